@@ -147,10 +147,13 @@ __device__ __forceinline__ void load_to_lds(const void* src, void* lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(at), "v"(src)
                : "memory", "m0");
 }
-// The wait is the builtin: the compiler then knows that its own earlier loads are
-// there too and does not wait for them among the next stage's.
+// The wait (for all but the wave's last LEFT loads, and for its LDS reads) is the
+// builtin: the compiler then knows that its own earlier loads are there too and
+// does not wait for them among the next stage's.
+template <int LEFT = 0>
 __device__ __forceinline__ void wait_lds_loads() {
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0), the other counters at their most
+  static_assert(LEFT < 64);
+  __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | (LEFT >> 4) << 14);  // vmcnt(LEFT), lgkmcnt(0)
   asm volatile("" ::: "memory");
 }
 

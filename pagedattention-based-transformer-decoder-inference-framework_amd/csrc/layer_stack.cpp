@@ -774,10 +774,13 @@ int LayerStack::moe(const Layer& l, int M, hipStream_t st) {
   g.lds = m.has_shared ? mm_pad(m.shared.ff) : 0;
   g.out = y_.p;
   g.ldo = ldx_;
-  g.max_n = 2 * std::max(m.expert.ff, m.has_shared ? m.shared.ff : 0);
+  g.shared_tiles = m.has_shared ? (M + r.tile_rows - 1) / r.tile_rows : 0;
+  g.routed_n = 2 * m.expert.ff;
+  g.shared_n = m.has_shared ? 2 * m.shared.ff : 0;
+  g.max_n = std::max(g.routed_n, g.shared_n);
   g.min_ks = (cfg_.width + mm_kstep(dt_) - 1) / mm_kstep(dt_);
   LLM_HIP_RET(mm_grouped_in(dt_, g, w_nt_, st));
-  g.max_n = cfg_.width;
+  g.routed_n = g.shared_n = g.max_n = cfg_.width;
   g.min_ks = (m.expert.ff + mm_kstep(dt_) - 1) / mm_kstep(dt_);
   LLM_HIP_RET(mm_grouped_out(dt_, g, w_nt_, st));
   return LLM_OK;

@@ -80,6 +80,8 @@ struct MmGrouped {
   int n_routed = 0, top = 0, M = 0;
   int max_tiles = 0;                // grid bound
   int tile_rows = 16;               // 16, 64 or 128: rows of a tile list entry
+  int routed_n = 0, shared_n = 0;   // columns of the routed groups, of the shared one
+  int shared_tiles = 0;             // list entries of the shared rows: the last ones
   int max_n = 0;                    // widest group's columns
   int min_ks = 0;
   const void* h = nullptr;          // [M][ldh] tokens' rows

@@ -6,8 +6,8 @@
 // Two kernels.  Decode rows stream: a block owns 16 MT rows x 16 NT columns, its
 // 8 waves split K and load A (row-major rows, 64 bytes per row and k-step) and W
 // (packed 1 KiB fragments) straight into registers, so every weight byte of the
-// product is in flight at once.  Prompt rows go through LDS in 128 x 128 (or 64 x
-// 128) blocks, both operands loaded from memory into LDS in fragment order.
+// product is in flight at once.  More rows go through LDS in blocks of 64 x 32 to
+// 128 x 256, both operands loaded from memory straight into LDS.
 // Grouped rows take either form; a tile list (built by the routing kernel) names
 // the group and rows of each row of the grid.
 // A and W share the k order inside a fragment, so the sum is exact whatever the
@@ -19,6 +19,7 @@
 #pragma once
 
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "mm.hpp"
@@ -114,10 +115,10 @@ struct Block {
 };
 
 template <typename T, int EPI>
-__device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_blocks) {
+__device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_block, int by) {
   Block<T> b;
   if constexpr (EPI == kGroupIn || EPI == kGroupOut) {
-    const MmTile t = p.g.tiles[blockIdx.y];
+    const MmTile t = p.g.tiles[by];
     const MmGroup g = p.g.groups[t.group];
     b.shared = t.group >= p.g.n_routed;
     b.m0 = t.row0;
@@ -143,7 +144,7 @@ __device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_blocks
     b.M = p.a.M;
     b.N = p.a.N;
     b.KS = p.KS;
-    b.m0 = (int)blockIdx.y * row_blocks;
+    b.m0 = by * row_block;
     b.glu = p.glu;
     if constexpr (EPI == kHeads) {
       b.A += blockIdx.z * p.heads.a_head;
@@ -153,9 +154,9 @@ __device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_blocks
   return b;
 }
 
-// This lane's 16 bytes of the first k-step of row m's fragments.
+// Row m of A (the last one for rows past it).
 template <typename T, int EPI>
-__device__ __forceinline__ const char* a_lane(const KernelArgs& p, const Block<T>& b, int m) {
+__device__ __forceinline__ const char* a_row(const KernelArgs& p, const Block<T>& b, int m) {
   m = min(m, b.M - 1);
   if constexpr (EPI == kGroupIn) {
     if (!b.shared) m = p.g.perm[m] / p.g.top;
@@ -169,9 +170,9 @@ __device__ __forceinline__ const char* a_lane(const KernelArgs& p, const Block<T
     int page = r.table[(size_t)r.slot[m] * r.max_tiles + min(pos / kPageTokens, r.max_tiles - 1)];
     page = min(max(page, 0), r.num_pages - 1);
     return static_cast<const char*>(r.pool) + (size_t)page * r.page_stride +
-           (size_t)(pos % kPageTokens) * r.row * sizeof(T) + 16 * (lane_id() >> 4);
+           (size_t)(pos % kPageTokens) * r.row * sizeof(T);
   }
-  return reinterpret_cast<const char*>(b.A + (size_t)m * b.lda) + 16 * (lane_id() >> 4);
+  return reinterpret_cast<const char*>(b.A + (size_t)m * b.lda);
 }
 
 template <int EPI>
@@ -189,6 +190,8 @@ struct RowOf {
   int m = -1;             // -1: no such row
   int at = 0, entry = 0;  // paged: place in the page, page-table entry of head 0 (-1: none)
   int pos = 0;
+  int out = 0;            // kGroupOut: the row's place in the output, its weight
+  float weight = 1.f;
 
   __device__ __forceinline__ RowOf() {}
   template <typename T>
@@ -201,6 +204,9 @@ struct RowOf {
       const int tile = pos / kPageTokens;
       at = pos % kPageTokens;
       entry = tile < e.max_tiles ? e.slot[m] * e.G * e.max_tiles + tile : -1;
+    } else if constexpr (EPI == kGroupOut) {
+      out = b.shared ? p.g.M * p.g.top + m : p.g.perm[m];
+      if (!b.shared) weight = p.g.weight[out];
     }
   }
 };
@@ -265,9 +271,8 @@ struct Target {
       T* d = static_cast<T*>(b.shared ? p.g.act_shared : p.g.act);
       p0 = d + (size_t)m * (b.shared ? p.g.lds : p.g.lda) + (n >> 1);
     } else if constexpr (EPI == kGroupOut) {
-      const int row = b.shared ? p.g.M * p.g.top + m : p.g.perm[m];
-      if (!b.shared) cs = p.g.weight[row];
-      float* d = p.g.out + (size_t)row * p.g.ldo + n;
+      cs = r.weight;
+      float* d = p.g.out + (size_t)r.out * p.g.ldo + n;
       p0 = d;
       p1 = n + 1 < b.N ? d + 1 : nullptr;
     } else if constexpr (EPI == kSplit) {
@@ -426,76 +431,268 @@ struct Target {
   }
 };
 
-// A column of 16 x 16 tiles of finished sums (tile i's rows m0 + 16 i .., columns
-// n0 ..) -> the epilogue, a column pair per lane.  Every lane of the wave takes
-// part; rows are what row_of() found for this lane.
-template <typename T, int EPI, int MT>
-struct TileRows {
-  RowOf<EPI> r[MT][2];
-  __device__ __forceinline__ TileRows(const KernelArgs& p, const Block<T>& b, int m0) {
-    const int lane = lane_id(), first = m0 + 4 * (lane >> 4) + (lane & 1 ? 2 : 0);
+// 16 MT rows from m0 on and 16 NT columns from n0 on, straight from the accumulators,
+// a column pair per lane: 64 bytes of a line per store, enough for fp32 results.
+// Every lane of the wave takes part.
+template <typename T, int EPI, int MT, int NT>
+__device__ __forceinline__ void emit_pairs(const KernelArgs& p, const Block<T>& b,
+                                           const f32x4 (&acc)[MT][NT], int m0, int n0) {
+  const int lane = lane_id(), first = m0 + 4 * (lane >> 4) + (lane & 1 ? 2 : 0);
+  const bool odd = lane & 1;
+  RowOf<EPI> rows[MT][2];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+  for (int i = 0; i < MT; ++i)
 #pragma unroll
-      for (int k = 0; k < 2; ++k) r[i][k] = RowOf<EPI>(p, b, first + 16 * i + k);
+    for (int r = 0; r < 2; ++r) rows[i][r] = RowOf<EPI>(p, b, first + 16 * i + r);
+#pragma unroll
+  for (int j = 0; j < NT; ++j) {
+    const int n = n0 + 16 * j + (lane & 14);
+    const ColOf<EPI> col(p, b, n);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const f32x4 c = acc[i][j];
+      f32x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = mov_dpp<0xB1>(c[r]);  // the neighbouring column
+#pragma unroll
+      for (int r = 0; r < 2; ++r) {
+        Target<T, EPI> t;
+        t.find(p, b, rows[i][r], col);
+        t.put(p, b, n, odd ? o[2 + r] : c[r], odd ? c[2 + r] : o[r]);
+      }
+    }
+  }
+}
+
+template <typename T>
+__device__ __forceinline__ void put_eight(T* p, const float (&v)[8]) {
+  constexpr int E = 16 / sizeof(T);
+  typedef T chunk_t __attribute__((ext_vector_type(E)));
+#pragma unroll
+  for (int k = 0; k < 8; k += E) {
+    chunk_t o;
+#pragma unroll
+    for (int e = 0; e < E; ++e) o[e] = (T)v[k + e];
+    *reinterpret_cast<chunk_t*>(p + k) = o;
+  }
+}
+// rows of ld elements that all start at 16 bytes
+template <typename T>
+__device__ __forceinline__ bool whole(const void* p, size_t ld) {
+  return ((reinterpret_cast<uintptr_t>(p) | ld * sizeof(T)) & 15) == 0;
+}
+
+// Where columns n .. n + 7 (n a multiple of 8) of a row go in stores of 16 bytes, and
+// what they still need.  ok: sizes and places allow it; else they go pair by pair.
+template <typename T, int EPI>
+struct Eight {
+  bool ok = false;
+  void* p0 = nullptr;  // NULL: nothing to write
+  void* p1 = nullptr;
+  bool turned = false;
+  float2 turn[4];
+
+  __device__ __forceinline__ void find(const KernelArgs& p, const Block<T>& b, const RowOf<EPI>& r,
+                                       const ColOf<EPI>& c) {
+    const int m = r.m, n = c.n;
+    ok = true;
+    if (m < 0 || n < 0) return;
+    ok = n + 8 <= b.N;
+    if constexpr (EPI == kGroupIn) {
+      const int ld = b.shared ? p.g.lds : p.g.lda;
+      T* d = static_cast<T*>(b.shared ? p.g.act_shared : p.g.act);
+      ok = ok && whole<T>(d, ld);
+      p0 = d + (size_t)m * ld + (n >> 1);
+    } else if constexpr (EPI == kGlu) {
+      ok = ok && whole<T>(p.split.t, p.split.ldt);
+      p0 = static_cast<T*>(p.split.t) + (size_t)m * p.split.ldt + (n >> 1);
+    } else if constexpr (EPI == kLatent) {
+      const MmLatent& e = p.lat;
+      ok = ok && ((e.D | e.rot) & 7) == 0 && whole<T>(e.q, e.ldq) && whole<float>(e.down, e.ldd);
+      if (c.part) {
+        p1 = e.down + (size_t)m * e.ldd + c.d;
+        return;
+      }
+      p0 = static_cast<T*>(e.q) + ((size_t)m * e.H + c.head) * e.ldq + c.d;
+      if (c.d < e.D) return;
+      ok = ok && whole<T>(e.q_lat, e.ld_lat) && whole<T>(nullptr, e.lat_rot);
+      p1 = static_cast<T*>(e.q_lat) + ((size_t)m * e.H + c.head) * e.ld_lat + e.lat_rot + (c.d - e.D);
+      if (ok) angles(e.turn + (size_t)m * (e.rot >> 1) + ((c.d - e.D) >> 1));
+    } else if constexpr (EPI == kQkv || EPI == kExpand) {
+      const MmQkv& e = p.q;
+      ok = ok && c.part < 2 && ((e.D | e.rot | e.Dp) & 7) == 0;
+      if (!ok) return;
+      if (c.d < e.rot) angles(e.turn + (size_t)m * (e.rot >> 1) + (c.d >> 1));
+      if (c.part == 0) {
+        p0 = static_cast<T*>(e.q) + ((size_t)m * e.H + c.head) * e.Dp + c.d;
+      } else if (r.entry >= 0) {
+        T* page = page_at<T>(e, e.k_pool, r.entry, c.head);
+        if (page) p0 = page + (size_t)r.at * e.Dp + c.d;
+      }
+    } else {
+      ok = false;
+    }
+  }
+
+  __device__ __forceinline__ void put(const KernelArgs& p, const Block<T>& b, int n, float (&v)[8]) const {
+    if constexpr (EPI == kGroupIn || EPI == kGlu) {
+      if (!p0) return;
+      typedef T half_t __attribute__((ext_vector_type(4)));
+      half_t o;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) o[k] = (T)glu(v[2 * k], v[2 * k + 1], b.glu);
+      *static_cast<half_t*>(p0) = o;
+    } else if constexpr (EPI == kLatent) {
+      if (!p0) {
+        if (p1) put_eight(static_cast<float*>(p1), v);
+        return;
+      }
+      rotate(v);
+      put_eight(static_cast<T*>(p0), v);
+      if (p1) put_eight(static_cast<T*>(p1), v);
+    } else if constexpr (EPI == kQkv || EPI == kExpand) {
+      if (!p0) return;
+      rotate(v);
+      put_eight(static_cast<T*>(p0), v);
+    }
+  }
+
+ private:
+  __device__ __forceinline__ void angles(const float2* t) {
+    turned = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) turn[k] = t[k];
+  }
+  __device__ __forceinline__ void rotate(float (&v)[8]) const {
+    if (!turned) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float v0 = v[2 * k], v1 = v[2 * k + 1];
+      v[2 * k] = v0 * turn[k].x - v1 * turn[k].y;
+      v[2 * k + 1] = v1 * turn[k].x + v0 * turn[k].y;
+    }
   }
 };
 
-template <typename T, int EPI, int MT, int NT>
-__device__ __forceinline__ void emit_column(const KernelArgs& p, const Block<T>& b,
-                                            const TileRows<T, EPI, MT>& rows, const f32x4 (&acc)[MT][NT],
-                                            int j, int m0, int n0) {
-  const int lane = lane_id();
-  const bool odd = lane & 1;
-  if constexpr (RowOf<EPI>::PAGED) {
-    // values lie token by token: a lane's four rows of its own column are one
-    // store where they are tokens 4 t .. 4 t + 3 of a sequence
-    if (n0 >= (p.q.H + p.q.G) * p.q.D) {
-      typedef T quad_t __attribute__((ext_vector_type(4)));
-      const ColOf<EPI> col(p, b, n0 + (lane & 15));
+// Value columns [c0, c1) of a block's sums: they lie token by token in their pages.
+// Rows of a few sequences: four tokens of a page that lie together are one store,
+// sixteen lanes a page's line.  Rows of many: a row per thread, so that its page is
+// looked up once for the columns it takes.
+template <typename T, int EPI, int ROWS, int STRIDE, int THREADS>
+__device__ __forceinline__ void emit_values(const KernelArgs& p, const Block<T>& b, const float* sums,
+                                            int first_col, int c0, int c1) {
+  const MmQkv& e = p.q;
+  const int rows = min(ROWS, b.M - b.m0);
+  if (rows <= 0 || c0 >= c1) return;
+  unsigned long long starts[ROWS / 64];  // rows that begin a sequence's
+  int sequences = 0;
 #pragma unroll
-      for (int i = 0; i < MT; ++i) {
-        const int m = m0 + 16 * i + 4 * (lane >> 4);
-        const RowOf<EPI> lo(p, b, m), hi(p, b, m + 3);
-        if (lo.m < 0 || col.n < 0) continue;
-        if (hi.m >= 0 && (lo.at & 3) == 0 && hi.pos == lo.pos + 3 && hi.entry == lo.entry) {
-          if (lo.entry < 0) continue;
-          T* page = page_at<T>(p.q, p.q.v_pool, lo.entry, col.head);
-          if (!page) continue;
-          quad_t v;
+  for (int h = 0; h < ROWS / 64; ++h) {
+    const int r = 64 * h + lane_id();
+    starts[h] = __ballot(r < rows && (r == 0 || e.slot[b.m0 + r] != e.slot[b.m0 + r - 1]));
+    sequences += __popcll(starts[h]);
+  }
+  const auto put = [&](const RowOf<EPI>& row, int r, int col) {
+    if (row.m < 0 || row.entry < 0) return;
+    const ColOf<EPI> c(p, b, col);
+    T* page = page_at<T>(e, e.v_pool, row.entry, c.head);
+    if (page)
+      page[(size_t)c.d * kPageTokens + v_page_slot(row.at, Kind<T>::BF16)] =
+          (T)sums[r * STRIDE + col - first_col];
+  };
+  if (sequences > 4) {
+    const int r = threadIdx.x % ROWS;
+    const RowOf<EPI> row(p, b, b.m0 + r);
+#pragma unroll 4
+    for (int col = c0 + threadIdx.x / ROWS; col < c1; col += THREADS / ROWS) put(row, r, col);
+    return;
+  }
+  typedef T quad_t __attribute__((ext_vector_type(4)));
 #pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (T)acc[i][j][r];
-          *reinterpret_cast<quad_t*>(page + (size_t)col.d * kPageTokens +
-                                     v_page_slot(lo.at, Kind<T>::BF16)) = v;
+  for (int h = 0; h < ROWS / 64; ++h) {
+    for (unsigned long long left = starts[h]; left; left &= left - 1) {
+      const int s0 = 64 * h + __ffsll(left) - 1;  // the sequence's rows: [s0, s1)
+      const unsigned long long after = left & (left - 1);
+      int s1 = after ? 64 * h + __ffsll(after) - 1 : rows;
+      if (!after && h + 1 < ROWS / 64 && starts[ROWS / 64 - 1]) s1 = 64 * (h + 1) + __ffsll(starts[ROWS / 64 - 1]) - 1;
+      const int pos0 = e.pos[b.m0 + s0], slot = e.slot[b.m0 + s0], off = pos0 & 3;
+      const int chunks = ((off + s1 - s0 + 3) / 4 + 15) / 16;  // of sixteen quads
+      for (int i = threadIdx.x; i < (c1 - c0) * chunks * 16; i += THREADS) {
+        const int rest = i >> 4, col = c0 + rest / chunks;
+        const int r0 = s0 + 4 * (16 * (rest % chunks) + (i & 15)) - off;
+        if (r0 >= s1) continue;
+        const int pos = pos0 + r0 - s0, tile = pos / kPageTokens;
+        if (tile >= e.max_tiles) continue;
+        const ColOf<EPI> c(p, b, col);
+        T* page = page_at<T>(e, e.v_pool, slot * e.G * e.max_tiles + tile, c.head);
+        if (!page) continue;
+        const float* v = sums + r0 * STRIDE + (col - first_col);
+        T* to = page + (size_t)c.d * kPageTokens + v_page_slot(pos % kPageTokens, Kind<T>::BF16);
+        if (r0 >= s0 && r0 + 4 <= s1) {
+          quad_t o;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) o[k] = (T)v[k * STRIDE];
+          *reinterpret_cast<quad_t*>(to) = o;
         } else {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const RowOf<EPI> row(p, b, m + r);
-            if (row.m < 0 || row.entry < 0) continue;
-            T* page = page_at<T>(p.q, p.q.v_pool, row.entry, col.head);
-            if (page)
-              page[(size_t)col.d * kPageTokens + v_page_slot(row.at, Kind<T>::BF16)] = (T)acc[i][j][r];
+          for (int k = 0; k < 4; ++k)
+            if (r0 + k >= s0 && r0 + k < s1) to[k] = (T)v[k * STRIDE];
+        }
+      }
+    }
+  }
+}
+
+// A block's finished sums, row by row in LDS -> the epilogue, eight columns of a row
+// per thread, so that stores are whole lines and a page or a head is looked up once
+// for eight columns (straight from the accumulators, a pair of columns per lane and
+// 16 to 32 bytes of a line per store: expansion of 2011 x 4096 x 512 58 us, now 36;
+// latent projections of 2011 x 3648 x 2048 45 us, now 37).
+template <typename T, int EPI, int ROWS, int COLS, int STRIDE, int THREADS>
+__device__ __forceinline__ void emit_block(const KernelArgs& p, const Block<T>& b, const float* sums,
+                                           int first_col) {
+  constexpr int ACROSS = COLS / 8, PER = ROWS * ACROSS / THREADS, BATCH = PER < 4 ? PER : 4;
+  static_assert(THREADS % ACROSS == 0 && PER >= 1 && PER % BATCH == 0);
+  const int row0 = threadIdx.x / ACROSS, col0 = threadIdx.x % ACROSS * 8, n = first_col + col0;
+  int end = b.N;  // of the columns that go by rows
+  if constexpr (RowOf<EPI>::PAGED) end = min(b.N, (p.q.H + p.q.G) * p.q.D);
+  if (n < end) {
+    const ColOf<EPI> c(p, b, n);
+#pragma unroll 1
+    for (int i0 = 0; i0 < PER; i0 += BATCH) {
+      RowOf<EPI> r[BATCH];
+      Eight<T, EPI> t[BATCH];
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) r[i] = RowOf<EPI>(p, b, b.m0 + row0 + (i0 + i) * (THREADS / ACROSS));
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) t[i].find(p, b, r[i], c);
+#pragma unroll
+      for (int i = 0; i < BATCH; ++i) {
+        if (r[i].m < 0) continue;
+        float v[8];
+        const float* s = sums + (size_t)(row0 + (i0 + i) * (THREADS / ACROSS)) * STRIDE + col0;
+#pragma unroll
+        for (int k = 0; k < 8; k += 4) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(s + k);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[k + e] = x[e];
+        }
+        if (t[i].ok) {
+          t[i].put(p, b, n, v);
+        } else {
+#pragma unroll 1
+          for (int k = 0; k < 8 && n + k < end; k += 2) {
+            Target<T, EPI> g;
+            g.find(p, b, r[i], ColOf<EPI>(p, b, n + k));
+            g.put(p, b, n + k, s[k], s[k + 1]);
           }
         }
       }
-      return;
     }
   }
-  const int n = n0 + (lane & 14);
-  const ColOf<EPI> col(p, b, n);
-#pragma unroll
-  for (int i = 0; i < MT; ++i) {
-    const f32x4 c = acc[i][j];
-    f32x4 o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = mov_dpp<0xB1>(c[r]);  // the neighbouring column
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      Target<T, EPI> t;
-      t.find(p, b, rows.r[i][r], col);
-      t.put(p, b, n, odd ? o[2 + r] : c[r], odd ? c[2 + r] : o[r]);
-    }
-  }
+  if constexpr (RowOf<EPI>::PAGED)
+    emit_values<T, EPI, ROWS, STRIDE, THREADS>(p, b, sums, first_col, max(first_col, end),
+                                               min(first_col + COLS, b.N));
 }
 
 // Decode rows (and short grouped tiles): a block owns 16 MT rows x 16 NT columns
@@ -507,14 +704,14 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
   constexpr int U = MT * NT >= 4 ? 2 : 4;  // k-steps per load batch
   const int lane = lane_id();
   const int w = wave_id_uniform();
-  const Block<T> b = block_of<T, EPI>(p, 16 * MT);
+  const Block<T> b = block_of<T, EPI>(p, 16 * MT, blockIdx.y);
   const int ntiles = (b.N + 15) >> 4;
   const int nt0 = (int)blockIdx.x * NT;
   if (nt0 >= ntiles) return;  // (groups differ in width)
 
   const char* ap[MT];
 #pragma unroll
-  for (int i = 0; i < MT; ++i) ap[i] = a_lane<T, EPI>(p, b, b.m0 + 16 * i + (lane & 15));
+  for (int i = 0; i < MT; ++i) ap[i] = a_row<T, EPI>(p, b, b.m0 + 16 * i + (lane & 15)) + 16 * (lane >> 4);
   const char* bp[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -612,73 +809,207 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
   }
 }
 
-// Prompt rows: a block of 16 MB rows x 128 columns, 4 waves as WM x (4 / WM).
-// Fragments go from memory straight into LDS (A gathered row by row, W linear),
-// two k-steps per stage, the next stage in flight while one is multiplied.
-template <typename T, int EPI, int MB, int WM>
-__global__ __launch_bounds__(256, 2) void mm_block_kernel(KernelArgs p) {
-  if constexpr (EPI == kGroupIn || EPI == kGroupOut)
-    if ((int)blockIdx.y >= *p.g.n_tiles) return;
-  constexpr int NB = 8, WN = 4 / WM, MT = MB / WM, NT = NB / WN;
-  constexpr int AW = MB / 4, BW = NB / 4;  // row / column tiles a wave loads
-  __shared__ u32x4 sa[2][2][MB][64];       // [stage][k-step][tile][lane]
-  __shared__ u32x4 sb[2][2][NB][64];
+// Workgroups go round the XCDs in turn.  Block id -> tile of an nx wide grid, in a
+// walk whose neighbours are the blocks of one XCD: they share rows of A and columns
+// of W in its L2, eight row blocks at a time.
+struct TileAt {
+  int x = 0, y = 0;
+};
+__device__ __forceinline__ TileAt xcd_tile(int id, int nx, int ny) {
+  const int total = nx * ny, xcd = id & 7, each = total >> 3, more = total & 7;
+  const int t = xcd * each + min(xcd, more) + (id >> 3);
+  const int group = t / (8 * nx), r = t - group * 8 * nx, rows = min(8, ny - 8 * group);
+  return {r / rows, 8 * group + r % rows};
+}
+
+// blocks of 16 NB columns in n columns
+__host__ __device__ __forceinline__ int group_across(int n, int NB) { return (n + 16 * NB - 1) / (16 * NB); }
+
+// A block of 16 MB rows x 16 NB columns, WM x WN waves.  Both operands
+// go from memory straight into LDS, ST stages of two k-steps in flight; while a
+// wave multiplies one k-step it reads the fragments of the next.  It waits for its
+// own loads of a stage alone; the barrier then makes them everyone's and frees the
+// stage that was read before.  The loads are spread among the matrix instructions:
+// issued together they hold up the wave while the matrix cores run dry.
+// A load of A takes 8 rows x 128 bytes, whole cache lines (16 rows x 64 bytes, the
+// fragment itself, took 1.7 times as long per byte); the 16-byte chunks of a row
+// are exchanged by (row / 2) so that a fragment's 16 rows lie in different banks.
+// Bound by the matrix cores waiting at the barriers: 2048 x 2048 x 6144 48.6 us, 1060
+// TFLOP/s (113 us with two k-steps loaded and waited for together in 128 x 128 blocks
+// of four waves); 2048 x 12288 x 2048 101 us (143), 700 x 2048 x 2048 12.3 us (32).
+template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
+__global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p) {
+  constexpr int WAVES = WM * WN, MT = MB / WM, NT = NB / WN;
+  constexpr int LOADS = 2 * (MB + NB) / WAVES;  // of a wave and stage, 1 KiB each
+  static_assert(2 * (MB + NB) % WAVES == 0);
+  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];  // per stage: A, two k-steps a tile; W, tile by tile
+  int id = blockIdx.y * gridDim.x + blockIdx.x;
+  TileAt tile;
+  if constexpr (EPI == kGroupIn || EPI == kGroupOut) {
+    // the shared expert's tiles (the last of the list, the most columns or k-steps)
+    // go first; each kind is dealt out over the XCDs by itself
+    const int across = group_across(p.g.shared_n, NB), shared = p.g.shared_tiles * across;
+    const int routed = *p.g.n_tiles - p.g.shared_tiles;
+    if (id < shared) {
+      tile = xcd_tile(id, across, p.g.shared_tiles);
+      tile.y += routed;
+    } else {
+      id -= shared;
+      const int nx = group_across(p.g.routed_n, NB);
+      if (id >= routed * nx) return;
+      tile = xcd_tile(id, nx, routed);
+    }
+  } else {
+    tile = xcd_tile(id, gridDim.x, gridDim.y);
+  }
   const int lane = lane_id();
   const int w = wave_id_uniform();
-  const Block<T> b = block_of<T, EPI>(p, 16 * MB);
+  const Block<T> b = block_of<T, EPI>(p, 16 * MB, tile.y);
   const int ntiles = (b.N + 15) >> 4;
-  const int nt0 = (int)blockIdx.x * NB;
-  if (nt0 >= ntiles) return;
+  const int nt0 = tile.x * NB;
+  const int KS = b.KS, stages = KS >> 1;
 
-  const char* ap[AW];
+  // load l of a stage: rows 8 l .. 8 l + 7 of A (l < 2 MB), then the two k-steps of
+  // each of W's column tiles
+  const char* src[LOADS];
+  const int l0 = w * LOADS;
 #pragma unroll
-  for (int i = 0; i < AW; ++i)
-    ap[i] = a_lane<T, EPI>(p, b, b.m0 + 16 * (w * AW + i) + (lane & 15));
-  const char* bp[BW];
-#pragma unroll
-  for (int j = 0; j < BW; ++j)
-    bp[j] = b.W + (size_t)min(nt0 + w * BW + j, ntiles - 1) * b.KS * 1024 + lane * 16;
-  auto issue = [&](int st, int ks) {
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (ks + u >= b.KS) break;
-#pragma unroll
-      for (int i = 0; i < AW; ++i) load_to_lds(ap[i] + (size_t)(ks + u) * 64, sa[st][u][w * AW + i]);
-#pragma unroll
-      for (int j = 0; j < BW; ++j)
-        load_to_lds(bp[j] + (size_t)(ks + u) * 1024, sb[st][u][w * BW + j]);
+  for (int i = 0; i < LOADS; ++i) {
+    const int l = l0 + i;
+    if (l < 2 * MB) {
+      const int r = 8 * l + (lane >> 3);
+      src[i] = a_row<T, EPI>(p, b, b.m0 + r) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    } else {
+      src[i] = b.W + (size_t)min(nt0 + (l >> 1) - MB, ntiles - 1) * KS * 1024 + (l & 1) * 1024 + lane * 16;
     }
+  }
+  auto issue = [&](int st, int i) {
+    load_to_lds(src[i], lds[st][l0 + i]);
+    src[i] += l0 + i < 2 * MB ? 128 : 2048;
   };
   const int wm = w / WN, wn = w % WN;
+  const bool rows_here = b.m0 + 16 * wm * MT < b.M;  // (short blocks: the others load and wait)
   f32x4 acc[MT][NT];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
     for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  auto mul = [&](int st, int u) {
+  struct Frags {
     u32x4 a[MT], c[NT];
+  };
+  const int ar = lane & 15;  // this lane's row of a fragment, and its chunks of the two k-steps
+  const int at0 = 8 * ar + ((lane >> 4) ^ (ar >> 1)), at1 = at0 ^ 4;
+  auto read = [&](Frags& f, int st, int u) {
 #pragma unroll
-    for (int i = 0; i < MT; ++i) a[i] = sa[st][u][wm * MT + i][lane];
+    for (int i = 0; i < MT; ++i) f.a[i] = (&lds[st][2 * (wm * MT + i)][0])[u ? at1 : at0];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) c[j] = sb[st][u][wn * NT + j][lane];
+    for (int j = 0; j < NT; ++j) f.c[j] = lds[st][2 * (MB + wn * NT + j) + u][lane];
+  };
+  // multiplies, with loads [FROM, TO) of stage st among the products
+  auto mul = [&](const Frags& f, int st, auto from, auto to) {
+    constexpr int FROM = decltype(from)::value, TO = decltype(to)::value, N = MT * NT;
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      if constexpr (TO > FROM) {
+#pragma unroll
+        for (int i = FROM; i < TO; ++i)
+          if ((i - FROM) * N / (TO - FROM) == t) {
+            issue(st, i);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      const int i = t / NT, j = t % NT;
+      acc[i][j] = Kind<T>::mma(f.a[i], f.c[j], acc[i][j]);
+    }
+  };
+  using Zero = std::integral_constant<int, 0>;
+  using Half = std::integral_constant<int, LOADS / 2>;
+  using All = std::integral_constant<int, LOADS>;
+  const Zero zero;
+  const Half half;
+  const All all;
+  if (stages > 0) {
+#pragma unroll
+    for (int s = 0; s < ST; ++s)
+      if (s < stages) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue(s, i);
+      }
+    Frags x, y;
+    if (stages >= ST) wait_lds_loads<(ST - 1) * LOADS>();
+    else wait_lds_loads<0>();
+    __builtin_amdgcn_s_barrier();
+    if (rows_here) {
+      read(x, 0, 0);
+      read(y, 0, 1);
+      mul(x, 0, zero, zero);
+    }
+    int st = 0;
+    auto landed = [&](int s) {  // stage s + 1 is there for everyone, stage s read out
+      if (s + ST <= stages) wait_lds_loads<(ST - 2) * LOADS>();
+      else wait_lds_loads<0>();
+      __builtin_amdgcn_s_barrier();
+    };
+    landed(0);
+    int s = 0;
+    for (; s + ST < stages; ++s) {
+      const int now = st;
+      st = st + 1 == ST ? 0 : st + 1;
+      if (rows_here) {
+        read(x, st, 0);
+        mul(y, now, zero, half);
+        read(y, st, 1);
+        mul(x, now, half, all);
+      } else {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue(now, i);
+      }
+      landed(s + 1);
+    }
+    for (; s + 1 < stages; ++s) {
+      st = st + 1 == ST ? 0 : st + 1;
+      if (rows_here) {
+        read(x, st, 0);
+        mul(y, 0, zero, zero);
+        read(y, st, 1);
+        mul(x, 0, zero, zero);
+      }
+      landed(s + 1);
+    }
+    if (rows_here) mul(y, 0, zero, zero);
+  }
+  if (KS & 1) {  // the last k-step of an odd number, from memory
+    Frags f;
 #pragma unroll
     for (int i = 0; i < MT; ++i)
+      f.a[i] = *reinterpret_cast<const u32x4*>(a_row<T, EPI>(p, b, b.m0 + 16 * (wm * MT + i) + ar) +
+                                               (size_t)(KS - 1) * 64 + 16 * (lane >> 4));
 #pragma unroll
-      for (int j = 0; j < NT; ++j) acc[i][j] = Kind<T>::mma(a[i], c[j], acc[i][j]);
-  };
-  issue(0, 0);
-  int st = 0;
-  for (int ks = 0; ks < b.KS; ks += 2, st ^= 1) {
-    wait_lds_loads();
-    __syncthreads();  // stage st has landed, stage st ^ 1 is read out
-    if (ks + 2 < b.KS) issue(st ^ 1, ks + 2);
-    mul(st, 0);
-    if (ks + 1 < b.KS) mul(st, 1);
+    for (int j = 0; j < NT; ++j)
+      f.c[j] = *reinterpret_cast<const u32x4*>(
+          b.W + ((size_t)min(nt0 + wn * NT + j, ntiles - 1) * KS + KS - 1) * 1024 + lane * 16);
+    mul(f, 0, zero, zero);
   }
-  const int m0 = b.m0 + 16 * wm * MT;
-  const TileRows<T, EPI, MT> rows(p, b, m0);
+  // 2048 x 12288 x 2048 with its activation 107 us by rows, 109 by pairs; 2011 x 8192
+  // split 80 and 77
+  constexpr bool BY_ROWS = EPI == kGroupIn || EPI == kGlu || EPI == kLatent || RowOf<EPI>::PAGED;
+  if constexpr (!BY_ROWS) {
+    emit_pairs<T, EPI>(p, b, acc, b.m0 + 16 * wm * MT, (nt0 + wn * NT) * 16);
+    return;
+  }
+  // (every wave has read its last fragments before the last barrier)
+  constexpr int STRIDE = 16 * NB + 4;
+  static_assert(sizeof(lds) >= sizeof(float) * 16 * MB * STRIDE);
+  float* sums = reinterpret_cast<float*>(&lds[0][0][0]);
 #pragma unroll
-  for (int j = 0; j < NT; ++j) emit_column(p, b, rows, acc, j, m0, (nt0 + wn * NT + j) * 16);
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sums[(16 * (wm * MT + i) + 4 * (lane >> 4) + r) * STRIDE + 16 * (wn * NT + j) + ar] = acc[i][j][r];
+  __syncthreads();
+  emit_block<T, EPI, 16 * MB, 16 * NB, STRIDE, 64 * WAVES>(p, b, sums, 16 * nt0);
 }
 
 template <int EPI>
@@ -693,11 +1024,53 @@ hipError_t stream(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <typename T, int EPI, int MB, int WM>
+template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
 hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
-  const dim3 grid((N + 127) / 128, row_blocks, heads_of<EPI>(p));
-  hipLaunchKernelGGL((mm_block_kernel<T, EPI, MB, WM>), grid, dim3(256), 0, st, p);
+  dim3 grid(group_across(N, NB), row_blocks, heads_of<EPI>(p));
+  if constexpr (EPI == kGroupIn || EPI == kGroupOut)
+    grid = dim3((p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, NB) +
+                p.g.shared_tiles * group_across(p.g.shared_n, NB));
+  hipLaunchKernelGGL((mm_block_kernel<T, EPI, MB, NB, WM, WN, ST>), grid, dim3(64 * WM * WN), 0,
+                     st, p);
   return hipGetLastError();
+}
+
+// A block form and the time of one round of its workgroups over the chip at K =
+// 2048, launch taken off (us).  A product takes the form with the least rounds x time:
+// 2048 x 12288: 3 rounds of 128 x 256, 101 us (128 x 128: 115); 2048 x 2048: one round
+// of 128 x 128, 21.5 us (128 x 256 leaves half the chip idle: 33); 700 x 2048: 64 x 128,
+// 12.2 us (128 x 128: 23); 64 x 12288: 64 x 64, 11.0 us (64 x 32: 13).
+template <typename T, int EPI>
+struct BlockForm {
+  int mb, nb;
+  float round;
+  hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
+};
+template <typename T, int EPI>
+hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipStream_t st) {
+  static constexpr BlockForm<T, EPI> forms[] = {{4, 2, 4.2f, blocks<T, EPI, 4, 2, 2, 2, 4>},
+                                                {4, 4, 6.2f, blocks<T, EPI, 4, 4, 2, 2, 3>},
+                                                {4, 8, 10.f, blocks<T, EPI, 4, 8, 2, 4, 4>},
+                                                {4, 16, 19.5f, blocks<T, EPI, 4, 16, 2, 4, 3>},
+                                                {8, 8, 18.5f, blocks<T, EPI, 8, 8, 4, 2, 3>},
+                                                {8, 16, 30.f, blocks<T, EPI, 8, 16, 2, 4, 3>}};
+  const BlockForm<T, EPI>* best = nullptr;
+  int best_y = 0;
+  float least = 0.f;
+  for (const BlockForm<T, EPI>& f : forms) {
+    if (f.mb < min_mb || f.mb > max_mb) continue;
+    const int y = (p.a.M + 16 * f.mb - 1) / (16 * f.mb);
+    int groups = group_across(N, f.nb) * y * heads_of<EPI>(p);
+    if constexpr (EPI == kGroupIn || EPI == kGroupOut)
+      groups = (p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, f.nb) +
+               p.g.shared_tiles * group_across(p.g.shared_n, f.nb);
+    const float cost = (float)((groups + 255) / 256) * f.round;
+    if (best && cost >= least) continue;
+    best = &f;
+    best_y = y;
+    least = cost;
+  }
+  return best->go(p, best_y, N, st);
 }
 
 template <typename T, int EPI>
@@ -705,41 +1078,40 @@ hipError_t launch(const KernelArgs& p, hipStream_t st) {
   const int M = p.a.M, N = p.a.N;
   const int ntiles = (N + 15) / 16;
   if (M <= 16) return stream<T, EPI, 1, 1>(p, 1, N, st);
-  if (M <= 64) {
-    // The form with the fewest rounds of workgroups over the chip, a round priced
-    // by its column tiles and the rows it reads: 64 x 12288 x 2048 17.4 us as 4 x 3
-    // tiles (one round) against 25.9 as 4 x 2, 64 x 8192 14.5 as 4 x 2 against 16.1.
-    struct Form {
-      int mt, nt;
-      float rows;
-      hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
-    };
-    static constexpr Form forms[] = {{1, 1, 0.5f, stream<T, EPI, 1, 1>}, {1, 2, 0.5f, stream<T, EPI, 1, 2>},
-                                     {2, 2, 1.5f, stream<T, EPI, 2, 2>}, {2, 3, 1.5f, stream<T, EPI, 2, 3>},
-                                     {4, 2, 3.f, stream<T, EPI, 4, 2>},  {4, 3, 3.f, stream<T, EPI, 4, 3>}};
-    const Form* best = nullptr;
-    int row_blocks = 0;
-    float least = 0.f;
-    for (const Form& f : forms) {
-      const int rb = (M + 16 * f.mt - 1) / (16 * f.mt);
-      const int groups = (ntiles + f.nt - 1) / f.nt * rb * heads_of<EPI>(p);
-      const float cost = (float)((groups + 255) / 256) * ((float)f.nt + f.rows);
-      if (best && cost >= least) continue;
-      best = &f;
-      least = cost;
-      row_blocks = rb;
-    }
-    return best->go(p, row_blocks, N, st);
-  }
   if constexpr (EPI == kSplit) {
     // narrow products: all columns in two blocks, so a row is read twice
-    if (ntiles <= 10 && (M + 31) / 32 * 2 < 1024) return stream<T, EPI, 2, 5>(p, (M + 31) / 32, N, st);
+    if (M > 64 && ntiles <= 10 && (M + 31) / 32 * 2 < 1024)
+      return stream<T, EPI, 2, 5>(p, (M + 31) / 32, N, st);
   }
-  // prompt rows: blocks once there are enough of them, else 32-row streams
-  const int n128 = (N + 127) / 128 * heads_of<EPI>(p);
-  if ((M + 127) / 128 * n128 >= 256) return blocks<T, EPI, 8, 2>(p, (M + 127) / 128, N, st);
-  if ((M + 63) / 64 * n128 >= 128) return blocks<T, EPI, 4, 1>(p, (M + 63) / 64, N, st);
-  return stream<T, EPI, 2, 1>(p, (M + 31) / 32, N, st);
+  // Blocks once the smallest of them are more than half a round, else streams:
+  // 64 x 6144 x 1024 5.1 us as blocks (streams 5.3), 64 x 2048 x 6144 10.7 as
+  // streams (blocks 15.4), 128 x 2048 x 6144 16.3 as streams (blocks 17.5).
+  if (M > 32 && (M + 63) / 64 * ((N + 31) / 32) * heads_of<EPI>(p) > 128)
+    return launch_block<T, EPI>(p, 4, 8, N, st);
+  // The stream form with the fewest rounds of workgroups, a round priced by its
+  // column tiles and the rows it reads.
+  struct Form {
+    int mt, nt;
+    float rows;
+    hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
+  };
+  static constexpr Form forms[] = {{1, 1, 0.5f, stream<T, EPI, 1, 1>},
+                                   {1, 2, 0.5f, stream<T, EPI, 1, 2>},
+                                   {2, 2, 1.5f, stream<T, EPI, 2, 2>},
+                                   {2, 3, 1.5f, stream<T, EPI, 2, 3>}};
+  const Form* best = nullptr;
+  int row_blocks = 0;
+  float least = 0.f;
+  for (const Form& f : forms) {
+    const int rb = (M + 16 * f.mt - 1) / (16 * f.mt);
+    const int groups = (ntiles + f.nt - 1) / f.nt * rb * heads_of<EPI>(p);
+    const float cost = (float)((groups + 255) / 256) * ((float)f.nt + f.rows);
+    if (best && cost >= least) continue;
+    best = &f;
+    least = cost;
+    row_blocks = rb;
+  }
+  return best->go(p, row_blocks, N, st);
 }
 
 template <typename T, int EPI>
@@ -747,8 +1119,8 @@ hipError_t launch_grouped(const MmGrouped& g, int w_nt, hipStream_t st) {
   KernelArgs p{};
   p.g = g;
   p.a.w_nt = w_nt;
-  if (g.tile_rows == 128) return blocks<T, EPI, 8, 2>(p, g.max_tiles, g.max_n, st);
-  if (g.tile_rows == 64) return blocks<T, EPI, 4, 1>(p, g.max_tiles, g.max_n, st);
+  if (g.tile_rows > 16)
+    return launch_block<T, EPI>(p, g.tile_rows / 16, g.tile_rows / 16, g.max_n, st);
   // few k-steps per wave are not worth eight of them
   return g.min_ks >= 16 ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
                         : stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st);

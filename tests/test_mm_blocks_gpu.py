@@ -1,0 +1,55 @@
+"""The block form of the layer-stack models' products (mm_impl.hpp) where it can go
+wrong: one k-step and odd numbers of them, rows and columns that end inside a block,
+heads that whole 16-byte stores fit and do not fit, blocks of one, a few and many
+sequences at places of a page that are no multiple of four, short expert tiles."""
+import numpy as np
+import pytest
+
+import _layer_stack as T
+import _nubosun as N
+from test_layer_stack_gpu import serve, tokens  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# width, attention, experts, portions of the sequences in each step
+GEFARAX = {
+    "one_k_step": (32, T.attn(heads=96, kv_heads=8, dim=24, vdim=16, rot=16), None,
+                   [[17] * 7, [1] * 7, [31] * 7]),
+    "odd_k_steps": (96, T.attn(heads=48, kv_heads=6, dim=40, vdim=24, rot=16),
+                    T.moe(experts=4, top=2, ff=136, shared=200), [[70, 131, 50], [3, 2, 5], [61, 66, 129]]),
+    "pairs": (128, T.attn(heads=64, kv_heads=4, dim=20, vdim=10, rot=12),
+              T.moe(experts=8, top=3, ff=36, shared=40), [[33], [65], [130]]),
+    "many_rows": (160, T.attn(heads=20, kv_heads=2, dim=72, vdim=64, rot=40),
+                  T.moe(experts=3, top=2, ff=264, shared=300), [[127, 129, 1, 2, 60], [300]]),
+    "wide": (1056, T.attn(heads=32, kv_heads=4, dim=64, vdim=64, rot=32),
+             T.moe(experts=2, top=1, ff=520, shared=1032), [[391], [44, 28]]),
+}
+
+
+def check(serve, cfg, w, dtype, portions):  # noqa: F811
+    n = max(len(p) for p in portions)
+    lens = [sum(p[i] for p in portions if i < len(p)) for i in range(n)]
+    requests = {i: tokens(cfg, lens[i], 7 + i) for i in range(n)}
+    eng = serve(cfg, w, dtype, max_tokens=64 * n + sum(lens), max_seqs=n)
+    got = T.replay(eng, requests, [list(enumerate(p)) for p in portions])
+    for i in range(n):
+        T.check_rows(got[i], T.logits(cfg, w, requests[i]), dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("name", GEFARAX)
+def test_grouped_query_blocks(serve, name, dtype):  # noqa: F811
+    width, a, m, portions = GEFARAX[name]
+    cfg = T.config([(a, m)], width=width)
+    w = T.weights(cfg, 3)
+    check(serve, cfg, T.clear_choices(w) if dtype == "bfloat16" else w, dtype, portions)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("mixer", [N.latent(heads=48, dim=32, rot=16, vdim=24, rank=96),
+                                   N.latent(heads=36, dim=20, rot=12, vdim=14, rank=72)],
+                         ids=["whole", "pairs"])
+def test_latent_blocks(serve, mixer, dtype):  # noqa: F811
+    """Also the expansion of cached rows (portions of 65 tokens and more)."""
+    cfg = N.config([(mixer, N.dense(ff=1100))], width=136)
+    check(serve, cfg, N.weights(cfg, 5), dtype, [[70, 131, 90], [66, 1, 129]])
