@@ -1,5 +1,5 @@
-// Device token sampling: temperature / top-k / top-p over
-// the vocabulary, one workgroup per row, the row held in registers + LDS.
+// Device token sampling: temperature / top-k / top-p over the vocabulary, one
+// workgroup per row, the row held in registers.
 //
 // Reference semantics restated:
 //   * temperature + softmax: top_k_top_p_filter (attention/top_k_top_p_filter.cuh:55-88):
@@ -16,15 +16,22 @@
 //   * greedy (T <= 0 or top_k == 1): argmax, first maximum wins
 //     (sample_from_logits, decoder/cuda_decoder.cu:7-14).
 //
-// The rank / mass thresholds are found by a bitwise radix search over the
-// (non-negative) fp32 probability bit patterns: 31 block-wide count or sum
-// reductions per threshold, no sort.
+// The rank and mass thresholds are patterns of (non-negative) fp32 probabilities,
+// found ten bits at a time from histograms in LDS: three passes over the registers
+// for each, where a search bit by bit took 31 passes and block reductions for each
+// (64 rows of 50,257, top_k 40 and top_p 0.9: 461 us, now 36 us).  Bound by the
+// latency of the passes and of the LDS atomics, one row being one workgroup.  Masses
+// are added as whole multiples of 2^-50, so their sums are exact to 2^-34 and do not
+// depend on the order of the atomics.
 #include "common.hpp"
 #include "row_ops.hpp"
 
 namespace llm {
 
-constexpr int kSampleThreads = 512;  // 8 waves: 256 VGPRs per lane available
+constexpr int kSampleThreads = 1024;
+constexpr int kSampleWaves = kSampleThreads / 64;
+constexpr int kSampleSeg = 4 * kSampleThreads;  // tokens of a segment: 256 per wave, 4 per lane
+constexpr int kBins = 1024;
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
   z += 0x9E3779B97F4A7C15ull;
@@ -70,174 +77,287 @@ __device__ __forceinline__ T block_reduce(T v, T* sh, Op op) {
   return t;
 }
 
-// Thread t owns the contiguous tokens [t*VPT, t*VPT + VPT) of the row.  The
-// first VPT_REG of them live in registers, the rest in LDS (VPT 128: 128 KiB,
-// [slot][thread] so each access is bank-conflict free).
-template <int VPT>
-struct RowVals {
-  // register slots; the rest in LDS: VPT 64 -> 32 + 64 KiB, VPT 128 -> 56 + 144 KiB
-  static constexpr int R = VPT <= 32 ? VPT : (VPT <= 64 ? 32 : 56);
-  float reg[R];
-  // volatile: re-read per use, so the compiler does not hoist the LDS half into
-  // registers across the radix-search loops (that spilled)
-  volatile float* lds;  // [(VPT - R)][kSampleThreads]
-  // f(i, value&): register slots unrolled, LDS slots in a rolled loop (dynamic
-  // LDS indexing is free; unrolling it only made the compiler hoist and spill)
-  template <typename F>
-  __device__ __forceinline__ void each(F f) {
+__device__ __forceinline__ void put_token(const SampleArgs& a, int r, int tok) {
+  a.out[r] = tok;
+  if (a.out2) a.out2[(size_t)r * a.out2_stride] = tok;
+}
+
+// p as a multiple of 2^-50 (p in [0, 1])
+__device__ __forceinline__ unsigned long long mass_of(uint32_t bits) {
+  const int e = (int)(bits >> 23) - 100;
+  const unsigned long long m = (bits & 0x7FFFFFu) | (bits >> 23 ? 0x800000u : 0u);
+  return e >= 0 ? m << e : e > -24 ? m >> -e : 0;
+}
+
+// Of histogram bins hist[0 .. kBins): the largest bin whose sum with all bins above
+// it reaches `want`, and what is still wanted of that bin.  bin -1: all together do
+// not.  One bin per thread; every thread gets the answer.
+template <typename W>
+struct Found {
+  int bin;
+  W left;
+};
+template <typename W>
+__device__ __forceinline__ Found<W> find_bin(const W* hist, W want, W* part, Found<W>* found) {
+  static_assert(kBins == kSampleThreads);
+  const int lane = lane_id(), w = threadIdx.x >> 6;
+  const W own = hist[threadIdx.x];
+  W sum = own;  // of this wave's bins from here on
 #pragma unroll
-    for (int i = 0; i < R; ++i) f(i, reg[i]);
+  for (int off = 1; off < 64; off <<= 1) {
+    const W o = __shfl_down(sum, off, 64);
+    if (lane + off < 64) sum += o;
+  }
+  if (lane == 0) part[w] = sum;
+  if (threadIdx.x == 0) *found = {-1, want};
+  __syncthreads();
+  for (int i = w + 1; i < kSampleWaves; ++i) sum += part[i];
+  if (sum >= want && sum - own < want) *found = {(int)threadIdx.x, want - (sum - own)};
+  __syncthreads();
+  return *found;
+}
+
+// The largest pattern of the values (from `floor` on) that the weights of the values
+// from it on reach `want`; 0: all together do not.
+template <int NS, typename W, typename F>
+__device__ __forceinline__ uint32_t find_pattern(const float (&v)[NS][4], uint32_t floor, W want, W* hist,
+                                                 W* part, Found<W>* found, F weight) {
+  uint32_t at = 0;
 #pragma unroll 1
-    for (int i = R; i < VPT; ++i) {
-      float v = lds[(i - R) * kSampleThreads + threadIdx.x];
-      f(i, v);
-      lds[(i - R) * kSampleThreads + threadIdx.x] = v;
+  for (int shift = 20; shift >= 0; shift -= 10) {
+    hist[threadIdx.x] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        uint32_t bits = __float_as_uint(v[s][j]);
+        asm volatile("" : "+v"(bits));  // (weights kept over the passes would not fit the registers)
+        if (bits != 0 && bits >= floor && bits >> shift >> 10 == at)
+          atomicAdd(&hist[bits >> shift & (kBins - 1)], weight(bits));
+      }
+    __syncthreads();
+    const Found<W> f = find_bin(hist, want, part, found);
+    if (f.bin < 0) return 0;
+    at = at << 10 | (uint32_t)f.bin;
+    want = f.left;
+    __syncthreads();
+  }
+  return at;
+}
+
+// temperature <= 0 or top_k 1: the first maximum
+__global__ __launch_bounds__(kSampleThreads) void sample_greedy_kernel(SampleArgs a) {
+  __shared__ float shf[kSampleWaves];
+  __shared__ int shi[kSampleWaves];
+  const float* lg = a.logits + (size_t)blockIdx.x * a.V;
+  float best = -INFINITY;
+  int bi = 0x7fffffff;
+#pragma unroll 8
+  for (int i = threadIdx.x; i < a.V; i += kSampleThreads) {
+    const float v = lg[i];
+    if (v > best) {
+      best = v;
+      bi = i;
     }
   }
-};
+  const float m = block_reduce(best, shf, [](float x, float y) { return fmaxf(x, y); });
+  int cand = (best == m) ? bi : 0x7fffffff;
+  cand = block_reduce(cand, shi, [](int x, int y) { return min(x, y); });
+  if (threadIdx.x == 0) put_token(a, blockIdx.x, cand == 0x7fffffff ? 0 : cand);
+}
 
-template <int VPT>
+// A thread's tokens: 4 of each of NS segments, 64 apart, so that loads are whole
+// lines and a wave's 256 tokens of a segment (a cell) follow one another.
+template <int NS>
 __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs a) {
-  __shared__ float shf[16];
-  __shared__ int shi[16];
-  __shared__ uint32_t shu[16];
-  extern __shared__ float spill[];
-  const int r = blockIdx.x;
+  __shared__ float shf[kSampleWaves];
+  __shared__ uint32_t ranks[kBins], rank_part[kSampleWaves];
+  __shared__ unsigned long long masses[kBins], mass_part[kSampleWaves];
+  __shared__ Found<uint32_t> rank_found;
+  __shared__ Found<unsigned long long> mass_found;
+  __shared__ float cells[NS * kSampleWaves];
+  __shared__ int cell;
+  __shared__ float cell_left;
+  const int r = blockIdx.x, lane = lane_id(), w = wave_id_uniform();
   const float* lg = a.logits + (size_t)r * a.V;
-  const int base = threadIdx.x * VPT;
-  RowVals<VPT> p;
-  p.lds = spill;
-  const bool greedy = a.temperature <= 0.f || a.top_k == 1;
-  p.each([&](int i, float& v) { v = base + i < a.V ? lg[base + i] : -INFINITY; });
-
-  if (greedy) {
-    float best = -INFINITY;
-    int bi = 0x7fffffff;
-    p.each([&](int i, float& v) {  // first max in the chunk
-      if (v > best) { best = v; bi = base + i; }
-    });
-    const float m = block_reduce(best, shf, [](float x, float y) { return fmaxf(x, y); });
-    int cand = (best == m) ? bi : 0x7fffffff;
-    cand = block_reduce(cand, shi, [](int x, int y) { return min(x, y); });
-    if (threadIdx.x == 0) {
-      const int tok = cand == 0x7fffffff ? 0 : cand;
-      a.out[r] = tok;
-      if (a.out2) a.out2[(size_t)r * a.out2_stride] = tok;
+  const auto token = [&](int s, int j) { return s * kSampleSeg + w * 256 + j * 64 + lane; };
+  const auto done = [&](int tok) { put_token(a, r, tok); };
+  float v[NS][4];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if ((s + 1) * kSampleSeg <= a.V) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[s][j] = lg[token(s, j)];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[s][j] = token(s, j) < a.V ? lg[token(s, j)] : -INFINITY;
     }
-    return;
   }
 
   // temperature + softmax (reference: logits /= T; exp(x - max); / (sum + 1e-6))
   float mloc = -INFINITY;
-  p.each([&](int, float& v) {
-    v = v / a.temperature;
-    mloc = fmaxf(mloc, v);
-  });
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[s][j] = v[s][j] / a.temperature;
+      mloc = fmaxf(mloc, v[s][j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   const float m = block_reduce(mloc, shf, [](float x, float y) { return fmaxf(x, y); });
   float sloc = 0.f;
-  p.each([&](int i, float& v) {
-    v = base + i < a.V ? expf(v - m) : 0.f;
-    sloc += v;
-  });
-  const float s = block_reduce(sloc, shf, [](float x, float y) { return x + y; });
-  const float inv = 1.0f / (s + 1e-6f);
-  p.each([&](int, float& v) { v = v * inv; });
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[s][j] = expf(v[s][j] - m);
+      sloc += v[s][j];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const float sum = block_reduce(sloc, shf, [](float x, float y) { return x + y; });
+  if (!(sum < INFINITY)) {  // a logit that is no number, or none that is finite
+    if (threadIdx.x == 0) done(0);
+    return;
+  }
+  const float inv = 1.0f / (sum + 1e-6f);
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[s][j] = v[s][j] * inv;
 
-  // top-k: bit pattern of the k-th largest probability (keep bits >= tk)
-  uint32_t tk = 0;
-  if (a.top_k > 0 && a.top_k < a.V) {
-    for (int bit = 30; bit >= 0; --bit) {
-      const uint32_t cand = tk | (1u << bit);
-      uint32_t c = 0;
-      p.each([&](int, float& v) { c += __float_as_uint(v) >= cand; });
-      c = block_reduce(c, shu, [](uint32_t x, uint32_t y) { return x + y; });
-      if (c >= (uint32_t)a.top_k) tk = cand;
+  // top-k: the largest pattern that top_k probabilities reach (fewer that are not
+  // zero: all stay).  top-p: the largest pattern whose probabilities and those above
+  // hold a mass of top_p; whatever lies below has at least that much ranked above it.
+  // What top-k drops cannot change that: where the mass that it leaves is less than
+  // top_p, top-p drops nothing more.
+  uint32_t least = 0;
+  if (a.top_k > 0 && a.top_k < a.V)
+    least = find_pattern<NS>(v, 0u, (uint32_t)a.top_k, ranks, rank_part, &rank_found,
+                             [](uint32_t) { return 1u; });
+  if (a.top_p < 1.0f)
+    least = max(least, find_pattern<NS>(v, least, mass_of(__float_as_uint(a.top_p)), masses, mass_part,
+                                        &mass_found, [](uint32_t bits) { return mass_of(bits); }));
+
+  // kept mass in token order: per cell, then over the cells
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    float part = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      v[s][j] = __float_as_uint(v[s][j]) >= least ? v[s][j] : 0.f;
+      part += v[s][j];
     }
+    if (__ballot(part > 0.f)) part = group_sum<64>(part);
+    if (lane == 0) cells[s * kSampleWaves + w] = part;
   }
-  // top-p: keep p_i iff the mass strictly above it is < top_p, i.e. bits > tp
-  // where tp is the largest pattern whose strictly-above mass is >= top_p
-  int64_t tp = -1;
-  if (a.top_p < 1.0f) {
-    auto mass_above = [&](uint32_t t) {
-      float ms = 0.f;
-      p.each([&](int, float& v) { ms += __float_as_uint(v) > t ? v : 0.f; });
-      return block_reduce(ms, shf, [](float x, float y) { return x + y; });
-    };
-    if (mass_above(0u) >= a.top_p) {
-      uint32_t t = 0;
-      for (int bit = 30; bit >= 0; --bit) {
-        const uint32_t cand = t | (1u << bit);
-        if (mass_above(cand) >= a.top_p) t = cand;
-      }
-      tp = t;
-    }
-  }
-  // kept mass in token-index order: thread partial sums, block exclusive scan
-  float part = 0.f;
-  p.each([&](int i, float& v) {
-    const uint32_t bits = __float_as_uint(v);
-    const bool keep = base + i < a.V && bits >= tk && (int64_t)bits > tp;
-    v = keep ? v : 0.f;
-    part += v;
-  });
-  __shared__ float scan[kSampleThreads];
-  scan[threadIdx.x] = part;
   __syncthreads();
-  for (int off = 1; off < kSampleThreads; off <<= 1) {  // Hillis-Steele inclusive scan
-    const float v = threadIdx.x >= off ? scan[threadIdx.x - off] : 0.f;
-    __syncthreads();
-    scan[threadIdx.x] += v;
-    __syncthreads();
-  }
-  const float Z = scan[kSampleThreads - 1];
-  const int ctr = a.counter ? a.counter[r] : a.counter0;
-  const float target = sample_uniform(a.seed, a.row0 + r, ctr) * Z;
-  const float lo = threadIdx.x ? scan[threadIdx.x - 1] : 0.f;
-  // the thread whose [lo, lo + part) holds target picks inside its chunk
-  int pick = 0x7fffffff;
-  if (part > 0.f && target >= lo && (target < lo + part || threadIdx.x == kSampleThreads - 1 ||
-                                     scan[threadIdx.x] >= Z)) {
-    float c = lo;
-    int last = -1;
-    p.each([&](int i, float& v) {  // ascending token index
-      if (v > 0.f) {
-        last = base + i;
-        c += v;
-        if (target < c && pick == 0x7fffffff) pick = base + i;
+  constexpr int CELLS = NS * kSampleWaves, PER = (CELLS + 63) / 64;
+  if (w == 0) {
+    float c[PER], own = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      c[i] = lane * PER + i < CELLS ? cells[lane * PER + i] : 0.f;
+      own += c[i];
+    }
+    float incl = own;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float o = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += o;
+    }
+    const float Z = __shfl(incl, 63, 64);
+    const int ctr = a.counter ? a.counter[r] : a.counter0;
+    const float target = sample_uniform(a.seed, a.row0 + r, ctr) * Z;
+    // the first cell whose end lies past the target, else (rounding at the top of the
+    // range) the last one that holds any mass
+    float lo = __shfl_up(incl, 1, 64);
+    if (lane == 0) lo = 0.f;
+    int hit = 0x7fffffff, last = -1;
+    float left = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (c[i] > 0.f) {
+        last = lane * PER + i;
+        if (hit == 0x7fffffff && target < lo + c[i]) {
+          hit = last;
+          left = target - lo;
+        }
       }
-    });
-    if (pick == 0x7fffffff) pick = last;  // rounding at the top of the range
+      lo += c[i];
+    }
+    int first = hit;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+      first = min(first, __shfl_xor(first, off, 64));
+      last = max(last, __shfl_xor(last, off, 64));
+    }
+    if (first != 0x7fffffff) {
+      if (hit == first) {
+        cell = first;
+        cell_left = left;
+      }
+    } else if (lane == 0) {
+      cell = last;
+      cell_left = INFINITY;
+    }
   }
-  pick = block_reduce(pick, shi, [](int x, int y) { return min(x, y); });
-  if (threadIdx.x == 0) {
-    const int tok = pick == 0x7fffffff ? 0 : pick;
-    a.out[r] = tok;
-    if (a.out2) a.out2[(size_t)r * a.out2_stride] = tok;
+  __syncthreads();
+  const int at = cell;
+  if (at < 0) {
+    if (threadIdx.x == 0) done(0);
+    return;
   }
+  if (w != at % kSampleWaves) return;
+  const float target = cell_left;
+  float lo = 0.f;
+  int pick = 0x7fffffff, last = -1;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (s != at / kSampleWaves) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float incl = v[s][j];
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const float o = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += o;
+      }
+      if (v[s][j] > 0.f) {
+        last = token(s, j);
+        if (target < lo + incl) pick = min(pick, token(s, j));
+      }
+      lo += __shfl(incl, 63, 64);
+    }
+  }
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+    pick = min(pick, __shfl_xor(pick, off, 64));
+    last = max(last, __shfl_xor(last, off, 64));
+  }
+  if (lane == 0) done(pick == 0x7fffffff ? last : pick);
 }
 
-template <int VPT>
-hipError_t launch_sample_vpt(const SampleArgs& a, int rows, hipStream_t st) {
-  constexpr size_t lds = (size_t)(VPT - RowVals<VPT>::R) * kSampleThreads * sizeof(float);
-  if constexpr (lds > 65536) {
-    static bool attr = false;
-    if (!attr) {
-      (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&sample_rows_kernel<VPT>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-      attr = true;
-    }
-  }
-  hipLaunchKernelGGL(sample_rows_kernel<VPT>, dim3(rows), dim3(kSampleThreads), lds, st, a);
+template <int NS>
+hipError_t launch_sample_segments(const SampleArgs& a, int rows, hipStream_t st) {
+  hipLaunchKernelGGL(sample_rows_kernel<NS>, dim3(rows), dim3(kSampleThreads), 0, st, a);
   return hipGetLastError();
 }
 
 hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t st) {
-  const int vpt = (a.V + kSampleThreads - 1) / kSampleThreads;
-  if (vpt <= 16) return launch_sample_vpt<16>(a, rows, st);
-  if (vpt <= 32) return launch_sample_vpt<32>(a, rows, st);
-  if (vpt <= 64) return launch_sample_vpt<64>(a, rows, st);
-  if (vpt <= 128) return launch_sample_vpt<128>(a, rows, st);
-  return hipErrorInvalidValue;
+  if (a.V > 16 * kSampleSeg) return hipErrorInvalidValue;
+  if (a.temperature <= 0.f || a.top_k == 1) {
+    hipLaunchKernelGGL(sample_greedy_kernel, dim3(rows), dim3(kSampleThreads), 0, st, a);
+    return hipGetLastError();
+  }
+  const int segments = (a.V + kSampleSeg - 1) / kSampleSeg;
+  if (segments <= 2) return launch_sample_segments<2>(a, rows, st);
+  if (segments <= 4) return launch_sample_segments<4>(a, rows, st);
+  if (segments <= 8) return launch_sample_segments<8>(a, rows, st);
+  if (segments <= 13) return launch_sample_segments<13>(a, rows, st);
+  return launch_sample_segments<16>(a, rows, st);
 }
 
 }  // namespace llm
@@ -249,7 +369,7 @@ extern "C" int sample_rows(const float* logits, int rows, int V, float temperatu
   LLM_REQUIRE(rows >= 0 && V > 0, "sample_rows: bad shape");
   if (rows == 0) return LLM_OK;
   LLM_REQUIRE(logits && out, "sample_rows: NULL pointer");
-  LLM_REQUIRE(V <= 128 * kSampleThreads, "sample_rows: V > 65536");
+  LLM_REQUIRE(V <= 16 * kSampleSeg, "sample_rows: V > 65536");
   LLM_REQUIRE(top_k >= 0 && top_p > 0.f && top_p <= 1.0f, "sample_rows: top_k >= 0, 0 < top_p <= 1");
   SampleArgs a{logits, V, temperature, top_k, top_p, seed, nullptr, counter, 0, out, nullptr, 0};
   LLM_HIP_RET(launch_sample_rows(a, rows, as_stream(stream)));

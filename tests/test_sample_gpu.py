@@ -1,0 +1,53 @@
+"""sample_rows where its segments, histograms and cells can go wrong: vocabularies at
+their borders, ties, masked and unusable logits, thresholds that keep one or all."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def draw(logits, T, k, p, counter=0):
+    import torch
+    import llm_capi
+    return llm_capi.sample_rows(torch.from_numpy(logits).cuda(), T, k, p, seed=5,
+                                counter=counter).cpu().numpy()
+
+
+@pytest.mark.parametrize("V", [1, 2, 63, 257, 4095, 4097, 8193, 16385, 32768, 53248, 53249, 65536])
+@pytest.mark.parametrize("T,k,p", [(0.8, 40, 0.9), (1.0, 0, 0.999), (1.3, 2, 1.0), (1.0, 0, 1.0),
+                                   (0.05, 300, 0.3), (0.0, 0, 1.0)])
+def test_vocabulary_borders(gpu, V, T, k, p):
+    from oracle.oracle import sample_rows
+    logits = (np.random.default_rng(V + k).standard_normal((5, V)) * 2).astype(np.float32)
+    for counter in (0, 9):
+        ref, margin = sample_rows(logits, T, k, p, seed=5, counter=counter)
+        got = draw(logits, T, k, p, counter)
+        # a draw this close to a boundary of the distribution may fall on either side
+        assert ((got == ref) | (margin < 1e-4)).all(), (got, ref, margin)
+
+
+def test_ties_stay_together(gpu):
+    """Equal probabilities share a rank: all of them stay, nothing below does."""
+    V = 20000
+    logits = np.full((1, V), -3.0, np.float32)
+    top = np.arange(17, V, 1999)
+    logits[0, top] = 2.0
+    seen = {int(draw(logits, 1.0, 3, 1.0, c)[0]) for c in range(200)}
+    assert seen <= set(top.tolist()) and len(seen) == len(top)
+    same = np.zeros((1, 300), np.float32)  # top_p of equal ones: the mass above each is 0
+    assert len({int(draw(same, 1.0, 0, 0.1, c)[0]) for c in range(300)}) > 100
+
+
+def test_masked_and_unusable_logits(gpu):
+    V = 9000
+    rng = np.random.default_rng(1)
+    logits = rng.standard_normal((4, V)).astype(np.float32)
+    logits[0, :] = -np.inf
+    logits[0, [5, 8190, 8999]] = [0.0, 1.0, 0.5]  # all others masked
+    logits[1, 77] = np.nan
+    logits[2, :] = -np.inf
+    logits[3, 4000] = 80.0  # the rest underflows to nothing
+    for c in range(20):
+        got = draw(logits, 1.0, 50, 0.95, c)
+        assert got[0] in (5, 8190, 8999) and got[1] == 0 and got[2] == 0 and got[3] == 4000
+    assert draw(logits, 1.0, 0, 0.3, 1)[0] == 8190
