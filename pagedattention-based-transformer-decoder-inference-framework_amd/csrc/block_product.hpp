@@ -1,0 +1,178 @@
+// The product of a block of 16 MB rows and 16 NB columns on MFMA, both operands
+// through LDS: the prompt-sized products of the layer-stack models (mm_impl.hpp) and
+// of the dense decoders (gemm_impl.hpp).
+#pragma once
+
+#include <type_traits>
+
+#include "common.hpp"
+
+namespace llm {
+
+// Workgroups go round the XCDs in turn.  Block id -> tile of an nx wide grid, in a
+// walk whose neighbours are the blocks of one XCD: they share rows of A and columns
+// of W in its L2, eight row blocks at a time.
+struct TileAt {
+  int x = 0, y = 0;
+};
+__device__ __forceinline__ TileAt xcd_tile(int id, int nx, int ny) {
+  const int total = nx * ny, xcd = id & 7, each = total >> 3, more = total & 7;
+  const int t = xcd * each + min(xcd, more) + (id >> 3);
+  const int group = t / (8 * nx), r = t - group * 8 * nx, rows = min(8, ny - 8 * group);
+  return {r / rows, 8 * group + r % rows};
+}
+
+// WM x WN waves.  A k-step is 64 bytes of every row and column (32 bf16 / fp16, 64
+// int8, 16 fp32), a fragment of 16 of them 1 KiB.  Both operands go from memory
+// straight into LDS, ST stages of two k-steps in flight; while a wave multiplies one
+// k-step it reads the fragments of the next.  It waits for its own loads of a stage
+// alone; the barrier then makes them everyone's and frees the stage that was read
+// before.  The loads are spread among the matrix instructions: issued together they
+// hold up the wave while the matrix cores run dry.
+// W is packed, fragment after fragment (w_tile(t): the first of column tile t).  A is
+// packed alike (A_PACKED; a_at(t): the first fragment of row tile t) or row-major
+// (a_at(r): row r).  Row-major, a load takes 8 rows x 128 bytes, whole cache lines (16
+// rows x 64 bytes, the fragment itself, took 1.7 times as long per byte); the 16-byte
+// chunks of a row are exchanged by (row / 2) so that a fragment's 16 rows lie in
+// different banks.  Addresses past the operands' ends are the callers' to avoid.
+// Bound by the matrix cores waiting at the barriers: 2048 x 2048 x 6144 48.6 us, 1060
+// TFLOP/s (113 us with two k-steps loaded and waited for together in 128 x 128 blocks
+// of four waves); 2048 x 12288 x 2048 101 us (143), 700 x 2048 x 2048 12.3 us (32).
+//
+// here: whether any of the wave's rows exist (the others load and wait).  When it
+// returns, nobody reads LDS any more.
+template <bool A_PACKED, int MB, int NB, int WM, int WN, int ST, typename Acc, typename A, typename W,
+          typename Mma>
+__device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64],
+                                              Acc (&acc)[MB / WM][NB / WN], int KS, bool here,
+                                              const A& a_at, const W& w_tile, const Mma& mma) {
+  constexpr int WAVES = WM * WN, MT = MB / WM, NT = NB / WN;
+  constexpr int LOADS = 2 * (MB + NB) / WAVES;  // of a wave and stage, 1 KiB each
+  static_assert(2 * (MB + NB) % WAVES == 0);
+  const int lane = lane_id(), w = wave_id_uniform();
+  const int wm = w / WN, wn = w % WN, stages = KS >> 1;
+
+  // load l of a stage: A (l < 2 MB), eight rows or a k-step of a tile, then the two
+  // k-steps of each of W's column tiles
+  const char* src[LOADS];
+  const int l0 = w * LOADS;
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int l = l0 + i;
+    if (l >= 2 * MB) {
+      src[i] = w_tile((l >> 1) - MB) + (l & 1) * 1024 + lane * 16;
+    } else if constexpr (A_PACKED) {
+      src[i] = a_at(l >> 1) + (l & 1) * 1024 + lane * 16;
+    } else {
+      const int r = 8 * l + (lane >> 3);
+      src[i] = a_at(r) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+    }
+  }
+  auto issue = [&](int st, int i) {
+    load_to_lds(src[i], lds[st][l0 + i]);
+    src[i] += !A_PACKED && l0 + i < 2 * MB ? 128 : 2048;
+  };
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+  struct Frags {
+    u32x4 a[MT], c[NT];
+  };
+  const int ar = lane & 15;  // row-major: this lane's row of a fragment, its chunks of the two k-steps
+  const int at0 = 8 * ar + ((lane >> 4) ^ (ar >> 1)), at1 = at0 ^ 4;
+  auto read = [&](Frags& f, int st, int u) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const u32x4* tile = &lds[st][2 * (wm * MT + i)][0];
+      f.a[i] = A_PACKED ? tile[u * 64 + lane] : tile[u ? at1 : at0];
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) f.c[j] = lds[st][2 * (MB + wn * NT + j) + u][lane];
+  };
+  // multiplies, with loads [FROM, TO) of stage st among the products
+  auto mul = [&](const Frags& f, int st, auto from, auto to) {
+    constexpr int FROM = decltype(from)::value, TO = decltype(to)::value, N = MT * NT;
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      if constexpr (TO > FROM) {
+#pragma unroll
+        for (int i = FROM; i < TO; ++i)
+          if ((i - FROM) * N / (TO - FROM) == t) {
+            issue(st, i);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+      }
+      const int i = t / NT, j = t % NT;
+      acc[i][j] = mma(f.a[i], f.c[j], acc[i][j]);
+    }
+  };
+  const std::integral_constant<int, 0> zero;
+  const std::integral_constant<int, LOADS / 2> half;
+  const std::integral_constant<int, LOADS> all;
+  if (stages > 0) {
+#pragma unroll
+    for (int s = 0; s < ST; ++s)
+      if (s < stages) {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue(s, i);
+      }
+    Frags x, y;
+    if (stages >= ST) wait_lds_loads<(ST - 1) * LOADS>();
+    else wait_lds_loads<0>();
+    __builtin_amdgcn_s_barrier();
+    if (here) {
+      read(x, 0, 0);
+      read(y, 0, 1);
+      mul(x, 0, zero, zero);
+    }
+    int st = 0;
+    auto landed = [&](int s) {  // stage s + 1 is there for everyone, stage s read out
+      if (s + ST <= stages) wait_lds_loads<(ST - 2) * LOADS>();
+      else wait_lds_loads<0>();
+      __builtin_amdgcn_s_barrier();
+    };
+    landed(0);
+    int s = 0;
+    for (; s + ST < stages; ++s) {
+      const int now = st;
+      st = st + 1 == ST ? 0 : st + 1;
+      if (here) {
+        read(x, st, 0);
+        mul(y, now, zero, half);
+        read(y, st, 1);
+        mul(x, now, half, all);
+      } else {
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) issue(now, i);
+      }
+      landed(s + 1);
+    }
+    for (; s + 1 < stages; ++s) {
+      st = st + 1 == ST ? 0 : st + 1;
+      if (here) {
+        read(x, st, 0);
+        mul(y, 0, zero, zero);
+        read(y, st, 1);
+        mul(x, 0, zero, zero);
+      }
+      landed(s + 1);
+    }
+    if (here) mul(y, 0, zero, zero);
+  }
+  if (KS & 1) {  // the last k-step of an odd number, from memory
+    Frags f;
+    const size_t at = (size_t)(KS - 1) * 1024 + lane * 16;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int t = wm * MT + i;
+      const char* p = A_PACKED ? a_at(t) + at : a_at(16 * t + ar) + (size_t)(KS - 1) * 64 + 16 * (lane >> 4);
+      f.a[i] = *reinterpret_cast<const u32x4*>(p);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j) f.c[j] = *reinterpret_cast<const u32x4*>(w_tile(wn * NT + j) + at);
+    mul(f, 0, zero, zero);
+  }
+}
+
+}  // namespace llm

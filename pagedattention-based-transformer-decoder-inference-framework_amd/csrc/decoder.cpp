@@ -142,13 +142,17 @@ struct llm_decoder {
   int enqueue_step(hipStream_t st);
   int run_step(const int32_t* tokens_host, float* logits_dev, int32_t* next_host, hipStream_t st);
 
-  // chunked prefill (llm_decoder_prefill): buffers for one chunk of tokens
-  static constexpr int kPrefillChunk = 512;
+  // chunked prefill (llm_decoder_prefill): buffers for one chunk of tokens.  Mixed
+  // steps and shapes without the MFMA prompt attention take up to kPrefillChunk; a
+  // prompt otherwise up to kPromptChunk, enough for its products to fill the chip
+  // (2048 tokens, 4 layers of 16 x 128: in chunks of 512 3,042 us, whole 2,262).
+  static constexpr int kPrefillChunk = 512, kPromptChunk = 2048;
   DevBuf<float> px, pq, po, ph1, psa;
   DevBuf<uint8_t> pact, pws;
   DevBuf<int32_t> pmeta;  // [4][chunk]: pos, ctx, page-table row, token
   size_t pws_bytes = 0;
   int pf_cap = 0;
+  int alloc_prefill(int C);
   int ensure_prefill(int C);
   int prefill(int row, const int32_t* toks, int n, hipStream_t st);
   int forward_mixed(const std::vector<StepSeq>& seqs, float* logits_dev, hipStream_t st);
@@ -808,8 +812,8 @@ int llm_decoder::oproj_range_status() {
 }
 
 // Buffers for one layer pass of C prompt tokens.
-int llm_decoder::ensure_prefill(int C) {
-  if (C <= pf_cap) return LLM_OK;
+int llm_decoder::alloc_prefill(int C) {
+  pf_cap = 0;
   const size_t C16 = ((size_t)C + 15) / 16 * 16;
   RET_IF(px.alloc((size_t)C * hid));
   RET_IF(pq.alloc((size_t)C * hid));
@@ -819,7 +823,7 @@ int llm_decoder::ensure_prefill(int C) {
   RET_IF(pact.alloc(C16 * std::max(hid, inter) * (wdtype == LLM_I8 ? 1 : 4)));  // F16: act, act2
   RET_IF(pmeta.alloc((size_t)4 * C));
   pws_bytes = 16;
-  for (int b = 1; b <= C; ++b)
+  for (int b = 1; b <= std::min(C, kPrefillChunk); ++b)
     pws_bytes = std::max(pws_bytes, pa_decode_workspace_bytes(b, H, D, max_tiles, 0));
   {  // the MFMA prefill's split partials (its split count is bounded at any p0)
     pa_kv_view v0;
@@ -830,6 +834,13 @@ int llm_decoder::ensure_prefill(int C) {
   RET_IF(pws.alloc(pws_bytes));
   pf_cap = C;
   return LLM_OK;
+}
+
+// A card that the cache fills has no room for the long chunk: the short one then.
+int llm_decoder::ensure_prefill(int C) {
+  if (C <= pf_cap) return LLM_OK;
+  const int rc = alloc_prefill(C);
+  return rc == LLM_ERR_OOM && C > kPrefillChunk ? alloc_prefill(kPrefillChunk) : rc;
 }
 
 // Chunked prefill of `n` prompt tokens of active row `row` (the reference's
@@ -846,8 +857,11 @@ int llm_decoder::prefill(int row, const int32_t* toks, int n, hipStream_t st) {
   LLM_REQUIRE(n >= 1 && toks, "prefill: need >= 1 token");
   LLM_REQUIRE(h_pos[row] + n < cfg.max_seq_len, "prefill: prompt exceeds max_seq_len");
   for (int i = 0; i < n; ++i) LLM_REQUIRE(toks[i] >= 0 && toks[i] < V, "prefill: token id out of range");
-  const int C = std::min(n, kPrefillChunk);
+  pa_kv_view v0;
+  RET_IF(kv_cache_view(kv, 0, &v0));
+  int C = std::min(n, pa_prefill_supported(&v0) ? kPromptChunk : kPrefillChunk);
   RET_IF(ensure_prefill(C));
+  C = std::min(C, pf_cap);
   KvCache* k = kv_impl(kv);
   std::vector<int32_t> meta((size_t)4 * C), pc(2);
   for (int c0 = 0; c0 < n; c0 += C) {

@@ -27,6 +27,7 @@
 //     row = 4*(lane>>4) + reg (cdna_hip_programming.md §3).
 #pragma once
 
+#include "block_product.hpp"
 #include "common.hpp"
 #include "gemm.hpp"
 #include "ln_wave.hpp"
@@ -580,6 +581,161 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
   gemm_tile<KIND, MT, NT, WAVES, DIAG, PRO>(a, bx, by, bz, (int)gridDim.z, (int)gridDim.x);
 }
 
+// Rows of a prompt: blocks of 16 MB rows x 16 NB columns through LDS
+// (block_product.hpp), compute-shaped where the kernel above is a weight stream.
+// int8, 2048 rows: x 6144 x 2048 with the KV append 71.5 us (177 as four streams of
+// 512 rows), x 8192 x 2048 63 (224), x 2048 x 2048 and x 2048 x 8192 31 on average
+// (91); bound as block_product, the append by its page stores besides.
+template <GemmKind KIND, bool A_PACKED, int MB, int NB, int WM, int WN, int ST>
+__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_block_kernel(GemmArgs a) {
+  using Tr = GemmTraits<KIND>;
+  using acc_t = typename Tr::acc_t;
+  using elem_t = typename Tr::elem_t;
+  constexpr int MT = MB / WM, NT = NB / WN, THREADS = 64 * WM * WN;
+  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
+  const TileAt tile = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y);
+  const int lane = lane_id(), w = wave_id_uniform(), wm = w / WN, wn = w % WN;
+  const int KS = a.KS, ntiles = (a.N + 15) >> 4, mtiles = (a.M + 15) >> 4;
+  const int m0 = tile.y * 16 * MB, nt0 = tile.x * NB;
+  acc_t acc[MT][NT];
+  block_product<A_PACKED, MB, NB, WM, WN, ST>(
+      lds, acc, KS, m0 + 16 * wm * MT < a.M,
+      [&](int r) {
+        const char* A = reinterpret_cast<const char*>(a.A);
+        return A_PACKED ? A + (size_t)min((m0 >> 4) + r, mtiles - 1) * KS * 1024
+                        : A + (size_t)min(m0 + r, a.M - 1) * a.lda * Tr::ESIZE;
+      },
+      [&](int t) {
+        return reinterpret_cast<const char*>(a.B) + (size_t)min(nt0 + t, ntiles - 1) * KS * 1024;
+      },
+      [](u32x4 x, u32x4 y, acc_t c) {
+        if constexpr (KIND == GemmKind::I8)
+          return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, x),
+                                                       __builtin_bit_cast(i32x4, y), c, 0, 0, 0);
+        else
+          return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x),
+                                                        __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
+      });
+  const auto finish = [&](elem_t s, float sa, float sw, float bias) {
+#pragma clang fp contract(off)  // y = acc * scale + bias rounded twice, as the reference
+    float y = (float)s;
+    if constexpr (KIND == GemmKind::I8) y = y * (sa * sw);
+    if (a.bias) y = y + bias;
+    return apply_act(y, a.act);
+  };
+  const bool rows_only = !a.kv.k_pool && !a.c16;
+  if (rows_only) {  // fp32 rows: 64 bytes of a line per store, straight from the accumulators
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+      const int first = m0 + 16 * (wm * MT + i) + 4 * (lane >> 4);
+      float sa[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sa[r] = KIND == GemmKind::I8 && a.sa ? a.sa[min(first + r, a.M - 1)] : 1.f;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        const int n = (nt0 + wn * NT + j) * 16 + (lane & 15);
+        if (n >= a.N) continue;
+        const float sw = KIND == GemmKind::I8 && a.sw ? a.sw[n] : 1.f, bias = a.bias ? a.bias[n] : 0.f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = first + r;
+          if (m >= a.M) continue;
+          if constexpr (KIND == GemmKind::I8)
+            if (a.acc_out) a.acc_out[(size_t)m * a.N + n] = acc[i][j][r];
+          if (a.C && n < a.c_cols) a.C[(size_t)m * a.c_ld + n] = finish(acc[i][j][r], sa[r], sw, bias);
+        }
+      }
+    }
+    return;
+  }
+  // Pages and packed fp16 rows: row by row through LDS (block_product has read it
+  // out), eight columns per thread, so that stores are 16 bytes and a page is looked
+  // up once for them.
+  constexpr int STRIDE = 16 * NB + 4;
+  static_assert(sizeof(lds) >= sizeof(elem_t) * 16 * MB * STRIDE);
+  elem_t* sums = reinterpret_cast<elem_t*>(&lds[0][0][0]);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        sums[(16 * (wm * MT + i) + 4 * (lane >> 4) + r) * STRIDE + 16 * (wn * NT + j) + (lane & 15)] =
+            acc[i][j][r];
+  __syncthreads();
+  constexpr int ACROSS = 2 * NB, STEP = THREADS / ACROSS, PER = 16 * MB / STEP, BATCH = PER < 4 ? PER : 4;
+  static_assert(THREADS % ACROSS == 0 && PER % BATCH == 0);
+  const int row0 = threadIdx.x / ACROSS, col0 = threadIdx.x % ACROSS * 8, n = nt0 * 16 + col0;
+  if (n >= a.N) return;  // (N is a multiple of 16)
+  const KvAppend& kv = a.kv;
+  const int hid = kv.H * kv.D, which = kv.k_pool && n >= hid ? n / hid : 0;  // 1: K, 2: V
+  const int head = which ? (n - which * hid) / kv.D : 0, d = which ? (n - which * hid) % kv.D : 0;
+  float sw[8], bias[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    sw[k] = KIND == GemmKind::I8 && a.sw ? a.sw[n + k] : 1.f;
+    bias[k] = a.bias ? a.bias[n + k] : 0.f;
+  }
+#pragma unroll 1
+  for (int i0 = 0; i0 < PER; i0 += BATCH) {
+    int pos[BATCH], page[BATCH];
+    float sa[BATCH];
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const int m = min(m0 + row0 + (i0 + i) * STEP, a.M - 1);
+      sa[i] = KIND == GemmKind::I8 && a.sa ? a.sa[m] : 1.f;
+      pos[i] = which ? kv.pos[m] : -1;
+      page[i] = which ? (kv.rows ? kv.rows[m] : m) : -1;  // the page-table row first
+    }
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const int row = page[i], t = pos[i] >= 0 ? pos[i] / kv.TS : 0;
+      page[i] = -1;
+      if (pos[i] >= 0 && row >= 0 && row < kv.num_beams && t < kv.max_tiles)
+        page[i] = kv.page_table[((size_t)row * kv.H + head) * kv.max_tiles + t];
+      if (page[i] >= kv.num_pages) page[i] = -1;
+    }
+#pragma unroll
+    for (int i = 0; i < BATCH; ++i) {
+      const int r = row0 + (i0 + i) * STEP, m = m0 + r;
+      if (m >= a.M) continue;
+      float y[8];
+      f16x8 h;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const elem_t s = sums[r * STRIDE + col0 + k];
+        if constexpr (KIND == GemmKind::I8)
+          if (a.acc_out) a.acc_out[(size_t)m * a.N + n + k] = s;
+        y[k] = finish(s, sa[i], sw[k], bias[k]);
+        h[k] = (_Float16)y[k];
+      }
+      if (a.C) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (n + k < a.c_cols) a.C[(size_t)m * a.c_ld + n + k] = y[k];
+      }
+      if (a.c16) *reinterpret_cast<f16x8*>(a.c16 + a_frag_off_f16(m, n, a.N >> 5)) = h;
+      if (page[i] >= 0) {
+        _Float16* pool = which == 2 ? kv.v_pool : kv.k_pool;
+        if ((kv.D & 7) == 0) {
+          *reinterpret_cast<f16x8*>(pool + (size_t)page[i] * kv.page_stride +
+                                    (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
+        } else {  // the eight columns reach into other heads
+#pragma unroll 1
+          for (int k = 0; k < 8; ++k) {
+            const int c = n - which * hid + k, hd = c / kv.D;
+            const int row = kv.rows ? kv.rows[m] : m;
+            const int pg = kv.page_table[((size_t)row * kv.H + hd) * kv.max_tiles + pos[i] / kv.TS];
+            if (pg >= 0 && pg < kv.num_pages)
+              pool[(size_t)pg * kv.page_stride + (size_t)(pos[i] % kv.TS) * kv.D + c % kv.D] = h[k];
+          }
+        }
+      }
+    }
+  }
+}
+
 // Repack W [K][N] (row-major) into per-(16-col tile, k-step) 1 KiB blocks,
 // lane l's 16 bytes = W[k0 + (l>>4)*EPL + j][n0 + (l&15)], j < EPL
 // (EPL = elements per lane: 16 int8 or 8 fp16); zero-padded past K / N.
@@ -733,10 +889,43 @@ inline bool narrow_decode_tile(const GemmArgs& a, int kstep, TileChoice& t) {
   return narrow_tile_for(a.M, a.N, a.KS * kstep, t);
 }
 
+// The block form with the least rounds of workgroups x time of a round (us at 32
+// k-steps, launch taken off).
+template <GemmKind KIND, bool A_PACKED>
+hipError_t launch_gemm_block(const GemmArgs& a, hipStream_t st) {
+  struct Form {
+    int mb, nb, threads;
+    float round;
+    void (*kernel)(GemmArgs);
+  };
+  static constexpr Form forms[] = {{4, 4, 256, 6.2f, gemm_block_kernel<KIND, A_PACKED, 4, 4, 2, 2, 3>},
+                                   {4, 8, 512, 10.f, gemm_block_kernel<KIND, A_PACKED, 4, 8, 2, 4, 4>},
+                                   {8, 8, 512, 18.5f, gemm_block_kernel<KIND, A_PACKED, 8, 8, 4, 2, 3>},
+                                   {8, 16, 512, 27.f, gemm_block_kernel<KIND, A_PACKED, 8, 16, 2, 4, 3>}};
+  const Form* best = nullptr;
+  dim3 grid;
+  float least = 0.f;
+  for (const Form& f : forms) {
+    const dim3 g((a.N + 16 * f.nb - 1) / (16 * f.nb), (a.M + 16 * f.mb - 1) / (16 * f.mb));
+    const float cost = (float)((g.x * g.y + 255) / 256) * f.round;
+    if (best && cost >= least) continue;
+    best = &f;
+    grid = g;
+    least = cost;
+  }
+  hipLaunchKernelGGL(best->kernel, grid, dim3(best->threads), 0, st, a);
+  return hipGetLastError();
+}
+
 template <GemmKind KIND>
 hipError_t launch_gemm(const GemmArgs& a_in, hipStream_t st, int nt_override = 0,
                        int waves_override = 0, int mrows_override = 0, int ks_override = 0) {
   GemmArgs a = a_in;
+  // rows of a prompt, once 64 x 64 blocks are more than half a round of workgroups
+  if (a.M > 64 && (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) > 128 && !a.ln_x && !a.partial &&
+      !a.ksplit2 && !a.stamps && reinterpret_cast<uintptr_t>(a.A) % 16 == 0 &&
+      nt_override + waves_override + mrows_override + ks_override == 0)
+    return a.a_packed ? launch_gemm_block<KIND, true>(a, st) : launch_gemm_block<KIND, false>(a, st);
   TileChoice tc{0, 0, 0};
   const bool narrow = nt_override == 0 && waves_override == 0 && mrows_override == 0 &&
                       narrow_decode_tile(a, GemmTraits<KIND>::KSTEP, tc);

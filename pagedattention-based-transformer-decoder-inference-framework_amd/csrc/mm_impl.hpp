@@ -19,8 +19,8 @@
 #pragma once
 
 #include <algorithm>
-#include <type_traits>
 
+#include "block_product.hpp"
 #include "common.hpp"
 #include "mm.hpp"
 
@@ -809,40 +809,14 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
   }
 }
 
-// Workgroups go round the XCDs in turn.  Block id -> tile of an nx wide grid, in a
-// walk whose neighbours are the blocks of one XCD: they share rows of A and columns
-// of W in its L2, eight row blocks at a time.
-struct TileAt {
-  int x = 0, y = 0;
-};
-__device__ __forceinline__ TileAt xcd_tile(int id, int nx, int ny) {
-  const int total = nx * ny, xcd = id & 7, each = total >> 3, more = total & 7;
-  const int t = xcd * each + min(xcd, more) + (id >> 3);
-  const int group = t / (8 * nx), r = t - group * 8 * nx, rows = min(8, ny - 8 * group);
-  return {r / rows, 8 * group + r % rows};
-}
-
 // blocks of 16 NB columns in n columns
 __host__ __device__ __forceinline__ int group_across(int n, int NB) { return (n + 16 * NB - 1) / (16 * NB); }
 
-// A block of 16 MB rows x 16 NB columns, WM x WN waves.  Both operands
-// go from memory straight into LDS, ST stages of two k-steps in flight; while a
-// wave multiplies one k-step it reads the fragments of the next.  It waits for its
-// own loads of a stage alone; the barrier then makes them everyone's and frees the
-// stage that was read before.  The loads are spread among the matrix instructions:
-// issued together they hold up the wave while the matrix cores run dry.
-// A load of A takes 8 rows x 128 bytes, whole cache lines (16 rows x 64 bytes, the
-// fragment itself, took 1.7 times as long per byte); the 16-byte chunks of a row
-// are exchanged by (row / 2) so that a fragment's 16 rows lie in different banks.
-// Bound by the matrix cores waiting at the barriers: 2048 x 2048 x 6144 48.6 us, 1060
-// TFLOP/s (113 us with two k-steps loaded and waited for together in 128 x 128 blocks
-// of four waves); 2048 x 12288 x 2048 101 us (143), 700 x 2048 x 2048 12.3 us (32).
+// A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).
 template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
 __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p) {
   constexpr int WAVES = WM * WN, MT = MB / WM, NT = NB / WN;
-  constexpr int LOADS = 2 * (MB + NB) / WAVES;  // of a wave and stage, 1 KiB each
-  static_assert(2 * (MB + NB) % WAVES == 0);
-  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];  // per stage: A, two k-steps a tile; W, tile by tile
+  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
   int id = blockIdx.y * gridDim.x + blockIdx.x;
   TileAt tile;
   if constexpr (EPI == kGroupIn || EPI == kGroupOut) {
@@ -866,130 +840,14 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p)
   const int w = wave_id_uniform();
   const Block<T> b = block_of<T, EPI>(p, 16 * MB, tile.y);
   const int ntiles = (b.N + 15) >> 4;
-  const int nt0 = tile.x * NB;
-  const int KS = b.KS, stages = KS >> 1;
-
-  // load l of a stage: rows 8 l .. 8 l + 7 of A (l < 2 MB), then the two k-steps of
-  // each of W's column tiles
-  const char* src[LOADS];
-  const int l0 = w * LOADS;
-#pragma unroll
-  for (int i = 0; i < LOADS; ++i) {
-    const int l = l0 + i;
-    if (l < 2 * MB) {
-      const int r = 8 * l + (lane >> 3);
-      src[i] = a_row<T, EPI>(p, b, b.m0 + r) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
-    } else {
-      src[i] = b.W + (size_t)min(nt0 + (l >> 1) - MB, ntiles - 1) * KS * 1024 + (l & 1) * 1024 + lane * 16;
-    }
-  }
-  auto issue = [&](int st, int i) {
-    load_to_lds(src[i], lds[st][l0 + i]);
-    src[i] += l0 + i < 2 * MB ? 128 : 2048;
-  };
+  const int nt0 = tile.x * NB, KS = b.KS;
   const int wm = w / WN, wn = w % WN;
-  const bool rows_here = b.m0 + 16 * wm * MT < b.M;  // (short blocks: the others load and wait)
   f32x4 acc[MT][NT];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  struct Frags {
-    u32x4 a[MT], c[NT];
-  };
-  const int ar = lane & 15;  // this lane's row of a fragment, and its chunks of the two k-steps
-  const int at0 = 8 * ar + ((lane >> 4) ^ (ar >> 1)), at1 = at0 ^ 4;
-  auto read = [&](Frags& f, int st, int u) {
-#pragma unroll
-    for (int i = 0; i < MT; ++i) f.a[i] = (&lds[st][2 * (wm * MT + i)][0])[u ? at1 : at0];
-#pragma unroll
-    for (int j = 0; j < NT; ++j) f.c[j] = lds[st][2 * (MB + wn * NT + j) + u][lane];
-  };
-  // multiplies, with loads [FROM, TO) of stage st among the products
-  auto mul = [&](const Frags& f, int st, auto from, auto to) {
-    constexpr int FROM = decltype(from)::value, TO = decltype(to)::value, N = MT * NT;
-#pragma unroll
-    for (int t = 0; t < N; ++t) {
-      if constexpr (TO > FROM) {
-#pragma unroll
-        for (int i = FROM; i < TO; ++i)
-          if ((i - FROM) * N / (TO - FROM) == t) {
-            issue(st, i);
-            __builtin_amdgcn_sched_barrier(0);
-          }
-      }
-      const int i = t / NT, j = t % NT;
-      acc[i][j] = Kind<T>::mma(f.a[i], f.c[j], acc[i][j]);
-    }
-  };
-  using Zero = std::integral_constant<int, 0>;
-  using Half = std::integral_constant<int, LOADS / 2>;
-  using All = std::integral_constant<int, LOADS>;
-  const Zero zero;
-  const Half half;
-  const All all;
-  if (stages > 0) {
-#pragma unroll
-    for (int s = 0; s < ST; ++s)
-      if (s < stages) {
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) issue(s, i);
-      }
-    Frags x, y;
-    if (stages >= ST) wait_lds_loads<(ST - 1) * LOADS>();
-    else wait_lds_loads<0>();
-    __builtin_amdgcn_s_barrier();
-    if (rows_here) {
-      read(x, 0, 0);
-      read(y, 0, 1);
-      mul(x, 0, zero, zero);
-    }
-    int st = 0;
-    auto landed = [&](int s) {  // stage s + 1 is there for everyone, stage s read out
-      if (s + ST <= stages) wait_lds_loads<(ST - 2) * LOADS>();
-      else wait_lds_loads<0>();
-      __builtin_amdgcn_s_barrier();
-    };
-    landed(0);
-    int s = 0;
-    for (; s + ST < stages; ++s) {
-      const int now = st;
-      st = st + 1 == ST ? 0 : st + 1;
-      if (rows_here) {
-        read(x, st, 0);
-        mul(y, now, zero, half);
-        read(y, st, 1);
-        mul(x, now, half, all);
-      } else {
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) issue(now, i);
-      }
-      landed(s + 1);
-    }
-    for (; s + 1 < stages; ++s) {
-      st = st + 1 == ST ? 0 : st + 1;
-      if (rows_here) {
-        read(x, st, 0);
-        mul(y, 0, zero, zero);
-        read(y, st, 1);
-        mul(x, 0, zero, zero);
-      }
-      landed(s + 1);
-    }
-    if (rows_here) mul(y, 0, zero, zero);
-  }
-  if (KS & 1) {  // the last k-step of an odd number, from memory
-    Frags f;
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-      f.a[i] = *reinterpret_cast<const u32x4*>(a_row<T, EPI>(p, b, b.m0 + 16 * (wm * MT + i) + ar) +
-                                               (size_t)(KS - 1) * 64 + 16 * (lane >> 4));
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-      f.c[j] = *reinterpret_cast<const u32x4*>(
-          b.W + ((size_t)min(nt0 + wn * NT + j, ntiles - 1) * KS + KS - 1) * 1024 + lane * 16);
-    mul(f, 0, zero, zero);
-  }
+  block_product<false, MB, NB, WM, WN, ST>(
+      lds, acc, KS, b.m0 + 16 * wm * MT < b.M,
+      [&](int r) { return a_row<T, EPI>(p, b, b.m0 + r); },
+      [&](int t) { return b.W + (size_t)min(nt0 + t, ntiles - 1) * KS * 1024; },
+      [](u32x4 x, u32x4 y, f32x4 c) { return Kind<T>::mma(x, y, c); });
   // 2048 x 12288 x 2048 with its activation 107 us by rows, 109 by pairs; 2011 x 8192
   // split 80 and 77
   constexpr bool BY_ROWS = EPI == kGroupIn || EPI == kGlu || EPI == kLatent || RowOf<EPI>::PAGED;
@@ -997,7 +855,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p)
     emit_pairs<T, EPI>(p, b, acc, b.m0 + 16 * wm * MT, (nt0 + wn * NT) * 16);
     return;
   }
-  // (every wave has read its last fragments before the last barrier)
+  // (block_product has read all of LDS before its last barrier)
   constexpr int STRIDE = 16 * NB + 4;
   static_assert(sizeof(lds) >= sizeof(float) * 16 * MB * STRIDE);
   float* sums = reinterpret_cast<float*>(&lds[0][0][0]);
@@ -1007,7 +865,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p)
     for (int j = 0; j < NT; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        sums[(16 * (wm * MT + i) + 4 * (lane >> 4) + r) * STRIDE + 16 * (wn * NT + j) + ar] = acc[i][j][r];
+        sums[(16 * (wm * MT + i) + 4 * (lane >> 4) + r) * STRIDE + 16 * (wn * NT + j) + (lane & 15)] = acc[i][j][r];
   __syncthreads();
   emit_block<T, EPI, 16 * MB, 16 * NB, STRIDE, 64 * WAVES>(p, b, sums, 16 * nt0);
 }

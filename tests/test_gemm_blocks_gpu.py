@@ -1,0 +1,51 @@
+"""The block form of i8_gemm / f16_gemm (rows of a prompt) at the edges of its tiles:
+exact int32 accumulators, fp16 sums within their rounding, rows with a stride, one
+k-step and odd numbers of them, and the same rows at an address that only the stream
+form takes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# enough columns for more than 128 blocks of 64 x 64
+SHAPES = [(65, 4352, 64), (127, 4160, 192), (129, 2832, 2048), (191, 2768, 320), (513, 1040, 64),
+          (640, 2304, 768), (1025, 528, 448), (2048, 272, 1088), (2047, 2048, 128)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("shift", [0, 4])
+def test_int8(gpu, M, N, K, shift):
+    import torch
+    import llm_capi
+    rng = np.random.default_rng(M + N + K)
+    A = rng.integers(-127, 128, (M, K + 32), dtype=np.int8)
+    W = rng.integers(-127, 128, (K, N), dtype=np.int8)
+    sa = rng.uniform(0.5, 2.0, M).astype(np.float32)
+    sw = rng.uniform(0.5, 2.0, N).astype(np.float32)
+    bias = (100 * rng.standard_normal(N)).astype(np.float32)
+    buf = torch.zeros(M * (K + 32) + 64, dtype=torch.int8, device="cuda")
+    a = buf[shift:shift + M * (K + 32)].view(M, K + 32)
+    a.copy_(torch.from_numpy(A))
+    dev = [torch.from_numpy(x).cuda() for x in (sa, sw, bias)]
+    packed = llm_capi.pack_weights(torch.from_numpy(W).cuda(), llm_capi.LLM_I8)
+    acc, C = llm_capi.i8_gemm(a[:, :K], packed, N, sa=dev[0], sw=dev[1], bias=dev[2], act=1)
+    ref = (torch.from_numpy(A[:, :K]).double() @ torch.from_numpy(W).double()).numpy()
+    assert np.array_equal(acc.cpu().numpy(), ref.astype(np.int32))
+    y = ref.astype(np.float32) * (sa[:, None] * sw) + bias
+    assert np.array_equal(C.cpu().numpy(), np.maximum(y, 0))
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_fp16(gpu, M, N, K):
+    import torch
+    import llm_capi
+    g = torch.Generator().manual_seed(M + K)
+    A = torch.randn((M, K + 8), generator=g).half()
+    W = torch.randn((K, N), generator=g).half()
+    bias = torch.randn(N, generator=g)
+    packed = llm_capi.pack_weights(W.cuda(), llm_capi.LLM_F16)
+    C = llm_capi.f16_gemm(A.cuda()[:, :K], packed, N, bias=bias.cuda()).cpu().double()
+    ref = A[:, :K].double() @ W.double() + bias.double()
+    # fp32 sums of K exact products in some order: K roundings of the largest partial sum
+    size = A[:, :K].double().abs() @ W.double().abs() + bias.double().abs()
+    assert ((C - ref).abs() <= 2.0 ** -23 * (K ** 0.5 + 2) * size).all()
