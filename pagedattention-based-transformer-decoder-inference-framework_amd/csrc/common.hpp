@@ -115,6 +115,17 @@ __device__ __forceinline__ float wave_max(float x) {
   return x;
 }
 
+// The largest of lanes l, l ^ 16, l ^ 32, l ^ 48 (the same lane of the wave's four
+// rows): two exchanges of rows between registers, no trip through LDS.
+__device__ __forceinline__ float rows_max(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
+  const uint32_t c = __builtin_bit_cast(uint32_t, y);
+  const auto h = __builtin_amdgcn_permlane32_swap(c, c, false, false);
+  return fmaxf(__builtin_bit_cast(float, (uint32_t)h[0]), __builtin_bit_cast(float, (uint32_t)h[1]));
+}
+
 // wave_max through DPP moves inside the 16-lane rows
 __device__ __forceinline__ float wave_max_dpp(float x) {
   x = fmaxf(x, mov_dpp<0xB1>(x));

@@ -458,8 +458,8 @@ int LayerStack::ensure_rows(int M) {
 }
 
 // The row tiles of one attention launch: the plan's sequences that bring few rows
-// per key/value head (big false) or many, split over their pages until the launch
-// holds about kTargetGroups workgroups; long tiles first.
+// per key/value head (big false) or many, split over their pages so that the launch
+// fills rounds of kTargetGroups workgroups; long tiles first.
 void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
                      std::vector<GqaItem>& items, std::vector<GqaMerge>& merges, Launch& l) {
   l = Launch();
@@ -481,6 +481,29 @@ void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
   // shape (and graph) while contexts grow
   const int least = p.latent ? kMinLatentPages : kMinSplitPages;
   const int common = std::min(want, (max_pages + least - 1) / least);
+  // Long tiles: pieces of `per` pages, the length for which the rounds of workgroups
+  // times it is least (a causal prompt's tiles differ in length; 2048 tokens, every
+  // tile in two or three, then in such pieces: 16 heads over 2 76 -> 63 us, 16 expanded
+  // heads of 192 85 -> 42 us).
+  int per = max_pages;
+  if (big) {
+    double lowest = 1e30;
+    for (int n = 1; n <= std::min(kMaxSplits, (max_pages + least - 1) / least); ++n) {
+      const int len = (max_pages + n - 1) / n;
+      long long pieces = 0;
+      for (const StepSeq& s : batch) {
+        if (!mine(s)) continue;
+        for (int r0 = 0; r0 < s.n * p.R; r0 += l.tile_rows) {
+          const int last = s.p0 + (std::min(r0 + l.tile_rows, s.n * p.R) - 1) / p.R;
+          pieces += (last / kPageTokens + len) / len;
+        }
+      }
+      const double cost = (double)((pieces * p.G + kTargetGroups - 1) / kTargetGroups) * len + 0.5 * n;
+      if (cost >= lowest) continue;
+      lowest = cost;
+      per = len;
+    }
+  }
   for (const StepSeq& s : batch) {
     const int rows = s.n * p.R;
     const int t0 = tok0;
@@ -491,7 +514,7 @@ void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
     for (int r0 = 0; r0 < rows; r0 += l.tile_rows) {
       const int last = s.p0 + (std::min(r0 + l.tile_rows, rows) - 1) / p.R;
       const int pages = last / kPageTokens + 1;
-      const int ns = big ? std::min(want, (pages + least - 1) / least) : common;
+      const int ns = big ? (pages + per - 1) / per : common;
       for (int k = 0; k < ns; ++k)
         items.push_back(GqaItem{t0, slot, s.p0, r0, rows, (int)((long long)pages * k / ns),
                                 (int)((long long)pages * (k + 1) / ns), ns > 1 ? l.parts + k : -1});

@@ -491,7 +491,9 @@ int llm::pa_merge_rows_internal(const float* part_acc, const float* part_ml, flo
                     rows ? rows->inv_scale : nullptr,
                     rows ? static_cast<_Float16*>(rows->out16) : nullptr, context_lens, B, H, D, T,
                     TS, pps, nsplit, max_tiles, rows ? rows->pack : 0, ctx_p0};
-  const int threads = 64 * std::min(16, H);  // one wave per head (heads > 16 loop)
+  // one wave per head (heads past 16 loop); a prompt's rows fill the chip by themselves,
+  // and four waves each leave room for four times the rows on a CU
+  const int threads = 64 * std::min(B >= 1024 ? 4 : 16, H);
   const size_t lds = (size_t)H * D * sizeof(float);
   if (D <= 64)
     hipLaunchKernelGGL(pa_merge_row_kernel<1>, dim3(B), dim3(threads), lds, st, mg);

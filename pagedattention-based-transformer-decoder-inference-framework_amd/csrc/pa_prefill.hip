@@ -1,24 +1,31 @@
 // Causal paged attention of a prompt chunk on MFMA (the reference's is_prefill
 // pass: AttentionCUDA's `is_prefill` flag, attention/attention_cuda.hpp:21,
 // with the maths of cpu_paged_attention_forward,
-// attention_cpu/cpu_attention_kernel.cpp:37-129, per query token; SURVEY §8f
-// row 4).
+// attention_cpu/cpu_attention_kernel.cpp:37-129, per query token).
 //
 // m query tokens of ONE sequence sit at positions p0 .. p0+m-1 and their K/V
 // are already in the sequence's pages (page-table row `row`).  Query i attends
 // to positions 0 .. p0+i.  The decode kernel computes the same thing with one
 // wave per (token, head), so each page is re-read once per query token; here a
-// workgroup of NW waves owns 16·NW consecutive queries of one head, stages
-// every 32-key block of K and V into LDS ONCE, and each wave runs
-//   S^T[32 keys][16 queries] = K · Q^T        (v_mfma_f32_16x16x32_f16)
-//   O^T[D][16 queries]     += V^T · P^T
+// workgroup of 4 waves owns 64 MT consecutive queries of one head, loads every
+// 64-key stage of K and V into LDS ONCE, and each wave runs
+//   S^T[32 keys][16 MT queries] = K · Q^T     (v_mfma_f32_16x16x32_f16)
+//   O^T[D][16 MT queries]     += V^T · P^T
 // with the flash online softmax (log2 units, as pa_split_kernel) in between.
+//
+// A stage goes from memory straight into LDS, one stage ahead, a wave loading
+// 16 keys, with their page looked up two stages ahead: the dependent loads
+// (page, keys) and a register pass per 32 keys were what bounded the first form
+// (2048 queries x 16 heads x 128, two key splits: 137 us, now 52 us).  The
+// 16-byte chunks of a row are exchanged by the key so that the 16 rows of a
+// fragment lie in different banks.  Now bound by the vector instructions of the
+// softmax beside the matrix cores, at two workgroups per CU.
 //
 // Orientation: keys are the MFMA row index of S^T, so the C layout of S^T
 // (lane l: rows 4(l>>4)+r, column l&15) already holds, per lane, 8 keys of ONE
 // query: that is the B operand of the P·V product once the 32 keys are taken
 // in the k order slot(key) = 8·((key&15)>>2) + 4·(key>>4) + (key&3).  V is
-// staged row-major and its V^T A operand, in that same key order, is two
+// row-major and its V^T A operand, in that same key order, is two
 // hardware-transposed LDS reads (ds_read_b64_tr_b16) per 16 dims.  The query is the lane's column in both
 // products, so the running max / sum / rescale are per lane (the 4 lanes of a
 // query agree after a 2-step max exchange).
@@ -33,6 +40,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 
 #include "common.hpp"
 #include "pa_decode.hpp"
@@ -61,254 +69,312 @@ struct PaPrefillArgs {
   float* part_ml;
 };
 
-constexpr int kKeyBlock = 32;
+constexpr int kStageKeys = 64;
+constexpr int kWaves = 4;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
-constexpr float kPScale = 16384.f;  // P enters the PV MFMA as p * 2^14 (hi + lo)
+constexpr float kPShift = 14.f, kPScale = 16384.f;  // P enters the PV MFMA as p * 2^14 (hi + lo)
 
 __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
   hi = (_Float16)x;
   lo = (_Float16)(x - (float)hi);
 }
 
-template <int D, int TS, int NW>
-__global__ __launch_bounds__(64 * NW) void pa_prefill_kernel(PaPrefillArgs a) {
-  constexpr int KB = kKeyBlock;
-  constexpr int KSTR = D + 8;   // K row stride (halves): conflict-free 16-B row reads
-  constexpr int VSTR = D + 16;  // V row stride (halves): 8·odd dwords, so the
-                                // 64 lanes of a transposed read hit 64 banks
-  constexpr int CPR = D / 8;    // 16-byte chunks per key row
-  constexpr int NCH = KB * CPR; // chunks per block, each of K and V
-  constexpr int NTH = 64 * NW;
-  constexpr int CPT = NCH / NTH;
-  constexpr int NKK = D / 32;   // k-steps of q.k
-  constexpr int ND = D / 16;    // 16-dim tiles of the output
-  static_assert(NCH % NTH == 0 && D % 32 == 0 && KB % TS == 0, "shape");
-  __shared__ __attribute__((aligned(16))) _Float16 Ks[KB * KSTR];
-  __shared__ __attribute__((aligned(16))) _Float16 Vs[KB * VSTR];
-  __shared__ int kval[KB];
+template <int D, int TS, int MT>
+__global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArgs a) {
+  constexpr int ROWB = 2 * D;                // bytes of a key's row
+  constexpr int CPR = D / 8;                 // its 16-byte chunks
+  constexpr int LOADS = 16 * ROWB / 1024;    // 1 KiB loads of a wave's 16 keys, each of K and V
+  constexpr int NKK = D / 32;                // k-steps of q.k
+  constexpr int ND = D / 16;                 // 16-dim tiles of the output
+  constexpr int QW = 16 * MT, QT = QW * kWaves;  // queries of a wave, of the workgroup
+  static_assert(D % 32 == 0 && TS % 16 == 0 && kStageKeys == 16 * kWaves, "shape");
+  __shared__ u32x4 lds[2][2][kStageKeys * CPR];  // [stage][K, V][key][chunk, exchanged]
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
+  const int lane = threadIdx.x & 63;
   const int w = wave_id_uniform();
   const int g = lane >> 4;
   const int c = lane & 15;
-  const int h = blockIdx.y;
-  const int qbase = blockIdx.x * 16 * NW;
-  const int qi = qbase + w * 16 + c;  // this lane's query (column of S^T / O^T)
-  const int qpos = a.p0 + qi;
-  const int lastpos = a.p0 + min(qbase + 16 * NW, a.m) - 1;  // last key any query here sees
+  // heads go round the XCDs: the tiles of a head share its K and V in one L2, and
+  // every XCD has long and short ones
+  const int h = blockIdx.x;
+  const int qbase = ((int)gridDim.y - 1 - (int)blockIdx.y) * QT;  // the longest first
+  const int q0 = qbase + w * QW;                                  // this wave's first query
+  const int lastpos = a.p0 + min(qbase + QT, a.m) - 1;  // last key any query here sees
+  const int wave_first = a.p0 + q0;
+  const int wave_last = q0 < a.m ? a.p0 + min(q0 + QW, a.m) - 1 : -1;
   const int split = blockIdx.z;
-  const int kb0 = split * a.pps * TS / KB;
-  const int nblk = min((split + 1) * a.pps * TS / KB, lastpos / KB + 1);
+  const int s0 = split * (a.pps * TS / kStageKeys);
+  const int s1 = min(a.nsplit > 1 ? (split + 1) * (a.pps * TS / kStageKeys) : INT_MAX,
+                     lastpos / kStageKeys + 1);
   // no query of this workgroup reaches this split: the merge never reads it
-  if (kb0 >= nblk) return;
+  if (s0 >= s1) return;
   const int32_t* pt = a.pt_row + (size_t)h * a.max_tiles;
+
+  // Lanes 0..3: the page of a stage's 16-key groups (-1: none, or past lastpos).
+  auto pages_of = [&](int s) -> int {
+    const int key = s * kStageKeys + 16 * (lane & 3), tile = key / TS;
+    const int pg = s < s1 && key <= lastpos && tile < a.max_tiles ? pt[tile] : -1;
+    return pg < a.num_pages ? pg : -1;
+  };
+  // LDS position of chunk `ch` of key k (0..15 of a group): 16 rows that read one
+  // chunk each meet 16 different bank groups, and so do 8 rows that read two
+  auto exchange = [](int k, int ch) { return ch ^ (CPR == 16 ? ((k << 1) | (k >> 3)) & 15 : (k >> 1) & 7); };
+  auto issue = [&](int buf, int s, int page) {  // this wave's 16 keys of stage s
+    const int key0 = s * kStageKeys + 16 * w, at = 16 * w * CPR;
+    if (page < 0) {  // masked: V = 0, since 0 * NaN would not be 0
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        lds[buf][0][at + 64 * i + lane] = u32x4{0u, 0u, 0u, 0u};
+        lds[buf][1][at + 64 * i + lane] = u32x4{0u, 0u, 0u, 0u};
+      }
+      return;
+    }
+    const size_t base = (size_t)page * a.page_stride + (size_t)(key0 % TS) * ROWB;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int row = (64 * i + lane) / CPR, ch = exchange(row, (64 * i + lane) % CPR);
+      // (rows past lastpos may never have been written: the last one that was, masked)
+      const size_t off = base + (size_t)min(row, lastpos - key0) * ROWB + 16 * ch;
+      load_to_lds(a.k_pool + off, &lds[buf][0][at + 64 * i]);
+      load_to_lds(a.v_pool + off, &lds[buf][1][at + 64 * i]);
+    }
+  };
+  int pages = pages_of(s0), next = pages_of(s0 + 1);
+  unsigned valid = (unsigned)__ballot(pages >= 0) & 15u;
+  issue(0, s0, __builtin_amdgcn_readlane(pages, w));
 
   // Q^T B-operand fragments: lane holds q[qi][32kk + 8g .. +7] (pre-scaled by
   // qscale), hi + lo.  The query's values are also scaled by a power of two
   // 2^(14-e) (|q|max < 2^e) so the lo halves stay clear of fp16 subnormals,
   // which the MFMA does not keep; S is scaled back exactly after the MFMA.
-  float qx[NKK][8];
-  float amax = 0.f;
+  f16x8 qh[MT][NKK], ql[MT][NKK];
+  float qinv[MT];
 #pragma unroll
-  for (int kk = 0; kk < NKK; ++kk) {
-    f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
-    if (qi < a.m) {
-      const float* qp = a.q + (size_t)qi * a.q_stride + h * D + 32 * kk + 8 * g;
-      x0 = *reinterpret_cast<const f32x4*>(qp);
-      x1 = *reinterpret_cast<const f32x4*>(qp + 4);
-    }
+  for (int t = 0; t < MT; ++t) {
+    const int qi = q0 + 16 * t + c;
+    float qx[NKK][8];
+    float amax = 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      qx[kk][e] = x0[e] * a.qscale;
-      qx[kk][4 + e] = x1[e] * a.qscale;
-      amax = fmaxf(amax, fmaxf(fabsf(qx[kk][e]), fabsf(qx[kk][4 + e])));
-    }
-  }
-  amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-  amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-  int qe = 0;
-  (void)frexpf(amax, &qe);  // amax < 2^qe (0 for amax == 0)
-  qe = min(max(qe, -100), 100);
-  const float qsc = ldexpf(1.f, 14 - qe), qinv = ldexpf(1.f, qe - 14);
-  f16x8 qh[NKK], ql[NKK];
-#pragma unroll
-  for (int kk = 0; kk < NKK; ++kk)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      _Float16 hi, lo;
-      split_f16(qx[kk][e] * qsc, hi, lo);
-      qh[kk][e] = hi;
-      ql[kk][e] = lo;
-    }
-
-  // Staging: chunk i of a thread = (key ch / CPR, dims 8 (ch % CPR)) of K and
-  // of V — rows coalesced, both stored row-major ([key][d]); the PV product
-  // reads V transposed with ds_read_b64_tr_b16.
-  u32x4 kr[CPT], vr[CPT];
-  int vok[CPT];
-  auto page_of = [&](int kg) -> int {  // page of key position kg, -1 if none / past lastpos
-    const int tile = kg / TS;
-    int pg = (kg <= lastpos && tile < a.max_tiles) ? pt[tile] : -1;
-    return (pg >= 0 && pg < a.num_pages) ? pg : -1;
-  };
-  auto load = [&](int kb) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int ch = tid + i * NTH;
-      const int key = ch / CPR, d0 = (ch % CPR) * 8;
-      const int kg = kb * KB + key;
-      const int pg = page_of(kg);
-      const size_t off = (size_t)pg * a.page_stride + ((kg % TS) * D + d0) * 2;
-      vok[i] = pg >= 0;
-      // masked keys stage V = 0: a never-written row may hold NaN (0 * NaN)
-      kr[i] = pg >= 0 ? *reinterpret_cast<const u32x4*>(a.k_pool + off) : u32x4{0u, 0u, 0u, 0u};
-      vr[i] = pg >= 0 ? *reinterpret_cast<const u32x4*>(a.v_pool + off) : u32x4{0u, 0u, 0u, 0u};
-    }
-  };
-  auto stage = [&]() {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int ch = tid + i * NTH;
-      const int key = ch / CPR, d0 = (ch % CPR) * 8;
-      *reinterpret_cast<u32x4*>(&Ks[key * KSTR + d0]) = kr[i];
-      *reinterpret_cast<u32x4*>(&Vs[key * VSTR + d0]) = vr[i];
-      if (d0 == 0) kval[key] = vok[i];
-    }
-  };
-
-  f32x4 O[ND];
-#pragma unroll
-  for (int nd = 0; nd < ND; ++nd) O[nd] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float mrun = kNegSentinel, lrun = 0.f;
-
-  load(kb0);
-  for (int kb = kb0; kb < nblk; ++kb) {
-    if (kb > kb0) __syncthreads();  // every wave is done reading block kb-1
-    stage();
-    __syncthreads();
-    if (kb + 1 < nblk) load(kb + 1);  // next block's loads fly during this block's math
-
-    // S^T: two 16-key tiles
-    f32x4 s[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kk = 0; kk < NKK; ++kk) {
-        const f16x8 kf = *reinterpret_cast<const f16x8*>(&Ks[(16 * t + c) * KSTR + 32 * kk + 8 * g]);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[kk], s[t], 0, 0, 0);
-        s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[kk], s[t], 0, 0, 0);
+    for (int kk = 0; kk < NKK; ++kk) {
+      f32x4 x0 = {0.f, 0.f, 0.f, 0.f}, x1 = x0;
+      if (qi < a.m) {
+        const float* qp = a.q + (size_t)qi * a.q_stride + h * D + 32 * kk + 8 * g;
+        x0 = *reinterpret_cast<const f32x4*>(qp);
+        x1 = *reinterpret_cast<const f32x4*>(qp + 4);
       }
-      s[t] *= qinv;
-    }
-    // causal + missing-page mask, online softmax (per query = per lane)
-    bool ok[2][4];
-    float mloc = kNegSentinel;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int key = 16 * t + 4 * g + r;
-        ok[t][r] = kval[key] != 0 && kb * KB + key <= qpos;
-        if (ok[t][r]) mloc = fmaxf(mloc, s[t][r]);
+      for (int e = 0; e < 4; ++e) {
+        qx[kk][e] = x0[e] * a.qscale;
+        qx[kk][4 + e] = x1[e] * a.qscale;
+        amax = fmaxf(amax, fmaxf(fabsf(qx[kk][e]), fabsf(qx[kk][4 + e])));
       }
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-    mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
-    const float mnew = fmaxf(mrun, mloc);
-    const float corr = __builtin_amdgcn_exp2f(mrun - mnew);
-    lrun *= corr;
+    }
+    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+    int qe = 0;
+    (void)frexpf(amax, &qe);  // amax < 2^qe (0 for amax == 0)
+    qe = min(max(qe, -100), 100);
+    const float qsc = ldexpf(1.f, 14 - qe);
+    qinv[t] = ldexpf(1.f, qe - 14);
 #pragma unroll
-    for (int nd = 0; nd < ND; ++nd) O[nd] *= corr;
-    f16x8 ph, pl;
+    for (int kk = 0; kk < NKK; ++kk)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float p = ok[t][r] ? __builtin_amdgcn_exp2f(s[t][r] - mnew) : 0.f;
-        lrun += p;
+      for (int e = 0; e < 8; ++e) {
         _Float16 hi, lo;
-        split_f16(p * kPScale, hi, lo);  // p <= 1: scaled clear of fp16 subnormals
-        ph[4 * t + r] = hi;
-        pl[4 * t + r] = lo;
+        split_f16(qx[kk][e] * qsc, hi, lo);
+        qh[t][kk][e] = hi;
+        ql[t][kk][e] = lo;
       }
-    mrun = mnew;
-    // O^T += V^T · P^T.  A operand lane l: V^T[d = 16nd + (l&15)][k 8g+j] =
-    // V[key(8g+j)][d], keys 4g..4g+3 then 16+4g..16+4g+3: two transposed
-    // reads of 4 V rows x 16 columns, lane 4q+p addressing row q, columns 4p..
+  }
+
+  f32x4 O[ND][MT];
+  float nrun[MT], lrun[MT];
 #pragma unroll
-    for (int nd = 0; nd < ND; ++nd) {
-      const int q4 = c >> 2, p4 = c & 3;
-      const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)&Vs[(4 * g + q4) * VSTR + 16 * nd + 4 * p4]);
-      const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)&Vs[(16 + 4 * g + q4) * VSTR + 16 * nd + 4 * p4]);
-      const f16x8 vf = __builtin_bit_cast(
-          f16x8, s16x8{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]});
-      O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, O[nd], 0, 0, 0);
-      O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, O[nd], 0, 0, 0);
+  for (int t = 0; t < MT; ++t) {
+    nrun[t] = kNegSentinel;
+    lrun[t] = 0.f;
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd) O[nd][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  int buf = 0;
+  for (int s = s0; s < s1; ++s, buf ^= 1) {
+    wait_lds_loads();
+    __syncthreads();  // stage s has landed, the other buffer is read out
+    const unsigned valid_next = (unsigned)__ballot(next >= 0) & 15u;
+    if (s + 1 < s1) issue(buf ^ 1, s + 1, __builtin_amdgcn_readlane(next, w));
+    next = pages_of(s + 2);
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const int key0 = s * kStageKeys + 32 * kb;
+      if (key0 > wave_last) break;
+      const unsigned here = valid >> (2 * kb) & 3u;  // of the block's two 16-key tiles
+      // S^T: two 16-key tiles
+      f32x4 sc[MT][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) sc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const u32x4* krow = &lds[buf][0][(32 * kb + 16 * u + c) * CPR];
+#pragma unroll
+        for (int kk = 0; kk < NKK; ++kk) {
+          const f16x8 kf = __builtin_bit_cast(f16x8, krow[exchange(c, 4 * kk + g)]);
+#pragma unroll
+          for (int t = 0; t < MT; ++t) {
+            sc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[t][kk], sc[t][u], 0, 0, 0);
+            sc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[t][kk], sc[t][u], 0, 0, 0);
+          }
+        }
+      }
+      // The products are read before the branch on `mask`: the compiler leaves out the
+      // wait for a matrix instruction whose result is first read behind one.
+      float mloc[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        mloc[t] = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) mloc[t] = fmaxf(mloc[t], sc[t][u][r]);
+        asm volatile("" : "+v"(mloc[t]));
+      }
+      // causal + missing-page mask
+      if (key0 + 31 > wave_first || here != 3u) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          mloc[t] = -INFINITY;
+#pragma unroll
+          for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              if (!(here >> u & 1u) || key0 + 16 * u + 4 * g + r > wave_first + 16 * t + c)
+                sc[t][u][r] = -INFINITY;
+              mloc[t] = fmaxf(mloc[t], sc[t][u][r]);
+            }
+        }
+      }
+      // online softmax (per query = per lane): p = 2^(s - n), n the running maximum
+      // less 14, so that p comes out scaled for the halves; s is scaled back in the same
+      // operation
+      f16x8 ph[MT], pl[MT];
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const float nloc = rows_max(mloc[t]) * qinv[t] - kPShift;
+        if (__any(nloc > nrun[t])) {
+          const float nnew = fmaxf(nrun[t], nloc);
+          const float corr = __builtin_amdgcn_exp2f(nrun[t] - nnew);
+          lrun[t] *= corr;
+#pragma unroll
+          for (int nd = 0; nd < ND; ++nd) O[nd][t] *= corr;
+          nrun[t] = nnew;
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float p = __builtin_amdgcn_exp2f(fmaf(sc[t][u][r], qinv[t], -nrun[t]));
+            lrun[t] += p;
+            _Float16 hi, lo;
+            split_f16(p, hi, lo);  // p <= 2^14: clear of fp16 subnormals
+            ph[t][4 * u + r] = hi;
+            pl[t][4 * u + r] = lo;
+          }
+      }
+      // O^T += V^T · P^T.  A operand lane l: V^T[d = 16nd + (l&15)][k 8g+j] =
+      // V[key(8g+j)][d], keys 4g..4g+3 then 16+4g..16+4g+3: two transposed
+      // reads of 4 V rows x 16 columns, lane 4q+p addressing row q, columns 4p..
+      const int vk = 4 * g + (c >> 2), p4 = c & 3;
+      const char* v0 = reinterpret_cast<const char*>(&lds[buf][1][(32 * kb + vk) * CPR]) + 8 * (p4 & 1);
+#pragma unroll
+      for (int nd = 0; nd < ND; ++nd) {
+        const char* at = v0 + 16 * exchange(vk, 2 * nd + (p4 >> 1));
+        const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)at);
+        const s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (__attribute__((address_space(3))) s16x4*)(at + 16 * ROWB));
+        const f16x8 vf = __builtin_bit_cast(
+            f16x8, s16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]});
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+          O[nd][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[t], O[nd][t], 0, 0, 0);
+          O[nd][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[t], O[nd][t], 0, 0, 0);
+        }
+      }
     }
+    valid = valid_next;
   }
 
   // the 4 lanes of a query hold partial sums over their keys
-  lrun += __shfl_xor(lrun, 16, 64);
-  lrun += __shfl_xor(lrun, 32, 64);
-  if (qi < a.m) {
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    lrun[t] += __shfl_xor(lrun[t], 16, 64);
+    lrun[t] += __shfl_xor(lrun[t], 32, 64);
+    lrun[t] *= 1.0f / kPScale;
+    const int qi = q0 + 16 * t + c;
+    if (qi >= a.m) continue;
     if (a.part_acc) {  // split partial state (unnormalised, log2 units)
       const size_t pidx = ((size_t)qi * a.H + h) * a.nsplit + split;
       float* o = a.part_acc + pidx * D + 4 * g;
 #pragma unroll
-      for (int nd = 0; nd < ND; ++nd) *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * (1.0f / kPScale);
-      if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{mrun, lrun};
+      for (int nd = 0; nd < ND; ++nd)
+        *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd][t] * (1.0f / kPScale);
+      if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{nrun[t] + kPShift, lrun[t]};
     } else {
-      const float inv = 1.0f / (lrun + 1e-6f) * (1.0f / kPScale);
+      const float inv = 1.0f / (lrun[t] + 1e-6f) * (1.0f / kPScale);
       float* o = a.out + (size_t)qi * a.out_stride + h * D + 4 * g;
 #pragma unroll
-      for (int nd = 0; nd < ND; ++nd) *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * inv;
+      for (int nd = 0; nd < ND; ++nd) *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd][t] * inv;
     }
   }
 }
 
 template <int D, int TS>
-hipError_t launch_prefill(const PaPrefillArgs& a, int nw, hipStream_t st) {
-  if (nw == 4) {
-    const dim3 grid((a.m + 63) / 64, a.H, a.nsplit);
-    hipLaunchKernelGGL((pa_prefill_kernel<D, TS, 4>), grid, dim3(256), 0, st, a);
-  } else {
-    const dim3 grid((a.m + 31) / 32, a.H, a.nsplit);
-    hipLaunchKernelGGL((pa_prefill_kernel<D, TS, 2>), grid, dim3(128), 0, st, a);
-  }
+hipError_t launch_prefill(const PaPrefillArgs& a, int mt, hipStream_t st) {
+  const int qt = 16 * mt * kWaves;
+  const dim3 grid(a.H, (a.m + qt - 1) / qt, a.nsplit);
+  if (mt == 2)
+    hipLaunchKernelGGL((pa_prefill_kernel<D, TS, 2>), grid, dim3(64 * kWaves), 0, st, a);
+  else
+    hipLaunchKernelGGL((pa_prefill_kernel<D, TS, 1>), grid, dim3(64 * kWaves), 0, st, a);
   return hipGetLastError();
 }
 
-// Launch geometry: NW waves (16 queries each) per workgroup; the key range is
-// split until the grid holds about kTargetWgs workgroups (4 per CU), in
-// splits of whole 32-key blocks and at least 2 blocks each.
-constexpr int kTargetWgs = 1024;
+// Launch geometry: 32 queries per wave, 16 where the chunk has few.  The key range is
+// cut into splits of `per` stages, the length for which the rounds of workgroups (2 per
+// CU) times their length is least, a split more counted as half a stage for its merge;
+// no more than split_bound of them a query (2048 queries x 16 heads: 11 stages, 512
+// workgroups in one round).
+constexpr int kRound = 512;
 struct PrefillPlan {
-  int nw, nsplit, pps;
+  int mt, nsplit, pps;
 };
+int queries_per_wg(int m) { return m > 64 ? 128 : 64; }
+int split_bound(int H, int m) {
+  const int nq = (m + queries_per_wg(m) - 1) / queries_per_wg(m);
+  return std::min(2 * kRound / std::max(nq * H, 1) + 1, 128);
+}
 PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   PrefillPlan p;
-#if LLM_TUNING
-  p.nw = env_int("LLM_PREFILL_NW", 4) == 2 ? 2 : 4;
-#else
-  p.nw = 4;
-#endif
-  const int TS = kv->page_size;
-  const int step = kKeyBlock / TS;  // tiles per key block
-  const int ntiles = (p0 + m + TS - 1) / TS;
-  const int nq = (m + 16 * p.nw - 1) / (16 * p.nw);
-  const int want = std::min(std::max(kTargetWgs / std::max(nq * kv->num_heads, 1), 1), 128);
-  int pps = (ntiles + want - 1) / want;
-  pps = std::max((pps + step - 1) / step * step, 2 * step);
-  p.pps = pps;
-  p.nsplit = std::max(1, std::min((ntiles + pps - 1) / pps, 128));
-  if (p.nsplit * pps < ntiles) {  // > 128 splits: lengthen them
-    p.pps = ((ntiles + 127) / 128 + step - 1) / step * step;
-    p.nsplit = (ntiles + p.pps - 1) / p.pps;
+  const int qt = queries_per_wg(m), H = kv->num_heads;
+  p.mt = qt / 64;
+  const int most = (p0 + m - 1) / kStageKeys + 1;
+  const int bound = split_bound(H, m);
+  int best = most;
+  double least = 1e30;
+  for (int n = 1; n <= std::min(bound, most); ++n) {
+    const int per = (most + n - 1) / n;
+    long long wgs = 0;
+    for (int q = 0; q < m; q += qt)
+      wgs += ((p0 + std::min(q + qt, m) - 1) / kStageKeys + per) / per;
+    const double cost = (double)((wgs * H + kRound - 1) / kRound) * per + 0.5 * (most + per - 1) / per;
+    if (cost < least) {
+      least = cost;
+      best = per;
+    }
   }
+  p.nsplit = (most + best - 1) / best;
+  p.pps = best * kStageKeys / kv->page_size;
   return p;
 }
 
@@ -324,6 +390,12 @@ size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m) {
   const PrefillPlan p = prefill_plan(kv, p0, m);
   if (p.nsplit <= 1) return 0;
   return (size_t)m * kv->num_heads * p.nsplit * (size_t)(kv->head_dim + 2) * sizeof(float);
+}
+
+size_t pa_prefill_ws_bound(const pa_kv_view* kv, int m) {
+  if (!pa_prefill_supported(kv) || m <= 0) return 0;
+  return (size_t)m * kv->num_heads * split_bound(kv->num_heads, m) * (size_t)(kv->head_dim + 2) *
+         sizeof(float);
 }
 
 int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, float* out,
@@ -378,9 +450,9 @@ int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, floa
   hipError_t e;
   const int TS = kv->page_size;
   if (D == 64)
-    e = TS == 16 ? launch_prefill<64, 16>(a, pl.nw, st) : launch_prefill<64, 32>(a, pl.nw, st);
+    e = TS == 16 ? launch_prefill<64, 16>(a, pl.mt, st) : launch_prefill<64, 32>(a, pl.mt, st);
   else
-    e = TS == 16 ? launch_prefill<128, 16>(a, pl.nw, st) : launch_prefill<128, 32>(a, pl.nw, st);
+    e = TS == 16 ? launch_prefill<128, 16>(a, pl.mt, st) : launch_prefill<128, 32>(a, pl.mt, st);
   if (e != hipSuccess) return fail(LLM_ERR_HIP, std::string("pa_prefill launch: ") + hipGetErrorString(e));
   if (split)
     return pa_merge_rows_internal(a.part_acc, a.part_ml, (rows && !rows->keep_out) ? nullptr : out,

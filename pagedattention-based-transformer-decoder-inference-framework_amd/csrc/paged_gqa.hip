@@ -123,8 +123,7 @@ struct Rows {
 #pragma unroll
         for (int r = 0; r < 4; ++r) mloc = fmaxf(mloc, s[t][u][r]);
       }
-      mloc = fmaxf(mloc, __shfl_xor(mloc, 16, 64));
-      mloc = fmaxf(mloc, __shfl_xor(mloc, 32, 64));
+      mloc = rows_max(mloc);
       if (__any(mloc > m[t])) {
         const float mnew = fmaxf(m[t], mloc);  // >= the sentinel: masked scores stay far below
         const float corr = __builtin_amdgcn_exp2f(m[t] - mnew);

@@ -89,6 +89,28 @@ def test_pa_prefill_vs_oracle(gpu, oracle, H, D, ts, p0, m, row, split):
     assert_parity(out, dec.cpu().numpy(), RTOL, ATOL_FRAC)
 
 
+@pytest.mark.parametrize("D,ts", [(64, 16), (64, 32), (128, 16), (128, 32)])
+@pytest.mark.parametrize("p0,m", [
+    (0, 63), (0, 64), (0, 65),      # 16 or 32 queries a wave
+    (0, 129), (95, 128),            # one query past a tile; a tile that ends inside a stage
+    (1, 127), (448, 65), (449, 256),  # stages of 64 keys: first and last full or one key long
+])
+def test_pa_prefill_tile_edges(gpu, oracle, D, ts, p0, m):
+    """Query tiles of 64 and 128, key stages of 64, pages missing inside a stage, keys past
+    the context never written; cut into pieces and in one pass."""
+    import llm_capi
+    rng = np.random.default_rng(p0 + 3 * m + D + ts)
+    H = 3
+    kp, vp, pt = _case(rng, rows=2, H=H, D=D, T=p0 + m, ts=ts, missing=0.1, nan_tail=True)
+    q = (rng.standard_normal((m, H, D)) * D ** -0.25).astype(np.float32)
+    ref = _oracle(oracle, q, kp, vp, pt, 1, p0)
+    for split in (True, False):
+        out = llm_capi.pa_prefill(_dev(q), _dev(kp), _dev(vp), _dev(pt), row=1, p0=p0,
+                                  split=split).cpu().numpy()
+        assert np.isfinite(out).all()
+        assert_parity(out, ref, RTOL, ATOL_FRAC)
+
+
 def test_pa_prefill_missing_pages_and_scale(gpu, oracle):
     import llm_capi
     rng = np.random.default_rng(11)
