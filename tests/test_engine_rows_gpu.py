@@ -1,0 +1,55 @@
+"""Logits rows of an engine step in the caller's memory: pageable memory goes through the
+engine's pinned pieces of 512 KiB, four at a time, memory that the runtime knows does not;
+both hold the same bytes."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import _layer_stack as T
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def eng(gpu, tmp_path_factory):
+    import engine
+    cfg = T.config([(T.attn(), None)], vocab=5003)
+    folder = T.save(tmp_path_factory.mktemp("model"), cfg, T.weights(cfg, 3))
+    with engine.Engine(folder, dtype="float32", max_seqs=4, max_tokens=1024,
+                       max_step_tokens=128) as e:
+        yield e
+
+
+def step(eng, entries, out):
+    from llm_capi import EngineEntry
+    arr, keep = (EngineEntry * len(entries))(), []
+    for i, (seq, tok, want) in enumerate(entries):
+        t, w = np.asarray(tok, np.int32), np.asarray(want, np.int32)
+        keep.append((t, w))
+        arr[i] = EngineEntry(seq, t.ctypes.data, t.size, w.ctypes.data, w.size)
+    eng._check(eng.lib.llm_engine_step(eng._h, arr, len(entries), ctypes.c_void_p(out)))
+
+
+# 26 rows of 20,012 bytes: just under one piece; 27 and 105: over one and over four; 128
+# in order, 127 in gaps, and a batch of two passes whose rows lie apart
+@pytest.mark.parametrize("lens,pick", [
+    ([1], None), ([26], None), ([27], None), ([105], None), ([128], None), ([60, 67], "odd"),
+    ([100, 90], "back"), ([3], "none"),
+])
+def test_rows_by_both_ways(eng, lens, pick):
+    import torch
+    rng = np.random.default_rng(len(lens) + lens[0])
+    toks = [rng.integers(0, eng.vocab, n) for n in lens]
+    wants = [{None: list(range(n)), "odd": list(range(1, n, 2)), "back": list(range(n))[::-1],
+              "none": []}[pick] for n in lens]
+    rows = sum(map(len, wants))
+    pinned = torch.full((max(rows, 1), eng.vocab), -7.0, pin_memory=True)
+    plain = np.full((max(rows, 1), eng.vocab), 7.0, np.float32)
+    for out in (pinned.data_ptr(), plain.ctypes.data):
+        seqs = [eng.open_seq() for _ in lens]
+        step(eng, [(s, t, w) for s, t, w in zip(seqs, toks, wants)], out)
+        for s in seqs:
+            eng.close_seq(s)
+    if rows:
+        np.testing.assert_array_equal(plain, pinned.numpy())
