@@ -116,7 +116,8 @@ struct PaMergeArgs {
   int B, H, D, T, TS, pps, nsplit, max_tiles;
 };
 
-template <int DPL>
+// RAGGED: the split launch dealt its splits out by need (ragged_plan).
+template <int DPL, bool RAGGED>
 __global__ __launch_bounds__(256) void pa_merge_kernel(PaMergeArgs a) {
   const int lane = lane_id();
   const int bh = blockIdx.x * 4 + wave_id_uniform();
@@ -127,11 +128,20 @@ __global__ __launch_bounds__(256) void pa_merge_kernel(PaMergeArgs a) {
   const int ntiles = min((Tb + a.TS - 1) / a.TS, a.max_tiles);
   const int pps = row_pps(a.pps, a.nsplit, ntiles);
   // pps < 0: every split holds a partial (beam launches: cost-balanced splits)
-  const int ns = a.pps < 0 ? a.nsplit : min(a.nsplit, (ntiles + pps - 1) / pps);
+  int held = a.nsplit, ns = a.pps < 0 ? a.nsplit : min(a.nsplit, (ntiles + pps - 1) / pps);
+  size_t at = (size_t)bh * a.nsplit;
+  if constexpr (RAGGED) {
+    const RaggedPlan p = ragged_plan(a.context_lens, a.B, a.T, a.TS, a.max_tiles, a.nsplit);
+    if (p.unit) {
+      const RowSplits r = ragged_find(p, [&](int row, int, int) { return row == b; });
+      held = r.count;
+      ns = (ntiles + p.unit - 1) / p.unit;
+      at = (size_t)r.first * a.H + (size_t)(bh % a.H) * r.count;
+    }
+  }
   float acc[DPL];
-  const float inv = merge_head<DPL, 16>(a.part_ml + (size_t)bh * a.nsplit * 2,
-                                        a.part_acc + (size_t)bh * a.nsplit * a.D, a.nsplit, ns,
-                                        a.D, acc);
+  const float inv =
+      merge_head<DPL, 16>(a.part_ml + at * 2, a.part_acc + at * a.D, held, ns, a.D, acc);
   float* o = a.out + (size_t)bh * a.D;
 #pragma unroll
   for (int j = 0; j < DPL; ++j) {
@@ -269,7 +279,11 @@ hipError_t launch_split(const PaSplitArgs& a, bool direct, hipStream_t st, bool*
   if constexpr (KVT != LLM_F16) {
     // other KV element types: the standard schedule (no beam-prefetch form)
     constexpr int ST = split_stages<D, TS, KVT>();
-    if (direct)
+    if (a.ragged)
+      hipLaunchKernelGGL((pa_split_kernel<D, TS, false, 16384, kKvLoadAux, ST, 0, false, false, KVT,
+                                          true, false, false, 0, false, false, false, true>),
+                         grid, block, 0, st, a);
+    else if (direct)
       hipLaunchKernelGGL((pa_split_kernel<D, TS, true, 16384, kKvLoadAux, ST, 0, false, false, KVT>),
                          grid, block, 0, st, a);
     else
@@ -310,6 +324,10 @@ hipError_t launch_split(const PaSplitArgs& a, bool direct, hipStream_t st, bool*
                                         false, true, LLM_F16, true, false, false, 0, false, true, true>),
                        grid, block, 0, st, a);
     *beam = true;
+  } else if (a.ragged) {
+    hipLaunchKernelGGL((pa_split_kernel<D, TS, false, 16384, kKvLoadAux, ST, 0, false, false, LLM_F16,
+                                        true, false, false, 0, false, false, false, true>),
+                       grid, block, 0, st, a);
   } else if (direct) {
     hipLaunchKernelGGL((pa_split_kernel<D, TS, true, 16384, kKvLoadAux, ST>), grid, block, 0, st, a);
   } else {
@@ -470,15 +488,21 @@ extern "C" size_t pa_decode_workspace_bytes(int B, int H, int D, int max_tiles,
 
 int llm::pa_merge_splits_internal(const float* part_acc, const float* part_ml, float* out,
                                   const int32_t* context_lens, int B, int H, int D, int T, int TS,
-                                  int pps, int nsplit, int max_tiles, hipStream_t st) {
+                                  int pps, int nsplit, int max_tiles, hipStream_t st,
+                                  bool ragged) {
   PaMergeArgs mg{part_acc, part_ml, out, context_lens, B, H, D, T, TS, pps, nsplit, max_tiles};
-  const dim3 grid((B * H + 3) / 4);
-  if (D <= 64)
-    hipLaunchKernelGGL(pa_merge_kernel<1>, grid, dim3(256), 0, st, mg);
-  else if (D <= 128)
-    hipLaunchKernelGGL(pa_merge_kernel<2>, grid, dim3(256), 0, st, mg);
-  else
-    hipLaunchKernelGGL(pa_merge_kernel<4>, grid, dim3(256), 0, st, mg);
+  const auto launch = [&](auto r) {
+    constexpr bool R = decltype(r)::value;
+    const dim3 grid((B * H + 3) / 4);
+    if (D <= 64)
+      hipLaunchKernelGGL((pa_merge_kernel<1, R>), grid, dim3(256), 0, st, mg);
+    else if (D <= 128)
+      hipLaunchKernelGGL((pa_merge_kernel<2, R>), grid, dim3(256), 0, st, mg);
+    else
+      hipLaunchKernelGGL((pa_merge_kernel<4, R>), grid, dim3(256), 0, st, mg);
+  };
+  if (ragged) launch(std::true_type{});
+  else launch(std::false_type{});
   LLM_HIP_RET(hipGetLastError());
   return LLM_OK;
 }
@@ -709,6 +733,7 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
   a.nsplit = nsplit;
   a.group = std::max(1, std::min(row_group, 4));
   a.qscale = sm_scale * kLog2e;
+  a.ragged = context_lens && !rows && !direct && row_group == 1 && pps_fixed <= 0 && B <= kRaggedRows;
   const bool wgm = wgm_ok && !direct && a.group == 1 && nsplit <= kWgmMaxSplits;
   if (!direct && !wgm) {  // (the workgroup merge keeps its splits' states in LDS)
     const size_t need = (size_t)B * H * nsplit * (size_t)(D + 2) * sizeof(float);
@@ -754,7 +779,7 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
                                   kv->max_tiles, st);
   if (!direct) {
     const int r = pa_merge_splits_internal(a.part_acc, a.part_ml, out, context_lens, B, H, D, T,
-                                           TS, beam ? -1 : pps_fixed, nsplit, kv->max_tiles, st);
+                                           TS, beam ? -1 : pps_fixed, nsplit, kv->max_tiles, st, a.ragged);
     if (r != LLM_OK) return r;
   }
   if (row_out) {  // single split: out is final; convert it in a row pass

@@ -101,7 +101,8 @@ struct PaSplitArgs {
   // workgroups (blockIdx b, b + 256, b + 512, b + 768 at C4) are then 4 split
   // pairs of 4 (group, head)s rather than 4 sequence pairs, and the splits of
   // one (group, head) share an XCD (blockIdx mod 8) and its L2.
-  int smaj;  // (last: the earlier fields keep their kernel-argument offsets)
+  int smaj;
+  bool ragged;  // host only: the RAGGED form (last two: the fields before keep their offsets)
 };
 
 constexpr int kWgmMaxSplits = 8;  // one merge batch (pa_merge_row_kernel's kMergeBatch)
@@ -114,6 +115,78 @@ constexpr int kMaxSplits = 128;  // split weights held in two registers per merg
 __device__ __forceinline__ int row_pps(int pps_fixed, int nsplit, int ntiles) {
   if (pps_fixed > 0) return pps_fixed;
   return min(max((ntiles + nsplit - 1) / nsplit, 1), kMaxPps);
+}
+
+// Splits of rows of different contexts (RAGGED, launches without row outputs): the same
+// B * nsplit splits a head, dealt out by need.  A row of n tiles gets ceil(n / unit) of
+// them, one at least, at unit = ceil(tiles of all rows / (B * (nsplit - 1))), which makes
+// no more than B * nsplit; equal counts leave the chip to the longest row (32 rows of 1 ..
+// 4096 tokens, half of them under 64: 16 heads of 128 bf16 53 us, so 35).  Where that
+// does not shorten the longest split, as for rows of one length, every row has nsplit.
+// Partials lie in the order (row, head, split) either way.  Lane l holds rows l, 64 + l, ...
+constexpr int kRaggedRows = 256;
+struct RaggedPlan {
+  int count[kRaggedRows / 64];  // splits of the lane's rows
+  int unit;                     // tiles of a split; 0: nsplit equal splits
+};
+struct RowSplits {
+  int row, first, count;  // first: splits of the rows before it
+};
+
+__device__ __forceinline__ int ragged_tiles(const int32_t* lens, int row, int T, int TS, int max_tiles) {
+  return min((min(max(lens[row], 0), T) + TS - 1) / TS, max_tiles);
+}
+
+__device__ __forceinline__ RaggedPlan ragged_plan(const int32_t* lens, int B, int T, int TS,
+                                                  int max_tiles, int nsplit) {
+  RaggedPlan p;
+  int total = 0, most = 0;
+#pragma unroll
+  for (int k = 0; k < kRaggedRows / 64; ++k) {
+    const int row = 64 * k + lane_id();
+    p.count[k] = row < B ? ragged_tiles(lens, row, T, TS, max_tiles) : 0;
+    total += p.count[k];
+    most = max(most, p.count[k]);
+  }
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    total += __shfl_xor(total, d, 64);
+    most = max(most, __shfl_xor(most, d, 64));
+  }
+  const int slots = B * (nsplit - 1);
+  const int unit = max((total + slots - 1) / slots, (most + kMaxSplits - 1) / kMaxSplits);
+  p.unit = __builtin_amdgcn_readfirstlane(unit < (most + nsplit - 1) / nsplit && unit <= kMaxPps ? unit : 0);
+#pragma unroll
+  for (int k = 0; k < kRaggedRows / 64; ++k)
+    if (64 * k + lane_id() < B)
+      p.count[k] = p.unit ? max((p.count[k] + p.unit - 1) / p.unit, 1) : nsplit;
+  return p;
+}
+
+// The row that `hit(row, splits before it, its splits)` names; row -1: none.
+template <typename Hit>
+__device__ __forceinline__ RowSplits ragged_find(const RaggedPlan& p, Hit hit) {
+  RowSplits r{-1, 0, 0};
+  int before = 0;
+#pragma unroll
+  for (int k = 0; k < kRaggedRows / 64; ++k) {
+    int sum = p.count[k];
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+      const int below = __shfl_up(sum, d, 64);
+      sum += lane_id() >= d ? below : 0;
+    }
+    const int first = before + sum - p.count[k];
+    const uint64_t at = __ballot(p.count[k] > 0 && hit(64 * k + lane_id(), first, p.count[k]));
+    if (at) {
+      const int l = __builtin_ctzll(at);
+      r.row = 64 * k + l;
+      r.first = __builtin_amdgcn_readlane(first, l);
+      r.count = __builtin_amdgcn_readlane(p.count[k], l);
+    }
+    before += __builtin_amdgcn_readlane(sum, 63);
+  }
+  return r;
 }
 
 // Pages per register stage: CHUNK_BYTES of K+V in flight per wave per stage.
@@ -187,7 +260,8 @@ constexpr int kKvLoadAux = 2;
 template <int D, int TS, bool DIRECT, int CHUNK_BYTES = 16384, int AUX = kKvLoadAux,
           int STAGES = 2, int MIN_WAVES = 0, bool LOAD_ONLY = false, bool BEAM = false,
           int KVT = LLM_F16, bool FULLPATH = true, bool WGM = false, bool OPROJ = false,
-          int RING = 0, bool STAMPS = false, bool INTERLEAVE = false, bool PRIO = false>
+          int RING = 0, bool STAMPS = false, bool INTERLEAVE = false, bool PRIO = false,
+          bool RAGGED = false>
 __global__ __launch_bounds__(WGM ? 64 * kWgmMaxSplits : 256)
 __attribute__((amdgpu_waves_per_eu(MIN_WAVES > 0 ? MIN_WAVES : 1)))
 void pa_split_kernel(PaSplitArgs a) {
@@ -213,10 +287,25 @@ void pa_split_kernel(PaSplitArgs a) {
   const int gi = wid % G;  // row within the group (fastest: adjacent waves)
   const int rest = wid / G;
   const int GH = BEAM && a.smaj ? ((a.B + 3) / 4) * a.H : 1;
-  const int s = BEAM && a.smaj ? rest / GH : rest % a.nsplit;
+  static_assert(!RAGGED || (!DIRECT && !BEAM && !WGM), "splits by need are a plain split form");
+  int s = BEAM && a.smaj ? rest / GH : rest % a.nsplit;
   const int gh = BEAM && a.smaj ? rest % GH : rest / a.nsplit;
-  const int h = gh % a.H;
-  const int b = (gh / a.H) * G + gi;
+  int h = gh % a.H;
+  int b = (gh / a.H) * G + gi;
+  int unit = 0;
+  if constexpr (RAGGED) {  // (group 1)
+    const RaggedPlan p = ragged_plan(a.context_lens, a.B, a.T, TS, a.max_tiles, a.nsplit);
+    unit = p.unit;
+    if (unit) {
+      const int slot = wid / a.H;
+      const RowSplits r = ragged_find(
+          p, [&](int, int first, int count) { return slot >= first && slot < first + count; });
+      if (r.row < 0) return;
+      b = r.row;
+      h = (wid - r.first * a.H) / r.count;
+      s = (wid - r.first * a.H) % r.count;
+    }
+  }
   // BEAM: the shared path runs only when all 4 rows exist, route to a valid
   // page-table row and hold the same context (a uniform decision: every wave
   // of the workgroup evaluates the same 4 rows, before any early return).
@@ -269,7 +358,8 @@ void pa_split_kernel(PaSplitArgs a) {
   }
   if (b >= a.B) return;
   const int bh = b * a.H + h;
-  const size_t pidx = (size_t)bh * a.nsplit + s;  // partial-state slot
+  // partial-state slot
+  const size_t pidx = RAGGED ? (size_t)wid : (size_t)bh * a.nsplit + s;
   const int r = a.beam_ids ? a.beam_ids[b] : b;
   int Tb = a.context_lens ? a.context_lens[b] : a.T;
   Tb = min(max(Tb, 0), a.T);
@@ -282,7 +372,7 @@ void pa_split_kernel(PaSplitArgs a) {
     tstride = a.nsplit;
     count = ntiles > s ? (ntiles - s + a.nsplit - 1) / a.nsplit : 0;
   } else {
-    const int pps = row_pps(a.pps, a.nsplit, ntiles);
+    const int pps = RAGGED && unit ? unit : row_pps(a.pps, a.nsplit, ntiles);
     tile0 = s * pps;
     count = min(pps, ntiles - tile0);
   }

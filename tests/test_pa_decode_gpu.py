@@ -118,6 +118,37 @@ def test_pa_decode_ragged_context_and_beams(gpu, oracle):
         np.testing.assert_array_equal(out[2], 0.0)  # empty context -> zeros
 
 
+# rows of different contexts: splits by need (one long row beside short ones, lengths at the
+# edges of a split and past T and the page table, 64 rows a register and 256 a launch), and
+# equal ones, which keep equal splits; 257 rows are dealt equally
+@pytest.mark.parametrize("B,H,D,T,ts,kind", [
+    (2, 4, 64, 3000, 16, "one"), (5, 3, 128, 2500, 16, "one"), (32, 2, 128, 4096, 16, "log"),
+    (64, 3, 64, 1500, 32, "log"), (65, 2, 64, 1500, 16, "log"), (256, 1, 128, 1200, 32, "log"),
+    (257, 1, 64, 1200, 16, "log"), (40, 2, 64, 2100, 16, "past"), (33, 2, 128, 1111, 16, "same"),
+    (7, 2, 64, 1500, 16, "none"),
+])
+def test_pa_decode_splits_by_need(gpu, oracle, B, H, D, T, ts, kind):
+    import llm_capi
+    rng = np.random.default_rng(B + T + D)
+    q, kp, vp, pt = _random_case(rng, B, H, D, T, ts, num_beams=3)
+    if kind == "past":
+        pt = pt[:, :, :-1].copy()
+    beam_ids = rng.integers(0, 3, B).astype(np.int32)
+    lens = {"one": np.full(B, 5), "log": np.exp(rng.uniform(0, np.log(T), B)), "same": np.full(B, T),
+            "past": rng.integers(0, 2 * T, B), "none": np.zeros(B)}[kind].astype(np.int32)
+    if kind in ("one", "log"):
+        lens[B // 2] = T
+        lens[0] = 0
+    ref = oracle.paged_attention(q, kp.astype(np.float32), vp.astype(np.float32), pt, T=T,
+                                 beam_ids=beam_ids, context_lens=np.minimum(lens, min(T, pt.shape[2] * ts)))
+    out = llm_capi.pa_decode(_dev(q), _dev(kp), _dev(vp), _dev(pt), T=T, beam_ids=_dev(beam_ids),
+                             context_lens=_dev(lens)).cpu().numpy()
+    if kind == "none":
+        np.testing.assert_array_equal(out, 0.0)
+    else:
+        assert_parity(out, ref, RTOL)
+
+
 def test_pa_decode_softmax_spike(gpu, oracle):
     """Force the online-softmax rescale: a key in a late page dominates."""
     import llm_capi
