@@ -13,14 +13,13 @@
 //
 // One workgroup per (row b, head h).  The whole row of scores lives in LDS
 // (T <= 8192), or, for longer rows, in the caller's workspace (the row's
-// scores and sort keys, pa_decode_ex_workspace_bytes; only its own workgroup
+// scores and the list of what stays, pa_decode_ex_workspace_bytes; only its own workgroup
 // touches them, so the barriers that order the LDS form order these too):
-// scores -> softmax -> (sort by (prob, index) descending ->
-// top-k / top-p mask) -> EOS threshold -> AV.  The sort key is
-// (prob bits << 32 | index): probabilities are >= 0, so the unsigned order of
-// the key is exactly std::greater on pair<float, int> — the order
-// apply_topk_topp_filter sorts by (attention_cpu/softmax_lut.cpp:233-256),
-// ties broken toward the larger index.
+// scores -> softmax -> (the cut of the ranking by (prob, index) descending ->
+// top-k / top-p mask) -> EOS threshold -> AV.  Probabilities are >= 0, so the
+// unsigned order of (prob bits, index) is exactly std::greater on
+// pair<float, int> — the order apply_topk_topp_filter sorts by
+// (attention_cpu/softmax_lut.cpp:233-256), ties broken toward the larger index.
 #include "common.hpp"
 #include "pa_decode.hpp"
 
@@ -47,13 +46,14 @@ struct PaFilterArgs {
   int num_pages, num_beams, max_tiles;
   size_t page_stride;  // elements from page p to page p + 1
   float temperature;
-  uint64_t* ws_key;   // [B*H][Tp] sort keys (the workspace form)
+  uint64_t* ws_key;   // [B*H][Tp] what stays (the workspace form)
   float* ws_sc;       // [B*H][Tp] scores / probabilities (the workspace form)
   int Tp;             // row stride of ws_key / ws_sc
   int top_k;
   float top_p;
   int eos;
   float eos_thr;
+  int lpt;  // lanes of a token's 16-byte pieces (a power of two); 0: rows that are no such pieces
 };
 
 template <int KVT>
@@ -66,6 +66,20 @@ __device__ __forceinline__ float kv_elem(const uint8_t* pool, size_t i) {
     return reinterpret_cast<const float*>(pool)[i];
   } else {
     return (float)reinterpret_cast<const int8_t*>(pool)[i];
+  }
+}
+
+// Element e of a 16-byte piece.
+template <int KVT>
+__device__ __forceinline__ float kv_elem(const u32x4& r, int e) {
+  if constexpr (KVT == LLM_F16) {
+    return (float)__builtin_bit_cast(f16x8, r)[e];
+  } else if constexpr (KVT == LLM_BF16) {
+    return __uint_as_float(e & 1 ? r[e >> 1] & 0xFFFF0000u : r[e >> 1] << 16);
+  } else if constexpr (KVT == LLM_F32) {
+    return __uint_as_float(r[e]);
+  } else {
+    return (float)((int32_t)(r[e >> 2] << (24 - 8 * (e & 3))) >> 24);
   }
 }
 
@@ -82,16 +96,102 @@ __device__ float block_reduce(float x, float* sh) {
   return r;
 }
 
+// The cut of the ranking by (probability, index) descending: entries at or above (bits,
+// index) stay.  Found digit by digit, 11 bits a pass, from a histogram of counts and masses
+// of the entries that agree so far.  Masses are whole numbers of 2^-44, so that their sums
+// do not depend on the order.
+constexpr int kDigitBits = 11, kDigits = 1 << kDigitBits;
+constexpr float kMassUnit = 17592186044416.f;  // 2^44
+static_assert(kDigits == 2 * kFilterThreads, "the scan gives every thread two digits");
+
+struct FilterHist {
+  uint64_t mass[kDigits];
+  uint32_t count[kDigits];
+};
+struct FilterCut {
+  uint64_t mass;         // of the entries above the digit's
+  uint32_t count, held;  // entries above the digit's, the digit's own
+  int digit;             // -1: the whole row stays
+};
+
+__device__ __forceinline__ uint64_t filter_mass(float p) { return p > 0.f ? (uint64_t)(p * kMassUnit) : 0; }
+
+// The digit, from the top, at which `need` entries (0: any number) or a mass of `limit`
+// (0: any) are reached; `from` holds what lies above the histogram.
+__device__ void filter_digit(const FilterHist& hist, uint32_t need, uint64_t limit,
+                             const FilterCut& from, FilterCut* out, uint64_t* sh_mass,
+                             uint32_t* sh_count) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int top = kDigits - 1 - 2 * tid;
+  const uint32_t c0 = hist.count[top], c1 = hist.count[top - 1];
+  const uint64_t m0 = hist.mass[top], m1 = hist.mass[top - 1];
+  uint32_t c = c0 + c1;
+  uint64_t m = m0 + m1;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t cu = __shfl_up(c, off, 64);
+    const uint64_t mu = __shfl_up((unsigned long long)m, off, 64);
+    if (lane >= off) {
+      c += cu;
+      m += mu;
+    }
+  }
+  if (lane == 63) {
+    sh_count[w] = c;
+    sh_mass[w] = m;
+  }
+  if (tid == 0) out->digit = -1;
+  __syncthreads();
+  c += from.count - c0 - c1;
+  m += from.mass - m0 - m1;
+  for (int i = 0; i < w; ++i) {
+    c += sh_count[i];
+    m += sh_mass[i];
+  }
+  const auto reached = [&](uint32_t n, uint64_t x) { return (need && n >= need) || (limit && x >= limit); };
+#pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const uint32_t n = k ? c1 : c0;
+    const uint64_t x = k ? m1 : m0;
+    if (!reached(c, m) && reached(c + n, m + x)) {
+      out->digit = top - k;
+      out->count = c;
+      out->mass = m;
+      out->held = n;
+    }
+    c += n;
+    m += x;
+  }
+  __syncthreads();
+}
+
+// One workgroup per (row, head).  The scores take one pass over K: 16-byte pieces, a
+// token's pieces in adjacent lanes, kScoreTokens tokens of a group in flight.  The entries
+// that stay are listed in the order of their index, and only their V rows are read, by all
+// lanes.  16 rows x 12 heads of 64, 2048 tokens, top 64: 70 us with a token a thread, a
+// sort of the row and a walk over all of it for the values, now 31.  Bound by the
+// latency of its steps; the 192 workgroups are one a CU.
+constexpr int kScoreTokens = 8, kValueTokens = 4;
+
 template <int KVT, bool WS>
 __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs a) {
+  constexpr int ES = KVT == LLM_F32 ? 4 : KVT == LLM_I8 ? 1 : 2;
+  constexpr int EPL = 16 / ES;
+  constexpr int kWaves = kFilterThreads / 64;
+  // scores, then probabilities; the sums of the values at the end
+  __shared__ float lsc[WS ? kWaves * 256 : kFilterMaxT];
+  // the histograms, then the list of what stays
+  __shared__ uint64_t llist[WS ? sizeof(FilterHist) / 8 : kFilterMaxT];
   __shared__ float qs[256];
-  __shared__ float lsc[WS ? 1 : kFilterMaxT];  // scores, then probabilities
-  __shared__ uint64_t lkey[WS ? kFilterThreads / 2 : kFilterMaxT];  // WS: the AV reduction only
-  __shared__ float sh[kFilterThreads / 64];
-  const int tid = threadIdx.x;
+  __shared__ float sh[kWaves];
+  __shared__ uint64_t sh_mass[kWaves];
+  __shared__ uint32_t sh_count[kWaves];
+  __shared__ FilterCut found;
+  static_assert(sizeof(FilterHist) <= sizeof(llist), "the histograms lie in the list's memory");
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.x;
   float* sc = WS ? a.ws_sc + (size_t)bh * a.Tp : lsc;
-  uint64_t* key = WS ? a.ws_key + (size_t)bh * a.Tp : lkey;
+  uint64_t* list = WS ? a.ws_key + (size_t)bh * a.Tp : llist;
   const int b = bh / a.H, h = bh % a.H;
   const int D = a.D;
   const int r = a.beam_ids ? a.beam_ids[b] : b;
@@ -105,21 +205,63 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
     const int p = table[tile];
     return (p < 0 || p >= a.num_pages) ? -1 : p;
   };
+  // element of (page, token in it)
+  auto at = [&](int page, int t) { return (size_t)page * a.page_stride + (size_t)(t % a.TS) * D; };
   for (int d = tid; d < D; d += kFilterThreads) qs[d] = a.q[(size_t)bh * D + d];
   __syncthreads();
+  // lanes per token, tokens of a wave at a time
+  const int lpt = a.lpt, tpw = lpt ? 64 / lpt : 0, c = lpt ? lane % lpt : 0, g = lpt ? lane / lpt : 0;
 
   // scores[t] = dot(q, k_t) / temperature; -1e9 where the tile is missing
   // (cpu_attention_kernel.cpp:61,68-86)
-  for (int t = tid; t < Tb; t += kFilterThreads) {
-    const int p = page_of(t);
-    float s = -1e9f;
-    if (p >= 0) {
-      const size_t base = (size_t)p * a.page_stride + (size_t)(t % a.TS) * D;
-      float dot = 0.f;
-      for (int d = 0; d < D; ++d) dot += qs[d] * kv_elem<KVT>(a.k_pool, base + d);
-      s = dot / a.temperature;
+  if (lpt) {
+    float qv[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) qv[e] = qs[c * EPL + e];
+    const int step = kScoreTokens * tpw;
+    int page[kScoreTokens];
+    auto pages = [&](int t0) {
+#pragma unroll
+      for (int u = 0; u < kScoreTokens; ++u) {
+        const int t = t0 + u * tpw + g;
+        page[u] = t < Tb ? page_of(t) : -1;
+      }
+    };
+    pages(w * step);
+    for (int t0 = w * step; t0 < Tb; t0 += kWaves * step) {
+      u32x4 k[kScoreTokens];
+      bool there[kScoreTokens];
+#pragma unroll
+      for (int u = 0; u < kScoreTokens; ++u) {
+        const int t = t0 + u * tpw + g;
+        there[u] = page[u] >= 0;
+        k[u] = u32x4{0u, 0u, 0u, 0u};
+        if (there[u])
+          k[u] = *reinterpret_cast<const u32x4*>(a.k_pool + at(page[u], t) * ES + c * 16);
+      }
+      pages(t0 + kWaves * step);
+#pragma unroll
+      for (int u = 0; u < kScoreTokens; ++u) {
+        float dot = 0.f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) dot = fmaf(qv[e], kv_elem<KVT>(k[u], e), dot);
+        for (int off = lpt >> 1; off; off >>= 1) dot += __shfl_xor(dot, off, 64);
+        const int t = t0 + u * tpw + g;
+        if (c == 0 && t < Tb) sc[t] = there[u] ? dot / a.temperature : -1e9f;
+      }
     }
-    sc[t] = s;
+  } else {
+    for (int t = tid; t < Tb; t += kFilterThreads) {
+      const int p = page_of(t);
+      float s = -1e9f;
+      if (p >= 0) {
+        const size_t base = at(p, t);
+        float dot = 0.f;
+        for (int d = 0; d < D; ++d) dot += qs[d] * kv_elem<KVT>(a.k_pool, base + d);
+        s = dot / a.temperature;
+      }
+      sc[t] = s;
+    }
   }
   __syncthreads();
   if (a.scores_out)
@@ -139,94 +281,151 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   sum = block_reduce<false>(sum, sh);
   const float inv = 1.0f / (sum + 1e-6f);
   for (int t = tid; t < Tb; t += kFilterThreads) sc[t] = sc[t] * inv;
-  __syncthreads();
 
   // apply_topk_topp_filter (softmax_lut.cpp:233-256): rank by (prob, index)
   // descending; zero rank >= top_k and every entry whose preceding mass
   // (cum of the higher-ranked probabilities) is >= top_p; no renormalisation.
+  uint32_t cut_bits = 0;
+  int cut_index = 0;
   if ((a.top_k > 0 || a.top_p < 1.0f) && Tb > 0) {
-    int Tp = 1;
-    while (Tp < Tb) Tp <<= 1;
-    for (int i = tid; i < Tp; i += kFilterThreads)
-      key[i] = i < Tb ? ((uint64_t)__float_as_uint(sc[i]) << 32) | (uint32_t)i : 0ull;
-    __syncthreads();
-    for (int k = 2; k <= Tp; k <<= 1)
-      for (int j = k >> 1; j > 0; j >>= 1) {
-        for (int i = tid; i < Tp; i += kFilterThreads) {
-          const int ixj = i ^ j;
-          if (ixj > i) {
-            const uint64_t x = key[i], y = key[ixj];
-            const bool desc = (i & k) == 0;
-            if (desc ? x < y : x > y) {
-              key[i] = y;
-              key[ixj] = x;
-            }
-          }
-        }
-        __syncthreads();
+    FilterHist& hist = *reinterpret_cast<FilterHist*>(llist);
+    const uint32_t k = a.top_k > 0 ? (uint32_t)a.top_k : 0u;
+    const uint64_t limit = a.top_p < 1.0f ? max((uint64_t)ceilf(a.top_p * kMassUnit), (uint64_t)1) : 0;
+    // digit `level` (0: the highest) of the bits, then of the index
+    const auto histogram = [&](auto digit_of) {
+      for (int i = tid; i < kDigits; i += kFilterThreads) {
+        hist.mass[i] = 0;
+        hist.count[i] = 0;
       }
-    // exclusive prefix of the sorted probabilities: each thread owns E
-    // consecutive ranks, then a block scan of the per-thread totals
-    const int E = (Tp + kFilterThreads - 1) / kFilterThreads;
-    const int i0 = tid * E;
-    float part = 0.f;
-    for (int e = 0; e < E; ++e)
-      if (i0 + e < Tb) part += __uint_as_float((uint32_t)(key[i0 + e] >> 32));
-    float incl = part;
-    const int lane = tid & 63, w = tid >> 6;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float y = __shfl_up(incl, off, 64);
-      if (lane >= off) incl += y;
+      __syncthreads();
+      for (int t = tid; t < Tb; t += kFilterThreads) {
+        const float p = sc[t];
+        const int d = digit_of(__float_as_uint(p), (uint32_t)t);
+        if (d < 0) continue;
+        atomicAdd(&hist.count[d], 1u);
+        atomicAdd(reinterpret_cast<unsigned long long*>(&hist.mass[d]),
+                  (unsigned long long)filter_mass(p));
+      }
+      __syncthreads();
+    };
+    FilterCut cut{0, 0, 0, 0};
+    bool all = false;
+    // three digits of the bits: 11, 11 and 10 of them
+    for (int level = 0; level < 3 && !all; ++level) {
+      const int shift = level == 0 ? 21 : level == 1 ? 10 : 0;
+      const uint32_t mask = level == 2 ? 1023u : 2047u;
+      const uint32_t above = level == 0 ? 0u : ~0u << (shift + (level == 2 ? 10 : 11));
+      histogram([&](uint32_t bits, uint32_t) {
+        return (bits & above) == cut_bits ? (int)(bits >> shift & mask) : -1;
+      });
+      filter_digit(hist, k, limit, cut, &found, sh_mass, sh_count);
+      all = found.digit < 0;
+      if (!all) {
+        cut = found;
+        cut_bits |= (uint32_t)cut.digit << shift;
+      }
+      __syncthreads();
     }
-    __syncthreads();
-    if (lane == 63) sh[w] = incl;
-    __syncthreads();
-    float before = incl - part;
-    for (int i = 0; i < w; ++i) before += sh[i];
-    float cum = before;
-    for (int e = 0; e < E; ++e) {
-      const int i = i0 + e;
-      if (i >= Tb) break;
-      const uint64_t kv = key[i];
-      if ((a.top_k > 0 && i >= a.top_k) || (a.top_p < 1.0f && cum >= a.top_p))
-        sc[(uint32_t)kv] = 0.f;
-      cum += __uint_as_float((uint32_t)(kv >> 32));
+    if (all) {
+      cut_bits = 0;
+    } else {
+      // of the equal ones at the cut the first `keep` stay, those of the largest index
+      const uint64_t each = filter_mass(__uint_as_float(cut_bits));
+      uint64_t keep = cut.held;
+      if (k) keep = min(keep, (uint64_t)(k - cut.count));
+      if (limit && each) keep = min(keep, (limit - cut.mass + each - 1) / each);
+      if (keep < cut.held) {
+        FilterCut from{0, 0, 0, 0};
+        uint32_t index = 0;
+        for (int level = 0; level < 3; ++level) {
+          const int shift = 22 - 11 * level;
+          const uint32_t above = level == 0 ? 0u : ~0u << (shift + 11);
+          histogram([&](uint32_t bits, uint32_t t) {
+            return bits == cut_bits && (t & above) == index ? (int)(t >> shift & 2047u) : -1;
+          });
+          filter_digit(hist, (uint32_t)keep, 0, from, &found, sh_mass, sh_count);
+          from = found;
+          index |= (uint32_t)from.digit << shift;
+          __syncthreads();
+        }
+        cut_index = (int)index;
+      }
     }
-    __syncthreads();
   }
+  __syncthreads();
+  const auto stays = [&](int t) -> float {
+    const float p = sc[t];
+    const uint32_t bits = __float_as_uint(p);
+    return bits > cut_bits || (bits == cut_bits && t >= cut_index) ? p : 0.f;
+  };
   // EOS hard threshold: keep only the EOS position when its weight exceeds it
-  if (a.eos >= 0 && a.eos < Tb && sc[a.eos] > a.eos_thr) {
-    const int eos = a.eos;
+  const bool only = a.eos >= 0 && a.eos < Tb && stays(a.eos) > a.eos_thr;
+  int n = 0;  // entries listed
+  for (int t0 = 0; t0 < a.T; t0 += kFilterThreads) {
+    const int t = t0 + tid;
+    const float p = t < Tb && !(only && t != a.eos) ? stays(t) : 0.f;
+    if (a.probs_out && t < a.T) a.probs_out[(size_t)bh * a.T + t] = p;
+    if (t0 >= Tb) continue;
+    const uint64_t kept = __ballot(p != 0.f);
+    if (lane == 0) sh_count[w] = (uint32_t)__popcll(kept);
     __syncthreads();
-    for (int t = tid; t < Tb; t += kFilterThreads)
-      if (t != eos) sc[t] = 0.f;
+    int before = n;
+    for (int i = 0; i < kWaves; ++i) {
+      before += i < w ? (int)sh_count[i] : 0;
+      n += (int)sh_count[i];
+    }
+    if (p != 0.f)
+      list[before + __popcll(kept & ((1ull << lane) - 1))] =
+          (uint64_t)__float_as_uint(p) << 32 | (uint32_t)t;
     __syncthreads();
   }
-  if (a.probs_out)
-    for (int t = tid; t < a.T; t += kFilterThreads)
-      a.probs_out[(size_t)bh * a.T + t] = t < Tb ? sc[t] : 0.f;
 
-  // out = sum_t p_t v_t over present tiles (cpu_attention_kernel.cpp:103-117):
-  // thread -> (dim d, token group g), groups summed in order at the end
-  const int G = kFilterThreads / D;
-  const int d = tid % D, g = tid / D;
-  float acc = 0.f;
-  if (g < G)
-    for (int t = g; t < Tb; t += G) {
-      const float p = sc[t];
-      if (p == 0.f) continue;
-      const int pg = page_of(t);
-      if (pg < 0) continue;
-      acc += p * kv_elem<KVT>(a.v_pool, (size_t)pg * a.page_stride + (size_t)(t % a.TS) * D + d);
+  // out = sum_t p_t v_t over present tiles (cpu_attention_kernel.cpp:103-117)
+  if (lpt) {
+    float acc[EPL];
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+    for (int j0 = w * tpw + g; j0 < n; j0 += kValueTokens * kWaves * tpw) {
+      u32x4 v[kValueTokens];
+      float p[kValueTokens];
+#pragma unroll
+      for (int u = 0; u < kValueTokens; ++u) {
+        const int j = j0 + u * kWaves * tpw;
+        const uint64_t item = j < n ? list[j] : 0;
+        const int t = (int)(uint32_t)item, pg = j < n ? page_of(t) : -1;
+        p[u] = pg < 0 ? 0.f : __uint_as_float((uint32_t)(item >> 32));
+        v[u] = u32x4{0u, 0u, 0u, 0u};
+        if (pg >= 0) v[u] = *reinterpret_cast<const u32x4*>(a.v_pool + at(pg, t) * ES + c * 16);
+      }
+#pragma unroll
+      for (int u = 0; u < kValueTokens; ++u)
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) acc[e] = fmaf(p[u], kv_elem<KVT>(v[u], e), acc[e]);
     }
-  float* red = reinterpret_cast<float*>(lkey);
+    for (int off = lpt; off < 64; off <<= 1)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+    if (g == 0)
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) lsc[w * D + c * EPL + e] = acc[e];
+  } else {
+    // thread -> (dim d, group g of the list), groups summed in order at the end
+    const int G = kFilterThreads / D, d = tid % D, gr = tid / D;
+    float acc = 0.f;
+    if (gr < G)
+      for (int j = gr; j < n; j += G) {
+        const int t = (int)(uint32_t)list[j], pg = page_of(t);
+        if (pg < 0) continue;
+        acc += __uint_as_float((uint32_t)(list[j] >> 32)) *
+               kv_elem<KVT>(a.v_pool, at(pg, t) + d);
+      }
+    if (gr < G) lsc[gr * D + d] = acc;
+  }
   __syncthreads();
-  if (g < G) red[g * D + d] = acc;
-  __syncthreads();
+  const int groups = lpt ? kWaves : kFilterThreads / D;
   if (tid < D) {
     float o = 0.f;
-    for (int gg = 0; gg < G; ++gg) o += red[gg * D + tid];
+    for (int i = 0; i < groups; ++i) o += lsc[i * D + tid];
     a.out[(size_t)bh * D + tid] = o;
   }
 }
@@ -309,6 +508,13 @@ extern "C" int pa_decode_ex(const pa_kv_view* kv, const float* q, float* out,
   a.top_p = opt->top_p;
   a.eos = opt->eos_token;
   a.eos_thr = opt->eos_threshold;
+  // rows of whole 16-byte pieces, at most a wave's lanes of them, where the pools allow
+  // 16-byte loads; other rows are read element by element
+  const int row_bytes = D * kv_elem_size(kv->kv_dtype), pieces = row_bytes / 16;
+  const bool whole = row_bytes % 16 == 0 && pieces <= 64 && (pieces & (pieces - 1)) == 0;
+  const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  a.lpt = whole && kv_view_page_stride(*kv) % 16 == 0 && aligned(kv->k_pool) && aligned(kv->v_pool)
+              ? pieces : 0;
   hipStream_t st = as_stream(stream);
   const dim3 grid(B * H), block(kFilterThreads);
 #define LLM_FILTER_LAUNCH(KVT)                                                  \

@@ -444,6 +444,46 @@ def test_pa_decode_ex_long_rows_vs_oracle(gpu, oracle, kv_dtype, top_k, top_p, e
     _check_scores(scores, rs)
 
 
+# rows read in 16-byte pieces (1, 2, 8 and 64 lanes a token) and element by element (6 pieces,
+# pages of 5 tokens), lengths around a round of tokens and the LDS form's last; spread: equal
+# weights, where the largest indices stay, and weights that all differ
+@pytest.mark.parametrize("kv_dtype,D,ts,T", [
+    ("float16", 8, 16, 1025), ("int8", 32, 16, 300), ("float16", 64, 16, 1024), ("float32", 256, 16, 511),
+    ("float16", 48, 16, 700), ("bfloat16", 64, 5, 1023), ("float16", 64, 16, 8192),
+    ("float16", 64, 16, 8193), ("float16", 64, 16, 1),
+])
+@pytest.mark.parametrize("spread", [0.0, 1.0])
+@pytest.mark.parametrize("top_k,top_p", [(5, 1.0), (0, 0.3), (400, 0.95)])
+def test_pa_decode_ex_cuts(gpu, oracle, kv_dtype, D, ts, T, spread, top_k, top_p):
+    import torch
+    import llm_capi
+    dt = getattr(torch, kv_dtype)
+    rng = np.random.default_rng(T + D)
+    B, H, nt = 2, 2, (T + ts - 1) // ts
+    q = (rng.standard_normal((B, H, D)) * spread * (0.1 if dt == torch.int8 else D ** -0.5)).astype(np.float32)
+    kd, kf = _kv_elems(rng, dt, (B * H * nt + 1, ts, D), 1.0)
+    vd, vf = _kv_elems(rng, dt, (B * H * nt + 1, ts, D), 1.0)
+    pt = rng.permutation(B * H * nt).astype(np.int32).reshape(B, H, nt)
+    lens = np.array([T, max(T - 3, 1)], np.int32)
+    ref, rp, _ = oracle.paged_attention(q, kf, vf, pt, T=T, context_lens=lens, top_k=top_k,
+                                        top_p=top_p, want_probs=True)
+    out, probs, _ = llm_capi.pa_decode_ex(_dev(q), kd, vd, _dev(pt), T=T, context_lens=_dev(lens),
+                                          top_k=top_k, top_p=top_p, want_probs=True)
+    out, probs = out.cpu().numpy(), probs.cpu().numpy()
+    kept, want = probs > 0, rp > 0
+    if top_p < 1.0:
+        # the mass above an entry decides: within fp32 rounding of a sum of T weights one
+        # entry, the last, may fall on either side
+        assert (kept != want).sum(-1).max() <= 1
+        same, both = (kept == want).all(-1), kept & want
+        out, ref, probs, rp = out[same], ref[same], probs * both, rp * both
+    else:
+        np.testing.assert_array_equal(kept, want)
+    if out.size:
+        assert_parity(out, ref, RTOL)
+    assert_parity(probs, rp, RTOL)
+
+
 def test_pa_decode_ex_workspace_form_equals_lds_form(gpu):
     """The same rows (<= 8192 tokens) through the LDS form (T 8192) and the
     workspace form (T 8193, the rows' context_lens unchanged): the same
