@@ -7,16 +7,16 @@
 // are already in the sequence's pages (page-table row `row`).  Query i attends
 // to positions 0 .. p0+i.  The decode kernel computes the same thing with one
 // wave per (token, head), so each page is re-read once per query token; here a
-// workgroup of 4 waves owns 64 MT consecutive queries of one head, loads every
+// workgroup of 4 waves owns 64 consecutive queries of one head, loads every
 // 64-key stage of K and V into LDS ONCE, and each wave runs
-//   S^T[32 keys][16 MT queries] = K · Q^T     (v_mfma_f32_16x16x32_f16)
-//   O^T[D][16 MT queries]     += V^T · P^T
+//   S^T[32 keys][16 queries] = K · Q^T     (v_mfma_f32_16x16x32_f16)
+//   O^T[D][16 queries]     += V^T · P^T
 // with the flash online softmax (log2 units, as pa_split_kernel) in between.
 //
 // A stage goes from memory straight into LDS, one stage ahead, a wave loading
 // 16 keys, with their page looked up two stages ahead: the dependent loads
 // (page, keys) and a register pass per 32 keys were what bounded the first form
-// (2048 queries x 16 heads x 128, two key splits: 137 us, now 52 us).  The
+// (2048 queries x 16 heads x 128: 137 us, now 58 us).  The
 // 16-byte chunks of a row are exchanged by the key so that the 16 rows of a
 // fragment lie in different banks.  Now bound by the vector instructions of the
 // softmax beside the matrix cores, at two workgroups per CU.
@@ -71,6 +71,7 @@ struct PaPrefillArgs {
 
 constexpr int kStageKeys = 64;
 constexpr int kWaves = 4;
+constexpr int kTileQueries = 16 * kWaves;  // of a workgroup
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
 constexpr float kPShift = 14.f, kPScale = 16384.f;  // P enters the PV MFMA as p * 2^14 (hi + lo)
@@ -80,14 +81,14 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
   lo = (_Float16)(x - (float)hi);
 }
 
-template <int D, int TS, int MT>
+template <int D, int TS>
 __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArgs a) {
   constexpr int ROWB = 2 * D;                // bytes of a key's row
   constexpr int CPR = D / 8;                 // its 16-byte chunks
   constexpr int LOADS = 16 * ROWB / 1024;    // 1 KiB loads of a wave's 16 keys, each of K and V
   constexpr int NKK = D / 32;                // k-steps of q.k
   constexpr int ND = D / 16;                 // 16-dim tiles of the output
-  constexpr int QW = 16 * MT, QT = QW * kWaves;  // queries of a wave, of the workgroup
+  constexpr int QW = 16, QT = kTileQueries;  // queries of a wave, of the workgroup
   static_assert(D % 32 == 0 && TS % 16 == 0 && kStageKeys == 16 * kWaves, "shape");
   __shared__ u32x4 lds[2][2][kStageKeys * CPR];  // [stage][K, V][key][chunk, exchanged]
 
@@ -148,11 +149,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
   // qscale), hi + lo.  The query's values are also scaled by a power of two
   // 2^(14-e) (|q|max < 2^e) so the lo halves stay clear of fp16 subnormals,
   // which the MFMA does not keep; S is scaled back exactly after the MFMA.
-  f16x8 qh[MT][NKK], ql[MT][NKK];
-  float qinv[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int qi = q0 + 16 * t + c;
+  f16x8 qh[NKK], ql[NKK];
+  float qinv;
+  {
+    const int qi = q0 + c;
     float qx[NKK][8];
     float amax = 0.f;
 #pragma unroll
@@ -176,27 +176,22 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
     (void)frexpf(amax, &qe);  // amax < 2^qe (0 for amax == 0)
     qe = min(max(qe, -100), 100);
     const float qsc = ldexpf(1.f, 14 - qe);
-    qinv[t] = ldexpf(1.f, qe - 14);
+    qinv = ldexpf(1.f, qe - 14);
 #pragma unroll
     for (int kk = 0; kk < NKK; ++kk)
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         _Float16 hi, lo;
         split_f16(qx[kk][e] * qsc, hi, lo);
-        qh[t][kk][e] = hi;
-        ql[t][kk][e] = lo;
+        qh[kk][e] = hi;
+        ql[kk][e] = lo;
       }
   }
 
-  f32x4 O[ND][MT];
-  float nrun[MT], lrun[MT];
+  f32x4 O[ND];
+  float nrun = kNegSentinel, lrun = 0.f;
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    nrun[t] = kNegSentinel;
-    lrun[t] = 0.f;
-#pragma unroll
-    for (int nd = 0; nd < ND; ++nd) O[nd][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
+  for (int nd = 0; nd < ND; ++nd) O[nd] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   int buf = 0;
   for (int s = s0; s < s1; ++s, buf ^= 1) {
@@ -211,76 +206,62 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
       if (key0 > wave_last) break;
       const unsigned here = valid >> (2 * kb) & 3u;  // of the block's two 16-key tiles
       // S^T: two 16-key tiles
-      f32x4 sc[MT][2];
+      f32x4 sc[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-#pragma unroll
-        for (int t = 0; t < MT; ++t) sc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        sc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
         const u32x4* krow = &lds[buf][0][(32 * kb + 16 * u + c) * CPR];
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
           const f16x8 kf = __builtin_bit_cast(f16x8, krow[exchange(c, 4 * kk + g)]);
-#pragma unroll
-          for (int t = 0; t < MT; ++t) {
-            sc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[t][kk], sc[t][u], 0, 0, 0);
-            sc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[t][kk], sc[t][u], 0, 0, 0);
-          }
+          sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, qh[kk], sc[u], 0, 0, 0);
+          sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[kk], sc[u], 0, 0, 0);
         }
       }
       // The products are read before the branch on `mask`: the compiler leaves out the
       // wait for a matrix instruction whose result is first read behind one.
-      float mloc[MT];
+      float mloc = -INFINITY;
 #pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        mloc[t] = -INFINITY;
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) mloc[t] = fmaxf(mloc[t], sc[t][u][r]);
-        asm volatile("" : "+v"(mloc[t]));
-      }
+        for (int r = 0; r < 4; ++r) mloc = fmaxf(mloc, sc[u][r]);
+      asm volatile("" : "+v"(mloc));
       // causal + missing-page mask
       if (key0 + 31 > wave_first || here != 3u) {
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          mloc[t] = -INFINITY;
-#pragma unroll
-          for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-              if (!(here >> u & 1u) || key0 + 16 * u + 4 * g + r > wave_first + 16 * t + c)
-                sc[t][u][r] = -INFINITY;
-              mloc[t] = fmaxf(mloc[t], sc[t][u][r]);
-            }
-        }
-      }
-      // online softmax (per query = per lane): p = 2^(s - n), n the running maximum
-      // less 14, so that p comes out scaled for the halves; s is scaled back in the same
-      // operation
-      f16x8 ph[MT], pl[MT];
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const float nloc = rows_max(mloc[t]) * qinv[t] - kPShift;
-        if (__any(nloc > nrun[t])) {
-          const float nnew = fmaxf(nrun[t], nloc);
-          const float corr = __builtin_amdgcn_exp2f(nrun[t] - nnew);
-          lrun[t] *= corr;
-#pragma unroll
-          for (int nd = 0; nd < ND; ++nd) O[nd][t] *= corr;
-          nrun[t] = nnew;
-        }
+        mloc = -INFINITY;
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            const float p = __builtin_amdgcn_exp2f(fmaf(sc[t][u][r], qinv[t], -nrun[t]));
-            lrun[t] += p;
-            _Float16 hi, lo;
-            split_f16(p, hi, lo);  // p <= 2^14: clear of fp16 subnormals
-            ph[t][4 * u + r] = hi;
-            pl[t][4 * u + r] = lo;
+            if (!(here >> u & 1u) || key0 + 16 * u + 4 * g + r > wave_first + c)
+              sc[u][r] = -INFINITY;
+            mloc = fmaxf(mloc, sc[u][r]);
           }
       }
+      // online softmax (per query = per lane): p = 2^(s - n), n the running maximum
+      // less 14, so that p comes out scaled for the halves; s is scaled back in the same
+      // operation
+      f16x8 ph, pl;
+      const float nloc = rows_max(mloc) * qinv - kPShift;
+      if (__any(nloc > nrun)) {
+        const float nnew = fmaxf(nrun, nloc);
+        const float corr = __builtin_amdgcn_exp2f(nrun - nnew);
+        lrun *= corr;
+#pragma unroll
+        for (int nd = 0; nd < ND; ++nd) O[nd] *= corr;
+        nrun = nnew;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[u][r], qinv, -nrun));
+          lrun += p;
+          _Float16 hi, lo;
+          split_f16(p, hi, lo);  // p <= 2^14: clear of fp16 subnormals
+          ph[4 * u + r] = hi;
+          pl[4 * u + r] = lo;
+        }
       // O^T += V^T · P^T.  A operand lane l: V^T[d = 16nd + (l&15)][k 8g+j] =
       // V[key(8g+j)][d], keys 4g..4g+3 then 16+4g..16+4g+3: two transposed
       // reads of 4 V rows x 16 columns, lane 4q+p addressing row q, columns 4p..
@@ -295,69 +276,57 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
             (__attribute__((address_space(3))) s16x4*)(at + 16 * ROWB));
         const f16x8 vf = __builtin_bit_cast(
             f16x8, s16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]});
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-          O[nd][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph[t], O[nd][t], 0, 0, 0);
-          O[nd][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[t], O[nd][t], 0, 0, 0);
-        }
+        O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, O[nd], 0, 0, 0);
+        O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, O[nd], 0, 0, 0);
       }
     }
     valid = valid_next;
   }
 
   // the 4 lanes of a query hold partial sums over their keys
+  lrun += __shfl_xor(lrun, 16, 64);
+  lrun += __shfl_xor(lrun, 32, 64);
+  lrun *= 1.0f / kPScale;
+  const int qi = q0 + c;
+  if (qi >= a.m) return;
+  if (a.part_acc) {  // split partial state (unnormalised, log2 units)
+    const size_t pidx = ((size_t)qi * a.H + h) * a.nsplit + split;
+    float* o = a.part_acc + pidx * D + 4 * g;
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    lrun[t] += __shfl_xor(lrun[t], 16, 64);
-    lrun[t] += __shfl_xor(lrun[t], 32, 64);
-    lrun[t] *= 1.0f / kPScale;
-    const int qi = q0 + 16 * t + c;
-    if (qi >= a.m) continue;
-    if (a.part_acc) {  // split partial state (unnormalised, log2 units)
-      const size_t pidx = ((size_t)qi * a.H + h) * a.nsplit + split;
-      float* o = a.part_acc + pidx * D + 4 * g;
+    for (int nd = 0; nd < ND; ++nd)
+      *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * (1.0f / kPScale);
+    if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{nrun + kPShift, lrun};
+  } else {
+    const float inv = 1.0f / (lrun + 1e-6f) * (1.0f / kPScale);
+    float* o = a.out + (size_t)qi * a.out_stride + h * D + 4 * g;
 #pragma unroll
-      for (int nd = 0; nd < ND; ++nd)
-        *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd][t] * (1.0f / kPScale);
-      if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{nrun[t] + kPShift, lrun[t]};
-    } else {
-      const float inv = 1.0f / (lrun[t] + 1e-6f) * (1.0f / kPScale);
-      float* o = a.out + (size_t)qi * a.out_stride + h * D + 4 * g;
-#pragma unroll
-      for (int nd = 0; nd < ND; ++nd) *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd][t] * inv;
-    }
+    for (int nd = 0; nd < ND; ++nd) *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * inv;
   }
 }
 
 template <int D, int TS>
-hipError_t launch_prefill(const PaPrefillArgs& a, int mt, hipStream_t st) {
-  const int qt = 16 * mt * kWaves;
-  const dim3 grid(a.H, (a.m + qt - 1) / qt, a.nsplit);
-  if (mt == 2)
-    hipLaunchKernelGGL((pa_prefill_kernel<D, TS, 2>), grid, dim3(64 * kWaves), 0, st, a);
-  else
-    hipLaunchKernelGGL((pa_prefill_kernel<D, TS, 1>), grid, dim3(64 * kWaves), 0, st, a);
+hipError_t launch_prefill(const PaPrefillArgs& a, hipStream_t st) {
+  const dim3 grid(a.H, (a.m + kTileQueries - 1) / kTileQueries, a.nsplit);
+  hipLaunchKernelGGL((pa_prefill_kernel<D, TS>), grid, dim3(64 * kWaves), 0, st, a);
   return hipGetLastError();
 }
 
-// Launch geometry: 32 queries per wave, 16 where the chunk has few.  The key range is
-// cut into splits of `per` stages, the length for which the rounds of workgroups (2 per
-// CU) times their length is least, a split more counted as half a stage for its merge;
-// no more than split_bound of them a query (2048 queries x 16 heads: 11 stages, 512
-// workgroups in one round).
+// The key range is cut into splits of `per` stages, the length for which the rounds of
+// workgroups (2 per CU) times their length is least, a split more counted as half a stage
+// for its merge; no more than split_bound of them a query.  32 queries a wave in place of
+// 16 (16 heads of 128, with the merge): 2048 queries 72 -> 70 us, but those after 2048 more
+// 120 -> 139, 1024 34 -> 36, 117 11 -> 14; heads of 64 2048 48 -> 60.
 constexpr int kRound = 512;
 struct PrefillPlan {
-  int mt, nsplit, pps;
+  int nsplit, pps;
 };
-int queries_per_wg(int m) { return m > 64 ? 128 : 64; }
 int split_bound(int H, int m) {
-  const int nq = (m + queries_per_wg(m) - 1) / queries_per_wg(m);
+  const int nq = (m + kTileQueries - 1) / kTileQueries;
   return std::min(2 * kRound / std::max(nq * H, 1) + 1, 128);
 }
 PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   PrefillPlan p;
-  const int qt = queries_per_wg(m), H = kv->num_heads;
-  p.mt = qt / 64;
+  const int H = kv->num_heads;
   const int most = (p0 + m - 1) / kStageKeys + 1;
   const int bound = split_bound(H, m);
   int best = most;
@@ -365,8 +334,8 @@ PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   for (int n = 1; n <= std::min(bound, most); ++n) {
     const int per = (most + n - 1) / n;
     long long wgs = 0;
-    for (int q = 0; q < m; q += qt)
-      wgs += ((p0 + std::min(q + qt, m) - 1) / kStageKeys + per) / per;
+    for (int q = 0; q < m; q += kTileQueries)
+      wgs += ((p0 + std::min(q + kTileQueries, m) - 1) / kStageKeys + per) / per;
     const double cost = (double)((wgs * H + kRound - 1) / kRound) * per + 0.5 * (most + per - 1) / per;
     if (cost < least) {
       least = cost;
@@ -450,9 +419,9 @@ int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, floa
   hipError_t e;
   const int TS = kv->page_size;
   if (D == 64)
-    e = TS == 16 ? launch_prefill<64, 16>(a, pl.mt, st) : launch_prefill<64, 32>(a, pl.mt, st);
+    e = TS == 16 ? launch_prefill<64, 16>(a, st) : launch_prefill<64, 32>(a, st);
   else
-    e = TS == 16 ? launch_prefill<128, 16>(a, pl.mt, st) : launch_prefill<128, 32>(a, pl.mt, st);
+    e = TS == 16 ? launch_prefill<128, 16>(a, st) : launch_prefill<128, 32>(a, st);
   if (e != hipSuccess) return fail(LLM_ERR_HIP, std::string("pa_prefill launch: ") + hipGetErrorString(e));
   if (split)
     return pa_merge_rows_internal(a.part_acc, a.part_ml, (rows && !rows->keep_out) ? nullptr : out,

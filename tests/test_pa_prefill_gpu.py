@@ -91,12 +91,12 @@ def test_pa_prefill_vs_oracle(gpu, oracle, H, D, ts, p0, m, row, split):
 
 @pytest.mark.parametrize("D,ts", [(64, 16), (64, 32), (128, 16), (128, 32)])
 @pytest.mark.parametrize("p0,m", [
-    (0, 63), (0, 64), (0, 65),      # 16 or 32 queries a wave
+    (0, 63), (0, 64), (0, 65),      # a full tile, one query less and one more
     (0, 129), (95, 128),            # one query past a tile; a tile that ends inside a stage
     (1, 127), (448, 65), (449, 256),  # stages of 64 keys: first and last full or one key long
 ])
 def test_pa_prefill_tile_edges(gpu, oracle, D, ts, p0, m):
-    """Query tiles of 64 and 128, key stages of 64, pages missing inside a stage, keys past
+    """Query tiles and key stages of 64, pages missing inside a stage, keys past
     the context never written; cut into pieces and in one pass."""
     import llm_capi
     rng = np.random.default_rng(p0 + 3 * m + D + ts)
