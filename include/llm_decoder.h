@@ -422,7 +422,7 @@ int llm_decoder_generate(llm_decoder* d, const int32_t* prompts, const int32_t* 
 
 /* Chunked prefill (the is_prefill pass of AttentionCUDA::forward,
  * attention/attention_cuda.hpp:21): append the n tokens (host ids) of active
- * row `row` at its next positions in one layer pass per chunk of <= 512 tokens
+ * row `row` at its next positions in one layer pass per chunk of <= 2048 tokens
  * (M = chunk weight GEMMs; causal paged attention per token), then set the
  * row's next token from the last token's logits, so llm_decoder_step(tokens =
  * NULL) continues decoding.  llm_decoder_generate uses it for every prompt. */
