@@ -232,14 +232,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   // zero: all stay).  top-p: the largest pattern whose probabilities and those above
   // hold a mass of top_p; whatever lies below has at least that much ranked above it.
   // What top-k drops cannot change that: where the mass that it leaves is less than
-  // top_p, top-p drops nothing more.
+  // top_p, top-p drops nothing more.  A top_p below the masses' unit wants one of it: the
+  // most probable alone have nothing ranked above them.
   uint32_t least = 0;
   if (a.top_k > 0 && a.top_k < a.V)
     least = find_pattern<NS>(v, 0u, (uint32_t)a.top_k, ranks, rank_part, &rank_found,
                              [](uint32_t) { return 1u; });
   if (a.top_p < 1.0f)
-    least = max(least, find_pattern<NS>(v, least, mass_of(__float_as_uint(a.top_p)), masses, mass_part,
-                                        &mass_found, [](uint32_t bits) { return mass_of(bits); }));
+    least = max(least, find_pattern<NS>(v, least, max(mass_of(__float_as_uint(a.top_p)), 1ull), masses,
+                                        mass_part, &mass_found,
+                                        [](uint32_t bits) { return mass_of(bits); }));
 
   // kept mass in token order: per cell, then over the cells
 #pragma unroll

@@ -51,3 +51,17 @@ def test_masked_and_unusable_logits(gpu):
         got = draw(logits, 1.0, 50, 0.95, c)
         assert got[0] in (5, 8190, 8999) and got[1] == 0 and got[2] == 0 and got[3] == 4000
     assert draw(logits, 1.0, 0, 0.3, 1)[0] == 8190
+
+
+@pytest.mark.parametrize("p", [9e-16, 8e-16, 1e-16, 1e-20, 1.2e-38, 1e-42])
+@pytest.mark.parametrize("k", [0, 50])
+def test_top_p_below_any_probability(gpu, p, k):
+    """A top_p that every mass exceeds leaves the most probable token, or its ties."""
+    rng = np.random.default_rng(11)
+    logits = rng.standard_normal((6, 9000)).astype(np.float32)
+    logits[5, [3, 4100, 8999]] = logits[5].max() + 1.0
+    logits[4] = 0.25
+    for c in range(12):
+        got = draw(logits, 1.0, k, p, c)
+        assert (got[:4] == logits[:4].argmax(1)).all() and got[5] in (3, 4100, 8999)
+    assert len({int(draw(logits[4:5], 1.0, k, p, c)[0]) for c in range(40)}) > 20  # all tied
