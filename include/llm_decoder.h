@@ -145,13 +145,15 @@ int pa_decode_grouped(const pa_kv_view* kv, const float* q, float* out, const in
  * K/V are already in the pages of page-table row `row`; query i attends to
  * positions 0 .. p0+i.  Equals pa_decode with B = m, beam_ids[i] = row,
  * context_lens[i] = p0 + i + 1 (within 1e-3 relative), but each K/V page is
- * read once per 32 queries instead of once per query (MFMA tiles).
+ * read once per 64 queries instead of once per query (MFMA tiles).
  * q, out: fp32 [m][H][D] with row strides q_stride / out_stride floats
  * (<= 0: H*D), 16-byte aligned.  fp16 pools, head_dim 64 or 128, page_size
  * 16 or 32 (else LLM_ERR_UNSUPPORTED; pa_decode covers every shape).
  * With workspace_bytes >= pa_prefill_workspace_bytes(kv, p0, m) (and
  * out_stride H*D) the key range is split over more workgroups and merged as
- * pa_decode's splits; with less (or NULL) it runs in one pass. */
+ * pa_decode's splits; with less (or NULL) it runs in one pass.  That size is
+ * enough for the same m at every shorter context: a caller may ask once, at
+ * the longest. */
 size_t pa_prefill_workspace_bytes(const pa_kv_view* kv, int p0, int m);
 int pa_prefill(const pa_kv_view* kv, const float* q, int q_stride, float* out, int out_stride,
                int row, int p0, int m, float sm_scale, void* workspace, size_t workspace_bytes,

@@ -828,7 +828,8 @@ int llm_decoder::alloc_prefill(int C) {
   {  // the MFMA prefill's split partials, at any p0
     pa_kv_view v0;
     RET_IF(kv_cache_view(kv, 0, &v0));
-    for (int b = 1; b <= C; ++b) pws_bytes = std::max(pws_bytes, pa_prefill_ws_bound(&v0, b));
+    for (int b = 1; b <= std::min(C, cfg.max_seq_len); ++b)
+      pws_bytes = std::max(pws_bytes, pa_prefill_ws_bytes(&v0, cfg.max_seq_len - b, b));
   }
   RET_IF(pws.alloc(pws_bytes));
   pf_cap = C;

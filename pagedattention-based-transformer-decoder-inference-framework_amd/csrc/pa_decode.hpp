@@ -90,9 +90,8 @@ int pa_merge_splits_internal(const float* part_acc, const float* part_ml, float*
 // (the o_proj input); without, one pass writes out and `rows` is converted by
 // the row quantiser.  `out` may be NULL only when it splits and rows is set.
 bool pa_prefill_supported(const pa_kv_view* kv);
+// (pa_prefill_ws_bytes: enough for m queries at p0 and at any shorter context)
 size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m);
-// The most of it over all p0.
-size_t pa_prefill_ws_bound(const pa_kv_view* kv, int m);
 int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, float* out,
                         int out_stride, int row, int p0, int m, float sm_scale, void* workspace,
                         size_t workspace_bytes, hipStream_t st, const PaRowOutputs* rows = nullptr);

@@ -354,17 +354,15 @@ bool pa_prefill_supported(const pa_kv_view* kv) {
          (kv->page_size == 16 || kv->page_size == 32);
 }
 
+// A plan has no more splits than split_bound and its stages allow, but fewer at one p0
+// than at a shorter one (2048 queries x 16 heads: three at p0 0, one from p0 2048 on), so
+// the size is of the most that any context up to this one takes.
 size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m) {
   if (!pa_prefill_supported(kv) || m <= 0 || p0 < 0) return 0;
-  const PrefillPlan p = prefill_plan(kv, p0, m);
-  if (p.nsplit <= 1) return 0;
-  return (size_t)m * kv->num_heads * p.nsplit * (size_t)(kv->head_dim + 2) * sizeof(float);
-}
-
-size_t pa_prefill_ws_bound(const pa_kv_view* kv, int m) {
-  if (!pa_prefill_supported(kv) || m <= 0) return 0;
-  return (size_t)m * kv->num_heads * split_bound(kv->num_heads, m) * (size_t)(kv->head_dim + 2) *
-         sizeof(float);
+  const int most = (int)(((long long)p0 + m - 1) / kStageKeys) + 1;
+  const int n = std::min(split_bound(kv->num_heads, m), most);
+  if (n <= 1) return 0;
+  return (size_t)m * kv->num_heads * n * (size_t)(kv->head_dim + 2) * sizeof(float);
 }
 
 int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, float* out,
@@ -387,7 +385,7 @@ int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, floa
               "pa_prefill: q and out must be 16-byte aligned");
   const bool row_out = rows && (rows->q || rows->out16);
   PrefillPlan pl = prefill_plan(kv, p0, m);
-  const size_t need = pa_prefill_ws_bytes(kv, p0, m);
+  const size_t need = (size_t)m * H * pl.nsplit * (size_t)(D + 2) * sizeof(float);
   const bool split = pl.nsplit > 1 && workspace && workspace_bytes >= need &&
                      (out == nullptr || out_stride == hid) &&
                      (!row_out || rows->pack);  // the merge writes packed o_proj inputs

@@ -154,3 +154,19 @@ def test_no_oracle_in_product_path():
     for p in list(PKG.rglob("*.py")) + list((PKG / "csrc").glob("*")) + [PKG / "Makefile"]:
         if p.is_file():
             assert not pat.search(p.read_text(errors="ignore")), p
+
+
+@pytest.mark.parametrize("H,D,ts", [(1, 64, 16), (12, 64, 16), (16, 128, 16), (16, 128, 32), (96, 128, 16)])
+def test_prefill_workspace_grows_with_the_context(H, D, ts):
+    """A workspace sized at the longest context does for all shorter ones: the split form
+    must not be lost for want of it."""
+    import llm_capi
+    lib = llm_capi.load()
+    v = llm_capi.PaKvView()
+    v.num_pages, v.page_size, v.head_dim, v.num_beams, v.num_heads, v.max_tiles = 1 << 20, ts, D, 1, H, 1 << 16
+    v.kv_dtype = llm_capi.LLM_F16
+    for m in (1, 17, 64, 65, 512, 1000, 2048, 4096):
+        sizes = [lib.pa_prefill_workspace_bytes(ctypes.byref(v), p0, m)
+                 for p0 in (0, 1, 15, 63, 64, 100, 500, 511, 1024, 2048, 4096, 10000, 65536)]
+        assert sizes == sorted(sizes), (m, sizes)
+    assert lib.pa_prefill_workspace_bytes(ctypes.byref(v), 4096, 64) > 0
