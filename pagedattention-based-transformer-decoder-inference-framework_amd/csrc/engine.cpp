@@ -70,9 +70,13 @@ struct Request {
 // takes its staging and the host's copy one after the other: 64 rows of 32,768 505 us,
 // so 157 us on the bus and 107 us of host copy beside it.  Eight pieces: a piece costs
 // 10 us of its own on the stream and 15 us to submit, most of it while the step still
-// runs, and the last one's host copy stands alone.
+// runs, and the last one's host copy stands alone.  Up to 1 MiB the runtime's way is the
+// faster one, its copy being one call (whole steps of small and large stacks: 1 row of
+// 32,768 135 and 138 us through the ring, 4 rows 175 and 181, 8 rows, 1 MiB, 316 and 327;
+// 16 rows 444 and 409).
 struct RowCopy {
   static constexpr size_t kPiece = 1 << 20, kLeast = 256 << 10;  // bytes of a piece, of a small one
+  static constexpr size_t kByRuntime = 1 << 20;  // a step's bytes that go the runtime's way
   static constexpr int kRing = 8;
   char* ring = nullptr;
   hipEvent_t arrived[kRing] = {};
@@ -113,7 +117,7 @@ struct RowCopy {
            hipStream_t st) {
     const size_t row_bytes = width * sizeof(float), total = rows.size() * row_bytes;
     if (!total) return finish(LLM_OK, st);
-    if (!ring || !pageable(host)) {
+    if (!ring || total <= kByRuntime || !pageable(host)) {
       for (size_t r = 0, n; r < rows.size(); r += n) {
         for (n = 1; r + n < rows.size() && rows[r + n] == rows[r] + n;) ++n;
         LLM_HIP_RET(hipMemcpyAsync(host + rows[r] * width, src + r * width, n * row_bytes,

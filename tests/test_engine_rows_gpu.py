@@ -1,6 +1,6 @@
-"""Logits rows of an engine step in the caller's memory: pageable memory goes through the
-engine's pinned pieces of 512 KiB, four at a time, memory that the runtime knows does not;
-both hold the same bytes."""
+"""Logits rows of an engine step in the caller's memory.  More than 1 MiB of them go to
+pageable memory through the engine's ring of eight pinned pieces (of 256 KiB to 1 MiB); less,
+and memory that the runtime knows, goes the runtime's way.  All hold the same bytes."""
 import ctypes
 
 import numpy as np
@@ -31,13 +31,7 @@ def step(eng, entries, out):
     eng._check(eng.lib.llm_engine_step(eng._h, arr, len(entries), ctypes.c_void_p(out)))
 
 
-# 26 rows of 20,012 bytes: just under one piece; 27 and 105: over one and over four; 128
-# in order, 127 in gaps, and a batch of two passes whose rows lie apart
-@pytest.mark.parametrize("lens,pick", [
-    ([1], None), ([26], None), ([27], None), ([105], None), ([128], None), ([60, 67], "odd"),
-    ([100, 90], "back"), ([3], "none"),
-])
-def test_rows_by_both_ways(eng, lens, pick):
+def check(eng, lens, pick):
     import torch
     rng = np.random.default_rng(len(lens) + lens[0])
     toks = [rng.integers(0, eng.vocab, n) for n in lens]
@@ -53,3 +47,34 @@ def test_rows_by_both_ways(eng, lens, pick):
             eng.close_seq(s)
     if rows:
         np.testing.assert_array_equal(plain, pinned.numpy())
+
+
+# rows of 20,012 bytes: one; 52 and 53: the last by the runtime and the first through the
+# ring; 105 and 128: five pieces; 127 in gaps, and a batch of two passes whose rows lie apart
+@pytest.mark.parametrize("lens,pick", [
+    ([1], None), ([26], None), ([52], None), ([53], None), ([105], None), ([128], None),
+    ([60, 67], "odd"), ([100, 90], "back"), ([3], "none"),
+])
+def test_rows_by_both_ways(eng, lens, pick):
+    check(eng, lens, pick)
+
+
+@pytest.fixture(scope="module")
+def wide(gpu, tmp_path_factory):
+    import engine
+    cfg = T.config([(T.attn(), None)], vocab=40009)
+    folder = T.save(tmp_path_factory.mktemp("wide"), cfg, T.weights(cfg, 4))
+    with engine.Engine(folder, dtype="float32", max_seqs=4, max_tokens=1024,
+                       max_step_tokens=128) as e:
+        yield e
+
+
+# rows of 160,036 bytes: 6 and 7 on both sides of 1 MiB; 52 just fill the ring's 8 MiB, 53
+# use a piece again, 105 (over 16 MiB) and 128 a piece for the third time; in gaps and back
+# to front, and 190 rows of two passes
+@pytest.mark.parametrize("lens,pick", [
+    ([6], None), ([7], None), ([52], None), ([53], None), ([105], None), ([128], None),
+    ([64, 64], "odd"), ([70, 58], "back"), ([100, 90], "back"), ([100, 90], None),
+])
+def test_pieces_used_again(wide, lens, pick):
+    check(wide, lens, pick)
