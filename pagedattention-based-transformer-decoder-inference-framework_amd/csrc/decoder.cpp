@@ -152,6 +152,7 @@ struct llm_decoder {
   DevBuf<int32_t> pmeta;  // [4][chunk]: pos, ctx, page-table row, token
   size_t pws_bytes = 0;
   int pf_cap = 0;
+  int prompt_chunk = kPromptChunk;  // kPrefillChunk once the card had no room for more
   int alloc_prefill(int C);
   int ensure_prefill(int C);
   int prefill(int row, const int32_t* toks, int n, hipStream_t st);
@@ -831,16 +832,22 @@ int llm_decoder::alloc_prefill(int C) {
     for (int b = 1; b <= std::min(C, cfg.max_seq_len); ++b)
       pws_bytes = std::max(pws_bytes, pa_prefill_ws_bytes(&v0, cfg.max_seq_len - b, b));
   }
+#if LLM_TUNING  // a card with room for that many rows
+  if (C > env_int("LLM_PREFILL_ROOM", C)) return fail(LLM_ERR_OOM, "decoder: LLM_PREFILL_ROOM");
+#endif
   RET_IF(pws.alloc(pws_bytes));
   pf_cap = C;
   return LLM_OK;
 }
 
-// A card that the cache fills has no room for the long chunk: the short one then.
+// A card that the cache fills has no room for the long chunk: the short one then, and
+// from then on, since every try frees all of these buffers and allocates them again.
 int llm_decoder::ensure_prefill(int C) {
   if (C <= pf_cap) return LLM_OK;
   const int rc = alloc_prefill(C);
-  return rc == LLM_ERR_OOM && C > kPrefillChunk ? alloc_prefill(kPrefillChunk) : rc;
+  if (rc != LLM_ERR_OOM || C <= kPrefillChunk) return rc;
+  prompt_chunk = kPrefillChunk;
+  return alloc_prefill(kPrefillChunk);
 }
 
 // Chunked prefill of `n` prompt tokens of active row `row` (the reference's
@@ -859,7 +866,7 @@ int llm_decoder::prefill(int row, const int32_t* toks, int n, hipStream_t st) {
   for (int i = 0; i < n; ++i) LLM_REQUIRE(toks[i] >= 0 && toks[i] < V, "prefill: token id out of range");
   pa_kv_view v0;
   RET_IF(kv_cache_view(kv, 0, &v0));
-  int C = std::min(n, pa_prefill_supported(&v0) ? kPromptChunk : kPrefillChunk);
+  int C = std::min(n, pa_prefill_supported(&v0) ? prompt_chunk : kPrefillChunk);
   RET_IF(ensure_prefill(C));
   C = std::min(C, pf_cap);
   KvCache* k = kv_impl(kv);

@@ -590,10 +590,10 @@ def _prefill_vs_stepping(make, prompts, V):
 
 
 def test_prefill_matches_token_by_token(gpu, oracle):
-    """Chunked prefill (one layer pass per <= 512-token chunk, causal attention
-    on the MFMA prefill kernel) leaves the same KV and state as feeding the
-    prompt one token per decode step; prompts of 600 (two chunks) and 37
-    tokens, ragged.  The prefill kernel's attention agrees with the decode
+    """Prefill (one layer pass per <= 2048-token chunk, causal attention on the
+    MFMA prefill kernel) leaves the same KV and state as feeding the prompt one
+    token per decode step; prompts of 600 and 37 tokens, ragged, a pass each
+    (more than one: test_prefill_later_passes).  The prefill kernel's attention agrees with the decode
     kernel to ~1e-6 (tests/test_pa_prefill_gpu.py); through the int8
     activations that is the free-running bar of this file (FREE_RUN_TOL)."""
     w = _int8_model(oracle, L=2, H=4, D=64, V=500, S=1024, seed=12)
@@ -607,6 +607,66 @@ def test_prefill_matches_token_by_token(gpu, oracle):
     for r in range(2):
         assert errs[r] < FREE_RUN_TOL, (r, errs[r])
         assert gaps[r] <= FREE_RUN_TOL, (r, gaps[r])
+
+
+@pytest.fixture(scope="module")
+def long_prompts(gpu, oracle):
+    """kind -> (decoders, a prompt of 2160 tokens, logits after stepping it token by
+    token, by tokens taken in)"""
+    torch = _torch()
+    import llm_decoder
+    rng = np.random.default_rng(21)
+    L, H, D, V, S = 2, 4, 64, 500, 2304
+    prompt = rng.integers(0, V, 2160).tolist()
+    w = _int8_model(oracle, L=L, H=H, D=D, V=V, S=S, seed=21)
+    wf = _f16_model(rng, L, H, D, V, S)
+    f = {k: np.ascontiguousarray(v) for k, v in wf.items() if k != "cfg"}
+    for k in ("emb", "wqkv", "wo", "w1", "w2"):
+        f[k] = f[k].view(np.uint16)
+
+    def f16(n):
+        dec = llm_decoder.CUDADecoder(L, H, D, H * D, V, S, max_batch=n)
+        dec.set_weights(f)
+        return dec
+
+    out = {}
+    for kind, make in (("int8", lambda n: _make_gpu_decoder(w, max_batch=n)), ("f16", f16)):
+        a, logits, seen = make(1), torch.empty((1, V), device="cuda"), {}
+        a.begin_synthetic(1, 0, 0, False)
+        for i, t in enumerate(prompt):
+            a.step([t], logits_ptr=logits.data_ptr())
+            if i + 1 in (2050, 2101, 2149, 2150):
+                torch.cuda.synchronize()
+                seen[i + 1] = logits[0].cpu().numpy().copy()
+        out[kind] = make, prompt, seen
+    return out
+
+
+@pytest.mark.parametrize("kind", ["int8", "f16"])
+@pytest.mark.parametrize("calls", [
+    (2049,), (2100,),  # a second pass of one token, of 52
+    (100, 2049),       # a whole pass and one token after 100 others
+    (600, 1548),       # both calls one pass, the second the longer one
+], ids=str)
+def test_prefill_later_passes(gpu, long_prompts, kind, calls):
+    """Prompts of more than one pass, by their length or by a second call: later
+    passes read the pages that earlier ones wrote, and reuse their buffers.  Bars as
+    for one pass: FREE_RUN_TOL where int8 activations may flip, 1e-3 in fp16."""
+    torch = _torch()
+    make, prompt, seen = long_prompts[kind]
+    b, at, n = make(2), 0, sum(calls)
+    b.begin_synthetic(2, 0, 0, False)
+    b.prefill(1, prompt[:7])  # (another row between them)
+    for m in calls:
+        b.prefill(0, prompt[at:at + m])
+        at += m
+    logits = torch.empty((2, len(seen[n + 1])), device="cuda")
+    b.step([prompt[n], prompt[7]], logits_ptr=logits.data_ptr())
+    torch.cuda.synchronize()
+    assert b.context_len(0) == n + 1
+    err = rel_err(logits[0].cpu().numpy(), seen[n + 1])
+    record("free_run", test=f"prefill_later_passes_{kind}", calls=list(calls), logit_err=err)
+    assert err < (FREE_RUN_TOL if kind == "int8" else 1e-3), err
 
 
 def test_prefill_decode_kernel_fallback(gpu, oracle):
