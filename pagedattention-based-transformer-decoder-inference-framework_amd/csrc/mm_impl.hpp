@@ -204,7 +204,14 @@ struct RowOf {
       const int tile = pos / kPageTokens;
       at = pos % kPageTokens;
       entry = tile < e.max_tiles ? e.slot[m] * e.G * e.max_tiles + tile : -1;
-    } else if constexpr (EPI == kGroupOut) {
+    }
+  }
+  // kGroupOut.  The stream kernel's rows do it in Target::find, behind one branch with the
+  // rest: behind one of its own the compiler waits for the weight, and so for the first
+  // loads of A and W, before it issues the next (fp32, a row: 18.0 us, now 14.1).
+  template <typename T>
+  __device__ __forceinline__ void look_up(const KernelArgs& p, const Block<T>& b) {
+    if constexpr (EPI == kGroupOut) {
       out = b.shared ? p.g.M * p.g.top + m : p.g.perm[m];
       if (!b.shared) weight = p.g.weight[out];
     }
@@ -259,6 +266,7 @@ struct Target {
   void* p1 = nullptr;  // the second column's place where it is not next to the first
   float cs = 1.f, sn = 0.f;  // rotation; kGroupOut: cs is the weight
 
+  template <bool LOOKED_UP = false>
   __device__ __forceinline__ void find(const KernelArgs& p, const Block<T>& b, const RowOf<EPI>& r,
                                        const ColOf<EPI>& c) {
     const int m = r.m, n = c.n;
@@ -271,8 +279,10 @@ struct Target {
       T* d = static_cast<T*>(b.shared ? p.g.act_shared : p.g.act);
       p0 = d + (size_t)m * (b.shared ? p.g.lds : p.g.lda) + (n >> 1);
     } else if constexpr (EPI == kGroupOut) {
-      cs = r.weight;
-      float* d = p.g.out + (size_t)r.out * p.g.ldo + n;
+      RowOf<EPI> at = r;
+      if constexpr (!LOOKED_UP) at.look_up(p, b);
+      cs = at.weight;
+      float* d = p.g.out + (size_t)at.out * p.g.ldo + n;
       p0 = d;
       p1 = n + 1 < b.N ? d + 1 : nullptr;
     } else if constexpr (EPI == kSplit) {
@@ -443,7 +453,10 @@ __device__ __forceinline__ void emit_pairs(const KernelArgs& p, const Block<T>& 
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
-    for (int r = 0; r < 2; ++r) rows[i][r] = RowOf<EPI>(p, b, first + 16 * i + r);
+    for (int r = 0; r < 2; ++r) {
+      rows[i][r] = RowOf<EPI>(p, b, first + 16 * i + r);
+      if (rows[i][r].m >= 0) rows[i][r].look_up(p, b);
+    }
 #pragma unroll
   for (int j = 0; j < NT; ++j) {
     const int n = n0 + 16 * j + (lane & 14);
@@ -457,7 +470,7 @@ __device__ __forceinline__ void emit_pairs(const KernelArgs& p, const Block<T>& 
 #pragma unroll
       for (int r = 0; r < 2; ++r) {
         Target<T, EPI> t;
-        t.find(p, b, rows[i][r], col);
+        t.template find<true>(p, b, rows[i][r], col);
         t.put(p, b, n, odd ? o[2 + r] : c[r], odd ? c[2 + r] : o[r]);
       }
     }
