@@ -120,7 +120,7 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
     Frags x, y;
     if (stages >= ST) wait_lds_loads<(ST - 1) * LOADS>();
     else wait_lds_loads<0>();
-    __builtin_amdgcn_s_barrier();
+    barrier_only();
     if (here) {
       read(x, 0, 0);
       read(y, 0, 1);
@@ -130,7 +130,7 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
     auto landed = [&](int s) {  // stage s + 1 is there for everyone, stage s read out
       if (s + ST <= stages) wait_lds_loads<(ST - 2) * LOADS>();
       else wait_lds_loads<0>();
-      __builtin_amdgcn_s_barrier();
+      barrier_only();
     };
     landed(0);
     int s = 0;

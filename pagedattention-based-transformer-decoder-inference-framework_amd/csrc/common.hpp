@@ -167,6 +167,13 @@ __device__ __forceinline__ void wait_lds_loads() {
   __builtin_amdgcn_s_waitcnt(0x0070 | (LEFT & 15) | (LEFT >> 4) << 14);  // vmcnt(LEFT), lgkmcnt(0)
   asm volatile("" ::: "memory");
 }
+// The workgroup's barrier without __syncthreads' wait for the loads in flight; no access
+// to memory moves over it.
+__device__ __forceinline__ void barrier_only() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 
 // Offset of activation element (m, k) in MFMA A-fragment order ("packed A"):
 // one contiguous 1 KiB block per (16-row tile, k-step), lane l of the block

@@ -718,19 +718,8 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_block_kernel(GemmArgs a)
       if (a.c16) *reinterpret_cast<f16x8*>(a.c16 + a_frag_off_f16(m, n, a.N >> 5)) = h;
       if (page[i] >= 0) {
         _Float16* pool = which == 2 ? kv.v_pool : kv.k_pool;
-        if ((kv.D & 7) == 0) {
-          *reinterpret_cast<f16x8*>(pool + (size_t)page[i] * kv.page_stride +
-                                    (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
-        } else {  // the eight columns reach into other heads
-#pragma unroll 1
-          for (int k = 0; k < 8; ++k) {
-            const int c = n - which * hid + k, hd = c / kv.D;
-            const int row = kv.rows ? kv.rows[m] : m;
-            const int pg = kv.page_table[((size_t)row * kv.H + hd) * kv.max_tiles + pos[i] / kv.TS];
-            if (pg >= 0 && pg < kv.num_pages)
-              pool[(size_t)pg * kv.page_stride + (size_t)(pos[i] % kv.TS) * kv.D + c % kv.D] = h[k];
-          }
-        }
+        *reinterpret_cast<f16x8*>(pool + (size_t)page[i] * kv.page_stride +
+                                  (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
       }
     }
   }
@@ -921,9 +910,11 @@ template <GemmKind KIND>
 hipError_t launch_gemm(const GemmArgs& a_in, hipStream_t st, int nt_override = 0,
                        int waves_override = 0, int mrows_override = 0, int ks_override = 0) {
   GemmArgs a = a_in;
-  // rows of a prompt, once 64 x 64 blocks are more than half a round of workgroups
+  // rows of a prompt, once 64 x 64 blocks are more than half a round of workgroups; pages
+  // of heads of whole eights, which a thread's eight columns do not leave
   if (a.M > 64 && (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) > 128 && !a.ln_x && !a.partial &&
       !a.ksplit2 && !a.stamps && reinterpret_cast<uintptr_t>(a.A) % 16 == 0 &&
+      (!a.kv.k_pool || a.kv.D % 8 == 0) &&
       nt_override + waves_override + mrows_override + ks_override == 0)
     return a.a_packed ? launch_gemm_block<KIND, true>(a, st) : launch_gemm_block<KIND, false>(a, st);
   TileChoice tc{0, 0, 0};
