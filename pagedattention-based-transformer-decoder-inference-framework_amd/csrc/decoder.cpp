@@ -840,10 +840,12 @@ int llm_decoder::alloc_prefill(int C) {
   return LLM_OK;
 }
 
-// A card that the cache fills has no room for the long chunk: the short one then, and
-// from then on, since every try frees all of these buffers and allocates them again.
+// Past the short chunk in whole ones: prompts a little longer each time would otherwise
+// free and allocate everything at every one.  A card that the cache fills has no room for
+// the long chunk: the short one then, and from then on, for the same reason.
 int llm_decoder::ensure_prefill(int C) {
   if (C <= pf_cap) return LLM_OK;
+  if (C > kPrefillChunk) C = (C + kPrefillChunk - 1) / kPrefillChunk * kPrefillChunk;
   const int rc = alloc_prefill(C);
   if (rc != LLM_ERR_OOM || C <= kPrefillChunk) return rc;
   prompt_chunk = kPrefillChunk;
