@@ -109,6 +109,29 @@ __device__ __forceinline__ float group_sum(float x) {
   return x;
 }
 
+// Inclusive scans over the wave's lanes (row shifts, then the rows' last lanes to the
+// rows behind), so lane 63 holds the total; wave_scan_max of values >= 0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int lanes_before(int x) {  // 0 where there is none
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_scan_add(int x) {
+  x += lanes_before<0x111, 0xF>(x);  // row_shr 1, 2, 4, 8
+  x += lanes_before<0x112, 0xF>(x);
+  x += lanes_before<0x114, 0xF>(x);
+  x += lanes_before<0x118, 0xF>(x);
+  x += lanes_before<0x142, 0xA>(x);  // row_bcast 15 into rows 1 and 3
+  return x + lanes_before<0x143, 0xC>(x);  // row_bcast 31 into rows 2 and 3
+}
+__device__ __forceinline__ int wave_scan_max(int x) {
+  x = max(x, lanes_before<0x111, 0xF>(x));
+  x = max(x, lanes_before<0x112, 0xF>(x));
+  x = max(x, lanes_before<0x114, 0xF>(x));
+  x = max(x, lanes_before<0x118, 0xF>(x));
+  x = max(x, lanes_before<0x142, 0xA>(x));
+  return max(x, lanes_before<0x143, 0xC>(x));
+}
+
 __device__ __forceinline__ float wave_max(float x) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off, 64));

@@ -39,22 +39,28 @@ struct PaMergeRowArgs {
 // from lane s by readlane.  acc[j] * the returned 1 / L is the output at dim
 // lane + 64 j; a head with no partial returns acc = 0.
 template <int DPL, int BATCH>
-__device__ __forceinline__ float merge_head(const float* ml, const float* pa, int nsplit, int ns,
-                                            int D, float (&acc)[DPL]) {
+struct MergeFirst {
+  float m0, l0, m1, l1, v[BATCH][DPL];
+  __device__ __forceinline__ void load(const float* ml, const float* pa, int nsplit, int D) {
+    const int lane = lane_id(), nsl = max(nsplit - 1, 0);
+    m0 = ml[2 * min(lane, nsl)], l0 = ml[2 * min(lane, nsl) + 1];
+    m1 = ml[2 * min(64 + lane, nsl)], l1 = ml[2 * min(64 + lane, nsl) + 1];
+#pragma unroll
+    for (int s2 = 0; s2 < BATCH; ++s2)
+#pragma unroll
+      for (int j = 0; j < DPL; ++j)
+        v[s2][j] = pa[(size_t)min(s2, nsl) * D + min(lane + 64 * j, D - 1)];
+  }
+};
+template <int DPL, int BATCH>
+__device__ __forceinline__ float merge_loaded(MergeFirst<DPL, BATCH>& f, const float* pa, int ns,
+                                              int D, float (&acc)[DPL]) {
   const int lane = lane_id();
-  const int nsl = max(nsplit - 1, 0);
-  const float m0r = ml[2 * min(lane, nsl)], l0r = ml[2 * min(lane, nsl) + 1];
-  const float m1r = ml[2 * min(64 + lane, nsl)], l1r = ml[2 * min(64 + lane, nsl) + 1];
-  float v[BATCH][DPL];
-#pragma unroll
-  for (int s2 = 0; s2 < BATCH; ++s2)
-#pragma unroll
-    for (int j = 0; j < DPL; ++j)
-      v[s2][j] = pa[(size_t)min(s2, nsl) * D + min(lane + 64 * j, D - 1)];
-  const float m0 = lane < ns ? m0r : kNegSentinel;
-  const float m1 = 64 + lane < ns ? m1r : kNegSentinel;
-  const float l0 = lane < ns ? l0r : 0.f;
-  const float l1 = 64 + lane < ns ? l1r : 0.f;
+  float (&v)[BATCH][DPL] = f.v;
+  const float m0 = lane < ns ? f.m0 : kNegSentinel;
+  const float m1 = 64 + lane < ns ? f.m1 : kNegSentinel;
+  const float l0 = lane < ns ? f.l0 : 0.f;
+  const float l1 = 64 + lane < ns ? f.l1 : 0.f;
 #pragma unroll
   for (int s2 = 0; s2 < BATCH; ++s2)
 #pragma unroll
@@ -103,6 +109,13 @@ __device__ __forceinline__ float merge_head(const float* ml, const float* pa, in
   }
   return 1.0f / (L + 1e-6f);
 }
+template <int DPL, int BATCH>
+__device__ __forceinline__ float merge_head(const float* ml, const float* pa, int nsplit, int ns,
+                                            int D, float (&acc)[DPL]) {
+  MergeFirst<DPL, BATCH> f;
+  f.load(ml, pa, nsplit, D);
+  return merge_loaded(f, pa, ns, D, acc);
+}
 
 // Split merge, fp32 output: one wave per (b, h), 4 per workgroup.  The first
 // 16 splits' partials come in the first round trip (the 8-row C3 step merges
@@ -123,25 +136,35 @@ __global__ __launch_bounds__(256) void pa_merge_kernel(PaMergeArgs a) {
   const int bh = blockIdx.x * 4 + wave_id_uniform();
   if (bh >= a.B * a.H) return;
   const int b = bh / a.H;
-  int Tb = a.context_lens ? a.context_lens[b] : a.T;
-  Tb = min(max(Tb, 0), a.T);
-  const int ntiles = min((Tb + a.TS - 1) / a.TS, a.max_tiles);
-  const int pps = row_pps(a.pps, a.nsplit, ntiles);
-  // pps < 0: every split holds a partial (beam launches: cost-balanced splits)
-  int held = a.nsplit, ns = a.pps < 0 ? a.nsplit : min(a.nsplit, (ntiles + pps - 1) / pps);
-  size_t at = (size_t)bh * a.nsplit;
+  const float* ml = a.part_ml + (size_t)bh * a.nsplit * 2;
+  const float* pa = a.part_acc + (size_t)bh * a.nsplit * a.D;
+  MergeFirst<DPL, 16> first;
+  first.load(ml, pa, a.nsplit, a.D);  // (of equal splits: they come while the plan is made)
+  int ns;
   if constexpr (RAGGED) {
     const RaggedPlan p = ragged_plan(a.context_lens, a.B, a.T, a.TS, a.max_tiles, a.nsplit);
+    const int ntiles = min((ragged_tokens(p, b) + a.TS - 1) >> __builtin_ctz(a.TS), a.max_tiles);
     if (p.unit) {
-      const RowSplits r = ragged_find(p, [&](int row, int, int) { return row == b; });
-      held = r.count;
+      const RowSplits r = ragged_find(p, a.B, [&](int row, int, int) { return row == b; });
+      const size_t at = (size_t)r.first * a.H + (size_t)(bh % a.H) * r.count;
+      ml = a.part_ml + at * 2;
+      pa = a.part_acc + at * a.D;
+      first.load(ml, pa, r.count, a.D);
       ns = (ntiles + p.unit - 1) / p.unit;
-      at = (size_t)r.first * a.H + (size_t)(bh % a.H) * r.count;
+    } else {
+      const int pps = row_pps(0, a.nsplit, ntiles);
+      ns = min(a.nsplit, (ntiles + pps - 1) / pps);
     }
+  } else {
+    int Tb = a.context_lens ? a.context_lens[b] : a.T;
+    Tb = min(max(Tb, 0), a.T);
+    const int ntiles = min((Tb + a.TS - 1) / a.TS, a.max_tiles);
+    const int pps = row_pps(a.pps, a.nsplit, ntiles);
+    // pps < 0: every split holds a partial (beam launches: cost-balanced splits)
+    ns = a.pps < 0 ? a.nsplit : min(a.nsplit, (ntiles + pps - 1) / pps);
   }
   float acc[DPL];
-  const float inv =
-      merge_head<DPL, 16>(a.part_ml + at * 2, a.part_acc + at * a.D, held, ns, a.D, acc);
+  const float inv = merge_loaded(first, pa, ns, a.D, acc);
   float* o = a.out + (size_t)bh * a.D;
 #pragma unroll
   for (int j = 0; j < DPL; ++j) {
@@ -733,7 +756,9 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
   a.nsplit = nsplit;
   a.group = std::max(1, std::min(row_group, 4));
   a.qscale = sm_scale * kLog2e;
-  a.ragged = context_lens && !rows && !direct && row_group == 1 && pps_fixed <= 0 && B <= kRaggedRows;
+  a.ragged = context_lens && !rows && !direct && row_group == 1 && pps_fixed <= 0 && B > 1 &&
+             B <= kRaggedRows && nsplit < kRaggedSplits &&
+             (ntiles_max + nsplit - 1) / nsplit >= kRaggedPages;
   const bool wgm = wgm_ok && !direct && a.group == 1 && nsplit <= kWgmMaxSplits;
   if (!direct && !wgm) {  // (the workgroup merge keeps its splits' states in LDS)
     const size_t need = (size_t)B * H * nsplit * (size_t)(D + 2) * sizeof(float);

@@ -121,70 +121,93 @@ __device__ __forceinline__ int row_pps(int pps_fixed, int nsplit, int ntiles) {
 // B * nsplit splits a head, dealt out by need.  A row of n tiles gets ceil(n / unit) of
 // them, one at least, at unit = ceil(tiles of all rows / (B * (nsplit - 1))), which makes
 // no more than B * nsplit; equal counts leave the chip to the longest row (32 rows of 1 ..
-// 4096 tokens, half of them under 64: 16 heads of 128 bf16 53 us, so 35).  Where that
-// does not shorten the longest split, as for rows of one length, every row has nsplit.
-// Partials lie in the order (row, head, split) either way.  Lane l holds rows l, 64 + l, ...
-constexpr int kRaggedRows = 256;
+// 4096 tokens, half of them under 64: 16 heads of 128 bf16 53 us, so 35).  No row gets more
+// than kRaggedSplits, the merge's first batch, which it loads at once: a split more in a
+// later one costs more than the shorter splits give (20 rows of 1 .. 8192, 4 heads of 64:
+// 17.6 us equal, 27 with up to 128 splits, 17.2 with 16).
+//
+// Where that does not pay every row has nsplit equal splits: on the host by the launch's
+// longest (kRaggedSplits of them already, or of fewer than kRaggedPages tiles: what can be
+// saved is less than the 1 us of a plan), on the device by the contexts.  There the tiles of
+// all rows have to be less than 0.4 of what rows of the longest's length would have (a third
+// of 64 rows at 4096 tokens, the others at 512, which is 0.41: by need 24.3 us, equal 22.4;
+// 64 rows of lengths spread over their logarithm, 0.15: 110 us become 63), and a split has to
+// come out at 0.6 of an equal one or less.  Partials lie in the order (row, head, split)
+// either way.  Lane l holds rows l, 64 + l, ...
+//
+// Every wave of both launches works the plan out, before its first page: a load of the
+// contexts and register moves, no division where nothing is gained.  64 rows of one length
+// 0.3 us longer than without a plan, the merge none (its first loads are under way); with
+// exchanges through LDS and a second load of the own context both together 1.4.
+constexpr int kRaggedRows = 256, kRaggedSplits = 16, kRaggedPages = 16;
 struct RaggedPlan {
-  int count[kRaggedRows / 64];  // splits of the lane's rows
-  int unit;                     // tiles of a split; 0: nsplit equal splits
+  int tokens[kRaggedRows / 64];  // contexts of the lane's rows
+  int count[kRaggedRows / 64];   // their splits
+  int unit;                      // tiles of a split; 0: nsplit equal splits
 };
 struct RowSplits {
   int row, first, count;  // first: splits of the rows before it
 };
 
-__device__ __forceinline__ int ragged_tiles(const int32_t* lens, int row, int T, int TS, int max_tiles) {
-  return min((min(max(lens[row], 0), T) + TS - 1) / TS, max_tiles);
-}
-
 __device__ __forceinline__ RaggedPlan ragged_plan(const int32_t* lens, int B, int T, int TS,
                                                   int max_tiles, int nsplit) {
   RaggedPlan p;
-  int total = 0, most = 0;
+  const int shift = __builtin_ctz(TS);  // (pages of 16 or 32 tokens)
+  int tiles[kRaggedRows / 64], total = 0, most = 0;
 #pragma unroll
   for (int k = 0; k < kRaggedRows / 64; ++k) {
-    const int row = 64 * k + lane_id();
-    p.count[k] = row < B ? ragged_tiles(lens, row, T, TS, max_tiles) : 0;
-    total += p.count[k];
-    most = max(most, p.count[k]);
+    p.tokens[k] = 64 * k < B ? min(max(lens[min(64 * k + lane_id(), B - 1)], 0), T) : 0;
   }
 #pragma unroll
-  for (int d = 1; d < 64; d *= 2) {
-    total += __shfl_xor(total, d, 64);
-    most = max(most, __shfl_xor(most, d, 64));
+  for (int k = 0; k < kRaggedRows / 64; ++k) {
+    tiles[k] = 64 * k + lane_id() < B ? min((p.tokens[k] + TS - 1) >> shift, max_tiles) : 0;
+    total += tiles[k];
+    most = max(most, tiles[k]);
   }
+  total = __builtin_amdgcn_readlane(wave_scan_add(total), 63);
+  most = __builtin_amdgcn_readlane(wave_scan_max(most), 63);
   const int slots = B * (nsplit - 1);
-  const int unit = max((total + slots - 1) / slots, (most + kMaxSplits - 1) / kMaxSplits);
-  p.unit = __builtin_amdgcn_readfirstlane(unit < (most + nsplit - 1) / nsplit && unit <= kMaxPps ? unit : 0);
+  p.unit = 0;
+  if (100LL * total * nsplit <= 40LL * most * slots && most > 0) {
+    const int unit = max((total + slots - 1) / slots, (most + kRaggedSplits - 1) / kRaggedSplits);
+    if (5 * unit * nsplit <= 3 * most) p.unit = __builtin_amdgcn_readfirstlane(unit);
+  }
 #pragma unroll
   for (int k = 0; k < kRaggedRows / 64; ++k)
-    if (64 * k + lane_id() < B)
-      p.count[k] = p.unit ? max((p.count[k] + p.unit - 1) / p.unit, 1) : nsplit;
+    p.count[k] = p.unit && 64 * k + lane_id() < B ? max((tiles[k] + p.unit - 1) / p.unit, 1) : 0;
   return p;
 }
 
-// The row that `hit(row, splits before it, its splits)` names; row -1: none.
+// The context of a row (the same one for the whole wave).
+__device__ __forceinline__ int ragged_tokens(const RaggedPlan& p, int row) {
+  int t = __builtin_amdgcn_readlane(p.tokens[0], row & 63);  // (not of a chosen one: an array in LDS)
+#pragma unroll
+  for (int k = 1; k < kRaggedRows / 64; ++k) {
+    const int u = __builtin_amdgcn_readlane(p.tokens[k], row & 63);
+    t = row >> 6 == k ? u : t;
+  }
+  return t;
+}
+
+// Of a plan with a unit: the row that `hit(row, splits before it, its splits)` names; row
+// -1: none.
 template <typename Hit>
-__device__ __forceinline__ RowSplits ragged_find(const RaggedPlan& p, Hit hit) {
+__device__ __forceinline__ RowSplits ragged_find(const RaggedPlan& p, int B, Hit hit) {
   RowSplits r{-1, 0, 0};
   int before = 0;
 #pragma unroll
   for (int k = 0; k < kRaggedRows / 64; ++k) {
-    int sum = p.count[k];
-#pragma unroll
-    for (int d = 1; d < 64; d *= 2) {
-      const int below = __shfl_up(sum, d, 64);
-      sum += lane_id() >= d ? below : 0;
+    if (64 * k < B) {
+      const int sum = wave_scan_add(p.count[k]), first = before + sum - p.count[k];
+      const uint64_t at = __ballot(p.count[k] > 0 && hit(64 * k + lane_id(), first, p.count[k]));
+      if (at) {
+        const int l = __builtin_ctzll(at);
+        r.row = 64 * k + l;
+        r.first = __builtin_amdgcn_readlane(first, l);
+        r.count = __builtin_amdgcn_readlane(p.count[k], l);
+      }
+      before += __builtin_amdgcn_readlane(sum, 63);
     }
-    const int first = before + sum - p.count[k];
-    const uint64_t at = __ballot(p.count[k] > 0 && hit(64 * k + lane_id(), first, p.count[k]));
-    if (at) {
-      const int l = __builtin_ctzll(at);
-      r.row = 64 * k + l;
-      r.first = __builtin_amdgcn_readlane(first, l);
-      r.count = __builtin_amdgcn_readlane(p.count[k], l);
-    }
-    before += __builtin_amdgcn_readlane(sum, 63);
   }
   return r;
 }
@@ -292,19 +315,20 @@ void pa_split_kernel(PaSplitArgs a) {
   const int gh = BEAM && a.smaj ? rest % GH : rest / a.nsplit;
   int h = gh % a.H;
   int b = (gh / a.H) * G + gi;
-  int unit = 0;
+  int unit = 0, tokens = 0;
   if constexpr (RAGGED) {  // (group 1)
     const RaggedPlan p = ragged_plan(a.context_lens, a.B, a.T, TS, a.max_tiles, a.nsplit);
     unit = p.unit;
     if (unit) {
       const int slot = wid / a.H;
       const RowSplits r = ragged_find(
-          p, [&](int, int first, int count) { return slot >= first && slot < first + count; });
+          p, a.B, [&](int, int first, int count) { return slot >= first && slot < first + count; });
       if (r.row < 0) return;
       b = r.row;
       h = (wid - r.first * a.H) / r.count;
       s = (wid - r.first * a.H) % r.count;
     }
+    tokens = ragged_tokens(p, min(b, a.B - 1));
   }
   // BEAM: the shared path runs only when all 4 rows exist, route to a valid
   // page-table row and hold the same context (a uniform decision: every wave
@@ -361,8 +385,8 @@ void pa_split_kernel(PaSplitArgs a) {
   // partial-state slot
   const size_t pidx = RAGGED ? (size_t)wid : (size_t)bh * a.nsplit + s;
   const int r = a.beam_ids ? a.beam_ids[b] : b;
-  int Tb = a.context_lens ? a.context_lens[b] : a.T;
-  Tb = min(max(Tb, 0), a.T);
+  int Tb = RAGGED ? tokens : a.context_lens ? a.context_lens[b] : a.T;
+  if constexpr (!RAGGED) Tb = min(max(Tb, 0), a.T);
   const int ntiles = min((Tb + TS - 1) / TS, a.max_tiles);
   int tile0, count;
   // tiles of the split: tile0 + j * tstride, j < count

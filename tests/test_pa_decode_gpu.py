@@ -562,3 +562,33 @@ def test_pa_decode_long_context_few_rows(gpu, oracle, B, H):
     assert_parity(out, ref, RTOL)
     with pytest.raises(llm_capi.LlmError, match="128 splits"):
         llm_capi.pa_decode(_dev(q), _dev(kp), _dev(vp), _dev(pt), T=T, pages_per_split=8)
+
+
+# one long row among short ones, or a third of them: by need where equal splits are of 16
+# pages or more, fewer than 16, and leave most of the chip idle; else a row's splits do not
+# depend on the other rows.  The last: 16 equal splits already, and a third of the rows long
+@pytest.mark.parametrize("B,H,D,T,long,by_need", [
+    (64, 4, 64, 2048, 1, True), (20, 16, 128, 4096, 1, True), (200, 2, 64, 4096, 20, True),
+    (2, 4, 64, 2048, 1, False), (20, 16, 128, 200, 1, False), (20, 4, 64, 8192, 1, False),
+    (64, 4, 64, 4096, 24, False),
+])
+def test_pa_decode_need_or_equal(gpu, oracle, B, H, D, T, long, by_need):
+    import llm_capi
+    rng = np.random.default_rng(B + T + D)
+    q, kp, vp, pt = _random_case(rng, B, H, D, T, 16, num_beams=2)
+    beam_ids = rng.integers(0, 2, B).astype(np.int32)
+    lens = rng.integers(1, 40, B).astype(np.int32)
+    lens[1:1 + long] = T
+    args = [_dev(a) for a in (q, kp, vp, pt)]
+
+    def run(contexts):
+        return llm_capi.pa_decode(*args, T=T, beam_ids=_dev(beam_ids),
+                                  context_lens=_dev(contexts)).cpu().numpy()
+
+    out, alone = run(lens), run(np.full(B, T, np.int32))
+    rows = np.unique([0, 1, long, min(long + 1, B - 1), B - 1])
+    ref = oracle.paged_attention(q[rows], kp.astype(np.float32), vp.astype(np.float32), pt, T=T,
+                                 beam_ids=beam_ids[rows], context_lens=lens[rows])
+    assert_parity(out[rows], ref, RTOL)
+    assert_parity(out[1:1 + long], alone[1:1 + long], RTOL)
+    assert np.array_equal(out[1], alone[1]) != by_need
