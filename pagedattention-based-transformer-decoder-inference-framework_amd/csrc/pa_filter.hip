@@ -53,7 +53,8 @@ struct PaFilterArgs {
   float top_p;
   int eos;
   float eos_thr;
-  int lpt;  // lanes of a token's 16-byte pieces (a power of two); 0: rows that are no such pieces
+  int lpt;    // lanes of a token's 16-byte pieces (a power of two); 0: rows that are no such pieces
+  int shift;  // log2 of TS; -1: no power of two (a division costs some 30 instructions)
 };
 
 template <int KVT>
@@ -165,6 +166,16 @@ __device__ void filter_digit(const FilterHist& hist, uint32_t need, uint64_t lim
   __syncthreads();
 }
 
+// Rows of up to kRankRow tokens: every entry's own count and mass of the entries above it,
+// each against all (kRankParts threads an entry), in place of the histograms, whose six
+// passes over the digits take 8 us however short the row is.  The same whole numbers.
+constexpr int kRankRow = 256, kRankParts = kFilterThreads / kRankRow;
+struct FilterRank {
+  uint64_t key[kRankRow], own[kRankRow];      // (probability bits, index); mass
+  uint64_t mass[kRankParts][kRankRow];        // of the part's entries above
+  uint32_t count[kRankParts][kRankRow];
+};
+
 // One workgroup per (row, head).  The scores take one pass over K: 16-byte pieces, a
 // token's pieces in adjacent lanes, kScoreTokens tokens of a group in flight.  The entries
 // that stay are listed in the order of their index, and only their V rows are read, by all
@@ -187,7 +198,8 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   __shared__ uint64_t sh_mass[kWaves];
   __shared__ uint32_t sh_count[kWaves];
   __shared__ FilterCut found;
-  static_assert(sizeof(FilterHist) <= sizeof(llist), "the histograms lie in the list's memory");
+  static_assert(sizeof(FilterHist) <= sizeof(llist) && sizeof(FilterRank) <= sizeof(llist),
+                "the histograms and ranks lie in the list's memory");
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.x;
   float* sc = WS ? a.ws_sc + (size_t)bh * a.Tp : lsc;
@@ -200,15 +212,16 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   const bool row_ok = r >= 0 && r < a.num_beams;
   const int32_t* table = a.page_table + ((size_t)(row_ok ? r : 0) * a.H + h) * a.max_tiles;
   auto page_of = [&](int t) -> int {  // KVTileCache::get (kv_tile_cache.hpp:21-26)
-    const int tile = t / a.TS;
+    const int tile = a.shift >= 0 ? t >> a.shift : t / a.TS;
     if (!row_ok || tile >= a.max_tiles) return -1;
     const int p = table[tile];
     return (p < 0 || p >= a.num_pages) ? -1 : p;
   };
   // element of (page, token in it)
-  auto at = [&](int page, int t) { return (size_t)page * a.page_stride + (size_t)(t % a.TS) * D; };
-  for (int d = tid; d < D; d += kFilterThreads) qs[d] = a.q[(size_t)bh * D + d];
-  __syncthreads();
+  auto at = [&](int page, int t) {
+    const int in = a.shift >= 0 ? t & ((1 << a.shift) - 1) : t % a.TS;
+    return (size_t)page * a.page_stride + (size_t)in * D;
+  };
   // lanes per token, tokens of a wave at a time
   const int lpt = a.lpt, tpw = lpt ? 64 / lpt : 0, c = lpt ? lane % lpt : 0, g = lpt ? lane / lpt : 0;
 
@@ -217,40 +230,52 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   if (lpt) {
     float qv[EPL];
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) qv[e] = qs[c * EPL + e];
-    const int step = kScoreTokens * tpw;
+    for (int e = 0; e < EPL; ++e) qv[e] = a.q[(size_t)bh * D + c * EPL + e];
+    // the waves take turns of tpw tokens each, so that short rows are spread over them
+    const int step = kWaves * tpw;
     int page[kScoreTokens];
     auto pages = [&](int t0) {
 #pragma unroll
       for (int u = 0; u < kScoreTokens; ++u) {
-        const int t = t0 + u * tpw + g;
+        const int t = t0 + u * step + g;
         page[u] = t < Tb ? page_of(t) : -1;
       }
     };
-    pages(w * step);
-    for (int t0 = w * step; t0 < Tb; t0 += kWaves * step) {
+    if (w * tpw < Tb) pages(w * tpw);
+    for (int t0 = w * tpw; t0 < Tb; t0 += kScoreTokens * step) {
       u32x4 k[kScoreTokens];
       bool there[kScoreTokens];
 #pragma unroll
       for (int u = 0; u < kScoreTokens; ++u) {
-        const int t = t0 + u * tpw + g;
+        const int t = t0 + u * step + g;
         there[u] = page[u] >= 0;
         k[u] = u32x4{0u, 0u, 0u, 0u};
         if (there[u])
           k[u] = *reinterpret_cast<const u32x4*>(a.k_pool + at(page[u], t) * ES + c * 16);
       }
-      pages(t0 + kWaves * step);
+      if (t0 + kScoreTokens * step < Tb) pages(t0 + kScoreTokens * step);
+      float dot[kScoreTokens];
 #pragma unroll
       for (int u = 0; u < kScoreTokens; ++u) {
-        float dot = 0.f;
+        dot[u] = 0.f;
+        if (t0 + u * step < Tb) {  // (the same for the wave)
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) dot = fmaf(qv[e], kv_elem<KVT>(k[u], e), dot);
-        for (int off = lpt >> 1; off; off >>= 1) dot += __shfl_xor(dot, off, 64);
-        const int t = t0 + u * tpw + g;
-        if (c == 0 && t < Tb) sc[t] = there[u] ? dot / a.temperature : -1e9f;
+          for (int e = 0; e < EPL; ++e) dot[u] = fmaf(qv[e], kv_elem<KVT>(k[u], e), dot[u]);
+        }
+      }
+      for (int off = lpt >> 1; off; off >>= 1)
+#pragma unroll
+        for (int u = 0; u < kScoreTokens; ++u)
+          if (t0 + u * step < Tb) dot[u] += __shfl_xor(dot[u], off, 64);
+#pragma unroll
+      for (int u = 0; u < kScoreTokens; ++u) {
+        const int t = t0 + u * step + g;
+        if (t0 + u * step < Tb && c == 0 && t < Tb) sc[t] = there[u] ? dot[u] / a.temperature : -1e9f;
       }
     }
   } else {
+    for (int d = tid; d < D; d += kFilterThreads) qs[d] = a.q[(size_t)bh * D + d];
+    __syncthreads();
     for (int t = tid; t < Tb; t += kFilterThreads) {
       const int p = page_of(t);
       float s = -1e9f;
@@ -287,10 +312,43 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   // (cum of the higher-ranked probabilities) is >= top_p; no renormalisation.
   uint32_t cut_bits = 0;
   int cut_index = 0;
-  if ((a.top_k > 0 || a.top_p < 1.0f) && Tb > 0) {
+  const bool cuts = (a.top_k > 0 || a.top_p < 1.0f) && Tb > 0;
+  const uint32_t k = a.top_k > 0 ? (uint32_t)a.top_k : 0u;
+  const uint64_t limit = a.top_p < 1.0f ? max((uint64_t)ceilf(a.top_p * kMassUnit), (uint64_t)1) : 0;
+  if (cuts && Tb <= kRankRow) {
+    FilterRank& rank = *reinterpret_cast<FilterRank*>(llist);
+    if (tid < Tb) {  // (the thread that wrote sc[tid])
+      rank.key[tid] = (uint64_t)__float_as_uint(sc[tid]) << 32 | (uint32_t)tid;
+      rank.own[tid] = filter_mass(sc[tid]);
+    }
+    __syncthreads();
+    const int i = tid % kRankRow, part = tid / kRankRow, each = (Tb + kRankParts - 1) / kRankParts;
+    if (i < Tb) {
+      const uint64_t key = rank.key[i];
+      const int end = min((part + 1) * each, Tb);
+      uint32_t n = 0;
+      uint64_t m = 0;
+      for (int j = part * each; j < end; ++j) {
+        const bool above = rank.key[j] > key;
+        n += above ? 1u : 0u;
+        m += above ? rank.own[j] : 0;
+      }
+      rank.count[part][i] = n;
+      rank.mass[part][i] = m;
+    }
+    __syncthreads();
+    if (tid < Tb) {
+      uint32_t n = 0;
+      uint64_t m = 0;
+#pragma unroll
+      for (int j = 0; j < kRankParts; ++j) {
+        n += rank.count[j][tid];
+        m += rank.mass[j][tid];
+      }
+      if ((k && n >= k) || (limit && m >= limit)) sc[tid] = 0.f;
+    }
+  } else if (cuts) {
     FilterHist& hist = *reinterpret_cast<FilterHist*>(llist);
-    const uint32_t k = a.top_k > 0 ? (uint32_t)a.top_k : 0u;
-    const uint64_t limit = a.top_p < 1.0f ? max((uint64_t)ceilf(a.top_p * kMassUnit), (uint64_t)1) : 0;
     // digit `level` (0: the highest) of the bits, then of the index
     const auto histogram = [&](auto digit_of) {
       for (int i = tid; i < kDigits; i += kFilterThreads) {
@@ -360,12 +418,13 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   };
   // EOS hard threshold: keep only the EOS position when its weight exceeds it
   const bool only = a.eos >= 0 && a.eos < Tb && stays(a.eos) > a.eos_thr;
-  int n = 0;  // entries listed
+  const bool whole = !cuts && !only;  // the row as it is: no list
+  int n = whole ? Tb : 0;             // entries listed
   for (int t0 = 0; t0 < a.T; t0 += kFilterThreads) {
     const int t = t0 + tid;
     const float p = t < Tb && !(only && t != a.eos) ? stays(t) : 0.f;
     if (a.probs_out && t < a.T) a.probs_out[(size_t)bh * a.T + t] = p;
-    if (t0 >= Tb) continue;
+    if (whole || t0 >= Tb) continue;
     const uint64_t kept = __ballot(p != 0.f);
     if (lane == 0) sh_count[w] = (uint32_t)__popcll(kept);
     __syncthreads();
@@ -380,6 +439,12 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
     __syncthreads();
   }
 
+  // entry j < n: (probability bits, index); a value of weight 0 is not read
+  const auto entry = [&](int j) -> uint64_t {
+    return whole ? (uint64_t)__float_as_uint(sc[j]) << 32 | (uint32_t)j : list[j];
+  };
+  const auto page_of_entry = [&](uint64_t e) { return e >> 32 ? page_of((int)(uint32_t)e) : -1; };
+
   // out = sum_t p_t v_t over present tiles (cpu_attention_kernel.cpp:103-117)
   if (lpt) {
     float acc[EPL];
@@ -391,8 +456,8 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
 #pragma unroll
       for (int u = 0; u < kValueTokens; ++u) {
         const int j = j0 + u * kWaves * tpw;
-        const uint64_t item = j < n ? list[j] : 0;
-        const int t = (int)(uint32_t)item, pg = j < n ? page_of(t) : -1;
+        const uint64_t item = j < n ? entry(j) : 0;
+        const int t = (int)(uint32_t)item, pg = page_of_entry(item);
         p[u] = pg < 0 ? 0.f : __uint_as_float((uint32_t)(item >> 32));
         v[u] = u32x4{0u, 0u, 0u, 0u};
         if (pg >= 0) v[u] = *reinterpret_cast<const u32x4*>(a.v_pool + at(pg, t) * ES + c * 16);
@@ -402,27 +467,31 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[e] = fmaf(p[u], kv_elem<KVT>(v[u], e), acc[e]);
     }
-    for (int off = lpt; off < 64; off <<= 1)
+    if (whole) __syncthreads();  // (the sums go over the probabilities)
+    if (w * tpw < n) {           // (the other waves' sums are not read)
+      for (int off = lpt; off < 64; off <<= 1)
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
-    if (g == 0)
+        for (int e = 0; e < EPL; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
+      if (g == 0)
 #pragma unroll
-      for (int e = 0; e < EPL; ++e) lsc[w * D + c * EPL + e] = acc[e];
+        for (int e = 0; e < EPL; ++e) lsc[w * D + c * EPL + e] = acc[e];
+    }
   } else {
     // thread -> (dim d, group g of the list), groups summed in order at the end
     const int G = kFilterThreads / D, d = tid % D, gr = tid / D;
     float acc = 0.f;
     if (gr < G)
       for (int j = gr; j < n; j += G) {
-        const int t = (int)(uint32_t)list[j], pg = page_of(t);
+        const uint64_t item = entry(j);
+        const int t = (int)(uint32_t)item, pg = page_of_entry(item);
         if (pg < 0) continue;
-        acc += __uint_as_float((uint32_t)(list[j] >> 32)) *
-               kv_elem<KVT>(a.v_pool, at(pg, t) + d);
+        acc += __uint_as_float((uint32_t)(item >> 32)) * kv_elem<KVT>(a.v_pool, at(pg, t) + d);
       }
+    if (whole) __syncthreads();
     if (gr < G) lsc[gr * D + d] = acc;
   }
   __syncthreads();
-  const int groups = lpt ? kWaves : kFilterThreads / D;
+  const int groups = lpt ? min(kWaves, (n + tpw - 1) / tpw) : kFilterThreads / D;
   if (tid < D) {
     float o = 0.f;
     for (int i = 0; i < groups; ++i) o += lsc[i * D + tid];
@@ -435,10 +504,11 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
 using namespace llm;
 
 namespace {
-// The longest row the filtered form takes: its power-of-two sort length must
-// stay an int (filter_row_stride), and 2^30 tokens is far past any context
+// The longest row the filtered form takes: the workspace's row stride, a power of two, must
+// stay an int, and 2^30 tokens is far past any context.  (A row needs T entries; callers
+// have sized the workspace by the power of two from the first version on.)
 constexpr int kFilterRowMaxT = 1 << 30;
-int filter_row_stride(int T) {  // the bitonic sort's power-of-two length, T <= kFilterRowMaxT
+int filter_row_stride(int T) {
   int Tp = 1;
   while (Tp < T) Tp <<= 1;
   return Tp;
@@ -508,6 +578,7 @@ extern "C" int pa_decode_ex(const pa_kv_view* kv, const float* q, float* out,
   a.top_p = opt->top_p;
   a.eos = opt->eos_token;
   a.eos_thr = opt->eos_threshold;
+  a.shift = (a.TS & (a.TS - 1)) == 0 ? __builtin_ctz((unsigned)a.TS) : -1;
   // rows of whole 16-byte pieces, at most a wave's lanes of them, where the pools allow
   // 16-byte loads; other rows are read element by element
   const int row_bytes = D * kv_elem_size(kv->kv_dtype), pieces = row_bytes / 16;

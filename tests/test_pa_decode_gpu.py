@@ -592,3 +592,37 @@ def test_pa_decode_need_or_equal(gpu, oracle, B, H, D, T, long, by_need):
     assert_parity(out[rows], ref, RTOL)
     assert_parity(out[1:1 + long], alone[1:1 + long], RTOL)
     assert np.array_equal(out[1], alone[1]) != by_need
+
+
+# rows ranked entry against entry (up to 256 tokens), in LDS and in the workspace, and the
+# first that are not; the row as it is, with a list, and with nothing but the EOS position
+@pytest.mark.parametrize("T", [1, 2, 63, 255, 256, 257, 9000])
+@pytest.mark.parametrize("D,ts", [(64, 16), (24, 7)])
+@pytest.mark.parametrize("opt", [
+    dict(top_k=1), dict(top_k=7, top_p=0.5), dict(top_p=0.9), dict(top_p=1e-20), dict(),
+    dict(eos_token=0, eos_threshold=1e-9), dict(eos_token=0, eos_threshold=2.0),
+], ids=str)
+def test_pa_decode_ex_short_rows(gpu, oracle, T, D, ts, opt):
+    import llm_capi
+    rng = np.random.default_rng(T + D)
+    B, H, nt = 4, 2, (T + ts - 1) // ts
+    q = (rng.standard_normal((B, H, D)) * D ** -0.5).astype(np.float32)
+    q[2] = 0  # all weights equal: the largest indices stay
+    kp = rng.standard_normal((B * H * nt, ts, D)).astype(np.float16)
+    vp = rng.standard_normal((B * H * nt, ts, D)).astype(np.float16)
+    pt = rng.permutation(B * H * nt).astype(np.int32).reshape(B, H, nt)
+    pt[1, 1, nt // 2] = -1
+    lens = np.minimum([T, 256, 200, 3], T).astype(np.int32)
+    ref, rp, _ = oracle.paged_attention(q, kp.astype(np.float32), vp.astype(np.float32), pt, T=T,
+                                        context_lens=lens, want_probs=True, **opt)
+    out, probs, _ = llm_capi.pa_decode_ex(*[_dev(a) for a in (q, kp, vp, pt)], T=T,
+                                          context_lens=_dev(lens), want_probs=True, **opt)
+    out, probs = out.cpu().numpy(), probs.cpu().numpy()
+    kept, want = probs > 0, rp > 0
+    # the mass above an entry decides: within fp32 rounding of a sum of T weights one entry,
+    # the last, may fall on either side
+    assert (kept != want).sum(-1).max() <= (1 if opt.get("top_p", 1.0) < 1.0 else 0)
+    same, both = (kept == want).all(-1), kept & want
+    if same.any():
+        assert_parity(out[same], ref[same], RTOL)
+    assert_parity(probs * both, rp * both, RTOL)
