@@ -540,7 +540,7 @@ int llm_decoder::layer_attn(int l, hipStream_t st, const Rows& R, PaPlan* plan) 
   view.page_table += (size_t)R.table_row0 * H * view.max_tiles;  // rows r0..
   view.num_beams -= R.table_row0;
   if (R.prefill_row >= 0 && !R.mixed && pa_prefill_supported(&view) && !plan) {
-    // one MFMA pass over the chunk (K/V pages read once per 32 queries), then
+    // one MFMA pass over the chunk (K/V pages read once per 64 queries), then
     // the o_proj input conversion the decode merge would have fused
     PaRowOutputs ro;
     ro.pack = 1;
