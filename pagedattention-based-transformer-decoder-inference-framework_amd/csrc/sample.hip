@@ -23,6 +23,8 @@
 // latency of the passes and of the LDS atomics, one row being one workgroup.  Masses
 // are added as whole multiples of 2^-50, so their sums are exact to 2^-34 and do not
 // depend on the order of the atomics.
+#include <utility>
+
 #include "common.hpp"
 #include "row_ops.hpp"
 
@@ -31,6 +33,7 @@ namespace llm {
 constexpr int kSampleThreads = 1024;
 constexpr int kSampleWaves = kSampleThreads / 64;
 constexpr int kSampleSeg = 4 * kSampleThreads;  // tokens of a segment: 256 per wave, 4 per lane
+constexpr int kSampleSegments = 16;             // of the longest row
 constexpr int kBins = 1024;
 
 __device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
@@ -347,19 +350,25 @@ hipError_t launch_sample_segments(const SampleArgs& a, int rows, hipStream_t st)
   hipLaunchKernelGGL(sample_rows_kernel<NS>, dim3(rows), dim3(kSampleThreads), 0, st, a);
   return hipGetLastError();
 }
+// A kernel for every number of segments: its passes walk all of its registers, so a row
+// takes the time of its own length (top_k 40 and top_p 0.9, us: 20,000 tokens 20 with 5
+// segments and 24 with 8; 40,000 30 with 10 and 34 with 13; 50,257 35 with 13).
+template <size_t... I>
+hipError_t launch_sample_n(std::index_sequence<I...>, int segments, const SampleArgs& a, int rows,
+                           hipStream_t st) {
+  using Launch = hipError_t (*)(const SampleArgs&, int, hipStream_t);
+  static constexpr Launch launch[] = {launch_sample_segments<(int)I + 1>...};
+  return launch[segments - 1](a, rows, st);
+}
 
 hipError_t launch_sample_rows(const SampleArgs& a, int rows, hipStream_t st) {
-  if (a.V > 16 * kSampleSeg) return hipErrorInvalidValue;
+  if (a.V > kSampleSegments * kSampleSeg) return hipErrorInvalidValue;
   if (a.temperature <= 0.f || a.top_k == 1) {
     hipLaunchKernelGGL(sample_greedy_kernel, dim3(rows), dim3(kSampleThreads), 0, st, a);
     return hipGetLastError();
   }
-  const int segments = (a.V + kSampleSeg - 1) / kSampleSeg;
-  if (segments <= 2) return launch_sample_segments<2>(a, rows, st);
-  if (segments <= 4) return launch_sample_segments<4>(a, rows, st);
-  if (segments <= 8) return launch_sample_segments<8>(a, rows, st);
-  if (segments <= 13) return launch_sample_segments<13>(a, rows, st);
-  return launch_sample_segments<16>(a, rows, st);
+  return launch_sample_n(std::make_index_sequence<kSampleSegments>(), (a.V + kSampleSeg - 1) / kSampleSeg, a,
+                         rows, st);
 }
 
 }  // namespace llm
@@ -371,7 +380,7 @@ extern "C" int sample_rows(const float* logits, int rows, int V, float temperatu
   LLM_REQUIRE(rows >= 0 && V > 0, "sample_rows: bad shape");
   if (rows == 0) return LLM_OK;
   LLM_REQUIRE(logits && out, "sample_rows: NULL pointer");
-  LLM_REQUIRE(V <= 16 * kSampleSeg, "sample_rows: V > 65536");
+  LLM_REQUIRE(V <= kSampleSegments * kSampleSeg, "sample_rows: V > 65536");
   LLM_REQUIRE(top_k >= 0 && top_p > 0.f && top_p <= 1.0f, "sample_rows: top_k >= 0, 0 < top_p <= 1");
   SampleArgs a{logits, V, temperature, top_k, top_p, seed, nullptr, counter, 0, out, nullptr, 0};
   LLM_HIP_RET(launch_sample_rows(a, rows, as_stream(stream)));

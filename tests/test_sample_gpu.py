@@ -26,6 +26,19 @@ def test_vocabulary_borders(gpu, V, T, k, p):
         assert ((got == ref) | (margin < 1e-4)).all(), (got, ref, margin)
 
 
+@pytest.mark.parametrize("segments", range(1, 17))
+def test_every_number_of_segments(gpu, segments):
+    """Rows of whole segments and of one token more than the form before takes."""
+    from oracle.oracle import sample_rows
+    for V in {4096 * segments, 4096 * (segments - 1) + 1}:
+        logits = (np.random.default_rng(V).standard_normal((3, V)) * 2).astype(np.float32)
+        logits[:, -1] = logits.max(1) + 3.0  # the last token is drawn now and then
+        for counter in range(4):
+            ref, margin = sample_rows(logits, 0.9, 60, 0.95, seed=5, counter=counter)
+            got = draw(logits, 0.9, 60, 0.95, counter)
+            assert ((got == ref) | (margin < 1e-4)).all(), (V, got, ref, margin)
+
+
 def test_ties_stay_together(gpu):
     """Equal probabilities share a rank: all of them stay, nothing below does."""
     V = 20000
