@@ -74,7 +74,7 @@ constexpr int kWaves = 4;
 constexpr int kTileQueries = 16 * kWaves;  // of a workgroup
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
-constexpr float kPShift = 14.f, kPScale = 16384.f;  // P enters the PV MFMA as p * 2^14 (hi + lo)
+constexpr float kPScale = 16384.f;  // P enters the PV MFMA as p * 2^14 (hi + lo)
 
 __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
   hi = (_Float16)x;
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
   }
 
   f32x4 O[ND];
-  float nrun = kNegSentinel, lrun = 0.f;
+  float mrun = kNegSentinel, lrun = 0.f;
 #pragma unroll
   for (int nd = 0; nd < ND; ++nd) O[nd] = f32x4{0.f, 0.f, 0.f, 0.f};
 
@@ -238,27 +238,28 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
             mloc = fmaxf(mloc, sc[u][r]);
           }
       }
-      // online softmax (per query = per lane): p = 2^(s - n), n the running maximum
-      // less 14, so that p comes out scaled for the halves; s is scaled back in the same
-      // operation
+      // online softmax (per query = per lane): p = 2^(s - m), m the running maximum; s is
+      // scaled back in the same operation.  (The scale of the halves in the exponent as well,
+      // 2^(s - m + 14), saves an instruction a value and rounds the exponent of the large p
+      // to 2^-21: 1.2 to 2 times the error of the result.)
       f16x8 ph, pl;
-      const float nloc = rows_max(mloc) * qinv - kPShift;
-      if (__any(nloc > nrun)) {
-        const float nnew = fmaxf(nrun, nloc);
-        const float corr = __builtin_amdgcn_exp2f(nrun - nnew);
+      const float mblk = rows_max(mloc) * qinv;
+      if (__any(mblk > mrun)) {
+        const float mnew = fmaxf(mrun, mblk);
+        const float corr = __builtin_amdgcn_exp2f(mrun - mnew);
         lrun *= corr;
 #pragma unroll
         for (int nd = 0; nd < ND; ++nd) O[nd] *= corr;
-        nrun = nnew;
+        mrun = mnew;
       }
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(sc[u][r], qinv, -nrun));
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[u][r], qinv, -mrun));
           lrun += p;
           _Float16 hi, lo;
-          split_f16(p, hi, lo);  // p <= 2^14: clear of fp16 subnormals
+          split_f16(p * kPScale, hi, lo);  // p <= 1: scaled clear of fp16 subnormals
           ph[4 * u + r] = hi;
           pl[4 * u + r] = lo;
         }
@@ -286,7 +287,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
   // the 4 lanes of a query hold partial sums over their keys
   lrun += __shfl_xor(lrun, 16, 64);
   lrun += __shfl_xor(lrun, 32, 64);
-  lrun *= 1.0f / kPScale;
   const int qi = q0 + c;
   if (qi >= a.m) return;
   if (a.part_acc) {  // split partial state (unnormalised, log2 units)
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
 #pragma unroll
     for (int nd = 0; nd < ND; ++nd)
       *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * (1.0f / kPScale);
-    if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{nrun + kPShift, lrun};
+    if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{mrun, lrun};
   } else {
     const float inv = 1.0f / (lrun + 1e-6f) * (1.0f / kPScale);
     float* o = a.out + (size_t)qi * a.out_stride + h * D + 4 * g;
