@@ -68,15 +68,14 @@ struct Request {
 // Logits rows to the caller's memory through a ring of pinned pieces: the host copies
 // one piece out while the next ones arrive.  A copy into pageable memory by the runtime
 // takes its staging and the host's copy one after the other: 64 rows of 32,768 505 us,
-// so 157 us on the bus and 107 us of host copy beside it.  Eight pieces: a piece costs
-// 10 us of its own on the stream and 15 us to submit, most of it while the step still
-// runs, and the last one's host copy stands alone.  Up to 1 MiB the runtime's way is the
-// faster one, its copy being one call (whole steps of small and large stacks: 1 row of
-// 32,768 135 and 138 us through the ring, 4 rows 175 and 181, 8 rows, 1 MiB, 316 and 327;
-// 16 rows 444 and 409).
+// so 157 us on the bus and 107 us of host copy beside it.  Pieces of 1 MiB: one costs 10 us
+// of its own on the stream and 15 us to submit, most of it while the step still runs, and
+// the last one's host copy stands alone.  (Smaller pieces for smaller steps: 14 rows of a
+// small stack 277 us a step, so 218; by the runtime 240.)  One piece behind a step's graph
+// is waited for by its stream: 1 row 123 us, by an event 129; behind launches by an event:
+// a prompt of 17 tokens 166 us, by the stream 180.  (By the runtime 123 and 197.)
 struct RowCopy {
-  static constexpr size_t kPiece = 1 << 20, kLeast = 256 << 10;  // bytes of a piece, of a small one
-  static constexpr size_t kByRuntime = 1 << 20;  // a step's bytes that go the runtime's way
+  static constexpr size_t kPiece = 1 << 20;  // bytes
   static constexpr int kRing = 8;
   char* ring = nullptr;
   hipEvent_t arrived[kRing] = {};
@@ -113,11 +112,12 @@ struct RowCopy {
     return true;
   }
   // Row r of src (`width` floats each) to host row rows[r]; returns when all are there.
-  int copy(float* host, const std::vector<size_t>& rows, const float* src, size_t width,
+  // graph: they come from a step that may be a captured one.
+  int copy(float* host, const std::vector<size_t>& rows, const float* src, size_t width, bool graph,
            hipStream_t st) {
     const size_t row_bytes = width * sizeof(float), total = rows.size() * row_bytes;
     if (!total) return finish(LLM_OK, st);
-    if (!ring || total <= kByRuntime || !pageable(host)) {
+    if (!ring || !pageable(host)) {
       for (size_t r = 0, n; r < rows.size(); r += n) {
         for (n = 1; r + n < rows.size() && rows[r + n] == rows[r] + n;) ++n;
         LLM_HIP_RET(hipMemcpyAsync(host + rows[r] * width, src + r * width, n * row_bytes,
@@ -125,24 +125,27 @@ struct RowCopy {
       }
       return finish(LLM_OK, st);
     }
-    const size_t share = (total / kRing + kLeast) / kLeast * kLeast;  // a whole ring
-    const size_t piece_bytes = std::min(share, kPiece), pieces = (total + piece_bytes - 1) / piece_bytes;
+    const size_t pieces = (total + kPiece - 1) / kPiece;
+    const bool by_event = pieces > 1 || !graph;
     const auto fetch = [&](size_t k) -> int {
-      const size_t at = k * piece_bytes;
+      const size_t at = k * kPiece;
       LLM_HIP_RET(hipMemcpyAsync(ring + k % kRing * kPiece, reinterpret_cast<const char*>(src) + at,
-                                 std::min(piece_bytes, total - at), hipMemcpyDeviceToHost, st));
-      LLM_HIP_RET(hipEventRecord(arrived[k % kRing], st));
+                                 std::min(kPiece, total - at), hipMemcpyDeviceToHost, st));
+      if (by_event) LLM_HIP_RET(hipEventRecord(arrived[k % kRing], st));
       return LLM_OK;
+    };
+    const auto wait = [&](size_t k) {
+      return by_event ? hipEventSynchronize(arrived[k % kRing]) : hipStreamSynchronize(st);
     };
     for (size_t k = 0; k < std::min<size_t>(pieces, kRing); ++k)
       if (const int rc = fetch(k)) return finish(rc, st);
     for (size_t k = 0; k < pieces; ++k) {
-      if (const hipError_t e = hipEventSynchronize(arrived[k % kRing])) {
+      if (const hipError_t e = wait(k)) {
         (void)finish(LLM_OK, st);
         LLM_HIP_RET(e);
       }
       const char* piece = ring + k % kRing * kPiece;
-      const size_t first = k * piece_bytes, end = std::min(first + piece_bytes, total);
+      const size_t first = k * kPiece, end = std::min(first + kPiece, total);
       for (size_t at = first; at < end;) {
         const size_t r = at / row_bytes, in = at % row_bytes;
         const size_t n = std::min(row_bytes - in, end - at);
@@ -262,7 +265,9 @@ int llm_engine::step(const llm_engine_entry* entries, int n, float* host) {
     }
     RET_IF(ensure_logits(rows.size()));
     RET_IF(model->forward(batch, logits.p, stream));
-    RET_IF(out.copy(host, rows, logits.p, V, stream));
+    bool single = true;  // one token a sequence: a decode step
+    for (const StepSeq& s : batch) single = single && s.n == 1;
+    RET_IF(out.copy(host, rows, logits.p, V, single, stream));
     for (const StepSeq& s : batch) seqs[s.slot].len = s.p0 + s.n;
     batch.clear();
     wants.clear();

@@ -1,6 +1,6 @@
-"""Logits rows of an engine step in the caller's memory.  More than 1 MiB of them go to
-pageable memory through the engine's ring of eight pinned pieces (of 256 KiB to 1 MiB); less,
-and memory that the runtime knows, goes the runtime's way.  All hold the same bytes."""
+"""Logits rows of an engine step in the caller's memory.  They go to pageable memory through
+the engine's ring of eight pinned pieces of 1 MiB, to memory that the runtime knows by its
+copy.  Both hold the same bytes."""
 import ctypes
 
 import numpy as np
@@ -49,8 +49,8 @@ def check(eng, lens, pick):
         np.testing.assert_array_equal(plain, pinned.numpy())
 
 
-# rows of 20,012 bytes: one; 52 and 53: the last by the runtime and the first through the
-# ring; 105 and 128: five pieces; 127 in gaps, and a batch of two passes whose rows lie apart
+# rows of 20,012 bytes: one; 52 and 53: the last in one piece and the first in two; 105 and
+# 128: three pieces; 127 in gaps, and a batch of two passes whose rows lie apart
 @pytest.mark.parametrize("lens,pick", [
     ([1], None), ([26], None), ([52], None), ([53], None), ([105], None), ([128], None),
     ([60, 67], "odd"), ([100, 90], "back"), ([3], "none"),
@@ -69,7 +69,7 @@ def wide(gpu, tmp_path_factory):
         yield e
 
 
-# rows of 160,036 bytes: 6 and 7 on both sides of 1 MiB; 52 just fill the ring's 8 MiB, 53
+# rows of 160,036 bytes: 6 and 7 on both sides of a piece; 52 just fill the ring's 8 MiB, 53
 # use a piece again, 105 (over 16 MiB) and 128 a piece for the third time; in gaps and back
 # to front, and 190 rows of two passes
 @pytest.mark.parametrize("lens,pick", [
