@@ -39,10 +39,17 @@ __device__ __forceinline__ TileAt xcd_tile(int id, int nx, int ny) {
 // TFLOP/s (113 us with two k-steps loaded and waited for together in 128 x 128 blocks
 // of four waves); 2048 x 12288 x 2048 101 us (143), 700 x 2048 x 2048 12.3 us (32).
 //
+// PARTS: K in eight parts, each summed from zero and then added to the parts before it.
+// One fp32 sum over all of K is off by 2 to 3 times as much as the streams' eight waves'
+// (fp16, K 8192: 5.7e-7 of the result, so 2.1e-7, streams 2.1e-7; an fp32 stack's prompt of
+// 100 tokens 1.5e-6, so 8.3e-7): a wave's registers hold both, and it costs fp16 products
+// 3 to 10 % (2048 x 6144 x 2048 74.0 -> 78.7 us, the 64-row streams 321), fp32 ones nothing.
+// Not for bf16, whose operands' rounding hides it, nor for int8, whose sums are exact.
+//
 // here: whether any of the wave's rows exist (the others load and wait).  When it
 // returns, nobody reads LDS any more.
-template <bool A_PACKED, int MB, int NB, int WM, int WN, int ST, typename Acc, typename A, typename W,
-          typename Mma>
+template <bool A_PACKED, bool PARTS, int MB, int NB, int WM, int WN, int ST, typename Acc, typename A,
+          typename W, typename Mma>
 __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64],
                                               Acc (&acc)[MB / WM][NB / WN], int KS, bool here,
                                               const A& a_at, const W& w_tile, const Mma& mma) {
@@ -107,6 +114,27 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
       acc[i][j] = mma(f.a[i], f.c[j], acc[i][j]);
     }
   };
+  Acc sum[PARTS ? MT : 1][PARTS ? NT : 1];
+  if constexpr (PARTS) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) sum[i][j] = Acc{0, 0, 0, 0};
+  }
+  // (PARTS) the part so far to the sum of parts
+  auto part = [&] {
+    if constexpr (PARTS) {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+          sum[i][j] += acc[i][j];
+          acc[i][j] = Acc{0, 0, 0, 0};
+        }
+    }
+  };
+  const int every = PARTS ? max((stages + 4) / 8, 1) : 1;  // stages of a part
+  int left = every;
   const std::integral_constant<int, 0> zero;
   const std::integral_constant<int, LOADS / 2> half;
   const std::integral_constant<int, LOADS> all;
@@ -146,6 +174,10 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) issue(now, i);
       }
+      if (PARTS && --left == 0) {
+        part();
+        left = every;
+      }
       landed(s + 1);
     }
     for (; s + 1 < stages; ++s) {
@@ -155,6 +187,10 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
         mul(y, 0, zero, zero);
         read(y, st, 1);
         mul(x, 0, zero, zero);
+      }
+      if (PARTS && --left == 0) {
+        part();
+        left = every;
       }
       landed(s + 1);
     }
@@ -172,6 +208,12 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
 #pragma unroll
     for (int j = 0; j < NT; ++j) f.c[j] = *reinterpret_cast<const u32x4*>(w_tile(wn * NT + j) + at);
     mul(f, 0, zero, zero);
+  }
+  if constexpr (PARTS) {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] += sum[i][j];
   }
 }
 

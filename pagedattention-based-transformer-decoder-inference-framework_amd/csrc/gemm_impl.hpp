@@ -598,7 +598,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_block_kernel(GemmArgs a)
   const int KS = a.KS, ntiles = (a.N + 15) >> 4, mtiles = (a.M + 15) >> 4;
   const int m0 = tile.y * 16 * MB, nt0 = tile.x * NB;
   acc_t acc[MT][NT];
-  block_product<A_PACKED, MB, NB, WM, WN, ST>(
+  block_product<A_PACKED, KIND == GemmKind::F16, MB, NB, WM, WN, ST>(
       lds, acc, KS, m0 + 16 * wm * MT < a.M,
       [&](int r) {
         const char* A = reinterpret_cast<const char*>(a.A);

@@ -856,7 +856,7 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p)
   const int nt0 = tile.x * NB, KS = b.KS;
   const int wm = w / WN, wn = w % WN;
   f32x4 acc[MT][NT];
-  block_product<false, MB, NB, WM, WN, ST>(
+  block_product<false, !Kind<T>::BF16, MB, NB, WM, WN, ST>(
       lds, acc, KS, b.m0 + 16 * wm * MT < b.M,
       [&](int r) { return a_row<T, EPI>(p, b, b.m0 + r); },
       [&](int t) { return b.W + (size_t)min(nt0 + t, ntiles - 1) * KS * 1024; },

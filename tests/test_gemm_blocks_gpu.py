@@ -49,3 +49,21 @@ def test_fp16(gpu, M, N, K):
     # fp32 sums of K exact products in some order: K roundings of the largest partial sum
     size = A[:, :K].double().abs() @ W.double().abs() + bias.double().abs()
     assert ((C - ref).abs() <= 2.0 ** -23 * (K ** 0.5 + 2) * size).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(700, 1024, 256), (512, 2304, 768), (320, 6144, 2048), (1024, 2048, 8192)])
+def test_fp16_sums_as_exact_as_the_streams(gpu, M, N, K):
+    """A block's sum over K goes in eight parts, as a stream's over its waves: off no more
+    than a tenth beyond the stream of the same rows (one sum over all of K: 1.4 to 2.7
+    times)."""
+    import torch
+    import llm_capi
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A = torch.randn((M, K), generator=g, device="cuda").half()
+    W = torch.randn((K, N), generator=g, device="cuda").half()
+    packed = llm_capi.pack_weights(W, llm_capi.LLM_F16)
+    ref = A.double() @ W.double()
+    blocks = llm_capi.f16_gemm(A, packed, N).double()
+    streams = torch.cat([llm_capi.f16_gemm(A[i:i + 64], packed, N).double() for i in range(0, M, 64)])
+    off = [((x - ref).norm() / ref.norm()).item() for x in (blocks, streams)]
+    assert off[0] <= 1.1 * off[1], off
