@@ -165,3 +165,27 @@ def test_pa_prefill_rejects_unsupported(gpu):
         kp, vp, pt = _case(rng, rows=1, H=2, D=64, T=20, ts=16)
         q = rng.standard_normal((100, 2, 64)).astype(np.float32)
         llm_capi.pa_prefill(_dev(q), _dev(kp), _dev(vp), _dev(pt), row=0, p0=0)
+
+
+@pytest.mark.parametrize("H,D,m", [(4, 64, 113), (16, 64, 300), (16, 128, 300), (4, 64, 1024)])
+def test_pa_prefill_as_exact_as_decode(gpu, H, D, m):
+    """Small scores, so that the weights' own rounding decides: against 64 bits off no more
+    than half as much again as the decode kernel over the same rows (whose weights stay
+    fp32; with the scale of the weights' halves in their exponent it was twice as much)."""
+    import torch
+    import llm_capi
+    g = torch.Generator(device="cuda").manual_seed(m)
+    nt = -(-m // 16)
+    kp, vp = (torch.randn((H * nt, 16, D), generator=g, device="cuda").half() for _ in "kv")
+    pt = torch.randperm(H * nt, generator=g, device="cuda").int().view(1, H, nt).contiguous()
+    q = torch.randn((m, H, D), generator=g, device="cuda") * 0.3 * D ** -0.5
+    k, v = (x[pt[0].long()].reshape(H, -1, D)[:, :m].double() for x in (kp, vp))
+    s = (q.double().transpose(0, 1) @ k.transpose(1, 2).contiguous()).masked_fill(
+        torch.ones((m, m), dtype=torch.bool, device="cuda").triu(1), -float("inf"))
+    e = torch.exp(s - s.amax(-1, keepdim=True))
+    ref = ((e / (e.sum(-1, keepdim=True) + 1e-6)) @ v).transpose(0, 1)
+    rows = torch.arange(m, dtype=torch.int32, device="cuda")
+    outs = (llm_capi.pa_prefill(q, kp, vp, pt, row=0, p0=0),
+            llm_capi.pa_decode(q, kp, vp, pt, T=m, beam_ids=torch.zeros_like(rows), context_lens=rows + 1))
+    off = [((x.double() - ref).norm() / ref.norm()).item() for x in outs]
+    assert off[0] <= 1.5 * off[1], off
