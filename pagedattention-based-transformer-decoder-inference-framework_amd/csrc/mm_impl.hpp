@@ -910,21 +910,24 @@ hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
 // 2048, launch taken off (us).  A product takes the form with the least rounds x time:
 // 2048 x 12288: 3 rounds of 128 x 256, 101 us (128 x 128: 115); 2048 x 2048: one round
 // of 128 x 128, 21.5 us (128 x 256 leaves half the chip idle: 33); 700 x 2048: 64 x 128,
-// 12.2 us (128 x 128: 23); 64 x 12288: 64 x 64, 11.0 us (64 x 32: 13).
+// 12.2 us (128 x 128: 23); 64 x 12288: 64 x 64, 11.0 us (64 x 32: 13).  fp32 blocks are
+// bound by the matrix cores and take the time of their area, the small ones, of which a CU
+// holds several, the time between two rounds: 2048 x 2048: two rounds of 64 x 128, 140 us
+// (128 x 128: 158); 700 x 6144: five of 64 x 64, 185 us (64 x 128: 207); K only scales all.
 template <typename T, int EPI>
 struct BlockForm {
   int mb, nb;
-  float round;
+  float bf16, fp32;
   hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
 };
 template <typename T, int EPI>
 hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipStream_t st) {
-  static constexpr BlockForm<T, EPI> forms[] = {{4, 2, 4.2f, blocks<T, EPI, 4, 2, 2, 2, 4>},
-                                                {4, 4, 6.2f, blocks<T, EPI, 4, 4, 2, 2, 3>},
-                                                {4, 8, 10.f, blocks<T, EPI, 4, 8, 2, 4, 4>},
-                                                {4, 16, 19.5f, blocks<T, EPI, 4, 16, 2, 4, 3>},
-                                                {8, 8, 18.5f, blocks<T, EPI, 8, 8, 4, 2, 3>},
-                                                {8, 16, 30.f, blocks<T, EPI, 8, 16, 2, 4, 3>}};
+  static constexpr BlockForm<T, EPI> forms[] = {{4, 2, 4.2f, 21.5f, blocks<T, EPI, 4, 2, 2, 2, 4>},
+                                                {4, 4, 6.2f, 37.f, blocks<T, EPI, 4, 4, 2, 2, 3>},
+                                                {4, 8, 10.f, 70.f, blocks<T, EPI, 4, 8, 2, 4, 4>},
+                                                {4, 16, 19.5f, 160.f, blocks<T, EPI, 4, 16, 2, 4, 3>},
+                                                {8, 8, 18.5f, 156.f, blocks<T, EPI, 8, 8, 4, 2, 3>},
+                                                {8, 16, 30.f, 293.f, blocks<T, EPI, 8, 16, 2, 4, 3>}};
   const BlockForm<T, EPI>* best = nullptr;
   int best_y = 0;
   float least = 0.f;
@@ -935,7 +938,7 @@ hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipS
     if constexpr (EPI == kGroupIn || EPI == kGroupOut)
       groups = (p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, f.nb) +
                p.g.shared_tiles * group_across(p.g.shared_n, f.nb);
-    const float cost = (float)((groups + 255) / 256) * f.round;
+    const float cost = (float)((groups + 255) / 256) * (Kind<T>::BF16 ? f.bf16 : f.fp32);
     if (best && cost >= least) continue;
     best = &f;
     best_y = y;
