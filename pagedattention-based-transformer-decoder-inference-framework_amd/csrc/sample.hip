@@ -36,13 +36,6 @@ constexpr int kSampleSeg = 4 * kSampleThreads;  // tokens of a segment: 256 per 
 constexpr int kSampleSegments = 16;             // of the longest row
 constexpr int kBins = 1024;
 
-__device__ __forceinline__ uint64_t splitmix64(uint64_t z) {
-  z += 0x9E3779B97F4A7C15ull;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  return z ^ (z >> 31);
-}
-
 // uniform in [0, 1) with 24 random bits (exactly representable in fp32)
 __host__ __device__ __forceinline__ float sample_uniform(uint64_t seed, int row, int counter) {
   uint64_t z = seed ^ ((uint64_t)(uint32_t)row << 32) ^ (uint64_t)(uint32_t)counter;
