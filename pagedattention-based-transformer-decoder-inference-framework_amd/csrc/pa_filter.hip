@@ -180,7 +180,7 @@ struct FilterRank {
 // token's pieces in adjacent lanes, kScoreTokens tokens of a group in flight.  The entries
 // that stay are listed in the order of their index, and only their V rows are read, by all
 // lanes.  16 rows x 12 heads of 64, 2048 tokens, top 64: 70 us with a token a thread, a
-// sort of the row and a walk over all of it for the values, now 31.  Bound by the
+// sort of the row and a walk over all of it for the values, now 30.  Bound by the
 // latency of its steps; the 192 workgroups are one a CU.
 constexpr int kScoreTokens = 8, kValueTokens = 4;
 

@@ -16,7 +16,7 @@
 // A stage goes from memory straight into LDS, one stage ahead, a wave loading
 // 16 keys, with their page looked up two stages ahead: the dependent loads
 // (page, keys) and a register pass per 32 keys were what bounded the first form
-// (2048 queries x 16 heads x 128: 137 us, now 58 us).  The
+// (2048 queries x 16 heads x 128: 137 us, now 61 us).  The
 // 16-byte chunks of a row are exchanged by the key so that the 16 rows of a
 // fragment lie in different banks.  Now bound by the vector instructions of the
 // softmax beside the matrix cores, at two workgroups per CU.
