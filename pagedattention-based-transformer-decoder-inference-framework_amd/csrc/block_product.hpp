@@ -29,6 +29,8 @@ __device__ __forceinline__ TileAt xcd_tile(int id, int nx, int ny) {
 // alone; the barrier then makes them everyone's and frees the stage that was read
 // before.  The loads are spread among the matrix instructions: issued together they
 // hold up the wave while the matrix cores run dry.
+// The matrix instruction takes W as its first operand: a lane's sums are four neighbouring
+// columns, 4 (lane >> 4) on, of row 16 i + (lane & 15) of A.
 // W is packed, fragment after fragment (w_tile(t): the first of column tile t).  A is
 // packed alike (A_PACKED; a_at(t): the first fragment of row tile t) or row-major
 // (a_at(r): row r).  Row-major, a load takes 8 rows x 128 bytes, whole cache lines (16
@@ -111,7 +113,7 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
           }
       }
       const int i = t / NT, j = t % NT;
-      acc[i][j] = mma(f.a[i], f.c[j], acc[i][j]);
+      acc[i][j] = mma(f.c[j], f.a[i], acc[i][j]);
     }
   };
   Acc sum[PARTS ? MT : 1][PARTS ? NT : 1];
@@ -215,6 +217,27 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
 #pragma unroll
       for (int j = 0; j < NT; ++j) acc[i][j] += sum[i][j];
   }
+}
+
+// us of `groups` blocks of which a CU holds `per` at once: at[n - 1] with n on every CU,
+// launch included.  A round of workgroups follows the one before, the last one with as many
+// a CU as are left.
+inline float rounds_us(long long groups, int per, const float (&at)[3]) {
+  const long long all = 256LL * per, full = groups / all, left = groups % all;
+  return (float)full * at[per - 1] + (left ? at[(left + 255) / 256 - 1] : 0.f);
+}
+
+// A wave's sums into the block's LDS, row by row: row m0 + 16 i + .., column n0 + 16 j + .. of
+// rows of STRIDE (a multiple of 4, not of 64: 16 lanes' 16 bytes lie in different banks).  What
+// the wave then reads of its own rows and columns it need not wait for others for.
+template <int STRIDE, int MT, int NT, typename Acc, typename E>
+__device__ __forceinline__ void spread_sums(const Acc (&acc)[MT][NT], E* sums, int m0, int n0) {
+  E* to = sums + (m0 + (lane_id() & 15)) * STRIDE + n0 + 4 * (lane_id() >> 4);
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) *reinterpret_cast<Acc*>(to + 16 * i * STRIDE + 16 * j) = acc[i][j];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 }  // namespace llm

@@ -583,15 +583,17 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
 
 // Rows of a prompt: blocks of 16 MB rows x 16 NB columns through LDS
 // (block_product.hpp), compute-shaped where the kernel above is a weight stream.
-// int8, 2048 rows: x 6144 x 2048 with the KV append 71.5 us (177 as four streams of
-// 512 rows), x 8192 x 2048 63 (224), x 2048 x 2048 and x 2048 x 8192 31 on average
-// (91); bound as block_product, the append by its page stores besides.
-template <GemmKind KIND, bool A_PACKED, int MB, int NB, int WM, int WN, int ST>
+// int8, 2048 rows: x 6144 x 2048 with the KV append 53 us (pages through the block's LDS and
+// looked up between its stores: 73), x 8192 x 2048 57 (64), x 2048 x 2048 and x 2048 x 8192
+// 30 on average (31); bound by the stores of fp32 rows (the products alone of 2048 x 6144 x
+// 2048: 24 us, with their rows 41).
+// ROWS: fp32 rows alone; else pages or packed fp16 rows too.
+template <GemmKind KIND, bool A_PACKED, bool ROWS, int MB, int NB, int WM, int WN, int ST>
 __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_block_kernel(GemmArgs a) {
   using Tr = GemmTraits<KIND>;
   using acc_t = typename Tr::acc_t;
   using elem_t = typename Tr::elem_t;
-  constexpr int MT = MB / WM, NT = NB / WN, THREADS = 64 * WM * WN;
+  constexpr int MT = MB / WM, NT = NB / WN;
   __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
   const TileAt tile = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y);
   const int lane = lane_id(), w = wave_id_uniform(), wm = w / WN, wn = w % WN;
@@ -616,111 +618,89 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void gemm_block_kernel(GemmArgs a)
           return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x),
                                                         __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
       });
-  const auto finish = [&](elem_t s, float sa, float sw, float bias) {
-#pragma clang fp contract(off)  // y = acc * scale + bias rounded twice, as the reference
-    float y = (float)s;
-    if constexpr (KIND == GemmKind::I8) y = y * (sa * sw);
-    if (a.bias) y = y + bias;
-    return apply_act(y, a.act);
-  };
-  const bool rows_only = !a.kv.k_pool && !a.c16;
-  if (rows_only) {  // fp32 rows: 64 bytes of a line per store, straight from the accumulators
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const int first = m0 + 16 * (wm * MT + i) + 4 * (lane >> 4);
-      float sa[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sa[r] = KIND == GemmKind::I8 && a.sa ? a.sa[min(first + r, a.M - 1)] : 1.f;
-#pragma unroll
-      for (int j = 0; j < NT; ++j) {
-        const int n = (nt0 + wn * NT + j) * 16 + (lane & 15);
-        if (n >= a.N) continue;
-        const float sw = KIND == GemmKind::I8 && a.sw ? a.sw[n] : 1.f, bias = a.bias ? a.bias[n] : 0.f;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = first + r;
-          if (m >= a.M) continue;
-          if constexpr (KIND == GemmKind::I8)
-            if (a.acc_out) a.acc_out[(size_t)m * a.N + n] = acc[i][j][r];
-          if (a.C && n < a.c_cols) a.C[(size_t)m * a.c_ld + n] = finish(acc[i][j][r], sa[r], sw, bias);
-        }
-      }
-    }
-    return;
-  }
-  // Pages and packed fp16 rows: row by row through LDS (block_product has read it
-  // out), eight columns per thread, so that stores are 16 bytes and a page is looked
-  // up once for them.
-  constexpr int STRIDE = 16 * NB + 4;
-  static_assert(sizeof(lds) >= sizeof(elem_t) * 16 * MB * STRIDE);
+  // The wave's sums through LDS (block_product has read it out), so that stores are 16
+  // bytes a lane, lines of a row by neighbouring lanes, and a lane has one set of C columns,
+  // whose scale, bias and page are found once.  All that is loaded is loaded before the
+  // first store: a load behind stores is waited for together with them.
+  constexpr int STRIDE = 16 * NB + 4, C = ROWS ? 4 : 8, ACROSS = 16 * NT / C, STEP = 64 / ACROSS,
+                PER = 16 * MT / STEP;
+  static_assert(sizeof(lds) >= sizeof(elem_t) * 16 * MB * STRIDE && 64 % ACROSS == 0 && PER >= 1);
   elem_t* sums = reinterpret_cast<elem_t*>(&lds[0][0][0]);
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sums[(16 * (wm * MT + i) + 4 * (lane >> 4) + r) * STRIDE + 16 * (wn * NT + j) + (lane & 15)] =
-            acc[i][j][r];
-  __syncthreads();
-  constexpr int ACROSS = 2 * NB, STEP = THREADS / ACROSS, PER = 16 * MB / STEP, BATCH = PER < 4 ? PER : 4;
-  static_assert(THREADS % ACROSS == 0 && PER % BATCH == 0);
-  const int row0 = threadIdx.x / ACROSS, col0 = threadIdx.x % ACROSS * 8, n = nt0 * 16 + col0;
+  spread_sums<STRIDE>(acc, sums, 16 * wm * MT, 16 * wn * NT);
+  const int row0 = 16 * wm * MT + lane / ACROSS, col0 = 16 * wn * NT + lane % ACROSS * C;
+  const int m = m0 + row0, n = 16 * nt0 + col0;  // this lane's rows m + STEP i, columns n .. n + C - 1
   if (n >= a.N) return;  // (N is a multiple of 16)
+  sums += row0 * STRIDE + col0;
   const KvAppend& kv = a.kv;
-  const int hid = kv.H * kv.D, which = kv.k_pool && n >= hid ? n / hid : 0;  // 1: K, 2: V
+  const int hid = kv.H * kv.D;
+  const int which = !ROWS && kv.k_pool && n >= hid ? n / hid : 0;  // 1: K, 2: V
   const int head = which ? (n - which * hid) / kv.D : 0, d = which ? (n - which * hid) % kv.D : 0;
-  float sw[8], bias[8];
+  float sa[PER], sw[C], bias[C];
+  int pos[PER], page[PER];
 #pragma unroll
-  for (int k = 0; k < 8; ++k) {
+  for (int k = 0; k < C; ++k) {
     sw[k] = KIND == GemmKind::I8 && a.sw ? a.sw[n + k] : 1.f;
     bias[k] = a.bias ? a.bias[n + k] : 0.f;
   }
-#pragma unroll 1
-  for (int i0 = 0; i0 < PER; i0 += BATCH) {
-    int pos[BATCH], page[BATCH];
-    float sa[BATCH];
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
-      const int m = min(m0 + row0 + (i0 + i) * STEP, a.M - 1);
-      sa[i] = KIND == GemmKind::I8 && a.sa ? a.sa[m] : 1.f;
-      pos[i] = which ? kv.pos[m] : -1;
-      page[i] = which ? (kv.rows ? kv.rows[m] : m) : -1;  // the page-table row first
-    }
+  for (int i = 0; i < PER; ++i) {
+    const int r = min(m + STEP * i, a.M - 1);
+    sa[i] = KIND == GemmKind::I8 && a.sa ? a.sa[r] : 1.f;
+    pos[i] = which ? kv.pos[r] : -1;
+    page[i] = which ? (kv.rows ? kv.rows[r] : r) : -1;  // the page-table row first
+  }
+  if constexpr (!ROWS) {
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
+    for (int i = 0; i < PER; ++i) {
       const int row = page[i], t = pos[i] >= 0 ? pos[i] / kv.TS : 0;
       page[i] = -1;
       if (pos[i] >= 0 && row >= 0 && row < kv.num_beams && t < kv.max_tiles)
         page[i] = kv.page_table[((size_t)row * kv.H + head) * kv.max_tiles + t];
       if (page[i] >= kv.num_pages) page[i] = -1;
     }
+  }
+  const bool vec = ((a.c_ld | a.c_cols) & 3) == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
 #pragma unroll
-    for (int i = 0; i < BATCH; ++i) {
-      const int r = row0 + (i0 + i) * STEP, m = m0 + r;
-      if (m >= a.M) continue;
-      float y[8];
+  for (int i = 0; i < PER; ++i) {
+#pragma clang fp contract(off)  // y = acc * scale + bias rounded twice, as the reference
+    const int r = m + STEP * i;
+    if (r >= a.M) break;
+    float y[C];
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      const elem_t s = sums[i * STEP * STRIDE + k];
+      if constexpr (KIND == GemmKind::I8)
+        if (a.acc_out) a.acc_out[(size_t)r * a.N + n + k] = s;
+      y[k] = (float)s;
+      if constexpr (KIND == GemmKind::I8) y[k] = y[k] * (sa[i] * sw[k]);
+      if (a.bias) y[k] = y[k] + bias[k];
+      y[k] = apply_act(y[k], a.act);
+    }
+    if (a.C && n < a.c_cols) {
+      float* to = a.C + (size_t)r * a.c_ld + n;
+      if (vec && n + C <= a.c_cols) {
+#pragma unroll
+        for (int k = 0; k < C; k += 4) {
+          const f32x4 v = {y[k], y[k + 1], y[k + 2], y[k + 3]};
+          // int8 blocks are short, and written past L2 their rows come too thick
+          // (2048 x 12288 x 2048 66 us, past L2 70)
+          if constexpr (KIND == GemmKind::I8 || !ROWS) *reinterpret_cast<f32x4*>(to + k) = v;
+          else store_through(to + k, __builtin_bit_cast(u32x4, v));
+        }
+      } else {
+#pragma unroll
+        for (int k = 0; k < C; ++k)
+          if (n + k < a.c_cols) to[k] = y[k];
+      }
+    }
+    if constexpr (!ROWS) {
       f16x8 h;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const elem_t s = sums[r * STRIDE + col0 + k];
-        if constexpr (KIND == GemmKind::I8)
-          if (a.acc_out) a.acc_out[(size_t)m * a.N + n + k] = s;
-        y[k] = finish(s, sa[i], sw[k], bias[k]);
-        h[k] = (_Float16)y[k];
-      }
-      if (a.C) {
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (n + k < a.c_cols) a.C[(size_t)m * a.c_ld + n + k] = y[k];
-      }
-      if (a.c16) *reinterpret_cast<f16x8*>(a.c16 + a_frag_off_f16(m, n, a.N >> 5)) = h;
-      if (page[i] >= 0) {
-        _Float16* pool = which == 2 ? kv.v_pool : kv.k_pool;
-        *reinterpret_cast<f16x8*>(pool + (size_t)page[i] * kv.page_stride +
-                                  (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
-      }
+      for (int k = 0; k < 8; ++k) h[k] = (_Float16)y[k];
+      if (a.c16) *reinterpret_cast<f16x8*>(a.c16 + a_frag_off_f16(r, n, a.N >> 5)) = h;
+      if (page[i] >= 0)
+        *reinterpret_cast<f16x8*>((which == 2 ? kv.v_pool : kv.k_pool) +
+                                  (size_t)page[i] * kv.page_stride + (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
     }
   }
 }
@@ -878,31 +858,36 @@ inline bool narrow_decode_tile(const GemmArgs& a, int kstep, TileChoice& t) {
   return narrow_tile_for(a.M, a.N, a.KS * kstep, t);
 }
 
-// The block form with the least rounds of workgroups x time of a round (us at 32
-// k-steps, launch taken off).
-template <GemmKind KIND, bool A_PACKED>
+// The block form whose rounds of workgroups take least; us of a round at K = 2048 with one,
+// two and three blocks a CU (mm_impl.hpp's forms, int8's by times of their own).
+template <GemmKind KIND, bool A_PACKED, bool ROWS>
 hipError_t launch_gemm_block(const GemmArgs& a, hipStream_t st) {
-  struct Form {
-    int mb, nb, threads;
-    float round;
-    void (*kernel)(GemmArgs);
-  };
-  static constexpr Form forms[] = {{4, 4, 256, 6.2f, gemm_block_kernel<KIND, A_PACKED, 4, 4, 2, 2, 3>},
-                                   {4, 8, 512, 10.f, gemm_block_kernel<KIND, A_PACKED, 4, 8, 2, 4, 4>},
-                                   {8, 8, 512, 18.5f, gemm_block_kernel<KIND, A_PACKED, 8, 8, 4, 2, 3>},
-                                   {8, 16, 512, 27.f, gemm_block_kernel<KIND, A_PACKED, 8, 16, 2, 4, 3>}};
-  const Form* best = nullptr;
+  void (*best)(GemmArgs) = nullptr;
   dim3 grid;
+  int threads = 0;
   float least = 0.f;
-  for (const Form& f : forms) {
-    const dim3 g((a.N + 16 * f.nb - 1) / (16 * f.nb), (a.M + 16 * f.mb - 1) / (16 * f.mb));
-    const float cost = (float)((g.x * g.y + 255) / 256) * f.round;
-    if (best && cost >= least) continue;
-    best = &f;
+  const auto consider = [&](int mb, int nb, int waves, int per, const float (&at)[3], void (*kernel)(GemmArgs)) {
+    const dim3 g((a.N + 16 * nb - 1) / (16 * nb), (a.M + 16 * mb - 1) / (16 * mb));
+    const float cost = rounds_us((long long)g.x * g.y, per, at);
+    if (best && cost >= least) return;
+    best = kernel;
     grid = g;
+    threads = 64 * waves;
     least = cost;
+  };
+  if constexpr (KIND == GemmKind::I8) {
+    consider(4, 4, 4, 3, {9.f, 10.7f, 14.f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 4, 2, 2, 3>);
+    consider(4, 8, 8, 1, {9.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 4>);
+    consider(4, 8, 8, 2, {9.7f, 14.4f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 3>);
+    consider(8, 8, 8, 1, {13.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 8, 4, 2, 3>);
+    consider(8, 16, 8, 1, {21.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 16, 2, 4, 3>);
+  } else {
+    consider(4, 8, 8, 1, {12.1f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 4>);
+    consider(4, 8, 8, 2, {12.6f, 20.1f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 3>);
+    consider(8, 8, 8, 1, {17.6f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 8, 4, 2, 3>);
+    consider(8, 16, 8, 1, {28.f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 16, 2, 4, 3>);
   }
-  hipLaunchKernelGGL(best->kernel, grid, dim3(best->threads), 0, st, a);
+  hipLaunchKernelGGL(best, grid, dim3(threads), 0, st, a);
   return hipGetLastError();
 }
 
@@ -916,7 +901,12 @@ hipError_t launch_gemm(const GemmArgs& a_in, hipStream_t st, int nt_override = 0
       !a.ksplit2 && !a.stamps && reinterpret_cast<uintptr_t>(a.A) % 16 == 0 &&
       (!a.kv.k_pool || a.kv.D % 8 == 0) &&
       nt_override + waves_override + mrows_override + ks_override == 0)
-    return a.a_packed ? launch_gemm_block<KIND, true>(a, st) : launch_gemm_block<KIND, false>(a, st);
+  {
+    const bool rows = !a.kv.k_pool && !a.c16;
+    if (a.a_packed)
+      return rows ? launch_gemm_block<KIND, true, true>(a, st) : launch_gemm_block<KIND, true, false>(a, st);
+    return rows ? launch_gemm_block<KIND, false, true>(a, st) : launch_gemm_block<KIND, false, false>(a, st);
+  }
   TileChoice tc{0, 0, 0};
   const bool narrow = nt_override == 0 && waves_override == 0 && mrows_override == 0 &&
                       narrow_decode_tile(a, GemmTraits<KIND>::KSTEP, tc);

@@ -69,10 +69,19 @@ struct KernelArgs {
   const float* bias;
 };
 
+// fp32 results take expf and the division; bf16 ones the hardware's 2^x and 1 / x, off by some
+// 1e-7 and at most 1e-6 where the exponent is large (the rounding to bf16: 4e-3): a vector
+// instruction takes a SIMD 4 cycles, a pair was 60 of them and is 25 (2048 x 12288 x 2048 of
+// blocks 95 -> 86 us, the results past L2 in the same step).  e^-alpha g past 2^120 leaves
+// nothing of any g.
+template <typename T>
 __device__ __forceinline__ float glu(float gate, float up, const GluParams& p) {
   const float g = fminf(gate, p.limit);
   const float u = fminf(fmaxf(up, -p.limit), p.limit);
-  return g / (1.f + expf(-p.alpha * g)) * (u + p.up_bias);
+  if constexpr (!Kind<T>::BF16) return g / (1.f + expf(-p.alpha * g)) * (u + p.up_bias);
+  const float a = -p.alpha * g, t = fminf(a * kLog2e, 120.f);
+  const float d = 1.f + __builtin_amdgcn_exp2f(t), r = __builtin_amdgcn_rcpf(d);
+  return g * r * (u + p.up_bias);
 }
 
 // log(1 + e^v) = max(v, 0) + log1p(e), e = e^-|v|; log1p(e) = 2 atanh(s) with
@@ -205,6 +214,21 @@ struct RowOf {
       at = pos % kPageTokens;
       entry = tile < e.max_tiles ? e.slot[m] * e.G * e.max_tiles + tile : -1;
     }
+  }
+  // of lane l
+  __device__ __forceinline__ RowOf from(int l) const {
+    RowOf r;
+    r.m = __shfl(m, l, 64);
+    if constexpr (PAGED) {
+      r.at = __shfl(at, l, 64);
+      r.entry = __shfl(entry, l, 64);
+      r.pos = __shfl(pos, l, 64);
+    }
+    if constexpr (EPI == kGroupOut) {
+      r.out = __shfl(out, l, 64);
+      r.weight = __shfl(weight, l, 64);
+    }
+    return r;
   }
   // kGroupOut.  The stream kernel's rows do it in Target::find, behind one branch with the
   // rest: behind one of its own the compiler waits for the weight, and so for the first
@@ -375,7 +399,7 @@ struct Target {
       if (p0) *static_cast<float*>(p0) = v0;
       if (p1) *static_cast<float*>(p1) = v1;
     } else if constexpr (EPI == kGroupIn || EPI == kGlu) {
-      if (p0) *static_cast<T*>(p0) = (T)glu(v0, v1, b.glu);
+      if (p0) *static_cast<T*>(p0) = (T)glu<T>(v0, v1, b.glu);
     } else if constexpr (EPI == kSplit) {
       if (!p0) return;
       if (n < p.split.n_t) put_pair(static_cast<T*>(p0), v0, v1);
@@ -441,42 +465,6 @@ struct Target {
   }
 };
 
-// 16 MT rows from m0 on and 16 NT columns from n0 on, straight from the accumulators,
-// a column pair per lane: 64 bytes of a line per store, enough for fp32 results.
-// Every lane of the wave takes part.
-template <typename T, int EPI, int MT, int NT>
-__device__ __forceinline__ void emit_pairs(const KernelArgs& p, const Block<T>& b,
-                                           const f32x4 (&acc)[MT][NT], int m0, int n0) {
-  const int lane = lane_id(), first = m0 + 4 * (lane >> 4) + (lane & 1 ? 2 : 0);
-  const bool odd = lane & 1;
-  RowOf<EPI> rows[MT][2];
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-      rows[i][r] = RowOf<EPI>(p, b, first + 16 * i + r);
-      if (rows[i][r].m >= 0) rows[i][r].look_up(p, b);
-    }
-#pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int n = n0 + 16 * j + (lane & 14);
-    const ColOf<EPI> col(p, b, n);
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-      const f32x4 c = acc[i][j];
-      f32x4 o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = mov_dpp<0xB1>(c[r]);  // the neighbouring column
-#pragma unroll
-      for (int r = 0; r < 2; ++r) {
-        Target<T, EPI> t;
-        t.template find<true>(p, b, rows[i][r], col);
-        t.put(p, b, n, odd ? o[2 + r] : c[r], odd ? c[2 + r] : o[r]);
-      }
-    }
-  }
-}
-
 template <typename T>
 __device__ __forceinline__ void put_eight(T* p, const float (&v)[8]) {
   constexpr int E = 16 / sizeof(T);
@@ -486,8 +474,19 @@ __device__ __forceinline__ void put_eight(T* p, const float (&v)[8]) {
     chunk_t o;
 #pragma unroll
     for (int e = 0; e < E; ++e) o[e] = (T)v[k + e];
-    *reinterpret_cast<chunk_t*>(p + k) = o;
+    // half of fp32's 32 bytes at a time would reach memory as parts of lines
+    if constexpr (E == 8) store_through(p + k, __builtin_bit_cast(u32x4, o));
+    else *reinterpret_cast<chunk_t*>(p + k) = o;
   }
+}
+template <typename T>
+__device__ __forceinline__ void put_four(T* p, f32x4 v) {
+  typedef T four_t __attribute__((ext_vector_type(4)));
+  four_t o;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) o[k] = (T)v[k];
+  if constexpr (sizeof(T) == 2) store_through(p, __builtin_bit_cast(u32x2, o));
+  else store_through(p, __builtin_bit_cast(u32x4, o));
 }
 // rows of ld elements that all start at 16 bytes
 template <typename T>
@@ -519,6 +518,11 @@ struct Eight {
     } else if constexpr (EPI == kGlu) {
       ok = ok && whole<T>(p.split.t, p.split.ldt);
       p0 = static_cast<T*>(p.split.t) + (size_t)m * p.split.ldt + (n >> 1);
+    } else if constexpr (EPI == kHeads) {
+      const MmHeads& e = p.heads;
+      ok = ok && whole<T>(e.C, e.ldc) && whole<T>(nullptr, e.c_head);
+      const int row = e.rows ? e.rows[m] : m;
+      p0 = static_cast<T*>(e.C) + (size_t)row * e.ldc + (size_t)blockIdx.z * e.c_head + n;
     } else if constexpr (EPI == kLatent) {
       const MmLatent& e = p.lat;
       ok = ok && ((e.D | e.rot) & 7) == 0 && whole<T>(e.q, e.ldq) && whole<float>(e.down, e.ldd);
@@ -553,8 +557,10 @@ struct Eight {
       typedef T half_t __attribute__((ext_vector_type(4)));
       half_t o;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = (T)glu(v[2 * k], v[2 * k + 1], b.glu);
+      for (int k = 0; k < 4; ++k) o[k] = (T)glu<T>(v[2 * k], v[2 * k + 1], b.glu);
       *static_cast<half_t*>(p0) = o;
+    } else if constexpr (EPI == kHeads) {
+      if (p0) put_eight(static_cast<T*>(p0), v);
     } else if constexpr (EPI == kLatent) {
       if (!p0) {
         if (p1) put_eight(static_cast<float*>(p1), v);
@@ -587,125 +593,258 @@ struct Eight {
   }
 };
 
+// Rows of a block that begin a sequence's: found before the product, for the value columns.
+template <int ROWS>
+struct Starts {
+  unsigned long long at[ROWS / 64];
+  int rows = 0, sequences = 0;
+
+  template <typename T>
+  __device__ __forceinline__ Starts(const MmQkv& e, const Block<T>& b) {
+    rows = min(ROWS, b.M - b.m0);
+#pragma unroll
+    for (int h = 0; h < ROWS / 64; ++h) {
+      const int r = 64 * h + lane_id();
+      at[h] = __ballot(r < rows && (r == 0 || e.slot[b.m0 + r] != e.slot[b.m0 + r - 1]));
+      sequences += __popcll(at[h]);
+    }
+  }
+};
+
+struct NoStarts {
+  template <typename T>
+  __device__ __forceinline__ NoStarts(const MmQkv&, const Block<T>&) {}
+};
+
 // Value columns [c0, c1) of a block's sums: they lie token by token in their pages.
 // Rows of a few sequences: four tokens of a page that lie together are one store,
-// sixteen lanes a page's line.  Rows of many: a row per thread, so that its page is
-// looked up once for the columns it takes.
-template <typename T, int EPI, int ROWS, int STRIDE, int THREADS>
+// sixteen lanes a page's line.  A thread's tokens stay the same over its columns, whose pages
+// are looked up together and before the stores: one by one, each look-up waited for the
+// store before it (2011 x 4096 x 512, half of it values: 37 us, now 29.5).
+// Rows of many: a row per thread, so that its page is looked up once for the columns it takes.
+template <typename T, int EPI, int ROWS, int COLS, int STRIDE, int THREADS>
 __device__ __forceinline__ void emit_values(const KernelArgs& p, const Block<T>& b, const float* sums,
-                                            int first_col, int c0, int c1) {
+                                            const Starts<ROWS>& starts, int first_col, int c0, int c1) {
   const MmQkv& e = p.q;
-  const int rows = min(ROWS, b.M - b.m0);
-  if (rows <= 0 || c0 >= c1) return;
-  unsigned long long starts[ROWS / 64];  // rows that begin a sequence's
-  int sequences = 0;
-#pragma unroll
-  for (int h = 0; h < ROWS / 64; ++h) {
-    const int r = 64 * h + lane_id();
-    starts[h] = __ballot(r < rows && (r == 0 || e.slot[b.m0 + r] != e.slot[b.m0 + r - 1]));
-    sequences += __popcll(starts[h]);
-  }
-  const auto put = [&](const RowOf<EPI>& row, int r, int col) {
-    if (row.m < 0 || row.entry < 0) return;
-    const ColOf<EPI> c(p, b, col);
-    T* page = page_at<T>(e, e.v_pool, row.entry, c.head);
-    if (page)
-      page[(size_t)c.d * kPageTokens + v_page_slot(row.at, Kind<T>::BF16)] =
-          (T)sums[r * STRIDE + col - first_col];
-  };
-  if (sequences > 4) {
+  if (starts.rows <= 0 || c0 >= c1) return;
+  if (starts.sequences > 4) {
     const int r = threadIdx.x % ROWS;
     const RowOf<EPI> row(p, b, b.m0 + r);
+    if (row.m < 0 || row.entry < 0) return;
 #pragma unroll 4
-    for (int col = c0 + threadIdx.x / ROWS; col < c1; col += THREADS / ROWS) put(row, r, col);
+    for (int col = c0 + threadIdx.x / ROWS; col < c1; col += THREADS / ROWS) {
+      const ColOf<EPI> c(p, b, col);
+      T* page = page_at<T>(e, e.v_pool, row.entry, c.head);
+      if (page)
+        page[(size_t)c.d * kPageTokens + v_page_slot(row.at, Kind<T>::BF16)] =
+            (T)sums[r * STRIDE + col - first_col];
+    }
     return;
   }
   typedef T quad_t __attribute__((ext_vector_type(4)));
+  constexpr int ACROSS = THREADS / 16, PER = COLS / ACROSS;
+  static_assert(COLS % ACROSS == 0);
 #pragma unroll
   for (int h = 0; h < ROWS / 64; ++h) {
-    for (unsigned long long left = starts[h]; left; left &= left - 1) {
+    for (unsigned long long left = starts.at[h]; left; left &= left - 1) {
       const int s0 = 64 * h + __ffsll(left) - 1;  // the sequence's rows: [s0, s1)
       const unsigned long long after = left & (left - 1);
-      int s1 = after ? 64 * h + __ffsll(after) - 1 : rows;
-      if (!after && h + 1 < ROWS / 64 && starts[ROWS / 64 - 1]) s1 = 64 * (h + 1) + __ffsll(starts[ROWS / 64 - 1]) - 1;
+      int s1 = after ? 64 * h + __ffsll(after) - 1 : starts.rows;
+      if (!after && h + 1 < ROWS / 64 && starts.at[ROWS / 64 - 1])
+        s1 = 64 * (h + 1) + __ffsll(starts.at[ROWS / 64 - 1]) - 1;
       const int pos0 = e.pos[b.m0 + s0], slot = e.slot[b.m0 + s0], off = pos0 & 3;
-      const int chunks = ((off + s1 - s0 + 3) / 4 + 15) / 16;  // of sixteen quads
-      for (int i = threadIdx.x; i < (c1 - c0) * chunks * 16; i += THREADS) {
-        const int rest = i >> 4, col = c0 + rest / chunks;
-        const int r0 = s0 + 4 * (16 * (rest % chunks) + (i & 15)) - off;
-        if (r0 >= s1) continue;
+      for (int r0 = s0 + 4 * (threadIdx.x & 15) - off; r0 - 4 * (int)(threadIdx.x & 15) < s1; r0 += 64) {
         const int pos = pos0 + r0 - s0, tile = pos / kPageTokens;
-        if (tile >= e.max_tiles) continue;
-        const ColOf<EPI> c(p, b, col);
-        T* page = page_at<T>(e, e.v_pool, slot * e.G * e.max_tiles + tile, c.head);
-        if (!page) continue;
-        const float* v = sums + r0 * STRIDE + (col - first_col);
-        T* to = page + (size_t)c.d * kPageTokens + v_page_slot(pos % kPageTokens, Kind<T>::BF16);
-        if (r0 >= s0 && r0 + 4 <= s1) {
-          quad_t o;
+        const bool here = r0 < s1 && tile < e.max_tiles;
+        T* to[PER];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) o[k] = (T)v[k * STRIDE];
-          *reinterpret_cast<quad_t*>(to) = o;
-        } else {
+        for (int j = 0; j < PER; ++j) {
+          const int col = c0 + threadIdx.x / 16 + j * ACROSS;
+          to[j] = nullptr;
+          if (!here || col >= c1) continue;
+          const ColOf<EPI> c(p, b, col);
+          T* page = page_at<T>(e, e.v_pool, slot * e.G * e.max_tiles + tile, c.head);
+          if (page) to[j] = page + (size_t)c.d * kPageTokens + v_page_slot(pos % kPageTokens, Kind<T>::BF16);
+        }
 #pragma unroll
-          for (int k = 0; k < 4; ++k)
-            if (r0 + k >= s0 && r0 + k < s1) to[k] = (T)v[k * STRIDE];
+        for (int j = 0; j < PER; ++j) {
+          if (!to[j]) continue;
+          const float* v = sums + r0 * STRIDE + (c0 + (int)threadIdx.x / 16 + j * ACROSS - first_col);
+          if (r0 >= s0 && r0 + 4 <= s1) {
+            quad_t o;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) o[k] = (T)v[k * STRIDE];
+            *reinterpret_cast<quad_t*>(to[j]) = o;
+          } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+              if (r0 + k >= s0 && r0 + k < s1) to[j][k] = (T)v[k * STRIDE];
+          }
         }
       }
     }
   }
 }
 
-// A block's finished sums, row by row in LDS -> the epilogue, eight columns of a row
-// per thread, so that stores are whole lines and a page or a head is looked up once
-// for eight columns (straight from the accumulators, a pair of columns per lane and
-// 16 to 32 bytes of a line per store: expansion of 2011 x 4096 x 512 58 us, now 36;
-// latent projections of 2011 x 3648 x 2048 45 us, now 37).
-template <typename T, int EPI, int ROWS, int COLS, int STRIDE, int THREADS>
-__device__ __forceinline__ void emit_block(const KernelArgs& p, const Block<T>& b, const float* sums,
-                                           int first_col) {
-  constexpr int ACROSS = COLS / 8, PER = ROWS * ACROSS / THREADS, BATCH = PER < 4 ? PER : 4;
-  static_assert(THREADS % ACROSS == 0 && PER >= 1 && PER % BATCH == 0);
-  const int row0 = threadIdx.x / ACROSS, col0 = threadIdx.x % ACROSS * 8, n = first_col + col0;
-  int end = b.N;  // of the columns that go by rows
+// Columns of a row that a thread finishes: 16 bytes of fp32 or of the element type, which
+// sixteen of (gate, up) make; pairs where a channel's history comes along.
+template <int EPI>
+constexpr int columns_each(int rows, int cols) {
+  return EPI == kConv ? 2
+         : EPI == kStore || EPI == kGroupOut || EPI == kSoftplus || EPI == kSplit ? 4
+         : (EPI == kGroupIn || EPI == kGlu) && 1024 / cols <= rows ? 16
+                                                                    : 8;
+}
+
+// A wave's ROWS x COLS finished sums, row by row in LDS -> the epilogue.  Stores are whole
+// lines of a row, 64 columns of it by neighbouring lanes (straight from the accumulators a
+// pair of columns a lane: bf16 2048 x 12288 x 2048 with fp32 results 101.5 us, now 95;
+// gate and up with their activation 103, now 86; the products alone 77), and a thread's rows
+// have one set of columns, whose bias, head and place are found once.  All that is loaded
+// is loaded before the first store: a load behind stores is waited for together with them.
+template <typename T, int EPI, int ROWS, int COLS, int STRIDE>
+__device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b, const float* sums,
+                                          const RowOf<EPI>& row, int m0, int n0) {
+  constexpr int E = columns_each<EPI>(ROWS, COLS), ACROSS = COLS / E, STEP = 64 / ACROSS, PER = ROWS / STEP;
+  static_assert(64 % ACROSS == 0 && PER >= 1);
+  const int lane = lane_id(), r0 = lane / ACROSS, c0 = lane % ACROSS * E, n = n0 + c0;
+  int end = b.N;  // of the columns that go by rows; the others are values
   if constexpr (RowOf<EPI>::PAGED) end = min(b.N, (p.q.H + p.q.G) * p.q.D);
-  if (n < end) {
+  RowOf<EPI> r[EPI == kConv ? 1 : PER];
+  if constexpr (EPI != kConv) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) r[i] = row.from(r0 + i * STEP);
+  }
+  if (n >= end) return;
+  sums += r0 * STRIDE + c0;
+  if constexpr (EPI == kConv) {
+    constexpr int BATCH = PER < 4 ? PER : 4;
     const ColOf<EPI> c(p, b, n);
 #pragma unroll 1
     for (int i0 = 0; i0 < PER; i0 += BATCH) {
-      RowOf<EPI> r[BATCH];
-      Eight<T, EPI> t[BATCH];
+      Target<T, EPI> t[BATCH];
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) r[i] = RowOf<EPI>(p, b, b.m0 + row0 + (i0 + i) * (THREADS / ACROSS));
-#pragma unroll
-      for (int i = 0; i < BATCH; ++i) t[i].find(p, b, r[i], c);
+      for (int i = 0; i < BATCH; ++i) t[i].find(p, b, RowOf<EPI>(p, b, m0 + r0 + (i0 + i) * STEP), c);
 #pragma unroll
       for (int i = 0; i < BATCH; ++i) {
-        if (r[i].m < 0) continue;
-        float v[8];
-        const float* s = sums + (size_t)(row0 + (i0 + i) * (THREADS / ACROSS)) * STRIDE + col0;
+        const float* s = sums + (i0 + i) * STEP * STRIDE;
+        t[i].put(p, b, n, s[0], s[1]);
+      }
+    }
+    return;
+  }
+  if constexpr (EPI == kSplit) {
+    const MmSplit& e = p.split;
+    const bool left = n < e.n_t, four = (e.n_t & 3) == 0 && n + 4 <= b.N;
+    const bool vec = four && (left ? ((reinterpret_cast<uintptr_t>(e.t) | e.ldt * sizeof(T)) &
+                                      (4 * sizeof(T) - 1)) == 0
+                                   : whole<float>(e.f, e.ldf));
 #pragma unroll
-        for (int k = 0; k < 8; k += 4) {
-          const f32x4 x = *reinterpret_cast<const f32x4*>(s + k);
+    for (int i = 0; i < PER; ++i) {
+      const int m = r[i].m;
+      if (m < 0) continue;
+      const f32x4 v = *reinterpret_cast<const f32x4*>(sums + i * STEP * STRIDE);
+      T* t = static_cast<T*>(e.t) + (size_t)m * e.ldt + n;
+      float* f = e.f + (size_t)m * e.ldf + (n - e.n_t);
+      if (!vec) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[k + e] = x[e];
+        for (int k = 0; k < 4; ++k) {
+          if (n + k >= b.N) break;
+          if (n + k < e.n_t) t[k] = (T)v[k];
+          else f[k] = v[k];
         }
-        if (t[i].ok) {
-          t[i].put(p, b, n, v);
-        } else {
+      } else if (!left) {
+        store_through(f, __builtin_bit_cast(u32x4, v));
+      } else {
+        put_four(t, v);
+      }
+    }
+  } else if constexpr (E == 4) {
+    float* C = EPI == kGroupOut ? p.g.out : p.a.C;
+    const size_t ldc = EPI == kGroupOut ? p.g.ldo : p.a.ldc;
+    const bool vec = whole<float>(C, ldc) && n + 4 <= b.N;
+    float bias[4];
+    if constexpr (EPI == kSoftplus)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) bias[k] = p.bias[min(n + k, b.N - 1)];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (r[i].m < 0) continue;
+      f32x4 v = *reinterpret_cast<const f32x4*>(sums + i * STEP * STRIDE);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if constexpr (EPI == kGroupOut) v[k] *= r[i].weight;
+        else if constexpr (EPI == kSoftplus) v[k] = softplus(v[k] + bias[k]);
+        else if (p.a.softcap > 0.f) v[k] = p.a.softcap * tanhf(v[k] / p.a.softcap);
+      }
+      float* to = C + (EPI == kGroupOut ? r[i].out : r[i].m) * ldc + n;
+      if (vec) {
+        store_through(to, __builtin_bit_cast(u32x4, v));
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (n + k < b.N) to[k] = v[k];
+      }
+    }
+  } else if constexpr (E == 16) {  // gate and up
+    const size_t ld = EPI == kGlu ? p.split.ldt : b.shared ? p.g.lds : p.g.lda;
+    T* act = static_cast<T*>(EPI == kGlu ? p.split.t : b.shared ? p.g.act_shared : p.g.act);
+    const bool vec = whole<T>(act, ld) && n + 16 <= b.N;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (r[i].m < 0) continue;
+      T* to = act + r[i].m * ld + (n >> 1);
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(sums + i * STEP * STRIDE + 2 * k);
+        v[k] = glu<T>(x[0], x[1], b.glu);
+        v[k + 1] = glu<T>(x[2], x[3], b.glu);
+      }
+      if (vec) {
+        put_eight(to, v);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (n + 2 * k < b.N) to[k] = (T)v[k];
+      }
+    }
+  } else {
+    const ColOf<EPI> c(p, b, n);
+    Eight<T, EPI> t[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) t[i].find(p, b, r[i], c);
+    bool rest = false;  // rows that go pair by pair
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (r[i].m < 0) continue;
+      const float* s = sums + i * STEP * STRIDE;
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; k += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(s + k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[k + e] = x[e];
+      }
+      if (t[i].ok) t[i].put(p, b, n, v);
+      else rest = true;
+    }
+    if (!rest) return;
 #pragma unroll 1
-          for (int k = 0; k < 8 && n + k < end; k += 2) {
-            Target<T, EPI> g;
-            g.find(p, b, r[i], ColOf<EPI>(p, b, n + k));
-            g.put(p, b, n + k, s[k], s[k + 1]);
-          }
-        }
+    for (int i = 0; i < PER; ++i) {
+      const RowOf<EPI> at(p, b, m0 + r0 + i * STEP);
+      Eight<T, EPI> e;
+      e.find(p, b, at, c);
+      if (at.m < 0 || e.ok) continue;
+      const float* s = sums + i * STEP * STRIDE;
+#pragma unroll 1
+      for (int k = 0; k < 8 && n + k < end; k += 2) {
+        Target<T, EPI> g;
+        g.find(p, b, at, ColOf<EPI>(p, b, n + k));
+        g.put(p, b, n + k, s[k], s[k + 1]);
       }
     }
   }
-  if constexpr (RowOf<EPI>::PAGED)
-    emit_values<T, EPI, ROWS, STRIDE, THREADS>(p, b, sums, first_col, max(first_col, end),
-                                               min(first_col + COLS, b.N));
 }
 
 // Decode rows (and short grouped tiles): a block owns 16 MT rows x 16 NT columns
@@ -828,7 +967,7 @@ __host__ __device__ __forceinline__ int group_across(int n, int NB) { return (n 
 // A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).
 template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
 __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p) {
-  constexpr int WAVES = WM * WN, MT = MB / WM, NT = NB / WN;
+  constexpr int MT = MB / WM, NT = NB / WN;
   __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
   int id = blockIdx.y * gridDim.x + blockIdx.x;
   TileAt tile;
@@ -855,32 +994,28 @@ __global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p)
   const int ntiles = (b.N + 15) >> 4;
   const int nt0 = tile.x * NB, KS = b.KS;
   const int wm = w / WN, wn = w % WN;
+  const int m0 = 16 * wm * MT, n0 = 16 * wn * NT;
+  RowOf<EPI> row(p, b, b.m0 + m0 + lane % (16 * MT));
+  if (row.m >= 0) row.look_up(p, b);
+  std::conditional_t<RowOf<EPI>::PAGED, Starts<16 * MB>, NoStarts> starts(p.q, b);
   f32x4 acc[MT][NT];
   block_product<false, !Kind<T>::BF16, MB, NB, WM, WN, ST>(
       lds, acc, KS, b.m0 + 16 * wm * MT < b.M,
       [&](int r) { return a_row<T, EPI>(p, b, b.m0 + r); },
       [&](int t) { return b.W + (size_t)min(nt0 + t, ntiles - 1) * KS * 1024; },
       [](u32x4 x, u32x4 y, f32x4 c) { return Kind<T>::mma(x, y, c); });
-  // 2048 x 12288 x 2048 with its activation 107 us by rows, 109 by pairs; 2011 x 8192
-  // split 80 and 77
-  constexpr bool BY_ROWS = EPI == kGroupIn || EPI == kGlu || EPI == kLatent || RowOf<EPI>::PAGED;
-  if constexpr (!BY_ROWS) {
-    emit_pairs<T, EPI>(p, b, acc, b.m0 + 16 * wm * MT, (nt0 + wn * NT) * 16);
-    return;
-  }
   // (block_product has read all of LDS before its last barrier)
   constexpr int STRIDE = 16 * NB + 4;
   static_assert(sizeof(lds) >= sizeof(float) * 16 * MB * STRIDE);
   float* sums = reinterpret_cast<float*>(&lds[0][0][0]);
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sums[(16 * (wm * MT + i) + 4 * (lane >> 4) + r) * STRIDE + 16 * (wn * NT + j) + (lane & 15)] = acc[i][j][r];
-  __syncthreads();
-  emit_block<T, EPI, 16 * MB, 16 * NB, STRIDE, 64 * WAVES>(p, b, sums, 16 * nt0);
+  spread_sums<STRIDE>(acc, sums, m0, n0);
+  emit_wave<T, EPI, 16 * MT, 16 * NT, STRIDE>(p, b, sums + m0 * STRIDE + n0, row, b.m0 + m0, 16 * nt0 + n0);
+  if constexpr (RowOf<EPI>::PAGED) {
+    const int first = max(16 * nt0, (p.q.H + p.q.G) * p.q.D), last = min(16 * (nt0 + NB), b.N);
+    if (first >= last) return;
+    __syncthreads();
+    emit_values<T, EPI, 16 * MB, 16 * NB, STRIDE, 64 * WM * WN>(p, b, sums, starts, 16 * nt0, first, last);
+  }
 }
 
 template <int EPI>
@@ -906,28 +1041,32 @@ hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
   return hipGetLastError();
 }
 
-// A block form and the time of one round of its workgroups over the chip at K =
-// 2048, launch taken off (us).  A product takes the form with the least rounds x time:
-// 2048 x 12288: 3 rounds of 128 x 256, 101 us (128 x 128: 115); 2048 x 2048: one round
-// of 128 x 128, 21.5 us (128 x 256 leaves half the chip idle: 33); 700 x 2048: 64 x 128,
-// 12.2 us (128 x 128: 23); 64 x 12288: 64 x 64, 11.0 us (64 x 32: 13).  fp32 blocks are
+// A block form, the blocks of it a CU holds (by their LDS), and the time of a round of them at
+// K = 2048 with one, two and three a CU (us, weights from memory).  A product takes the form
+// whose rounds take least.  Two blocks of 64 x 128 a CU hide each other's first loads and last
+// stores, so there are two depths of them: 2048 x 2560 28.7 us (four stages, one a CU: 33.8),
+// 1000 x 2048 12.3 (three stages: 13.2).  2048 x 12288: 3 rounds of 128 x 256, 83 us with the
+// activation (128 x 128: 110); 2048 x 2048: one round of 128 x 128, 17.1 us (128 x 256 leaves
+// half the chip idle: 26.4); 700 x 2048: 64 x 128, 12.0 us (128 x 128: 17.3).  fp32 blocks are
 // bound by the matrix cores and take the time of their area, the small ones, of which a CU
 // holds several, the time between two rounds: 2048 x 2048: two rounds of 64 x 128, 140 us
 // (128 x 128: 158); 700 x 6144: five of 64 x 64, 185 us (64 x 128: 207); K only scales all.
 template <typename T, int EPI>
 struct BlockForm {
-  int mb, nb;
-  float bf16, fp32;
+  int mb, nb, per;
+  float bf16[3], fp32;
   hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
 };
 template <typename T, int EPI>
 hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipStream_t st) {
-  static constexpr BlockForm<T, EPI> forms[] = {{4, 2, 4.2f, 21.5f, blocks<T, EPI, 4, 2, 2, 2, 4>},
-                                                {4, 4, 6.2f, 37.f, blocks<T, EPI, 4, 4, 2, 2, 3>},
-                                                {4, 8, 10.f, 70.f, blocks<T, EPI, 4, 8, 2, 4, 4>},
-                                                {4, 16, 19.5f, 160.f, blocks<T, EPI, 4, 16, 2, 4, 3>},
-                                                {8, 8, 18.5f, 156.f, blocks<T, EPI, 8, 8, 4, 2, 3>},
-                                                {8, 16, 30.f, 293.f, blocks<T, EPI, 8, 16, 2, 4, 3>}};
+  static constexpr BlockForm<T, EPI> forms[] = {
+      {4, 2, 3, {10.8f, 12.1f, 15.6f}, 21.5f, blocks<T, EPI, 4, 2, 4, 1, 4>},
+      {4, 4, 3, {13.3f, 15.4f, 20.4f}, 37.f, blocks<T, EPI, 4, 4, 2, 2, 3>},
+      {4, 8, 1, {12.1f}, 70.f, blocks<T, EPI, 4, 8, 2, 4, 4>},
+      {4, 8, 2, {12.6f, 20.1f}, 1e9f, blocks<T, EPI, 4, 8, 2, 4, 3>},
+      {4, 16, 1, {18.7f}, 160.f, blocks<T, EPI, 4, 16, 2, 4, 3>},
+      {8, 8, 1, {17.6f}, 156.f, blocks<T, EPI, 8, 8, 4, 2, 3>},
+      {8, 16, 1, {28.f}, 293.f, blocks<T, EPI, 8, 16, 2, 4, 3>}};
   const BlockForm<T, EPI>* best = nullptr;
   int best_y = 0;
   float least = 0.f;
@@ -938,7 +1077,7 @@ hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipS
     if constexpr (EPI == kGroupIn || EPI == kGroupOut)
       groups = (p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, f.nb) +
                p.g.shared_tiles * group_across(p.g.shared_n, f.nb);
-    const float cost = (float)((groups + 255) / 256) * (Kind<T>::BF16 ? f.bf16 : f.fp32);
+    const float cost = Kind<T>::BF16 ? rounds_us(groups, f.per, f.bf16) : (float)((groups + 255) / 256) * f.fp32;
     if (best && cost >= least) continue;
     best = &f;
     best_y = y;

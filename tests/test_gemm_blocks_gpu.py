@@ -51,6 +51,14 @@ def test_fp16(gpu, M, N, K):
     assert ((C - ref).abs() <= 2.0 ** -23 * (K ** 0.5 + 2) * size).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(257, 10944, 64), (257, 11024, 192), (257, 11248, 320)])
+def test_two_blocks_a_cu(gpu, M, N, K):
+    """257 to 512 blocks of 64 x 128: the form of three stages, with one k-step, odd and even
+    numbers of stages."""
+    test_int8(gpu, M, N, K, 0)
+    test_fp16(gpu, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(700, 1024, 256), (512, 2304, 768), (320, 6144, 2048), (1024, 2048, 8192)])
 def test_fp16_sums_as_exact_as_the_streams(gpu, M, N, K):
     """A block's sum over K goes in eight parts, as a stream's over its waves: off no more

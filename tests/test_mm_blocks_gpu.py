@@ -53,3 +53,10 @@ def test_latent_blocks(serve, mixer, dtype):  # noqa: F811
     """Also the expansion of cached rows (portions of 65 tokens and more)."""
     cfg = N.config([(mixer, N.dense(ff=1100))], width=136)
     check(serve, cfg, N.weights(cfg, 5), dtype, [[70, 131, 90], [66, 1, 129]])
+
+
+@pytest.mark.parametrize("ff,rows", [(4640, 385), (4668, 385)])
+def test_two_blocks_a_cu(serve, ff, rows):  # noqa: F811
+    """gate and up in 257 to 512 blocks of 64 x 128 (three stages), rows of 16 bytes and not."""
+    cfg = N.config([(N.latent(heads=4, dim=32, rot=16, vdim=32, rank=64), N.dense(ff=ff))], width=96)
+    check(serve, cfg, N.weights(cfg, 11), "bfloat16", [[rows]])
