@@ -97,6 +97,26 @@ __device__ __forceinline__ float mov_dpp(float x) {
       float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
 }
 
+// x and the x of lane l ^ 16 (l ^ 32), in some order: an exchange of rows between registers,
+// no trip through LDS.
+struct LanePair {
+  float a, b;
+};
+__device__ __forceinline__ LanePair with_lane16(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+}
+__device__ __forceinline__ LanePair with_lane32(float x) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, x);
+  const auto r = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+  return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
+}
+__device__ __forceinline__ float add(LanePair p) { return p.a + p.b; }
+__device__ __forceinline__ float larger(LanePair p) { return fmaxf(p.a, p.b); }
+// The largest of lanes l, l ^ 16, l ^ 32, l ^ 48 (the same lane of the wave's four rows).
+__device__ __forceinline__ float rows_max(float x) { return larger(with_lane32(larger(with_lane16(x)))); }
+
 // Sum over aligned groups of G lanes (G in {2,4,8,16,32,64}); every lane of a
 // group ends with the identical total (commutative butterfly).
 template <int G>
@@ -105,8 +125,8 @@ __device__ __forceinline__ float group_sum(float x) {
   if constexpr (G >= 4) x += mov_dpp<0x4E>(x);   // quad_perm [2,3,0,1]
   if constexpr (G >= 8) x += mov_dpp<0x141>(x);  // row_half_mirror
   if constexpr (G >= 16) x += mov_dpp<0x140>(x); // row_mirror
-  if constexpr (G >= 32) x += __shfl_xor(x, 16, 64);
-  if constexpr (G >= 64) x += __shfl_xor(x, 32, 64);
+  if constexpr (G >= 32) x = add(with_lane16(x));
+  if constexpr (G >= 64) x = add(with_lane32(x));
   return x;
 }
 
@@ -139,25 +159,13 @@ __device__ __forceinline__ float wave_max(float x) {
   return x;
 }
 
-// The largest of lanes l, l ^ 16, l ^ 32, l ^ 48 (the same lane of the wave's four
-// rows): two exchanges of rows between registers, no trip through LDS.
-__device__ __forceinline__ float rows_max(float x) {
-  const uint32_t b = __builtin_bit_cast(uint32_t, x);
-  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-  const float y = fmaxf(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1]));
-  const uint32_t c = __builtin_bit_cast(uint32_t, y);
-  const auto h = __builtin_amdgcn_permlane32_swap(c, c, false, false);
-  return fmaxf(__builtin_bit_cast(float, (uint32_t)h[0]), __builtin_bit_cast(float, (uint32_t)h[1]));
-}
-
 // wave_max through DPP moves inside the 16-lane rows
 __device__ __forceinline__ float wave_max_dpp(float x) {
   x = fmaxf(x, mov_dpp<0xB1>(x));
   x = fmaxf(x, mov_dpp<0x4E>(x));
   x = fmaxf(x, mov_dpp<0x141>(x));
   x = fmaxf(x, mov_dpp<0x140>(x));
-  x = fmaxf(x, __shfl_xor(x, 16, 64));
-  return fmaxf(x, __shfl_xor(x, 32, 64));
+  return rows_max(x);
 }
 
 __device__ __forceinline__ float wave_sum(float x) {

@@ -160,72 +160,73 @@ struct GemmTraits<GemmKind::F16> {
 // the LDS image of A (ln_row_stride) and, for I8, the row scales into sa_lds:
 // ln_wave.hpp, bit-identical to the LayerNorm launch.  One wave per row (rows
 // w, w + WAVES, ...), two rows' loads in flight; gamma / beta loaded once.
-template <GemmKind KIND, int ROWS, int WAVES>
-__device__ __forceinline__ void ln_prologue(const GemmArgs& a, int m0, uint8_t* alds,
-                                            float* sa_lds) {
+// CPL: float4 chunks per lane that cover K, so that a row of 256 is not worked on as
+// one of 2048; a wave without a row does nothing, and rows past M stay as they are (each
+// row of A makes its own row of C).  One row of 256: PENDING_F.
+template <GemmKind KIND, int ROWS, int WAVES, int CPL>
+__device__ __forceinline__ void ln_prologue_rows(const GemmArgs& a, int m0, uint8_t* alds, float* sa_lds) {
   constexpr int ESIZE = GemmTraits<KIND>::ESIZE;
-  constexpr int CPL = 8;  // float4 chunks per lane (K <= 2048, ln_fusable)
   const int lane = lane_id();
   const int w = wave_id_uniform();
   const int K = a.K;
   const int K4 = K >> 2;
   const int stride = ln_row_stride(K, ESIZE);
+  const int rows = min(ROWS, a.M - m0);
+  if (w >= rows) return;
   // ln_g == NULL: quantise only (I8: the fp32 rows are the attention output,
   // the o_proj prologue replacing the merge launch's per-row quantisation)
   const bool do_ln = a.ln_g != nullptr;
-  LnRow<CPL> gm, bt;
+  LnRow<CPL> x[2], gm, bt;
+  const auto load = [&](int r, LnRow<CPL>& v) {
+    if (a.ln_emb)
+      ln_wave_load_f16(ln_embed_row(a.ln_emb, a.ln_tok, m0 + r, a.ln_V, K), K4, true, v);
+    else
+      ln_wave_load(a.ln_x + (size_t)(m0 + r) * K, K4, true, v);
+  };
+  const auto finish = [&](int r, LnRow<CPL>& v) {
+    float am;
+    if (do_ln) {
+      am = ln_wave_compute(v, gm, bt, K, a.ln_eps);
+    } else {
+      am = 0.f;
+#pragma unroll
+      for (int j = 0; j < CPL; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(v.v[j][e]));
+      am = ln_wave_max(am);
+    }
+    uint8_t* rowp = alds + (size_t)r * stride;
+    const float scale = 127.f / (am + 1e-6f);
+#pragma unroll
+    for (int j = 0; j < CPL; ++j) {
+      const int c = 64 * j + lane;  // consecutive lanes, consecutive dwords
+      if (c >= K4) continue;
+      if constexpr (KIND == GemmKind::I8)
+        *reinterpret_cast<uint32_t*>(rowp + 4 * c) = ln_quant4(v.v[j], scale);
+      else
+        *reinterpret_cast<ln_f16x4*>(rowp + 8 * c) = ln_half4(v.v[j]);
+    }
+    if (KIND == GemmKind::I8 && lane == 0) sa_lds[r] = 1.0f / scale;
+  };
+  load(w, x[0]);
   ln_wave_load(a.ln_g, K4, do_ln, gm);
   ln_wave_load(a.ln_b, K4, do_ln, bt);
-  for (int r0 = w; r0 < ROWS; r0 += 2 * WAVES) {
-    LnRow<CPL> x[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int r = r0 + q * WAVES;
-      const int m = m0 + r;
-      const bool ok = r < ROWS && m < a.M;
-      if (a.ln_emb)
-        ln_wave_load_f16(ok ? ln_embed_row(a.ln_emb, a.ln_tok, m, a.ln_V, K) : a.ln_emb, K4, ok,
-                         x[q]);
-      else
-        ln_wave_load(a.ln_x + (size_t)m * K, K4, ok, x[q]);
-    }
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int r = r0 + q * WAVES;
-      if (r >= ROWS) break;
-      const bool mok = m0 + r < a.M;  // rows past M: zero A (their outputs are not stored)
-      float am;
-      if (do_ln) {
-        am = ln_wave_compute(x[q], gm, bt, K, a.ln_eps);
-      } else {
-        am = 0.f;
-#pragma unroll
-        for (int j = 0; j < CPL; ++j)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(x[q].v[j][e]));
-        am = ln_wave_max(am);
-      }
-      uint8_t* rowp = alds + (size_t)r * stride;
-      if constexpr (KIND == GemmKind::I8) {
-        const float scale = 127.f / (am + 1e-6f);
-#pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-          const int c = 64 * j + lane;  // consecutive lanes, consecutive dwords
-          if (c < K4)
-            *reinterpret_cast<uint32_t*>(rowp + 4 * c) = mok ? ln_quant4(x[q].v[j], scale) : 0u;
-        }
-        if (lane == 0) sa_lds[r] = mok ? 1.0f / scale : 0.f;
-      } else {
-#pragma unroll
-        for (int j = 0; j < CPL; ++j) {
-          const int c = 64 * j + lane;
-          if (c < K4)
-            *reinterpret_cast<ln_f16x4*>(rowp + 8 * c) =
-                mok ? ln_half4(x[q].v[j]) : ln_f16x4{0, 0, 0, 0};
-        }
-      }
-    }
+  for (int r = w;;) {
+    if (r + WAVES < rows) load(r + WAVES, x[1]);
+    finish(r, x[0]);
+    if (r + WAVES >= rows) break;
+    finish(r + WAVES, x[1]);
+    r += 2 * WAVES;
+    if (r >= rows) break;
+    load(r, x[0]);
   }
+}
+template <GemmKind KIND, int ROWS, int WAVES>
+__device__ __forceinline__ void ln_prologue(const GemmArgs& a, int m0, uint8_t* alds, float* sa_lds) {
+  if (a.K <= 256) ln_prologue_rows<KIND, ROWS, WAVES, 1>(a, m0, alds, sa_lds);
+  else if (a.K <= 512) ln_prologue_rows<KIND, ROWS, WAVES, 2>(a, m0, alds, sa_lds);
+  else if (a.K <= 1024) ln_prologue_rows<KIND, ROWS, WAVES, 4>(a, m0, alds, sa_lds);
+  else ln_prologue_rows<KIND, ROWS, WAVES, 8>(a, m0, alds, sa_lds);  // (K <= 2048, ln_fusable)
 }
 
 // One workgroup's tile (column block bx, row block by, k slice bz of nz);

@@ -27,8 +27,7 @@ __device__ __forceinline__ float ln_wave_max(float x) {
   x = fmaxf(x, mov_dpp<0x4E>(x));   // quad_perm [2,3,0,1]
   x = fmaxf(x, mov_dpp<0x141>(x));  // row_half_mirror
   x = fmaxf(x, mov_dpp<0x140>(x));  // row_mirror
-  x = fmaxf(x, __shfl_xor(x, 16, 64));
-  return fmaxf(x, __shfl_xor(x, 32, 64));
+  return rows_max(x);
 }
 
 template <int CPL>
