@@ -78,3 +78,34 @@ def wide(gpu, tmp_path_factory):
 ])
 def test_pieces_used_again(wide, lens, pick):
     check(wide, lens, pick)
+
+
+@pytest.mark.parametrize("tokens,want", [
+    (np.array([5, 6, 7], np.int32), [2, 0]), ([5, 6, 7], (1,)), ((5, 6, 7), range(3)),
+    (np.array([5, 9, 6, 9, 7, 9], np.int32)[::2], np.array([[1], [2]])),
+    (np.array([5, 6, 7]), np.array([0, 2], np.int32)), (np.array([5.0, 6.0, 7.0]), []),
+    ([np.int64(5), 6, 7], [True])])
+def test_entries_of_every_kind(eng, tokens, want):
+    """Entries that the native way takes and those it leaves to the general one."""
+    def run(entries):
+        s = eng.open_seq()
+        try:
+            return eng.step([(s, *entries)])
+        finally:
+            eng.close_seq(s)
+    places = [int(p) for p in np.asarray(want, np.int32).reshape(-1)]
+    all_rows = run((np.array([5, 6, 7], np.int32), np.array([0, 1, 2], np.int32)))
+    got = run((tokens, want))
+    assert got.shape == (len(places), eng.vocab) and got.dtype == np.float32
+    np.testing.assert_array_equal(got, all_rows[places])
+
+
+@pytest.mark.parametrize("bad", [([5], [1]), ([1 << 20], [0]), ([], []), ([5], [-1])])
+def test_refused_entries(eng, bad):
+    s = eng.open_seq()
+    with pytest.raises(Exception, match="engine step"):
+        eng.step([(s, *bad)])
+    assert eng.seq_len(s) == 0
+    eng.close_seq(s)
+    with pytest.raises(Exception, match="not open"):
+        eng.step([(s, [5], [0])])
