@@ -16,13 +16,15 @@
 //   * greedy (T <= 0 or top_k == 1): argmax, first maximum wins
 //     (sample_from_logits, decoder/cuda_decoder.cu:7-14).
 //
-// The rank and mass thresholds are patterns of (non-negative) fp32 probabilities,
-// found ten bits at a time from histograms in LDS: three passes over the registers
-// for each, where a search bit by bit took 31 passes and block reductions for each
-// (64 rows of 50,257, top_k 40 and top_p 0.9: 461 us, now 36 us).  Bound by the
-// latency of the passes and of the LDS atomics, one row being one workgroup.  Masses
-// are added as whole multiples of 2^-50, so their sums are exact to 2^-34 and do not
-// depend on the order of the atomics.
+// The rank and mass thresholds are patterns of (non-negative) fp32 probabilities.
+// A small top_k leaves few tokens that can matter, and these are ranked one against
+// the other (pick_few).  Else they are found ten bits at a time from histograms in
+// LDS: three passes over the registers for each.  64 rows of 50,257, top_k 40 and top_p
+// 0.9: 35 us by histograms, now 21 (top_k 50 alone 31 and 20, top_p 0.95 alone 35, neither
+// 15).  Bound by the vector instructions over a row's registers, one row being one
+// workgroup: the softmax, then the passes.  Masses are added as whole
+// multiples of 2^-50, so their sums are exact to 2^-34 and do not depend on the order
+// of the atomics.
 #include <utility>
 
 #include "common.hpp"
@@ -142,6 +144,102 @@ __device__ __forceinline__ uint32_t find_pattern(const float (&v)[NS][4], uint32
   return at;
 }
 
+// The thresholds of a top_k of at most kFewK, where no more than kFew tokens can be among
+// the top_k: the row's threads form 128 groups of eight, and top_k groups' largest values
+// are at least the top_k-th largest of the groups' largest, so nothing below that is kept.
+// What is left is counted against one another: a value's rank and the mass above it.
+// False: too many left, or groups without a value; nothing is found then.  Both thresholds
+// are what find_pattern gives.
+constexpr int kFewK = 64, kFew = 256, kGroups = kSampleThreads / 8;
+struct Few {
+  float most[kGroups];
+  uint32_t bits[kFew];
+  unsigned long long mass[kFew];
+  float floor;
+  int count;
+  uint32_t rank_least, mass_least;
+};
+template <int NS>
+__device__ __forceinline__ bool pick_few(const float (&v)[NS][4], int top_k, unsigned long long want, Few& few,
+                                         uint32_t* least) {
+  const int t = threadIdx.x;
+  float top = 0.f;
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) top = fmaxf(top, v[s][j]);
+  top = fmaxf(top, mov_dpp<0xB1>(top));
+  top = fmaxf(top, mov_dpp<0x4E>(top));
+  top = fmaxf(top, mov_dpp<0x141>(top));
+  if (t % 8 == 0) few.most[t / 8] = top;
+  if (t == 0) {
+    few.floor = 0.f;
+    few.count = 0;
+    few.rank_least = few.mass_least = 0;
+  }
+  __syncthreads();
+  {  // eight threads a group, each against sixteen others
+    const int g = t / 8, h0 = t % 8 * (kGroups / 8);
+    int above = 0;
+#pragma unroll
+    for (int k = 0; k < kGroups / 8; k += 4) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(&few.most[h0 + k]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) above += o[e] > top || (o[e] == top && h0 + k + e < g);
+    }
+    above += __builtin_amdgcn_mov_dpp(above, 0xB1, 0xF, 0xF, true);
+    above += __builtin_amdgcn_mov_dpp(above, 0x4E, 0xF, 0xF, true);
+    above += __builtin_amdgcn_mov_dpp(above, 0x141, 0xF, 0xF, true);
+    if (t % 8 == 0 && above == top_k - 1) few.floor = top;
+  }
+  __syncthreads();
+  const float floor = few.floor;
+  if (!(floor > 0.f)) return false;
+  if (top >= floor) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (v[s][j] >= floor) {
+          const int at = atomicAdd(&few.count, 1);
+          if (at < kFew) {
+            few.bits[at] = __float_as_uint(v[s][j]);
+            few.mass[at] = mass_of(__float_as_uint(v[s][j]));
+          }
+        }
+  }
+  __syncthreads();
+  const int n = few.count;
+  if (n > kFew) return false;
+  // four threads a value
+  const uint32_t own = t / 4 < n ? few.bits[t / 4] : 0u;
+  int above = 0, same = 0;
+  unsigned long long mass_above = 0, mass_same = 0;
+  if (own)
+    for (int i = t % 4; i < n; i += 4) {
+      const uint32_t o = few.bits[i];
+      const unsigned long long m = few.mass[i];
+      above += o > own;
+      same += o == own;
+      mass_above += o > own ? m : 0;
+      mass_same += o == own ? m : 0;
+    }
+#pragma unroll
+  for (int off = 1; off < 4; off <<= 1) {
+    above += __shfl_xor(above, off, 64);
+    same += __shfl_xor(same, off, 64);
+    mass_above += __shfl_xor(mass_above, off, 64);
+    mass_same += __shfl_xor(mass_same, off, 64);
+  }
+  if (own && above < top_k && above + same >= top_k) few.rank_least = own;
+  // (a value below the top_k-th counts for nothing: what is above it holds the mass already,
+  // or nothing more is dropped)
+  if (own && mass_above < want && mass_above + mass_same >= want) few.mass_least = own;
+  __syncthreads();
+  *least = max(few.rank_least, few.mass_least);
+  return true;
+}
+
 // temperature <= 0 or top_k 1: the first maximum
 __global__ __launch_bounds__(kSampleThreads) void sample_greedy_kernel(SampleArgs a) {
   __shared__ float shf[kSampleWaves];
@@ -175,6 +273,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   __shared__ float cells[NS * kSampleWaves];
   __shared__ int cell;
   __shared__ float cell_left;
+  __shared__ __attribute__((aligned(16))) Few few;
   const int r = blockIdx.x, lane = lane_id(), w = wave_id_uniform();
   const float* lg = a.logits + (size_t)r * a.V;
   const auto token = [&](int s, int j) { return s * kSampleSeg + w * 256 + j * 64 + lane; };
@@ -192,12 +291,16 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   }
 
   // temperature + softmax (reference: logits /= T; exp(x - max); / (sum + 1e-6))
+  // The product with 1 / T in 64 bits is off by 2^-52 of the quotient, which lies no nearer
+  // than 2^-49 to the middle of two floats: rounded, it is the quotient (a division takes
+  // four times the cycles).
+  const double by = 1.0 / (double)a.temperature;
   float mloc = -INFINITY;
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      v[s][j] = v[s][j] / a.temperature;
+      v[s][j] = (float)((double)v[s][j] * by);
       mloc = fmaxf(mloc, v[s][j]);
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -231,12 +334,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   // top_p, top-p drops nothing more.  A top_p below the masses' unit wants one of it: the
   // most probable alone have nothing ranked above them.
   uint32_t least = 0;
-  if (a.top_k > 0 && a.top_k < a.V)
+  const unsigned long long want = a.top_p < 1.0f ? max(mass_of(__float_as_uint(a.top_p)), 1ull) : ~0ull;
+  const bool few_found =
+      a.top_k > 0 && a.top_k < a.V && a.top_k <= kFewK && pick_few(v, a.top_k, want, few, &least);
+  if (!few_found && a.top_k > 0 && a.top_k < a.V)
     least = find_pattern<NS>(v, 0u, (uint32_t)a.top_k, ranks, rank_part, &rank_found,
                              [](uint32_t) { return 1u; });
-  if (a.top_p < 1.0f)
-    least = max(least, find_pattern<NS>(v, least, max(mass_of(__float_as_uint(a.top_p)), 1ull), masses,
-                                        mass_part, &mass_found,
+  if (!few_found && a.top_p < 1.0f)
+    least = max(least, find_pattern<NS>(v, least, want, masses, mass_part, &mass_found,
                                         [](uint32_t bits) { return mass_of(bits); }));
 
   // kept mass in token order: per cell, then over the cells

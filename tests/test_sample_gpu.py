@@ -78,3 +78,31 @@ def test_top_p_below_any_probability(gpu, p, k):
         got = draw(logits, 1.0, k, p, c)
         assert (got[:4] == logits[:4].argmax(1)).all() and got[5] in (3, 4100, 8999)
     assert len({int(draw(logits[4:5], 1.0, k, p, c)[0]) for c in range(40)}) > 20  # all tied
+
+
+@pytest.mark.parametrize("k", [2, 5, 63, 64, 65])
+@pytest.mark.parametrize("p", [0.5, 0.97, 1.0])
+@pytest.mark.parametrize("shape", ["spread", "one_group", "few_groups", "many_ties", "many_near", "flat"])
+def test_few_tokens_left(gpu, shape, k, p):
+    """A small top_k: its tokens spread out, in one group of eight threads, in fewer groups
+    than top_k; more equal or near ones than are ranked one against the other."""
+    from oracle.oracle import sample_rows
+    V = 12500
+    rng = np.random.default_rng(k)
+    logits = rng.standard_normal((3, V)).astype(np.float32)
+    at = np.arange(V)
+    group = (at // 256 % 16) * 8 + at % 64 // 8
+    if shape == "one_group":
+        logits[:, group == 19] += 6.0
+    elif shape == "few_groups":
+        logits[:, group >= 40] = -np.inf
+    elif shape == "many_ties":
+        logits[:, rng.permutation(V)[:900]] = 3.5
+    elif shape == "many_near":
+        logits[:, rng.permutation(V)[:2000]] = 3.0 + 1e-3 * rng.standard_normal((3, 2000)).astype(np.float32)
+    elif shape == "flat":
+        logits[:] = 0.0
+    for counter in range(6):
+        ref, margin = sample_rows(logits, 0.7, k, p, seed=5, counter=counter)
+        got = draw(logits, 0.7, k, p, counter)
+        assert ((got == ref) | (margin < 1e-4)).all(), (got, ref, margin)
