@@ -113,7 +113,12 @@ __device__ __forceinline__ LanePair with_lane32(float x) {
   return {__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])};
 }
 __device__ __forceinline__ float add(LanePair p) { return p.a + p.b; }
-__device__ __forceinline__ float larger(LanePair p) { return fmaxf(p.a, p.b); }
+// (fmaxf of what comes as bits takes two more instructions to quiet a NaN)
+__device__ __forceinline__ float larger(LanePair p) {
+  float x;
+  asm("v_max_f32 %0, %1, %2" : "=v"(x) : "v"(p.a), "v"(p.b));
+  return x;
+}
 // The largest of lanes l, l ^ 16, l ^ 32, l ^ 48 (the same lane of the wave's four rows).
 __device__ __forceinline__ float rows_max(float x) { return larger(with_lane32(larger(with_lane16(x)))); }
 

@@ -8,18 +8,22 @@
 // to positions 0 .. p0+i.  The decode kernel computes the same thing with one
 // wave per (token, head), so each page is re-read once per query token; here a
 // workgroup of 4 waves owns 64 consecutive queries of one head, loads every
-// 64-key stage of K and V into LDS ONCE, and each wave runs
+// stage of K and V (32 keys; 64 where D is 64) into LDS ONCE, and each wave runs
 //   S^T[32 keys][16 queries] = K · Q^T     (v_mfma_f32_16x16x32_f16)
 //   O^T[D][16 queries]     += V^T · P^T
 // with the flash online softmax (log2 units, as pa_split_kernel) in between.
 //
-// A stage goes from memory straight into LDS, one stage ahead, a wave loading
-// 16 keys, with their page looked up two stages ahead: the dependent loads
-// (page, keys) and a register pass per 32 keys were what bounded the first form
-// (2048 queries x 16 heads x 128: 137 us, now 61 us).  The
-// 16-byte chunks of a row are exchanged by the key so that the 16 rows of a
-// fragment lie in different banks.  Now bound by the vector instructions of the
-// softmax beside the matrix cores, at two workgroups per CU.
+// A stage goes from memory straight into LDS, one stage ahead, its loads shared
+// out among the waves, with the pages of 64 groups of 16 keys looked up a lane each.
+// The 16-byte chunks of a row are exchanged by the key so that the 16 rows of a
+// fragment lie in different banks.
+//
+// Bound by the vector instructions of the softmax and the matrix cores, each on its own
+// wave: what counts is waves to choose from and few instructions.  2048 queries x 16
+// heads x 128: 61 us with stages of 64 keys, two waves a SIMD; 55 with half the LDS and
+// four waves; 49 with the maximum moved only when it grew by more than 1, halves made
+// by conversions in pairs, LDS offsets in the instructions and page lookups in one
+// load (1410 -> 1090 vector instructions a wave and 1000 keys).
 //
 // Orientation: keys are the MFMA row index of S^T, so the C layout of S^T
 // (lane l: rows 4(l>>4)+r, column l&15) already holds, per lane, 8 keys of ONE
@@ -41,6 +45,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "common.hpp"
 #include "pa_decode.hpp"
@@ -69,7 +74,7 @@ struct PaPrefillArgs {
   float* part_ml;
 };
 
-constexpr int kStageKeys = 64;
+constexpr int stage_keys(int D) { return D == 64 ? 64 : 32; }
 constexpr int kWaves = 4;
 constexpr int kTileQueries = 16 * kWaves;  // of a workgroup
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -81,15 +86,28 @@ __device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
   lo = (_Float16)(x - (float)hi);
 }
 
+// Two values' fp16 halves (the asm: the compiler makes each hi a second time for its lo).
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint32_t& lo) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, f16x2));
+  asm("" : "+v"(hi));
+  const f16x2 h = __builtin_bit_cast(f16x2, hi);
+  lo = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(x - (float)h[0]), (_Float16)(y - (float)h[1])});
+}
+
 template <int D, int TS>
-__global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArgs a) {
+__global__ __launch_bounds__(64 * kWaves, 4) void pa_prefill_kernel(PaPrefillArgs a) {
   constexpr int ROWB = 2 * D;                // bytes of a key's row
   constexpr int CPR = D / 8;                 // its 16-byte chunks
-  constexpr int LOADS = 16 * ROWB / 1024;    // 1 KiB loads of a wave's 16 keys, each of K and V
+  constexpr int kStageKeys = stage_keys(D);
+  constexpr int OWN = kStageKeys / kWaves;   // keys of a stage that a wave loads, of one page
+  constexpr int LOADS = OWN * ROWB / 1024;   // its loads of 1 KiB, each of K and V
+  constexpr int BLOCKS = kStageKeys / 32, GROUPS = kStageKeys / 16;
   constexpr int NKK = D / 32;                // k-steps of q.k
   constexpr int ND = D / 16;                 // 16-dim tiles of the output
   constexpr int QW = 16, QT = kTileQueries;  // queries of a wave, of the workgroup
-  static_assert(D % 32 == 0 && TS % 16 == 0 && kStageKeys == 16 * kWaves, "shape");
+  static_assert(D % 32 == 0 && TS % 16 == 0 && 16 % OWN == 0 && OWN * ROWB % 1024 == 0, "shape");
   __shared__ u32x4 lds[2][2][kStageKeys * CPR];  // [stage][K, V][key][chunk, exchanged]
 
   const int lane = threadIdx.x & 63;
@@ -112,17 +130,17 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
   if (s0 >= s1) return;
   const int32_t* pt = a.pt_row + (size_t)h * a.max_tiles;
 
-  // Lanes 0..3: the page of a stage's 16-key groups (-1: none, or past lastpos).
-  auto pages_of = [&](int s) -> int {
-    const int key = s * kStageKeys + 16 * (lane & 3), tile = key / TS;
-    const int pg = s < s1 && key <= lastpos && tile < a.max_tiles ? pt[tile] : -1;
+  // Lane i: the page of the split's 16-key group `group` + i (-1: none, or past lastpos).
+  auto pages_from = [&](int group) -> int {
+    const int key = s0 * kStageKeys + 16 * (group + lane), tile = key / TS;
+    const int pg = key <= lastpos && tile < a.max_tiles ? pt[tile] : -1;
     return pg < a.num_pages ? pg : -1;
   };
   // LDS position of chunk `ch` of key k (0..15 of a group): 16 rows that read one
   // chunk each meet 16 different bank groups, and so do 8 rows that read two
   auto exchange = [](int k, int ch) { return ch ^ (CPR == 16 ? ((k << 1) | (k >> 3)) & 15 : (k >> 1) & 7); };
-  auto issue = [&](int buf, int s, int page) {  // this wave's 16 keys of stage s
-    const int key0 = s * kStageKeys + 16 * w, at = 16 * w * CPR;
+  auto issue = [&](int buf, int s, int page) {  // this wave's keys of stage s
+    const int key0 = s * kStageKeys + OWN * w / 16 * 16, at = OWN * w * CPR;  // (of their group)
     if (page < 0) {  // masked: V = 0, since 0 * NaN would not be 0
 #pragma unroll
       for (int i = 0; i < LOADS; ++i) {
@@ -132,18 +150,23 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
       return;
     }
     const size_t base = (size_t)page * a.page_stride + (size_t)(key0 % TS) * ROWB;
+    const uint8_t *k = a.k_pool + base, *v = a.v_pool + base;  // of all lanes
+    const uint32_t last = lastpos - key0;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const int row = (64 * i + lane) / CPR, ch = exchange(row, (64 * i + lane) % CPR);
+      const uint32_t row = OWN * w % 16 + (64 * i + lane) / CPR, ch = exchange(row, (64 * i + lane) % CPR);
       // (rows past lastpos may never have been written: the last one that was, masked)
-      const size_t off = base + (size_t)min(row, lastpos - key0) * ROWB + 16 * ch;
-      load_to_lds(a.k_pool + off, &lds[buf][0][at + 64 * i]);
-      load_to_lds(a.v_pool + off, &lds[buf][1][at + 64 * i]);
+      const uint32_t off = min(row, last) * ROWB + 16 * ch;
+      load_to_lds(k + off, &lds[buf][0][at + 64 * i]);
+      load_to_lds(v + off, &lds[buf][1][at + 64 * i]);
     }
   };
-  int pages = pages_of(s0), next = pages_of(s0 + 1);
-  unsigned valid = (unsigned)__ballot(pages >= 0) & 15u;
-  issue(0, s0, __builtin_amdgcn_readlane(pages, w));
+  constexpr unsigned ALL = (1u << GROUPS) - 1;
+  const int own = OWN * w / 16;  // the group of this wave's keys
+  int pages = pages_from(0), more = pages_from(64);
+  unsigned long long there = __ballot(pages >= 0);
+  unsigned valid = (unsigned)there & ALL;
+  issue(0, s0, __builtin_amdgcn_readlane(pages, own));
 
   // Q^T B-operand fragments: lane holds q[qi][32kk + 8g .. +7] (pre-scaled by
   // qscale), hi + lo.  The query's values are also scaled by a power of two
@@ -189,22 +212,40 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
   }
 
   f32x4 O[ND];
-  float mrun = kNegSentinel, lrun = 0.f;
+  float mrun = kNegSentinel, mtop = kNegSentinel, lrun = 0.f;
 #pragma unroll
   for (int nd = 0; nd < ND; ++nd) O[nd] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  int buf = 0;
-  for (int s = s0; s < s1; ++s, buf ^= 1) {
+  // V's place in LDS for 16 dims of the first block.  A operand lane l: V^T[d = 16nd +
+  // (l&15)][k 8g+j] = V[key(8g+j)][d], keys 4g..4g+3 then 16+4g..16+4g+3: two transposed reads
+  // of 4 V rows x 16 columns, lane 4q+p addressing row q, columns 4p..
+  uint32_t vat[ND];
+#pragma unroll
+  for (int nd = 0; nd < ND; ++nd) {
+    const int vk = 4 * g + (c >> 2), p4 = c & 3;
+    vat[nd] = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4*)&lds[0][0][0] + vk * ROWB +
+              16 * exchange(vk, 2 * nd + (p4 >> 1)) + 8 * (p4 & 1);
+  }
+
+  // stage s of the split, in buffer BUF: known, its LDS offsets are in the instructions
+  auto stage = [&](auto BUF, int s) {
+    constexpr int buf = decltype(BUF)::value;
     wait_lds_loads();
     __syncthreads();  // stage s has landed, the other buffer is read out
-    const unsigned valid_next = (unsigned)__ballot(next >= 0) & 15u;
-    if (s + 1 < s1) issue(buf ^ 1, s + 1, __builtin_amdgcn_readlane(next, w));
-    next = pages_of(s + 2);
+    const int at = (s + 1 - s0) * GROUPS % 64;  // the next one's groups
+    if (at == 0) {
+      pages = more;
+      more = pages_from((s + 1 - s0) * GROUPS + 64);
+      there = __ballot(pages >= 0);
+    }
+    const unsigned here_all = valid;
+    valid = (unsigned)(there >> at) & ALL;
+    if (s + 1 < s1) issue(buf ^ 1, s + 1, __builtin_amdgcn_readlane(pages, at + own));
 #pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
+    for (int kb = 0; kb < BLOCKS; ++kb) {
       const int key0 = s * kStageKeys + 32 * kb;
       if (key0 > wave_last) break;
-      const unsigned here = valid >> (2 * kb) & 3u;  // of the block's two 16-key tiles
+      const unsigned here = here_all >> (2 * kb) & 3u;  // of the block's two 16-key tiles
       // S^T: two 16-key tiles
       f32x4 sc[2];
 #pragma unroll
@@ -238,14 +279,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
             mloc = fmaxf(mloc, sc[u][r]);
           }
       }
-      // online softmax (per query = per lane): p = 2^(s - m), m the running maximum; s is
-      // scaled back in the same operation.  (The scale of the halves in the exponent as well,
+      // online softmax (per query = per lane): p = 2^(s - m), m the running maximum or up to 1
+      // less (p <= 2, its scaled halves below 2^15), so that few blocks move what is summed; s
+      // is scaled back in the same operation.  (The scale of the halves in the exponent as well,
       // 2^(s - m + 14), saves an instruction a value and rounds the exponent of the large p
       // to 2^-21: 1.2 to 2 times the error of the result.)
-      f16x8 ph, pl;
+      uint32_t ph[4], pl[4];
       const float mblk = rows_max(mloc) * qinv;
-      if (__any(mblk > mrun)) {
-        const float mnew = fmaxf(mrun, mblk);
+      mtop = fmaxf(mtop, mblk);
+      if (__any(mblk > mrun + 1.f)) {
+        const float mnew = mtop;
         const float corr = __builtin_amdgcn_exp2f(mrun - mnew);
         lrun *= corr;
 #pragma unroll
@@ -253,35 +296,40 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
         mrun = mnew;
       }
 #pragma unroll
-      for (int u = 0; u < 2; ++u)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(fmaf(sc[u][r], qinv, -mrun));
-          lrun += p;
-          _Float16 hi, lo;
-          split_f16(p * kPScale, hi, lo);  // p <= 1: scaled clear of fp16 subnormals
-          ph[4 * u + r] = hi;
-          pl[4 * u + r] = lo;
-        }
-      // O^T += V^T · P^T.  A operand lane l: V^T[d = 16nd + (l&15)][k 8g+j] =
-      // V[key(8g+j)][d], keys 4g..4g+3 then 16+4g..16+4g+3: two transposed
-      // reads of 4 V rows x 16 columns, lane 4q+p addressing row q, columns 4p..
-      const int vk = 4 * g + (c >> 2), p4 = c & 3;
-      const char* v0 = reinterpret_cast<const char*>(&lds[buf][1][(32 * kb + vk) * CPR]) + 8 * (p4 & 1);
+      for (int i = 0; i < 4; ++i) {
+        const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[i / 2][i % 2 * 2], qinv, -mrun));
+        const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[i / 2][i % 2 * 2 + 1], qinv, -mrun));
+        lrun += p0;
+        lrun += p1;
+        split_pair(p0 * kPScale, p1 * kPScale, ph[i], pl[i]);  // clear of fp16 subnormals
+      }
+      const f16x8 phi = __builtin_bit_cast(f16x8, u32x4{ph[0], ph[1], ph[2], ph[3]});
+      const f16x8 plo = __builtin_bit_cast(f16x8, u32x4{pl[0], pl[1], pl[2], pl[3]});
+      // O^T += V^T · P^T
 #pragma unroll
       for (int nd = 0; nd < ND; ++nd) {
-        const char* at = v0 + 16 * exchange(vk, 2 * nd + (p4 >> 1));
-        const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (__attribute__((address_space(3))) s16x4*)at);
+        const uint32_t at = vat[nd] + (2 * buf + 1) * sizeof(lds[0][0]) + 32 * kb * ROWB;
+        const s16x4 x = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)at);
         const s16x4 y = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (__attribute__((address_space(3))) s16x4*)(at + 16 * ROWB));
         const f16x8 vf = __builtin_bit_cast(
             f16x8, s16x8{x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]});
-        O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, ph, O[nd], 0, 0, 0);
-        O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl, O[nd], 0, 0, 0);
+        O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, phi, O[nd], 0, 0, 0);
+        O[nd] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, plo, O[nd], 0, 0, 0);
       }
     }
-    valid = valid_next;
+  };
+  for (int s = s0;;) {
+    stage(std::integral_constant<int, 0>{}, s);
+    if (++s >= s1) break;
+    stage(std::integral_constant<int, 1>{}, s);
+    if (++s >= s1) break;
+  }
+  {
+    const float corr = __builtin_amdgcn_exp2f(mrun - mtop);
+    lrun *= corr;
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd) O[nd] *= corr;
   }
 
   // the 4 lanes of a query hold partial sums over their keys
@@ -295,7 +343,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void pa_prefill_kernel(PaPrefillArg
 #pragma unroll
     for (int nd = 0; nd < ND; ++nd)
       *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * (1.0f / kPScale);
-    if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{mrun, lrun};
+    if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{mtop, lrun};
   } else {
     const float inv = 1.0f / (lrun + 1e-6f) * (1.0f / kPScale);
     float* o = a.out + (size_t)qi * a.out_stride + h * D + 4 * g;
@@ -312,21 +360,21 @@ hipError_t launch_prefill(const PaPrefillArgs& a, hipStream_t st) {
 }
 
 // The key range is cut into splits of `per` stages, the length for which the rounds of
-// workgroups (2 per CU) times their length is least, a split more counted as half a stage
+// workgroups (4 per CU) times their length is least, a split more counted as half a stage
 // for its merge; no more than split_bound of them a query.  32 queries a wave in place of
 // 16 (16 heads of 128, with the merge): 2048 queries 72 -> 70 us, but those after 2048 more
 // 120 -> 139, 1024 34 -> 36, 117 11 -> 14; heads of 64 2048 48 -> 60.
-constexpr int kRound = 512;
+constexpr int kRound = 1024;
 struct PrefillPlan {
   int nsplit, pps;
 };
 int split_bound(int H, int m) {
   const int nq = (m + kTileQueries - 1) / kTileQueries;
-  return std::min(2 * kRound / std::max(nq * H, 1) + 1, 128);
+  return std::min(kRound / std::max(nq * H, 1) + 1, 128);
 }
 PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   PrefillPlan p;
-  const int H = kv->num_heads;
+  const int H = kv->num_heads, kStageKeys = stage_keys(kv->head_dim);
   const int most = (p0 + m - 1) / kStageKeys + 1;
   const int bound = split_bound(H, m);
   int best = most;
@@ -359,7 +407,7 @@ bool pa_prefill_supported(const pa_kv_view* kv) {
 // the size is of the most that any context up to this one takes.
 size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m) {
   if (!pa_prefill_supported(kv) || m <= 0 || p0 < 0) return 0;
-  const int most = (int)(((long long)p0 + m - 1) / kStageKeys) + 1;
+  const int most = (int)(((long long)p0 + m - 1) / stage_keys(kv->head_dim)) + 1;
   const int n = std::min(split_bound(kv->num_heads, m), most);
   if (n <= 1) return 0;
   return (size_t)m * kv->num_heads * n * (size_t)(kv->head_dim + 2) * sizeof(float);

@@ -14,7 +14,13 @@
 //              ahead, and are merged through LDS.  A decoded token of a group of
 //              8 heads is 8 rows: its K and V are read once for the group.
 //   many rows  gqa_rows_kernel: every wave owns 16 MT rows; the workgroup loads
-//              each page into LDS once, in fragment order, one stage ahead.
+//              each page into LDS once, in fragment order, one stage ahead.  Bound by
+//              the softmax's vector instructions beside the matrix cores, and by the
+//              waves there are to run the one while others wait: in bf16 8 waves of 16
+//              rows, four waves a SIMD (2048 tokens, 16 heads of 128 over 2: 4 waves of
+//              32 rows 65 us, 8 of 16 with the class's own sizes known 51, maxima that
+//              move only when they grew by more than 8 47; 16 heads of 192 / 128: 43 us,
+//              36, 35).
 //
 // The probabilities stay fp32 up to the product: in bf16 they enter it as
 // hi + lo halves.  Scores, maxima and sums are fp32 in log2 units.  A sink is
@@ -55,8 +61,19 @@ __device__ __forceinline__ f32x4 dot_step(u32x4 a, u32x4 b, f32x4 c) {
   }
 }
 
-// The rows one wave works on.  CK, CV: largest Dp and Dvp of the class.
-template <typename T, int CK, int CV, int MT>
+// Two probabilities' bf16 halves: hi, and what it leaves.
+__device__ __forceinline__ uint32_t bf16_pair(float x, float y) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{x, y}, bf16x2));
+}
+__device__ __forceinline__ void split_bf16(float x, float y, uint32_t& hi, uint32_t& lo) {
+  hi = bf16_pair(x, y);
+  lo = bf16_pair(x - __builtin_bit_cast(float, hi << 16), y - __builtin_bit_cast(float, hi & 0xffff0000u));
+}
+
+// The rows one wave works on.  CK, CV: largest Dp and Dvp of the class; WHOLE: its own.
+template <typename T, int CK, int CV, int MT, bool WHOLE = false>
 struct Rows {
   static constexpr int KSTEP = Att<T>::KSTEP, KT = Att<T>::KT, KEYS = 16 * KT;
   static constexpr int NK = CK / KSTEP, ND = CV / 16;
@@ -81,6 +98,7 @@ struct Rows {
       for (int k = 0; k < NK; ++k) {
         const int d = k * KSTEP + g * (KSTEP / 4);
         q[t][k] = ok && d < a.Dp ? *reinterpret_cast<const u32x4*>(qp + d) : u32x4{0u, 0u, 0u, 0u};
+        if (a.scale < 0.f) q[t][k] ^= sizeof(T) == 2 ? 0x80008000u : 0x80000000u;
       }
       m[t] = kNegSentinel;
       l[t] = 0.f;
@@ -90,7 +108,7 @@ struct Rows {
   }
 
   // One block of KEYS keys from position key0: kf(u, k) and vf(n) give its
-  // fragments; mask: some row ends inside it.
+  // fragments; mask: some row ends inside it.  scale2 > 0 (the queries have the scale's sign).
   template <typename KF, typename VF>
   __device__ __forceinline__ void attend(const GqaArgs& a, int key0, bool mask, float scale2, KF kf,
                                          VF vf) {
@@ -102,7 +120,7 @@ struct Rows {
       for (int t = 0; t < MT; ++t) s[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int k = 0; k < NK; ++k)
-        if (k * KSTEP < a.Dp) {
+        if (WHOLE || k * KSTEP < a.Dp) {
           const u32x4 x = kf(u, k);
 #pragma unroll
           for (int t = 0; t < MT; ++t) s[t][u] = dot_step<T>(x, q[t][k], s[t][u]);
@@ -111,53 +129,57 @@ struct Rows {
     u32x4 hi[MT], lo[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
-      float mloc = kNegSentinel;
+      // The products are read before the branch on `mask`: the compiler leaves out the
+      // wait for a matrix instruction whose result is first read behind one.
+      float mloc = -INFINITY;
 #pragma unroll
-      for (int u = 0; u < KT; ++u) {
-        s[t][u] *= scale2;
-        if (mask) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (key0 + 16 * u + 4 * g + r > pos[t]) s[t][u][r] = 2.f * kNegSentinel;
-        }
+      for (int u = 0; u < KT; ++u)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mloc = fmaxf(mloc, s[t][u][r]);
+      asm volatile("" : "+v"(mloc));
+      if (mask) {
+        mloc = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < KT; ++u)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (key0 + 16 * u + 4 * g + r > pos[t]) s[t][u][r] = -INFINITY;
+            mloc = fmaxf(mloc, s[t][u][r]);
+          }
       }
-      mloc = rows_max(mloc);
-      if (__any(mloc > m[t])) {
+      mloc = rows_max(mloc) * scale2;
+      // (what is summed moves when a maximum grew by more than 8: p <= 256, floats as exact)
+      if (__any(mloc > m[t] + 8.f)) {
         const float mnew = fmaxf(m[t], mloc);  // >= the sentinel: masked scores stay far below
         const float corr = __builtin_amdgcn_exp2f(m[t] - mnew);
         l[t] *= corr;
 #pragma unroll
         for (int n = 0; n < ND; ++n)
-          if (16 * n < a.Dvp) o[n][t] *= corr;
+          if (WHOLE || 16 * n < a.Dvp) o[n][t] *= corr;
         m[t] = mnew;
       }
 #pragma unroll
       for (int u = 0; u < KT; ++u)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          s[t][u][r] = __builtin_amdgcn_exp2f(s[t][u][r] - m[t]);
+          s[t][u][r] = __builtin_amdgcn_exp2f(fmaf(s[t][u][r], scale2, -m[t]));
           l[t] += s[t][u][r];
         }
       if constexpr (sizeof(T) == 2) {
-        bf16x8 h, w;
 #pragma unroll
-        for (int u = 0; u < KT; ++u)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            h[4 * u + r] = (__bf16)s[t][u][r];
-            w[4 * u + r] = (__bf16)(s[t][u][r] - (float)h[4 * u + r]);
-          }
-        hi[t] = __builtin_bit_cast(u32x4, h);
-        lo[t] = __builtin_bit_cast(u32x4, w);
+        for (int i = 0; i < 4; ++i) {
+          uint32_t h, w;
+          split_bf16(s[t][i / 2][i % 2 * 2], s[t][i / 2][i % 2 * 2 + 1], h, w);
+          hi[t][i] = h;
+          lo[t][i] = w;
+        }
       } else {
         hi[t] = __builtin_bit_cast(u32x4, s[t][0]);
       }
     }
 #pragma unroll
     for (int n = 0; n < ND; ++n)
-      if (16 * n < a.Dvp) {
+      if (WHOLE || 16 * n < a.Dvp) {
         const u32x4 x = vf(n);
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
@@ -271,7 +293,7 @@ __global__ __launch_bounds__(64 * kWaves, C < 256 ? 2 : 1) void gqa_split_kernel
                      : u32x4{0u, 0u, 0u, 0u};
     }
   };
-  const float scale2 = a.scale * kLog2e;
+  const float scale2 = fmaxf(fabsf(a.scale) * kLog2e, 1e-30f);  // (0: -inf stays what it is)
   RowsT row;
   Block x, y;
   int b = b0 + w;
@@ -342,23 +364,24 @@ __global__ __launch_bounds__(64 * kWaves, C < 256 ? 2 : 1) void gqa_split_kernel
   row.write(a, it, kvh, 0, rows, 16);
 }
 
-// Keys a stage of the row kernel holds: 32 KiB of K and V fragments at most.
+// Keys a stage of the row kernel holds: 40 KiB of K and V fragments at most, so that a CU
+// holds two workgroups.
 template <typename T, int CK, int CV>
 constexpr int stage_keys() {
   int n = kPageTokens;
-  while (n * (CK + CV) * (int)sizeof(T) > 32768) n /= 2;
+  while (n * (CK + CV) * (int)sizeof(T) > 40960) n /= 2;
   return n;
 }
 
-template <typename T, int CK, int CV, int MT>
-__global__ __launch_bounds__(64 * kWaves, 2) void gqa_rows_kernel(GqaArgs a) {
-  using RowsT = Rows<T, CK, CV, MT>;
+template <typename T, int CK, int CV, int MT, int W, bool WHOLE>
+__global__ __launch_bounds__(64 * W, W / 2) void gqa_rows_kernel(GqaArgs a) {
+  using RowsT = Rows<T, CK, CV, MT, WHOLE>;
   constexpr int KSTEP = RowsT::KSTEP, KT = RowsT::KT, KEYS = RowsT::KEYS;
   constexpr int NK = RowsT::NK, ND = RowsT::ND;
   constexpr int SK = stage_keys<T, CK, CV>(), SPP = kPageTokens / SK;
-  constexpr int FK = SK / 16 * NK, FV = SK / KEYS * ND, FW = (FK + FV) / kWaves;
-  constexpr int TR = 16 * MT * kWaves;
-  static_assert(SK % KEYS == 0 && (FK + FV) % kWaves == 0, "whole fragments per wave");
+  constexpr int FK = SK / 16 * NK, FV = SK / KEYS * ND, FW = (FK + FV + W - 1) / W;
+  constexpr int TR = 16 * MT * W;
+  static_assert(SK % KEYS == 0, "whole blocks");
   __shared__ u32x4 lds[2][FK + FV][64];
 
   const int lane = lane_id(), w = wave_id_uniform();
@@ -388,19 +411,20 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gqa_rows_kernel(GqaArgs a) {
 #pragma unroll
     for (int i = 0; i < FW; ++i) {
       const int f = w * FW + i;
+      if ((FK + FV) % W && f >= FK + FV) break;
       if (f < FK) {
         const int t = f / NK, k = f % NK, d = k * KSTEP + g * (KSTEP / 4);
-        if (k * KSTEP < a.Dp)
+        if (WHOLE || k * KSTEP < a.Dp)
           load_to_lds(kp + (size_t)16 * t * a.Dp + (d < a.Dp ? d : 0), lds[buf][f]);
       } else {
         const int kb = (f - FK) / ND, n = (f - FK) % ND;
-        if (16 * n < a.Dvp)
+        if (WHOLE || 16 * n < a.Dvp)
           load_to_lds(vp + kb * KEYS + (size_t)min(16 * n + c, a.Dvp - 1) * kPageTokens,
                       lds[buf][f]);
       }
     }
   };
-  const float scale2 = a.scale * kLog2e;
+  const float scale2 = fmaxf(fabsf(a.scale) * kLog2e, 1e-30f);  // (0: -inf stays what it is)
   RowsT row;
   auto page_of = [&](int s) { return page_at(a, pt, s / SPP, s < s1); };
   int page = page_of(s0), next = page_of(s0 + 1), buf = 0;
@@ -494,11 +518,13 @@ hipError_t split(const GqaArgs& a, hipStream_t st) {
   return merge<T>(a, 16, st);
 }
 
-template <typename T, int CK, int CV, int MT>
+template <typename T, int CK, int CV, int MT, int W = kWaves>
 hipError_t rows(const GqaArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((gqa_rows_kernel<T, CK, CV, MT>), dim3(a.n_items, a.G), dim3(64 * kWaves), 0, st, a);
+  void (*const kernel)(GqaArgs) = a.Dp == CK && a.Dvp == CV ? gqa_rows_kernel<T, CK, CV, MT, W, true>
+                                                            : gqa_rows_kernel<T, CK, CV, MT, W, false>;
+  hipLaunchKernelGGL(kernel, dim3(a.n_items, a.G), dim3(64 * W), 0, st, a);
   if (hipError_t e = hipGetLastError()) return e;
-  return merge<T>(a, 16 * MT * kWaves, st);
+  return merge<T>(a, 16 * MT * W, st);
 }
 
 template <typename T>
@@ -508,8 +534,9 @@ hipError_t launch(const GqaArgs& a, int tile_rows, hipStream_t st) {
     return d <= 64 ? split<T, 64>(a, st) : d <= 128 ? split<T, 128>(a, st) : split<T, 256>(a, st);
   if constexpr (sizeof(T) == 2) {
     if (tile_rows == 128) {
-      if (d <= 64) return rows<T, 64, 64, 2>(a, st);
-      return d <= 128 ? rows<T, 128, 128, 2>(a, st) : rows<T, 192, 128, 2>(a, st);
+      if (d <= 64) return rows<T, 64, 64, 1, 8>(a, st);
+      if (a.Dp <= 96 && a.Dvp <= 64) return rows<T, 96, 64, 1, 8>(a, st);
+      return d <= 128 ? rows<T, 128, 128, 1, 8>(a, st) : rows<T, 192, 128, 1, 8>(a, st);
     }
   }
   if (d <= 64) return rows<T, 64, 64, 1>(a, st);

@@ -97,6 +97,26 @@ def test_attention_alone(serve, name, dtype):
     T.check_rows(got, want, dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (96, 64), (96, 48), (128, 128), (112, 128), (192, 128),
+                                      (160, 96)])
+@pytest.mark.parametrize("scale", [0.15, 0.5, -0.4, 0.0])
+def test_prompt_attention_classes(serve, dtype, dim, vdim, scale):
+    """Head sizes that are a class of the row kernel and sizes inside one; maxima that
+    hardly move and ones that jump, a scale below and at zero."""
+    # q and k rounded to 8 bits move a score of products of 64 to 192 normal values by some
+    # scale * sqrt(192) * 2^-9 * sqrt(2) / sqrt(3), 0.01 of every weight at 0.5 (24 bits:
+    # 2e-7); at 2 it would be BF16_TOL itself, and past FP32_TOL in the worst rows
+    cfg = one_layer(T.attn(heads=4, kv_heads=2, dim=dim, vdim=vdim, rot=32, scale=scale))
+    w = T.weights(cfg, 7)
+    t = tokens(cfg, 150, 8)
+    eng = serve(cfg, w, dtype)
+    want = T.logits(cfg, w, t)
+    T.check_rows(run_whole(eng, t), want, dtype)
+    got = T.replay(eng, {0: t}, [[(0, n)] for n in (33, 70, 46, 1)])[0]
+    T.check_rows(got, want, dtype)
+
+
 @pytest.mark.parametrize("sink", [-30.0, 0.0, 6.0, 40.0])
 def test_sink(serve, sink):
     """From no weight to nearly all of it; a sink that is left out, scaled or
