@@ -244,6 +244,93 @@ __global__ __launch_bounds__(1024) void pa_merge_row_kernel(PaMergeRowArgs a) {
   if (threadIdx.x == 0) a.inv_scale[b] = 1.0f / scale;
 }
 
+// The same for a prompt's rows: many of them, few splits each.  A thread takes four
+// neighbouring values of QPT quads, of every split one 16-byte load, and keeps them to the
+// quantisation; it works out its head's weights itself, two to four exponentials in most
+// prompts.  Bound by the partials' bytes (2048 rows of 16 x 128, three splits at most, int8
+// out: 22 us by a wave a head and values through LDS, all splits' places read, now 11).
+template <int QPT>
+__global__ __launch_bounds__(256) void pa_merge_prompt_kernel(PaMergeRowArgs a) {
+  __shared__ float sh[4];
+  const int b = blockIdx.x, hid = a.H * a.D, step = blockDim.x;
+  const int ntiles = min((min(a.ctx_p0 + b + 1, a.T) + a.TS - 1) / a.TS, a.max_tiles);
+  const int ns = min(a.nsplit, (ntiles + a.pps - 1) / a.pps);
+  f32x4 v[QPT];
+  const auto merge = [&](auto N) {  // N: the row's splits, 0: more than the cases below
+    constexpr int AT_ONCE = decltype(N)::value ? decltype(N)::value : 4;
+#pragma unroll
+    for (int i = 0; i < QPT; ++i) {
+      const int at = 4 * (threadIdx.x + i * step), h = at / a.D;
+      v[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (at >= hid) continue;
+      const size_t first = ((size_t)b * a.H + h) * a.nsplit;
+      const float2* ml = reinterpret_cast<const float2*>(a.part_ml) + first;
+      const float* pa = a.part_acc + first * a.D + at % a.D;
+      float M = kNegSentinel, L = 0.f;
+      if constexpr (decltype(N)::value == 0)
+#pragma unroll 4
+        for (int s = AT_ONCE; s < ns; ++s) M = fmaxf(M, ml[s].x);
+      f32x4 x[AT_ONCE];
+      float2 st[AT_ONCE];
+#pragma unroll
+      for (int s = 0; s < AT_ONCE; ++s) {
+        x[s] = *reinterpret_cast<const f32x4*>(pa + (size_t)s * a.D);
+        st[s] = ml[s];
+      }
+#pragma unroll
+      for (int s = 0; s < AT_ONCE; ++s) M = fmaxf(M, st[s].x);
+#pragma unroll
+      for (int s = 0; s < AT_ONCE; ++s) {
+        const float w = __builtin_amdgcn_exp2f(st[s].x - M);
+        L += st[s].y * w;
+        v[i] += x[s] * w;
+      }
+      if constexpr (decltype(N)::value == 0)
+#pragma unroll 4
+        for (int s = AT_ONCE; s < ns; ++s) {
+          const float w = __builtin_amdgcn_exp2f(ml[s].x - M);
+          L += ml[s].y * w;
+          v[i] += *reinterpret_cast<const f32x4*>(pa + (size_t)s * a.D) * w;
+        }
+      v[i] *= M <= 0.5f * kNegSentinel ? 0.f : 1.0f / (L + 1e-6f);
+    }
+  };
+  switch (ns) {
+    case 1: merge(std::integral_constant<int, 1>{}); break;
+    case 2: merge(std::integral_constant<int, 2>{}); break;
+    case 3: merge(std::integral_constant<int, 3>{}); break;
+    case 4: merge(std::integral_constant<int, 4>{}); break;
+    default: merge(std::integral_constant<int, 0>{});
+  }
+  float am = 0.f;
+#pragma unroll
+  for (int i = 0; i < QPT; ++i) {
+    const int at = 4 * (threadIdx.x + i * step);
+    if (at >= hid) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) am = fmaxf(am, fabsf(v[i][e]));
+    if (a.out) *reinterpret_cast<f32x4*>(a.out + (size_t)b * hid + at) = v[i];
+    if (a.out16)
+      *reinterpret_cast<ln_f16x4*>(
+          a.out16 + (a.pack ? a_frag_off_f16(b, at, hid >> 5) : (size_t)b * hid + at)) = ln_half4(v[i]);
+  }
+  if (!a.q) return;
+  am = ln_wave_max(am);
+  if (lane_id() == 0) sh[wave_id_uniform()] = am;
+  __syncthreads();
+  am = sh[0];
+  for (int i = 1; i < step >> 6; ++i) am = fmaxf(am, sh[i]);
+  const float scale = 127.f / (am + 1e-6f);
+#pragma unroll
+  for (int i = 0; i < QPT; ++i) {
+    const int at = 4 * (threadIdx.x + i * step);
+    if (at < hid)
+      *reinterpret_cast<uint32_t*>(
+          a.q + (a.pack ? a_frag_off_i8(b, at, hid >> 6) : (size_t)b * hid + at)) = ln_quant4(v[i], scale);
+  }
+  if (threadIdx.x == 0) a.inv_scale[b] = 1.0f / scale;
+}
+
 namespace {
 
 constexpr int kMinPps = 8;
@@ -538,6 +625,18 @@ int llm::pa_merge_rows_internal(const float* part_acc, const float* part_ml, flo
                     rows ? rows->inv_scale : nullptr,
                     rows ? static_cast<_Float16*>(rows->out16) : nullptr, context_lens, B, H, D, T,
                     TS, pps, nsplit, max_tiles, rows ? rows->pack : 0, ctx_p0};
+  // a prompt's rows (more splits a row than 16: one after the other they cost more than the
+  // waves of a row that take a head each)
+  const int quads = H * D / 4;
+  if (ctx_p0 >= 0 && !context_lens && pps > 0 && nsplit <= 16 && D % 64 == 0 && quads <= 1024) {
+    const int per_row = std::min((quads + 63) / 64 * 64, 256);
+    const auto kernel = quads <= 256   ? pa_merge_prompt_kernel<1>
+                        : quads <= 512 ? pa_merge_prompt_kernel<2>
+                                       : pa_merge_prompt_kernel<4>;
+    hipLaunchKernelGGL(kernel, dim3(B), dim3(per_row), 0, st, mg);
+    LLM_HIP_RET(hipGetLastError());
+    return LLM_OK;
+  }
   // one wave per head (heads past 16 loop); a prompt's rows fill the chip by themselves,
   // and four waves each leave room for four times the rows on a CU
   const int threads = 64 * std::min(B >= 1024 ? 4 : 16, H);

@@ -117,6 +117,19 @@ def test_prompt_attention_classes(serve, dtype, dim, vdim, scale):
     T.check_rows(got, want, dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim,vdim", [(24, 7), (64, 64), (80, 72), (128, 128), (256, 200)])
+def test_prompt_merges(serve, dtype, dim, vdim):
+    """Tiles cut into pieces, of up to 16, 32 and 64 lanes a row, whole quads of a row and not."""
+    cfg = one_layer(T.attn(heads=4, kv_heads=2, dim=dim, vdim=vdim, rot=10, scale=dim ** -0.5))
+    w = T.weights(cfg, 9)
+    t = tokens(cfg, 900, 10)
+    eng = serve(cfg, w, dtype, max_tokens=2048)
+    want = T.logits(cfg, w, t)
+    T.check_rows(run_whole(eng, t), want, dtype)
+    T.check_rows(T.replay(eng, {0: t}, [[(0, 700)], [(0, 200)]])[0], want, dtype)
+
+
 @pytest.mark.parametrize("sink", [-30.0, 0.0, 6.0, 40.0])
 def test_sink(serve, sink):
     """From no weight to nearly all of it; a sink that is left out, scaled or

@@ -111,6 +111,24 @@ def test_pa_prefill_tile_edges(gpu, oracle, D, ts, p0, m):
         assert_parity(out, ref, RTOL, ATOL_FRAC)
 
 
+@pytest.mark.parametrize("H,D", [(2, 64), (7, 64), (12, 64), (16, 128), (31, 128), (33, 128)])
+@pytest.mark.parametrize("p0,m", [(0, 300), (900, 70), (2000, 17)])
+def test_pa_prefill_merges(gpu, oracle, H, D, p0, m):
+    """Rows of one to many splits and of one to four quads a thread, some past the prompt
+    merge's widest; rows whose pages are missing altogether."""
+    import llm_capi
+    rng = np.random.default_rng(H + p0 + m)
+    kp, vp, pt = _case(rng, rows=1, H=H, D=D, T=p0 + m, ts=16)
+    pt[0, H // 2] = -1
+    q = (rng.standard_normal((m, H, D)) * D ** -0.25).astype(np.float32)
+    out = llm_capi.pa_prefill(_dev(q), _dev(kp), _dev(vp), _dev(pt), row=0, p0=p0).cpu().numpy()
+    assert (out[:, H // 2] == 0).all()
+    at = np.r_[0:m:max(1, m // 5), m - 1]  # rows of their own contexts
+    for i in at:
+        ref = _oracle(oracle, q[i:i + 1], kp, vp, pt, 0, p0 + int(i))
+        assert_parity(out[i:i + 1], ref, RTOL, ATOL_FRAC)
+
+
 def test_pa_prefill_missing_pages_and_scale(gpu, oracle):
     import llm_capi
     rng = np.random.default_rng(11)
