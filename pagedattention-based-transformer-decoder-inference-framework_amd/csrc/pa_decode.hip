@@ -252,7 +252,8 @@ __global__ __launch_bounds__(1024) void pa_merge_row_kernel(PaMergeRowArgs a) {
 template <int QPT>
 __global__ __launch_bounds__(256) void pa_merge_prompt_kernel(PaMergeRowArgs a) {
   __shared__ float sh[4];
-  const int b = blockIdx.x, hid = a.H * a.D, step = blockDim.x;
+  const int b = a.pack ? packed_row(blockIdx.x, gridDim.x) : blockIdx.x;
+  const int hid = a.H * a.D, step = blockDim.x;
   const int ntiles = min((min(a.ctx_p0 + b + 1, a.T) + a.TS - 1) / a.TS, a.max_tiles);
   const int ns = min(a.nsplit, (ntiles + a.pps - 1) / a.pps);
   f32x4 v[QPT];
