@@ -370,7 +370,7 @@ __global__ __launch_bounds__(256) void fill_random_f16_kernel(_Float16* __restri
   for (; i < n; i += stride) {
     const size_t page = i / page_elems;
     struct alignas(2 * E) {
-      _Float16 x[E];
+      uint16_t x[E];
     } out;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
@@ -381,7 +381,11 @@ __global__ __launch_bounds__(256) void fill_random_f16_kernel(_Float16* __restri
       float u = 0.f;
 #pragma unroll
       for (int k = 0; k < 4; ++k) u += (float)((z >> (16 * k)) & 0xFFFF) * (1.0f / 65536.0f);
-      out.x[e] = (_Float16)((u - 2.0f) * 1.7320508f * scale);
+      // (rounded once: which the compiler takes, this or a product and a conversion, would
+      // depend on E)
+      uint32_t h;
+      asm("v_fma_mixlo_f16 %0, %1, %2, 0\n\ts_nop 0" : "=v"(h) : "v"((u - 2.0f) * 1.7320508f), "s"(scale));
+      out.x[e] = (uint16_t)h;
     }
     *reinterpret_cast<decltype(out)*>(p + page * page_stride + (i - page * page_elems)) = out;
   }

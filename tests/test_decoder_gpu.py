@@ -773,3 +773,33 @@ def test_forced_hidden_2048_tile_forms(gpu, oracle, rows):
     _, worst, n_vals, n_flips = _forced_lockstep(dec, OracleDecoder(oracle, w, rows), taps,
                                                  prompts, gen=4, V=512)
     assert n_flips < 1e-3 * n_vals, (n_flips, n_vals)
+
+
+@pytest.mark.parametrize("max_batch,max_seq", [(1, 40), (4, 2048)])  # a thread an element, and eight
+def test_synthetic_context_bits(gpu, oracle, max_batch, max_seq):
+    """The random context of a seed: splitmix64, the sum of its four 16-bit parts, one rounding
+    to fp16 of the scaled value."""
+    import ctypes
+
+    import llm_capi
+    from _util import hip_copy_to_host
+    w = _int8_model(oracle, S=max_seq)
+    dec = _make_gpu_decoder(w, max_batch)
+    dec.begin_synthetic(1, 0, 9, False)
+    lib, kv = llm_capi.load(), ctypes.c_void_p(dec.kv_handle)
+    pages, ts, D = lib.kv_cache_num_pages(kv), 16, w["cfg"]["D"]
+    pool = np.empty((pages, 2, ts, D), np.float16)
+    hip_copy_to_host(pool, lib.kv_cache_k_pool(kv))
+    n = pages * ts * D
+    at = np.r_[0:min(n, 5000), max(0, n - 5000):n]
+    for which, scale in ((0, np.float32(0.05)), (1, np.float32(1.0))):
+        with np.errstate(over="ignore"):
+            z = np.uint64(9 * 2 + 1 + which) + np.uint64(0x9E3779B97F4A7C15) * (at.astype(np.uint64) + np.uint64(1))
+            z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+            z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        z ^= z >> np.uint64(31)
+        u = sum(((z >> np.uint64(16 * k)) & np.uint64(0xFFFF)).astype(np.float64) for k in range(4)) / 65536
+        x = (u - 2).astype(np.float32) * np.float32(1.7320508)
+        want = (x.astype(np.float64) * np.float64(scale)).astype(np.float16)
+        got = pool[:, which].reshape(-1)[at]
+        assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), which
