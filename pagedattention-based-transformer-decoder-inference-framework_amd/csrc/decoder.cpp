@@ -133,6 +133,7 @@ struct llm_decoder {
   bool oproj_fusable(const struct Rows& R);
   bool wgm_quant_ok(const struct Rows& R);
   bool fc2_split(const struct Rows& R) const;
+  bool fc2_quant_prologue(const struct Rows& R) const;
   int layer_post(int l, hipStream_t st, const struct Rows& R);
   struct Rows step_rows(int r0, int n, uint8_t* ws);
   int step_head(hipStream_t st, int r0, int n);
@@ -534,6 +535,16 @@ bool llm_decoder::fc2_split(const Rows& R) const {
          !ln_fusable(wdtype, R.n, hid) && inter / 64 >= 16;
 }
 
+// INT8 decode rows whose fc2 quantises its own input: a row for each of the prologue's waves,
+// of an intermediate size that its registers hold.  Every workgroup of fc2 does it again, which
+// costs less than the quantising launch up to there (us a step of 8 layers, launch and prologue,
+// hidden 256: 1 row 190 and 180, 8 rows 203 and 193, 16 rows 223 and 225; 512: 208 and 197, 229
+// and 225, 257 and 266).
+bool llm_decoder::fc2_quant_prologue(const Rows& R) const {
+  return wdtype == LLM_I8 && R.prefill_row < 0 && R.n <= 8 && !fc2_split(R) &&
+         quant_prologue_ok(R.n, hid, inter);
+}
+
 int llm_decoder::layer_attn(int l, hipStream_t st, const Rows& R, PaPlan* plan) {
   pa_kv_view view;
   RET_IF(kv_cache_view(kv, l, &view));
@@ -625,14 +636,22 @@ int llm_decoder::layer_post(int l, hipStream_t st, const Rows& R) {
   g.C16 = nullptr;
   if (!i8) g.A = R.act2;
   // quantise h1 -> mlp_fc2 (+b2)
-  if (i8)
-    LLM_HIP_RET(launch_quantize_rows(R.h1, R.n, inter, static_cast<int8_t*>(R.act), R.sa, st, 1));
-  RET_IF(tap(l, 3, R, inter, st));
+  const bool qpro2 = fc2_quant_prologue(R);
+  if (qpro2) {
+    g.ln_x = R.h1;
+    g.ln_quant_only = 1;
+    if (tap_q) { g.act_out = R.act; g.sa_out = R.sa; }
+  } else {
+    if (i8)
+      LLM_HIP_RET(launch_quantize_rows(R.h1, R.n, inter, static_cast<int8_t*>(R.act), R.sa, st, 1));
+    RET_IF(tap(l, 3, R, inter, st));
+  }
   g.W_packed = w2.p + sz_2 * l; g.N = hid; g.K = inter; g.C = R.x;
   g.bias = b2.p + lh; g.act = LLM_ACT_NONE;
   if (i8) g.sw = sw2.p + lh;
   g.ksplit2 = split_fc2 ? 1 : 0;  // (x was zeroed by the LN2 launch)
-  return weight_gemm(g, st);
+  RET_IF(weight_gemm(g, st));
+  return qpro2 ? tap(l, 3, R, inter, st) : LLM_OK;
 }
 
 // Rows r0 .. r0 + n - 1 of the decode-step buffers.

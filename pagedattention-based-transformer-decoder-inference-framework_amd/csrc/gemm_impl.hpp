@@ -162,7 +162,8 @@ struct GemmTraits<GemmKind::F16> {
 // w, w + WAVES, ...), two rows' loads in flight; gamma / beta loaded once.
 // CPL: float4 chunks per lane that cover K, so that a row of 256 is not worked on as
 // one of 2048; a wave without a row does nothing, and rows past M stay as they are (each
-// row of A makes its own row of C).  One row of 256: PENDING_F.
+// row of A makes its own row of C).  1 x 768 x 256 with its KV append 7.5 us, now 4.3; 1 x 256 x
+// 256 behind the attention 5.0, now 3.5.
 template <GemmKind KIND, int ROWS, int WAVES, int CPL>
 __device__ __forceinline__ void ln_prologue_rows(const GemmArgs& a, int m0, uint8_t* alds, float* sa_lds) {
   constexpr int ESIZE = GemmTraits<KIND>::ESIZE;
