@@ -106,8 +106,8 @@ struct llm_decoder {
   float* tap_s = nullptr;
   int tap(int l, int stage, const struct Rows& R, int K, hipStream_t st);
   int layer_norm_into(WeightGemm& g, const struct Rows& R, const float* gamma, const float* beta,
-                      hipStream_t st, float* zero_x = nullptr);
-  LnSource embed_src;  // set by step_head: the next LayerNorm reads E[token] rows
+                      hipStream_t st);
+  LnSource embed_src;  // set by embed_rows: the next LayerNorm reads E[token] rows
 
   ~llm_decoder() {
     if (h_oflag) (void)hipHostFree(h_oflag);
@@ -136,7 +136,7 @@ struct llm_decoder {
   bool fc2_quant_prologue(const struct Rows& R) const;
   int layer_post(int l, hipStream_t st, const struct Rows& R);
   struct Rows step_rows(int r0, int n, uint8_t* ws);
-  int step_head(hipStream_t st, int r0, int n);
+  void embed_rows(const int32_t* tok);
   int step_tail(hipStream_t st, int r0, int n);
   int next_tokens(const float* xr, int n, int r0, const int32_t* ctr, hipStream_t st,
                   int32_t* adv_pos = nullptr, int32_t* adv_ctx = nullptr);
@@ -451,18 +451,17 @@ int llm_decoder::layer_pre(int l, hipStream_t st, const Rows& R) {
 // the rows' A image fits in LDS (decode rows), else a LayerNorm (+ quant)
 // launch writing the packed A the GEMM reads.
 int llm_decoder::layer_norm_into(WeightGemm& g, const Rows& R, const float* gamma,
-                                 const float* beta, hipStream_t st, float* zero_x) {
-  // the step's first LayerNorm reads the token embedding rows (step_head)
+                                 const float* beta, hipStream_t st) {
+  // the first LayerNorm reads the token embedding rows (embed_rows)
   LnSource src = embed_src;
   embed_src = LnSource{};
-  src.zero_x = zero_x;  // (the LayerNorm launch only: the caller checks fc2_split)
   if (R.prefill_row < 0 && ln_fusable(wdtype, R.n, hid)) {
     g.ln_x = R.x; g.ln_g = gamma; g.ln_b = beta; g.ln_eps = 1e-5f;
     g.ln_emb = src.emb; g.ln_tok = src.tok; g.ln_V = src.V;
     if (tap_q) { g.act_out = R.act; g.sa_out = R.sa; }  // the taps read A and the scales back
     return LLM_OK;
   }
-  const LnSource* pp = src.emb || src.zero_x ? &src : nullptr;
+  const LnSource* pp = src.emb ? &src : nullptr;
   if (wdtype == LLM_I8)
     LLM_HIP_RET(launch_layernorm_quant(R.x, R.n, hid, gamma, beta, 1e-5f, nullptr,
                                        static_cast<int8_t*>(R.act), R.sa, st, 1, pp));
@@ -522,17 +521,18 @@ bool llm_decoder::wgm_quant_ok(const Rows& R) {
 // 128 column tiles leave half the CUs idle, so it runs as two k slices that
 // each add their dequantised half into x (fp32 atomics; two addends commute,
 // so x is the same bits whichever lands first).  x must be zero when fc2
-// starts: the LN2 launch, the last reader of the o_proj output in x, writes
-// zeros over the rows after loading them.  Standalone (scripts/tune_gemm_sk.py,
+// starts: fc1 is the last reader of the o_proj output in x, and the launch that
+// quantises fc1's rows sets it to zero.  Standalone (scripts/tune_gemm_sk.py,
 // profiles/r05/gemm_small_m.txt): fc2 at M = 8 6.86 -> 5.67 us, M = 16 7.53 ->
 // 5.95 us.
-// Round 6: also at 33..64 rows when inter >= 16384 (C5's fc2, K 16384): every
+// 4 layers of hidden 768: 126 -> 124 us a step of one row, 155.5 -> 153 of 16.
+// Also at 33..64 rows when inter >= 16384 (C5's fc2, K 16384): every
 // workgroup of the one-slice form reads all of A, 1 MB, the k slices half of
 // it (gemm_impl.hpp narrow_decode_tile).
 bool llm_decoder::fc2_split(const Rows& R) const {
   return wdtype == LLM_I8 && R.prefill_row < 0 &&
          (R.n <= 16 || (R.n > 32 && R.n <= 64 && inter >= 16384)) &&
-         !ln_fusable(wdtype, R.n, hid) && inter / 64 >= 16;
+         inter / 64 >= 16 && !fc2_quant_prologue(R);
 }
 
 // INT8 decode rows whose fc2 quantises its own input: a row for each of the prologue's waves,
@@ -541,8 +541,7 @@ bool llm_decoder::fc2_split(const Rows& R) const {
 // hidden 256: 1 row 190 and 180, 8 rows 203 and 193, 16 rows 223 and 225; 512: 208 and 197, 229
 // and 225, 257 and 266).
 bool llm_decoder::fc2_quant_prologue(const Rows& R) const {
-  return wdtype == LLM_I8 && R.prefill_row < 0 && R.n <= 8 && !fc2_split(R) &&
-         quant_prologue_ok(R.n, hid, inter);
+  return wdtype == LLM_I8 && R.prefill_row < 0 && R.n <= 8 && quant_prologue_ok(R.n, hid, inter);
 }
 
 int llm_decoder::layer_attn(int l, hipStream_t st, const Rows& R, PaPlan* plan) {
@@ -618,7 +617,7 @@ int llm_decoder::layer_post(int l, hipStream_t st, const Rows& R) {
   RET_IF(tap(l, 1, R, hid, st));
   // LN2 -> mlp_fc1 (+b1, ReLU)
   const bool split_fc2 = fc2_split(R);
-  RET_IF(layer_norm_into(g, R, ln2_g.p + lh, ln2_b.p + lh, st, split_fc2 ? R.x : nullptr));
+  RET_IF(layer_norm_into(g, R, ln2_g.p + lh, ln2_b.p + lh, st));
   g.W_packed = w1.p + sz_1 * l; g.N = inter; g.K = hid;
   g.bias = b1.p + (size_t)l * inter; g.act = LLM_ACT_RELU;
   if (i8) {
@@ -643,13 +642,14 @@ int llm_decoder::layer_post(int l, hipStream_t st, const Rows& R) {
     if (tap_q) { g.act_out = R.act; g.sa_out = R.sa; }
   } else {
     if (i8)
-      LLM_HIP_RET(launch_quantize_rows(R.h1, R.n, inter, static_cast<int8_t*>(R.act), R.sa, st, 1));
+      LLM_HIP_RET(launch_quantize_rows(R.h1, R.n, inter, static_cast<int8_t*>(R.act), R.sa, st, 1,
+                                       split_fc2 ? R.x : nullptr, hid));
     RET_IF(tap(l, 3, R, inter, st));
   }
   g.W_packed = w2.p + sz_2 * l; g.N = hid; g.K = inter; g.C = R.x;
   g.bias = b2.p + lh; g.act = LLM_ACT_NONE;
   if (i8) g.sw = sw2.p + lh;
-  g.ksplit2 = split_fc2 ? 1 : 0;  // (x was zeroed by the LN2 launch)
+  g.ksplit2 = split_fc2 ? 1 : 0;  // (x was zeroed by the quantising launch)
   RET_IF(weight_gemm(g, st));
   return qpro2 ? tap(l, 3, R, inter, st) : LLM_OK;
 }
@@ -717,16 +717,13 @@ int llm_decoder::next_tokens(const float* xr, int n, int r0, const int32_t* ctr,
   return LLM_OK;
 }
 
-// The step's embedding: no launch of its own; layer 0's first LayerNorm
-// (launch or GEMM prologue) reads E[token] rows directly (embed_src).
-int llm_decoder::step_head(hipStream_t st, int r0, int n) {
-  (void)st;
+// The embedding of rows of tokens: no launch of its own; layer 0's first LayerNorm
+// (launch or GEMM prologue) reads E[token] rows directly.
+void llm_decoder::embed_rows(const int32_t* tok) {
   embed_src = LnSource{};
   embed_src.emb = reinterpret_cast<const _Float16*>(emb.p);
-  embed_src.tok = tokens.p + r0;
+  embed_src.tok = tok;
   embed_src.V = V;
-  (void)n;
-  return LLM_OK;
 }
 
 int llm_decoder::step_tail(hipStream_t st, int r0, int n) {
@@ -738,7 +735,7 @@ int llm_decoder::enqueue_step(hipStream_t st) {
   Rows R = step_rows(0, batch, attn_ws.p);
   if (oproj_fusable(R)) R.oacc = oacc.p, R.oproj_out = R.x, R.oflag = oflag.p;
   R.wgm_quant = wgm_quant_ok(R);
-  RET_IF(step_head(st, 0, batch));
+  embed_rows(tokens.p);
   for (int l = 0; l < L; ++l) {
     RET_IF(layer_pre(l, st, R));
     RET_IF(layer_attn(l, st, R));
@@ -917,8 +914,7 @@ int llm_decoder::prefill(int row, const int32_t* toks, int n, hipStream_t st) {
     R.prefill_row = row;
     R.prefill_p0 = p0;
     R.attn_ws = pws.p; R.attn_ws_bytes = pws_bytes;
-    LLM_HIP_RET(launch_embed(emb.p, pmeta.p + 3 * C, m, hid, V, px.p, st));
-    embed_src = LnSource{};  // (a failed step enqueue could have left it set)
+    embed_rows(pmeta.p + 3 * C);
     for (int l = 0; l < L; ++l) {
       RET_IF(layer_pre(l, st, R));
       RET_IF(layer_attn(l, st, R));
@@ -985,8 +981,7 @@ int llm_decoder::forward_mixed(const std::vector<StepSeq>& seqs, float* logits_d
   R.prefill_row = seqs[0].slot;
   R.prefill_p0 = seqs[0].p0;
   R.attn_ws = pws.p; R.attn_ws_bytes = pws_bytes;
-  LLM_HIP_RET(launch_embed(emb.p, pmeta.p + 3 * C, n, hid, V, px.p, st));
-  embed_src = LnSource{};
+  embed_rows(pmeta.p + 3 * C);
   for (int l = 0; l < L; ++l) {
     RET_IF(layer_pre(l, st, R));
     RET_IF(layer_attn(l, st, R));

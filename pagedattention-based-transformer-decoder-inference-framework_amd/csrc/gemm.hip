@@ -86,7 +86,9 @@ extern "C" int f16_gemm(const void* A, int lda, const void* W_packed, float* C, 
 // at only ~80-120 GB/s (scripts/micro/bcast_read.hip: 256 KB per workgroup
 // +2.2 us, 512 KB +6.4 us).  Same-box A/B of the decode step
 // (scripts/gpu_ab.sh): C2 (16 rows x 768, 48 KB) +1.5-5 %; C4 (32 x 2048,
-// 256 KB) -7 %; C3 (64 x 2048, 512 KB) -4 %.  So: at most 64 KB of rows.
+// 256 KB) -7 %; C3 (64 x 2048, 512 KB) -4 %.  So: at most 64 KB of rows, tiles
+// counted whole: a row of 2048 takes its wave longer than the launch (4 layers, 1 row: 185 us a
+// step with the launches, 192 without; 8 rows 192 and 224).
 bool llm::ln_fusable(int dtype, int M, int K) {
   const int es = dtype == LLM_I8 ? 1 : 2;
   if (K % 16 != 0 || (K * es) % 256 != 0 || K > 2048) return false;

@@ -66,15 +66,12 @@ struct WeightGemm {
   int ksplit2 = 0;
 };
 
-// Input of a LayerNorm when it is not x: embedding rows E[tok[r]] (the decode
-// step's first LayerNorm reads the token embedding directly, no embed launch).
+// Input of a LayerNorm when it is not x: embedding rows E[tok[r]] (a step's or a prompt's
+// first LayerNorm reads the token embedding directly, no embed launch).
 struct LnSource {
   const _Float16* emb = nullptr;
   const int32_t* tok = nullptr;
   int V = 0;
-  // optional (x rows only): the launch writes zeros over the rows it read,
-  // once they are loaded (the next GEMM accumulates into them: ksplit2)
-  float* zero_x = nullptr;
 };
 
 int weight_gemm(const WeightGemm& g, hipStream_t st);

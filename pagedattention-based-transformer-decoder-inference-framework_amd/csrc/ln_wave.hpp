@@ -64,7 +64,7 @@ __device__ __forceinline__ void ln_wave_load_f16(const _Float16* __restrict__ ro
   }
 }
 
-// Embedding row of token id tok (clamped to [0, V), as embed_kernel).
+// Embedding row of token id tok (clamped to [0, V)).
 __device__ __forceinline__ const _Float16* ln_embed_row(const _Float16* E, const int32_t* tok,
                                                         int m, int V, int K) {
   int t = tok[m];

@@ -130,10 +130,11 @@ __device__ __forceinline__ uint32_t pack4_i8(f32x4 y, float scale) {
 }
 
 // pack = 1: q / out16 are written in packed-A order (a_frag_off_*), else row-major.
+// zero: rows of zero_n4 quads set to zero on the way.
 template <int VPT>
 __global__ __launch_bounds__(kRowThreads) void quantize_rows_v_kernel(
     const float* __restrict__ x, int cols, int8_t* __restrict__ q, float* __restrict__ inv_scale,
-    int pack) {
+    int pack, f32x4* __restrict__ zero, int zero_n4) {
   __shared__ float sh[4];
   const int r = pack ? packed_row(blockIdx.x, gridDim.x) : blockIdx.x;
   const int n4 = cols >> 2;
@@ -162,6 +163,8 @@ __global__ __launch_bounds__(kRowThreads) void quantize_rows_v_kernel(
     }
   }
   if (threadIdx.x == 0) inv_scale[r] = 1.0f / scale;
+  if (zero)
+    for (int c = threadIdx.x; c < zero_n4; c += kRowThreads) zero[(size_t)r * zero_n4 + c] = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
 // LayerNorm (+ int8 quantisation) launch, one 256-thread workgroup per row:
@@ -174,7 +177,7 @@ __global__ __launch_bounds__(kRowThreads) void quantize_rows_v_kernel(
 // q / out16 in packed-A order when pack.
 template <int VPT>
 __global__ __launch_bounds__(kRowThreads) void layernorm_rows_kernel(
-    const float* x /* not restrict: pp.zero_x may point at it (fc2_split) */, int rows, int cols, const float* __restrict__ gamma,
+    const float* __restrict__ x, int rows, int cols, const float* __restrict__ gamma,
     const float* __restrict__ beta, float eps, float* __restrict__ out, int8_t* __restrict__ q,
     float* __restrict__ inv_scale, _Float16* __restrict__ out16, int pack, LnSource pp) {
   __shared__ float sh[4];
@@ -183,7 +186,7 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_rows_kernel(
   const f32x4* g4 = reinterpret_cast<const f32x4*>(gamma);
   const f32x4* b4 = reinterpret_cast<const f32x4*>(beta);
   f32x4 v[VPT], gv[VPT], bv[VPT];
-  if (pp.emb) {  // x = E[tok[r]] (embed_kernel's values, not stored)
+  if (pp.emb) {  // x = E[tok[r]] (TokenEmbedding::forward, decoder/token_embedding.hpp:19-26)
     typedef _Float16 h4 __attribute__((ext_vector_type(4)));
     const h4* er = reinterpret_cast<const h4*>(ln_embed_row(pp.emb, pp.tok, r, pp.V, cols));
 #pragma unroll
@@ -210,13 +213,6 @@ __global__ __launch_bounds__(kRowThreads) void layernorm_rows_kernel(
 #pragma unroll
   for (int i = 0; i < VPT; ++i) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
   const float mean = block_sum_fast(s, sh) / (float)cols;
-  if (pp.zero_x && !pp.emb) {  // (after the barrier in block_sum_fast: every thread's loads are done)
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      const int c = threadIdx.x + i * kRowThreads;
-      if (c < n4) reinterpret_cast<f32x4*>(pp.zero_x + (size_t)r * cols)[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
   float vs = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
@@ -312,19 +308,6 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_kernel(const float* __r
   }
 }
 
-// x[b] = float(E[tok[b]]) (TokenEmbedding::forward, decoder/token_embedding.hpp:19-26).
-__global__ __launch_bounds__(kRowThreads) void embed_kernel(const _Float16* __restrict__ E,
-                                                            const int32_t* __restrict__ tok,
-                                                            int hid, int V,
-                                                            float* __restrict__ x) {
-  const int b = blockIdx.x;
-  int t = tok[b];
-  t = t < 0 ? 0 : (t >= V ? V - 1 : t);
-  const _Float16* e = E + (size_t)t * hid;
-  float* xr = x + (size_t)b * hid;
-  for (int i = threadIdx.x; i < hid; i += blockDim.x) xr[i] = (float)e[i];
-}
-
 // pack_cols > 0: y is packed-A fp16 of rows of pack_cols (x row-major [n / pack_cols][pack_cols]).
 __global__ void to_f16_kernel(const float* __restrict__ x, size_t n, _Float16* __restrict__ y,
                               int pack_cols) {
@@ -395,16 +378,18 @@ __global__ __launch_bounds__(256) void fill_random_f16_kernel(_Float16* __restri
 // host launchers (internal)
 // ---------------------------------------------------------------------------
 hipError_t launch_quantize_rows(const float* x, int rows, int cols, int8_t* q, float* inv,
-                                hipStream_t st, int pack) {
+                                hipStream_t st, int pack, float* zero, int zero_cols) {
   const dim3 g(rows), b(kRowThreads);
-  const int v = row_vpt(cols);
+  const int v = row_vpt(cols), zn = zero_cols / 4;
+  f32x4* const z = reinterpret_cast<f32x4*>(zero);
   if (pack && (v == 0 || cols % 64 != 0)) return hipErrorInvalidValue;
+  if (zero && (v == 0 || zero_cols % 4 != 0)) return hipErrorInvalidValue;
   switch (v) {
-    case 1: hipLaunchKernelGGL(quantize_rows_v_kernel<1>, g, b, 0, st, x, cols, q, inv, pack); break;
-    case 2: hipLaunchKernelGGL(quantize_rows_v_kernel<2>, g, b, 0, st, x, cols, q, inv, pack); break;
-    case 4: hipLaunchKernelGGL(quantize_rows_v_kernel<4>, g, b, 0, st, x, cols, q, inv, pack); break;
-    case 8: hipLaunchKernelGGL(quantize_rows_v_kernel<8>, g, b, 0, st, x, cols, q, inv, pack); break;
-    case 16: hipLaunchKernelGGL(quantize_rows_v_kernel<16>, g, b, 0, st, x, cols, q, inv, pack); break;
+    case 1: hipLaunchKernelGGL(quantize_rows_v_kernel<1>, g, b, 0, st, x, cols, q, inv, pack, z, zn); break;
+    case 2: hipLaunchKernelGGL(quantize_rows_v_kernel<2>, g, b, 0, st, x, cols, q, inv, pack, z, zn); break;
+    case 4: hipLaunchKernelGGL(quantize_rows_v_kernel<4>, g, b, 0, st, x, cols, q, inv, pack, z, zn); break;
+    case 8: hipLaunchKernelGGL(quantize_rows_v_kernel<8>, g, b, 0, st, x, cols, q, inv, pack, z, zn); break;
+    case 16: hipLaunchKernelGGL(quantize_rows_v_kernel<16>, g, b, 0, st, x, cols, q, inv, pack, z, zn); break;
     default: hipLaunchKernelGGL(quantize_rows_kernel, g, b, 0, st, x, cols, q, inv); break;
   }
   return hipGetLastError();
@@ -465,13 +450,6 @@ hipError_t launch_argmax(const float* logits, int rows, int V, int32_t* out, int
                          int out2_stride, hipStream_t st) {
   hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(kArgmaxThreads), 0, st, logits, V, out, out2,
                      out2_stride);
-  return hipGetLastError();
-}
-
-hipError_t launch_embed(const void* E, const int32_t* tok, int rows, int hid, int V, float* x,
-                        hipStream_t st) {
-  hipLaunchKernelGGL(embed_kernel, dim3(rows), dim3(kRowThreads), 0, st,
-                     static_cast<const _Float16*>(E), tok, hid, V, x);
   return hipGetLastError();
 }
 

@@ -10,8 +10,9 @@ namespace llm {
 
 // pack = 1: int8 / fp16 outputs in packed-A order (common.hpp a_frag_off_*;
 // needs cols % 64 == 0), consumed by the weight GEMMs with a_packed.
+// zero (optional): as many rows of zero_cols floats set to zero on the way.
 hipError_t launch_quantize_rows(const float* x, int rows, int cols, int8_t* q, float* inv,
-                                hipStream_t st, int pack = 0);
+                                hipStream_t st, int pack = 0, float* zero = nullptr, int zero_cols = 0);
 struct LnSource;
 // pp (optional): read the rows as embedding rows E[tok[r]] instead of x
 // (gemm.hpp LnSource)
@@ -25,8 +26,6 @@ hipError_t launch_to_f16(const float* x, size_t n, void* y, hipStream_t st, int 
 hipError_t launch_advance(int32_t* pos, int32_t* ctx, int n, hipStream_t st);
 hipError_t launch_argmax(const float* logits, int rows, int V, int32_t* out, int32_t* out2,
                          int out2_stride, hipStream_t st);
-hipError_t launch_embed(const void* E, const int32_t* tok, int rows, int hid, int V, float* x,
-                        hipStream_t st);
 hipError_t launch_scatter_i32(int32_t* dst, const int64_t* idx, const int32_t* val, int n,
                               hipStream_t st);
 // LM head (csrc/lm_head.hip): logits = x . E^T (E packed by launch_lm_pack); with part_val/part_idx also the
