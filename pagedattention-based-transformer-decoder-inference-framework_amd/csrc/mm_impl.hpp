@@ -1090,6 +1090,11 @@ template <typename T, int EPI>
 hipError_t launch(const KernelArgs& p, hipStream_t st) {
   const int M = p.a.M, N = p.a.N;
   const int ntiles = (N + 15) / 16;
+  // A model's head: blocks of two tiles, which read A half as often, by four waves of twice the
+  // k-steps (32768 x 2048, 16 rows 31.2 us by the form below, 27.2 by eight waves, 25.8 so; one
+  // row 31.6, 30.2, 29.9)
+  if constexpr (EPI == kStore && Kind<T>::BF16)
+    if (M <= 16 && ntiles >= 2048) return stream<T, EPI, 1, 2, 4>(p, 1, N, st);
   if (M <= 16) return stream<T, EPI, 1, 1>(p, 1, N, st);
   if constexpr (EPI == kSplit) {
     // narrow products: all columns in two blocks, so a row is read twice
@@ -1134,9 +1139,12 @@ hipError_t launch_grouped(const MmGrouped& g, int w_nt, hipStream_t st) {
   p.a.w_nt = w_nt;
   if (g.tile_rows > 16)
     return launch_block<T, EPI>(p, g.tile_rows / 16, g.tile_rows / 16, g.max_n, st);
-  // few k-steps per wave are not worth eight of them
-  return g.min_ks >= 16 ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
-                        : stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st);
+  if constexpr (!Kind<T>::BF16)  // (and more parts make fp32 sums more exact)
+    return g.min_ks >= 16 ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
+                          : stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st);
+  return g.min_ks >= 64   ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
+         : g.min_ks >= 32 ? stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st)
+                          : stream<T, EPI, 1, 1, 2>(p, g.max_tiles, g.max_n, st);
 }
 
 }  // namespace

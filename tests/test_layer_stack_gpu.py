@@ -66,6 +66,21 @@ def test_norm_and_head_alone(serve, dtype):
     T.check_rows(run_whole(serve(cfg, w, dtype), t), T.logits(cfg, w, t), dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("vocab", [32752, 32753, 32785])
+def test_wide_head(serve, dtype, vocab):
+    """The head's forms around 2,048 column tiles, whole pairs of them and not, and of rows."""
+    cfg = one_layer(width=136, vocab=vocab)
+    w = T.weights(cfg, 11)
+    t = tokens(cfg, 20, 12)
+    eng = serve(cfg, w, dtype)
+    want = T.logits(cfg, w, t)
+    for rows in ([19], list(range(3, 19)), list(range(20))):
+        s = eng.open_seq()
+        T.check_rows(eng.step([(s, t, rows)]), want[rows], dtype)
+        eng.close_seq(s)
+
+
 ATTENTION = {
     "plain": T.attn(rot=0),
     "rotary": T.attn(scaling=None),
