@@ -53,65 +53,48 @@ py::array_t<T, py::array::c_style | py::array::forcecast> arr(const py::dict& w,
   return a;
 }
 
-// int32 values of a list, a tuple or a buffer, as they lie where they can; false: of another
-// kind (the caller's general way takes it, or refuses it).
-class Int32s {
- public:
-  Int32s() = default;
-  Int32s(Int32s&& o) noexcept : view_(o.view_), held_(o.held_), data(o.data), at(o.at), n(o.n) { o.held_ = false; }
-  Int32s(const Int32s&) = delete;
-  ~Int32s() {
-    if (held_) PyBuffer_Release(&view_);
-  }
-  bool take(PyObject* o, std::vector<int32_t>& pool) {
-    if (PyList_CheckExact(o) || PyTuple_CheckExact(o)) {
-      const Py_ssize_t size = PySequence_Fast_GET_SIZE(o);
-      PyObject** items = PySequence_Fast_ITEMS(o);
-      at = pool.size();
-      for (Py_ssize_t i = 0; i < size; ++i) {
-        int over = 0;
-        if (!PyLong_CheckExact(items[i])) return false;
-        const long v = PyLong_AsLongAndOverflow(items[i], &over);
-        if (over || v != (int32_t)v) return false;
-        pool.push_back((int32_t)v);
-      }
-      n = (int)size;
-      return true;
+// int32 values of a list, a tuple or a buffer, appended to `pool` (a step reads them without the
+// interpreter's lock, when another thread may write the caller's array).  False: of another kind
+// (the caller's general way takes it, or refuses it).
+bool append_int32s(PyObject* o, std::vector<int32_t>& pool) {
+  if (PyList_CheckExact(o) || PyTuple_CheckExact(o)) {
+    const Py_ssize_t size = PySequence_Fast_GET_SIZE(o);
+    PyObject** items = PySequence_Fast_ITEMS(o);
+    for (Py_ssize_t i = 0; i < size; ++i) {
+      int over = 0;
+      if (!PyLong_CheckExact(items[i])) return false;
+      const long v = PyLong_AsLongAndOverflow(items[i], &over);
+      if (over || v != (int32_t)v) return false;
+      pool.push_back((int32_t)v);
     }
-    if (!PyObject_CheckBuffer(o)) return false;
-    if (PyObject_GetBuffer(o, &view_, PyBUF_FORMAT | PyBUF_C_CONTIGUOUS) != 0) {
-      PyErr_Clear();
-      return false;
-    }
-    held_ = true;
-    if (view_.ndim != 1 || view_.itemsize != 4 || !view_.format || std::string(view_.format) != "i" ||
-        view_.shape[0] > INT32_MAX)
-      return false;
-    data = static_cast<const int32_t*>(view_.buf);
-    n = (int)view_.shape[0];
     return true;
   }
-
- private:
-  Py_buffer view_{};
-  bool held_ = false;
-
- public:
-  const int32_t* data = nullptr;  // NULL: at `at` in the pool
-  size_t at = 0;
-  int n = 0;
-};
+  if (!PyObject_CheckBuffer(o)) return false;
+  Py_buffer view;
+  if (PyObject_GetBuffer(o, &view, PyBUF_FORMAT | PyBUF_C_CONTIGUOUS) != 0) {
+    PyErr_Clear();
+    return false;
+  }
+  const bool ok = view.ndim == 1 && view.itemsize == 4 && view.format && view.format[0] == 'i' &&
+                  view.format[1] == 0 && view.shape[0] <= INT32_MAX;
+  if (ok) {
+    const int32_t* v = static_cast<const int32_t*>(view.buf);
+    pool.insert(pool.end(), v, v + view.shape[0]);
+  }
+  PyBuffer_Release(&view);
+  return ok;
+}
 
 // llm_engine_step (the function at `step`, of the library the engine is from) over
 // [(seq, tokens, want)]: (status, logits), or None for entries that are not tuples of an int
-// and two Int32s.  64 entries of one token 9 us; built in Python 71.
+// and two lists of int32.  64 entries of one token 9 us; built in Python 71.
 py::object engine_step(uintptr_t step, uintptr_t engine, py::handle entries, int vocab) {
   PyObject* e = entries.ptr();
   if (!PyList_CheckExact(e) && !PyTuple_CheckExact(e)) return py::none();
   const Py_ssize_t count = PySequence_Fast_GET_SIZE(e);
-  std::vector<Int32s> lists(2 * (size_t)count);
   std::vector<llm_engine_entry> out((size_t)count + 1);
   std::vector<int32_t> pool;
+  std::vector<size_t> at(2 * (size_t)count + 1, 0);  // where a list begins
   pool.reserve(2 * (size_t)count);
   py::ssize_t rows = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
@@ -122,16 +105,17 @@ py::object engine_step(uintptr_t step, uintptr_t engine, py::handle entries, int
     const long seq = PyLong_AsLongAndOverflow(PyTuple_GET_ITEM(t, 0), &over);
     if (over || seq != (int)seq) return py::none();
     out[i].seq = (int)seq;
-    for (int k = 0; k < 2; ++k)
-      if (!lists[2 * i + k].take(PyTuple_GET_ITEM(t, 1 + k), pool)) return py::none();
-    rows += lists[2 * i + 1].n;
+    for (int k = 0; k < 2; ++k) {
+      if (!append_int32s(PyTuple_GET_ITEM(t, 1 + k), pool)) return py::none();
+      at[2 * i + k + 1] = pool.size();
+    }
+    rows += (py::ssize_t)(at[2 * i + 2] - at[2 * i + 1]);
   }
   for (Py_ssize_t i = 0; i < count; ++i) {
-    const Int32s &t = lists[2 * i], &w = lists[2 * i + 1];
-    out[i].tokens = t.data ? t.data : pool.data() + t.at;
-    out[i].n = t.n;
-    out[i].want = w.data ? w.data : pool.data() + w.at;
-    out[i].n_want = w.n;
+    out[i].tokens = pool.data() + at[2 * i];
+    out[i].n = (int)(at[2 * i + 1] - at[2 * i]);
+    out[i].want = pool.data() + at[2 * i + 1];
+    out[i].n_want = (int)(at[2 * i + 2] - at[2 * i + 1]);
   }
   py::array_t<float> logits({rows, (py::ssize_t)vocab});
   float* to = rows ? logits.mutable_data() : nullptr;
