@@ -573,7 +573,8 @@ __global__ __launch_bounds__(256) void gqa_merge_rows_kernel(GqaArgs a, int TR) 
 template <typename T>
 hipError_t merge(const GqaArgs& a, int tile_rows, hipStream_t st) {
   if (a.n_merges <= 0) return hipSuccess;
-  if (tile_rows > 16 && a.Dv <= 256) {
+  // (tiles of many splits: eight of them in flight a wave, below)
+  if (tile_rows > 16 && a.Dv <= 256 && a.n_items <= 8 * a.n_merges) {
     const auto go = [&](auto kernel, int rows) {
       hipLaunchKernelGGL(kernel, dim3(a.n_merges, a.G, std::max(tile_rows / rows / 2, 1)), dim3(256), 0, st,
                          a, tile_rows);
