@@ -775,6 +775,59 @@ def test_forced_hidden_2048_tile_forms(gpu, oracle, rows):
     assert n_flips < 1e-3 * n_vals, (n_flips, n_vals)
 
 
+@pytest.mark.parametrize("H,D,rows", [(4, 64, 1), (4, 64, 8), (4, 64, 9), (8, 64, 8), (8, 64, 9),
+                                      (12, 64, 1), (12, 64, 16), (12, 64, 17), (16, 128, 3)])
+def test_forced_fc2_forms(gpu, oracle, H, D, rows):
+    """fc2 that quantises its own input (hidden up to 512, 8 rows), in two slices behind the
+    quantising launch (up to 16 rows, every width) and in one."""
+    from oracle.oracle import OracleDecoder
+    w = _int8_model(oracle, L=2, H=H, D=D, V=512, S=24, seed=43)
+    dec = _make_gpu_decoder(w, max_batch=rows)
+    taps = _Taps(dec, w, rows)
+    rng = np.random.default_rng(rows)
+    prompts = [list(rng.integers(0, 512, 3)) for _ in range(rows)]
+    _, _, n_vals, n_flips = _forced_lockstep(dec, OracleDecoder(oracle, w, rows), taps, prompts,
+                                             gen=3, V=512)
+    assert n_flips < 1e-3 * n_vals, (n_flips, n_vals)
+
+
+@pytest.mark.parametrize("H,D", [(4, 64), (16, 128)])
+@pytest.mark.parametrize("n", [127, 128, 129, 300])
+def test_packed_rows_of_prompts(gpu, H, D, n):
+    """Every row of a packed matrix of one to a few groups of 128 rows, its own values and scale."""
+    import torch
+
+    # the prompt's last token sees every row: one that went astray shows in its logits, against
+    # the same tokens one by one
+    import llm_decoder
+    hid, V, rng = H * D, 600, np.random.default_rng(n)
+    L, w = 2, {}
+    w["emb"] = rng.standard_normal((V, hid)).astype(np.float16).view(np.uint16)
+    for k in ("ln1_g", "ln2_g"):
+        w[k] = (1 + 0.1 * rng.standard_normal((L, hid))).astype(np.float32)
+    for k, c in (("ln1_b", hid), ("ln2_b", hid), ("b1", 4 * hid), ("b2", hid)):
+        w[k] = (0.1 * rng.standard_normal((L, c))).astype(np.float32)
+    for k, K, N in (("wqkv", hid, 3 * hid), ("wo", hid, hid), ("w1", hid, 4 * hid), ("w2", 4 * hid, hid)):
+        w[k] = (K ** -0.5 * rng.standard_normal((L, K, N))).astype(np.float16).view(np.uint16)
+    out = []
+    for whole in (True, False):
+        dec = llm_decoder.CUDADecoder(L, H, D, hid, V, n + 8, max_batch=1, attn_scale=D ** -0.5)
+        dec.set_weights(w)
+        dec.begin_synthetic(1, 0, 0, False)
+        ids = np.random.default_rng(n).integers(0, V, n + 1).tolist()
+        logits = torch.empty((1, V), device="cuda")
+        if whole:
+            dec.prefill(0, ids[:n])
+        else:
+            for t in ids[:n]:
+                dec.step([t])
+        dec.step([ids[n]], logits_ptr=logits.data_ptr())
+        torch.cuda.synchronize()
+        out.append(logits.cpu().numpy())
+    # fp16 products either way: two roundings of their inputs in another order
+    assert rel_err(out[0], out[1]) < 5e-3, rel_err(out[0], out[1])
+
+
 @pytest.mark.parametrize("max_batch,max_seq", [(1, 40), (4, 2048)])  # a thread an element, and eight
 def test_synthetic_context_bits(gpu, oracle, max_batch, max_seq):
     """The random context of a seed: splitmix64, the sum of its four 16-bit parts, one rounding
