@@ -248,7 +248,7 @@ __global__ __launch_bounds__(1024) void pa_merge_row_kernel(PaMergeRowArgs a) {
 // neighbouring values of QPT quads, of every split one 16-byte load, and keeps them to the
 // quantisation; it works out its head's weights itself, two to four exponentials in most
 // prompts.  Bound by the partials' bytes (2048 rows of 16 x 128, three splits at most, int8
-// out: 22 us by a wave a head and values through LDS, all splits' places read, now 11).
+// out: 22 us by a wave a head and values through LDS, all splits' places read, now 10).
 template <int QPT>
 __global__ __launch_bounds__(256) void pa_merge_prompt_kernel(PaMergeRowArgs a) {
   __shared__ float sh[4];

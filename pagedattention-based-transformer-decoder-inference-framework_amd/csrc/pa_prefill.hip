@@ -362,8 +362,9 @@ hipError_t launch_prefill(const PaPrefillArgs& a, hipStream_t st) {
 // The key range is cut into splits of `per` stages, the length for which the rounds of
 // workgroups (4 per CU) times their length is least, a split more counted as half a stage
 // for its merge; no more than split_bound of them a query.  32 queries a wave in place of
-// 16 (16 heads of 128, with the merge): 2048 queries 72 -> 70 us, but those after 2048 more
-// 120 -> 139, 1024 34 -> 36, 117 11 -> 14; heads of 64 2048 48 -> 60.
+// 16 (16 heads of 128, with the merge; two waves a SIMD, of 32 queries there can be no more):
+// 2048 queries 72 -> 70 us, but those after 2048 more 120 -> 139, 1024 34 -> 36, 117 11 -> 14;
+// heads of 64 2048 48 -> 60.
 constexpr int kRound = 1024;
 struct PrefillPlan {
   int nsplit, pps;
