@@ -69,19 +69,10 @@ struct KernelArgs {
   const float* bias;
 };
 
-// fp32 results take expf and the division; bf16 ones the hardware's 2^x and 1 / x, off by some
-// 1e-7 and at most 1e-6 where the exponent is large (the rounding to bf16: 4e-3): a vector
-// instruction takes a SIMD 4 cycles, a pair was 60 of them and is 25 (2048 x 12288 x 2048 of
-// blocks 95 -> 86 us, the results past L2 in the same step).  e^-alpha g past 2^120 leaves
-// nothing of any g.
-template <typename T>
 __device__ __forceinline__ float glu(float gate, float up, const GluParams& p) {
   const float g = fminf(gate, p.limit);
   const float u = fminf(fmaxf(up, -p.limit), p.limit);
-  if constexpr (!Kind<T>::BF16) return g / (1.f + expf(-p.alpha * g)) * (u + p.up_bias);
-  const float a = -p.alpha * g, t = fminf(a * kLog2e, 120.f);
-  const float d = 1.f + __builtin_amdgcn_exp2f(t), r = __builtin_amdgcn_rcpf(d);
-  return g * r * (u + p.up_bias);
+  return g / (1.f + expf(-p.alpha * g)) * (u + p.up_bias);
 }
 
 // log(1 + e^v) = max(v, 0) + log1p(e), e = e^-|v|; log1p(e) = 2 atanh(s) with
@@ -399,7 +390,7 @@ struct Target {
       if (p0) *static_cast<float*>(p0) = v0;
       if (p1) *static_cast<float*>(p1) = v1;
     } else if constexpr (EPI == kGroupIn || EPI == kGlu) {
-      if (p0) *static_cast<T*>(p0) = (T)glu<T>(v0, v1, b.glu);
+      if (p0) *static_cast<T*>(p0) = (T)glu(v0, v1, b.glu);
     } else if constexpr (EPI == kSplit) {
       if (!p0) return;
       if (n < p.split.n_t) put_pair(static_cast<T*>(p0), v0, v1);
@@ -557,7 +548,7 @@ struct Eight {
       typedef T half_t __attribute__((ext_vector_type(4)));
       half_t o;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) o[k] = (T)glu<T>(v[2 * k], v[2 * k + 1], b.glu);
+      for (int k = 0; k < 4; ++k) o[k] = (T)glu(v[2 * k], v[2 * k + 1], b.glu);
       *static_cast<half_t*>(p0) = o;
     } else if constexpr (EPI == kHeads) {
       if (p0) put_eight(static_cast<T*>(p0), v);
@@ -798,8 +789,8 @@ __device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b
 #pragma unroll
       for (int k = 0; k < 8; k += 2) {
         const f32x4 x = *reinterpret_cast<const f32x4*>(sums + i * STEP * STRIDE + 2 * k);
-        v[k] = glu<T>(x[0], x[1], b.glu);
-        v[k + 1] = glu<T>(x[2], x[3], b.glu);
+        v[k] = glu(x[0], x[1], b.glu);
+        v[k + 1] = glu(x[2], x[3], b.glu);
       }
       if (vec) {
         put_eight(to, v);
