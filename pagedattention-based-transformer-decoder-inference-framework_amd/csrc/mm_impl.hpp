@@ -839,8 +839,10 @@ __device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b
 }
 
 // Decode rows (and short grouped tiles): a block owns 16 MT rows x 16 NT columns
-// and its WK waves split K, adding through LDS in a fixed order.
-template <typename T, int EPI, int MT, int NT, int WK>
+// and its WK waves split K, adding through LDS in a fixed order.  K is summed in PARTS parts,
+// PARTS / WK of them by a wave one after the other: a wave that streams more of K sums it no
+// further in one piece, and the bits do not depend on how many waves there are.
+template <typename T, int EPI, int MT, int NT, int WK, int PARTS>
 __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kernel(KernelArgs p) {
   if constexpr (EPI == kGroupIn || EPI == kGroupOut)
     if ((int)blockIdx.y >= *p.g.n_tiles) return;
@@ -870,6 +872,28 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
   // the same A lines at once.
   const int wr = (w + (int)blockIdx.x) % WK;
   const int ks0 = wr * b.KS / WK, ks1 = (wr + 1) * b.KS / WK;
+  constexpr int OWN = PARTS / WK;
+  static_assert(PARTS % WK == 0, "whole parts a wave");
+  __shared__ float red[PARTS][MT * NT][4][64];
+  int part = wr * OWN;  // the one being summed
+  auto put_part = [&] {
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[part][i * NT + j][r][lane] = acc[i][j][r];
+  };
+  auto end_parts = [&](int k) {  // (a wave's last part ends with the wave)
+    while (part < wr * OWN + OWN - 1 && (part + 1) * b.KS / PARTS <= k) {
+      put_part();
+      ++part;
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
   struct Batch {
     u32x4 a[U][MT], b[U][NT];
   };
@@ -895,17 +919,18 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
       }
     }
   };
-  auto mul = [&](const Batch& x) {
+  auto mul = [&](const Batch& x, int ks) {
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int u = 0; u < U; ++u) {
+      if constexpr (OWN > 1) end_parts(ks + u);
 #pragma unroll
       for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = Kind<T>::mma(x.a[u][i], x.b[u][j], acc[i][j]);
+    }
   };
   // thread t finishes column pairs t, t + THREADS, ...: 8 pairs a row, 128 a tile
   constexpr int PAIRS = MT * NT * 128, THREADS = 64 * WK, EPT = (PAIRS + THREADS - 1) / THREADS;
-  __shared__ float red[WK][MT * NT][4][64];
   Target<T, EPI> target[EPT];
   Batch x, y;
   if (ks0 < ks1) load(x, ks0);
@@ -919,22 +944,18 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
   if (ks0 < ks1) {
     for (int ks = ks0;;) {
       if (ks + U < ks1) load(y, ks + U);
-      mul(x);
+      mul(x, ks);
       ks += U;
       if (ks >= ks1) break;
       if (ks + U < ks1) load(x, ks + U);
-      mul(y);
+      mul(y, ks);
       ks += U;
       if (ks >= ks1) break;
     }
   }
 
-#pragma unroll
-  for (int i = 0; i < MT; ++i)
-#pragma unroll
-    for (int j = 0; j < NT; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) red[wr][i * NT + j][r][lane] = acc[i][j][r];
+  if constexpr (OWN > 1) end_parts(b.KS);
+  put_part();
   __syncthreads();
 #pragma unroll
   for (int e = 0; e < EPT; ++e) {
@@ -943,7 +964,7 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
     const int t = pr >> 7, row = (pr >> 3) & 15, col = (pr & 7) * 2;
     float2 s = {0.f, 0.f};
 #pragma unroll
-    for (int k = 0; k < WK; ++k) {
+    for (int k = 0; k < PARTS; ++k) {
       const float2 v = *reinterpret_cast<const float2*>(&red[k][t][row & 3][(row >> 2) * 16 + col]);
       s.x += v.x;
       s.y += v.y;
@@ -1014,10 +1035,10 @@ int heads_of(const KernelArgs& p) {
   return EPI == kHeads ? p.heads.heads : 1;
 }
 
-template <typename T, int EPI, int MT, int NT, int WK = 8>
+template <typename T, int EPI, int MT, int NT, int WK = 8, int PARTS = WK>
 hipError_t stream(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
   const dim3 grid(((N + 15) / 16 + NT - 1) / NT, row_blocks, heads_of<EPI>(p));
-  hipLaunchKernelGGL((mm_stream_kernel<T, EPI, MT, NT, WK>), grid, dim3(64 * WK), 0, st, p);
+  hipLaunchKernelGGL((mm_stream_kernel<T, EPI, MT, NT, WK, PARTS>), grid, dim3(64 * WK), 0, st, p);
   return hipGetLastError();
 }
 
@@ -1130,12 +1151,20 @@ hipError_t launch_grouped(const MmGrouped& g, int w_nt, hipStream_t st) {
   p.a.w_nt = w_nt;
   if (g.tile_rows > 16)
     return launch_block<T, EPI>(p, g.tile_rows / 16, g.tile_rows / 16, g.max_n, st);
-  if constexpr (!Kind<T>::BF16)  // (and more parts make fp32 sums more exact)
-    return g.min_ks >= 16 ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
-                          : stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st);
-  return g.min_ks >= 64   ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
-         : g.min_ks >= 32 ? stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st)
-                          : stream<T, EPI, 1, 1, 2>(p, g.max_tiles, g.max_n, st);
+  // bf16: at least eight k-steps a wave (an expert's output product of 32 k-steps over 37 tiles
+  // 26 us by eight waves, 20.5 by four; of 16 over 52 15.2, 10.5 by two), the sums in as many
+  // parts as by eight.  Two waves a workgroup are too few in flight while a CU has but two or
+  // three workgroups: 16 k-steps 4.0 us by eight waves, 4.7 by two over 64 x 5 workgroups, 4.1
+  // and 5.1 over 64 x 9, 6.0 and 5.3 over 64 x 13.
+  if constexpr (Kind<T>::BF16) {
+    const bool few = g.max_tiles * ((g.max_n + 15) / 16) <= 640;
+    if (g.min_ks >= 32 && g.min_ks < 64) return stream<T, EPI, 1, 1, 4, 8>(p, g.max_tiles, g.max_n, st);
+    if (g.min_ks < 32 && !few)
+      return g.min_ks >= 16 ? stream<T, EPI, 1, 1, 2, 8>(p, g.max_tiles, g.max_n, st)
+                            : stream<T, EPI, 1, 1, 2, 4>(p, g.max_tiles, g.max_n, st);
+  }
+  return g.min_ks >= 16 ? stream<T, EPI, 1, 1>(p, g.max_tiles, g.max_n, st)
+                        : stream<T, EPI, 1, 1, 4>(p, g.max_tiles, g.max_n, st);
 }
 
 }  // namespace

@@ -1,4 +1,5 @@
-"""The layer-stack models' products (mm_impl.hpp): the activation at gates of any size."""
+"""Products of few rows in bf16 (mm_impl.hpp): the activation at gates of any size, and sums
+over K that do not depend on what else the launch works on."""
 import numpy as np
 import pytest
 
@@ -36,3 +37,22 @@ def test_gates_far_from_zero(serve, kind, rows, dtype):  # noqa: F811
     with np.errstate(over="ignore"):
         want = T.logits(cfg, w, t)
     T.check_rows(run_whole(serve(cfg, w, dtype), t), want, dtype)
+
+
+@pytest.mark.parametrize("width,experts,rows", [(96, 2, 1), (96, 2, 5), (1088, 8, 1), (1088, 8, 16)])
+def test_sums_of_experts_whatever_the_others_width(serve, width, experts, rows):  # noqa: F811
+    """A shared expert of 64 k-steps beside routed ones of 16, 32 and 64, whose output is
+    nothing: the same bits, by eight, four and two waves a workgroup (these past 640)."""
+    first = base = None
+    for ff in (2048, 1024, 512):
+        cfg = T.config([(T.attn(), T.moe(experts=experts, ff=ff, shared=2048))], width=width)
+        w = T.weights(cfg, 5)
+        base = base or w
+        w = {k: w[k] if ".mlp.e" in k else base[k] for k in w}
+        for e in range(experts):
+            w[f"l0.mlp.e{e}.down"] = 0 * w[f"l0.mlp.e{e}.down"]
+        eng = serve(cfg, w, "bfloat16", name=f"m{ff}")
+        s = eng.open_seq()
+        tap = eng.step_taps([(s, tokens(cfg, rows, 6), [0])])[1]
+        first = tap if first is None else first
+        np.testing.assert_array_equal(tap.view(np.uint32), first.view(np.uint32))
