@@ -1102,11 +1102,16 @@ template <typename T, int EPI>
 hipError_t launch(const KernelArgs& p, hipStream_t st) {
   const int M = p.a.M, N = p.a.N;
   const int ntiles = (N + 15) / 16;
-  // A model's head: blocks of two tiles, which read A half as often, by four waves of twice the
-  // k-steps (32768 x 2048, 16 rows 31.2 us by the form below, 27.2 by eight waves, 25.8 so; one
-  // row 31.6, 30.2, 29.9)
+  // A model's head: blocks of two tiles read A half as often, which counts once A's rows are
+  // many beside a block's weights; four waves of two parts each stream more of K (us by one
+  // tile and eight waves / two and four).  16 rows, K 1024: 1000 tiles 10.0 / 9.0, 2048 18.6 /
+  // 15.0, 4000 33.9 / 26.4; K 2048: 16.9 / 14.7, 31.7 / 26.3, 59.2 / 49.0; K 4096: 31.2 / 30.7,
+  // 60.1 / 58.0, 114 / 103.  8 rows: 2048 tiles 15.3 / 14.1, 26.1 / 25.5, 47.5 / 56.0; 12 rows
+  // of K 4096 53.5 / 57.8.  One row: 13.4 / 13.8, 24.3 / 24.5, 44.5 / 53.7.  512 tiles of 16
+  // rows: 6.0 / 6.2, 9.4 / 8.9, 16.7 / 17.0.
   if constexpr (EPI == kStore && Kind<T>::BF16)
-    if (M <= 16 && ntiles >= 2048) return stream<T, EPI, 1, 2, 4>(p, 1, N, st);
+    if (M <= 16 && M > (p.KS > 64 ? 14 : 8) && p.KS <= 128 && ntiles >= 1000)
+      return stream<T, EPI, 1, 2, 4, 8>(p, 1, N, st);
   if (M <= 16) return stream<T, EPI, 1, 1>(p, 1, N, st);
   if constexpr (EPI == kSplit) {
     // narrow products: all columns in two blocks, so a row is read twice

@@ -56,3 +56,22 @@ def test_sums_of_experts_whatever_the_others_width(serve, width, experts, rows):
         tap = eng.step_taps([(s, tokens(cfg, rows, 6), [0])])[1]
         first = tap if first is None else first
         np.testing.assert_array_equal(tap.view(np.uint32), first.view(np.uint32))
+
+
+@pytest.mark.parametrize("width", [72, 512])
+def test_sums_of_the_head_whatever_its_width(serve, width):  # noqa: F811
+    """Logits of the first tokens of heads of 999 column tiles and of more, one row to 16: the
+    same bits."""
+    cfg = T.config([(T.attn(), None)], width=width, vocab=32768)
+    w = T.weights(cfg, 7)
+    t = tokens({"vocab": 15984}, 16, 8)
+    first = None
+    for vocab in (15984, 16001, 32752, 32768):
+        v = dict(w, embed=w["embed"][:vocab], head=w["head"][:vocab])
+        eng = serve(dict(cfg, vocab=vocab), v, "bfloat16", name=f"m{vocab}")
+        for rows in (range(16), [15], range(8), range(9)):
+            s = eng.open_seq()
+            out = eng.step([(s, t, list(rows))])[:, :15984]
+            eng.close_seq(s)
+            first = out if first is None else first
+            np.testing.assert_array_equal(out.view(np.uint32), first[list(rows)].view(np.uint32))
