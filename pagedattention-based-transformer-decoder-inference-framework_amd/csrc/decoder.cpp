@@ -524,15 +524,16 @@ bool llm_decoder::wgm_quant_ok(const Rows& R) {
 // starts: fc1 is the last reader of the o_proj output in x, and the launch that
 // quantises fc1's rows sets it to zero.  Standalone (scripts/tune_gemm_sk.py,
 // profiles/r05/gemm_small_m.txt): fc2 at M = 8 6.86 -> 5.67 us, M = 16 7.53 ->
-// 5.95 us.
-// 4 layers of hidden 768: 126 -> 124 us a step of one row, 155.5 -> 153 of 16.
+// 5.95 us.  Not at widths whose LayerNorms are prologues (ln_fusable): one exact
+// sum there, the same bits in a step of any number of rows (in two slices 4 layers
+// of hidden 768 were 126 -> 124 us a step of one row, 155.5 -> 153 of 16).
 // Also at 33..64 rows when inter >= 16384 (C5's fc2, K 16384): every
 // workgroup of the one-slice form reads all of A, 1 MB, the k slices half of
 // it (gemm_impl.hpp narrow_decode_tile).
 bool llm_decoder::fc2_split(const Rows& R) const {
   return wdtype == LLM_I8 && R.prefill_row < 0 &&
          (R.n <= 16 || (R.n > 32 && R.n <= 64 && inter >= 16384)) &&
-         inter / 64 >= 16 && !fc2_quant_prologue(R);
+         !ln_fusable(wdtype, R.n, hid) && inter / 64 >= 16 && !fc2_quant_prologue(R);
 }
 
 // INT8 decode rows whose fc2 quantises its own input: a row for each of the prologue's waves,

@@ -779,7 +779,7 @@ def test_forced_hidden_2048_tile_forms(gpu, oracle, rows):
                                       (12, 64, 1), (12, 64, 16), (12, 64, 17), (16, 128, 3)])
 def test_forced_fc2_forms(gpu, oracle, H, D, rows):
     """fc2 that quantises its own input (hidden up to 512, 8 rows), in two slices behind the
-    quantising launch (up to 16 rows, every width) and in one."""
+    quantising launch (up to 16 rows of hidden past 1,024) and in one."""
     from oracle.oracle import OracleDecoder
     w = _int8_model(oracle, L=2, H=H, D=D, V=512, S=24, seed=43)
     dec = _make_gpu_decoder(w, max_batch=rows)
@@ -789,6 +789,25 @@ def test_forced_fc2_forms(gpu, oracle, H, D, rows):
     _, _, n_vals, n_flips = _forced_lockstep(dec, OracleDecoder(oracle, w, rows), taps, prompts,
                                              gen=3, V=512)
     assert n_flips < 1e-3 * n_vals, (n_flips, n_vals)
+
+
+@pytest.mark.parametrize("H,D,batches", [(4, 64, (33, 17, 16, 9, 8, 1)), (8, 64, (32, 17, 16, 9, 8, 1))])
+def test_fc2_sums_whatever_the_batch(gpu, oracle, H, D, batches):
+    """One exact sum of fc2 over all of K where the LayerNorms are prologues: a token's rows
+    after every layer are the same bits and scales in a step of any number of rows."""
+    w = _int8_model(oracle, L=4, H=H, D=D, V=512, S=24, seed=47)
+    first = {}
+    for rows in batches:
+        dec = _make_gpu_decoder(w, max_batch=rows)
+        taps = _Taps(dec, w, rows)
+        dec.begin_synthetic(rows, 0, 0, False)
+        dec.step([(7 + 31 * r) % 512 for r in range(rows)])
+        _torch().cuda.synchronize()
+        q, s = taps.read(rows)
+        for r in range(rows):
+            got = first.setdefault(r, (q[:, :, r], s[:, :, r].view(np.uint32)))
+            np.testing.assert_array_equal(s[:, :, r].view(np.uint32), got[1], err_msg=f"row {r} of {rows}")
+            np.testing.assert_array_equal(q[:, :, r], got[0], err_msg=f"row {r} of {rows}")
 
 
 @pytest.mark.parametrize("H,D", [(4, 64), (16, 128)])
