@@ -55,10 +55,14 @@ class Engine:
         self.lib = lib or llm_capi.load()
         self._h = c_void_p()
         self._native_step, self._step_at = None, 0
-        if lib is None:  # (with the engine's library alone, steps are built here)
-            from llm_decoder import engine_step
-            self._native_step = engine_step
-            self._step_at = ctypes.cast(self.lib.llm_engine_step, c_void_p).value
+        # (without the module, or with the engine's library alone, steps are built here)
+        if self.lib is llm_capi._lib:
+            try:
+                from llm_decoder import engine_step
+                self._native_step = engine_step
+                self._step_at = ctypes.cast(self.lib.llm_engine_step, c_void_p).value
+            except ImportError:
+                pass
         cfg = EngineConfig(DTYPES[dtype], max_seqs, max_tokens, max_seq_len, max_step_tokens)
         self._check(self.lib.llm_engine_create(os.fsencode(str(model_dir)), ctypes.byref(cfg),
                                                ctypes.byref(self._h)))

@@ -109,3 +109,27 @@ def test_refused_entries(eng, bad):
     eng.close_seq(s)
     with pytest.raises(Exception, match="not open"):
         eng.step([(s, [5], [0])])
+
+
+def test_without_the_extension_module(eng, tmp_path, monkeypatch):
+    """The C library alone, or a module built for another Python: steps go the general way."""
+    import sys
+
+    import engine
+    import llm_capi
+    cfg = T.config([(T.attn(), None)], vocab=5003)
+    T.save(tmp_path / "m", cfg, T.weights(cfg, 3))
+
+    def step(e):
+        seq = e.open_seq()
+        out = e.step([(seq, np.array([5, 6, 7], np.int32), [0, 2])])
+        e.close_seq(seq)
+        return out
+    want = step(eng)
+    with engine.Engine(tmp_path / "m", dtype="float32", max_tokens=256, lib=llm_capi.load()) as e:
+        assert e._native_step  # the default library, named or not
+        np.testing.assert_array_equal(step(e), want)
+    monkeypatch.setitem(sys.modules, "llm_decoder", None)
+    with engine.Engine(tmp_path / "m", dtype="float32", max_tokens=256) as e:
+        assert not e._native_step
+        np.testing.assert_array_equal(step(e), want)
