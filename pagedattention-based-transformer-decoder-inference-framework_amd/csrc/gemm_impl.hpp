@@ -861,7 +861,12 @@ inline bool narrow_decode_tile(const GemmArgs& a, int kstep, TileChoice& t) {
 }
 
 // The block form whose rounds of workgroups take least; us of a round at K = 2048 with one,
-// two and three blocks a CU (mm_impl.hpp's forms, int8's by times of their own).
+// two and three blocks a CU (mm_impl.hpp's forms, int8's by times of their own; fp16's are 1.4
+// times bf16's in every form, for sums in eight parts).  Timed over 65 to 2048 rows, 1024 to
+// 12288 columns and K 256 to 8192, the form so chosen is on average 0 to 2 % off the best from K
+// 1024 on, 2 to 10 % below.  fp16 blocks of 64 x 64 are faster than 64 x 128 at small K (1000 x
+// 1024 x 256 8.3 and 11.4 us, 130 x 4096 x 512 8.0 and 9.3, x 2048 15.7 and 15.9; a prompt of 250
+// rows, qkv of K 1024 11.4 and 12.2) and 5 % slower from K 4096 on.
 template <GemmKind KIND, bool A_PACKED, bool ROWS>
 hipError_t launch_gemm_block(const GemmArgs& a, hipStream_t st) {
   void (*best)(GemmArgs) = nullptr;
@@ -884,6 +889,8 @@ hipError_t launch_gemm_block(const GemmArgs& a, hipStream_t st) {
     consider(8, 8, 8, 1, {13.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 8, 4, 2, 3>);
     consider(8, 16, 8, 1, {21.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 16, 2, 4, 3>);
   } else {
+    if (a.K <= 2048)
+      consider(4, 4, 4, 3, {11.4f, 13.7f, 18.9f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 4, 2, 2, 3>);
     consider(4, 8, 8, 1, {12.1f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 4>);
     consider(4, 8, 8, 2, {12.6f, 20.1f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 3>);
     consider(8, 8, 8, 1, {17.6f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 8, 4, 2, 3>);
@@ -902,8 +909,7 @@ hipError_t launch_gemm(const GemmArgs& a_in, hipStream_t st, int nt_override = 0
   if (a.M > 64 && (long long)((a.M + 63) / 64) * ((a.N + 63) / 64) > 128 && !a.ln_x && !a.partial &&
       !a.ksplit2 && !a.stamps && reinterpret_cast<uintptr_t>(a.A) % 16 == 0 &&
       (!a.kv.k_pool || a.kv.D % 8 == 0) &&
-      nt_override + waves_override + mrows_override + ks_override == 0)
-  {
+      nt_override + waves_override + mrows_override + ks_override == 0) {
     const bool rows = !a.kv.k_pool && !a.c16;
     if (a.a_packed)
       return rows ? launch_gemm_block<KIND, true, true>(a, st) : launch_gemm_block<KIND, true, false>(a, st);
