@@ -1062,40 +1062,36 @@ hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
 // half the chip idle: 26.4); 700 x 2048: 64 x 128, 12.0 us (128 x 128: 17.3).  fp32 blocks are
 // bound by the matrix cores and take the time of their area, the small ones, of which a CU
 // holds several, the time between two rounds: 2048 x 2048: two rounds of 64 x 128, 140 us
-// (128 x 128: 158); 700 x 6144: five of 64 x 64, 185 us (64 x 128: 207); K only scales all.
-template <typename T, int EPI>
-struct BlockForm {
-  int mb, nb, per;
-  float bf16[3], fp32;
-  hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
-};
+// (128 x 128: 158); 700 x 6144: five of 64 x 64, 185 us (64 x 128: 207).  Of other K the order
+// is nearly the same: over 65 to 2048 rows and 1024 to 12288 columns of bf16 the form so chosen is
+// on average 0.1 to 0.3 % off the best from K 1024 to 8192, 0.8 % at 512, 2.3 % at 256.
 template <typename T, int EPI>
 hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipStream_t st) {
-  static constexpr BlockForm<T, EPI> forms[] = {
-      {4, 2, 3, {10.8f, 12.1f, 15.6f}, 21.5f, blocks<T, EPI, 4, 2, 4, 1, 4>},
-      {4, 4, 3, {13.3f, 15.4f, 20.4f}, 37.f, blocks<T, EPI, 4, 4, 2, 2, 3>},
-      {4, 8, 1, {12.1f}, 70.f, blocks<T, EPI, 4, 8, 2, 4, 4>},
-      {4, 8, 2, {12.6f, 20.1f}, 1e9f, blocks<T, EPI, 4, 8, 2, 4, 3>},
-      {4, 16, 1, {18.7f}, 160.f, blocks<T, EPI, 4, 16, 2, 4, 3>},
-      {8, 8, 1, {17.6f}, 156.f, blocks<T, EPI, 8, 8, 4, 2, 3>},
-      {8, 16, 1, {28.f}, 293.f, blocks<T, EPI, 8, 16, 2, 4, 3>}};
-  const BlockForm<T, EPI>* best = nullptr;
+  hipError_t (*best)(const KernelArgs&, int, int, hipStream_t) = nullptr;
   int best_y = 0;
   float least = 0.f;
-  for (const BlockForm<T, EPI>& f : forms) {
-    if (f.mb < min_mb || f.mb > max_mb) continue;
-    const int y = (p.a.M + 16 * f.mb - 1) / (16 * f.mb);
-    int groups = group_across(N, f.nb) * y * heads_of<EPI>(p);
+  const auto consider = [&](int mb, int nb, int per, const float (&bf16)[3], float fp32,
+                            hipError_t (*go)(const KernelArgs&, int, int, hipStream_t)) {
+    if (mb < min_mb || mb > max_mb) return;
+    const int y = (p.a.M + 16 * mb - 1) / (16 * mb);
+    int groups = group_across(N, nb) * y * heads_of<EPI>(p);
     if constexpr (EPI == kGroupIn || EPI == kGroupOut)
-      groups = (p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, f.nb) +
-               p.g.shared_tiles * group_across(p.g.shared_n, f.nb);
-    const float cost = Kind<T>::BF16 ? rounds_us(groups, f.per, f.bf16) : (float)((groups + 255) / 256) * f.fp32;
-    if (best && cost >= least) continue;
-    best = &f;
+      groups = (p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, nb) +
+               p.g.shared_tiles * group_across(p.g.shared_n, nb);
+    const float cost = Kind<T>::BF16 ? rounds_us(groups, per, bf16) : (float)((groups + 255) / 256) * fp32;
+    if (best && cost >= least) return;
+    best = go;
     best_y = y;
     least = cost;
-  }
-  return best->go(p, best_y, N, st);
+  };
+  consider(4, 2, 3, {10.8f, 12.1f, 15.6f}, 21.5f, blocks<T, EPI, 4, 2, 4, 1, 4>);
+  consider(4, 4, 3, {13.3f, 15.4f, 20.4f}, 37.f, blocks<T, EPI, 4, 4, 2, 2, 3>);
+  consider(4, 8, 1, {12.1f}, 70.f, blocks<T, EPI, 4, 8, 2, 4, 4>);
+  if constexpr (Kind<T>::BF16) consider(4, 8, 2, {12.6f, 20.1f}, 0.f, blocks<T, EPI, 4, 8, 2, 4, 3>);
+  consider(4, 16, 1, {18.7f}, 160.f, blocks<T, EPI, 4, 16, 2, 4, 3>);
+  consider(8, 8, 1, {17.6f}, 156.f, blocks<T, EPI, 8, 8, 4, 2, 3>);
+  consider(8, 16, 1, {28.f}, 293.f, blocks<T, EPI, 8, 16, 2, 4, 3>);
+  return best(p, best_y, N, st);
 }
 
 template <typename T, int EPI>
