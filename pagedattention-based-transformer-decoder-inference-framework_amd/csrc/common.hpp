@@ -229,6 +229,12 @@ __device__ __forceinline__ void barrier_only() {
 // layout of v_mfma_i32_16x16x64_i8 / v_mfma_f32_16x16x32_f16, so the GEMM
 // reads each fragment with one coalesced buffer_load_dwordx4.
 // KS = k-steps per row (K/64 for int8, K/32 for fp16).  Offsets in elements.
+__host__ __device__ __forceinline__ size_t a_frag_off_i8(int m, int k, int KS) {
+  return ((size_t)((m >> 4) * KS + (k >> 6)) * 64 + (m & 15) + 16 * ((k & 63) >> 4)) * 16 + (k & 15);
+}
+__host__ __device__ __forceinline__ size_t a_frag_off_f16(int m, int k, int KS) {
+  return ((size_t)((m >> 4) * KS + (k >> 5)) * 64 + (m & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
 // The row of a workgroup that writes one of `rows` packed rows: workgroups go round the 8
 // XCDs, and a packed tile's 16 rows lie 16 bytes each in its lines, so that rows in their own
 // order leave parts of lines in every XCD's L2 (int8 2048 x 8192: 33 MB written for 17).  128
@@ -236,12 +242,6 @@ __device__ __forceinline__ void barrier_only() {
 __device__ __forceinline__ int packed_row(int block, int rows) {
   const int first = block & ~127;
   return first + 128 <= rows ? first + 16 * (block & 7) + (block >> 3 & 15) : block;
-}
-__host__ __device__ __forceinline__ size_t a_frag_off_i8(int m, int k, int KS) {
-  return ((size_t)((m >> 4) * KS + (k >> 6)) * 64 + (m & 15) + 16 * ((k & 63) >> 4)) * 16 + (k & 15);
-}
-__host__ __device__ __forceinline__ size_t a_frag_off_f16(int m, int k, int KS) {
-  return ((size_t)((m >> 4) * KS + (k >> 5)) * 64 + (m & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
 }
 
 }  // namespace llm

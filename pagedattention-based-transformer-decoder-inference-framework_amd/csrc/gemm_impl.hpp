@@ -158,8 +158,8 @@ struct GemmTraits<GemmKind::F16> {
 // zero), bit 1 = no epilogue (wave 0 stores one word per workgroup).
 // LayerNorm (+ int8 quantisation) of this workgroup's ROWS rows of ln_x into
 // the LDS image of A (ln_row_stride) and, for I8, the row scales into sa_lds:
-// ln_wave.hpp, bit-identical to the LayerNorm launch.  One wave per row (rows
-// w, w + WAVES, ...), two rows' loads in flight; gamma / beta loaded once.
+// ln_wave.hpp: the LayerNorm launch's steps, its two sums in another order.  One wave per row
+// (rows w, w + WAVES, ...), two rows' loads in flight; gamma / beta loaded once.
 // CPL: float4 chunks per lane that cover K, so that a row of 256 is not worked on as
 // one of 2048; a wave without a row does nothing, and rows past M stay as they are (each
 // row of A makes its own row of C).  1 x 768 x 256 with its KV append 7.5 us, now 4.3; 1 x 256 x

@@ -259,14 +259,11 @@ __global__ __launch_bounds__(64 * kWaves, 4) void pa_prefill_kernel(PaPrefillArg
           sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf, ql[kk], sc[u], 0, 0, 0);
         }
       }
-      // The products are read before the branch on `mask`: the compiler leaves out the
-      // wait for a matrix instruction whose result is first read behind one.
       float mloc = -INFINITY;
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 4; ++r) mloc = fmaxf(mloc, sc[u][r]);
-      asm volatile("" : "+v"(mloc));
       // causal + missing-page mask
       if (key0 + 31 > wave_first || here != 3u) {
         mloc = -INFINITY;
