@@ -813,7 +813,7 @@ def test_fc2_sums_whatever_the_batch(gpu, oracle, H, D, batches):
 @pytest.mark.parametrize("H,D", [(4, 64), (16, 128)])
 @pytest.mark.parametrize("n", [127, 128, 129, 300])
 def test_packed_rows_of_prompts(gpu, H, D, n):
-    """Every row of a packed matrix of one to a few groups of 128 rows, its own values and scale."""
+    """Every row of a packed fp16 matrix of one to a few groups of 128 rows."""
     import torch
 
     # the prompt's last token sees every row: one that went astray shows in its logits, against
@@ -845,6 +845,37 @@ def test_packed_rows_of_prompts(gpu, H, D, n):
         out.append(logits.cpu().numpy())
     # fp16 products either way: two roundings of their inputs in another order
     assert rel_err(out[0], out[1]) < 5e-3, rel_err(out[0], out[1])
+
+
+@pytest.mark.parametrize("H,D", [(4, 64), (16, 128)])
+@pytest.mark.parametrize("n", [127, 128, 129, 300])
+def test_packed_int8_rows_of_prompts(gpu, oracle, H, D, n):
+    """Every packed int8 row with its own scale: K and V of every token of a prompt against the
+    same tokens one by one.  The first layer's follow the LayerNorm's rows, whose sums are added
+    in another order; the second's also the attention's and fc1's.  An int8 step is 1/127 of a
+    row's largest value, some 0.03 of its rms: three rows whose values were all a step apart
+    would move a product by 0.055 of its rms, one value of 256 by 0.002.  Another token's row
+    is off by 1.4, its scale by as much as it differs."""
+    from types import SimpleNamespace
+    from _util import decoder_kv_to_oracle
+    w = _int8_model(oracle, L=2, H=H, D=D, V=600, S=n + 8, seed=53)
+    ids = np.random.default_rng(n).integers(0, 600, n).tolist()
+    got = []
+    for whole in (True, False):
+        dec = _make_gpu_decoder(w, max_batch=1)
+        dec.begin_synthetic(1, 0, 0, False)
+        if whole:
+            dec.prefill(0, ids)
+        else:
+            for t in ids:
+                dec.step([t])
+        _torch().cuda.synchronize()
+        kv = np.zeros((2, 2, 1, H, (n + 15) // 16 * 16, D), np.float32)
+        decoder_kv_to_oracle(dec, SimpleNamespace(cfg={"L": 2}, kv=lambda l, i: kv[l, i]), 1, n)
+        got.append(kv[:, :, 0, :, :n])
+    for layer, tol in ((0, 2e-3), (1, 0.055)):
+        d = np.sqrt(((got[0][layer] - got[1][layer]) ** 2).mean((1, 3)) / (got[1][layer] ** 2).mean((1, 3)))
+        assert d.max() < tol, (layer, d.argmax(), d.max())
 
 
 @pytest.mark.parametrize("max_batch,max_seq", [(1, 40), (4, 2048)])  # a thread an element, and eight
