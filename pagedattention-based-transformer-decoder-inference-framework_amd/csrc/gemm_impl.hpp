@@ -589,9 +589,11 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
 // looked up between its stores: 73), x 8192 x 2048 57 (64), x 2048 x 2048 and x 2048 x 8192
 // 30 on average (31); bound by the stores of fp32 rows (the products alone of 2048 x 6144 x
 // 2048: 24 us, with their rows 41).
-// ROWS: fp32 rows alone; else pages or packed fp16 rows too.
+// ROWS: fp32 rows alone; else pages or packed fp16 rows too.  Two waves a SIMD in the bounds:
+// with one, 64 x 64 blocks of four waves get their sums in accumulation registers and move them
+// out and back at every stage (200 x 3072 x 4096, weights in L2: int8 16.1 us, now 12.3).
 template <GemmKind KIND, bool A_PACKED, bool ROWS, int MB, int NB, int WM, int WN, int ST>
-__global__ __launch_bounds__(64 * WM * WN, 1) void gemm_block_kernel(GemmArgs a) {
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_block_kernel(GemmArgs a) {
   using Tr = GemmTraits<KIND>;
   using acc_t = typename Tr::acc_t;
   using elem_t = typename Tr::elem_t;
@@ -863,10 +865,8 @@ inline bool narrow_decode_tile(const GemmArgs& a, int kstep, TileChoice& t) {
 // The block form whose rounds of workgroups take least; us of a round at K = 2048 with one,
 // two and three blocks a CU (mm_impl.hpp's forms, int8's by times of their own; fp16's are 1.4
 // times bf16's in every form, for sums in eight parts).  Timed over 65 to 2048 rows, 1024 to
-// 12288 columns and K 256 to 8192, the form so chosen is on average 0 to 2 % off the best from K
-// 1024 on, 2 to 10 % below.  fp16 blocks of 64 x 64 are faster than 64 x 128 at small K (1000 x
-// 1024 x 256 8.3 and 11.4 us, 130 x 4096 x 512 8.0 and 9.3, x 2048 15.7 and 15.9; a prompt of 250
-// rows, qkv of K 1024 11.4 and 12.2) and 5 % slower from K 4096 on.
+// 12288 columns and K 256 to 8192, the form so chosen is on average 0 to 4 % off the best from K
+// 1024 on, 4 to 14 % below (int8 most).
 template <GemmKind KIND, bool A_PACKED, bool ROWS>
 hipError_t launch_gemm_block(const GemmArgs& a, hipStream_t st) {
   void (*best)(GemmArgs) = nullptr;
@@ -889,8 +889,7 @@ hipError_t launch_gemm_block(const GemmArgs& a, hipStream_t st) {
     consider(8, 8, 8, 1, {13.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 8, 4, 2, 3>);
     consider(8, 16, 8, 1, {21.5f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 16, 2, 4, 3>);
   } else {
-    if (a.K <= 2048)
-      consider(4, 4, 4, 3, {11.4f, 13.7f, 18.9f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 4, 2, 2, 3>);
+    consider(4, 4, 4, 3, {11.4f, 13.7f, 18.9f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 4, 2, 2, 3>);
     consider(4, 8, 8, 1, {12.1f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 4>);
     consider(4, 8, 8, 2, {12.6f, 20.1f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 4, 8, 2, 4, 3>);
     consider(8, 8, 8, 1, {17.6f}, gemm_block_kernel<KIND, A_PACKED, ROWS, 8, 8, 4, 2, 3>);

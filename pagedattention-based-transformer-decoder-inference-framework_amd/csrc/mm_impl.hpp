@@ -976,9 +976,10 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
 // blocks of 16 NB columns in n columns
 __host__ __device__ __forceinline__ int group_across(int n, int NB) { return (n + 16 * NB - 1) / (16 * NB); }
 
-// A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).
+// A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).  Two waves a SIMD in
+// the bounds, for the blocks of four waves (gemm_impl.hpp, gemm_block_kernel).
 template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
-__global__ __launch_bounds__(64 * WM * WN, 1) void mm_block_kernel(KernelArgs p) {
+__global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p) {
   constexpr int MT = MB / WM, NT = NB / WN;
   __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
   int id = blockIdx.y * gridDim.x + blockIdx.x;
