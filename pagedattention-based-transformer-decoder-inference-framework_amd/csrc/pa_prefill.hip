@@ -358,7 +358,8 @@ hipError_t launch_prefill(const PaPrefillArgs& a, hipStream_t st) {
 
 // The key range is cut into splits of `per` stages, the length for which the rounds of
 // workgroups (4 per CU) times their length is least, a split more counted as half a stage
-// for its merge; no more than split_bound of them a query.  32 queries a wave in place of
+// for its merge; no more than split_bound of them a query, and one of up to 64 keys (16 heads of
+// 128, 64 queries: 7.4 us, in two splits 10.2).  32 queries a wave in place of
 // 16 (16 heads of 128, with the merge; two waves a SIMD, of 32 queries there can be no more):
 // 2048 queries 72 -> 70 us, but those after 2048 more 120 -> 139, 1024 34 -> 36, 117 11 -> 14;
 // heads of 64 2048 48 -> 60.
@@ -377,7 +378,7 @@ PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   const int bound = split_bound(H, m);
   int best = most;
   double least = 1e30;
-  for (int n = 1; n <= std::min(bound, most); ++n) {
+  for (int n = 1; n <= (p0 + m <= 64 ? 1 : std::min(bound, most)); ++n) {
     const int per = (most + n - 1) / n;
     long long wgs = 0;
     for (int q = 0; q < m; q += kTileQueries)

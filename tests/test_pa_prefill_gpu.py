@@ -129,6 +129,19 @@ def test_pa_prefill_merges(gpu, oracle, H, D, p0, m):
         assert_parity(out[i:i + 1], ref, RTOL, ATOL_FRAC)
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("p0,m", [(0, 33), (0, 64), (31, 33), (50, 1)])
+def test_pa_prefill_short_contexts_are_one_split(gpu, D, p0, m):
+    """Up to 64 keys: the same bits with a workspace and without, no merge behind it."""
+    import llm_capi
+    rng = np.random.default_rng(p0 + m)
+    kp, vp, pt = _case(rng, rows=1, H=16, D=D, T=p0 + m, ts=16)
+    q = _dev((rng.standard_normal((m, 16, D)) * D ** -0.25).astype(np.float32))
+    k, v, t = _dev(kp), _dev(vp), _dev(pt)
+    whole, split = (llm_capi.pa_prefill(q, k, v, t, row=0, p0=p0, split=s).cpu().numpy() for s in (False, True))
+    np.testing.assert_array_equal(split.view(np.uint32), whole.view(np.uint32))
+
+
 def test_pa_prefill_missing_pages_and_scale(gpu, oracle):
     import llm_capi
     rng = np.random.default_rng(11)
