@@ -106,3 +106,15 @@ def test_few_tokens_left(gpu, shape, k, p):
         ref, margin = sample_rows(logits, 0.7, k, p, seed=5, counter=counter)
         got = draw(logits, 0.7, k, p, counter)
         assert ((got == ref) | (margin < 1e-4)).all(), (got, ref, margin)
+
+
+@pytest.mark.parametrize("V", [255, 1057, 1600, 2047, 2048, 2816, 4096])
+@pytest.mark.parametrize("k", [2, 6, 24, 50, 64])
+def test_short_rows(gpu, V, k):
+    """Rows of about as many groups of eight threads as top_k, and of fewer."""
+    from oracle.oracle import sample_rows
+    logits = (2 * np.random.default_rng(V + k).standard_normal((5, V))).astype(np.float32)
+    for p in (0.6, 1.0):
+        ref, margin = sample_rows(logits, 0.8, k, p, seed=5, counter=k)
+        got = draw(logits, 0.8, k, p, k)
+        assert ((got == ref) | (margin < 1e-4)).all(), (got, ref, margin)
