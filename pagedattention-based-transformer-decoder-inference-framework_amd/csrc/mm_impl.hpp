@@ -690,7 +690,7 @@ constexpr int columns_each(int rows, int cols) {
 // A wave's ROWS x COLS finished sums, row by row in LDS -> the epilogue.  Stores are whole
 // lines of a row, 64 columns of it by neighbouring lanes (straight from the accumulators a
 // pair of columns a lane: bf16 2048 x 12288 x 2048 with fp32 results 101.5 us, now 95;
-// gate and up with their activation 103, now 86; the products alone 77), and a thread's rows
+// 2011 rows of gate and up with their activation 108, now 105; the products alone 77), and a thread's rows
 // have one set of columns, whose bias, head and place are found once.  All that is loaded
 // is loaded before the first store: a load behind stores is waited for together with them.
 template <typename T, int EPI, int ROWS, int COLS, int STRIDE>
@@ -1058,8 +1058,8 @@ hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
 // K = 2048 with one, two and three a CU (us, weights from memory).  A product takes the form
 // whose rounds take least.  Two blocks of 64 x 128 a CU hide each other's first loads and last
 // stores, so there are two depths of them: 2048 x 2560 28.7 us (four stages, one a CU: 33.8),
-// 1000 x 2048 12.3 (three stages: 13.2).  2048 x 12288: 3 rounds of 128 x 256, 83 us with the
-// activation (128 x 128: 110); 2048 x 2048: one round of 128 x 128, 17.1 us (128 x 256 leaves
+// 1000 x 2048 12.3 (three stages: 13.2).  2048 x 12288: 3 rounds of 128 x 256, 97 us with the
+// activation (128 x 128: 119); 2048 x 2048: one round of 128 x 128, 17.1 us (128 x 256 leaves
 // half the chip idle: 26.4); 700 x 2048: 64 x 128, 12.0 us (128 x 128: 17.3).  fp32 blocks are
 // bound by the matrix cores and take the time of their area, the small ones, of which a CU
 // holds several, the time between two rounds: 2048 x 2048: two rounds of 64 x 128, 140 us
