@@ -96,11 +96,12 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint3
   lo = __builtin_bit_cast(uint32_t, f16x2{(_Float16)(x - (float)h[0]), (_Float16)(y - (float)h[1])});
 }
 
-template <int D, int TS>
-__global__ __launch_bounds__(64 * kWaves, 4) void pa_prefill_kernel(PaPrefillArgs a) {
+// KEYS: of a stage; 4 workgroups' stages fill a CU's LDS where these are stage_keys(D), 2 else.
+template <int D, int TS, int KEYS>
+__global__ __launch_bounds__(64 * kWaves, KEYS == stage_keys(D) ? 4 : 2) void pa_prefill_kernel(PaPrefillArgs a) {
   constexpr int ROWB = 2 * D;                // bytes of a key's row
   constexpr int CPR = D / 8;                 // its 16-byte chunks
-  constexpr int kStageKeys = stage_keys(D);
+  constexpr int kStageKeys = KEYS;
   constexpr int OWN = kStageKeys / kWaves;   // keys of a stage that a wave loads, of one page
   constexpr int LOADS = OWN * ROWB / 1024;   // its loads of 1 KiB, each of K and V
   constexpr int BLOCKS = kStageKeys / 32, GROUPS = kStageKeys / 16;
@@ -352,14 +353,19 @@ __global__ __launch_bounds__(64 * kWaves, 4) void pa_prefill_kernel(PaPrefillArg
 template <int D, int TS>
 hipError_t launch_prefill(const PaPrefillArgs& a, hipStream_t st) {
   const dim3 grid(a.H, (a.m + kTileQueries - 1) / kTileQueries, a.nsplit);
-  hipLaunchKernelGGL((pa_prefill_kernel<D, TS>), grid, dim3(64 * kWaves), 0, st, a);
+  // one pass of few workgroups: 64 keys a stage, half the barriers, as no others fill the waits
+  // (16 heads of 128: 17 queries after 4,000 114 -> 100 us, 2,048 after 2,048 147 -> 134)
+  const bool alone = a.nsplit == 1 && (long long)grid.x * grid.y <= 512;
+  hipLaunchKernelGGL((alone ? pa_prefill_kernel<D, TS, 64> : pa_prefill_kernel<D, TS, stage_keys(D)>), grid,
+                     dim3(64 * kWaves), 0, st, a);
   return hipGetLastError();
 }
 
 // The key range is cut into splits of `per` stages, the length for which the rounds of
-// workgroups (4 per CU) times their length is least, a split more counted as half a stage
-// for its merge; no more than split_bound of them a query, and one of up to 64 keys (16 heads of
-// 128, 64 queries: 7.4 us, in two splits 10.2).  32 queries a wave in place of
+// workgroups (4 per CU) times their length is least, a split more counted as half a stage, a
+// whole one where many rows write short ones, and more than 16 of them, which pa_merge_row_kernel
+// merges, as four; no more than split_bound of them a query, and one of up to 64 keys (16 heads
+// of 128, 64 queries: 7.4 us, in two splits 10.2).  32 queries a wave in place of
 // 16 (16 heads of 128, with the merge; two waves a SIMD, of 32 queries there can be no more):
 // 2048 queries 72 -> 70 us, but those after 2048 more 120 -> 139, 1024 34 -> 36, 117 11 -> 14;
 // heads of 64 2048 48 -> 60.
@@ -376,6 +382,10 @@ PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   const int H = kv->num_heads, kStageKeys = stage_keys(kv->head_dim);
   const int most = (p0 + m - 1) / kStageKeys + 1;
   const int bound = split_bound(H, m);
+  // us by splits, heads of 128.  4 heads, 64 queries after 8,000: 12 28.5, 16 24.8, 20 26.2, 32
+  // 25.5; 32 heads: 8 46.3, 16 43.7, 23 50.0.  32 heads, 128 queries after 3,000: 4 36.9, 8 35.7,
+  // 14 41.9; 4 heads, 300 queries: 3 11.9, 5 11.6.
+  const double split = kv->head_dim == 128 && m * H >= 1500 ? 1.0 : 0.5, many = 4.0;
   int best = most;
   double least = 1e30;
   for (int n = 1; n <= (p0 + m <= 64 ? 1 : std::min(bound, most)); ++n) {
@@ -383,7 +393,8 @@ PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
     long long wgs = 0;
     for (int q = 0; q < m; q += kTileQueries)
       wgs += ((p0 + std::min(q + kTileQueries, m) - 1) / kStageKeys + per) / per;
-    const double cost = (double)((wgs * H + kRound - 1) / kRound) * per + 0.5 * (most + per - 1) / per;
+    const double cost = (double)((wgs * H + kRound - 1) / kRound) * per + split * (most + per - 1) / per +
+                        (n > 16 ? many : 0.0);
     if (cost < least) {
       least = cost;
       best = per;

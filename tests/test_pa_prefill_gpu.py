@@ -129,6 +129,21 @@ def test_pa_prefill_merges(gpu, oracle, H, D, p0, m):
         assert_parity(out[i:i + 1], ref, RTOL, ATOL_FRAC)
 
 
+@pytest.mark.parametrize("H,p0,m", [(2, 0, 65), (2, 4095, 17), (2, 8190, 70), (12, 1000, 128), (16, 2040, 1), (33, 0, 1000)])
+def test_pa_prefill_stages(gpu, oracle, H, p0, m):
+    """One pass by stages of 64 keys where workgroups are few (of 32 past 512), splits of many
+    short stages: contexts that end inside a stage, more than 16 splits' worth of keys."""
+    import llm_capi
+    rng = np.random.default_rng(p0 + m)
+    kp, vp, pt = _case(rng, rows=1, H=H, D=128, T=p0 + m, ts=16, nan_tail=True)
+    q = (rng.standard_normal((m, H, 128)) * 128 ** -0.25).astype(np.float32)
+    k, v, t = _dev(kp), _dev(vp), _dev(pt)
+    for split in (False, True):
+        out = llm_capi.pa_prefill(_dev(q), k, v, t, row=0, p0=p0, split=split).cpu().numpy()
+        for i in {0, m // 2, m - 1}:
+            assert_parity(out[i:i + 1], _oracle(oracle, q[i:i + 1], kp, vp, pt, 0, p0 + i), RTOL, ATOL_FRAC)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("p0,m", [(0, 33), (0, 64), (31, 33), (50, 1)])
 def test_pa_prefill_short_contexts_are_one_split(gpu, D, p0, m):
