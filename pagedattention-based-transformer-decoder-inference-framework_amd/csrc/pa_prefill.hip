@@ -362,13 +362,13 @@ hipError_t launch_prefill(const PaPrefillArgs& a, hipStream_t st) {
 }
 
 // The key range is cut into splits of `per` stages, the length for which the rounds of
-// workgroups (4 per CU) times their length is least, a split more counted as half a stage, a
-// whole one where many rows write short ones, and more than 16 of them, which pa_merge_row_kernel
-// merges, as four; no more than split_bound of them a query, and one of up to 64 keys (16 heads
-// of 128, 64 queries: 7.4 us, in two splits 10.2).  32 queries a wave in place of
-// 16 (16 heads of 128, with the merge; two waves a SIMD, of 32 queries there can be no more):
-// 2048 queries 72 -> 70 us, but those after 2048 more 120 -> 139, 1024 34 -> 36, 117 11 -> 14;
-// heads of 64 2048 48 -> 60.
+// workgroups (4 per CU) times their length is least.  A split more counts as half a stage, a
+// whole one where many rows with a long context before them write short splits, and more than 16,
+// which pa_merge_row_kernel merges, as four besides.  No more than split_bound of them a query,
+// and one of up to 64 keys (16 heads of 128, 64 queries: 7.4 us, in two splits 10.2).
+// 32 queries a wave in place of 16 (16 heads of 128, with the merge; two waves a SIMD, of 32
+// queries there can be no more): 2048 queries 72 -> 70 us, but those after 2048 more 120 -> 139,
+// 1024 34 -> 36, 117 11 -> 14; heads of 64 2048 48 -> 60.
 constexpr int kRound = 1024;
 struct PrefillPlan {
   int nsplit, pps;
@@ -384,8 +384,8 @@ PrefillPlan prefill_plan(const pa_kv_view* kv, int p0, int m) {
   const int bound = split_bound(H, m);
   // us by splits, heads of 128.  4 heads, 64 queries after 8,000: 12 28.5, 16 24.8, 20 26.2, 32
   // 25.5; 32 heads: 8 46.3, 16 43.7, 23 50.0.  32 heads, 128 queries after 3,000: 4 36.9, 8 35.7,
-  // 14 41.9; 4 heads, 300 queries: 3 11.9, 5 11.6.
-  const double split = kv->head_dim == 128 && m * H >= 1500 ? 1.0 : 0.5, many = 4.0;
+  // 14 41.9; 16 heads, 200 queries alone, whose rows have half of them: 3 12.9, 4 12.4.
+  const double split = kv->head_dim == 128 && m * H >= 1500 && p0 >= m ? 1.0 : 0.5, many = 4.0;
   int best = most;
   double least = 1e30;
   for (int n = 1; n <= (p0 + m <= 64 ? 1 : std::min(bound, most)); ++n) {
