@@ -583,56 +583,37 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_kernel(GemmArgs a) {
   gemm_tile<KIND, MT, NT, WAVES, DIAG, PRO>(a, bx, by, bz, (int)gridDim.z, (int)gridDim.x);
 }
 
-// Rows of a prompt: blocks of 16 MB rows x 16 NB columns through LDS
-// (block_product.hpp), compute-shaped where the kernel above is a weight stream.
-// int8, 2048 rows: x 6144 x 2048 with the KV append 53 us (pages through the block's LDS and
-// looked up between its stores: 73), x 8192 x 2048 57 (64), x 2048 x 2048 and x 2048 x 8192
-// 30 on average (31); bound by the stores of fp32 rows (the products alone of 2048 x 6144 x
-// 2048: 24 us, with their rows 41).
-// ROWS: fp32 rows alone; else pages or packed fp16 rows too.  Two waves a SIMD in the bounds:
-// with one, 64 x 64 blocks of four waves get their sums in accumulation registers and move them
-// out and back at every stage (200 x 3072 x 4096, weights in L2: int8 16.1 us, now 12.3).
-template <GemmKind KIND, bool A_PACKED, bool ROWS, int MB, int NB, int WM, int WN, int ST>
-__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_block_kernel(GemmArgs a) {
-  using Tr = GemmTraits<KIND>;
-  using acc_t = typename Tr::acc_t;
-  using elem_t = typename Tr::elem_t;
-  constexpr int MT = MB / WM, NT = NB / WN;
-  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
-  const TileAt tile = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y);
-  const int lane = lane_id(), w = wave_id_uniform(), wm = w / WN, wn = w % WN;
-  const int KS = a.KS, ntiles = (a.N + 15) >> 4, mtiles = (a.M + 15) >> 4;
-  const int m0 = tile.y * 16 * MB, nt0 = tile.x * NB;
-  acc_t acc[MT][NT];
-  block_product<A_PACKED, KIND == GemmKind::F16, MB, NB, WM, WN, ST>(
-      lds, acc, KS, m0 + 16 * wm * MT < a.M,
-      [&](int r) {
-        const char* A = reinterpret_cast<const char*>(a.A);
-        return A_PACKED ? A + (size_t)min((m0 >> 4) + r, mtiles - 1) * KS * 1024
-                        : A + (size_t)min(m0 + r, a.M - 1) * a.lda * Tr::ESIZE;
-      },
-      [&](int t) {
-        return reinterpret_cast<const char*>(a.B) + (size_t)min(nt0 + t, ntiles - 1) * KS * 1024;
-      },
-      [](u32x4 x, u32x4 y, acc_t c) {
-        if constexpr (KIND == GemmKind::I8)
-          return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, x),
-                                                       __builtin_bit_cast(i32x4, y), c, 0, 0, 0);
-        else
-          return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x),
-                                                        __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
-      });
-  // The wave's sums through LDS (block_product has read it out), so that stores are 16
-  // bytes a lane, lines of a row by neighbouring lanes, and a lane has one set of C columns,
-  // whose scale, bias and page are found once.  All that is loaded is loaded before the
-  // first store: a load behind stores is waited for together with them.
-  constexpr int STRIDE = 16 * NB + 4, C = ROWS ? 4 : 8, ACROSS = 16 * NT / C, STEP = 64 / ACROSS,
-                PER = 16 * MT / STEP;
-  static_assert(sizeof(lds) >= sizeof(elem_t) * 16 * MB * STRIDE && 64 % ACROSS == 0 && PER >= 1);
-  elem_t* sums = reinterpret_cast<elem_t*>(&lds[0][0][0]);
-  spread_sums<STRIDE>(acc, sums, 16 * wm * MT, 16 * wn * NT);
-  const int row0 = 16 * wm * MT + lane / ACROSS, col0 = 16 * wn * NT + lane % ACROSS * C;
-  const int m = m0 + row0, n = 16 * nt0 + col0;  // this lane's rows m + STEP i, columns n .. n + C - 1
+// The operands of a block: row m0 + r of A (packed: row tile r from m0 on; the last one for those
+// past it), column tile t, their product.
+template <GemmKind KIND, bool A_PACKED>
+__device__ __forceinline__ const char* block_rows(const GemmArgs& a, int m0, int r) {
+  const char* A = reinterpret_cast<const char*>(a.A);
+  return A_PACKED ? A + (size_t)min((m0 >> 4) + r, ((a.M + 15) >> 4) - 1) * a.KS * 1024
+                  : A + (size_t)min(m0 + r, a.M - 1) * a.lda * GemmTraits<KIND>::ESIZE;
+}
+__device__ __forceinline__ const char* block_columns(const GemmArgs& a, int t) {
+  return reinterpret_cast<const char*>(a.B) + (size_t)min(t, ((a.N + 15) >> 4) - 1) * a.KS * 1024;
+}
+template <GemmKind KIND, typename Acc>
+__device__ __forceinline__ Acc block_mma(u32x4 x, u32x4 y, Acc c) {
+  if constexpr (KIND == GemmKind::I8)
+    return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(i32x4, x), __builtin_bit_cast(i32x4, y), c, 0,
+                                                 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), c, 0,
+                                                  0, 0);
+}
+
+// A wave's sums of EM rows and EN columns, row m0 and column n0 on, in LDS rows of STRIDE -> C, packed
+// rows, pages.  Stores are 16 bytes a lane, lines of a row by neighbouring lanes, and a lane has one
+// set of C columns, whose scale, bias and page are found once.  All that is loaded is loaded before
+// the first store: a load behind stores is waited for together with them.
+template <GemmKind KIND, bool ROWS, int EM, int EN, int STRIDE, typename E>
+__device__ __forceinline__ void emit_sums(const GemmArgs& a, E* sums, int m0, int n0) {
+  constexpr int C = ROWS ? 4 : 8, ACROSS = EN / C, STEP = 64 / ACROSS, PER = EM / STEP;
+  static_assert(64 % ACROSS == 0 && PER >= 1);
+  const int lane = lane_id(), row0 = lane / ACROSS, col0 = lane % ACROSS * C;
+  const int m = m0 + row0, n = n0 + col0;  // this lane's rows m + STEP i, columns n .. n + C - 1
   if (n >= a.N) return;  // (N is a multiple of 16)
   sums += row0 * STRIDE + col0;
   const KvAppend& kv = a.kv;
@@ -664,49 +645,129 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_block_kernel(GemmArgs a)
     }
   }
   const bool vec = ((a.c_ld | a.c_cols) & 3) == 0 && reinterpret_cast<uintptr_t>(a.C) % 16 == 0;
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
+  // FINISHED: LDS holds what `value` made of the sums already.
+  const auto value = [&](E s, float s_row, int k) {
 #pragma clang fp contract(off)  // y = acc * scale + bias rounded twice, as the reference
-    const int r = m + STEP * i;
-    if (r >= a.M) break;
-    float y[C];
+    float y = (float)s;
+    if constexpr (KIND == GemmKind::I8) y = y * (s_row * sw[k]);
+    return a.bias ? y + bias[k] : y;
+  };
+  const auto put_rows = [&](auto finished) {
 #pragma unroll
-    for (int k = 0; k < C; ++k) {
-      const elem_t s = sums[i * STEP * STRIDE + k];
-      if constexpr (KIND == GemmKind::I8)
-        if (a.acc_out) a.acc_out[(size_t)r * a.N + n + k] = s;
-      y[k] = (float)s;
-      if constexpr (KIND == GemmKind::I8) y[k] = y[k] * (sa[i] * sw[k]);
-      if (a.bias) y[k] = y[k] + bias[k];
-      y[k] = apply_act(y[k], a.act);
-    }
-    if (a.C && n < a.c_cols) {
-      float* to = a.C + (size_t)r * a.c_ld + n;
-      if (vec && n + C <= a.c_cols) {
+    for (int i = 0; i < PER; ++i) {
+      const int r = m + STEP * i;
+      if (r >= a.M) break;
+      float y[C];
 #pragma unroll
-        for (int k = 0; k < C; k += 4) {
-          const f32x4 v = {y[k], y[k + 1], y[k + 2], y[k + 3]};
-          // int8 blocks are short, and written past L2 their rows come too thick
-          // (2048 x 12288 x 2048 66 us, past L2 70)
-          if constexpr (KIND == GemmKind::I8 || !ROWS) *reinterpret_cast<f32x4*>(to + k) = v;
-          else store_through(to + k, __builtin_bit_cast(u32x4, v));
+      for (int k = 0; k < C; ++k) {
+        const E s = sums[i * STEP * STRIDE + k];
+        if constexpr (decltype(finished)::value) {
+          y[k] = __builtin_bit_cast(float, s);
+        } else {
+          y[k] = value(s, sa[i], k);
+          if (a.act == LLM_ACT_RELU) y[k] = fmaxf(y[k], 0.f);
         }
-      } else {
+      }
+      if (a.C && n < a.c_cols) {
+        float* to = a.C + (size_t)r * a.c_ld + n;
+        if (vec && n + C <= a.c_cols) {
 #pragma unroll
-        for (int k = 0; k < C; ++k)
-          if (n + k < a.c_cols) to[k] = y[k];
+          for (int k = 0; k < C; k += 4) {
+            const f32x4 v = {y[k], y[k + 1], y[k + 2], y[k + 3]};
+            // int8 blocks are short, and written past L2 their rows come too thick
+            // (2048 x 12288 x 2048 66 us, past L2 70)
+            if constexpr (KIND == GemmKind::I8 || !ROWS) *reinterpret_cast<f32x4*>(to + k) = v;
+            else store_through(to + k, __builtin_bit_cast(u32x4, v));
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < C; ++k)
+            if (n + k < a.c_cols) to[k] = y[k];
+        }
+      }
+      if constexpr (!ROWS) {
+        f16x8 h;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) h[k] = (_Float16)y[k];
+        if (a.c16) *reinterpret_cast<f16x8*>(a.c16 + a_frag_off_f16(r, n, a.N >> 5)) = h;
+        if (page[i] >= 0)
+          *reinterpret_cast<f16x8*>((which == 2 ? kv.v_pool : kv.k_pool) +
+                                    (size_t)page[i] * kv.page_stride + (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
       }
     }
-    if constexpr (!ROWS) {
-      f16x8 h;
+  };
+  if constexpr (KIND == GemmKind::I8)
+    if (a.acc_out) {
+      const bool whole = reinterpret_cast<uintptr_t>(a.acc_out) % 16 == 0;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) h[k] = (_Float16)y[k];
-      if (a.c16) *reinterpret_cast<f16x8*>(a.c16 + a_frag_off_f16(r, n, a.N >> 5)) = h;
-      if (page[i] >= 0)
-        *reinterpret_cast<f16x8*>((which == 2 ? kv.v_pool : kv.k_pool) +
-                                  (size_t)page[i] * kv.page_stride + (size_t)(pos[i] % kv.TS) * kv.D + d) = h;
+      for (int i = 0; i < PER; ++i) {
+        const int r = m + STEP * i;
+        if (r >= a.M) break;
+#pragma unroll
+        for (int k = 0; k < C; k += 4) {
+          const i32x4 s = *reinterpret_cast<const i32x4*>(sums + i * STEP * STRIDE + k);
+          int32_t* to = a.acc_out + (size_t)r * a.N + n + k;
+          if (whole) {
+            *reinterpret_cast<i32x4*>(to) = s;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) to[e] = s[e];
+          }
+        }
+      }
+    }
+  if (a.act != LLM_ACT_GELU) {
+    put_rows(std::false_type());
+    return;
+  }
+  // GELU first and by a loop: in line at every element its code made 40 of the 44 KB of a 128 x 256
+  // block's kernel, now 17 to 28, which a launch finds in no cache (2048 x 4096 int8: K 256 18.6 us,
+  // now 13.7; K 2048 29, 24)
+#pragma unroll 1
+  for (int i = 0; i < PER; ++i) {
+    const int r = m + STEP * i;
+    if (r >= a.M) break;
+    const float s_row = KIND == GemmKind::I8 && a.sa ? a.sa[r] : 1.f;
+#pragma unroll
+    for (int k = 0; k < C; ++k) {
+      E& s = sums[i * STEP * STRIDE + k];
+      s = __builtin_bit_cast(E, apply_act(value(s, s_row, k), LLM_ACT_GELU));
     }
   }
+  put_rows(std::true_type());
+}
+
+// Rows of a prompt: blocks of 16 MB rows x 16 NB columns through LDS
+// (block_product.hpp), compute-shaped where the kernel above is a weight stream.
+// int8, 2048 rows: x 6144 x 2048 with the KV append 46.7 us (GELU's code in line for every element,
+// 40 KB of it to be jumped over and found in no cache: 52), x 8192 x 2048 45.9 (54.4), x 2048 x 2048
+// and x 2048 x 8192 27 on average (29.3); bound by the stores of fp32 rows (the products alone of
+// 2048 x 6144 x 2048: 24 us, with their rows 41).
+// ROWS: fp32 rows alone; else pages or packed fp16 rows too.  Two waves a SIMD in the bounds:
+// with one, 64 x 64 blocks of four waves get their sums in accumulation registers and move them
+// out and back at every stage (200 x 3072 x 4096, weights in L2: int8 16.1 us, now 12.3).
+template <GemmKind KIND, bool A_PACKED, bool ROWS, int MB, int NB, int WM, int WN, int ST>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_block_kernel(GemmArgs a) {
+  using Tr = GemmTraits<KIND>;
+  using acc_t = typename Tr::acc_t;
+  using elem_t = typename Tr::elem_t;
+  constexpr int MT = MB / WM, NT = NB / WN;
+  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
+  const TileAt tile = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x, gridDim.y);
+  const int w = wave_id_uniform(), wm = w / WN, wn = w % WN;
+  const int m0 = tile.y * 16 * MB, nt0 = tile.x * NB;
+  acc_t acc[MT][NT];
+  block_product<A_PACKED, KIND == GemmKind::F16, MB, NB, WM, WN, ST>(
+      lds, acc, a.KS, m0 + 16 * wm * MT < a.M,
+      [&](int r) { return block_rows<KIND, A_PACKED>(a, m0, r); },
+      [&](int t) { return block_columns(a, nt0 + t); },
+      [](u32x4 x, u32x4 y, acc_t c) { return block_mma<KIND>(x, y, c); });
+  // (block_product has read LDS out)
+  constexpr int STRIDE = 16 * NB + 4;
+  static_assert(sizeof(lds) >= sizeof(elem_t) * 16 * MB * STRIDE);
+  elem_t* sums = reinterpret_cast<elem_t*>(&lds[0][0][0]) + 16 * wm * MT * STRIDE + 16 * wn * NT;
+  spread_sums<STRIDE>(acc, sums, 0, 0);
+  emit_sums<KIND, ROWS, 16 * MT, 16 * NT, STRIDE>(a, sums, m0 + 16 * wm * MT, 16 * (nt0 + wn * NT));
 }
 
 // Repack W [K][N] (row-major) into per-(16-col tile, k-step) 1 KiB blocks,

@@ -758,6 +758,28 @@ __device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b
     if constexpr (EPI == kSoftplus)
 #pragma unroll
       for (int k = 0; k < 4; ++k) bias[k] = p.bias[min(n + k, b.N - 1)];
+    const auto put = [&](int row, f32x4 v) {
+      float* to = C + row * ldc + n;
+      if (vec) {
+        store_through(to, __builtin_bit_cast(u32x4, v));
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          if (n + k < b.N) to[k] = v[k];
+      }
+    };
+    if (EPI == kStore && p.a.softcap > 0.f) {  // a model's head: apart, tanhf's code is long
+#pragma unroll 1
+      for (int i = 0; i < PER; ++i) {
+        const int row = m0 + r0 + i * STEP;
+        if (row >= b.M) break;
+        f32x4 v = *reinterpret_cast<const f32x4*>(sums + i * STEP * STRIDE);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = p.a.softcap * tanhf(v[k] / p.a.softcap);
+        put(row, v);
+      }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       if (r[i].m < 0) continue;
@@ -766,16 +788,8 @@ __device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b
       for (int k = 0; k < 4; ++k) {
         if constexpr (EPI == kGroupOut) v[k] *= r[i].weight;
         else if constexpr (EPI == kSoftplus) v[k] = softplus(v[k] + bias[k]);
-        else if (p.a.softcap > 0.f) v[k] = p.a.softcap * tanhf(v[k] / p.a.softcap);
       }
-      float* to = C + (EPI == kGroupOut ? r[i].out : r[i].m) * ldc + n;
-      if (vec) {
-        store_through(to, __builtin_bit_cast(u32x4, v));
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if (n + k < b.N) to[k] = v[k];
-      }
+      put(EPI == kGroupOut ? r[i].out : r[i].m, v);
     }
   } else if constexpr (E == 16) {  // gate and up
     const size_t ld = EPI == kGlu ? p.split.ldt : b.shared ? p.g.lds : p.g.lda;

@@ -75,3 +75,46 @@ def test_fp16_sums_as_exact_as_the_streams(gpu, M, N, K):
     streams = torch.cat([llm_capi.f16_gemm(A[i:i + 64], packed, N).double() for i in range(0, M, 64)])
     off = [((x - ref).norm() / ref.norm()).item() for x in (blocks, streams)]
     assert off[0] <= 1.1 * off[1], off
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 4352, 64), (191, 2768, 320), (1025, 1040, 448)])
+@pytest.mark.parametrize("act", [0, 1, 2])
+def test_activations_with_and_without_sums(gpu, M, N, K, act):
+    """The activations of a block's epilogue, with whole sums at 16 bytes, beside them and not asked for:
+    the same C, and scale, bias and activation of the exact sums (GELU within its erf's rounding)."""
+    import torch
+    import llm_capi
+    rng = np.random.default_rng(M + N + act)
+    A = torch.from_numpy(rng.integers(-127, 128, (M, K), dtype=np.int8))
+    W = torch.from_numpy(rng.integers(-127, 128, (K, N), dtype=np.int8))
+    sa, sw, bias = (torch.from_numpy(x.astype(np.float32)) for x in
+                    (rng.uniform(0.5, 2.0, M) / 127, rng.uniform(0.5, 2.0, N) / 127, rng.standard_normal(N)))
+    a, s, w, b = A.cuda(), sa.cuda(), sw.cuda(), bias.cuda()
+    packed = llm_capi.pack_weights(W.cuda(), llm_capi.LLM_I8)
+    lib, p = llm_capi.load(), llm_capi.ptr
+    whole = A.double() @ W.double()
+    y = whole.float() * (sa[:, None] * sw) + bias
+    ref = y if act == 0 else y.relu() if act == 1 else 0.5 * y.double() * (1 + torch.erf(y.double() * 0.5 ** 0.5))
+    out = []
+    for shift in (0, 1, None):
+        C = torch.empty((M, N), device="cuda")
+        sums = torch.zeros(M * N + 4, dtype=torch.int32, device="cuda")
+        at = None if shift is None else sums[shift:].data_ptr()
+        llm_capi.check(lib.i8_gemm(p(a), K, p(packed), at, p(C), M, N, K, p(s), p(w), p(b), act,
+                                   llm_capi.stream_ptr(None)))
+        out.append(C.cpu())
+        if shift is not None:
+            assert torch.equal(sums[shift:shift + M * N].view(M, N).cpu().double(), whole)
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+    if act < 2:
+        assert torch.equal(out[0], ref)
+    else:  # y / sqrt 2, erff and two products: a few roundings of y, and of 1 + erf where it cancels
+        assert ((out[0].double() - ref).abs() <= 2.0 ** -21 * y.double().abs()).all()
+    h = torch.randn((M, K), generator=torch.Generator().manual_seed(K)).half()
+    w16 = (W.float() / 127).half()
+    C = llm_capi.f16_gemm(h.cuda(), llm_capi.pack_weights(w16.cuda(), llm_capi.LLM_F16), N, bias=b, act=act).cpu().double()
+    x = h.double() @ w16.double() + bias.double()
+    ref = x if act == 0 else x.relu() if act == 1 else 0.5 * x * (1 + torch.erf(x * 0.5 ** 0.5))
+    size = h.double().abs() @ w16.double().abs() + bias.double().abs()
+    # as test_fp16; GELU's slope is at most 1.13
+    assert ((C - ref).abs() <= 1.13 * 2.0 ** -23 * (K ** 0.5 + 2) * size + 2.0 ** -21 * x.abs()).all()
