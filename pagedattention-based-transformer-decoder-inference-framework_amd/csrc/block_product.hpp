@@ -219,6 +219,159 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
   }
 }
 
+// The same product by waves side by side, each of all 16 MB rows and 16 NT columns of its own:
+// a wave alone reads its columns of W, so they come from memory straight into its registers,
+// AHEAD k-steps ahead, and LDS holds A alone, ST stages of two k-steps.  Of a k-step a wave reads
+// MB KiB from LDS for MB NT products (128 x 256: 32 KiB a block, the form above 64 KiB and W's
+// 16 KiB written besides), and the block takes 64 KiB of LDS in place of 147: two a CU, whose
+// first loads and last stores each other's products hide.  A fragment of A is read for the
+// next k-step right behind its last product.  Sums are added in the order of the form above:
+// the same bits.
+// Amid a model, its code cold: 2011 x 12288 x 2048 bf16 with its activation 100 us, now
+// 87; 2011 x 2048 x 2048 to 6144 40, 34; 32 experts' gate and up of 2048 tokens 146, 131.  Of the matrix
+// cores' time while a CU is busy 54 % were used, now 73, at the clock that the card's power leaves
+// (1.95 GHz; the products alone, out of registers, reach 2.0 PFLOP/s).
+// AHEAD k-steps of W: the compiler waits for them as if A's loads between were none, so that 4 are
+// 2 and 8 are 3.5; 128 x 128 alone on a CU needs the 8 (2011 x 2048 x 6144 58.7 us, 53.1), 128 x 256 has
+// registers for 4.
+// A is row-major, a_at as above; w_at(j): the wave's column tile j.  When it returns, nobody reads LDS any more.
+template <int MB, int NT, int WAVES, int ST, int AHEAD, typename Acc, typename A, typename W, typename Mma>
+__device__ __forceinline__ void strip_product(u32x4 (&lds)[ST][2 * MB][64], Acc (&acc)[MB][NT], int KS,
+                                              const A& a_at, const W& w_at, const Mma& mma) {
+  constexpr int LOADS = 2 * MB / WAVES;  // of A by a wave and stage
+  static_assert(2 * MB % WAVES == 0 && LOADS % 2 == 0 && MB >= 2 + LOADS / 2 && ST >= 3 &&
+                AHEAD >= 4 && AHEAD % 2 == 0 && (ST - 1) * LOADS + AHEAD * NT < 64);
+  const int lane = lane_id(), w = wave_id_uniform(), stages = KS >> 1, last = stages - 1;
+  const int ar = lane & 15;  // as above
+  const int at0 = 8 * ar + ((lane >> 4) ^ (ar >> 1)), at1 = at0 ^ 4;
+  const char* src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int r = 8 * (w * LOADS + i) + (lane >> 3);
+    src[i] = a_at(r) + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+  }
+  const char* wp[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j) wp[j] = w_at(j);
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = Acc{0, 0, 0, 0};
+  if (stages > 0) {
+    // loads [from, to) of stage s; behind the end the last one again, which nobody reads
+    auto load_a = [&](int s, int slot, int from, int to) {
+      const size_t at = (size_t)min(s, last) * 128;
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i)
+        if (i >= from && i < to) load_to_lds(src[i] + at, lds[slot][w * LOADS + i]);
+    };
+    u32x4 a[MB], b[AHEAD][NT];
+    auto load_w = [&](int k, u32x4 (&f)[NT]) {
+      const size_t at = (size_t)min(k, 2 * last + 1) * 1024;
+#pragma unroll
+      for (int j = 0; j < NT; ++j) f[j] = *reinterpret_cast<const u32x4*>(wp[j] + at + lane * 16);
+    };
+    auto read_a = [&](int i, int slot, int u) {
+      const u32x4* tile = &lds[slot][2 * i][0];
+      a[i] = tile[u ? at1 : at0];
+    };
+    load_a(0, 0, 0, LOADS);
+    load_w(0, b[0]);
+#pragma unroll
+    for (int s = 1; s < ST - 1; ++s) load_a(s, s, 0, LOADS);
+    load_a(ST - 1, ST - 1, 0, LOADS / 2);
+#pragma unroll
+    for (int k = 1; k < AHEAD; ++k) load_w(k, b[k]);
+    __builtin_amdgcn_sched_barrier(0);
+    wait_lds_loads<(ST - 1) * LOADS - LOADS / 2 + AHEAD * NT>();  // stage 0: what was issued behind it may fly
+    barrier_only();
+#pragma unroll
+    for (int i = 0; i < MB; ++i) read_a(i, 0, 0);
+    int slot = 0, before = ST - 1;  // of stage s, of stage s - 1
+    auto stage = [&](int s, u32x4 (&b0)[NT], u32x4 (&b1)[NT]) {
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {  // the other half of the loads into the slot that was freed last
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = mma(b0[j], a[i], acc[i][j]);
+        read_a(i, slot, 1);
+        if (i < LOADS / 2) load_a(s + ST - 1, before, LOADS / 2 + i, LOADS / 2 + i + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_w(2 * s + AHEAD, b0);
+      __builtin_amdgcn_sched_barrier(0);
+      before = slot;
+      slot = slot + 1 == ST ? 0 : slot + 1;
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = mma(b1[j], a[i], acc[i][j]);
+        if (i == 1) {
+          // The reads of stage s are done, the wave's loads of stage s + 1 there.  Behind them it has
+          // issued stages s + 2 .. s + ST - 1 and 2 ST - 3 k-steps of W (s = 0: AHEAD, s = 1: more)
+          __builtin_amdgcn_sched_barrier(0);
+          wait_lds_loads<(ST - 2) * LOADS + (AHEAD < 2 * ST - 3 ? AHEAD : 2 * ST - 3) * NT>();
+          barrier_only();
+          read_a(0, slot, 0);
+          read_a(1, slot, 0);
+        } else if (i > 1) {
+          read_a(i, slot, 0);
+          if (i - 2 < LOADS / 2) load_a(s + ST, before, i - 2, i - 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      load_w(2 * s + AHEAD + 1, b1);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int s = 0;
+    for (; s + AHEAD / 2 <= stages; s += AHEAD / 2) {
+#pragma unroll
+      for (int i = 0; i < AHEAD / 2; ++i) stage(s + i, b[2 * i], b[2 * i + 1]);
+    }
+#pragma unroll
+    for (int i = 0; i < AHEAD / 2 - 1; ++i)
+      if (s + i < stages) stage(s + i, b[2 * i], b[2 * i + 1]);
+    wait_lds_loads<0>();
+    barrier_only();
+  }
+  if (KS & 1) {  // the last k-step of an odd number, from memory
+    const size_t at = (size_t)(KS - 1) * 1024 + lane * 16;
+    u32x4 b[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) b[j] = *reinterpret_cast<const u32x4*>(wp[j] + at);
+#pragma unroll
+    for (int i = 0; i < MB; ++i) {
+      const char* p = a_at(16 * i + ar) + (size_t)(KS - 1) * 64 + 16 * (lane >> 4);
+      const u32x4 a = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[i][j] = mma(b[j], a, acc[i][j]);
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// The sums of strips, SR row tiles at a time from tile i0 on, to `emit(i0, part)`, of which there is
+// one copy: they move down to the first registers.  It says whether to go on.
+template <int SR, int MB, int NT, typename Acc, typename Emit>
+__device__ __forceinline__ void strip_rows(const Acc (&acc)[MB][NT], const Emit& emit) {
+  static_assert(MB % SR == 0);
+  Acc part[MB / SR][SR][NT];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) part[i / SR][i % SR][j] = acc[i][j];
+#pragma unroll 1
+  for (int i0 = 0; i0 < MB; i0 += SR) {
+    if (!emit(i0, part[0])) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read before the next ones come
+#pragma unroll
+    for (int s = 0; s + 1 < MB / SR; ++s)
+#pragma unroll
+      for (int i = 0; i < SR; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) part[s][i][j] = part[s + 1][i][j];
+  }
+}
+
 // us of `groups` blocks of which a CU holds `per` at once: at[n - 1] with n on every CU,
 // launch included.  A round of workgroups follows the one before, the last one with as many
 // a CU as are left.

@@ -990,14 +990,10 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
 // blocks of 16 NB columns in n columns
 __host__ __device__ __forceinline__ int group_across(int n, int NB) { return (n + 16 * NB - 1) / (16 * NB); }
 
-// A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).  Two waves a SIMD in
-// the bounds, for the blocks of four waves (gemm_impl.hpp, gemm_block_kernel).
-template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
-__global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p) {
-  constexpr int MT = MB / WM, NT = NB / WN;
-  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
+// The tile of this workgroup; false: there is none for it.
+template <int EPI, int NB>
+__device__ __forceinline__ bool tile_of(const KernelArgs& p, TileAt& tile) {
   int id = blockIdx.y * gridDim.x + blockIdx.x;
-  TileAt tile;
   if constexpr (EPI == kGroupIn || EPI == kGroupOut) {
     // the shared expert's tiles (the last of the list, the most columns or k-steps)
     // go first; each kind is dealt out over the XCDs by itself
@@ -1009,12 +1005,23 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p)
     } else {
       id -= shared;
       const int nx = group_across(p.g.routed_n, NB);
-      if (id >= routed * nx) return;
+      if (id >= routed * nx) return false;
       tile = xcd_tile(id, nx, routed);
     }
   } else {
     tile = xcd_tile(id, gridDim.x, gridDim.y);
   }
+  return true;
+}
+
+// A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).  Two waves a SIMD in
+// the bounds, for the blocks of four waves (gemm_impl.hpp, gemm_block_kernel).
+template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
+__global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p) {
+  constexpr int MT = MB / WM, NT = NB / WN;
+  __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
+  TileAt tile;
+  if (!tile_of<EPI, NB>(p, tile)) return;
   const int lane = lane_id();
   const int w = wave_id_uniform();
   const Block<T> b = block_of<T, EPI>(p, 16 * MB, tile.y);
@@ -1045,6 +1052,48 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p)
   }
 }
 
+// Epilogues that strips take: a wave alone on its SIMD waits for every load and transcendental of
+// the others (2011 x 4096 x 512 to pages 28.7 us by blocks, 44 by strips; x 4096 x 128 with softplus
+// 16.4, 22; queries to be turned 38.4, 40.9).
+template <typename T, int EPI>
+constexpr bool by_strips() {
+  return Kind<T>::BF16 && (EPI == kStore || EPI == kSplit || EPI == kGlu || EPI == kHeads || EPI == kGroupIn ||
+                           EPI == kGroupOut);
+}
+
+// A block of 16 MB rows x 16 NT WAVES columns by strips (block_product.hpp, strip_product).  A
+// wave's sums leave a quarter of its rows at a time through its part of LDS, by one copy of the
+// epilogue to which they are handed down: a launch finds its code in no cache (2011 x 2048 x 2048
+// amid a model, a copy for each quarter 35 KB: 27.5 us; one, 12 KB: 20.4; blocks of eight waves
+// 25.5).
+template <typename T, int EPI, int MB, int NT, int WAVES, int ST, int AHEAD>
+__global__ __launch_bounds__(64 * WAVES, 2) void mm_strip_kernel(KernelArgs p) {
+  constexpr int NB = NT * WAVES, SR = MB / 4, STRIDE = 16 * NT + 4;
+  __shared__ u32x4 lds[ST][2 * MB][64];
+  static_assert(by_strips<T, EPI>() && sizeof(lds) >= sizeof(float) * WAVES * 16 * SR * STRIDE);
+  TileAt tile;
+  if (!tile_of<EPI, NB>(p, tile)) return;
+  const int w = wave_id_uniform();
+  const Block<T> b = block_of<T, EPI>(p, 16 * MB, tile.y);
+  const int ntiles = (b.N + 15) >> 4, nt0 = tile.x * NB + w * NT, KS = b.KS;
+  f32x4 acc[MB][NT];
+  strip_product<MB, NT, WAVES, ST, AHEAD>(
+      lds, acc, KS, [&](int r) { return a_row<T, EPI>(p, b, b.m0 + r); },
+      [&](int j) { return b.W + (size_t)min(nt0 + j, ntiles - 1) * KS * 1024; },
+      [](u32x4 x, u32x4 y, f32x4 c) { return Kind<T>::mma(x, y, c); });
+  if (16 * nt0 >= b.N) return;
+  float* sums = reinterpret_cast<float*>(&lds[0][0][0]) + w * 16 * SR * STRIDE;
+  strip_rows<SR>(acc, [&](int i0, const f32x4(&part)[SR][NT]) {
+    const int m0 = b.m0 + 16 * i0;
+    if (m0 >= b.M) return false;
+    RowOf<EPI> row(p, b, m0 + lane_id() % (16 * SR));
+    if (row.m >= 0) row.look_up(p, b);
+    spread_sums<STRIDE>(part, sums, 0, 0);
+    emit_wave<T, EPI, 16 * SR, 16 * NT, STRIDE>(p, b, sums, row, m0, 16 * nt0);
+    return true;
+  });
+}
+
 template <int EPI>
 int heads_of(const KernelArgs& p) {
   return EPI == kHeads ? p.heads.heads : 1;
@@ -1057,14 +1106,25 @@ hipError_t stream(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <int EPI>
+dim3 block_grid(const KernelArgs& p, int row_blocks, int N, int NB) {
+  if constexpr (EPI == kGroupIn || EPI == kGroupOut)
+    return dim3((p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, NB) +
+                p.g.shared_tiles * group_across(p.g.shared_n, NB));
+  return dim3(group_across(N, NB), row_blocks, heads_of<EPI>(p));
+}
+
 template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
 hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
-  dim3 grid(group_across(N, NB), row_blocks, heads_of<EPI>(p));
-  if constexpr (EPI == kGroupIn || EPI == kGroupOut)
-    grid = dim3((p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, NB) +
-                p.g.shared_tiles * group_across(p.g.shared_n, NB));
-  hipLaunchKernelGGL((mm_block_kernel<T, EPI, MB, NB, WM, WN, ST>), grid, dim3(64 * WM * WN), 0,
-                     st, p);
+  hipLaunchKernelGGL((mm_block_kernel<T, EPI, MB, NB, WM, WN, ST>), block_grid<EPI>(p, row_blocks, N, NB),
+                     dim3(64 * WM * WN), 0, st, p);
+  return hipGetLastError();
+}
+
+template <typename T, int EPI, int MB, int NT, int WAVES, int ST, int AHEAD>
+hipError_t strips(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
+  hipLaunchKernelGGL((mm_strip_kernel<T, EPI, MB, NT, WAVES, ST, AHEAD>), block_grid<EPI>(p, row_blocks, N, NT * WAVES),
+                     dim3(64 * WAVES), 0, st, p);
   return hipGetLastError();
 }
 
@@ -1074,7 +1134,12 @@ hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
 // stores, so there are two depths of them: 2048 x 2560 28.7 us (four stages, one a CU: 33.8),
 // 1000 x 2048 12.3 (three stages: 13.2).  2048 x 12288: 3 rounds of 128 x 256, 97 us with the
 // activation (128 x 128: 119); 2048 x 2048: one round of 128 x 128, 17.1 us (128 x 256 leaves
-// half the chip idle: 26.4); 700 x 2048: 64 x 128, 12.0 us (128 x 128: 17.3).  fp32 blocks are
+// half the chip idle: 26.4); 700 x 2048: 64 x 128, 12.0 us (128 x 128: 17.3).  By strips 128 x 256
+// and 128 x 128 where a CU has two of them (with weights and code from memory, two a CU, K 256 / 512 /
+// 1024 / 2048 / 4096: 128 x 256 19.6 / 24.6 / 35.9 / 62.6 / 112 us, two rounds of blocks 20.8 / 28.4 / 40.6
+// / 65.7 / 120; 128 x 128 11.0 / 15.0 / 21.5 / 34.6 / 67.4, blocks 13.1 / 17.2 / 25.4 / 40.7 / 70.2), and
+// alone from K 1024 on (128 x 128 7.4 / 9.1 / 12.2 / 19.3 / 33.1, blocks 6.6 / 8.6 / 12.7 / 20.3 / 35.1).
+// fp32 blocks are
 // bound by the matrix cores and take the time of their area, the small ones, of which a CU
 // holds several, the time between two rounds: 2048 x 2048: two rounds of 64 x 128, 140 us
 // (128 x 128: 158); 700 x 6144: five of 64 x 64, 185 us (64 x 128: 207).  Of other K the order
@@ -1085,14 +1150,14 @@ hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipS
   hipError_t (*best)(const KernelArgs&, int, int, hipStream_t) = nullptr;
   int best_y = 0;
   float least = 0.f;
+  const bool long_k = (EPI == kGroupIn || EPI == kGroupOut ? p.g.min_ks : p.KS) >= 32;
   const auto consider = [&](int mb, int nb, int per, const float (&bf16)[3], float fp32,
-                            hipError_t (*go)(const KernelArgs&, int, int, hipStream_t)) {
+                            hipError_t (*go)(const KernelArgs&, int, int, hipStream_t), bool strip = false) {
     if (mb < min_mb || mb > max_mb) return;
     const int y = (p.a.M + 16 * mb - 1) / (16 * mb);
-    int groups = group_across(N, nb) * y * heads_of<EPI>(p);
-    if constexpr (EPI == kGroupIn || EPI == kGroupOut)
-      groups = (p.g.max_tiles - p.g.shared_tiles) * group_across(p.g.routed_n, nb) +
-               p.g.shared_tiles * group_across(p.g.shared_n, nb);
+    const dim3 g = block_grid<EPI>(p, y, N, nb);
+    const int groups = g.x * g.y * g.z;
+    if (strip && groups <= 256 && !long_k) return;
     const float cost = Kind<T>::BF16 ? rounds_us(groups, per, bf16) : (float)((groups + 255) / 256) * fp32;
     if (best && cost >= least) return;
     best = go;
@@ -1106,6 +1171,10 @@ hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipS
   consider(4, 16, 1, {18.7f}, 160.f, blocks<T, EPI, 4, 16, 2, 4, 3>);
   consider(8, 8, 1, {17.6f}, 156.f, blocks<T, EPI, 8, 8, 4, 2, 3>);
   consider(8, 16, 1, {28.f}, 293.f, blocks<T, EPI, 8, 16, 2, 4, 3>);
+  if constexpr (by_strips<T, EPI>()) {
+    consider(8, 8, 2, {17.f, 31.f}, 0.f, strips<T, EPI, 8, 2, 4, 4, 8>, true);
+    consider(8, 16, 2, {27.f, 53.f}, 0.f, strips<T, EPI, 8, 4, 4, 4, 4>, true);
+  }
   return best(p, best_y, N, st);
 }
 

@@ -60,3 +60,20 @@ def test_two_blocks_a_cu(serve, ff, rows):  # noqa: F811
     """gate and up in 257 to 512 blocks of 64 x 128 (three stages), rows of 16 bytes and not."""
     cfg = N.config([(N.latent(heads=4, dim=32, rot=16, vdim=32, rank=64), N.dense(ff=ff))], width=96)
     check(serve, cfg, N.weights(cfg, 11), "bfloat16", [[rows]])
+
+
+@pytest.mark.parametrize("ff,width", [(13000, 64), (13000, 96), (13000, 224), (9000, 160), (9000, 288),
+                                      (9000, 320), (9000, 448)])
+def test_strips(serve, ff, width):  # noqa: F811
+    """gate and up by strips, 385 to 512 blocks of 128 x 256 or 513 to 768 of 128 x 128: one to seven stages,
+    a last k-step alone, rows and columns that end inside a block."""
+    cfg = N.config([(N.latent(heads=4, dim=32, rot=16, vdim=32, rank=64), N.dense(ff=ff))], width=width)
+    check(serve, cfg, N.weights(cfg, 13), "bfloat16", [[500]])
+
+
+@pytest.mark.parametrize("ff,shared,width", [(7000, 1100, 160), (1056, 2080, 1056)])
+def test_expert_strips(serve, ff, shared, width):  # noqa: F811
+    """Tiles of 128 rows that end early; the routed and the shared experts' K at their own lengths."""
+    cfg = T.config([(T.attn(heads=8, kv_heads=2, dim=32, vdim=32, rot=16), T.moe(experts=2, top=1, ff=ff, shared=shared))],
+                   width=width)
+    check(serve, cfg, T.clear_choices(T.weights(cfg, 17)), "bfloat16", [[500]])
