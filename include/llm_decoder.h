@@ -560,6 +560,13 @@ typedef struct llm_engine_entry {
  * when nothing is wanted).  A failed step leaves the sequences' lengths as
  * they were. */
 int llm_engine_step(llm_engine* e, const llm_engine_entry* entries, int n, float* logits);
+
+/* Pinned memory for the logits of steps, which reach it by one copy over the bus:
+ * `bytes` of it, or NULL (no engine lives, 64 MiB are lent or held, or there is none)
+ * for the caller to take memory of its own.  Given back from any thread, also after
+ * the engine's end, when nothing reads it any more. */
+void* llm_host_rows_take(size_t bytes);
+void llm_host_rows_give(void* at);
 /* The residual stream after every layer run of each following step of at most
  * max_step_tokens tokens: tap, host [layer runs][tokens][width]; NULL: off. */
 int llm_engine_set_tap(llm_engine* e, float* tap);

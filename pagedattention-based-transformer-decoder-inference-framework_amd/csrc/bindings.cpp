@@ -117,8 +117,21 @@ py::object engine_step(uintptr_t step, uintptr_t engine, py::handle entries, int
     out[i].want = pool.data() + at[2 * i + 1];
     out[i].n_want = (int)(at[2 * i + 2] - at[2 * i + 1]);
   }
-  py::array_t<float> logits({rows, (py::ssize_t)vocab});
-  float* to = rows ? logits.mutable_data() : nullptr;
+  // From 64 KiB on rows arrive in pinned memory that the array holds, while there is some
+  const size_t bytes = (size_t)rows * (size_t)vocab * sizeof(float);
+  float* to = nullptr;
+  if (bytes >= 65536) {
+    py::gil_scoped_release nogil;
+    to = static_cast<float*>(llm_host_rows_take(bytes));
+  }
+  py::array_t<float> logits = [&] {
+    if (!to) return py::array_t<float>({rows, (py::ssize_t)vocab});
+    std::unique_ptr<float, void (*)(void*)> own(to, llm_host_rows_give);
+    py::capsule base(to, llm_host_rows_give);
+    own.release();
+    return py::array_t<float>({rows, (py::ssize_t)vocab}, to, base);
+  }();
+  if (!to && rows) to = logits.mutable_data();
   int rc;
   {
     py::gil_scoped_release nogil;

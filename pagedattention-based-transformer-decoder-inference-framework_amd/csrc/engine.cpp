@@ -12,6 +12,7 @@
 
 #include "common.hpp"
 #include "dev_buf.hpp"
+#include "host_rows.hpp"
 #include "model.hpp"
 #include "row_ops.hpp"
 
@@ -120,9 +121,13 @@ struct RowCopy {
     if (!ring || !pageable(host)) {
       for (size_t r = 0, n; r < rows.size(); r += n) {
         for (n = 1; r + n < rows.size() && rows[r + n] == rows[r] + n;) ++n;
-        LLM_HIP_RET(hipMemcpyAsync(host + rows[r] * width, src + r * width, n * row_bytes,
-                                   hipMemcpyDeviceToHost, st));
+        if (const hipError_t e = hipMemcpyAsync(host + rows[r] * width, src + r * width, n * row_bytes,
+                                                hipMemcpyDeviceToHost, st)) {
+          (void)finish(LLM_OK, st);
+          LLM_HIP_RET(e);
+        }
       }
+      if (!graph && ring && hipEventRecord(arrived[0], st) == hipSuccess) (void)hipEventSynchronize(arrived[0]);
       return finish(LLM_OK, st);
     }
     const size_t pieces = (total + kPiece - 1) / kPiece;
@@ -182,6 +187,7 @@ struct llm_engine {
   DevBuf<int32_t> draw;   // [rows] draw counters
   size_t rows_cap = 0;
   RowCopy out;
+  bool counted = false;  // among the engines that host rows are kept for
 
   std::deque<std::unique_ptr<Request>> waiting;
   std::vector<std::unique_ptr<Request>> running;
@@ -193,6 +199,7 @@ struct llm_engine {
     if (stream) (void)hipStreamSynchronize(stream);
     model.reset();
     if (stream) (void)hipStreamDestroy(stream);
+    if (counted) host_rows_engine_ends();
   }
   int ensure_logits(size_t rows) {
     if (rows <= rows_cap) return LLM_OK;
@@ -420,6 +427,8 @@ extern "C" int llm_engine_create(const char* model_dir, const llm_engine_config*
   LLM_HIP_RET(hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking));
   RET_IF(e->ensure_logits((size_t)std::max(16, cfg->max_seqs)));
   e->out.init();
+  host_rows_engine_begins((size_t)cfg->max_seqs * e->model->vocab() * sizeof(float));
+  e->counted = true;
   *out = e.release();
   return LLM_OK;
 }

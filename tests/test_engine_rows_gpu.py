@@ -133,3 +133,38 @@ def test_without_the_extension_module(eng, tmp_path, monkeypatch):
     with engine.Engine(tmp_path / "m", dtype="float32", max_tokens=256) as e:
         assert not e._native_step
         np.testing.assert_array_equal(step(e), want)
+
+
+def test_returned_rows_stay(gpu, tmp_path):
+    """Arrays of one step stay as they are through the next ones, past the 64 MiB that are pinned
+    at most, and past the engine; from several threads at once."""
+    import threading
+    import engine
+    cfg = T.config([(T.attn(), None)], vocab=5003)
+    folder = T.save(tmp_path, cfg, T.weights(cfg, 3))
+    held, lock = [], threading.Lock()
+
+    def serve(seed):
+        rng = np.random.default_rng(seed)
+        with engine.Engine(folder, dtype="float32", max_seqs=2, max_tokens=512) as e:
+            for n in [3, 4] + [200] * 12:  # 60,036 and 80,048 bytes; 4.0 MB
+                s = e.open_seq()
+                toks = rng.integers(0, e.vocab, n)
+                out = e.step([(s, toks, list(range(n)))])
+                e.close_seq(s)
+                plain = np.empty_like(out)
+                s = e.open_seq()
+                step(e, [(s, toks, list(range(n)))], plain.ctypes.data)
+                e.close_seq(s)
+                with lock:
+                    held.append((out, plain))
+
+    threads = [threading.Thread(target=serve, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(held) == 28
+    for out, plain in held:
+        assert out.flags.writeable and out.flags.c_contiguous
+        np.testing.assert_array_equal(out, plain)
