@@ -20,11 +20,15 @@
 // A small top_k leaves few tokens that can matter, and these are ranked one against
 // the other (pick_few).  Else they are found ten bits at a time from histograms in
 // LDS: three passes over the registers for each.  64 rows of 50,257, top_k 40 and top_p
-// 0.9: 35 us by histograms, now 21 (top_k 50 alone 31 and 20, top_p 0.95 alone 35, neither
+// 0.9: 35 us by histograms, now 19.7 (top_k 50 alone 31 and 19, top_p 0.95 alone 34, neither
 // 15).  Bound by the vector instructions over a row's registers, one row being one
-// workgroup: the softmax, then the passes.  Masses are added as whole
+// workgroup: of 37,000 clocks the exponentials take 11,600, the temperature 3,600, the loads
+// 5,200, the choice of the few 9,500, cells and draw 6,400.  A row over several workgroups would need
+// its maximum and its sum from all of them, in the present order: two launches more, 13 us by
+// the same count, and memory that the entry point does not have.  Masses are added as whole
 // multiples of 2^-50, so their sums are exact to 2^-34 and do not depend on the order
 // of the atomics.
+#include <type_traits>
 #include <utility>
 
 #include "common.hpp"
@@ -63,16 +67,48 @@ struct SampleArgs {
   int out2_stride;
 };
 
+// Of lanes l, l ^ 32, l ^ 16, .. l ^ 1, in that order: exchanges between registers (behind lane ^ 8
+// lanes l and l ^ 8 hold the same, so that a rotation by 4 is an exchange too).
+template <int CTRL>
+__device__ __forceinline__ int mov_lanes(int x) {
+  return __builtin_amdgcn_mov_dpp(x, CTRL, 0xF, 0xF, true);
+}
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  static_assert(sizeof(T) == 4);
+  const auto as_int = [](T x) { return __builtin_bit_cast(int, x); };
+  const auto as_t = [](int x) { return __builtin_bit_cast(T, x); };
+  const LanePair p = with_lane32(__builtin_bit_cast(float, v));
+  v = op(__builtin_bit_cast(T, p.a), __builtin_bit_cast(T, p.b));
+  const LanePair q = with_lane16(__builtin_bit_cast(float, v));
+  v = op(__builtin_bit_cast(T, q.a), __builtin_bit_cast(T, q.b));
+  v = op(v, as_t(mov_lanes<0x128>(as_int(v))));  // row_ror 8, 4
+  v = op(v, as_t(mov_lanes<0x124>(as_int(v))));
+  v = op(v, as_t(mov_lanes<0x4E>(as_int(v))));   // quad_perm [2,3,0,1], [1,0,3,2]
+  return op(v, as_t(mov_lanes<0xB1>(as_int(v))));
+}
+
 template <typename T, typename Op>
 __device__ __forceinline__ T block_reduce(T v, T* sh, Op op) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
+  v = wave_reduce(v, op);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
   __syncthreads();
   T t = sh[0];
   for (int i = 1; i < kSampleThreads / 64; ++i) t = op(t, sh[i]);  // fixed order
   return t;
+}
+
+// expf of x <= 0, the same bits for every x (compared over all of them, infinity and NaN too): 2^(x
+// log2 e) with the product in two parts.  Without expf's test for large x 64 rows of 50,257 take 0.4 us
+// less.
+__device__ __forceinline__ float exp_below(float x) {
+#pragma clang fp contract(off)
+  const float t = x * kLog2e;
+  const float lo = fmaf(x, 0x1.4ae0bep-26f, fmaf(x, kLog2e, -t));
+  const float r = rintf(t);
+  const float e = ldexpf(__builtin_amdgcn_exp2f((t - r) + lo), (int)r);
+  return x < -103.27893f ? 0.f : e;
 }
 
 __device__ __forceinline__ void put_token(const SampleArgs& a, int r, int tok) {
@@ -159,15 +195,35 @@ struct Few {
   int count;
   uint32_t rank_least, mass_least;
 };
+// What a value counts: those above it and beside it, and their masses.
+struct Above {
+  int above = 0, same = 0;
+  unsigned long long mass_above = 0, mass_same = 0;
+
+  template <int CTRL>
+  __device__ __forceinline__ void add_lane() {
+    above += mov_lanes<CTRL>(above);
+    same += mov_lanes<CTRL>(same);
+    mass_above += lane<CTRL>(mass_above);
+    mass_same += lane<CTRL>(mass_same);
+  }
+  template <int CTRL>
+  static __device__ __forceinline__ unsigned long long lane(unsigned long long x) {
+    return (unsigned long long)(uint32_t)mov_lanes<CTRL>((int)(x >> 32)) << 32 | (uint32_t)mov_lanes<CTRL>((int)x);
+  }
+};
+// v times `inv` are the probabilities; seg receives a thread's largest v of each segment.
 template <int NS>
-__device__ __forceinline__ bool pick_few(const float (&v)[NS][4], int top_k, unsigned long long want, Few& few,
-                                         uint32_t* least) {
+__device__ __forceinline__ bool pick_few(const float (&v)[NS][4], float inv, int top_k, unsigned long long want,
+                                         Few& few, float (&seg)[NS], uint32_t* least) {
   const int t = threadIdx.x;
   float top = 0.f;
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) top = fmaxf(top, v[s][j]);
+  for (int s = 0; s < NS; ++s) {
+    seg[s] = fmaxf(fmaxf(v[s][0], v[s][1]), fmaxf(v[s][2], v[s][3]));
+    top = fmaxf(top, seg[s]);
+  }
+  top *= inv;
   top = fmaxf(top, mov_dpp<0xB1>(top));
   top = fmaxf(top, mov_dpp<0x4E>(top));
   top = fmaxf(top, mov_dpp<0x141>(top));
@@ -179,62 +235,70 @@ __device__ __forceinline__ bool pick_few(const float (&v)[NS][4], int top_k, uns
   }
   __syncthreads();
   {  // eight threads a group, each against sixteen others
-    const int g = t / 8, h0 = t % 8 * (kGroups / 8);
-    int above = 0;
+    const int h0 = t % 8 * (kGroups / 8);
+    int above = 0, from = 0;
 #pragma unroll
     for (int k = 0; k < kGroups / 8; k += 4) {
       const f32x4 o = *reinterpret_cast<const f32x4*>(&few.most[h0 + k]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) above += o[e] > top || (o[e] == top && h0 + k + e < g);
+      for (int e = 0; e < 4; ++e) {
+        above += o[e] > top;
+        from += o[e] >= top;
+      }
     }
-    above += __builtin_amdgcn_mov_dpp(above, 0xB1, 0xF, 0xF, true);
-    above += __builtin_amdgcn_mov_dpp(above, 0x4E, 0xF, 0xF, true);
-    above += __builtin_amdgcn_mov_dpp(above, 0x141, 0xF, 0xF, true);
-    if (t % 8 == 0 && above == top_k - 1) few.floor = top;
+    above += mov_lanes<0xB1>(above);
+    from += mov_lanes<0xB1>(from);
+    above += mov_lanes<0x4E>(above);
+    from += mov_lanes<0x4E>(from);
+    above += mov_lanes<0x141>(above);
+    from += mov_lanes<0x141>(from);
+    if (t % 8 == 0 && above < top_k && from >= top_k) few.floor = top;  // (equal ones write the same)
   }
   __syncthreads();
   const float floor = few.floor;
   if (!(floor > 0.f)) return false;
-  if (top >= floor) {
+  // (v times inv reaches the floor only from `low` on, whose product is 2^-22 below it; products
+  // with few bits round further)
+  const float low = floor < 0x1p-100f ? 0.f : floor / inv * (1.f - 0x1p-22f);
 #pragma unroll
-    for (int s = 0; s < NS; ++s)
+  for (int s = 0; s < NS; ++s) {
+    if (!__ballot(seg[s] >= low)) continue;  // most waves have none in most segments
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (v[s][j] >= floor) {
-          const int at = atomicAdd(&few.count, 1);
-          if (at < kFew) {
-            few.bits[at] = __float_as_uint(v[s][j]);
-            few.mass[at] = mass_of(__float_as_uint(v[s][j]));
-          }
-        }
+    for (int j = 0; j < 4; ++j) {
+      const float p = v[s][j] * inv;
+      if (p >= floor) {
+        const int at = atomicAdd(&few.count, 1);
+        if (at < kFew) few.bits[at] = __float_as_uint(p);
+      }
+    }
   }
   __syncthreads();
   const int n = few.count;
   if (n > kFew) return false;
-  // four threads a value
-  const uint32_t own = t / 4 < n ? few.bits[t / 4] : 0u;
-  int above = 0, same = 0;
-  unsigned long long mass_above = 0, mass_same = 0;
+  if (t < n) few.mass[t] = mass_of(few.bits[t]);
+  __syncthreads();
+  // as many threads a value as n leaves, four at least
+  const int per = n <= 64 ? 16 : n <= 128 ? 8 : 4, at = t / per;
+  const uint32_t own = at < n ? few.bits[at] : 0u;
+  Above a;
   if (own)
-    for (int i = t % 4; i < n; i += 4) {
+#pragma unroll 4
+    for (int i = t % per; i < n; i += per) {
       const uint32_t o = few.bits[i];
       const unsigned long long m = few.mass[i];
-      above += o > own;
-      same += o == own;
-      mass_above += o > own ? m : 0;
-      mass_same += o == own ? m : 0;
+      a.above += o > own;
+      a.same += o == own;
+      a.mass_above += o > own ? m : 0;
+      a.mass_same += o == own ? m : 0;
     }
-#pragma unroll
-  for (int off = 1; off < 4; off <<= 1) {
-    above += __shfl_xor(above, off, 64);
-    same += __shfl_xor(same, off, 64);
-    mass_above += __shfl_xor(mass_above, off, 64);
-    mass_same += __shfl_xor(mass_same, off, 64);
-  }
-  if (own && above < top_k && above + same >= top_k) few.rank_least = own;
+  a.add_lane<0xB1>();
+  a.add_lane<0x4E>();
+  if (per >= 8) a.add_lane<0x141>();  // row_half_mirror, row_mirror
+  if (per >= 16) a.add_lane<0x140>();
+  if (own && a.above < top_k && a.above + a.same >= top_k) few.rank_least = own;
   // (a value below the top_k-th counts for nothing: what is above it holds the mass already,
   // or nothing more is dropped)
-  if (own && mass_above < want && mass_above + mass_same >= want) few.mass_least = own;
+  if (own && a.mass_above < want && a.mass_above + a.mass_same >= want) few.mass_least = own;
   __syncthreads();
   *least = max(few.rank_least, few.mass_least);
   return true;
@@ -278,6 +342,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   const float* lg = a.logits + (size_t)r * a.V;
   const auto token = [&](int s, int j) { return s * kSampleSeg + w * 256 + j * 64 + lane; };
   const auto done = [&](int tok) { put_token(a, r, tok); };
+  const float u = sample_uniform(a.seed, a.row0 + r, a.counter ? a.counter[r] : a.counter0);
   float v[NS][4];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
@@ -311,7 +376,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   for (int s = 0; s < NS; ++s) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      v[s][j] = expf(v[s][j] - m);
+      v[s][j] = exp_below(v[s][j] - m);
       sloc += v[s][j];
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -322,10 +387,6 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
     return;
   }
   const float inv = 1.0f / (sum + 1e-6f);
-#pragma unroll
-  for (int s = 0; s < NS; ++s)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[s][j] = v[s][j] * inv;
 
   // top-k: the largest pattern that top_k probabilities reach (fewer that are not
   // zero: all stay).  top-p: the largest pattern whose probabilities and those above
@@ -339,27 +400,42 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
   // too low a value or none.  40 rows of 1,057 tokens, top_k 50: 9.9 us, 11.3 with the attempt;
   // 64 of 1,600: 10.7 and 13.8)
   const int groups = min(kGroups, a.V / 256 * 8);
+  float seg[NS];
   const bool few_found = a.top_k > 0 && a.top_k < a.V && a.top_k <= min(kFewK, groups / 4 * 3) &&
-                         pick_few(v, a.top_k, want, few, &least);
-  if (!few_found && a.top_k > 0 && a.top_k < a.V)
-    least = find_pattern<NS>(v, 0u, (uint32_t)a.top_k, ranks, rank_part, &rank_found,
-                             [](uint32_t) { return 1u; });
-  if (!few_found && a.top_p < 1.0f)
-    least = max(least, find_pattern<NS>(v, least, want, masses, mass_part, &mass_found,
-                                        [](uint32_t bits) { return mass_of(bits); }));
-
-  // kept mass in token order: per cell, then over the cells
+                         pick_few(v, inv, a.top_k, want, few, seg, &least);
+  if (!few_found) {
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    float part = 0.f;
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[s][j] = __float_as_uint(v[s][j]) >= least ? v[s][j] : 0.f;
-      part += v[s][j];
-    }
-    if (__ballot(part > 0.f)) part = group_sum<64>(part);
-    if (lane == 0) cells[s * kSampleWaves + w] = part;
+      for (int j = 0; j < 4; ++j) v[s][j] = v[s][j] * inv;
+    if (a.top_k > 0 && a.top_k < a.V)
+      least = find_pattern<NS>(v, 0u, (uint32_t)a.top_k, ranks, rank_part, &rank_found,
+                               [](uint32_t) { return 1u; });
+    if (a.top_p < 1.0f)
+      least = max(least, find_pattern<NS>(v, least, want, masses, mass_part, &mass_found,
+                                          [](uint32_t bits) { return mass_of(bits); }));
   }
+
+  // kept mass in token order: per cell, then over the cells.  Of the few only the segments that
+  // hold some are walked.
+  const auto keep = [&](auto by_seg) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      float part = 0.f;
+      if (!decltype(by_seg)::value || __ballot(__float_as_uint(seg[s] * inv) >= least)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float p = decltype(by_seg)::value ? v[s][j] * inv : v[s][j];
+          v[s][j] = __float_as_uint(p) >= least ? p : 0.f;
+          part += v[s][j];
+        }
+        if (__ballot(part > 0.f)) part = group_sum<64>(part);
+      }
+      if (lane == 0) cells[s * kSampleWaves + w] = part;
+    }
+  };
+  if (few_found) keep(std::true_type());
+  else keep(std::false_type());
   __syncthreads();
   constexpr int CELLS = NS * kSampleWaves, PER = (CELLS + 63) / 64;
   if (w == 0) {
@@ -376,8 +452,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
       if (lane >= off) incl += o;
     }
     const float Z = __shfl(incl, 63, 64);
-    const int ctr = a.counter ? a.counter[r] : a.counter0;
-    const float target = sample_uniform(a.seed, a.row0 + r, ctr) * Z;
+    const float target = u * Z;
     // the first cell whose end lies past the target, else (rounding at the top of the
     // range) the last one that holds any mass
     float lo = __shfl_up(incl, 1, 64);
@@ -395,12 +470,8 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
       }
       lo += c[i];
     }
-    int first = hit;
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-      first = min(first, __shfl_xor(first, off, 64));
-      last = max(last, __shfl_xor(last, off, 64));
-    }
+    const int first = wave_reduce(hit, [](int x, int y) { return min(x, y); });
+    last = wave_reduce(last, [](int x, int y) { return max(x, y); });
     if (first != 0x7fffffff) {
       if (hit == first) {
         cell = first;
@@ -418,32 +489,39 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(SampleArgs 
     return;
   }
   if (w != at % kSampleWaves) return;
+  // the wave's four of that segment, by one copy of what follows: with one for every segment the
+  // kernel of 13 was 58 KB, now 42
+  const int which = at / kSampleWaves;
+  float x[4] = {};
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    if (s == which) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = v[s][j];
+    }
   const float target = cell_left;
-  float lo = 0.f;
-  int pick = 0x7fffffff, last = -1;
+  float lo = 0.f, incl[4];
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    if (s != at / kSampleWaves) continue;
+  for (int j = 0; j < 4; ++j) {
+    incl[j] = x[j];
+    if (!__ballot(x[j] > 0.f)) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float incl = v[s][j];
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const float o = __shfl_up(incl, off, 64);
-        if (lane >= off) incl += o;
-      }
-      if (v[s][j] > 0.f) {
-        last = token(s, j);
-        if (target < lo + incl) pick = min(pick, token(s, j));
-      }
-      lo += __shfl(incl, 63, 64);
+    for (int off = 1; off < 64; off <<= 1) {
+      const float o = __shfl_up(incl[j], off, 64);
+      if (lane >= off) incl[j] += o;
     }
   }
+  int pick = 0x7fffffff, last = -1;
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
-    pick = min(pick, __shfl_xor(pick, off, 64));
-    last = max(last, __shfl_xor(last, off, 64));
+  for (int j = 0; j < 4; ++j) {
+    if (x[j] > 0.f) {
+      last = token(which, j);
+      if (target < lo + incl[j]) pick = min(pick, token(which, j));
+    }
+    lo += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, incl[j]), 63));
   }
+  pick = wave_reduce(pick, [](int p, int q) { return min(p, q); });
+  last = wave_reduce(last, [](int p, int q) { return max(p, q); });
   if (lane == 0) done(pick == 0x7fffffff ? last : pick);
 }
 

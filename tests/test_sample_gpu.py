@@ -82,10 +82,12 @@ def test_top_p_below_any_probability(gpu, p, k):
 
 @pytest.mark.parametrize("k", [2, 5, 63, 64, 65])
 @pytest.mark.parametrize("p", [0.5, 0.97, 1.0])
-@pytest.mark.parametrize("shape", ["spread", "one_group", "few_groups", "many_ties", "many_near", "flat"])
+@pytest.mark.parametrize("shape", ["spread", "one_group", "few_groups", "many_ties", "many_near", "flat",
+                                   "some_near", "tiny"])
 def test_few_tokens_left(gpu, shape, k, p):
     """A small top_k: its tokens spread out, in one group of eight threads, in fewer groups
-    than top_k; more equal or near ones than are ranked one against the other."""
+    than top_k; 70 to 256 equal or near ones, and more than are ranked one against the other;
+    all but one below the least normal number."""
     from oracle.oracle import sample_rows
     V = 12500
     rng = np.random.default_rng(k)
@@ -100,6 +102,10 @@ def test_few_tokens_left(gpu, shape, k, p):
         logits[:, rng.permutation(V)[:900]] = 3.5
     elif shape == "many_near":
         logits[:, rng.permutation(V)[:2000]] = 3.0 + 1e-3 * rng.standard_normal((3, 2000)).astype(np.float32)
+    elif shape == "some_near":
+        logits[:, rng.permutation(V)[:190]] = 5.0 + 1e-3 * rng.standard_normal((3, 190)).astype(np.float32)
+    elif shape == "tiny":
+        logits[:, 777] = 66.0
     elif shape == "flat":
         logits[:] = 0.0
     for counter in range(6):
