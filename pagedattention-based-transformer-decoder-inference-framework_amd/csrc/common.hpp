@@ -159,13 +159,6 @@ __device__ __forceinline__ int wave_scan_max(int x) {
 }
 
 __device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off, 64));
-  return x;
-}
-
-// wave_max through DPP moves inside the 16-lane rows
-__device__ __forceinline__ float wave_max_dpp(float x) {
   x = fmaxf(x, mov_dpp<0xB1>(x));
   x = fmaxf(x, mov_dpp<0x4E>(x));
   x = fmaxf(x, mov_dpp<0x141>(x));
@@ -173,10 +166,29 @@ __device__ __forceinline__ float wave_max_dpp(float x) {
   return rows_max(x);
 }
 
+// op over lanes l, l ^ 32, l ^ 16, .. l ^ 1, in that order: exchanges between registers, no trips through
+// LDS (behind lane ^ 8 lanes l and l ^ 8 hold the same, so that a rotation by 4 is an exchange
+// too).
+template <int CTRL>
+__device__ __forceinline__ int mov_lanes(int x) {
+  return __builtin_amdgcn_mov_dpp(x, CTRL, 0xF, 0xF, true);
+}
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce(T v, Op op) {
+  static_assert(sizeof(T) == 4);
+  const auto as_int = [](T x) { return __builtin_bit_cast(int, x); };
+  const auto as_t = [](int x) { return __builtin_bit_cast(T, x); };
+  const LanePair p = with_lane32(__builtin_bit_cast(float, v));
+  v = op(__builtin_bit_cast(T, p.a), __builtin_bit_cast(T, p.b));
+  const LanePair q = with_lane16(__builtin_bit_cast(float, v));
+  v = op(__builtin_bit_cast(T, q.a), __builtin_bit_cast(T, q.b));
+  v = op(v, as_t(mov_lanes<0x128>(as_int(v))));  // row_ror 8, 4
+  v = op(v, as_t(mov_lanes<0x124>(as_int(v))));
+  v = op(v, as_t(mov_lanes<0x4E>(as_int(v))));  // quad_perm [2,3,0,1], [1,0,3,2]
+  return op(v, as_t(mov_lanes<0xB1>(as_int(v))));
+}
 __device__ __forceinline__ float wave_sum(float x) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off, 64);
-  return x;
+  return wave_reduce(x, [](float a, float b) { return a + b; });
 }
 
 __device__ __forceinline__ int wave_id_uniform() {

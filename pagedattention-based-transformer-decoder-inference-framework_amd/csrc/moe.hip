@@ -33,7 +33,7 @@ __device__ __forceinline__ void choose(const RouteArgs& a, int m, int32_t* choic
     float best = key[0];
 #pragma unroll
     for (int j = 1; j < LE; ++j) best = fmaxf(best, key[j]);
-    best = wave_max_dpp(best);
+    best = wave_max(best);
     // the lowest expert that has it (scores that are not numbers match nothing:
     // any valid expert then)
     int be = k;

@@ -224,7 +224,7 @@ __global__ __launch_bounds__(1024) void pa_merge_row_kernel(PaMergeRowArgs a) {
     }
   }
   if (!a.q) return;
-  am = ln_wave_max(am);  // DPP (wave_max shuffles through LDS)
+  am = ln_wave_max(am);
   if (lane == 0) sh[w] = am;
   __syncthreads();
   am = sh[0];

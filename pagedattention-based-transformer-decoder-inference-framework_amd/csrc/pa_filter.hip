@@ -24,8 +24,8 @@
 #include "pa_decode.hpp"
 
 #include <algorithm>
-
 #include <string>
+#include <type_traits>
 
 namespace llm {
 
@@ -86,7 +86,7 @@ __device__ __forceinline__ float kv_elem(const u32x4& r, int e) {
 
 // Block-wide reduction of one value per thread (all threads get the result).
 template <bool MAX>
-__device__ float block_reduce(float x, float* sh) {
+__device__ __forceinline__ float block_reduce(float x, float* sh) {
   x = MAX ? wave_max(x) : wave_sum(x);
   const int w = threadIdx.x >> 6;
   __syncthreads();
@@ -117,38 +117,62 @@ struct FilterCut {
 
 __device__ __forceinline__ uint64_t filter_mass(float p) { return p > 0.f ? (uint64_t)(p * kMassUnit) : 0; }
 
+// x of the lane that a row shift or a broadcast of a row's last lane names; 0 where there is none
+// or in rows outside ROWS
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t lane_from(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xF, true);
+}
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint64_t lane_from(uint64_t x) {
+  return (uint64_t)lane_from<CTRL, ROWS>((uint32_t)(x >> 32)) << 32 | lane_from<CTRL, ROWS>((uint32_t)x);
+}
+// sums over the lanes up to one's own, in rows of 16 lanes, then over the wave
+template <typename T>
+__device__ __forceinline__ T row_scan(T x) {
+  x += lane_from<0x111>(x);
+  x += lane_from<0x112>(x);
+  x += lane_from<0x114>(x);
+  x += lane_from<0x118>(x);
+  return x;
+}
+template <typename T>
+__device__ __forceinline__ T wave_scan(T x) {
+  x = row_scan(x);
+  x += lane_from<0x142, 0xA>(x);  // row_bcast 15
+  x += lane_from<0x143, 0xC>(x);  // row_bcast 31
+  return x;
+}
+__device__ __forceinline__ uint32_t lane_value(uint32_t x, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, l);
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t x, int l) {
+  return (uint64_t)lane_value((uint32_t)(x >> 32), l) << 32 | lane_value((uint32_t)x, l);
+}
+
 // The digit, from the top, at which `need` entries (0: any number) or a mass of `limit`
-// (0: any) are reached; `from` holds what lies above the histogram.
-__device__ void filter_digit(const FilterHist& hist, uint32_t need, uint64_t limit,
-                             const FilterCut& from, FilterCut* out, uint64_t* sh_mass,
-                             uint32_t* sh_count) {
+// (0: any) are reached; `from` holds what lies above the histogram.  Sums over lanes by register
+// moves, those over the waves before one's own too (6,400 clocks a digit by
+// shuffles and a walk over the waves, now 4,200).
+__device__ __forceinline__ void filter_digit(const FilterHist& hist, uint32_t need, uint64_t limit,
+                                             const FilterCut& from, FilterCut* out, uint64_t* sh_mass,
+                                             uint32_t* sh_count) {
+  static_assert(kFilterThreads / 64 <= 16, "a row of lanes sums the waves");
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int top = kDigits - 1 - 2 * tid;
   const uint32_t c0 = hist.count[top], c1 = hist.count[top - 1];
   const uint64_t m0 = hist.mass[top], m1 = hist.mass[top - 1];
-  uint32_t c = c0 + c1;
-  uint64_t m = m0 + m1;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const uint32_t cu = __shfl_up(c, off, 64);
-    const uint64_t mu = __shfl_up((unsigned long long)m, off, 64);
-    if (lane >= off) {
-      c += cu;
-      m += mu;
-    }
-  }
+  uint32_t c = wave_scan(c0 + c1);
+  uint64_t m = wave_scan(m0 + m1);
   if (lane == 63) {
     sh_count[w] = c;
     sh_mass[w] = m;
   }
   if (tid == 0) out->digit = -1;
   __syncthreads();
-  c += from.count - c0 - c1;
-  m += from.mass - m0 - m1;
-  for (int i = 0; i < w; ++i) {
-    c += sh_count[i];
-    m += sh_mass[i];
-  }
+  const bool before = lane < w;  // (w < 16)
+  c += lane_value(row_scan(before ? sh_count[lane] : 0u), 15) + from.count - c0 - c1;
+  m += lane_value(row_scan(before ? sh_mass[lane] : (uint64_t)0), 15) + from.mass - m0 - m1;
   const auto reached = [&](uint32_t n, uint64_t x) { return (need && n >= need) || (limit && x >= limit); };
 #pragma unroll
   for (int k = 0; k < 2; ++k) {
@@ -176,30 +200,180 @@ struct FilterRank {
   uint32_t count[kRankParts][kRankRow];
 };
 
+// A small top_k: the row's threads form 128 groups of eight; the top_k-th largest of the groups'
+// largest entries has top_k entries from it on, so that whatever stays is among those.  Where
+// they are few they are ranked one against the other, in place of the histograms (16 rows x 12
+// heads of 2048, top 64 and 0.9: 8.8 us of 30, now 3.8).  The same whole numbers.
+constexpr int kFewK = 64, kFew = 256, kFewGroups = kFilterThreads / 8;
+struct FilterFew {
+  uint64_t key[kFew], mass[kFew];  // (probability bits, index); mass
+  float most[kFewGroups];
+  uint32_t index[kFew];            // of what stays; ~0: it does not
+  uint64_t cut;
+  float floor;
+  uint32_t count;
+};
+template <int CTRL>
+__device__ __forceinline__ uint32_t lane_sum(uint32_t x) {
+  return x + (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ uint64_t lane_sum(uint64_t x) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)x, CTRL, 0xF, 0xF, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(x >> 32), CTRL, 0xF, 0xF, true);
+  return x + ((uint64_t)hi << 32 | lo);
+}
+// over 4, 8 or 16 neighbouring lanes: exchanges inside quads, half rows, rows
+template <typename T>
+__device__ __forceinline__ T lanes_sum(T x, int per) {
+  x = lane_sum<0xB1>(x);
+  x = lane_sum<0x4E>(x);
+  if (per >= 8) x = lane_sum<0x141>(x);
+  if (per >= 16) x = lane_sum<0x140>(x);
+  return x;
+}
+// sc[0 .. Tb): probabilities, `most` the largest of this thread's (t = tid, tid + kFilterThreads,
+// ..).  Lists what stays in the order of its index and gives the least of it; 0: too many, or
+// groups without an entry; nothing is found then.
+__device__ __forceinline__ int filter_few(const float* sc, int Tb, float most, uint32_t k, uint64_t limit, FilterFew& few,
+                          uint64_t* list, uint32_t* cut_bits, int* cut_index) {
+  const int tid = threadIdx.x;
+  most = fmaxf(most, mov_dpp<0xB1>(most));
+  most = fmaxf(most, mov_dpp<0x4E>(most));
+  most = fmaxf(most, mov_dpp<0x141>(most));
+  if (tid % 8 == 0) few.most[tid / 8] = most;
+  if (tid == 0) {
+    few.floor = 0.f;
+    few.count = 0;
+  }
+  __syncthreads();
+  {  // eight threads a group, each against sixteen others
+    const int h0 = tid % 8 * (kFewGroups / 8);
+    uint32_t above = 0, from = 0;
+#pragma unroll
+    for (int i = 0; i < kFewGroups / 8; i += 4) {
+      const f32x4 o = *reinterpret_cast<const f32x4*>(&few.most[h0 + i]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        above += o[e] > most;
+        from += o[e] >= most;
+      }
+    }
+    above = lanes_sum(above, 8);
+    from = lanes_sum(from, 8);
+    if (tid % 8 == 0 && above < k && from >= k) few.floor = most;  // (equal ones write the same)
+  }
+  __syncthreads();
+  const float floor = few.floor;
+  if (!(floor > 0.f)) return 0;
+  if (most >= floor)
+    for (int t = tid; t < Tb; t += kFilterThreads) {
+      const float p = sc[t];
+      if (!(p >= floor)) continue;
+      const uint32_t at = atomicAdd(&few.count, 1u);
+      if (at < kFew) {
+        few.key[at] = (uint64_t)__float_as_uint(p) << 32 | (uint32_t)t;
+        few.mass[at] = filter_mass(p);
+      }
+    }
+  __syncthreads();
+  const uint32_t n = few.count;
+  if (n > kFew) return 0;
+  // as many threads an entry as n leaves, four at least
+  const int per = n <= 64 ? 16 : n <= 128 ? 8 : 4;
+  const uint32_t i = (uint32_t)(tid / per);
+  const uint64_t key = i < n ? few.key[i] : 0;
+  uint32_t above = 0;
+  uint64_t mass = 0;
+  if (i < n)
+#pragma unroll 4
+    for (uint32_t j = tid % per; j < n; j += per) {
+      const bool over = few.key[j] > key;
+      const uint64_t m = few.mass[j];
+      above += over;
+      mass += over ? m : 0;
+    }
+  above = lanes_sum(above, per);
+  mass = lanes_sum(mass, per);
+  const bool stays = i < n && above < k && (!limit || mass < limit);
+  if (i < n && tid % per == 0) few.index[i] = stays ? (uint32_t)key : ~0u;
+  __syncthreads();
+  uint32_t before = 0, all = 0;
+#pragma unroll 4
+  for (uint32_t j = tid % per; j < n; j += per) {
+    const uint32_t index = few.index[j];
+    all += index != ~0u;
+    before += index < (uint32_t)key;
+  }
+  all = lanes_sum(all, per);
+  before = lanes_sum(before, per);
+  if (stays && tid % per == 0) {
+    list[before] = key;
+    if (above == all - 1) few.cut = key;
+  }
+  if (tid == 0) few.count = all;
+  __syncthreads();
+  *cut_bits = (uint32_t)(few.cut >> 32);
+  *cut_index = (int)(uint32_t)few.cut;
+  return (int)few.count;
+}
+
 // One workgroup per (row, head).  The scores take one pass over K: 16-byte pieces, a
-// token's pieces in adjacent lanes, kScoreTokens tokens of a group in flight.  The entries
+// token's pieces in adjacent lanes, 8 or 16 tokens of a group in flight.  The entries
 // that stay are listed in the order of their index, and only their V rows are read, by all
 // lanes.  16 rows x 12 heads of 64, 2048 tokens, top 64: 70 us with a token a thread, a
-// sort of the row and a walk over all of it for the values, now 30.  Bound by the
+// sort of the row and a walk over all of it for the values, now 21.4: 11 of them the scores.  Bound by the
 // latency of its steps; the 192 workgroups are one a CU.
-constexpr int kScoreTokens = 8, kValueTokens = 4;
+constexpr int kValueTokens = 4;
 
-template <int KVT, bool WS>
+// x of lane l ^ OFF
+template <int OFF>
+__device__ __forceinline__ float lane_xor(float x) {
+  if constexpr (OFF == 4)
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), 4 << 10 | 31));
+  else
+    return mov_dpp<OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : 0x128>(x);  // quad_perm, row_ror 8
+}
+// Sums of x[0 .. N) over lanes c, each lane giving half of what it holds to lane c ^ OFF, then OFF / 2:
+// in the order in which a whole exchange at every step would add them.
+template <int OFF, int N>
+__device__ __forceinline__ void halve_sums(float* x, int c) {
+  static_assert(OFF <= 8);
+  if constexpr (N == 1) {
+    x[0] += lane_xor<OFF>(x[0]);
+  } else {
+    const bool up = (c & OFF) != 0;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const float keep = up ? x[i + N / 2] : x[i], give = up ? x[i] : x[i + N / 2];
+      x[i] = keep + lane_xor<OFF>(give);
+    }
+  }
+  if constexpr (OFF > 1) halve_sums<OFF / 2, (N > 1 ? N / 2 : 1)>(x, c);
+}
+
+// FORM: kShort: rows of up to kRankRow tokens, a kernel of its own that is a third of the code (which
+// a launch waits for) and of the LDS, so that a CU holds two; kLds; kWs.
+// (top 50 of 100 tokens, 12 heads: one row 11.9 us in the LDS form, 10.8 in this; 32 rows 22.3, 20.0)
+enum FilterForm { kShort, kLds, kWs };
+template <int KVT, FilterForm FORM>
 __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs a) {
+  constexpr bool WS = FORM == kWs, SHORT = FORM == kShort;
   constexpr int ES = KVT == LLM_F32 ? 4 : KVT == LLM_I8 ? 1 : 2;
   constexpr int EPL = 16 / ES;
   constexpr int kWaves = kFilterThreads / 64;
   // scores, then probabilities; the sums of the values at the end
-  __shared__ float lsc[WS ? kWaves * 256 : kFilterMaxT];
+  __shared__ float lsc[FORM != kLds ? kWaves * 256 : kFilterMaxT];
   // the histograms, then the list of what stays
-  __shared__ uint64_t llist[WS ? sizeof(FilterHist) / 8 : kFilterMaxT];
+  __shared__ uint64_t llist[SHORT ? sizeof(FilterRank) / 8 : WS ? sizeof(FilterHist) / 8 : kFilterMaxT];
   __shared__ float qs[256];
   __shared__ float sh[kWaves];
   __shared__ uint64_t sh_mass[kWaves];
   __shared__ uint32_t sh_count[kWaves];
   __shared__ FilterCut found;
-  static_assert(sizeof(FilterHist) <= sizeof(llist) && sizeof(FilterRank) <= sizeof(llist),
-                "the histograms and ranks lie in the list's memory");
+  static_assert(sizeof(FilterRank) <= sizeof(llist) && kFewK * 8 + sizeof(FilterFew) <= sizeof(llist) &&
+                    (SHORT || sizeof(FilterHist) <= sizeof(llist)),
+                "the histograms and ranks lie in the list's memory, the few behind their list");
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int bh = blockIdx.x;
   float* sc = WS ? a.ws_sc + (size_t)bh * a.Tp : lsc;
@@ -233,46 +407,67 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
     for (int e = 0; e < EPL; ++e) qv[e] = a.q[(size_t)bh * D + c * EPL + e];
     // the waves take turns of tpw tokens each, so that short rows are spread over them
     const int step = kWaves * tpw;
-    int page[kScoreTokens];
-    auto pages = [&](int t0) {
+    // N tokens of a group in flight; LPT lanes a token where that is known (0: lpt)
+    const auto scores = [&](auto n_tokens, auto lanes) {
+      constexpr int N = decltype(n_tokens)::value, LPT = decltype(lanes)::value;
+      int page[N];
+      auto pages = [&](int t0) {
 #pragma unroll
-      for (int u = 0; u < kScoreTokens; ++u) {
-        const int t = t0 + u * step + g;
-        page[u] = t < Tb ? page_of(t) : -1;
-      }
-    };
-    if (w * tpw < Tb) pages(w * tpw);
-    for (int t0 = w * tpw; t0 < Tb; t0 += kScoreTokens * step) {
-      u32x4 k[kScoreTokens];
-      bool there[kScoreTokens];
+        for (int u = 0; u < N; ++u) {
+          const int t = t0 + u * step + g;
+          page[u] = t < Tb ? page_of(t) : -1;
+        }
+      };
+      if (w * tpw < Tb) pages(w * tpw);
+      for (int t0 = w * tpw; t0 < Tb; t0 += N * step) {
+        u32x4 k[N];
+        uint32_t there = 0;
 #pragma unroll
-      for (int u = 0; u < kScoreTokens; ++u) {
-        const int t = t0 + u * step + g;
-        there[u] = page[u] >= 0;
-        k[u] = u32x4{0u, 0u, 0u, 0u};
-        if (there[u])
-          k[u] = *reinterpret_cast<const u32x4*>(a.k_pool + at(page[u], t) * ES + c * 16);
-      }
-      if (t0 + kScoreTokens * step < Tb) pages(t0 + kScoreTokens * step);
-      float dot[kScoreTokens];
+        for (int u = 0; u < N; ++u) {
+          const int t = t0 + u * step + g;
+          k[u] = u32x4{0u, 0u, 0u, 0u};
+          if (page[u] >= 0) {
+            there |= 1u << u;
+            k[u] = *reinterpret_cast<const u32x4*>(a.k_pool + at(page[u], t) * ES + c * 16);
+          }
+        }
+        if (t0 + N * step < Tb) pages(t0 + N * step);
+        float dot[N];
 #pragma unroll
-      for (int u = 0; u < kScoreTokens; ++u) {
-        dot[u] = 0.f;
-        if (t0 + u * step < Tb) {  // (the same for the wave)
+        for (int u = 0; u < N; ++u) {
+          dot[u] = 0.f;
+          if (t0 + u * step < Tb) {  // (the same for the wave)
 #pragma unroll
-          for (int e = 0; e < EPL; ++e) dot[u] = fmaf(qv[e], kv_elem<KVT>(k[u], e), dot[u]);
+            for (int e = 0; e < EPL; ++e) dot[u] = fmaf(qv[e], kv_elem<KVT>(k[u], e), dot[u]);
+          }
+        }
+        if constexpr (LPT > 0) {
+          // every exchange halves the tokens a lane holds: lane c ends with those from c N / LPT on
+          halve_sums<LPT / 2, N>(dot, c);
+#pragma unroll
+          for (int i = 0; i < max(N / LPT, 1); ++i) {
+            const int u = c * N / LPT + i, t = t0 + u * step + g;
+            if (t < Tb) sc[t] = there >> u & 1 ? dot[i] / a.temperature : -1e9f;
+          }
+        } else {
+          for (int off = lpt >> 1; off; off >>= 1)
+#pragma unroll
+            for (int u = 0; u < N; ++u)
+              if (t0 + u * step < Tb) dot[u] += __shfl_xor(dot[u], off, 64);
+#pragma unroll
+          for (int u = 0; u < N; ++u) {
+            const int t = t0 + u * step + g;
+            if (t0 + u * step < Tb && c == 0 && t < Tb) sc[t] = there >> u & 1 ? dot[u] / a.temperature : -1e9f;
+          }
         }
       }
-      for (int off = lpt >> 1; off; off >>= 1)
-#pragma unroll
-        for (int u = 0; u < kScoreTokens; ++u)
-          if (t0 + u * step < Tb) dot[u] += __shfl_xor(dot[u], off, 64);
-#pragma unroll
-      for (int u = 0; u < kScoreTokens; ++u) {
-        const int t = t0 + u * step + g;
-        if (t0 + u * step < Tb && c == 0 && t < Tb) sc[t] = there[u] ? dot[u] / a.temperature : -1e9f;
-      }
-    }
+    };
+    const std::integral_constant<int, 8> eight;
+    const std::integral_constant<int, 16> sixteen;
+    const bool turns = Tb > 8 * step;  // (12 heads of 64, 16 rows of 2048: 28,400 clocks by 8 tokens, 23,400)
+    if (!SHORT && lpt == 8 && turns) scores(sixteen, eight);
+    else if (!SHORT && lpt == 16 && turns) scores(sixteen, sixteen);
+    else scores(eight, std::integral_constant<int, 0>());
   } else {
     for (int d = tid; d < D; d += kFilterThreads) qs[d] = a.q[(size_t)bh * D + d];
     __syncthreads();
@@ -305,7 +500,12 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   }
   sum = block_reduce<false>(sum, sh);
   const float inv = 1.0f / (sum + 1e-6f);
-  for (int t = tid; t < Tb; t += kFilterThreads) sc[t] = sc[t] * inv;
+  float most = 0.f;
+  for (int t = tid; t < Tb; t += kFilterThreads) {
+    const float p = sc[t] * inv;
+    sc[t] = p;
+    most = fmaxf(most, p);
+  }
 
   // apply_topk_topp_filter (softmax_lut.cpp:233-256): rank by (prob, index)
   // descending; zero rank >= top_k and every entry whose preceding mass
@@ -315,7 +515,14 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   const bool cuts = (a.top_k > 0 || a.top_p < 1.0f) && Tb > 0;
   const uint32_t k = a.top_k > 0 ? (uint32_t)a.top_k : 0u;
   const uint64_t limit = a.top_p < 1.0f ? max((uint64_t)ceilf(a.top_p * kMassUnit), (uint64_t)1) : 0;
-  if (cuts && Tb <= kRankRow) {
+  // (rows of fewer groups than that find too low a bound or none)
+  const bool try_few = !SHORT && k && k <= kFewK && Tb > kRankRow && (int)k <= min(Tb, kFilterThreads) / 8 / 4 * 3;
+  int n_few = 0;
+  if (try_few)
+    n_few = filter_few(sc, Tb, most, k, limit, *reinterpret_cast<FilterFew*>(llist + kFewK), list, &cut_bits,
+                       &cut_index);
+  if (n_few) {
+  } else if (cuts && (SHORT || Tb <= kRankRow)) {
     FilterRank& rank = *reinterpret_cast<FilterRank*>(llist);
     if (tid < Tb) {  // (the thread that wrote sc[tid])
       rank.key[tid] = (uint64_t)__float_as_uint(sc[tid]) << 32 | (uint32_t)tid;
@@ -347,7 +554,7 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
       }
       if ((k && n >= k) || (limit && m >= limit)) sc[tid] = 0.f;
     }
-  } else if (cuts) {
+  } else if (!SHORT && cuts) {
     FilterHist& hist = *reinterpret_cast<FilterHist*>(llist);
     // digit `level` (0: the highest) of the bits, then of the index
     const auto histogram = [&](auto digit_of) {
@@ -420,7 +627,12 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   const bool only = a.eos >= 0 && a.eos < Tb && stays(a.eos) > a.eos_thr;
   const bool whole = !cuts && !only;  // the row as it is: no list
   int n = whole ? Tb : 0;             // entries listed
-  for (int t0 = 0; t0 < a.T; t0 += kFilterThreads) {
+  if (n_few && !only) {               // the list is there
+    n = n_few;
+    if (a.probs_out)
+      for (int t = tid; t < a.T; t += kFilterThreads)
+        a.probs_out[(size_t)bh * a.T + t] = t < Tb ? stays(t) : 0.f;
+  } else for (int t0 = 0; t0 < a.T; t0 += kFilterThreads) {
     const int t = t0 + tid;
     const float p = t < Tb && !(only && t != a.eos) ? stays(t) : 0.f;
     if (a.probs_out && t < a.T) a.probs_out[(size_t)bh * a.T + t] = p;
@@ -591,9 +803,11 @@ extern "C" int pa_decode_ex(const pa_kv_view* kv, const float* q, float* out,
 #define LLM_FILTER_LAUNCH(KVT)                                                  \
   do {                                                                          \
     if (ws_form)                                                                \
-      hipLaunchKernelGGL((pa_filter_kernel<KVT, true>), grid, block, 0, st, a);  \
+      hipLaunchKernelGGL((pa_filter_kernel<KVT, kWs>), grid, block, 0, st, a);   \
+    else if (T <= kRankRow)                                                     \
+      hipLaunchKernelGGL((pa_filter_kernel<KVT, kShort>), grid, block, 0, st, a); \
     else                                                                        \
-      hipLaunchKernelGGL((pa_filter_kernel<KVT, false>), grid, block, 0, st, a); \
+      hipLaunchKernelGGL((pa_filter_kernel<KVT, kLds>), grid, block, 0, st, a);  \
   } while (0)
   switch (kv->kv_dtype) {
     case LLM_F16: LLM_FILTER_LAUNCH(LLM_F16); break;

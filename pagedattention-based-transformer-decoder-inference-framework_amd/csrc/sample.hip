@@ -67,27 +67,6 @@ struct SampleArgs {
   int out2_stride;
 };
 
-// Of lanes l, l ^ 32, l ^ 16, .. l ^ 1, in that order: exchanges between registers (behind lane ^ 8
-// lanes l and l ^ 8 hold the same, so that a rotation by 4 is an exchange too).
-template <int CTRL>
-__device__ __forceinline__ int mov_lanes(int x) {
-  return __builtin_amdgcn_mov_dpp(x, CTRL, 0xF, 0xF, true);
-}
-template <typename T, typename Op>
-__device__ __forceinline__ T wave_reduce(T v, Op op) {
-  static_assert(sizeof(T) == 4);
-  const auto as_int = [](T x) { return __builtin_bit_cast(int, x); };
-  const auto as_t = [](int x) { return __builtin_bit_cast(T, x); };
-  const LanePair p = with_lane32(__builtin_bit_cast(float, v));
-  v = op(__builtin_bit_cast(T, p.a), __builtin_bit_cast(T, p.b));
-  const LanePair q = with_lane16(__builtin_bit_cast(float, v));
-  v = op(__builtin_bit_cast(T, q.a), __builtin_bit_cast(T, q.b));
-  v = op(v, as_t(mov_lanes<0x128>(as_int(v))));  // row_ror 8, 4
-  v = op(v, as_t(mov_lanes<0x124>(as_int(v))));
-  v = op(v, as_t(mov_lanes<0x4E>(as_int(v))));   // quad_perm [2,3,0,1], [1,0,3,2]
-  return op(v, as_t(mov_lanes<0xB1>(as_int(v))));
-}
-
 template <typename T, typename Op>
 __device__ __forceinline__ T block_reduce(T v, T* sh, Op op) {
   v = wave_reduce(v, op);

@@ -626,3 +626,39 @@ def test_pa_decode_ex_short_rows(gpu, oracle, T, D, ts, opt):
     if same.any():
         assert_parity(out[same], ref[same], RTOL)
     assert_parity(probs * both, rp * both, RTOL)
+
+
+# a top_k that few entries can reach: rows at the fewest groups for it and past the LDS form, 8,
+# 16 and 32 lanes a token, pages that recur (equal weights, at the cut too), missing ones, ends
+# inside a round of tokens
+@pytest.mark.parametrize("kv_dtype,D,T", [("float16", 64, 257), ("float16", 64, 512), ("float16", 128, 2047),
+                                          ("float32", 64, 1500), ("float32", 128, 1111),
+                                          ("bfloat16", 64, 8192), ("float16", 64, 8200)])
+@pytest.mark.parametrize("opt", [
+    dict(top_k=2), dict(top_k=24), dict(top_k=48), dict(top_k=64), dict(top_k=64, top_p=0.3),
+    dict(top_k=40, eos_token=100, eos_threshold=1e-9), dict(top_k=40, eos_token=100, eos_threshold=2.0),
+], ids=str)
+def test_pa_decode_ex_few(gpu, oracle, kv_dtype, D, T, opt):
+    import torch
+    import llm_capi
+    ts, B, H = 16, 4, 2
+    nt = (T + ts - 1) // ts
+    rng = np.random.default_rng(T + D)
+    q = (rng.standard_normal((B, H, D)) * 2.0 * D ** -0.5).astype(np.float32)
+    kd, kf = _kv_elems(rng, getattr(torch, kv_dtype), (B * H * nt, ts, D), 1.0)
+    vd, vf = _kv_elems(rng, getattr(torch, kv_dtype), (B * H * nt, ts, D), 1.0)
+    pt = rng.permutation(B * H * nt).astype(np.int32).reshape(B, H, nt)
+    pt[1] = pt[1][:, np.arange(nt) // 3 * 3]  # every page three times
+    pt[2, :, 1::5] = -1
+    lens = np.array([T, T, T, max(T - 37, 257)], np.int32)
+    ref, rp, _ = oracle.paged_attention(q, kf, vf, pt, T=T, context_lens=lens, want_probs=True, **opt)
+    out, probs, _ = llm_capi.pa_decode_ex(_dev(q), kd, vd, _dev(pt), T=T, context_lens=_dev(lens),
+                                          want_probs=True, **opt)
+    out, probs = out.cpu().numpy(), probs.cpu().numpy()
+    kept, want = probs > 0, rp > 0
+    # as above
+    assert (kept != want).sum(-1).max() <= (1 if opt.get("top_p", 1.0) < 1.0 else 0)
+    same, both = (kept == want).all(-1), kept & want
+    assert same.any()
+    assert_parity(out[same], ref[same], RTOL)
+    assert_parity(probs * both, rp * both, RTOL)
