@@ -187,6 +187,18 @@ __device__ __forceinline__ T wave_reduce(T v, Op op) {
   v = op(v, as_t(mov_lanes<0x4E>(as_int(v))));  // quad_perm [2,3,0,1], [1,0,3,2]
   return op(v, as_t(mov_lanes<0xB1>(as_int(v))));
 }
+// x of lane l ^ OFF, OFF 1, 2, 4 or 8
+template <int OFF>
+__device__ __forceinline__ int lane_xor(int x) {
+  if constexpr (OFF == 4)
+    return __builtin_amdgcn_ds_swizzle(x, 4 << 10 | 31);
+  else
+    return mov_lanes<OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : 0x128>(x);  // quad_perm, row_ror 8
+}
+template <int OFF>
+__device__ __forceinline__ float lane_xor(float x) {
+  return __builtin_bit_cast(float, lane_xor<OFF>(__builtin_bit_cast(int, x)));
+}
 __device__ __forceinline__ float wave_sum(float x) {
   return wave_reduce(x, [](float a, float b) { return a + b; });
 }

@@ -70,6 +70,8 @@ struct llm_decoder {
   DevBuf<float> lm_pv;    // [max_batch][lm_nwg] LM-head argmax partials
   DevBuf<int32_t> lm_pi;
   int lm_nwg = 0;
+  DevBuf<uint64_t> lm_key;  // [max_batch][kChoiceStride], 0 between launches (HeadChoice)
+  DevBuf<uint32_t> lm_arrived;  // [max_batch]
   DevBuf<int8_t> qa;
   DevBuf<uint16_t> a16;
   // FP16: the fused o_proj's int64 columns [max_batch][hid] (zero between
@@ -201,6 +203,10 @@ extern "C" int llm_decoder_create(const llm_decoder_config* cfg_in, llm_decoder*
   d->lm_nwg = lm_head_workgroups(d->V);
   RET_IF(d->lm_pv.alloc((size_t)B * d->lm_nwg));
   RET_IF(d->lm_pi.alloc((size_t)B * d->lm_nwg));
+  RET_IF(d->lm_key.alloc((size_t)B * kChoiceStride));
+  RET_IF(d->lm_arrived.alloc((size_t)B));
+  LLM_HIP_RET(hipMemset(d->lm_key.p, 0, sizeof(uint64_t) * d->lm_key.n));
+  LLM_HIP_RET(hipMemset(d->lm_arrived.p, 0, sizeof(uint32_t) * d->lm_arrived.n));
   RET_IF(d->sa.alloc((size_t)B));
   const size_t B16 = ((size_t)B + 15) / 16 * 16;  // packed-A tiles are 16 rows
   RET_IF(d->qa.alloc(B16 * std::max(hid, inter)));
@@ -707,6 +713,13 @@ int llm_decoder::next_tokens(const float* xr, int n, int r0, const int32_t* ctr,
   const bool sample = temperature > 0.f && top_k != 1;
   float* pv = lm_pv.p + (size_t)r0 * lm_nwg;
   int32_t* pi = lm_pi.p + (size_t)r0 * lm_nwg;
+  if (!sample && lm_head_chooses(n, hid)) {
+    HeadChoice c;
+    c.key = lm_key.p + (size_t)r0 * kChoiceStride; c.arrived = lm_arrived.p + r0;
+    c.out = tokens.p + r0; c.pos = adv_pos; c.ctx = adv_ctx;
+    LLM_HIP_RET(launch_lm_head(xr, emb_packed.p, lg, n, V, hid, nullptr, nullptr, st, c));
+    return LLM_OK;
+  }
   LLM_HIP_RET(launch_lm_head(xr, emb_packed.p, lg, n, V, hid, sample ? nullptr : pv, pi, st));
   if (sample) {
     LLM_HIP_RET(launch_sample(lg, n, r0, V, temperature, top_k, top_p, sample_seed, ctr,

@@ -1,5 +1,5 @@
 // Tied-embedding LM head + greedy argmax for decode (logits = x . E^T, the
-// LM head the reference lacks: SURVEY Appendix A #20; argmax = sample_from_logits,
+// LM head the reference lacks; argmax = sample_from_logits,
 // decoder/cuda_decoder.cu:7-14).
 //
 // x is fp32 [M][K] (M <= 64 per row block).  E fp16 [V][K] is the embedding
@@ -24,7 +24,9 @@
 //
 // The epilogue writes the logits and a per-(row, workgroup) (max, first
 // index) pair; argmax_partials_kernel reduces those pairs per row (first
-// maximum wins), so greedy decoding never re-reads the [M][V] logits.
+// maximum wins), so greedy decoding never re-reads the [M][V] logits.  Up to 16
+// rows the workgroups meet in one 64-bit key a row instead and the last of them
+// writes the token (HeadChoice): no launch behind the head.
 #include "common.hpp"
 #include "row_ops.hpp"
 
@@ -55,9 +57,19 @@ struct LmHeadArgs {
   int32_t* part_idx;  // [M][nwg]
   int M, V, K, nwg;
   int tiles;  // vocabulary tiles (computing waves) per workgroup, <= kLmWaves
+  HeadChoice choice;  // (lm_head_x1_kernel) key: not NULL: the rows' tokens, not the partials
   int mode;  // 0; tuning build (LLM_LM_MODE): bit0 skip MFMA, bit1 skip x staging, bit2 skip
              // E loads; bit3: E with the default cache policy (kept) instead of nt
 };
+
+// The first maximum of 16 neighbouring lanes' (value, index), by lanes l ^ 1, 2, 4, 8
+template <int OFF = 1>
+__device__ __forceinline__ void first_max(float& v, int& i) {
+  const float ov = lane_xor<OFF>(v);
+  const int oi = lane_xor<OFF>(i);
+  if (ov > v || (ov == v && oi < i)) { v = ov; i = oi; }
+  if constexpr (OFF < 8) first_max<OFF * 2>(v, i);
+}
 
 // MT = 16-row tiles of x per workgroup (1, 2 or 4); WAVES waves, each NTW
 // vocabulary tiles (16 rows of E) per k-step against one read of the x
@@ -209,12 +221,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_head_kernel(LmHeadArgs a) {
         // max over this wave's 16 vocabulary rows (lanes sharing lane>>4), first index on ties
         float bv = n < a.V ? v : -INFINITY;
         int bi = n < a.V ? n : 0x7fffffff;
-#pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-          const float ov = __shfl_xor(bv, off, 64);
-          const int oi = __shfl_xor(bi, off, 64);
-          if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-        }
+        first_max(bv, bi);
         if ((lane & 15) == 0 && t < WAVES * NTW) { pv[t][row] = bv; pi[t][row] = bi; }
       }
     }
@@ -312,35 +319,67 @@ __global__ __launch_bounds__(1024) void lm_head_x1_kernel(LmHeadArgs a) {
     }
   }
   // acc lane l, reg r: x row m0 + 4 (l >> 4) + r, vocabulary row 16 ntile + (l & 15)
-  const int n = mine ? ntile * 16 + (lane & 15) : a.V;
+  const int n = mine ? ntile * 16 + (lane & 15) : a.V, rows = min(a.M - m0, 16);
+  const bool choose = a.part_val || a.choice.key;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
+    if (r >= rows) break;
     const int row = 4 * (lane >> 4) + r;
     const float v = acc[r];
-    if (a.logits && m0 + row < a.M && n < a.V) a.logits[(size_t)(m0 + row) * a.V + n] = v;
-    if (a.part_val) {
+    if (a.logits && row < rows && n < a.V) a.logits[(size_t)(m0 + row) * a.V + n] = v;
+    if (choose) {
       float bv = n < a.V ? v : -INFINITY;
       int bi = n < a.V ? n : 0x7fffffff;
-#pragma unroll
-      for (int off = 1; off < 16; off <<= 1) {
-        const float ov = __shfl_xor(bv, off, 64);
-        const int oi = __shfl_xor(bi, off, 64);
-        if (ov > bv || (ov == bv && oi < bi)) { bv = ov; bi = oi; }
-      }
+      first_max(bv, bi);
       if ((lane & 15) == 0) { pv[w][row] = bv; pi[w][row] = bi; }
     }
   }
-  if (!a.part_val) return;
+  if (!choose) return;
   __syncthreads();
-  if (threadIdx.x < 16 && m0 + (int)threadIdx.x < a.M) {
-    const int row = threadIdx.x;
-    float bv = pv[0][row];
-    int bi = pi[0][row];
-    for (int ww = 1; ww < a.tiles; ++ww)  // tiles in increasing vocabulary order
+  if (w) return;
+  const int row = lane;
+  float bv = -INFINITY;
+  int bi = 0x7fffffff;
+  if (row < rows) {
+    bv = pv[0][row];
+    bi = pi[0][row];
+#pragma unroll
+    for (int ww = 1; ww < kLmWaves; ++ww)  // tiles in increasing vocabulary order (past `tiles`: -inf)
       if (pv[ww][row] > bv) { bv = pv[ww][row]; bi = pi[ww][row]; }
-    a.part_val[(size_t)(m0 + row) * a.nwg + blockIdx.x] = bv;
-    a.part_idx[(size_t)(m0 + row) * a.nwg + blockIdx.x] = bi;
+    if (a.part_val) {
+      a.part_val[(size_t)(m0 + row) * a.nwg + blockIdx.x] = bv;
+      a.part_idx[(size_t)(m0 + row) * a.nwg + blockIdx.x] = bi;
+    }
   }
+  if (!a.choice.key) return;
+  // The order of argmax_partials_kernel: by value (-0 and 0 alike), then the smaller index; not a
+  // number and no entry at all: 0.  Every maximum's old value is waited for before this workgroup
+  // is counted (one whose result nobody reads would not be), so that the last one counted finds
+  // them all.  Keys and counter are left as they were found, 0.
+  const HeadChoice& c = a.choice;
+  unsigned long long* key = reinterpret_cast<unsigned long long*>(c.key) + (size_t)row * kChoiceStride;
+  if (row < rows) {
+    const uint32_t bits = __float_as_uint(bv + 0.f);
+    const uint32_t order = bits >> 31 ? ~bits : bits | 0x80000000u;
+    const unsigned long long mine_is =
+        bv != bv || bi == 0x7fffffff ? 0ull : (unsigned long long)order << 32 | (uint32_t)~bi;
+    const unsigned long long old =
+        __hip_atomic_fetch_max(key, mine_is, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" ::"v"((uint32_t)old), "v"((uint32_t)(old >> 32)) : "memory");
+  }
+  uint32_t before = 0;
+  if (lane == 0) before = __hip_atomic_fetch_add(c.arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (__builtin_amdgcn_readfirstlane(before) != (uint32_t)a.nwg - 1) return;
+  if (row < rows) {
+    const unsigned long long best =
+        __hip_atomic_exchange(key, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    c.out[row] = best ? (int32_t)~(uint32_t)best : 0;
+    if (c.pos) {
+      c.pos[row] += 1;
+      c.ctx[row] += 1;
+    }
+  }
+  if (lane == 0) __hip_atomic_store(c.arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Per row: the first maximum over the workgroup partials (in vocabulary order).
@@ -436,6 +475,22 @@ __global__ void lm_pack_kernel(const _Float16* __restrict__ E, _Float16* __restr
   }
 }
 
+namespace {
+int lm_mode() {
+#if LLM_TUNING
+  static const int mode = env_int("LLM_LM_MODE", 0) | (env_int("LLM_LM_FORM", 0) ? 256 : 0);
+  return mode;
+#else
+  return 0;
+#endif
+}
+}  // namespace
+
+// us of a head and its choice, V 50257: 1 row of K 256 8.3 + 3.9 in two launches, 7.6 in one; 16 rows of K 768
+// 18.3 + 4.0 and 20.0 (an arrival and a maximum a row from 242 workgroups).  More rows than a tile keep
+// two launches: their blocks would meet in as many keys and counters again.
+bool lm_head_chooses(int M, int K) { return M <= 16 && K <= 2048 && lm_mode() == 0; }
+
 size_t lm_head_packed_bytes(int V, int K) { return (size_t)((V + 15) / 16) * (K / 32) * 1024; }
 
 hipError_t launch_lm_pack(const void* E, void* P, int V, int K, hipStream_t st) {
@@ -447,17 +502,10 @@ hipError_t launch_lm_pack(const void* E, void* P, int V, int K, hipStream_t st) 
 }
 
 hipError_t launch_lm_head(const float* x, const void* E, float* logits, int M, int V, int K,
-                          float* part_val, int32_t* part_idx, hipStream_t st) {
-#if LLM_TUNING
-  static const int mode = [] {
-    const char* v = std::getenv("LLM_LM_MODE");
-    return v ? std::atoi(v) : 0;
-  }();
-#else
-  constexpr int mode = 0;
-#endif
+                          float* part_val, int32_t* part_idx, hipStream_t st,
+                          const HeadChoice& choice) {
   LmHeadArgs a{x, static_cast<const _Float16*>(E), logits, part_val, part_idx, M, V, K,
-               lm_head_workgroups(V), lm_head_tiles(V), mode};
+               lm_head_workgroups(V), lm_head_tiles(V), choice, lm_mode() & 255};
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   const dim3 grid(a.nwg, (M + 16 * mt - 1) / (16 * mt));
   // 16 waves x 1 vocabulary tile.  The tuning build's LLM_LM_FORM=1 (8 waves x
@@ -465,14 +513,14 @@ hipError_t launch_lm_head(const float* x, const void* E, float* logits, int M, i
   // at every row count (C3 / C4 / C2 shapes 58.7 / 46.1 / 16.3 vs 56.0 / 43.8 /
   // 15.9 us, profiles/r03/lm_head_forms.txt): the LDS reads do not bound it.
 #if LLM_TUNING
-  if (env_int("LLM_LM_FORM", 0)) {
+  if (lm_mode() & 256) {
     if (mt == 1) hipLaunchKernelGGL((lm_head_kernel<1, 8, 2>), grid, dim3(512), 0, st, a);
     else if (mt == 2) hipLaunchKernelGGL((lm_head_kernel<2, 8, 2>), grid, dim3(512), 0, st, a);
     else hipLaunchKernelGGL((lm_head_kernel<4, 8, 2>), grid, dim3(512), 0, st, a);
     return hipGetLastError();
   }
 #endif
-  if (mt == 1 && a.K <= 2048 && mode == 0) {
+  if (mt == 1 && a.K <= 2048 && lm_mode() == 0) {
     const size_t lds = (size_t)(a.K / 32) * 2 * 64 * sizeof(u32x4);
     hipLaunchKernelGGL(lm_head_x1_kernel, grid, dim3(1024), lds, st, a);
   } else if (mt == 1) hipLaunchKernelGGL((lm_head_kernel<1, 16, 1>), grid, dim3(1024), 0, st, a);

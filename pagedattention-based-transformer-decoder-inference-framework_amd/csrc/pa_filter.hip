@@ -326,14 +326,6 @@ __device__ __forceinline__ int filter_few(const float* sc, int Tb, float most, u
 // latency of its steps; the 192 workgroups are one a CU.
 constexpr int kValueTokens = 4;
 
-// x of lane l ^ OFF
-template <int OFF>
-__device__ __forceinline__ float lane_xor(float x) {
-  if constexpr (OFF == 4)
-    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), 4 << 10 | 31));
-  else
-    return mov_dpp<OFF == 1 ? 0xB1 : OFF == 2 ? 0x4E : 0x128>(x);  // quad_perm, row_ror 8
-}
 // Sums of x[0 .. N) over lanes c, each lane giving half of what it holds to lane c ^ OFF, then OFF / 2:
 // in the order in which a whole exchange at every step would add them.
 template <int OFF, int N>

@@ -33,8 +33,21 @@ hipError_t launch_scatter_i32(int32_t* dst, const int64_t* idx, const int32_t* v
 int lm_head_workgroups(int V);
 size_t lm_head_packed_bytes(int V, int K);
 hipError_t launch_lm_pack(const void* E, void* P, int V, int K, hipStream_t st);  // E -> packed
+// Where the head itself writes the greedy tokens (lm_head_chooses(M, K), no partials then): a key
+// of kChoiceStride words a row and one counter, all 0 before and after, of no other launch
+// that may run beside it.  pos / ctx (optional): the decode step's position advance.
+constexpr int kChoiceStride = 16;
+struct HeadChoice {
+  uint64_t* key = nullptr;
+  uint32_t* arrived = nullptr;
+  int32_t* out = nullptr;
+  int32_t* pos = nullptr;
+  int32_t* ctx = nullptr;
+};
+bool lm_head_chooses(int M, int K);
 hipError_t launch_lm_head(const float* x, const void* E, float* logits, int M, int V, int K,
-                          float* part_val, int32_t* part_idx, hipStream_t st);
+                          float* part_val, int32_t* part_idx, hipStream_t st,
+                          const HeadChoice& choice = HeadChoice());
 hipError_t launch_argmax_partials(const float* part_val, const int32_t* part_idx, int M, int nwg,
                                   int32_t* out, hipStream_t st, int32_t* pos = nullptr,
                                   int32_t* ctx = nullptr);

@@ -245,6 +245,26 @@ def test_generate_after_set_sampling_is_greedy(gpu, oracle):
     assert differ > 0
 
 
+@pytest.mark.parametrize("rows", [1, 5, 16, 17])
+@pytest.mark.parametrize("V,period", [(16, 5), (300, 7), (5000, 37), (5000, 0)])
+def test_greedy_tokens_of_equal_logits(gpu, oracle, rows, V, period):
+    """Logits that stand in many tiles and workgroups (embedding rows repeated; period 0: all
+    zero): the token is the first of the largest, at every step."""
+    torch = _torch()
+    w = _int8_model(oracle, L=1, H=2, D=64, V=V, S=32, seed=V + rows)
+    emb = w["emb"].copy()
+    w["emb"] = emb[np.arange(V) % period] if period else np.zeros_like(emb)
+    dec = _make_gpu_decoder(w, max_batch=rows)
+    dec.begin_synthetic(rows, 0, 0, False)
+    logits = torch.empty((rows, V), device="cuda")
+    tok = [(3 * b) % V for b in range(rows)]
+    for _ in range(6):
+        tok = dec.step(tok, logits_ptr=logits.data_ptr())
+        torch.cuda.synchronize()
+        assert list(tok) == logits.cpu().numpy().argmax(1).tolist()
+        tok = [(t + b) % V for b, t in enumerate(tok)]
+
+
 def test_generate_call_forms(gpu, oracle):
     w = _int8_model(oracle, L=1, H=2, D=64, V=300, S=48, seed=3)
     dec = _make_gpu_decoder(w, max_batch=4)
