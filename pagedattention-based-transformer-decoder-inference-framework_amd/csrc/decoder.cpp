@@ -42,6 +42,26 @@ using namespace llm;
 // read and cleared (llm_decoder::report_range)
 __global__ void take_flag_kernel(int* f) { f[1] = atomicExch(f, 0); }
 
+// Up to kPut words and the place of a step's logits, out of the launch's own arguments: one launch in
+// place of copies from pageable memory before a step and of the logits' copy behind it (which a
+// captured step needs, since its own arguments are fixed).  A prompt of 113 tokens and 16 steps
+// of one row, 2 layers of hidden 256: 1,191 us, now 1,137.
+constexpr int kPut = 128;
+struct StepPut {
+  int32_t* to;
+  int32_t* to2;  // (optional) takes v2
+  float** place; // (optional) takes logits
+  float* logits;
+  int n;
+  int32_t v2, v[kPut];
+};
+__global__ __launch_bounds__(kPut) void step_put_kernel(StepPut a) {
+  const int i = threadIdx.x;
+  if (i < a.n) a.to[i] = a.v[i];
+  if (i == 0 && a.to2) *a.to2 = a.v2;
+  if (i == 0 && a.place) *a.place = a.logits;
+}
+
 struct llm_decoder {
   llm_decoder_config cfg{};
   int L = 0, H = 0, D = 0, hid = 0, inter = 0, V = 0, TS = 0, max_tiles = 0, maxB = 0;
@@ -72,6 +92,8 @@ struct llm_decoder {
   int lm_nwg = 0;
   DevBuf<uint64_t> lm_key;  // [max_batch][kChoiceStride], 0 between launches (HeadChoice)
   DevBuf<uint32_t> lm_arrived;  // [max_batch]
+  DevBuf<float*> logits_at;     // [1] the step's logits go there, if not null (step_put_kernel)
+  bool logits_set = false;      // logits_at is not null
   DevBuf<int8_t> qa;
   DevBuf<uint16_t> a16;
   // FP16: the fused o_proj's int64 columns [max_batch][hid] (zero between
@@ -141,7 +163,8 @@ struct llm_decoder {
   void embed_rows(const int32_t* tok);
   int step_tail(hipStream_t st, int r0, int n);
   int next_tokens(const float* xr, int n, int r0, const int32_t* ctr, hipStream_t st,
-                  int32_t* adv_pos = nullptr, int32_t* adv_ctx = nullptr);
+                  int32_t* adv_pos = nullptr, int32_t* adv_ctx = nullptr,
+                  float* const* place = nullptr);
   int enqueue_step(hipStream_t st);
   int run_step(const int32_t* tokens_host, float* logits_dev, int32_t* next_host, hipStream_t st);
 
@@ -206,6 +229,8 @@ extern "C" int llm_decoder_create(const llm_decoder_config* cfg_in, llm_decoder*
   RET_IF(d->lm_key.alloc((size_t)B * kChoiceStride));
   RET_IF(d->lm_arrived.alloc((size_t)B));
   LLM_HIP_RET(hipMemset(d->lm_key.p, 0, sizeof(uint64_t) * d->lm_key.n));
+  RET_IF(d->logits_at.alloc(1));
+  LLM_HIP_RET(hipMemset(d->logits_at.p, 0, sizeof(float*)));
   LLM_HIP_RET(hipMemset(d->lm_arrived.p, 0, sizeof(uint32_t) * d->lm_arrived.n));
   RET_IF(d->sa.alloc((size_t)B));
   const size_t B16 = ((size_t)B + 15) / 16 * 16;  // packed-A tiles are 16 rows
@@ -708,7 +733,7 @@ int llm_decoder::tap(int l, int stage, const Rows& R, int K, hipStream_t st) {
 // adv_pos / adv_ctx (optional): advance the rows' positions afterwards (fused
 // into the argmax launch; a launch of its own after a draw, which reads them).
 int llm_decoder::next_tokens(const float* xr, int n, int r0, const int32_t* ctr, hipStream_t st,
-                             int32_t* adv_pos, int32_t* adv_ctx) {
+                             int32_t* adv_pos, int32_t* adv_ctx, float* const* place) {
   float* lg = logits.p + (size_t)r0 * V;
   const bool sample = temperature > 0.f && top_k != 1;
   float* pv = lm_pv.p + (size_t)r0 * lm_nwg;
@@ -717,10 +742,12 @@ int llm_decoder::next_tokens(const float* xr, int n, int r0, const int32_t* ctr,
     HeadChoice c;
     c.key = lm_key.p + (size_t)r0 * kChoiceStride; c.arrived = lm_arrived.p + r0;
     c.out = tokens.p + r0; c.pos = adv_pos; c.ctx = adv_ctx;
-    LLM_HIP_RET(launch_lm_head(xr, emb_packed.p, lg, n, V, hid, nullptr, nullptr, st, c));
+    LLM_HIP_RET(launch_lm_head(xr, emb_packed.p, lg, n, V, hid, nullptr, nullptr, st, c,
+                               place));
     return LLM_OK;
   }
-  LLM_HIP_RET(launch_lm_head(xr, emb_packed.p, lg, n, V, hid, sample ? nullptr : pv, pi, st));
+  LLM_HIP_RET(launch_lm_head(xr, emb_packed.p, lg, n, V, hid, sample ? nullptr : pv, pi, st, {},
+                             sample ? nullptr : place));  // (a draw reads them here)
   if (sample) {
     LLM_HIP_RET(launch_sample(lg, n, r0, V, temperature, top_k, top_p, sample_seed, ctr,
                               tokens.p + r0, st));
@@ -741,7 +768,8 @@ void llm_decoder::embed_rows(const int32_t* tok) {
 }
 
 int llm_decoder::step_tail(hipStream_t st, int r0, int n) {
-  return next_tokens(x.p + (size_t)r0 * hid, n, r0, pos.p + r0, st, pos.p + r0, ctx.p + r0);
+  return next_tokens(x.p + (size_t)r0 * hid, n, r0, pos.p + r0, st, pos.p + r0, ctx.p + r0,
+                     logits_at.p);
 }
 
 // One decode step of all active rows (captured into the step graph).
@@ -756,6 +784,22 @@ int llm_decoder::enqueue_step(hipStream_t st) {
     RET_IF(layer_post(l, st, R));
   }
   return step_tail(st, 0, batch);
+}
+
+// Memory of the current device that a kernel can write `bytes` of as floats; what is not (other
+// devices' memory, the host's, an allocation too small) is left to the copy, and to its checks.
+static bool kernel_writes(const void* p, size_t bytes) {
+  hipPointerAttribute_t at{};
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  int dev = -1;
+  const bool ok = reinterpret_cast<uintptr_t>(p) % alignof(float) == 0 && hipGetDevice(&dev) == hipSuccess &&
+                  hipPointerGetAttributes(&at, p) == hipSuccess && at.type == hipMemoryTypeDevice &&
+                  at.device == dev &&
+                  hipMemGetAddressRange(&base, &size, const_cast<void*>(p)) == hipSuccess &&
+                  (size_t)(static_cast<const char*>(p) - static_cast<char*>(base)) + bytes <= size;
+  if (!ok) (void)hipGetLastError();
+  return ok;
 }
 
 int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t* next_host,
@@ -774,8 +818,21 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
   if (tokens_host) {
     for (int b = 0; b < batch; ++b)
       LLM_REQUIRE(tokens_host[b] >= 0 && tokens_host[b] < V, "decoder: token id out of range");
-    LLM_HIP_RET(hipMemcpyAsync(tokens.p, tokens_host, sizeof(int32_t) * batch,
-                               hipMemcpyHostToDevice, st));
+  }
+  const bool sample = temperature > 0.f && top_k != 1;
+  const bool direct = logits_dev && !sample && kernel_writes(logits_dev, sizeof(float) * batch * V);
+  if (tokens_host || direct || logits_set) {
+    for (int b0 = 0; b0 == 0 || (tokens_host && b0 < batch); b0 += kPut) {
+      StepPut a{};
+      a.to = tokens.p + b0;
+      a.n = tokens_host ? std::min(kPut, batch - b0) : 0;
+      std::copy_n(tokens_host + b0, a.n, a.v);
+      if (b0 == 0) a.place = logits_at.p;
+      a.logits = direct ? logits_dev : nullptr;
+      hipLaunchKernelGGL(step_put_kernel, dim3(1), dim3(kPut), 0, st, a);
+      LLM_HIP_RET(hipGetLastError());
+    }
+    logits_set = direct;
   }
   if (!use_graph) {
     RET_IF(enqueue_step(st));
@@ -799,7 +856,7 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
     LLM_HIP_RET(hipGraphLaunch(graph, st));
   }
   for (int b = 0; b < batch; ++b) h_pos[b] += 1;
-  if (logits_dev)
+  if (logits_dev && !direct)
     LLM_HIP_RET(hipMemcpyAsync(logits_dev, logits.p, sizeof(float) * batch * V,
                                hipMemcpyDeviceToDevice, st));
   if (next_host) {
@@ -902,7 +959,7 @@ int llm_decoder::prefill(int row, const int32_t* toks, int n, hipStream_t st) {
   RET_IF(ensure_prefill(C));
   C = std::min(C, pf_cap);
   KvCache* k = kv_impl(kv);
-  std::vector<int32_t> meta((size_t)4 * C), pc(2);
+  std::vector<int32_t> meta((size_t)4 * C);
   for (int c0 = 0; c0 < n; c0 += C) {
     const int m = std::min(C, n - c0);
     const int p0 = h_pos[row];
@@ -937,12 +994,13 @@ int llm_decoder::prefill(int row, const int32_t* toks, int n, hipStream_t st) {
     h_pos[row] = p0 + m;
     if (c0 + m == n) {  // last token: logits -> the row's next token, decode state
       RET_IF(next_tokens(px.p + (size_t)(m - 1) * hid, 1, row, pmeta.p + (m - 1), st));
-      pc[0] = p0 + m;
-      pc[1] = p0 + m + 1;
-      LLM_HIP_RET(hipMemcpyAsync(pos.p + row, &pc[0], sizeof(int32_t), hipMemcpyHostToDevice, st));
-      LLM_HIP_RET(hipMemcpyAsync(ctx.p + row, &pc[1], sizeof(int32_t), hipMemcpyHostToDevice, st));
+      StepPut a{};
+      a.to = pos.p + row; a.n = 1; a.v[0] = p0 + m;
+      a.to2 = ctx.p + row; a.v2 = p0 + m + 1;
+      hipLaunchKernelGGL(step_put_kernel, dim3(1), dim3(kPut), 0, st, a);
+      LLM_HIP_RET(hipGetLastError());
     }
-    LLM_HIP_RET(hipStreamSynchronize(st));  // meta / pc staging reused next chunk
+    LLM_HIP_RET(hipStreamSynchronize(st));  // meta staging reused next chunk
   }
   return LLM_OK;
 }
@@ -1014,6 +1072,20 @@ int llm_decoder::forward_mixed(const std::vector<StepSeq>& seqs, float* logits_d
   return LLM_OK;
 }
 
+// The rows' state at start_pos and the fused o_proj's columns and flag, empty: one launch (beginning a
+// sequence 75 us with a copy or a fill for each, now 38).
+__global__ __launch_bounds__(256) void reset_rows_kernel(int32_t* pos, int32_t* ctx, int32_t* tokens, int batch,
+                                                         int start_pos, long long* oacc, size_t columns, int* oflag) {
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < (size_t)batch) {
+    pos[i] = start_pos;
+    ctx[i] = start_pos + 1;
+    tokens[i] = 0;
+  }
+  if (i < columns) oacc[i] = 0;
+  if (i == 0 && oflag) *oflag = 0;
+}
+
 static int reset_rows(llm_decoder* d, int batch, int start_pos) {
   LLM_REQUIRE(batch > 0 && batch <= d->maxB, "decoder: batch must be in [1, max_batch]");
   RET_IF(kv_cache_clear(d->kv));
@@ -1022,13 +1094,12 @@ static int reset_rows(llm_decoder* d, int batch, int start_pos) {
   d->row_group = 1;
   d->h_pos.assign(d->maxB, 0);
   for (int b = 0; b < batch; ++b) d->h_pos[b] = start_pos;
-  if (d->oacc.p) LLM_HIP_RET(hipMemset(d->oacc.p, 0, sizeof(long long) * d->oacc.n));
-  if (d->oflag.p) LLM_HIP_RET(hipMemset(d->oflag.p, 0, sizeof(int)));
   d->range_clamped = 0;
-  std::vector<int32_t> pos(batch, start_pos), ctx(batch, start_pos + 1), tok(batch, 0);
-  LLM_HIP_RET(hipMemcpy(d->pos.p, pos.data(), sizeof(int32_t) * batch, hipMemcpyHostToDevice));
-  LLM_HIP_RET(hipMemcpy(d->ctx.p, ctx.data(), sizeof(int32_t) * batch, hipMemcpyHostToDevice));
-  LLM_HIP_RET(hipMemcpy(d->tokens.p, tok.data(), sizeof(int32_t) * batch, hipMemcpyHostToDevice));
+  const size_t columns = d->oacc.p ? d->oacc.n : 0;
+  const unsigned blocks = (unsigned)((std::max(columns, (size_t)batch) + 255) / 256);
+  hipLaunchKernelGGL(reset_rows_kernel, dim3(blocks), dim3(256), 0, nullptr, d->pos.p, d->ctx.p, d->tokens.p, batch,
+                     start_pos, d->oacc.p, columns, d->oflag.p);
+  LLM_HIP_RET(hipGetLastError());
   LLM_HIP_RET(hipDeviceSynchronize());
   return LLM_OK;
 }

@@ -57,10 +57,16 @@ struct LmHeadArgs {
   int32_t* part_idx;  // [M][nwg]
   int M, V, K, nwg;
   int tiles;  // vocabulary tiles (computing waves) per workgroup, <= kLmWaves
+  float* const* place;  // where the logits go instead, if it holds a pointer (or NULL)
   HeadChoice choice;  // (lm_head_x1_kernel) key: not NULL: the rows' tokens, not the partials
   int mode;  // 0; tuning build (LLM_LM_MODE): bit0 skip MFMA, bit1 skip x staging, bit2 skip
              // E loads; bit3: E with the default cache policy (kept) instead of nt
 };
+
+__device__ __forceinline__ float* logits_of(const LmHeadArgs& a) {
+  float* p = a.place ? *a.place : nullptr;
+  return p ? p : a.logits;
+}
 
 // The first maximum of 16 neighbouring lanes' (value, index), by lanes l ^ 1, 2, 4, 8
 template <int OFF = 1>
@@ -84,6 +90,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_head_kernel(LmHeadArgs a) {
   const int lane = lane_id();
   const int w = wave_id_uniform();
   const int m0 = blockIdx.y * 16 * MT;
+  float* const logits = logits_of(a);
   const int KS = a.K / 32;
   const int ntiles = (a.V + 15) / 16;
   const auto ers = __builtin_amdgcn_make_buffer_rsrc(
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(WAVES * 64) void lm_head_kernel(LmHeadArgs a) {
     for (int r = 0; r < 4; ++r) {
       const int row = mt * 16 + 4 * (lane >> 4) + r;
       const float v = acc[j][mt][r];
-      if (a.logits && m0 + row < a.M && n < a.V) a.logits[(size_t)(m0 + row) * a.V + n] = v;
+      if (logits && m0 + row < a.M && n < a.V) logits[(size_t)(m0 + row) * a.V + n] = v;
       if (a.part_val) {
         // max over this wave's 16 vocabulary rows (lanes sharing lane>>4), first index on ties
         float bv = n < a.V ? v : -INFINITY;
@@ -254,6 +261,7 @@ __global__ __launch_bounds__(1024) void lm_head_x1_kernel(LmHeadArgs a) {
   const int lane = lane_id();
   const int w = wave_id_uniform();
   const int m0 = blockIdx.y * 16;
+  float* const logits = logits_of(a);
   const int KS = a.K / 32;
   const int ntiles = (a.V + 15) / 16;
   const auto ers = __builtin_amdgcn_make_buffer_rsrc(
@@ -326,7 +334,7 @@ __global__ __launch_bounds__(1024) void lm_head_x1_kernel(LmHeadArgs a) {
     if (r >= rows) break;
     const int row = 4 * (lane >> 4) + r;
     const float v = acc[r];
-    if (a.logits && row < rows && n < a.V) a.logits[(size_t)(m0 + row) * a.V + n] = v;
+    if (logits && row < rows && n < a.V) logits[(size_t)(m0 + row) * a.V + n] = v;
     if (choose) {
       float bv = n < a.V ? v : -INFINITY;
       int bi = n < a.V ? n : 0x7fffffff;
@@ -503,9 +511,9 @@ hipError_t launch_lm_pack(const void* E, void* P, int V, int K, hipStream_t st) 
 
 hipError_t launch_lm_head(const float* x, const void* E, float* logits, int M, int V, int K,
                           float* part_val, int32_t* part_idx, hipStream_t st,
-                          const HeadChoice& choice) {
+                          const HeadChoice& choice, float* const* place) {
   LmHeadArgs a{x, static_cast<const _Float16*>(E), logits, part_val, part_idx, M, V, K,
-               lm_head_workgroups(V), lm_head_tiles(V), choice, lm_mode() & 255};
+               lm_head_workgroups(V), lm_head_tiles(V), place, choice, lm_mode() & 255};
   const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
   const dim3 grid(a.nwg, (M + 16 * mt - 1) / (16 * mt));
   // 16 waves x 1 vocabulary tile.  The tuning build's LLM_LM_FORM=1 (8 waves x

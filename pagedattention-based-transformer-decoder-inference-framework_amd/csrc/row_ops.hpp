@@ -45,9 +45,10 @@ struct HeadChoice {
   int32_t* ctx = nullptr;
 };
 bool lm_head_chooses(int M, int K);
+// place (optional): device word; where it holds a pointer, the logits go there
 hipError_t launch_lm_head(const float* x, const void* E, float* logits, int M, int V, int K,
                           float* part_val, int32_t* part_idx, hipStream_t st,
-                          const HeadChoice& choice = HeadChoice());
+                          const HeadChoice& choice = HeadChoice(), float* const* place = nullptr);
 hipError_t launch_argmax_partials(const float* part_val, const int32_t* part_idx, int M, int nwg,
                                   int32_t* out, hipStream_t st, int32_t* pos = nullptr,
                                   int32_t* ctx = nullptr);

@@ -265,6 +265,34 @@ def test_greedy_tokens_of_equal_logits(gpu, oracle, rows, V, period):
         tok = [(t + b) % V for b, t in enumerate(tok)]
 
 
+@pytest.mark.parametrize("rows", [1, 17, 130])
+def test_logits_places(gpu, oracle, rows):
+    """The same logits wherever they go: a buffer that starts at any float, pinned host memory,
+    the last floats of an allocation, nowhere in between; a step without any leaves them alone."""
+    torch = _torch()
+    V = 300
+    w = _int8_model(oracle, L=1, H=2, D=64, V=V, S=32, seed=rows)
+    dec = _make_gpu_decoder(w, max_batch=rows)
+    toks = [[(7 * s + b) % V for b in range(rows)] for s in range(6)]
+    n = rows * V
+    want = torch.empty((6, rows, V), device="cuda")
+    dec.begin_synthetic(rows, 0, 0, False)
+    ids = [list(dec.step(t, logits_ptr=want[i].data_ptr())) for i, t in enumerate(toks)]
+    assert ids == want.cpu().numpy().argmax(2).tolist()
+    odd = torch.zeros(n + 3, device="cuda")
+    pinned = torch.zeros(n, pin_memory=True)
+    dec.begin_synthetic(rows, 0, 0, False)
+    for i, place in enumerate([odd[1:n + 1], None, pinned, odd[3:], None, odd[:n]]):
+        before = odd.clone()
+        got = dec.step(toks[i], logits_ptr=0 if place is None else place.data_ptr())
+        torch.cuda.synchronize()
+        assert list(got) == ids[i]
+        if place is None:
+            assert torch.equal(odd, before)
+        else:
+            assert torch.equal(place.cpu(), want[i].cpu().reshape(-1))
+
+
 def test_generate_call_forms(gpu, oracle):
     w = _int8_model(oracle, L=1, H=2, D=64, V=300, S=48, seed=3)
     dec = _make_gpu_decoder(w, max_batch=4)
