@@ -1623,7 +1623,7 @@ class DecoderModel final : public StepModel {
   long long free_tokens() const override {
     return kv_cache_free_pages(d_->kv) / ((long long)d_->L * d_->H) * d_->TS;
   }
-  int forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st) override {
+  int forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st, float*) override {
     std::lock_guard<std::mutex> g(d_->mu);
     return d_->forward_mixed(batch, logits, st);
   }

@@ -112,6 +112,33 @@ struct RowCopy {
     (void)hipGetLastError();
     return true;
   }
+  // Where the head's blocks store the rows over the bus themselves, while others still read weights:
+  // pinned memory that has room for all of them, one after the other; null: nowhere.  Up to 4 MiB
+  // (us a step behind a copy and so, two layers, blocks of memory in turn: 1 row of 32,768 161 and
+  // 151, 8 rows 191 and 174, 32 rows 280 and 264; 48 rows 333 and 341, 64 rows 379 and 393: there the
+  // blocks end together, and the copy engine writes faster into pages of the host that change).
+  static constexpr size_t kMostStored = 4 << 20;
+  static float* place(float* host, const std::vector<size_t>& rows, size_t width) {
+    for (size_t r = 1; r < rows.size(); ++r)
+      if (rows[r] != rows[0] + r) return nullptr;
+    if (rows.empty() || !host || rows.size() * width * sizeof(float) > kMostStored) return nullptr;
+    float* at = host + rows[0] * width;
+    hipPointerAttribute_t is{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    const bool ok = hipPointerGetAttributes(&is, at) == hipSuccess && is.type == hipMemoryTypeHost &&
+                    is.devicePointer && reinterpret_cast<uintptr_t>(is.devicePointer) % 16 == 0 &&
+                    hipMemGetAddressRange(&base, &size, is.devicePointer) == hipSuccess &&
+                    (size_t)(static_cast<char*>(is.devicePointer) - static_cast<char*>(base)) +
+                            rows.size() * width * sizeof(float) <= size;
+    if (!ok) (void)hipGetLastError();
+    return ok ? static_cast<float*>(is.devicePointer) : nullptr;
+  }
+  // The step's own stores to the host are done.
+  int wait(bool graph, hipStream_t st) {
+    if (!graph && ring && hipEventRecord(arrived[0], st) == hipSuccess) (void)hipEventSynchronize(arrived[0]);
+    return finish(LLM_OK, st);
+  }
   // Row r of src (`width` floats each) to host row rows[r]; returns when all are there.
   // graph: they come from a step that may be a captured one.
   int copy(float* host, const std::vector<size_t>& rows, const float* src, size_t width, bool graph,
@@ -127,8 +154,7 @@ struct RowCopy {
           LLM_HIP_RET(e);
         }
       }
-      if (!graph && ring && hipEventRecord(arrived[0], st) == hipSuccess) (void)hipEventSynchronize(arrived[0]);
-      return finish(LLM_OK, st);
+      return wait(graph, st);
     }
     const size_t pieces = (total + kPiece - 1) / kPiece;
     const bool by_event = pieces > 1 || !graph;
@@ -271,10 +297,14 @@ int llm_engine::step(const llm_engine_entry* entries, int n, float* host) {
       batch[i].n_want = (int)wants[i].size();
     }
     RET_IF(ensure_logits(rows.size()));
-    RET_IF(model->forward(batch, logits.p, stream));
+    float* place = model->writes_place() ? RowCopy::place(host, rows, V) : nullptr;
+    if (const int rc = model->forward(batch, logits.p, stream, place)) {
+      if (place) (void)hipStreamSynchronize(stream);  // nothing writes there any more
+      return rc;
+    }
     bool single = true;  // one token a sequence: a decode step
     for (const StepSeq& s : batch) single = single && s.n == 1;
-    RET_IF(out.copy(host, rows, logits.p, V, single, stream));
+    RET_IF(place ? out.wait(single, stream) : out.copy(host, rows, logits.p, V, single, stream));
     for (const StepSeq& s : batch) seqs[s.slot].len = s.p0 + s.n;
     batch.clear();
     wants.clear();

@@ -532,7 +532,8 @@ void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
     });
 }
 
-int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want, hipStream_t st) {
+int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want, float* place_at,
+                           hipStream_t st) {
   // pieces of the block besides the token rows, in their places
   std::vector<std::pair<size_t, std::vector<uint8_t>>> pieces;
   size_t at = 0, part_o = 0, part_ml = 0;
@@ -554,6 +555,7 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
   at_slot_ = take((size_t)M * 4);
   at_seq0_ = take((size_t)M * 4);
   at_want_ = take((size_t)n_want * 4);
+  at_place_ = take(sizeof place_at);
   for (auto& pp : plans_) {
     Plan& p = *pp;
     for (int b = 0; b < 2; ++b) {
@@ -629,6 +631,7 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
   int32_t* slot = reinterpret_cast<int32_t*>(h_meta_ + at_slot_);
   int32_t* seq0 = reinterpret_cast<int32_t*>(h_meta_ + at_seq0_);
   int32_t* want = reinterpret_cast<int32_t*>(h_meta_ + at_want_);
+  std::memcpy(h_meta_ + at_place_, &place_at, sizeof place_at);
   int m = 0, w = 0;
   for (const StepSeq& s : batch) {
     const int first = m;
@@ -895,13 +898,14 @@ int LayerStack::enqueue(int M, int n_want, float* logits, hipStream_t st) {
   a.K = cfg_.width;
   a.w_nt = w_nt_;
   a.C = logits;
+  a.C_at = meta<float*>(at_place_);
   a.ldc = cfg_.vocab;
   a.softcap = cfg_.logit_softcap;
   LLM_HIP_RET(mm(dt_, a, st));
   return LLM_OK;
 }
 
-int LayerStack::forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st) {
+int LayerStack::forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st, float* place) {
   int M = 0, n_want = 0;
   bool decode = true;
   single_ = true;
@@ -931,7 +935,7 @@ int LayerStack::forward(const std::vector<StepSeq>& batch, float* logits, hipStr
         RET_IF(g->kv.prepare_append(s.slot, t * kPageTokens));
     RET_IF(g->kv.sync(st));
   }
-  RET_IF(build_meta(batch, M, n_want, st));
+  RET_IF(build_meta(batch, M, n_want, place, st));
   if (!use_graph_ || !decode || tap_) return enqueue(M, n_want, logits, st);
 
   std::vector<long long> key{M, (long long)reinterpret_cast<uintptr_t>(logits)};

@@ -40,7 +40,8 @@ class LayerStack final : public StepModel {
     for (const auto& g : geos_) n = std::min(n, g->kv.free_count() / ((long long)g->layers * g->G));
     return n * kPageTokens;
   }
-  int forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st) override;
+  int forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st, float* place) override;
+  bool writes_place() const override { return true; }
   int release(int slot) override;
   int layer_runs() const override { return (int)runs_.size(); }
   int width() const override { return cfg_.width; }
@@ -158,7 +159,8 @@ class LayerStack final : public StepModel {
   int pack_rows(const SafeTensors& f, const std::vector<std::pair<std::string, int>>& parts, int K,
                 const std::vector<int32_t>* map, uint8_t* dst);
   int ensure_rows(int M);
-  int build_meta(const std::vector<StepSeq>& batch, int M, int n_want, hipStream_t st);
+  int build_meta(const std::vector<StepSeq>& batch, int M, int n_want, float* place,
+                 hipStream_t st);
   void cut(const std::vector<StepSeq>& batch, Plan& p, bool big, std::vector<GqaItem>& items,
            std::vector<GqaMerge>& merges, Launch& l);
   // rows and scratch pages of the portions whose keys are expanded
@@ -221,7 +223,7 @@ class LayerStack final : public StepModel {
   uint8_t* h_meta_ = nullptr;
   size_t meta_cap_ = 0;
   hipEvent_t meta_done_ = nullptr;
-  size_t at_tok_ = 0, at_pos_ = 0, at_slot_ = 0, at_seq0_ = 0, at_want_ = 0;
+  size_t at_tok_ = 0, at_pos_ = 0, at_slot_ = 0, at_seq0_ = 0, at_want_ = 0, at_place_ = 0;
   bool single_ = false;  // every entry of the step is one token
   float* tap_ = nullptr;
 

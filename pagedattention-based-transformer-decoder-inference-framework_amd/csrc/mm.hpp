@@ -101,6 +101,7 @@ struct MmArgs {
   int M = 0, N = 0, K = 0;
   int w_nt = 0;             // weights streamed once per step (not kept in cache)
   float* C = nullptr;       // [M][ldc]
+  float* const* C_at = nullptr;  // (mm only) device word: in place of C, if it holds a pointer
   int ldc = 0;
   float softcap = 0.f;      // C = softcap tanh(C / softcap) when set
 };

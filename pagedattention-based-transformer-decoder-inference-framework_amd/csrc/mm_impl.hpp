@@ -69,6 +69,14 @@ struct KernelArgs {
   const float* bias;
 };
 
+// Where a plain product goes.  A captured head's rows have another place at every step (16 rows of
+// 32,768 logits: 26 us into device memory and a copy of 38 over the bus behind it, 51 as the
+// blocks' own stores to the host's memory).
+__device__ __forceinline__ float* stored_to(const KernelArgs& p) {
+  float* c = p.a.C_at ? *p.a.C_at : nullptr;
+  return c ? c : p.a.C;
+}
+
 __device__ __forceinline__ float glu(float gate, float up, const GluParams& p) {
   const float g = fminf(gate, p.limit);
   const float u = fminf(fmaxf(up, -p.limit), p.limit);
@@ -287,7 +295,7 @@ struct Target {
     const int m = r.m, n = c.n;
     if (m < 0 || n < 0) return;
     if constexpr (EPI == kStore) {
-      float* d = p.a.C + (size_t)m * p.a.ldc + n;
+      float* d = stored_to(p) + (size_t)m * p.a.ldc + n;
       p0 = d;
       p1 = n + 1 < b.N ? d + 1 : nullptr;
     } else if constexpr (EPI == kGroupIn) {
@@ -751,7 +759,7 @@ __device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b
       }
     }
   } else if constexpr (E == 4) {
-    float* C = EPI == kGroupOut ? p.g.out : p.a.C;
+    float* C = EPI == kGroupOut ? p.g.out : EPI == kStore ? stored_to(p) : p.a.C;
     const size_t ldc = EPI == kGroupOut ? p.g.ldo : p.a.ldc;
     const bool vec = whole<float>(C, ldc) && n + 4 <= b.N;
     float bias[4];

@@ -35,8 +35,12 @@ class StepModel {
   virtual long long free_tokens() const = 0;
   // Run the batch (all entries together, from what earlier steps left in the
   // slots) and write the wanted rows' logits, in order, to logits[rows][vocab]
-  // on the device.  At most max_step_tokens() tokens.  Enqueued on `st`.
-  virtual int forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st) = 0;
+  // on the device.  At most max_step_tokens() tokens.  Enqueued on `st`.  A model that
+  // writes_place() writes them to `place` instead, if there is one: memory for all of the rows
+  // that a kernel can write (the host's).
+  virtual int forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st,
+                      float* place = nullptr) = 0;
+  virtual bool writes_place() const { return false; }
   // Give back what the slot holds.
   virtual int release(int slot) = 0;
   // The residual stream after every layer of the next forwards, copied to the

@@ -168,3 +168,35 @@ def test_returned_rows_stay(gpu, tmp_path):
     for out, plain in held:
         assert out.flags.writeable and out.flags.c_contiguous
         np.testing.assert_array_equal(out, plain)
+
+
+@pytest.mark.parametrize("vocab", [5003, 40000])
+@pytest.mark.parametrize("rows", [1, 9, 16, 17, 33])
+def test_decode_rows_in_turns(gpu, tmp_path, rows, vocab):
+    """One captured step whose rows go to pinned memory, to pageable memory and to a buffer
+    that begins at any float, in turns: the same bytes; nothing behind the rows is written."""
+    import engine
+    import torch
+    cfg = T.config([(T.attn(), None)], vocab=vocab)
+    folder = T.save(tmp_path, cfg, T.weights(cfg, 3))
+    n = rows * vocab
+    with engine.Engine(folder, dtype="bfloat16", max_seqs=2 * rows, max_tokens=32 * 2 * rows) as e:
+        rng = np.random.default_rng(rows)
+        toks = rng.integers(0, vocab, (6, rows))
+        plain, pinned = np.empty(n, np.float32), torch.empty(n + 8, pin_memory=True)
+        want = []
+        for places in ["plain"] * 6, ["aligned", "plain", "odd", "aligned", "plain", "odd"]:
+            seqs = [e.open_seq() for _ in range(rows)]
+            for i, place in enumerate(places):
+                pinned.fill_(-7.0)
+                at = {"aligned": 0, "odd": 3}.get(place)
+                out = plain.ctypes.data if at is None else pinned.data_ptr() + 4 * at
+                step(e, [(s, [t], [0]) for s, t in zip(seqs, toks[i])], out)
+                got = (plain if at is None else pinned.numpy()[at:at + n]).copy()
+                if len(want) < 6:
+                    want.append(got)
+                np.testing.assert_array_equal(got, want[i])
+                if at is not None:
+                    assert (pinned[:at] == -7.0).all() and (pinned[at + n:] == -7.0).all()
+            for s in seqs:
+                e.close_seq(s)
