@@ -39,9 +39,8 @@ struct KvCache {
   std::vector<std::vector<int32_t>> free_lists;
   long long zone_pages = 0;
   std::vector<std::pair<int32_t, int32_t>> cow;  // (src page, dst page) copies pending
-  int64_t* d_idx = nullptr;
-  int32_t* d_val = nullptr;
-  int64_t* h_idx = nullptr;
+  bool stage(size_t n);
+  int64_t* h_idx = nullptr;  // pinned, read by the device
   int32_t* h_val = nullptr;
   size_t staging_cap = 0;
   hipEvent_t staging_done = nullptr;

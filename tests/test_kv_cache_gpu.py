@@ -70,6 +70,36 @@ def test_kv_cache_alloc_fork_cow(gpu):
         lib.kv_cache_destroy(h)
 
 
+@pytest.mark.parametrize("tiles,beams", [(1, 1), (64, 1), (64, 2), (256, 4), (512, 4), (700, 8)])
+def test_table_on_the_device(gpu, tiles, beams):
+    """Few and many changed entries (2 layers x 16 heads of 700 tiles, 8 beams), past 16,384 of
+    them too, twice: the device's table is the host's."""
+    import torch
+    import llm_capi
+    lib = llm_capi.load()
+    h = ctypes.c_void_p()
+    L, H, NT = 2, 16, 700
+    llm_capi.check(lib.kv_cache_create(L, 8, H, 16, 16, NT, L * H * beams * tiles, ctypes.byref(h)))
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    try:
+        for part in (max(tiles // 2, 1), tiles):
+            for b in range(beams):
+                llm_capi.check(lib.kv_cache_reserve(h, b, 16 * part))
+            llm_capi.check(lib.kv_cache_sync(h, None))
+            torch.cuda.synchronize()
+            for l in range(L):
+                got = np.empty((8, H, NT), np.int32)
+                assert hip.hipMemcpy(got.ctypes.data, lib.kv_cache_page_table(h, l), got.nbytes, 2) == 0
+                assert (got[:beams, :, :part] >= 0).all() and (got[:beams, :, part:] == -1).all()
+                assert (got[beams:] == -1).all()
+                for b, hh, t in [(0, 0, 0), (beams - 1, H - 1, part - 1), (beams // 2, 3, part // 2)]:
+                    assert got[b, hh, t] == lib.kv_cache_lookup(h, l, b, hh, t)
+                assert len(np.unique(got[:beams, :, :part])) == beams * H * part
+    finally:
+        lib.kv_cache_destroy(h)
+
+
 class _RefLru:
     """KVTileCache<T>::register_tile / update_lru / evict_if_needed
     (kv_cache/kv_tile_cache.cpp:64-98) restated over tile keys: which tiles
