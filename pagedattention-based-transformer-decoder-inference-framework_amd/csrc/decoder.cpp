@@ -1146,8 +1146,8 @@ extern "C" int llm_decoder_begin_synthetic(llm_decoder* d, int batch, int contex
   RET_IF(kv_cache_sync(d->kv, d->stream));
   // seeded random fp16 K/V over the whole pools (K scaled so q.k ~ O(1))
   const size_t np = (size_t)k->num_pages, pe = k->page_elems, ps = k->page_stride() / k->es;
-  LLM_HIP_RET(launch_fill_random_f16(k->k_pool, np, pe, ps, seed * 2 + 1, 0.05f, d->stream));
-  LLM_HIP_RET(launch_fill_random_f16(k->v_pool, np, pe, ps, seed * 2 + 2, 1.0f, d->stream));
+  LLM_HIP_RET(launch_fill_random_f16({k->k_pool, seed * 2 + 1, 0.05f}, {k->v_pool, seed * 2 + 2, 1.0f}, np, pe, ps,
+                                     d->stream));
   LLM_HIP_RET(hipStreamSynchronize(d->stream));
   return LLM_OK;
 }
@@ -1182,8 +1182,8 @@ extern "C" int llm_decoder_begin_beams(llm_decoder* d, int num_seqs, int beam_wi
   }
   RET_IF(kv_cache_sync(d->kv, d->stream));
   const size_t np = (size_t)k->num_pages, pe = k->page_elems, ps = k->page_stride() / k->es;
-  LLM_HIP_RET(launch_fill_random_f16(k->k_pool, np, pe, ps, seed * 2 + 1, 0.05f, d->stream));
-  LLM_HIP_RET(launch_fill_random_f16(k->v_pool, np, pe, ps, seed * 2 + 2, 1.0f, d->stream));
+  LLM_HIP_RET(launch_fill_random_f16({k->k_pool, seed * 2 + 1, 0.05f}, {k->v_pool, seed * 2 + 2, 1.0f}, np, pe, ps,
+                                     d->stream));
   LLM_HIP_RET(hipStreamSynchronize(d->stream));
   d->row_group = beam_width;
   d->graph_batch = -1;  // re-capture: the attention launch depends on row_group

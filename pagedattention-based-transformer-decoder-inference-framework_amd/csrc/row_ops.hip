@@ -342,12 +342,16 @@ __global__ void scatter_i32_kernel(int32_t* __restrict__ dst, const int64_t* __r
 // Element i of the n = pages * page_elems lands at p[(i / page_elems) *
 // page_stride + i % page_elems] (page_stride in elements: a pool whose pages
 // interleave with another pool's).
-// E values a thread, neighbours of one page: 8 where pages are whole eights, 16 bytes a store.
-// Bound by the 64-bit products (34 MB 50 us with a division for every element's place, so 28).
+// Two pools a launch (blockIdx.y).  E values a thread, neighbours of one page: 8 where pages are whole
+// eights, 16 bytes a store.  The uniforms are whole numbers of 2^-16, so their sum is one of integers.
+// Bound by the 64-bit products (2 x 34 MB 100 us with a division for every element's place, 56 with
+// the uniforms added as floats, so 31).
 template <int E>
-__global__ __launch_bounds__(256) void fill_random_f16_kernel(_Float16* __restrict__ p, size_t n,
-                                                              size_t page_elems, size_t page_stride,
-                                                              uint64_t seed, float scale) {
+__global__ __launch_bounds__(256) void fill_random_f16_kernel(RandomFill f0, RandomFill f1, size_t n,
+                                                              size_t page_elems, size_t page_stride) {
+  _Float16* p = static_cast<_Float16*>(blockIdx.y ? f1.p : f0.p);
+  const uint64_t seed = blockIdx.y ? f1.seed : f0.seed;
+  const float scale = blockIdx.y ? f1.scale : f0.scale;
   size_t i = E * ((size_t)blockIdx.x * blockDim.x + threadIdx.x);
   const size_t stride = E * (size_t)gridDim.x * blockDim.x;
   for (; i < n; i += stride) {
@@ -355,15 +359,21 @@ __global__ __launch_bounds__(256) void fill_random_f16_kernel(_Float16* __restri
     struct alignas(2 * E) {
       uint16_t x[E];
     } out;
+    constexpr uint64_t kStep = 0x9E3779B97F4A7C15ull;
+    const uint64_t z0 = seed + kStep * (i + 1);
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      uint64_t z = seed + 0x9E3779B97F4A7C15ull * (i + e + 1);
+      uint64_t z = z0 + kStep * e;
       z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
       z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
       z ^= z >> 31;
-      float u = 0.f;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) u += (float)((z >> (16 * k)) & 0xFFFF) * (1.0f / 65536.0f);
+      typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+      const u16x2 ones = {1, 1};
+      const uint32_t sum =
+          __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, (uint32_t)z), ones,
+                                 __builtin_amdgcn_udot2(__builtin_bit_cast(u16x2, (uint32_t)(z >> 32)), ones, 0u, false),
+                                 false);
+      const float u = (float)sum * (1.0f / 65536.0f);
       // (rounded once: which the compiler takes, this or a product and a conversion, would
       // depend on E)
       uint32_t h;
@@ -460,17 +470,17 @@ hipError_t launch_scatter_i32(int32_t* dst, const int64_t* idx, const int32_t* v
   return hipGetLastError();
 }
 
-hipError_t launch_fill_random_f16(void* p, size_t pages, size_t page_elems, size_t page_stride,
-                                  uint64_t seed, float scale, hipStream_t st) {
+hipError_t launch_fill_random_f16(const RandomFill& k, const RandomFill& v, size_t pages, size_t page_elems,
+                                  size_t page_stride, hipStream_t st) {
   const size_t n = pages * page_elems;
   if (n == 0) return hipSuccess;
   // (few elements: a thread each, or the chip is idle)
-  const bool eights = n >= (1u << 20) && ((page_elems | page_stride) & 7) == 0 && reinterpret_cast<uintptr_t>(p) % 16 == 0;
+  const bool eights = n >= (1u << 20) && ((page_elems | page_stride) & 7) == 0 &&
+                      (reinterpret_cast<uintptr_t>(k.p) | reinterpret_cast<uintptr_t>(v.p)) % 16 == 0;
   const size_t threads = eights ? n / 8 : n;
   const size_t blocks = std::min<size_t>((threads + 255) / 256, 65536);
   hipLaunchKernelGGL((eights ? fill_random_f16_kernel<8> : fill_random_f16_kernel<1>),
-                     dim3((unsigned)blocks), dim3(256), 0, st,
-                     static_cast<_Float16*>(p), n, page_elems, page_stride, seed, scale);
+                     dim3((unsigned)blocks, 2), dim3(256), 0, st, k, v, n, page_elems, page_stride);
   return hipGetLastError();
 }
 

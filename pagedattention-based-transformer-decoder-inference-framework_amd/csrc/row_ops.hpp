@@ -58,7 +58,12 @@ hipError_t launch_sample(const float* logits, int rows, int row0, int V, float t
                          int32_t* out, hipStream_t st);
 // Seeded uniform (variance-1 x scale) fp16 over `pages` pages of page_elems
 // elements, page p at p + p * page_stride elements.
-hipError_t launch_fill_random_f16(void* p, size_t pages, size_t page_elems, size_t page_stride,
-                                  uint64_t seed, float scale, hipStream_t st);
+struct RandomFill {  // a pool to be filled
+  void* p;
+  uint64_t seed;
+  float scale;
+};
+hipError_t launch_fill_random_f16(const RandomFill& k, const RandomFill& v, size_t pages, size_t page_elems,
+                                  size_t page_stride, hipStream_t st);
 
 }  // namespace llm

@@ -265,6 +265,34 @@ def test_greedy_tokens_of_equal_logits(gpu, oracle, rows, V, period):
         tok = [(t + b) % V for b, t in enumerate(tok)]
 
 
+@pytest.mark.parametrize("H,D,page,S", [(4, 64, 16, 40), (3, 64, 5, 77), (16, 128, 16, 600)])
+def test_synthetic_pools(gpu, H, D, page, S):
+    """begin_synthetic's pools, a value and eight values a thread: the sum of four 16-bit uniforms of
+    splitmix64, rounded once with its scale."""
+    import ctypes
+    import llm_capi
+    import llm_decoder
+    dec = llm_decoder.INT8Decoder(1, H, D, H * D, 300, S, max_batch=1, page_size=page)
+    dec.begin_synthetic(1, 3, 77, False)
+    lib, kv = llm_capi.load(), ctypes.c_void_p(dec.kv_handle)
+    pages, stride = lib.kv_cache_num_pages(kv), lib.kv_cache_page_stride(kv)
+    hip = ctypes.CDLL("libamdhip64.so")
+    hip.hipMemcpy.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int]
+    got = np.empty((pages, stride // 2), np.float16)
+    assert hip.hipMemcpy(got.ctypes.data, lib.kv_cache_k_pool(kv), got.nbytes, 2) == 0
+    n = pages * page * D
+    for at, seed, scale in (0, 155, 0.05), (page * D, 156, 1.0):
+        with np.errstate(over="ignore"):
+            z = np.uint64(seed) + np.uint64(0x9E3779B97F4A7C15) * np.arange(1, n + 1, dtype=np.uint64)
+            z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+            z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        z ^= z >> np.uint64(31)
+        u = sum(((z >> np.uint64(16 * k)) & np.uint64(0xFFFF)).astype(np.float32) for k in range(4)) / np.float32(65536)
+        x = (u - np.float32(2)) * np.float32(1.7320508)
+        want = (x.astype(np.float64) * np.float64(np.float32(scale))).astype(np.float16)
+        np.testing.assert_array_equal(got[:, at:at + page * D].reshape(-1).view(np.uint16), want.view(np.uint16))
+
+
 @pytest.mark.parametrize("rows", [1, 17, 130])
 def test_logits_places(gpu, oracle, rows):
     """The same logits wherever they go: a buffer that starts at any float, pinned host memory,
