@@ -238,6 +238,7 @@ extern "C" int llm_decoder_create(const llm_decoder_config* cfg_in, llm_decoder*
   if (hipHostMalloc(reinterpret_cast<void**>(&d->h_prompt), sizeof(int32_t) * llm_decoder::kPromptChunk,
                     hipHostMallocDefault) == hipSuccess) {
     d->h_prompt_cap = llm_decoder::kPromptChunk;
+    std::fill_n(d->h_prompt, d->h_prompt_cap, 0);  // (the host's first use of its pages)
   } else {  // no memory to pin: tokens go by copies
     d->h_prompt = nullptr;
     (void)hipGetLastError();

@@ -31,7 +31,7 @@
 
 namespace llm {
 
-// Changed entries that have pinned memory from the start, 192 KB.
+// Changed entries that have pinned memory from the start, at most 192 KB.
 constexpr size_t kScattered = 16384;
 
 // src [n][H][D] rows (element type E) for token positions pos0..pos0+n-1 of `beam`.
@@ -88,7 +88,9 @@ int KvCache::init(int L_, int beams_, int H_, int D_, int TS_, int max_tiles_, l
   refcount.assign((size_t)num_pages, 0);
   reset_free_lists();
   LLM_HIP_RET(hipEventCreateWithFlags(&staging_done, hipEventDisableTiming));
-  (void)stage(std::min<size_t>(entries, kScattered));  // (not in the first step: 170 us)
+  // (not in the first step, which it would cost 170 us; a page's first use by the host takes 2 us)
+  if (stage(std::min<size_t>(entries, kScattered)))
+    std::memset(h_idx, 0, staging_cap * (sizeof(int64_t) + sizeof(int32_t)));
   return LLM_OK;
 }
 
@@ -103,7 +105,6 @@ KvCache::~KvCache() {
   if (k_pool) (void)hipFree(k_pool);  // v_pool lives in the same allocation
   if (d_table) (void)hipFree(d_table);
   if (h_idx) (void)hipHostFree(h_idx);
-  if (h_val) (void)hipHostFree(h_val);
   if (staging_done) (void)hipEventDestroy(staging_done);
 }
 
@@ -252,17 +253,17 @@ void KvCache::release_beam(int beam) {
 // Pinned memory for n entries; false: there is none.
 bool KvCache::stage(size_t n) {
   if (n <= staging_cap) return true;
+  const size_t cap = std::max(n, 2 * staging_cap);
   if (h_idx) (void)hipHostFree(h_idx);
-  if (h_val) (void)hipHostFree(h_val);
   h_idx = nullptr;
   h_val = nullptr;
   staging_cap = 0;
-  const size_t cap = std::max(n, kScattered);
-  if (hipHostMalloc(&h_idx, cap * sizeof(int64_t), hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc(&h_val, cap * sizeof(int32_t), hipHostMallocDefault) != hipSuccess) {
+  if (hipHostMalloc(&h_idx, cap * (sizeof(int64_t) + sizeof(int32_t)), hipHostMallocDefault) != hipSuccess) {
+    h_idx = nullptr;
     (void)hipGetLastError();
     return false;
   }
+  h_val = reinterpret_cast<int32_t*>(h_idx + cap);
   staging_cap = cap;
   return true;
 }

@@ -41,7 +41,7 @@ struct KvCache {
   std::vector<std::pair<int32_t, int32_t>> cow;  // (src page, dst page) copies pending
   bool stage(size_t n);
   int64_t* h_idx = nullptr;  // pinned, read by the device
-  int32_t* h_val = nullptr;
+  int32_t* h_val = nullptr;  // behind them
   size_t staging_cap = 0;
   hipEvent_t staging_done = nullptr;
   std::mutex mu;
