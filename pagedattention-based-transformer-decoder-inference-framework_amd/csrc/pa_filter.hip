@@ -203,11 +203,13 @@ struct FilterRank {
 // A small top_k: the row's threads form 128 groups of eight; the top_k-th largest of the groups'
 // largest entries has top_k entries from it on, so that whatever stays is among those.  Where
 // they are few they are ranked one against the other, in place of the histograms (16 rows x 12
-// heads of 2048, top 64 and 0.9: 8.8 us of 30, now 3.8).  The same whole numbers.
+// heads of 2048, top 64 and 0.9: 8.8 us of 30, now 3.8).  The same whole numbers.  Its memory is the
+// histograms' too: where it finds nothing they go over it behind a barrier of its own, as a wave
+// that still read `count` would find it cleared and stay for barriers that no other meets.
 constexpr int kFewK = 64, kFew = 256, kFewGroups = kFilterThreads / 8;
 struct FilterFew {
   uint64_t key[kFew], mass[kFew];  // (probability bits, index); mass
-  float most[kFewGroups];
+  alignas(16) float most[kFewGroups];
   uint32_t index[kFew];            // of what stays; ~0: it does not
   uint64_t cut;
   float floor;
@@ -265,7 +267,10 @@ __device__ __forceinline__ int filter_few(const float* sc, int Tb, float most, u
   }
   __syncthreads();
   const float floor = few.floor;
-  if (!(floor > 0.f)) return 0;
+  if (!(floor > 0.f)) {
+    __syncthreads();
+    return 0;
+  }
   if (most >= floor)
     for (int t = tid; t < Tb; t += kFilterThreads) {
       const float p = sc[t];
@@ -278,7 +283,10 @@ __device__ __forceinline__ int filter_few(const float* sc, int Tb, float most, u
     }
   __syncthreads();
   const uint32_t n = few.count;
-  if (n > kFew) return 0;
+  if (n > kFew) {
+    __syncthreads();
+    return 0;
+  }
   // as many threads an entry as n leaves, four at least
   const int per = n <= 64 ? 16 : n <= 128 ? 8 : 4;
   const uint32_t i = (uint32_t)(tid / per);
@@ -357,12 +365,13 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   // scores, then probabilities; the sums of the values at the end
   __shared__ float lsc[FORM != kLds ? kWaves * 256 : kFilterMaxT];
   // the histograms, then the list of what stays
-  __shared__ uint64_t llist[SHORT ? sizeof(FilterRank) / 8 : WS ? sizeof(FilterHist) / 8 : kFilterMaxT];
+  __shared__ alignas(16) uint64_t llist[SHORT ? sizeof(FilterRank) / 8 : WS ? sizeof(FilterHist) / 8 : kFilterMaxT];
   __shared__ float qs[256];
   __shared__ float sh[kWaves];
   __shared__ uint64_t sh_mass[kWaves];
   __shared__ uint32_t sh_count[kWaves];
   __shared__ FilterCut found;
+  static_assert(kFewK * 8 % alignof(FilterFew) == 0 && alignof(FilterFew) <= 16);
   static_assert(sizeof(FilterRank) <= sizeof(llist) && kFewK * 8 + sizeof(FilterFew) <= sizeof(llist) &&
                     (SHORT || sizeof(FilterHist) <= sizeof(llist)),
                 "the histograms and ranks lie in the list's memory, the few behind their list");

@@ -662,3 +662,41 @@ def test_pa_decode_ex_few(gpu, oracle, kv_dtype, D, T, opt):
     assert same.any()
     assert_parity(out[same], ref[same], RTOL)
     assert_parity(probs * both, rp * both, RTOL)
+
+
+# more equal weights at the bound than are ranked one against the other: the row's cut comes from
+# the histograms, whose memory those attempts share
+@pytest.mark.parametrize("top_k", [1, 2, 63, 64])
+@pytest.mark.parametrize("T,equal", [(300, 300), (300, 257), (2048, 2048), (2048, 257), (2048, 600),
+                                     (8200, 8200), (8200, 400)])
+def test_pa_decode_ex_many_equal(gpu, oracle, T, equal, top_k):
+    import llm_capi
+    ts, B, H, D = 16, 24, 12, 64
+    nt = (T + ts - 1) // ts
+    rng = np.random.default_rng(T + equal + top_k)
+    q = np.tile((rng.standard_normal(D) * D ** -0.5).astype(np.float32), (B, H, 1))
+    # one row's pages, shared by all rows and heads: `equal` tokens of the largest score
+    k = (0.3 * rng.standard_normal((nt * ts, D))).astype(np.float16)
+    strong = rng.permutation(T)[:equal]
+    k[strong] = (q[0, 0] * (2.0 / np.linalg.norm(q[0, 0]) ** 2)).astype(np.float16)
+    k = k.reshape(nt, ts, D)
+    v = rng.standard_normal((nt, ts, D)).astype(np.float16)
+    pt = np.tile(np.arange(nt, dtype=np.int32), (B, H, 1))
+    for top_p in (1.0, 0.02):
+        opt = dict(top_k=top_k, top_p=top_p)
+        ref, rp, _ = oracle.paged_attention(q[:1, :1], k.astype(np.float32), v.astype(np.float32), pt[:1, :1], T=T,
+                                            want_probs=True, **opt)
+        out, probs, _ = llm_capi.pa_decode_ex(_dev(q), _dev(k), _dev(v), _dev(pt), T=T, want_probs=True, **opt)
+        out, probs = out.cpu().numpy(), probs.cpu().numpy()
+        # the top_k of the largest index, and of them what top_p leaves (a rounding of the reference's
+        # running sum may take one more or less)
+        want = np.sort(strong)[-min(top_k, equal):]
+        cut = (probs > 0).sum(-1)
+        assert (np.abs(cut - (rp > 0).sum()) <= (1 if top_p < 1.0 else 0)).all()
+        for b in range(B):
+            for h in range(H):
+                np.testing.assert_array_equal(np.flatnonzero(probs[b, h]), want[len(want) - cut[b, h]:])
+        assert (out == out[:1, :1]).all() and (probs == probs[:1, :1]).all()
+        if cut[0, 0] == (rp > 0).sum():
+            assert_parity(out[:1, :1], ref, RTOL)
+            assert_parity(probs[:1, :1], rp, RTOL)
