@@ -618,7 +618,7 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
       }
     }
   }
-  __syncthreads();
+  if (!n_few) __syncthreads();  // (the few end with theirs, and nothing they hold is written again)
   const auto stays = [&](int t) -> float {
     const float p = sc[t];
     const uint32_t bits = __float_as_uint(p);
@@ -656,6 +656,11 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
   const auto entry = [&](int j) -> uint64_t {
     return whole ? (uint64_t)__float_as_uint(sc[j]) << 32 | (uint32_t)j : list[j];
   };
+  // The values' sums go over the probabilities, where the loop above has its barriers behind its reads
+  // of them, or there is one below; behind the few, whose probabilities others may still be reading.
+  constexpr int kBehind = kFewK + sizeof(FilterFew) / 8;
+  static_assert(FORM != kLds || kBehind * 8 + kWaves * 256 * sizeof(float) <= sizeof(llist));
+  float* sums = FORM == kLds && n_few && !only ? reinterpret_cast<float*>(llist + kBehind) : lsc;
   const auto page_of_entry = [&](uint64_t e) { return e >> 32 ? page_of((int)(uint32_t)e) : -1; };
 
   // out = sum_t p_t v_t over present tiles (cpu_attention_kernel.cpp:103-117)
@@ -680,14 +685,14 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[e] = fmaf(p[u], kv_elem<KVT>(v[u], e), acc[e]);
     }
-    if (whole) __syncthreads();  // (the sums go over the probabilities)
-    if (w * tpw < n) {           // (the other waves' sums are not read)
+    if (whole) __syncthreads();
+    if (w * tpw < n) {  // (the other waves' sums are not read)
       for (int off = lpt; off < 64; off <<= 1)
 #pragma unroll
         for (int e = 0; e < EPL; ++e) acc[e] += __shfl_xor(acc[e], off, 64);
       if (g == 0)
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) lsc[w * D + c * EPL + e] = acc[e];
+        for (int e = 0; e < EPL; ++e) sums[w * D + c * EPL + e] = acc[e];
     }
   } else {
     // thread -> (dim d, group g of the list), groups summed in order at the end
@@ -701,13 +706,13 @@ __global__ __launch_bounds__(kFilterThreads) void pa_filter_kernel(PaFilterArgs 
         acc += __uint_as_float((uint32_t)(item >> 32)) * kv_elem<KVT>(a.v_pool, at(pg, t) + d);
       }
     if (whole) __syncthreads();
-    if (gr < G) lsc[gr * D + d] = acc;
+    if (gr < G) sums[gr * D + d] = acc;
   }
   __syncthreads();
   const int groups = lpt ? min(kWaves, (n + tpw - 1) / tpw) : kFilterThreads / D;
   if (tid < D) {
     float o = 0.f;
-    for (int i = 0; i < groups; ++i) o += lsc[i * D + tid];
+    for (int i = 0; i < groups; ++i) o += sums[i * D + tid];
     a.out[(size_t)bh * D + tid] = o;
   }
 }

@@ -700,3 +700,37 @@ def test_pa_decode_ex_many_equal(gpu, oracle, T, equal, top_k):
         if cut[0, 0] == (rp > 0).sum():
             assert_parity(out[:1, :1], ref, RTOL)
             assert_parity(probs[:1, :1], rp, RTOL)
+
+
+# the weights that stay are those of the row without a cut, to the bit, wherever the values' sums
+# come to lie (wide heads: over the weights' first half)
+@pytest.mark.parametrize("kv_dtype,D,T", [("bfloat16", 256, 8190), ("float32", 256, 4100), ("float16", 100, 8190),
+                                          ("float16", 64, 8190), ("bfloat16", 256, 8200)])
+@pytest.mark.parametrize("opt", [dict(top_k=64), dict(top_k=5, top_p=0.01), dict(top_k=64, eos_token=3000, eos_threshold=2.0)],
+                         ids=str)
+def test_pa_decode_ex_weights_to_the_bit(gpu, kv_dtype, D, T, opt):
+    import torch
+    import llm_capi
+    ts, B, H = 16, 24, 12
+    nt = (T + ts - 1) // ts
+    g = torch.Generator(device="cuda").manual_seed(T + D)
+    q = torch.randn((B, H, D), generator=g, device="cuda") * D ** -0.5
+    k, v = (torch.randn((2 * nt, ts, D), generator=g, device="cuda").to(getattr(torch, kv_dtype)) for _ in range(2))
+    pt = torch.stack([torch.randperm(2 * nt, generator=g, device="cuda")[:nt] for _ in range(B * H)]).int()
+    pt = pt.view(B, H, nt)
+    _, whole, _ = llm_capi.pa_decode_ex(q, k, v, pt, T=T, want_probs=True)
+    out, probs, _ = llm_capi.pa_decode_ex(q, k, v, pt, T=T, want_probs=True, **opt)
+    # by weight, equal ones by their index
+    key = whole.view(torch.int32).long() << 32 | torch.arange(T, device="cuda")
+    kept = (probs > 0).sum(-1, keepdim=True)
+    if opt.get("top_p", 1.0) == 1.0:
+        assert (kept == opt["top_k"]).all()
+    assert (kept > 0).all() and (kept <= opt["top_k"]).all()
+    least = key.topk(64, -1).values.gather(-1, kept - 1)
+    assert torch.equal(probs, torch.where(key >= least, whole, torch.zeros_like(whole)))
+    tokens = pt.long().repeat_interleave(ts, -1)[..., :T] * ts + torch.arange(T, device="cuda") % ts
+    index = probs.topk(64, -1)
+    rows = v.view(-1, D)[tokens.gather(-1, index.indices)].double()
+    ref = (index.values.double()[..., None] * rows).sum(-2).float()
+    assert_parity(out.cpu().numpy(), ref.cpu().numpy(), RTOL)
+
