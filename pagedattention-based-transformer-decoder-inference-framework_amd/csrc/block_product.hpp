@@ -219,6 +219,41 @@ __device__ __forceinline__ void block_product(u32x4 (&lds)[ST][2 * (MB + NB)][64
   }
 }
 
+// A strip's loads (strip_product) in the order of its code: those that a wave has issued behind A's of
+// stage `at` + 1 when it waits for these in stage `at`.  Stages behind the last whole AHEAD / 2 load no W.
+constexpr int strip_behind(int ST, int LOADS, int NT, int AHEAD, int stages, int at) {
+  int n = 0, there = 0;
+  const auto a = [&](int s, int loads) {
+    n += loads;
+    if (s == at + 1) there = n;
+  };
+  a(0, LOADS);
+  n += NT;
+  for (int s = 1; s < ST - 1; ++s) a(s, LOADS);
+  a(ST - 1, LOADS / 2);
+  n += (AHEAD - 1) * NT;
+  for (int s = 0;; ++s) {
+    const int w = s < stages / (AHEAD / 2) * (AHEAD / 2) ? NT : 0;
+    a(s + ST - 1, LOADS / 2);
+    n += w;
+    if (s == at) return n - there;
+    a(s + ST, LOADS / 2);
+    n += w;
+  }
+}
+// How many may still fly there, with W's loads in the stage and without.
+constexpr int strip_left(int ST, int LOADS, int NT, int AHEAD, bool w) {
+  return (ST - 2) * LOADS + (!w ? 0 : AHEAD < 2 * ST - 3 ? AHEAD : 2 * ST - 3) * NT;
+}
+constexpr bool strip_waits(int ST, int LOADS, int NT, int AHEAD) {
+  for (int stages = 1; stages <= 4 * AHEAD; ++stages)
+    for (int s = 0; s < stages; ++s)
+      if (strip_left(ST, LOADS, NT, AHEAD, s < stages / (AHEAD / 2) * (AHEAD / 2)) >
+          strip_behind(ST, LOADS, NT, AHEAD, stages, s))
+        return false;
+  return true;
+}
+
 // The same product by waves side by side, each of all 16 MB rows and 16 NT columns of its own:
 // a wave alone reads its columns of W, so they come from memory straight into its registers,
 // AHEAD k-steps ahead, and LDS holds A alone, ST stages of two k-steps.  Of a k-step a wave reads
@@ -240,7 +275,8 @@ __device__ __forceinline__ void strip_product(u32x4 (&lds)[ST][2 * MB][64], Acc 
                                               const A& a_at, const W& w_at, const Mma& mma) {
   constexpr int LOADS = 2 * MB / WAVES;  // of A by a wave and stage
   static_assert(2 * MB % WAVES == 0 && LOADS % 2 == 0 && MB >= 2 + LOADS / 2 && ST >= 3 &&
-                AHEAD >= 4 && AHEAD % 2 == 0 && (ST - 1) * LOADS + AHEAD * NT < 64);
+                AHEAD >= 4 && AHEAD % 2 == 0 && (ST - 1) * LOADS + AHEAD * NT < 64 &&
+                strip_waits(ST, LOADS, NT, AHEAD));
   const int lane = lane_id(), w = wave_id_uniform(), stages = KS >> 1, last = stages - 1;
   const int ar = lane & 15;  // as above
   const int at0 = 8 * ar + ((lane >> 4) ^ (ar >> 1)), at1 = at0 ^ 4;
@@ -288,7 +324,9 @@ __device__ __forceinline__ void strip_product(u32x4 (&lds)[ST][2 * MB][64], Acc 
 #pragma unroll
     for (int i = 0; i < MB; ++i) read_a(i, 0, 0);
     int slot = 0, before = ST - 1;  // of stage s, of stage s - 1
-    auto stage = [&](int s, u32x4 (&b0)[NT], u32x4 (&b1)[NT]) {
+    // tail: W is there for all stages that are left; none of it is loaded
+    auto stage = [&](auto tail, int s, u32x4 (&b0)[NT], u32x4 (&b1)[NT]) {
+      constexpr bool TAIL = decltype(tail)::value;
 #pragma unroll
       for (int i = 0; i < MB; ++i) {  // the other half of the loads into the slot that was freed last
 #pragma unroll
@@ -297,7 +335,7 @@ __device__ __forceinline__ void strip_product(u32x4 (&lds)[ST][2 * MB][64], Acc 
         if (i < LOADS / 2) load_a(s + ST - 1, before, LOADS / 2 + i, LOADS / 2 + i + 1);
         __builtin_amdgcn_sched_barrier(0);
       }
-      load_w(2 * s + AHEAD, b0);
+      if constexpr (!TAIL) load_w(2 * s + AHEAD, b0);
       __builtin_amdgcn_sched_barrier(0);
       before = slot;
       slot = slot + 1 == ST ? 0 : slot + 1;
@@ -307,9 +345,10 @@ __device__ __forceinline__ void strip_product(u32x4 (&lds)[ST][2 * MB][64], Acc 
         for (int j = 0; j < NT; ++j) acc[i][j] = mma(b1[j], a[i], acc[i][j]);
         if (i == 1) {
           // The reads of stage s are done, the wave's loads of stage s + 1 there.  Behind them it has
-          // issued stages s + 2 .. s + ST - 1 and 2 ST - 3 k-steps of W (s = 0: AHEAD, s = 1: more)
+          // issued stages s + 2 .. s + ST - 1 and 2 ST - 3 k-steps of W (s = 0: AHEAD, s = 1: more); in the
+          // tail fewer of W, of which it counts none
           __builtin_amdgcn_sched_barrier(0);
-          wait_lds_loads<(ST - 2) * LOADS + (AHEAD < 2 * ST - 3 ? AHEAD : 2 * ST - 3) * NT>();
+          wait_lds_loads<strip_left(ST, LOADS, NT, AHEAD, !TAIL)>();
           barrier_only();
           read_a(0, slot, 0);
           read_a(1, slot, 0);
@@ -319,17 +358,17 @@ __device__ __forceinline__ void strip_product(u32x4 (&lds)[ST][2 * MB][64], Acc 
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      load_w(2 * s + AHEAD + 1, b1);
+      if constexpr (!TAIL) load_w(2 * s + AHEAD + 1, b1);
       __builtin_amdgcn_sched_barrier(0);
     };
     int s = 0;
     for (; s + AHEAD / 2 <= stages; s += AHEAD / 2) {
 #pragma unroll
-      for (int i = 0; i < AHEAD / 2; ++i) stage(s + i, b[2 * i], b[2 * i + 1]);
+      for (int i = 0; i < AHEAD / 2; ++i) stage(std::false_type(), s + i, b[2 * i], b[2 * i + 1]);
     }
 #pragma unroll
     for (int i = 0; i < AHEAD / 2 - 1; ++i)
-      if (s + i < stages) stage(s + i, b[2 * i], b[2 * i + 1]);
+      if (s + i < stages) stage(std::true_type(), s + i, b[2 * i], b[2 * i + 1]);
     wait_lds_loads<0>();
     barrier_only();
   }

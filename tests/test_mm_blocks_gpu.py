@@ -63,10 +63,11 @@ def test_two_blocks_a_cu(serve, ff, rows):  # noqa: F811
 
 
 @pytest.mark.parametrize("ff,width", [(13000, 64), (13000, 96), (13000, 224), (9000, 160), (9000, 288),
-                                      (9000, 320), (9000, 448)])
+                                      (9000, 320), (9000, 384), (9000, 448), (13000, 352), (9000, 1088),
+                                      (9000, 1152)])
 def test_strips(serve, ff, width):  # noqa: F811
-    """gate and up by strips, 385 to 512 blocks of 128 x 256 or 513 to 768 of 128 x 128: one to seven stages,
-    a last k-step alone, rows and columns that end inside a block."""
+    """gate and up by strips, 385 to 512 blocks of 128 x 256 or 513 to 768 of 128 x 128: one to seven stages
+    and 17 and 18, a last k-step alone, rows and columns that end inside a block."""
     cfg = N.config([(N.latent(heads=4, dim=32, rot=16, vdim=32, rank=64), N.dense(ff=ff))], width=width)
     check(serve, cfg, N.weights(cfg, 13), "bfloat16", [[500]])
 
