@@ -1095,15 +1095,21 @@ int llm_decoder::forward_mixed(const std::vector<StepSeq>& seqs, float* logits_d
   return LLM_OK;
 }
 
-// The rows' state at start_pos and the fused o_proj's columns and flag, empty: one launch (beginning a
-// sequence 75 us with a copy or a fill for each, now 38).
+// The rows' state at start_pos and what is empty between launches (the fused o_proj's columns and
+// flag, the head's keys and counters of all `rows`), whatever became of the launches before: one
+// launch (beginning a sequence 75 us with a copy or a fill for each, now 38).
 __global__ __launch_bounds__(256) void reset_rows_kernel(int32_t* pos, int32_t* ctx, int32_t* tokens, int batch,
-                                                         int start_pos, long long* oacc, size_t columns, int* oflag) {
+                                                         int start_pos, long long* oacc, size_t columns, int* oflag,
+                                                         uint64_t* key, uint32_t* arrived, int rows) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (i < (size_t)batch) {
     pos[i] = start_pos;
     ctx[i] = start_pos + 1;
     tokens[i] = 0;
+  }
+  if (i < (size_t)rows) {
+    key[i * kChoiceStride] = 0;
+    arrived[i] = 0;
   }
   if (i < columns) oacc[i] = 0;
   if (i == 0 && oflag) *oflag = 0;
@@ -1119,13 +1125,26 @@ static int reset_rows(llm_decoder* d, int batch, int start_pos) {
   for (int b = 0; b < batch; ++b) d->h_pos[b] = start_pos;
   d->range_clamped = 0;
   const size_t columns = d->oacc.p ? d->oacc.n : 0;
-  const unsigned blocks = (unsigned)((std::max(columns, (size_t)batch) + 255) / 256);
+  const unsigned blocks = (unsigned)((std::max(columns, (size_t)d->maxB) + 255) / 256);
   hipLaunchKernelGGL(reset_rows_kernel, dim3(blocks), dim3(256), 0, nullptr, d->pos.p, d->ctx.p, d->tokens.p, batch,
-                     start_pos, d->oacc.p, columns, d->oflag.p);
+                     start_pos, d->oacc.p, columns, d->oflag.p, d->lm_key.p, d->lm_arrived.p, d->maxB);
   LLM_HIP_RET(hipGetLastError());
   LLM_HIP_RET(hipDeviceSynchronize());
   return LLM_OK;
 }
+
+#if LLM_TUNING
+// The head's words as a launch that was cut short would leave them (tests).
+extern "C" int llm_decoder_tune_head_words(llm_decoder* d, uint32_t arrived, uint64_t key) {
+  std::lock_guard<std::mutex> g(d->mu);
+  const std::vector<uint32_t> n(d->lm_arrived.n, arrived);
+  const std::vector<uint64_t> k(d->lm_key.n, key);
+  LLM_HIP_RET(hipDeviceSynchronize());
+  LLM_HIP_RET(hipMemcpy(d->lm_arrived.p, n.data(), n.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+  LLM_HIP_RET(hipMemcpy(d->lm_key.p, k.data(), k.size() * sizeof(uint64_t), hipMemcpyHostToDevice));
+  return LLM_OK;
+}
+#endif
 
 extern "C" int llm_decoder_begin_synthetic(llm_decoder* d, int batch, int context_len,
                                            uint64_t seed, int shuffle) {

@@ -309,3 +309,32 @@ def _generate_and_rerun(lib, dec):
     lib.llm_decoder_oproj_status(dec, ctypes.byref(clamped), ctypes.byref(nz))
     run = lib.llm_decoder_run_attention(dec, 0, None)
     return rc, out, (sync_rc, clamped.value, nz.value), (run, lib.llm_decoder_sync(dec))
+
+
+def _tokens_and_generate(words, lib, dec):
+    """Greedy tokens of prompts that are prefilled row by row and stepped together, on a decoder
+    whose head's words are first set as a launch that was cut short would leave them."""
+    lib.llm_decoder_generate.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
+                                         ctypes.c_int, ctypes.c_float, ctypes.c_void_p]
+    if words:
+        lib.llm_decoder_tune_head_words.argtypes = [ctypes.c_void_p, ctypes.c_uint32, ctypes.c_uint64]
+        assert lib.llm_decoder_tune_head_words(dec, *words) == 0
+    B, n_gen, plen = 3, 6, 20
+    prompts = np.arange(B * plen, dtype=np.int32).reshape(B, plen)
+    out = np.full((B, n_gen), -1, np.int32)
+    assert lib.llm_decoder_generate(dec, prompts.ctypes.data, np.full(B, plen, np.int32).ctypes.data, plen, B, n_gen,
+                                    ctypes.c_float(1.0), out.ctypes.data) == 0
+    assert lib.llm_decoder_sync(dec) == 0
+    return out
+
+
+def test_sequences_begin_with_empty_head_words(gpu):
+    """The greedy tokens are the same whatever earlier launches left in the head's keys and counters."""
+    import functools
+    import llm_capi
+    L, H, D, V, B = 2, 4, 64, 300, 3
+    w = _model(np.random.default_rng(3), L, H, D, V)
+    got = [_guard_run(llm_capi.load_tune(), w, L, H, D, V, B, 1, fuse=False,
+                      after=functools.partial(_tokens_and_generate, words))[4]
+           for words in (None, (3, 0), (0, 2 ** 63 + 7))]
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
