@@ -35,6 +35,7 @@
 #include "model.hpp"
 #include "pa_decode.hpp"
 #include "row_ops.hpp"
+#include "step_put.hpp"
 
 using namespace llm;
 
@@ -42,19 +43,6 @@ using namespace llm;
 // read and cleared (llm_decoder::report_range)
 __global__ void take_flag_kernel(int* f) { f[1] = atomicExch(f, 0); }
 
-// Up to kPut words and the place of a step's logits, out of the launch's own arguments: one launch in
-// place of copies from pageable memory before a step and of the logits' copy behind it (which a
-// captured step needs, since its own arguments are fixed).  A prompt of 113 tokens and 16 steps
-// of one row, 2 layers of hidden 256: 1,191 us, now 1,137.
-constexpr int kPut = 128;
-struct StepPut {
-  int32_t* to;
-  int32_t* to2;  // (optional) takes v2
-  float** place; // (optional) takes logits
-  float* logits;
-  int n;
-  int32_t v2, v[kPut];
-};
 __global__ __launch_bounds__(kPut) void step_put_kernel(StepPut a) {
   const int i = threadIdx.x;
   if (i < a.n) a.to[i] = a.v[i];
@@ -846,19 +834,12 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
   }
   const bool sample = temperature > 0.f && top_k != 1;
   const bool direct = logits_dev && !sample && kernel_writes(logits_dev, sizeof(float) * batch * V);
-  if (tokens_host || direct || logits_set) {
-    for (int b0 = 0; b0 == 0 || (tokens_host && b0 < batch); b0 += kPut) {
-      StepPut a{};
-      a.to = tokens.p + b0;
-      a.n = tokens_host ? std::min(kPut, batch - b0) : 0;
-      std::copy_n(tokens_host + b0, a.n, a.v);
-      if (b0 == 0) a.place = logits_at.p;
-      a.logits = direct ? logits_dev : nullptr;
-      hipLaunchKernelGGL(step_put_kernel, dim3(1), dim3(kPut), 0, st, a);
-      LLM_HIP_RET(hipGetLastError());
-    }
-    logits_set = direct;
-  }
+  RET_IF(put_step(tokens_host, batch, tokens.p, logits_at.p, direct ? logits_dev : nullptr, logits_set,
+                  [&](const StepPut& a) -> int {
+                    hipLaunchKernelGGL(step_put_kernel, dim3(1), dim3(kPut), 0, st, a);
+                    LLM_HIP_RET(hipGetLastError());
+                    return LLM_OK;
+                  }));
   if (!use_graph) {
     RET_IF(enqueue_step(st));
   } else {
