@@ -164,11 +164,11 @@ struct llm_decoder {
   int layer_post(int l, hipStream_t st, const struct Rows& R);
   struct Rows step_rows(int r0, int n, uint8_t* ws);
   void embed_rows(const int32_t* tok);
-  int step_tail(hipStream_t st, int r0, int n);
+  int step_tail(hipStream_t st, int r0, int n, float* const* place, float* to);
   int next_tokens(const float* xr, int n, int r0, const int32_t* ctr, hipStream_t st,
                   int32_t* adv_pos = nullptr, int32_t* adv_ctx = nullptr,
-                  float* const* place = nullptr);
-  int enqueue_step(hipStream_t st);
+                  float* const* place = nullptr, float* to = nullptr);
+  int enqueue_step(hipStream_t st, float* const* place, float* to);
   int run_step(const int32_t* tokens_host, float* logits_dev, int32_t* next_host, hipStream_t st);
 
   // chunked prefill (llm_decoder_prefill): buffers for one chunk of tokens.  Mixed
@@ -740,15 +740,15 @@ int llm_decoder::tap(int l, int stage, const Rows& R, int K, hipStream_t st) {
   return LLM_OK;
 }
 
-// LM head + token choice for rows r0.. (x rows given): logits into the step's
-// logits buffer; greedy ids from the LM head's fused argmax partials, or a
+// LM head + token choice for rows r0.. (x rows given): logits to `to` (greedy
+// rows; null: the step's logits buffer) or where `place` says; greedy ids from the LM head's fused argmax partials, or a
 // device draw (sample_rows) with the rows' positions as draw counters.
 // adv_pos / adv_ctx (optional): advance the rows' positions afterwards (fused
 // into the argmax launch; a launch of its own after a draw, which reads them).
 int llm_decoder::next_tokens(const float* xr, int n, int r0, const int32_t* ctr, hipStream_t st,
-                             int32_t* adv_pos, int32_t* adv_ctx, float* const* place) {
-  float* lg = logits.p + (size_t)r0 * V;
+                             int32_t* adv_pos, int32_t* adv_ctx, float* const* place, float* to) {
   const bool sample = temperature > 0.f && top_k != 1;
+  float* lg = to && !sample ? to : logits.p + (size_t)r0 * V;
   float* pv = lm_pv.p + (size_t)r0 * lm_nwg;
   int32_t* pi = lm_pi.p + (size_t)r0 * lm_nwg;
   if (!sample && lm_head_chooses(n, hid)) {
@@ -780,13 +780,13 @@ void llm_decoder::embed_rows(const int32_t* tok) {
   embed_src.V = V;
 }
 
-int llm_decoder::step_tail(hipStream_t st, int r0, int n) {
+int llm_decoder::step_tail(hipStream_t st, int r0, int n, float* const* place, float* to) {
   return next_tokens(x.p + (size_t)r0 * hid, n, r0, pos.p + r0, st, pos.p + r0, ctx.p + r0,
-                     logits_at.p);
+                     place, to);
 }
 
 // One decode step of all active rows (captured into the step graph).
-int llm_decoder::enqueue_step(hipStream_t st) {
+int llm_decoder::enqueue_step(hipStream_t st, float* const* place, float* to) {
   Rows R = step_rows(0, batch, attn_ws.p);
   if (oproj_fusable(R)) R.oacc = oacc.p, R.oproj_out = R.x, R.oflag = oflag.p;
   R.wgm_quant = wgm_quant_ok(R);
@@ -796,7 +796,7 @@ int llm_decoder::enqueue_step(hipStream_t st) {
     RET_IF(layer_attn(l, st, R));
     RET_IF(layer_post(l, st, R));
   }
-  return step_tail(st, 0, batch);
+  return step_tail(st, 0, batch, place, to);
 }
 
 // Memory of the current device that a kernel can write `bytes` of as floats; what is not (other
@@ -834,21 +834,24 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
   }
   const bool sample = temperature > 0.f && top_k != 1;
   const bool direct = logits_dev && !sample && kernel_writes(logits_dev, sizeof(float) * batch * V);
-  RET_IF(put_step(tokens_host, batch, tokens.p, logits_at.p, direct ? logits_dev : nullptr, logits_set,
+  // The place comes with a step of the decoder's own graph; a step by launches has it in its arguments, so
+  // that a program that captured some does not write where a later step's logits went.
+  float* to = direct ? logits_dev : nullptr;
+  RET_IF(put_step(tokens_host, batch, tokens.p, logits_at.p, use_graph ? to : nullptr, logits_set,
                   [&](const StepPut& a) -> int {
                     hipLaunchKernelGGL(step_put_kernel, dim3(1), dim3(kPut), 0, st, a);
                     LLM_HIP_RET(hipGetLastError());
                     return LLM_OK;
                   }));
   if (!use_graph) {
-    RET_IF(enqueue_step(st));
+    RET_IF(enqueue_step(st, nullptr, to));
   } else {
     if (graph_batch != batch) {
       if (graph) { (void)hipGraphExecDestroy(graph); graph = nullptr; }
       hipGraph_t g;
       LLM_HIP_RET(hipStreamSynchronize(st));
       LLM_HIP_RET(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      int rc = enqueue_step(stream);
+      int rc = enqueue_step(stream, logits_at.p, nullptr);
       hipError_t e = hipStreamEndCapture(stream, &g);
       if (rc) return rc;
       if (e != hipSuccess)

@@ -321,6 +321,44 @@ def test_logits_places(gpu, oracle, rows):
             assert torch.equal(place.cpu(), want[i].cpu().reshape(-1))
 
 
+def test_captured_steps_leave_other_logits_alone(gpu, oracle, monkeypatch):
+    """Steps by launches (LLM_GRAPH=0) that a program captures: one without logits writes none, one
+    with logits writes its own, whatever places the steps between the replays had."""
+    torch = _torch()
+    monkeypatch.setenv("LLM_GRAPH", "0")
+    rows, V = 2, 300
+    w = _int8_model(oracle, L=1, H=2, D=64, V=V, S=32, seed=9)
+    dec = _make_gpu_decoder(w, max_batch=rows)
+    own, other = torch.zeros((2, rows, V), device="cuda")
+    want = torch.empty((2, rows, V), device="cuda")
+    dec.begin_synthetic(rows, 0, 0, False)  # (one page of 16 tokens)
+    for i in range(2):
+        dec.step([3, 4] if i else [1, 2], logits_ptr=want[i].data_ptr())
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    graphs = []
+    for logits in (0, own.data_ptr()):
+        dec.begin_synthetic(rows, 0, 0, False)
+        dec.step([1, 2])
+        graphs.append(torch.cuda.CUDAGraph())
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graphs[-1], stream=stream):
+            dec.step([3, 4], logits, stream.cuda_stream, False)
+    for logits in (other.data_ptr(), 0):
+        for g in graphs:
+            dec.begin_synthetic(rows, 0, 0, False)
+            dec.step([1, 2], logits_ptr=logits)
+            torch.cuda.synchronize()
+            if logits:
+                assert torch.equal(other, want[0])
+            own.fill_(-7.0)
+            other.fill_(-7.0)
+            g.replay()
+            torch.cuda.synchronize()
+            assert (other == -7.0).all()
+            assert torch.equal(own, want[1]) if g is graphs[1] else (own == -7.0).all()
+
+
 def test_generate_call_forms(gpu, oracle):
     w = _int8_model(oracle, L=1, H=2, D=64, V=300, S=48, seed=3)
     dec = _make_gpu_decoder(w, max_batch=4)
