@@ -20,43 +20,70 @@ struct Block {
   char* p = nullptr;
   size_t size = 0;
   bool lent = false;
+  uint64_t used = 0;  // the last take while it was lent
 };
 
 struct Pool {
   static constexpr size_t kMost = (size_t)64 << 20;     // all blocks, lent or free
   static constexpr size_t kAhead = (size_t)8 << 20;     // a block made with an engine
   static constexpr size_t kUnit = (size_t)256 << 10;
+  // A free block makes room for another after that many takes without it: results of two sizes in
+  // turn, which do not both fit, would else free and pin a block at every step (60 MiB: 30 us and 15
+  // to 900).  The one without a block takes memory of its own.
+  static constexpr uint64_t kIdle = 64;
   std::mutex mu;
   std::vector<Block> blocks;
-  size_t total = 0;
+  size_t total = 0;  // of blocks, and of those being made
+  uint64_t takes = 0;
   int engines = 0;
 
-  // Free blocks of up to 4 times the size, so that small results do not hold large blocks.
+  static bool fits(const Block& b, size_t bytes) {
+    // (up to 4 times the size, so that small results do not hold large blocks)
+    return !b.lent && b.size >= bytes && b.size <= 4 * bytes + kUnit;
+  }
   Block* find(size_t bytes) {
     Block* best = nullptr;
     for (Block& b : blocks)
-      if (!b.lent && b.size >= bytes && b.size <= 4 * bytes + kUnit && (!best || b.size < best->size)) best = &b;
+      if (fits(b, bytes) && (!best || b.size < best->size)) best = &b;
     return best;
   }
-  void drop(size_t i) {
-    (void)hipHostFree(blocks[i].p);
+  char* remove(size_t i) {
+    char* p = blocks[i].p;
     total -= blocks[i].size;
     blocks.erase(blocks.begin() + i);
+    return p;
   }
-  Block* make(size_t bytes) {
+  bool idle(const Block& b) const { return !b.lent && takes - b.used >= kIdle; }
+  // A new block; null: there is no room or none to pin.  `mu` is not held while memory is pinned or
+  // given back, so that nobody's take or give waits for it.
+  char* make(size_t bytes, bool lent, std::unique_lock<std::mutex>& lock) {
     const size_t size = (bytes + kUnit - 1) / kUnit * kUnit;
-    for (size_t i = blocks.size(); i-- > 0 && total + size > kMost;)
-      if (!blocks[i].lent) drop(i);
-    if (total + size > kMost) return nullptr;
-    Block b;
-    if (hipHostMalloc(reinterpret_cast<void**>(&b.p), size, hipHostMallocDefault) != hipSuccess) {
+    size_t free = 0;
+    for (const Block& b : blocks) free += idle(b) ? b.size : 0;
+    if (total - free + size > kMost) return nullptr;
+    std::vector<char*> out;
+    while (total + size > kMost) {
+      size_t oldest = blocks.size();
+      for (size_t i = 0; i < blocks.size(); ++i)
+        if (idle(blocks[i]) && (oldest == blocks.size() || blocks[i].used < blocks[oldest].used)) oldest = i;
+      out.push_back(remove(oldest));
+    }
+    total += size;
+    lock.unlock();
+    for (char* p : out) (void)hipHostFree(p);
+    void* p = nullptr;
+    if (hipHostMalloc(&p, size, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
+      p = nullptr;
+    }
+    if (p && !lent) std::memset(p, 0, size);  // the host's first touch of a page costs 1.5 us
+    lock.lock();
+    if (!p) {
+      total -= size;
       return nullptr;
     }
-    b.size = size;
-    total += size;
-    blocks.push_back(b);
-    return &blocks.back();
+    blocks.push_back({static_cast<char*>(p), size, lent, takes});
+    return static_cast<char*>(p);
   }
 };
 Pool& pool() {
@@ -66,28 +93,28 @@ Pool& pool() {
 
 }  // namespace
 
-// Two blocks: a caller holds one step's rows while the next one runs.  The host's first touch
-// of a page costs 1.5 us.
+// Two blocks: a caller holds one step's rows while the next one runs.
 void host_rows_engine_begins(size_t bytes) {
   Pool& p = pool();
-  std::lock_guard<std::mutex> g(p.mu);
+  std::unique_lock<std::mutex> lock(p.mu);
   ++p.engines;
   if (bytes > Pool::kAhead) return;
   int ready = 0;
-  for (const Block& b : p.blocks) ready += !b.lent && b.size >= bytes && b.size <= 4 * bytes + Pool::kUnit;
-  for (; ready < 2; ++ready) {
-    Block* b = p.make(bytes);
-    if (!b) return;
-    std::memset(b->p, 0, b->size);
-  }
+  for (const Block& b : p.blocks) ready += Pool::fits(b, bytes);
+  for (; ready < 2; ++ready)
+    if (!p.make(bytes, false, lock)) return;
 }
 
 void host_rows_engine_ends() {
   Pool& p = pool();
-  std::lock_guard<std::mutex> g(p.mu);
-  if (--p.engines > 0) return;
-  for (size_t i = p.blocks.size(); i-- > 0;)
-    if (!p.blocks[i].lent) p.drop(i);
+  std::vector<char*> out;
+  {
+    std::lock_guard<std::mutex> g(p.mu);
+    if (--p.engines > 0) return;
+    for (size_t i = p.blocks.size(); i-- > 0;)
+      if (!p.blocks[i].lent) out.push_back(p.remove(i));
+  }
+  for (char* b : out) (void)hipHostFree(b);
 }
 
 }  // namespace llm
@@ -96,22 +123,28 @@ using namespace llm;
 
 extern "C" void* llm_host_rows_take(size_t bytes) {
   Pool& p = pool();
-  std::lock_guard<std::mutex> g(p.mu);
-  if (p.engines == 0 || bytes == 0) return nullptr;
-  Block* b = p.find(bytes);
-  if (!b) b = p.make(bytes);
-  if (!b) return nullptr;
-  b->lent = true;
-  return b->p;
+  std::unique_lock<std::mutex> lock(p.mu);
+  if (p.engines == 0 || bytes == 0 || bytes > Pool::kMost) return nullptr;
+  ++p.takes;
+  if (Block* b = p.find(bytes)) {
+    b->lent = true;
+    b->used = p.takes;
+    return b->p;
+  }
+  return p.make(bytes, true, lock);
 }
 
 extern "C" void llm_host_rows_give(void* at) {
   Pool& p = pool();
-  std::lock_guard<std::mutex> g(p.mu);
-  for (size_t i = 0; i < p.blocks.size(); ++i)
-    if (p.blocks[i].p == at && p.blocks[i].lent) {
-      p.blocks[i].lent = false;
-      if (p.engines == 0) p.drop(i);
-      return;
-    }
+  {
+    std::lock_guard<std::mutex> g(p.mu);
+    size_t i = 0;
+    while (i < p.blocks.size() && !(p.blocks[i].p == at && p.blocks[i].lent)) ++i;
+    if (i == p.blocks.size()) return;
+    p.blocks[i].lent = false;
+    p.blocks[i].used = p.takes;
+    if (p.engines > 0) return;
+    (void)p.remove(i);
+  }
+  (void)hipHostFree(at);
 }

@@ -51,3 +51,67 @@ int main() {
 }
 """)
     assert out == ["ok"]
+
+
+def test_pinned_rows_of_two_sizes_in_turns(tmp_path):
+    """Results that do not fit the pool together: no block is pinned or given back at every step, the
+    bound holds, and sizes that are no longer asked for make room."""
+    out = run(tmp_path, """
+#include <atomic>
+#include <cstdio>
+#include <cstdlib>
+#include <thread>
+#include <hip/hip_runtime.h>
+#include "host_rows.hpp"
+#include "llm_decoder.h"
+std::atomic<int> pinned{0}, given{0};
+extern "C" hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  ++pinned;
+  *p = std::malloc(n);
+  return hipSuccess;
+}
+extern "C" hipError_t hipHostFree(void* p) {
+  ++given;
+  std::free(p);
+  return hipSuccess;
+}
+extern "C" hipError_t hipGetLastError() { return hipSuccess; }
+const size_t MB = 1 << 20;
+int turns(size_t a, size_t b, int n) {
+  int none = 0;
+  for (int i = 0; i < n; ++i)
+    for (size_t bytes : {a, b}) {
+      void* p = llm_host_rows_take(bytes);
+      none += !p;
+      llm_host_rows_give(p);
+    }
+  return none;
+}
+int main() {
+  if (llm_host_rows_take(MB)) return 1;  // no engine
+  llm::host_rows_engine_begins(8 * MB);
+  if (pinned != 2) return 2;
+  const int none = turns(60 * MB, 10 * MB, 400);
+  if (pinned + given > 2 + 20 || none < 300 || none > 500) return 3;
+  const int before = pinned;
+  if (turns(10 * MB, 12 * MB, 400) > 200 || pinned - before > 3) return 4;  // 60 MiB made room
+  if (turns(4 * MB, 14 * MB, 400) > 200) return 5;
+  void* held[80];
+  for (void*& p : held) p = llm_host_rows_take(MB);  // 64 MiB at most
+  int have = 0;
+  for (void* p : held) have += p != nullptr;
+  if (have > 64 || have < 16) return 6;
+  std::thread t[4];
+  for (std::thread& x : t)
+    x = std::thread([] {
+      for (int i = 0; i < 500; ++i) llm_host_rows_give(llm_host_rows_take((1 + i % 7) * MB));
+    });
+  for (std::thread& x : t) x.join();
+  llm::host_rows_engine_ends();
+  if (pinned - given != have) return 7;
+  for (void* p : held) llm_host_rows_give(p);
+  if (pinned != given) return 8;
+  std::puts("ok");
+}
+""", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-Wno-error", "-pthread", str(CSRC / "host_rows.cpp"))
+    assert out == ["ok"]
