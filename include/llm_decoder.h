@@ -567,6 +567,8 @@ int llm_engine_step(llm_engine* e, const llm_engine_entry* entries, int n, float
  * the engine's end, when nothing reads it any more. */
 void* llm_host_rows_take(size_t bytes);
 void llm_host_rows_give(void* at);
+/* The bytes at `at`, if llm_host_rows_take gave it and it was not given back; else 0. */
+size_t llm_host_rows_held(const void* at);
 /* The residual stream after every layer run of each following step of at most
  * max_step_tokens tokens: tap, host [layer runs][tokens][width]; NULL: off. */
 int llm_engine_set_tap(llm_engine* e, float* tap);

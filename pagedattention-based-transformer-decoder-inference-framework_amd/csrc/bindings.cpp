@@ -20,14 +20,21 @@
 // Errors: any non-zero C-ABI status raises RuntimeError with llm_last_error().
 // The GIL is released around device work; each decoder serialises its own
 // calls with an internal mutex (KVTileCache's std::mutex, kv_tile_cache.hpp:73).
+#define NPY_NO_DEPRECATED_API NPY_1_22_API_VERSION
+#define NPY_TARGET_VERSION NPY_1_22_API_VERSION
+#include <numpy/arrayobject.h>
 #include <pybind11/numpy.h>
 #include <pybind11/pybind11.h>
 #include <pybind11/stl.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <cstdlib>
+#include <cstring>
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "llm_decoder.h"
@@ -85,6 +92,54 @@ bool append_int32s(PyObject* o, std::vector<int32_t>& pool) {
   return ok;
 }
 
+// numpy's handler of arrays whose rows lie in pinned memory: they own it as other arrays do theirs
+// (resize in place takes memory of the host's).
+struct PinnedRows {
+  static inline thread_local void* next = nullptr;  // what the next array takes
+  static void* take(void*, size_t n) { return next ? std::exchange(next, nullptr) : std::malloc(n); }
+  static void* take_zeroed(void*, size_t n, size_t size) { return std::calloc(n, size); }
+  static void give(void*, void* p, size_t) {
+    if (llm_host_rows_held(p)) llm_host_rows_give(p);
+    else std::free(p);
+  }
+  static void* resize(void*, void* p, size_t n) {
+    const size_t held = llm_host_rows_held(p);
+    if (!held) return std::realloc(p, n);
+    void* to = std::malloc(n);
+    if (!to) return nullptr;
+    std::memcpy(to, p, std::min(held, n));
+    llm_host_rows_give(p);
+    return to;
+  }
+  static PyObject* handler() {
+    static PyDataMem_Handler h = {"llm_decoder rows", 1, {nullptr, take, take_zeroed, resize, give}};
+    static PyObject* capsule = nullptr;
+    if (!capsule && _import_array() == 0) capsule = PyCapsule_New(&h, "mem_handler", nullptr);
+    return capsule;
+  }
+  // An array over `at`, which llm_host_rows_take gave.
+  static py::array_t<float> array(void* at, py::ssize_t rows, py::ssize_t width) {
+    struct Scope {
+      PyObject* before;
+      explicit Scope(void* at) : before(nullptr) {
+        next = at;
+        if (PyObject* h = handler()) before = PyDataMem_SetHandler(h);
+      }
+      ~Scope() {
+        if (next) llm_host_rows_give(std::exchange(next, nullptr));
+        if (!before) return;
+        PyObject *type, *value, *trace;  // (an error on its way stays)
+        PyErr_Fetch(&type, &value, &trace);
+        Py_XDECREF(PyDataMem_SetHandler(before));
+        Py_DECREF(before);
+        PyErr_Restore(type, value, trace);
+      }
+    } scope(at);
+    if (!scope.before) throw py::error_already_set();
+    return py::array_t<float>({rows, width});
+  }
+};
+
 // llm_engine_step (the function at `step`, of the library the engine is from) over
 // [(seq, tokens, want)]: (status, logits), or None for entries that are not tuples of an int
 // and two lists of int32.  64 entries of one token 9 us; built in Python 71.
@@ -124,13 +179,7 @@ py::object engine_step(uintptr_t step, uintptr_t engine, py::handle entries, int
     py::gil_scoped_release nogil;
     to = static_cast<float*>(llm_host_rows_take(bytes));
   }
-  py::array_t<float> logits = [&] {
-    if (!to) return py::array_t<float>({rows, (py::ssize_t)vocab});
-    std::unique_ptr<float, void (*)(void*)> own(to, llm_host_rows_give);
-    py::capsule base(to, llm_host_rows_give);
-    own.release();
-    return py::array_t<float>({rows, (py::ssize_t)vocab}, to, base);
-  }();
+  py::array_t<float> logits = to ? PinnedRows::array(to, rows, vocab) : py::array_t<float>({rows, (py::ssize_t)vocab});
   if (!to && rows) to = logits.mutable_data();
   int rc;
   {

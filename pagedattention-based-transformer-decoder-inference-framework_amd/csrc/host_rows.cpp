@@ -134,6 +134,14 @@ extern "C" void* llm_host_rows_take(size_t bytes) {
   return p.make(bytes, true, lock);
 }
 
+extern "C" size_t llm_host_rows_held(const void* at) {
+  Pool& p = pool();
+  std::lock_guard<std::mutex> g(p.mu);
+  for (const Block& b : p.blocks)
+    if (b.p == at && b.lent) return b.size;
+  return 0;
+}
+
 extern "C" void llm_host_rows_give(void* at) {
   Pool& p = pool();
   {

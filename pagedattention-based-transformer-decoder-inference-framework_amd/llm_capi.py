@@ -150,6 +150,7 @@ _SIGS = {
     "llm_engine_step": (c_int, [c_void_p, ctypes.POINTER(EngineEntry), c_int, c_void_p]),
     "llm_host_rows_take": (c_void_p, [c_size_t]),
     "llm_host_rows_give": (None, [c_void_p]),
+    "llm_host_rows_held": (c_size_t, [c_void_p]),
     "llm_engine_set_tap": (c_int, [c_void_p, c_void_p]),
     "llm_engine_layer_runs": (c_int, [c_void_p]),
     "llm_engine_width": (c_int, [c_void_p]),

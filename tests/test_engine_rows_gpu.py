@@ -200,3 +200,27 @@ def test_decode_rows_in_turns(gpu, tmp_path, rows, vocab):
                     assert (pinned[:at] == -7.0).all() and (pinned[at + n:] == -7.0).all()
             for s in seqs:
                 e.close_seq(s)
+
+
+def test_returned_rows_resize_in_place(gpu, tmp_path):
+    """A step's array owns its rows, in pinned memory or not: it resizes in place, grows and shrinks,
+    and later steps' rows are theirs."""
+    import engine
+    cfg = T.config([(T.attn(), None)], vocab=5003)
+    with engine.Engine(T.save(tmp_path, cfg, T.weights(cfg, 3)), dtype="float32", max_seqs=2, max_tokens=512) as e:
+        for n in (3, 4, 60):  # 60,036 and 80,048 bytes; 1.2 MB
+            outs = []
+            for _ in range(3):
+                s = e.open_seq()
+                outs.append(e.step([(s, np.arange(n), list(range(n)))]))
+                e.close_seq(s)
+            want = outs[0].copy()
+            assert outs[0].flags.owndata and outs[0].base is None
+            outs[0].resize((2 * n, e.vocab), refcheck=False)
+            outs[1].resize((n - 2, e.vocab), refcheck=False)
+            outs[1].resize((n - 1, e.vocab), refcheck=False)
+            np.testing.assert_array_equal(outs[0][:n], want)
+            assert not outs[0][n:].any() and not outs[1][n - 2:].any()
+            np.testing.assert_array_equal(outs[1][:n - 2], want[:n - 2])
+            np.testing.assert_array_equal(outs[2], want)
+            assert np.zeros(100000).flags.owndata  # (other arrays are as ever)
