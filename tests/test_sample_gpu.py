@@ -124,3 +124,19 @@ def test_short_rows(gpu, V, k):
         ref, margin = sample_rows(logits, 0.8, k, p, seed=5, counter=k)
         got = draw(logits, 0.8, k, p, k)
         assert ((got == ref) | (margin < 1e-4)).all(), (got, ref, margin)
+
+
+def test_exp_below_is_expf(gpu):
+    """The sampler's exponential (tuning build) has expf's bits for every number that is not
+    positive, minus infinity and NaN among them."""
+    import ctypes
+    import torch
+    import llm_capi
+    lib = llm_capi.load_tune()
+    lib.exp_below_differs.argtypes = [ctypes.c_uint32, ctypes.c_uint, ctypes.c_void_p, ctypes.c_void_p]
+    differ = torch.zeros(2, dtype=torch.int32, device="cuda")
+    # 2^31 patterns with a sign; 0 and what comes with it in a workgroup, so small that it is 1; NaN
+    for first, blocks in ((0x80000000, 1 << 23), (0, 1), (0x7F800001, (0x7FFFFFFF - 0x7F800001) // 256)):
+        llm_capi.check(lib.exp_below_differs(first, blocks, differ.data_ptr(), None), lib)
+        torch.cuda.synchronize()
+        assert differ.tolist() == [0, 0], (hex(first), [hex(x & 0xFFFFFFFF) for x in differ.tolist()])
