@@ -170,9 +170,10 @@ def test_returned_rows_stay(gpu, tmp_path):
         np.testing.assert_array_equal(out, plain)
 
 
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("vocab", [5003, 40000])
 @pytest.mark.parametrize("rows", [1, 9, 16, 17, 33])
-def test_decode_rows_in_turns(gpu, tmp_path, rows, vocab):
+def test_decode_rows_in_turns(gpu, tmp_path, rows, vocab, dtype):
     """One captured step whose rows go to pinned memory, to pageable memory and to a buffer
     that begins at any float, in turns: the same bytes; nothing behind the rows is written."""
     import engine
@@ -180,7 +181,7 @@ def test_decode_rows_in_turns(gpu, tmp_path, rows, vocab):
     cfg = T.config([(T.attn(), None)], vocab=vocab)
     folder = T.save(tmp_path, cfg, T.weights(cfg, 3))
     n = rows * vocab
-    with engine.Engine(folder, dtype="bfloat16", max_seqs=2 * rows, max_tokens=32 * 2 * rows) as e:
+    with engine.Engine(folder, dtype=dtype, max_seqs=2 * rows, max_tokens=32 * 2 * rows) as e:
         rng = np.random.default_rng(rows)
         toks = rng.integers(0, vocab, (6, rows))
         plain, pinned = np.empty(n, np.float32), torch.empty(n + 8, pin_memory=True)
