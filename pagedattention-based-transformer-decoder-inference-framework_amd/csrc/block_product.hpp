@@ -263,9 +263,9 @@ constexpr bool strip_waits(int ST, int LOADS, int NT, int AHEAD) {
 // next k-step right behind its last product.  Sums are added in the order of the form above:
 // the same bits.
 // Amid a model, its code cold: 2011 x 12288 x 2048 bf16 with its activation 100 us, now
-// 87; 2011 x 2048 x 2048 to 6144 40, 34; 32 experts' gate and up of 2048 tokens 146, 131.  Of the matrix
-// cores' time while a CU is busy 54 % were used, now 73, at the clock that the card's power leaves
-// (1.95 GHz; the products alone, out of registers, reach 2.0 PFLOP/s).
+// 87; 2011 x 2048 x 2048 to 6144 40, 34; 32 experts' gate and up of 2048 tokens 146, 131.  The first
+// uses the matrix cores for 62 % of the time that a CU is busy, at 1.85 GHz (kernels without products
+// run at 2.3 to 2.4; products alone, out of registers, reach 2.0 PFLOP/s).
 // AHEAD k-steps of W: the compiler waits for them as if A's loads between were none, so that 4 are
 // 2 and 8 are 3.5; 128 x 128 alone on a CU needs the 8 (2011 x 2048 x 6144 58.7 us, 53.1), 128 x 256 has
 // registers for 4.
