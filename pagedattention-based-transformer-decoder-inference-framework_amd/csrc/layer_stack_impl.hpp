@@ -130,9 +130,9 @@ class LayerStack final : public StepModel {
              Dp == o.Dp && Dv == o.Dv && Dvp == o.Dvp;
     }
   };
-  // Layers whose scans take chunks of one size.
+  // Layers whose scans have as many channels and states.
   struct ScanPlan {
-    int chunk = 0;
+    int inner = 0, state = 0;
     int n_items = 0, n_chunks = 0, n_carry = 0, parts = 0;
     size_t items_at = 0, chunks_at = 0, carry_at = 0;
   };

@@ -17,13 +17,13 @@ namespace llm {
 int LayerStack::init_mamba(Layer& l) {
   const MambaSpec& m = l.s.mamba;
   const int ldc = mm_pad(m.inner);
-  const int chunk = scan_chunk(m.state);
   int k = 0;
   for (; k < (int)scans_.size(); ++k)
-    if (scans_[k].chunk == chunk) break;
+    if (scans_[k].inner == m.inner && scans_[k].state == m.state) break;
   if (k == (int)scans_.size()) {
     scans_.emplace_back();
-    scans_.back().chunk = chunk;
+    scans_.back().inner = m.inner;
+    scans_.back().state = m.state;
   }
   l.scan = k;
   ld_xz_ = std::max(ld_xz_, 2 * ldc);
@@ -70,13 +70,15 @@ void LayerStack::plan_scan(const std::vector<StepSeq>& batch, ScanPlan& p,
                            std::vector<ScanItem>& items, std::vector<ScanItem>& chunks,
                            std::vector<ScanCarry>& carry) {
   p.parts = 0;
-  int seq0 = 0;
+  int seq0 = 0, tokens = 0;
+  for (const StepSeq& s : batch) tokens += s.n;
+  const int chunk = scan_chunk(p.inner, p.state, tokens);
   for (const StepSeq& s : batch) {
-    const int n = (s.n + p.chunk - 1) / p.chunk;
+    const int n = (s.n + chunk - 1) / chunk;
     for (int k = 0; k < n; ++k) {
       ScanItem it;
-      it.tok0 = seq0 + k * p.chunk;
-      it.n = std::min(p.chunk, s.n - k * p.chunk);
+      it.tok0 = seq0 + k * chunk;
+      it.n = std::min(chunk, s.n - k * chunk);
       it.seq0 = seq0;
       it.seq_n = s.n;
       it.slot = s.slot;

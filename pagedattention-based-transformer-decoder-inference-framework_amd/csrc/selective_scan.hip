@@ -14,7 +14,7 @@ namespace {
 
 constexpr int kThreads = 256;
 
-constexpr int chunk_of(int padded_state) { return std::min(64, 4096 / padded_state); }
+constexpr int chunk_of(int padded_state) { return std::min(32, 4096 / padded_state); }
 
 // within 3 ulp: exp2 and the reciprocal are the hardware's
 __device__ __forceinline__ float silu(float v) {
@@ -275,10 +275,21 @@ hipError_t launch(int dtype, const ScanArgs& a, const ScanItem* items, int n, hi
 
 }  // namespace
 
-int scan_chunk(int state) {
+// A chunk is one serial chain of tokens a lane (about 0.3 us each, most of it latency that other
+// waves fill), and costs three passes over its state (end state, carried, read again).  So chunks
+// as long as still make kFull workgroups, at least 8 tokens, at most 32, in fours as the kernel
+// takes them.  Step of a latent and a scan layer, us, chunks of 64 / 32 / 16 / 8 tokens, of the
+// rule's: 4,096 channels of 16 states, 100 tokens 322 / 303 / 286 / 283, 283; 333 tokens 377 /
+// 360 / 342 / 341, 339; 700 tokens 464 / 443 / 438 / 451, 437; 2,048 tokens 711 / 696 / 705 / 727,
+// 696; 2,048 channels, 100 tokens 212 / 191 / 179 / 174, 174; 2,048 tokens 392 / 378 / 386 / 407, 378.
+int scan_chunk(int inner, int state, int tokens) {
+  constexpr int kFull = 448;
   int p = 8;
   while (p < state) p *= 2;
-  return chunk_of(p);
+  const int channels = kThreads / std::max(1, p / 32);  // of a workgroup
+  const long long blocks = (inner + channels - 1) / channels;
+  const long long n = (tokens * blocks + 4 * kFull - 1) / (4 * kFull) * 4;
+  return (int)std::min<long long>(std::max<long long>(n, 8), chunk_of(p));
 }
 
 hipError_t scan(int dtype, const ScanArgs& a, const ScanItem* items, int n, hipStream_t st) {

@@ -56,8 +56,8 @@ struct ScanArgs {
   float* sum_dt = nullptr;    // [parts][ldc]
 };
 constexpr int kMaxScanState = 256;
-// Tokens a chunk may hold.
-int scan_chunk(int state);
+// Tokens a chunk of a batch of that many takes.
+int scan_chunk(int inner, int state, int tokens);
 hipError_t scan(int dtype, const ScanArgs& a, const ScanItem* items, int n, hipStream_t st);
 // End states of chunks from zero (the first chunk of a sequence: from its slot).
 hipError_t scan_chunks(int dtype, const ScanArgs& a, const ScanItem* items, int n, hipStream_t st);

@@ -159,6 +159,16 @@ def test_selective_scan_alone(serve, name, dtype):  # noqa: F811
     check_cuts(serve(cfg, w, dtype), cfg, w, t, dtype, [2, 1, 2, 2, 1, 3, 66, 5, 64, 1, 1, 2, 60] + [1] * 20)
 
 
+@pytest.mark.parametrize("n", [9, 209, 211, 317, 424, 530, 633, 740, 866])
+def test_chunks_of_a_scan(serve, n):  # noqa: F811
+    """Chunks of 8 tokens to 32, by how many tokens a batch has, last ones of one token to a
+    whole chunk; the state they leave decides the tokens that follow."""
+    cfg = N.config([(N.mamba(inner=4100, state=16), None)], width=40, streams=1)
+    w = N.weights(cfg, 47)
+    t = tokens(cfg, n + 2, 48)
+    check_cuts(serve(cfg, w), cfg, w, t, "float32", [n, 1, 1])
+
+
 @pytest.mark.parametrize("state", [8, 128])
 def test_memory_of_the_first_token(serve, state):  # noqa: F811
     """Slow decay and a strong first input: the token at position 0 decides rows
