@@ -783,6 +783,40 @@ def test_prefill_later_passes(gpu, long_prompts, kind, calls):
     assert err < (FREE_RUN_TOL if kind == "int8" else 1e-3), err
 
 
+@pytest.mark.parametrize("D", [64, 256])  # the prompt kernel; the decode kernel's rows
+@pytest.mark.parametrize("L", [1, 2])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32, 33, 64, 65, 113])
+def test_prefill_last_rows(gpu, n, L, D):
+    """The token that a prompt leaves for the next step, and the step after it: the last layer runs on
+    the last 16 rows of a prompt or fewer.  fp16, so the bars of test_prefill_later_passes."""
+    torch = _torch()
+    import llm_decoder
+    rng = np.random.default_rng(22)
+    H, V, S = 2, 300, 128
+    w = _f16_model(rng, L, H, D, V, S)
+    d = {k: np.ascontiguousarray(v) for k, v in w.items() if k != "cfg"}
+    for k in ("emb", "wqkv", "wo", "w1", "w2"):
+        d[k] = d[k].view(np.uint16)
+    a, b = (llm_decoder.CUDADecoder(L, H, D, H * D, V, S, max_batch=1) for _ in range(2))
+    logits = torch.empty((2, 1, V), device="cuda")
+    prompt = rng.integers(0, V, n).tolist()
+    for dec in (a, b):
+        dec.set_weights(d)
+        dec.begin_synthetic(1, 0, 0, False)
+    for t in prompt:
+        ida = a.step([t], want_next=True)
+    idb = torch.empty(1, dtype=torch.int32, device="cuda")
+    b.prefill(0, prompt)
+    b.copy_next_ids(idb.data_ptr())
+    torch.cuda.synchronize()
+    assert idb.tolist() == ida
+    for i, dec in enumerate((a, b)):
+        dec.step(None, logits_ptr=logits[i].data_ptr())
+    torch.cuda.synchronize()
+    la, lb = logits.cpu().numpy()
+    assert rel_err(lb, la) < 1e-3, rel_err(lb, la)
+
+
 def test_prefill_decode_kernel_fallback(gpu, oracle):
     """Head dims the MFMA prefill kernel does not take (D = 256) prefill
     through the decode kernel, one row per prompt token (beam_ids = the row,
