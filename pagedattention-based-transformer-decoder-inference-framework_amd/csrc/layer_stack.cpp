@@ -426,6 +426,7 @@ int LayerStack::ensure_rows(int M) {
   clear_graphs();
   rows_ = 0;
   RET_IF(alloc_zero(x_, (size_t)n * std::max(cfg_.streams, 1) * ldx_));
+  RET_IF(alloc_zero(x_tail_, (size_t)(n / kTailShare) * std::max(cfg_.streams, 1) * ldx_));
   RET_IF(alloc_zero(h_, (size_t)n * ldx_ * es_));
   // (a product may read whole k-steps past the last row's end)
   const size_t slack = (size_t)64 * es_;
@@ -460,16 +461,16 @@ int LayerStack::ensure_rows(int M) {
 // The row tiles of one attention launch: the plan's sequences that bring few rows
 // per key/value head (big false) or many, split over their pages so that the launch
 // fills rounds of kTargetGroups workgroups; long tiles first.
-void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
+void LayerStack::cut(const std::vector<Portion>& batch, const Plan& p, bool big,
                      std::vector<GqaItem>& items, std::vector<GqaMerge>& merges, Launch& l) {
   l = Launch();
   l.tile_rows = big ? p.big_tile : p.small_tile;
-  const auto mine = [&](const StepSeq& s) {
+  const auto mine = [&](const Portion& s) {
     return s.n >= p.min_n && s.n <= p.max_n && ((s.n * p.R > p.small_max) == big);
   };
   long long tiles = 0;
-  int max_pages = 1, tok0 = 0, entry = 0;
-  for (const StepSeq& s : batch) {
+  int max_pages = 1, entry = 0;
+  for (const Portion& s : batch) {
     if (!mine(s)) continue;
     const int rows = s.n * p.R;
     tiles += (rows + l.tile_rows - 1) / l.tile_rows;
@@ -491,7 +492,7 @@ void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
     for (int n = 1; n <= std::min(kMaxSplits, (max_pages + least - 1) / least); ++n) {
       const int len = (max_pages + n - 1) / n;
       long long pieces = 0;
-      for (const StepSeq& s : batch) {
+      for (const Portion& s : batch) {
         if (!mine(s)) continue;
         for (int r0 = 0; r0 < s.n * p.R; r0 += l.tile_rows) {
           const int last = s.p0 + (std::min(r0 + l.tile_rows, s.n * p.R) - 1) / p.R;
@@ -504,10 +505,8 @@ void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
       per = len;
     }
   }
-  for (const StepSeq& s : batch) {
+  for (const Portion& s : batch) {
     const int rows = s.n * p.R;
-    const int t0 = tok0;
-    tok0 += s.n;
     const int slot = p.expand ? entry : s.slot;  // expanded keys have a table of their own
     entry += s.n >= p.min_n && s.n <= p.max_n;
     if (!mine(s)) continue;
@@ -516,11 +515,11 @@ void LayerStack::cut(const std::vector<StepSeq>& batch, Plan& p, bool big,
       const int pages = last / kPageTokens + 1;
       const int ns = big ? (pages + per - 1) / per : common;
       for (int k = 0; k < ns; ++k)
-        items.push_back(GqaItem{t0, slot, s.p0, r0, rows, (int)((long long)pages * k / ns),
+        items.push_back(GqaItem{s.tok0, s.out0, slot, s.p0, r0, rows, (int)((long long)pages * k / ns),
                                 (int)((long long)pages * (k + 1) / ns), ns > 1 ? l.parts + k : -1});
       l.n_items += ns;
       if (ns > 1) {
-        merges.push_back(GqaMerge{t0, r0, rows, l.parts, ns});
+        merges.push_back(GqaMerge{s.out0, r0, rows, l.parts, ns});
         l.n_merges += 1;
         l.parts += ns;
       }
@@ -556,19 +555,34 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
   at_seq0_ = take((size_t)M * 4);
   at_want_ = take((size_t)n_want * 4);
   at_place_ = take(sizeof place_at);
+  const auto launch_of = [&](const std::vector<Portion>& portions, const Plan& p, bool big, Launch& l) {
+    std::vector<GqaItem> items;
+    std::vector<GqaMerge> merges;
+    cut(portions, p, big, items, merges, l);
+    l.items_at = place(items);
+    l.merges_at = place(merges);
+    const size_t rows = (size_t)l.parts * p.G * l.tile_rows;
+    part_o = std::max(part_o, rows * p.max_pd);
+    part_ml = std::max(part_ml, rows * 2);
+  };
+  std::vector<Portion> all, wanted;
+  for (const StepSeq& s : batch) {
+    const int m = all.empty() ? 0 : all.back().tok0 + all.back().n;
+    all.push_back(Portion{s.slot, s.p0, s.n, m, m});
+    if (tail_.on && s.n_want)
+      wanted.push_back(Portion{s.slot, s.p0 + s.n - 1, 1, m + s.n - 1, (int)wanted.size()});
+  }
+  const Layer& last = *layers_[runs_.back().layer];
+  tail_.small = tail_.big = Launch();
+  tail_.n_scan = 0;
+  if (last.plan >= 0) {
+    launch_of(wanted, *plans_[last.plan], false, tail_.small);
+    launch_of(wanted, *plans_[last.plan], true, tail_.big);
+  }
   for (auto& pp : plans_) {
     Plan& p = *pp;
-    for (int b = 0; b < 2; ++b) {
-      Launch& l = b ? p.big : p.small;
-      std::vector<GqaItem> items;
-      std::vector<GqaMerge> merges;
-      cut(batch, p, b != 0, items, merges, l);
-      l.items_at = place(items);
-      l.merges_at = place(merges);
-      const size_t rows = (size_t)l.parts * p.G * l.tile_rows;
-      part_o = std::max(part_o, rows * p.max_pd);
-      part_ml = std::max(part_ml, rows * 2);
-    }
+    launch_of(all, p, false, p.small);
+    launch_of(all, p, true, p.big);
     if (p.latent) {
       std::vector<int32_t> rows;
       int m = 0;
@@ -599,11 +613,18 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
   for (ScanPlan& p : scans_) {
     std::vector<ScanItem> items, chunks;
     std::vector<ScanCarry> carry;
-    plan_scan(batch, p, items, chunks, carry);
+    plan_scan(batch, false, p, items, chunks, carry);
     p.items_at = place(items);
     p.chunks_at = place(chunks);
     p.carry_at = place(carry);
     parts = std::max(parts, (size_t)p.parts);
+    if (!tail_.on || last.scan < 0 || &p != &scans_[last.scan]) continue;
+    items.clear();
+    ScanPlan again = p;
+    again.parts = 0;
+    plan_scan(batch, true, again, items, chunks, carry);
+    tail_.n_scan = (int)items.size();
+    tail_.scan_at = place(items);
   }
   if (part_o > part_o_.n || part_ml > part_ml_.n || at > meta_cap_ ||
       parts * carry_floats_ > carry_.n) {
@@ -649,7 +670,7 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
   return LLM_OK;
 }
 
-int LayerStack::attention(const Layer& l, const Run& r, int M, hipStream_t st) {
+int LayerStack::attention(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st) {
   const AttentionSpec& a = l.s.attn;
   Geometry& g = *geos_[l.geo];
   const KvCache& kv = g.kv;
@@ -682,6 +703,7 @@ int LayerStack::attention(const Layer& l, const Run& r, int M, hipStream_t st) {
   e.v_pool = kv.v_pool;
   e.page_stride = kv.page_stride();
   LLM_HIP_RET(mm_qkv(dt_, p, e, st));
+  if (tail && tail->n == 0) return LLM_OK;
 
   const Plan& plan = *plans_[l.plan];
   const int ldo = mm_pad(a.heads * a.vdim);
@@ -704,7 +726,7 @@ int LayerStack::attention(const Layer& l, const Run& r, int M, hipStream_t st) {
   q.sink = a.sink ? l.sink.p : nullptr;
   q.part_o = part_o_.p;
   q.part_ml = part_ml_.p;
-  for (const Launch* c : {&plan.small, &plan.big}) {
+  for (const Launch* c : {tail ? &tail->small : &plan.small, tail ? &tail->big : &plan.big}) {
     if (c->n_items == 0) continue;
     q.items = meta<GqaItem>(c->items_at);
     q.n_items = c->n_items;
@@ -713,7 +735,7 @@ int LayerStack::attention(const Layer& l, const Run& r, int M, hipStream_t st) {
     LLM_HIP_RET(gqa_attention(dt_, q, c->tile_rows, st));
   }
 
-  return out_product(l, att_.p, ldo, a.heads * a.vdim, M, st);
+  return out_product(l, att_.p, ldo, a.heads * a.vdim, tail ? tail->n : M, st);
 }
 
 int LayerStack::out_product(const Layer& l, const void* A, int lda, int K, int M, hipStream_t st) {
@@ -855,20 +877,33 @@ int LayerStack::enqueue(int M, int n_want, float* logits, hipStream_t st) {
     const Layer& l = *layers_[r.layer];
     if (r.again && cfg_.loop_adds_embedding) n.embed = 2;
     LLM_HIP_RET(enter(l.norm1, l.hc1));
+    const Tail* tail = tail_.on && i + 1 == runs_.size() ? &tail_ : nullptr;
     switch (l.s.mixer) {
-      case Mixer::kAttention: RET_IF(attention(l, r, M, st)); break;
-      case Mixer::kLatent: RET_IF(latent(l, r, M, st)); break;
-      case Mixer::kMamba: RET_IF(mamba(l, r, M, st)); break;
+      case Mixer::kAttention: RET_IF(attention(l, r, M, tail, st)); break;
+      case Mixer::kLatent: RET_IF(latent(l, r, M, tail, st)); break;
+      case Mixer::kMamba: RET_IF(mamba(l, r, M, tail, st)); break;
     }
+    if (n_want == 0 && tail) return LLM_OK;
     leave(l.norm1b, l.ls1, l.hc1, 1, false);
+    if (tail) {  // from here on row i is wanted row i
+      n.rows = meta<int32_t>(at_want_);
+      n.M = n_want;
+      n.y_rows = 1;
+      n.x_out = x_tail_.p;
+    }
     if (l.s.has_mlp) {
       LLM_HIP_RET(enter(l.norm2, l.hc2));
+      const int rows = tail ? n_want : M;
       if (l.s.dense) {
-        RET_IF(ffn(l, M, st));
+        RET_IF(ffn(l, rows, st));
         leave(l.norm2b, l.ls2, l.hc2, 1, false);
       } else {
-        RET_IF(moe(l, M, st));
+        RET_IF(moe(l, rows, st));
         leave(l.norm2b, l.ls2, l.hc2, l.s.moe.top, l.s.moe.has_shared);
+      }
+      if (tail) {
+        n.x = x_tail_.p;
+        n.M = n.M_y = n_want;
       }
     }
     if (tap_) {
@@ -885,8 +920,11 @@ int LayerStack::enqueue(int M, int n_want, float* logits, hipStream_t st) {
     }
   }
   if (n_want == 0) return LLM_OK;
-  n.rows = meta<int32_t>(at_want_);
-  n.M = n_want;
+  if (n.x != x_tail_.p) {
+    n.rows = meta<int32_t>(at_want_);
+    n.M = n_want;
+    n.x_out = nullptr;
+  }
   n.w_pre = final_norm_.p;
   LLM_HIP_RET(rms_norm_step(dt_, n, st));
   MmArgs a;
@@ -907,7 +945,7 @@ int LayerStack::enqueue(int M, int n_want, float* logits, hipStream_t st) {
 
 int LayerStack::forward(const std::vector<StepSeq>& batch, float* logits, hipStream_t st, float* place) {
   int M = 0, n_want = 0;
-  bool decode = true;
+  bool decode = true, lasts = true;  // lasts: no row is wanted but sequences' last new ones
   single_ = true;
   std::vector<char> seen(opt_.max_seqs, 0);
   for (const StepSeq& s : batch) {
@@ -923,6 +961,7 @@ int LayerStack::forward(const std::vector<StepSeq>& batch, float* logits, hipStr
     n_want += s.n_want;
     single_ = single_ && s.n == 1;
     decode = decode && s.n == 1 && s.n_want == 1;
+    lasts = lasts && (s.n_want == 0 || (s.n_want == 1 && s.want[0] == s.n - 1));
   }
   LLM_REQUIRE(M >= 1 && M <= cap_ && n_want <= M, "step: too many tokens");
   LLM_REQUIRE(n_want == 0 || logits, "step: logits is NULL");
@@ -935,6 +974,8 @@ int LayerStack::forward(const std::vector<StepSeq>& batch, float* logits, hipStr
         RET_IF(g->kv.prepare_append(s.slot, t * kPageTokens));
     RET_IF(g->kv.sync(st));
   }
+  tail_.on = !tap_ && lasts && n_want <= M / kTailShare;
+  tail_.n = n_want;
   RET_IF(build_meta(batch, M, n_want, place, st));
   if (!use_graph_ || !decode || tap_) return enqueue(M, n_want, logits, st);
 

@@ -137,6 +137,17 @@ class LayerStack final : public StepModel {
     size_t items_at = 0, chunks_at = 0, carry_at = 0;
   };
 
+  // The last layer of a step that wants few of its rows (at most one of kTailShare, and of a sequence
+  // the last) runs on those alone, past what it leaves in the cache: no other row of its output is read.
+  static constexpr int kTailShare = 16;
+  struct Tail {
+    bool on = false;
+    int n = 0;           // wanted rows
+    Launch small, big;   // attention of the wanted rows, a portion each
+    int n_scan = 0;
+    size_t scan_at = 0;
+  };
+
   int init_latent(Layer& l);
   int init_mamba(Layer& l);
   int find_rope(const RopeSpec& spec, int* index);
@@ -161,18 +172,24 @@ class LayerStack final : public StepModel {
   int ensure_rows(int M);
   int build_meta(const std::vector<StepSeq>& batch, int M, int n_want, float* place,
                  hipStream_t st);
-  void cut(const std::vector<StepSeq>& batch, Plan& p, bool big, std::vector<GqaItem>& items,
+  // n tokens of one sequence in a row, and the row their attention goes to
+  struct Portion {
+    int slot, p0, n, tok0, out0;
+  };
+  void cut(const std::vector<Portion>& batch, const Plan& p, bool big, std::vector<GqaItem>& items,
            std::vector<GqaMerge>& merges, Launch& l);
   // rows and scratch pages of the portions whose keys are expanded
   void plan_expansion(const std::vector<StepSeq>& batch, Plan& p, std::vector<int32_t>& pos,
                       std::vector<int32_t>& slot, std::vector<int32_t>& entry,
                       std::vector<int32_t>& table);
-  void plan_scan(const std::vector<StepSeq>& batch, ScanPlan& p, std::vector<ScanItem>& items,
+  // tail: only the wanted rows put out
+  void plan_scan(const std::vector<StepSeq>& batch, bool tail, ScanPlan& p, std::vector<ScanItem>& items,
                  std::vector<ScanItem>& chunks, std::vector<ScanCarry>& carry);
   int enqueue(int M, int n_want, float* logits, hipStream_t st);
-  int attention(const Layer& l, const Run& r, int M, hipStream_t st);
-  int latent(const Layer& l, const Run& r, int M, hipStream_t st);
-  int mamba(const Layer& l, const Run& r, int M, hipStream_t st);
+  // Mixers of M rows.  tail: state of all rows, output (y_ row i) of the wanted ones
+  int attention(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st);
+  int latent(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st);
+  int mamba(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st);
   int out_product(const Layer& l, const void* A, int lda, int K, int M, hipStream_t st);
   int moe(const Layer& l, int M, hipStream_t st);
   int ffn(const Layer& l, int M, hipStream_t st);
@@ -195,6 +212,7 @@ class LayerStack final : public StepModel {
   std::vector<Run> runs_;
   std::vector<std::unique_ptr<Plan>> plans_;
   std::vector<ScanPlan> scans_;
+  Tail tail_;
   DevBuf<uint16_t> emb_;
   DevBuf<float> final_norm_;
   DevBuf<uint8_t> head_;
@@ -205,7 +223,7 @@ class LayerStack final : public StepModel {
   // step buffers, sized for rows_ tokens
   int rows_ = 0;
   int ld_q_ = 0, ld_att_ = 0, ld_act_ = 0, ld_shared_ = 0, max_top_ = 0, max_e_ = 0;
-  DevBuf<float> x_, y_, z_, weight_, part_o_, part_ml_, tap_rows_;
+  DevBuf<float> x_, x_tail_, y_, z_, weight_, part_o_, part_ml_, tap_rows_;
   DevBuf<uint8_t> h_, q_, att_, act_, act_shared_;
   // latent: queries in the latent space, values in it, projected-down rows
   int ld_qlat_ = 0, ld_olat_ = 0, ld_down_ = 0;

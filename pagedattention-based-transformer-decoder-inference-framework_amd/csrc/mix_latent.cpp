@@ -128,14 +128,16 @@ void LayerStack::plan_expansion(const std::vector<StepSeq>& batch, Plan& p,
   p.x_pages = page;
 }
 
-int LayerStack::latent(const Layer& l, const Run& r, int M, hipStream_t st) {
+int LayerStack::latent(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st) {
   const LatentSpec& a = l.s.latent;
   const Geometry& g = *geos_[l.geo];
   const int dim = up(a.dim, 2), rank = up(a.rank, 2), Dp = up(dim + a.rot_dim, 8);
   const int ld_att = mm_pad(a.heads * a.vdim);
   const float2* turn = l.rope >= 0 ? ropes_[l.rope]->turn.p : nullptr;
   const Plan& near = *plans_[l.plan];
-  const Plan* far = l.plan_x >= 0 && plans_[l.plan_x]->x_rows > 0 ? plans_[l.plan_x].get() : nullptr;
+  const Plan* far =
+      !tail && l.plan_x >= 0 && plans_[l.plan_x]->x_rows > 0 ? plans_[l.plan_x].get() : nullptr;
+  const int near_rows = tail ? tail->n : near.n_rows;
 
   MmArgs p;
   p.A = h_.p;
@@ -194,13 +196,13 @@ int LayerStack::latent(const Layer& l, const Run& r, int M, hipStream_t st) {
     q.merges = meta<GqaMerge>(c.merges_at);
     q.n_merges = c.n_merges;
   };
-  if (near.n_rows > 0) {
+  if (near_rows > 0) {
     const int ld_lat = a.heads * g.Dp, ldv = mm_pad(a.rank);
     MmArgs b;
     b.A = q_.p;
     b.lda = a.heads * Dp;
     b.W = l.absorb.p;
-    b.M = near.n_rows;
+    b.M = near_rows;
     b.N = a.rank;
     b.K = a.dim;
     b.w_nt = w_nt_;
@@ -211,7 +213,7 @@ int LayerStack::latent(const Layer& l, const Run& r, int M, hipStream_t st) {
     hd.C = q_lat_.p;
     hd.ldc = ld_lat;
     hd.c_head = g.Dp;
-    hd.rows = near.n_rows == M ? nullptr : meta<int32_t>(near.rows_at);
+    hd.rows = tail ? meta<int32_t>(at_want_) : near.n_rows == M ? nullptr : meta<int32_t>(near.rows_at);
     LLM_HIP_RET(mm_heads(dt_, b, hd, st));
 
     q.q = q_lat_.p;
@@ -226,7 +228,7 @@ int LayerStack::latent(const Layer& l, const Run& r, int M, hipStream_t st) {
     q.G = 1;
     q.Dp = g.Dp;
     q.Dv = a.rank;
-    for (const Launch* c : {&near.small, &near.big}) {
+    for (const Launch* c : {tail ? &tail->small : &near.small, tail ? &tail->big : &near.big}) {
       if (c->n_items == 0) continue;
       at(*c);
       LLM_HIP_RET(latent_attention(dt_, q, c->tile_rows, st));
@@ -239,6 +241,7 @@ int LayerStack::latent(const Layer& l, const Run& r, int M, hipStream_t st) {
     b.K = a.rank;
     hd.a_head = ldv;
     hd.w_head = l.value_head;
+    if (tail) hd.rows = nullptr;  // they stand side by side now
     hd.C = att_.p;
     hd.ldc = ld_att;
     hd.c_head = a.vdim;
@@ -304,7 +307,8 @@ int LayerStack::latent(const Layer& l, const Run& r, int M, hipStream_t st) {
       LLM_HIP_RET(gqa_attention(dt_, q, c->tile_rows, st));
     }
   }
-  return out_product(l, att_.p, ld_att, a.heads * a.vdim, M, st);
+  if (tail && tail->n == 0) return LLM_OK;
+  return out_product(l, att_.p, ld_att, a.heads * a.vdim, tail ? tail->n : M, st);
 }
 
 }  // namespace llm

@@ -66,41 +66,49 @@ int LayerStack::load_mamba(const SafeTensors& f, const std::string& mix, Layer& 
   return upload_vec(l.A, t);
 }
 
-void LayerStack::plan_scan(const std::vector<StepSeq>& batch, ScanPlan& p,
+void LayerStack::plan_scan(const std::vector<StepSeq>& batch, bool tail, ScanPlan& p,
                            std::vector<ScanItem>& items, std::vector<ScanItem>& chunks,
                            std::vector<ScanCarry>& carry) {
   p.parts = 0;
   int seq0 = 0, tokens = 0;
   for (const StepSeq& s : batch) tokens += s.n;
   const int chunk = scan_chunk(p.inner, p.state, tokens);
+  int wanted = 0;
   for (const StepSeq& s : batch) {
     const int n = (s.n + chunk - 1) / chunk;
-    for (int k = 0; k < n; ++k) {
+    // The last chunk's end state goes where the first one's start state is, in one launch: a copy
+    // of that, made with the end states, is read instead.
+    const int start = n > 1 && s.p0 > 0 ? p.parts + n - 1 : -1;
+    for (int k = tail ? n - 1 : 0; k < n; ++k) {
       ScanItem it;
-      it.tok0 = seq0 + k * chunk;
+      it.tok0 = it.out0 = seq0 + k * chunk;
       it.n = std::min(chunk, s.n - k * chunk);
       it.seq0 = seq0;
       it.seq_n = s.n;
       it.slot = s.slot;
       it.p0 = s.p0;
-      it.part = k > 0 ? p.parts + k - 1 : -1;
+      it.part = k > 0 ? p.parts + k - 1 : start;
       it.last = k == n - 1;
+      it.start = -1;
+      if (tail) it.out0 = s.n_want ? wanted++ : -1;
       items.push_back(it);
       if (k == n - 1) continue;
       it.part = p.parts + k;
       it.last = k == 0;
+      it.start = k == 0 ? start : -1;
       chunks.push_back(it);
     }
     if (n > 2) carry.push_back(ScanCarry{p.parts, n - 1});
-    p.parts += n - 1;
+    p.parts += n - 1 + (start >= 0);
     seq0 += s.n;
   }
+  if (tail) return;
   p.n_items = (int)items.size();
   p.n_chunks = (int)chunks.size();
   p.n_carry = (int)carry.size();
 }
 
-int LayerStack::mamba(const Layer& l, const Run& r, int M, hipStream_t st) {
+int LayerStack::mamba(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st) {
   const MambaSpec& m = l.s.mamba;
   const int ldc = mm_pad(m.inner), low = up(m.dt_rank, 2), state = up(m.state, 2);
   const int ld_low = mm_pad(m.dt_rank);
@@ -203,10 +211,15 @@ int LayerStack::mamba(const Layer& l, const Run& r, int M, hipStream_t st) {
   }
   c.carry = carry_.p;
   c.sum_dt = sum_dt_.p;
+  c.last_only = tail != nullptr;
   LLM_HIP_RET(scan_chunks(dt_, c, meta<ScanItem>(p.chunks_at), p.n_chunks, st));
   LLM_HIP_RET(scan_carry(c, meta<ScanCarry>(p.carry_at), p.n_carry, st));
-  LLM_HIP_RET(scan(dt_, c, meta<ScanItem>(p.items_at), p.n_items, st));
-  return out_product(l, gated_.p, ldc, m.inner, M, st);
+  if (!tail) {
+    LLM_HIP_RET(scan(dt_, c, meta<ScanItem>(p.items_at), p.n_items, st));
+    return out_product(l, gated_.p, ldc, m.inner, M, st);
+  }
+  LLM_HIP_RET(scan(dt_, c, meta<ScanItem>(tail->scan_at), tail->n_scan, st));
+  return tail->n > 0 ? out_product(l, gated_.p, ldc, m.inner, tail->n, st) : LLM_OK;
 }
 
 }  // namespace llm

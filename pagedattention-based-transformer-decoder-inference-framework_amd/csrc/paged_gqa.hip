@@ -225,7 +225,7 @@ struct Rows {
         den = l[t] * f + __builtin_amdgcn_exp2f(s2 - m2);
       }
       f /= den;
-      T* dst = static_cast<T*>(a.out) + (size_t)(it.tok0 + tok) * a.ldo +
+      T* dst = static_cast<T*>(a.out) + (size_t)(it.out0 + tok) * a.ldo +
              (size_t)head * (a.ldh ? a.ldh : a.Dv);
 #pragma unroll
       for (int n = 0; n < ND; ++n)
@@ -493,7 +493,7 @@ __global__ __launch_bounds__(256) void gqa_merge_kernel(GqaArgs a, int TR) {
           if (lane + 64 * j < a.Dv) acc[j] += ws * v[u][j];
       }
     }
-    T* dst = static_cast<T*>(a.out) + (size_t)(it.tok0 + tok) * a.ldo +
+    T* dst = static_cast<T*>(a.out) + (size_t)(it.out0 + tok) * a.ldo +
              (size_t)head * (a.ldh ? a.ldh : a.Dv);
 #pragma unroll
     for (int j = 0; j < MAXD / 64; ++j)
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(256) void gqa_merge_rows_kernel(GqaArgs a, int TR) 
         acc += x[k] * w;
       }
     }
-    T* dst = static_cast<T*>(a.out) + (size_t)(it.tok0 + tok) * a.ldo + (size_t)head * ldh + d;
+    T* dst = static_cast<T*>(a.out) + (size_t)(it.out0 + tok) * a.ldo + (size_t)head * ldh + d;
     if (vec) {
       *reinterpret_cast<quad_t*>(dst) =
           quad_t{(T)(acc[0] / den), (T)(acc[1] / den), (T)(acc[2] / den), (T)(acc[3] / den)};

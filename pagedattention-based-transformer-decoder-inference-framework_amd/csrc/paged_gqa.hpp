@@ -17,6 +17,7 @@ namespace llm {
 // pages [page0, page1).
 struct GqaItem {
   int32_t tok0;   // batch row of the sequence's first new token
+  int32_t out0;   // its row of `out`
   int32_t slot;   // page-table row
   int32_t p0;     // its position
   int32_t row0, nrows;
@@ -25,7 +26,7 @@ struct GqaItem {
 };
 // The splits of one row tile: parts part0 .. part0 + nsplit - 1.
 struct GqaMerge {
-  int32_t tok0, row0, nrows, part0, nsplit;
+  int32_t out0, row0, nrows, part0, nsplit;
 };
 
 struct GqaArgs {

@@ -292,7 +292,7 @@ __global__ __launch_bounds__(64 * kWaves, sizeof(T) == 2 && NK * MT < 72 ? 2 : 1
       den = l[t] * f + __builtin_amdgcn_exp2f(s2 - m2);
     }
     f /= den;
-    T* dst = static_cast<T*>(a.out) + (size_t)(it.tok0 + tok) * a.ldo +
+    T* dst = static_cast<T*>(a.out) + (size_t)(it.out0 + tok) * a.ldo +
              (size_t)head * (a.ldh ? a.ldh : a.Dv);
 #pragma unroll
     for (int n = 0; n < NDW; ++n)

@@ -36,7 +36,9 @@ __global__ __launch_bounds__(THREADS) void norm_step_kernel(NormStep a) {
   const int i = blockIdx.x;
   const int m = a.rows ? a.rows[i] : i;
   const int nv = a.ldx >> 2;
-  float* xr = a.x + (size_t)m * (SM > 0 ? a.streams : 1) * a.ldx;
+  const size_t x_row = (size_t)(SM > 0 ? a.streams : 1) * a.ldx;
+  const float* xr = a.x + m * x_row;
+  float* xw = a.rows ? a.x_out ? a.x_out + i * x_row : nullptr : a.x + m * x_row;
   f32x4 x[NV];
   // up to 4 streams fly with the other loads; more are read where they are mixed
   constexpr bool EARLY = SM > 0 && SM <= 4 && NV * SM <= 16;
@@ -90,14 +92,15 @@ __global__ __launch_bounds__(THREADS) void norm_step_kernel(NormStep a) {
   f32x4 y[NV];
   if (a.y) {
     float ss = 0.f;
+    const int my = a.y_rows ? i : m;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int c = threadIdx.x + j * THREADS;
       f32x4 s = {0.f, 0.f, 0.f, 0.f};
       if (c < nv) {
-        const float* y0 = a.y + (size_t)m * a.parts * a.ldy + 4 * c;
+        const float* y0 = a.y + (size_t)my * a.parts * a.ldy + 4 * c;
         if (a.shared)
-          s = *reinterpret_cast<const f32x4*>(a.y + ((size_t)a.M_y * a.parts + m) * a.ldy + 4 * c);
+          s = *reinterpret_cast<const f32x4*>(a.y + ((size_t)a.M_y * a.parts + my) * a.ldy + 4 * c);
         for (int q = 0; q < a.parts; q += 4) {  // four parts' loads in flight
           f32x4 v[4];
 #pragma unroll
@@ -139,11 +142,11 @@ __global__ __launch_bounds__(THREADS) void norm_step_kernel(NormStep a) {
         if (c < nv) x[j] += embed_at(c);
       }
     }
-    if ((a.y || a.embed) && !a.rows) {
+    if ((a.y || a.embed) && xw) {
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
         const int c = threadIdx.x + j * THREADS;
-        if (c < nv) *reinterpret_cast<f32x4*>(xr + 4 * c) = x[j];
+        if (c < nv) *reinterpret_cast<f32x4*>(xw + 4 * c) = x[j];
       }
     }
   } else {
@@ -151,7 +154,7 @@ __global__ __launch_bounds__(THREADS) void norm_step_kernel(NormStep a) {
     __syncthreads();  // coef
     const int S = a.streams;
     const float *mix = coef, *out = coef + S * S, *in = out + S;
-    const bool store = (a.y || a.embed) && !a.rows;
+    const bool store = (a.y || a.embed) && xw;
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int c = threadIdx.x + j * THREADS;
@@ -172,7 +175,7 @@ __global__ __launch_bounds__(THREADS) void norm_step_kernel(NormStep a) {
         for (int s = 0; s < SN; ++s)
           if (s < S) v += mix[s * S + t] * old[s];
         if (a.embed == 2) v += e;
-        if (store) *reinterpret_cast<f32x4*>(xr + (size_t)t * a.ldx + 4 * c) = v;
+        if (store) *reinterpret_cast<f32x4*>(xw + (size_t)t * a.ldx + 4 * c) = v;
         x[j] += in[t] * v;
       }
       if (a.u) *reinterpret_cast<f32x4*>(a.u + (size_t)i * a.ldx + 4 * c) = x[j];

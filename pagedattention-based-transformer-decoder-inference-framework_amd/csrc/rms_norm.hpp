@@ -43,9 +43,11 @@ struct NormStep {
   void* h = nullptr;
   int ldh = 0;
   // rows (optional): only these rows of x, h row i = row rows[i]; M = their
-  // number, M_y the tokens y was written for
+  // number, M_y the tokens y was written for (y_rows: for those rows alone, y row i);
+  // x itself stays, the new rows go to x_out row i if that is set
   const int32_t* rows = nullptr;
-  int M_y = 0;
+  int M_y = 0, y_rows = 0;
+  float* x_out = nullptr;
   int streams = 0;                // 0: one residual, no mixing
   const float* hc_mix = nullptr;  // [streams][streams], from first
   const float* hc_out = nullptr;  // [streams]

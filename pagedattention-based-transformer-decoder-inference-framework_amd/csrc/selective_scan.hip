@@ -70,6 +70,14 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(ScanArgs a, const ScanIt
   const float D = PASS == kEmit ? a.D[c] : 0.f;
   __syncthreads();
 
+  if constexpr (PASS == kChunk)
+    if (it.start >= 0 && ok) {
+      float* dst = a.carry + (size_t)it.start * a.state * a.ldc;
+#pragma unroll
+      for (int k = 0; k < NS; ++k)
+        if (n0 + k < a.state) dst[(size_t)(n0 + k) * a.ldc + c] = S[k];
+    }
+
   float sum = 0.f;
   auto work = [&](const Rows& r, int t0) {
 #pragma unroll
@@ -97,7 +105,8 @@ __global__ __launch_bounds__(kThreads) void scan_kernel(ScanArgs a, const ScanIt
 #pragma unroll
         for (int off = LC; off < 64; off *= 2) v += __shfl_xor(v, off, 64);
         v = (v + D * r.x[u]) * silu(r.z[u]);
-        if (ok && sp == 0) static_cast<T*>(a.out)[(size_t)(it.tok0 + t) * a.ldo + c] = (T)v;
+        const int to = a.last_only ? t == n - 1 ? it.out0 : -1 : it.out0 + t;
+        if (ok && sp == 0 && to >= 0) static_cast<T*>(a.out)[(size_t)to * a.ldo + c] = (T)v;
       } else {
         sum += dt;
       }

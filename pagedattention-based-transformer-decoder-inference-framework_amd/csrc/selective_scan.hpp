@@ -24,7 +24,9 @@ struct ScanItem {
   int32_t p0;           // position of the sequence's first new token (0: starts from zero)
   int32_t part;         // scan: carried state to start from (-1: the slot's)
                         // chunk pass: where the end state goes; the first chunk has `last` 1
+  int32_t start;        // chunk pass: where its start state goes too (-1: nowhere)
   int32_t last;         // scan: the sequence's last chunk, its end state goes to the slot
+  int32_t out0;         // scan: output row of the first token; with last_only of the last one, -1: none
 };
 // Parts part0 .. part0 + n - 1 of one sequence, part0 already true.
 struct ScanCarry {
@@ -46,6 +48,7 @@ struct ScanArgs {
   const float* D = nullptr;   // [ldc]
   void* out = nullptr;        // [M][ldo]
   int ldo = 0;
+  int last_only = 0;          // items put out their last token alone
   float* slots = nullptr;     // [slots][state][ldc]
   // inputs of the convolution, to be kept for the next step (taps 0: not here)
   int taps = 0;

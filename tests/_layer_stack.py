@@ -163,6 +163,29 @@ def replay(eng, requests, schedule):
     return {i: np.concatenate(v) for i, v in got.items() if v}
 
 
+def check_last_rows(eng, cfg, w, dtype, a, b):
+    """Steps that want few of their rows, sequences' last ones or none: prompts alone and beside
+    one another, beside a decoded token, portions that nothing is wanted of, then single tokens of
+    both.  a and b: tokens of two sequences, 100 and 130 or more."""
+    sa, sb = eng.open_seq(), eng.open_seq()
+    at, got = {sa: 0, sb: 0}, {sa: [], sb: []}
+    seqs = {sa: a, sb: b}
+    for step in ([(sa, 70, 1), (sb, 40, 0)], [(sb, 33, 0)], [(sa, 1, 1), (sb, 34, 1)], [(sa, 20, 0)],
+                 [(sb, 16, 1)], [(sa, 3, 0), (sb, 1, 0)], [(sa, 1, 1), (sb, 1, 1)], [(sa, 1, 1), (sb, 1, 1)]):
+        entries = [(s, seqs[s][at[s]:at[s] + n], [n - 1] if want else []) for s, n, want in step]
+        out = np.asarray(eng.step(entries))
+        row = 0
+        for s, n, want in step:
+            at[s] += n
+            if want:
+                got[s].append((at[s] - 1, out[row]))
+                row += 1
+    for s, rows in got.items():
+        full = logits(cfg, w, seqs[s][:at[s]])
+        check_rows(np.stack([x for _, x in rows]), full[[i for i, _ in rows]], dtype)
+        eng.close_seq(s)
+
+
 def random_schedule(requests, live, seed):
     """Mixed steps: some requests decode, others bring portions, some pause."""
     rng = np.random.default_rng(seed)

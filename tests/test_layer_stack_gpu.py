@@ -251,6 +251,23 @@ def test_portions(serve, name, sizes, dtype):
     T.check_rows(got, T.logits(cfg, w, t), dtype)
 
 
+LAST = {
+    "attention": [(T.attn(), T.moe()), (T.attn(heads=6, kv_heads=3), None)],
+    "experts": [(T.attn(), None), (T.attn(), T.moe())],
+    "no_shared_expert": [(T.attn(), T.moe(shared=0))],
+    "many_heads": [(T.attn(heads=70, kv_heads=1, dim=16, vdim=8, rot=8), T.moe(experts=5, top=2))],
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", sorted(LAST))
+def test_last_layer_of_few_wanted_rows(serve, name, dtype):
+    """The wanted rows alone go through the last layer; its cache holds every token."""
+    cfg = T.config(LAST[name])
+    w = model_weights(cfg, 49, dtype)
+    T.check_last_rows(serve(cfg, w, dtype), cfg, w, dtype, tokens(cfg, 110, 50), tokens(cfg, 140, 51))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", sorted(MODELS))
 def test_mixed_batches_with_pages_and_slots_used_again(serve, name, dtype):

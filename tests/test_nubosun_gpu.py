@@ -207,6 +207,27 @@ def test_repeated_layers(serve, loop):  # noqa: F811
     check_cuts(serve(cfg, w), cfg, w, t, "float32", [50] + [1] * 40)
 
 
+LAST = {
+    "latent": [(N.mamba(), None), (N.latent(), None)],
+    "latent_and_dense": [(N.latent(), None), (N.latent(), N.dense())],
+    "latent_expands": [(N.latent(heads=2, dim=8, vdim=8, rank=128), N.dense()),
+                       (N.latent(heads=2, dim=8, vdim=8, rank=128), N.dense())],
+    "many_heads": [(N.latent(heads=70, dim=8, vdim=6, rot=4, rank=24), N.dense())],
+    "scan": [(N.latent(), N.dense()), (N.mamba(), None)],
+    "scan_and_dense": [(N.mamba(state=40), None), (N.mamba(), N.dense())],
+    "scan_alone": [(N.mamba(), None)],
+}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", sorted(LAST))
+def test_last_layer_of_few_wanted_rows(serve, name, dtype):  # noqa: F811
+    """The wanted rows alone go through the last layer; its cache and states hold every token."""
+    cfg = N.config(LAST[name], streams=5 if name == "scan_and_dense" else 3)
+    w = N.weights(cfg, 49)
+    T.check_last_rows(serve(cfg, w, dtype), cfg, w, dtype, tokens(cfg, 110, 50), tokens(cfg, 140, 51))
+
+
 def test_residual_after_every_layer(serve):  # noqa: F811
     cfg = N.config([(N.latent(), N.dense()), (N.mamba(), None)], loop=(0, 2, 2), width=100)
     w = N.weights(cfg, 21)
