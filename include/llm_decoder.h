@@ -502,8 +502,9 @@ int llm_decoder_set_taps(llm_decoder* d, int8_t* q_dev, float* s_dev);
  * LLM_PA_FORM_WG_MERGE when their fp32-row plan is one (a quantise launch
  * follows it), else LLM_PA_FORM_SPLIT_MERGE_ROW; beam groups
  * LLM_PA_FORM_SPLIT_MERGE_ROW | LLM_PA_FORM_BEAM.  FP16
- * decoders whose launch merges in the workgroup (2..8 splits, head_dim <= 128,
- * <= 64 heads) run o_proj inside it: LLM_PA_FORM_WG_MERGE | LLM_PA_FORM_OPROJ. */
+ * decoders (head_dim <= 128, <= 64 heads) whose launch merges in the workgroup
+ * run o_proj inside it: LLM_PA_FORM_WG_MERGE | LLM_PA_FORM_OPROJ; LLM_PA_FORM_DIRECT
+ * and LLM_PA_FORM_SPLIT_MERGE_ROW write its packed fp16 input. */
 int llm_decoder_attention_plan(llm_decoder* d, int* nsplit, int* form);
 /* Enqueue layer `layer`'s attention launch of the decoder's step on `stream`
  * (NULL: the decoder's) -- the same kernels, grid and outputs as inside the

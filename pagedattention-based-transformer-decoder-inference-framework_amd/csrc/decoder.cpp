@@ -157,6 +157,7 @@ struct llm_decoder {
   int layer_pre(int l, hipStream_t st, const struct Rows& R);
   int layer_attn(int l, hipStream_t st, const struct Rows& R, PaPlan* plan = nullptr);
   bool quant_prologue(const struct Rows& R) const;
+  bool oproj_shape(const struct Rows& R) const;
   bool oproj_fusable(const struct Rows& R);
   bool wgm_quant_ok(const struct Rows& R);
   bool fc2_split(const struct Rows& R) const;
@@ -525,6 +526,11 @@ bool llm_decoder::quant_prologue(const Rows& R) const {
          quant_prologue_ok(R.n, hid, hid);
 }
 
+bool llm_decoder::oproj_shape(const Rows& R) const {
+  return wdtype == LLM_F16 && R.prefill_row < 0 && R.row_group == 1 && !R.beam_rows && wo_heads.p && D <= 128 &&
+         H <= 64 && oproj_fuse_on();
+}
+
 // FP16 decode rows whose o_proj the attention's workgroup merge can run
 // (pa_decode.hip, OPROJ): each (row, head) workgroup multiplies its merged
 // head by W_o's rows for that head and adds the products into the int64
@@ -533,9 +539,7 @@ bool llm_decoder::quant_prologue(const Rows& R) const {
 // Needs the workgroup-merge form (2..8 splits), head_dim <= 128 and <= 64
 // heads; otherwise the o_proj GEMM runs as before.
 bool llm_decoder::oproj_fusable(const Rows& R) {
-  if (wdtype != LLM_F16 || R.prefill_row >= 0 || R.row_group != 1 || R.beam_rows || !wo_heads.p ||
-      D > 128 || H > 64 || !oproj_fuse_on())
-    return false;
+  if (!oproj_shape(R)) return false;
   Rows r = R;
   r.oacc = oacc.p;
   r.oproj_out = R.x;
@@ -629,6 +633,7 @@ int llm_decoder::layer_attn(int l, hipStream_t st, const Rows& R, PaPlan* plan) 
     ro.out16 = tap_q ? R.act : nullptr;  // the taps read the packed o_proj input
   } else {
     ro.out16 = R.act;
+    if (oproj_shape(R)) ro.o_n = hid;
   }
   if (R.row_group >= 4 && beam_steal_on()) ro.beam_ctr = beam_ctr.p;
   RET_IF(pa_decode_internal(&view, R.q, hid, R.o, R.beam_rows, R.ctx, R.n, H, D, cfg.max_seq_len,

@@ -537,6 +537,50 @@ int choose_nsplit(int B, int H, int ntiles, int pps_fixed, long long resident,
   return (int)std::min(ns, max_nsplit(B, H, ntiles));
 }
 
+// The FP16 decoder's attention and what its o_proj is: `nsplit` splits that a workgroup merges and
+// multiplies by the head's rows of W_o (fused), splits and a merge launch, or one split, both with an
+// o_proj GEMM after them.  `nsplit` in: what the rules above give; their fused form (2..8) may become any
+// of the three, the others stay what they are (the fused sums have a range, the GEMM's none).
+//
+// Lines from steps of 2 to 3 layers, rows x heads of D, the longest sequence held T, sequences that fill it
+// unless said; us a step, before -> now (with them the best fixed choice):
+//  * a fused workgroup reads D x hidden of W_o whatever its row's length, and its 4 waves (8 where that
+//    is 256 KB or more: two rounds of columns for 8) fit the chip 512 (256) times.  Past that one split of up
+//    to 128 pages: 64 x 16 of 128 T 720 476 -> 422, 48 x 12 of 64 T 720 194 -> 182, T 1,920 286 -> 261; below
+//    it where contexts are short for their W_o: 16 x 16 of 128 T 133 225 -> 196, 1 x 16 of 128 195 -> 176,
+//    but T 320 235 -> 223 by 8 waves, one split 219 (22 pages: the line).
+//  * few pairs of long rows leave CUs idle, so splits over more workgroups: 4 x 16 of 128 T 1,920 241 ->
+//    216, T 8,192 with 2,048 held 246 -> 222; 16 x 4 of 64 T 8,300 180 -> 151 by 12.  Heads of 64 with 17 to
+//    64 pairs do so past 8,192 tokens, as a step's sequences may be far shorter than T (T 7,144 with 1,000
+//    held: 4 x 16 of 64 by 4 waves 120, 12 splits 134).  And 16 of them at most, 12 from 33 pairs on, not 24
+//    to 64 (1 x 8 of 128 T 7,144 with 1,000 held 103 -> 94, T 12,144 with 6,000 129 -> 118).
+//  * else 4 waves: 16 x 12 of 64 T 8,192 with 2,048 held 162 -> 156 (by 8), T 2,720 167 -> 161 (by 3).
+//    Up to 32 KB of W_o, which one wave's columns cover, 2 to 4 as before (64 x 4 of 64 T 1,920 175; by 4 179).
+struct F16Form {
+  int nsplit;
+  bool fused;
+};
+F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
+  const long long kb = (long long)D * hidden * 2 / 1024;  // of W_o a head
+  const bool fits = nsplit >= 2 && nsplit <= kWgmMaxSplits;
+  const long long one = kb >= 512 ? std::max<long long>(bh > 256 ? 80 : bh > 128 ? 22 : 0, 13 * kb / 512)
+                        : kb >= 256 ? (bh > 256 ? 20 : 0)
+                                    : (bh > 400 ? 25 : bh > 256 ? 10 : 0);
+  if (fits && tiles <= kMaxPps && (bh > 512 || tiles <= one)) return {1, false};
+  const bool apart = D > 64 ? bh <= 128 && tiles > (kb >= 512 || bh <= 64 ? 45 : 200)
+                            : tiles > (bh <= 16 ? 110 : bh <= 64 ? 512 : INT_MAX);
+  if (nsplit > 1 && apart) {
+    int n = bh <= 32 ? (fits ? 8 : 16) : bh > 64 || (D > 64 && tiles <= 256) ? 8 : 12;
+    if (!fits) n = std::min(n, nsplit);
+    if ((long long)n * kMaxPps >= tiles) return {n, false};
+  }
+  if (!fits) return {nsplit, false};
+  if (tiles <= 4 * kMaxPps && bh > (kb >= 512 ? 400 : 512) && kb >= 256) return {4, false};
+  int n = kb >= 512 || (kb >= 256 && bh <= 256) ? 8 : kb <= 32 ? std::min(nsplit, 4) : 4;
+  while (n < kWgmMaxSplits && (long long)n * kMaxPps < tiles) n *= 2;
+  return {std::min(n, kWgmMaxSplits), true};
+}
+
 template <int D, int TS, int KVT>
 long long resident_for() {
   if constexpr (kv_shape_ok(D, TS, kv_elem_bytes<KVT>()))
@@ -767,7 +811,7 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
                           (long long)B * H * nsplit == resident_launch &&
                           (ntiles_max + nsplit - 1) / nsplit <= 2 * kShortPps;
   if (half_round) nsplit = (nsplit + 1) / 2;
-  const bool wgm_ok = ((row_out && rows->out16 && !rows->q) || oproj || f32_rows) && row_group == 1 &&
+  bool wgm_ok = ((row_out && rows->out16 && !rows->q) || oproj || f32_rows) && row_group == 1 &&
                       kv->kv_dtype == LLM_F16 && tn.wg_merge && !half_round;
   if (wgm_ok && pps_fixed <= 0 && !f32_rows) {
     const int nw = choose_nsplit(B, H, ntiles_max, 0, resident_launch, kWgmShortPps);
@@ -777,6 +821,11 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
     int nw = 2;
     while (nw < nsplit && nw < kWgmMaxSplits) nw *= 2;
     if (nw >= nsplit && (long long)nw * kMaxPps >= ntiles_max) nsplit = nw;
+  }
+  if (wgm_ok && pps_fixed <= 0 && rows->o_n > 0 && tn.wgm_splits <= 0) {
+    const F16Form f = f16_step_form((long long)B * H, D, rows->o_n, ntiles_max, nsplit);
+    wgm_ok = f.fused;  // (the workspace holds max_nsplit splits; a workgroup merge needs none)
+    nsplit = f.fused ? f.nsplit : (int)std::min<long long>(f.nsplit, max_nsplit(B, H, ntiles_max));
   }
   // tuning build: forced split counts of beam-group launches and of the
   // workgroup-merge eligible ones (fp16 row outputs, dynamic splits)
@@ -888,6 +937,13 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
       a.o_flag = rows->o_flag;
     }
   }
+  // one split of fp16 pages writes the o_proj's fp16 rows itself
+  const bool direct16 = direct && row_out && rows->out16 && !rows->q && !rows->keep_out &&
+                        kv->kv_dtype == LLM_F16;
+  if (direct16) {
+    a.out16 = static_cast<_Float16*>(rows->out16);
+    a.pack = rows->pack;
+  }
   hipError_t e;
   bool beam = false;  // the beam kernel ran: every split holds a partial
   switch (D) {
@@ -897,7 +953,7 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
     default: e = dispatch_kvt<256>(a, kv->kv_dtype, TS, direct, st, &beam); break;
   }
   if (e != hipSuccess) return fail(LLM_ERR_HIP, std::string("pa_split launch: ") + hipGetErrorString(e));
-  if (wgm) return LLM_OK;
+  if (wgm || direct16) return LLM_OK;
   if (row_out && !direct)
     return pa_merge_rows_internal(a.part_acc, a.part_ml, rows->keep_out ? out : nullptr, rows,
                                   context_lens, -1, B, H, D, T, TS, beam ? -1 : pps_fixed, nsplit,

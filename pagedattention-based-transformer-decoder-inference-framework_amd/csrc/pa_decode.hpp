@@ -32,7 +32,7 @@ struct PaRowOutputs {
   long long* o_acc = nullptr;
   float* o_x = nullptr;
   const void* wo_heads = nullptr;
-  int o_n = 0;
+  int o_n = 0;  // > 0 without o_acc: the same rows after a plan that did not fuse (f16_step_form)
   // device int set to 1 when a head's term left the accumulator's range and was
   // clamped (common.hpp oacc_term); required with o_acc
   int* o_flag = nullptr;

@@ -56,7 +56,7 @@ struct PaSplitArgs {
   const int32_t* page_table;
   const float* q;
   int q_stride;     // elements between consecutive rows b of q
-  float* out;       // DIRECT: final output [B][H][D]
+  float* out;       // DIRECT: final output [B][H][D] (out16 set: that instead)
   float* part_acc;  // [B*H*nsplit][D]
   float* part_ml;   // [B*H*nsplit][2]
   const int32_t* beam_ids;
@@ -478,6 +478,24 @@ void pa_split_kernel(PaSplitArgs a) {
   const int c = lane % LPT;
   const int g = lane / LPT;
 
+  // DIRECT: this lane's piece of the finished row, fp32 or (out16) the o_proj's fp16 input
+  const auto put_direct = [&](const float (&v)[EPL]) {
+    if constexpr (EPL == 8) {
+      if (a.out16) {
+        f16x8 pk;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pk[e] = (_Float16)v[e];
+        const int k0 = h * D + c * EPL, hid = a.H * D;
+        *reinterpret_cast<f16x8*>(a.out16 + (a.pack ? a_frag_off_f16(b, k0, hid >> 5) : (size_t)b * hid + k0)) = pk;
+        return;
+      }
+    }
+    float* o = a.out + (size_t)bh * D + c * EPL;
+#pragma unroll
+    for (int e = 0; e < EPL; e += 4)
+      *reinterpret_cast<f32x4*>(o + e) = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
+  };
+
   if (count <= 0) {
     if constexpr (BEAM && !DIRECT) {
       // the merge of a beam launch reads every split: an empty one holds
@@ -493,11 +511,8 @@ void pa_split_kernel(PaSplitArgs a) {
       }
     }
     if constexpr (DIRECT) {
-      if (lane < LPT) {
-        float* o = a.out + (size_t)bh * D + c * EPL;
-#pragma unroll
-        for (int e = 0; e < EPL; e += 4) *reinterpret_cast<f32x4*>(o + e) = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
+      const float zero[EPL] = {};
+      if (lane < LPT) put_direct(zero);
     }
     if constexpr (!WGM) return;
     count = 0;  // WGM: no partial (the merge reads splits < ns only), but meet the workgroup
@@ -954,11 +969,9 @@ void pa_split_kernel(PaSplitArgs a) {
   if (lane < LPT) {
     if constexpr (DIRECT) {
       const float inv = 1.0f / (l + 1e-6f);
-      float* o = a.out + (size_t)bh * D + c * EPL;
 #pragma unroll
-      for (int e = 0; e < EPL; e += 4)
-        *reinterpret_cast<f32x4*>(o + e) =
-            f32x4{acc[e] * inv, acc[e + 1] * inv, acc[e + 2] * inv, acc[e + 3] * inv};
+      for (int e = 0; e < EPL; ++e) acc[e] *= inv;
+      put_direct(acc);
     } else {
       float* o = a.part_acc + pidx * D + c * EPL;
 #pragma unroll

@@ -167,6 +167,37 @@ def test_fused_oproj(gpu, ctx, H, D, ts):
         assert np.mean(fa != fg) < 0.05, np.mean(fa != fg)
 
 
+@pytest.mark.parametrize("B,H,D,S,nsplit,form", [
+    (3, 4, 64, 70, 1, 0),       # one split, its fp16 rows written by itself
+    (64, 12, 64, 700, 1, 0),    # past 512 pairs too
+    (16, 16, 128, 150, 1, 0),   # short for the W_o a head has
+    (16, 4, 64, 300, 3, 35),    # few columns: 2 to 4 waves
+    (16, 12, 64, 700, 4, 35), (16, 12, 64, 8191, 4, 35), (16, 12, 64, 8300, 11, 2),
+    (16, 16, 128, 700, 8, 35),
+    (4, 16, 128, 1900, 8, 2), (4, 16, 128, 4500, 12, 2), (1, 8, 128, 8192, 16, 2),
+    (32, 16, 128, 2100, 4, 2),
+], ids=str)
+def test_f16_step_forms(gpu, B, H, D, S, nsplit, form):
+    """The forms an FP16 decoder's attention takes by rows, heads and the longest sequence, one and
+    several tiles of each split and none: step 0 against the o_proj GEMM behind the splits that a
+    decoder without the fused one has, at test_fused_oproj's bar."""
+    import llm_decoder
+    import llm_capi
+    from _util import rel_err
+    L, V = 1, 300
+    w = _model(np.random.default_rng(6), L, H, D, V)
+    dec = llm_decoder.CUDADecoder(L, H, D, H * D, V, S, max_batch=B)
+    dec.set_weights({k: v.view(np.uint16) if v.dtype == np.float16 else v for k, v in w.items()})
+    dec.begin_synthetic(B, 1, 77, True)
+    assert tuple(dec.attention_plan()) == (nsplit, form)
+    del dec
+    for ctx in (0, 17, min(S - 2, 1100)):
+        got = _run(llm_capi.load(), w, L, H, D, V, S, B, ctx, 1, True)
+        ref = _run(llm_capi.load_tune(), w, L, H, D, V, S, B, ctx, 1, False, fuse=False)
+        assert np.isfinite(got).all()
+        assert rel_err(got, ref) < 1e-3, (ctx, rel_err(got, ref))
+
+
 def _guard_run(lib, w, L, H, D, V, B, steps, fuse, splits=3, after=None):
     """Fused-o_proj range guard runs (tuning build, forced split count, context
     0 so each row's attention output is exactly its new V row): per step the
