@@ -581,6 +581,31 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
   return {std::min(n, kWgmMaxSplits), true};
 }
 
+// fp32 rows that the o_proj quantises (hidden up to 2,048): splits that a workgroup merges (2..8) or a
+// merge launch does.  `nsplit` in: what the rules above give; half_round's stay.  Whole rounds of waves
+// make 9 to 95 splits of few pairs, most of them empty where the sequences are short of the longest held,
+// T, and merged in odd batches.  Steps of 2 layers, rows x heads of D, T (held), us, before -> now:
+//  * at most 16 up to 64 pairs (24 of more than 8 pairs of 128 past 9,600 tokens): 1 x 4 of 64 T 7,144 (1,000) 68 -> 62, T 12,144 (6,000) 93 -> 75; 1 x 16 of
+//    128 T 7,144 (1,000) 134 -> 125, T 4,520 (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 11, 16
+//    in place of more: 16 x 4 of 64 T 4,520 (4,500) 97 -> 95, T 7,144 (1,000) 80 -> 77;
+//  * 8 up to 128: 8 x 16 of 128 T 4,520 (4,500) 243 -> 220, 32 x 4 of 64 146 -> 133; past that merged in the
+//    workgroup: 16 x 12 of 64 T 8,192 (2,048) 140 -> 133, T 12,144 (6,000) 217 -> 194;
+//  * more than 256 pairs of 64: 4 in place of 8 (64 x 12 T 8,192 (2,048) 275 -> 257, 32 x 12 186 -> 177), and
+//    past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
+struct F32Form {
+  int nsplit;
+  bool wgm;
+};
+F32Form f32_step_form(long long bh, int D, int tiles, int nsplit) {
+  const bool wgm = nsplit <= kWgmMaxSplits;
+  if (nsplit >= 2 && bh > 512 && tiles <= kMaxPps) return {1, false};
+  if (wgm) return {D <= 64 && bh > 256 && tiles <= 4 * kMaxPps ? std::min(nsplit, 4) : nsplit, true};
+  const int few = D > 64 && bh > 8 && tiles > 600 ? 24 : 16;
+  const int n = bh <= 32 ? std::min(nsplit, few) : bh <= 64 ? (nsplit > 12 ? 16 : 12) : 8;
+  if ((long long)n * kMaxPps < tiles) return {nsplit, false};
+  return {n, bh > 128};
+}
+
 template <int D, int TS, int KVT>
 long long resident_for() {
   if constexpr (kv_shape_ok(D, TS, kv_elem_bytes<KVT>()))
@@ -826,6 +851,11 @@ int llm::pa_decode_internal(const pa_kv_view* kv, const float* q, int q_stride, 
     const F16Form f = f16_step_form((long long)B * H, D, rows->o_n, ntiles_max, nsplit);
     wgm_ok = f.fused;  // (the workspace holds max_nsplit splits; a workgroup merge needs none)
     nsplit = f.fused ? f.nsplit : (int)std::min<long long>(f.nsplit, max_nsplit(B, H, ntiles_max));
+  }
+  if (wgm_ok && pps_fixed <= 0 && f32_rows && H * D <= 2048 && tn.wgm_splits <= 0) {
+    const F32Form f = f32_step_form((long long)B * H, D, ntiles_max, nsplit);
+    wgm_ok = f.wgm;
+    nsplit = f.wgm ? f.nsplit : (int)std::min<long long>(f.nsplit, max_nsplit(B, H, ntiles_max));
   }
   // tuning build: forced split counts of beam-group launches and of the
   // workgroup-merge eligible ones (fp16 row outputs, dynamic splits)

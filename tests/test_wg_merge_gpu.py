@@ -198,6 +198,42 @@ def test_f16_step_forms(gpu, B, H, D, S, nsplit, form):
         assert rel_err(got, ref) < 1e-3, (ctx, rel_err(got, ref))
 
 
+@pytest.mark.parametrize("B,H,D,S,nsplit,form", [
+    (64, 12, 64, 700, 1, 0), (48, 12, 64, 8100, 4, 3), (16, 12, 64, 8300, 8, 3),  # past 512, 256, 128 pairs
+    (1, 4, 64, 12100, 16, 1), (1, 16, 128, 12100, 24, 1), (4, 12, 64, 4600, 12, 1), (16, 4, 64, 7100, 16, 1),
+    (8, 16, 128, 4600, 8, 1), (2, 3, 64, 90, 1, 0), (16, 16, 128, 700, 2, 3),
+], ids=str)
+def test_int8_step_forms(gpu, oracle, B, H, D, S, nsplit, form):
+    """The forms of fp32 rows for the quantising o_proj: against the same step of a decoder that holds
+    other sequences too, at lengths with and without splits of no tiles.  An activation on the edge of
+    two int8 values may take the other: the free-running bar of test_decoder_gpu.py."""
+    import torch
+    from _util import rel_err
+    from test_decoder_gpu import FREE_RUN_TOL, _int8_model, _make_gpu_decoder
+    w = _int8_model(oracle, L=1, H=H, D=D, V=300, S=S, seed=31)
+    prompt = np.random.default_rng(32).integers(0, 300, min(S - 2, 700)).tolist()
+    out = []
+    for rows in (B, 1 if B > 1 else 7):  # the first row alone, or with others: other splits
+        dec = _make_gpu_decoder(w, max_batch=rows)
+        dec.begin_synthetic(rows, 0, 0, False)
+        if rows == B:
+            assert tuple(dec.attention_plan()) == (nsplit, form)
+        logits = torch.empty((rows, 300), device="cuda")
+        got = []
+        at = 0
+        for n in (0, 17, len(prompt) - 1):
+            if n > at:
+                for r in range(min(rows, 2)):
+                    dec.prefill(r, prompt[at:n])
+            dec.step([prompt[n]] * rows, logits_ptr=logits.data_ptr())
+            torch.cuda.synchronize()
+            got.append(logits[0].cpu().numpy())
+            at = n + 1
+        out.append(np.stack(got))
+    assert np.isfinite(out[0]).all()
+    assert rel_err(out[0], out[1]) < FREE_RUN_TOL, rel_err(out[0], out[1])
+
+
 def _guard_run(lib, w, L, H, D, V, B, steps, fuse, splits=3, after=None):
     """Fused-o_proj range guard runs (tuning build, forced split count, context
     0 so each row's attention output is exactly its new V row): per step the
