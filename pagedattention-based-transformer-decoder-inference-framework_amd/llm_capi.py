@@ -227,18 +227,38 @@ def stream_ptr(stream=None):
     return ctypes.c_void_p(s.cuda_stream)
 
 
+def _stream(stream):
+    """stream_ptr as a plain number, without a torch.cuda.Stream for the current one (3.2 us a
+    call of 18 for a short row's attention, now 0.3)."""
+    import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if stream is not None or raw is None or not torch.cuda.is_initialized():
+        return (stream if stream is not None else torch.cuda.current_stream()).cuda_stream
+    return raw(torch.cuda.current_device())
+
+
 def ptr(t) -> ctypes.c_void_p:
     return ctypes.c_void_p(0 if t is None else t.data_ptr())
 
 
+def _at(t):
+    return None if t is None else t.data_ptr()
+
+
+_kv_dtypes = None
+
+
 def kv_dtype_of(t) -> int:
     """llm_dtype of a torch KV pool tensor (fp16, bf16, fp32 or int8)."""
-    import torch
-    m = {torch.float16: LLM_F16, torch.bfloat16: LLM_BF16, torch.float32: LLM_F32,
-         torch.int8: LLM_I8}
-    if t.dtype not in m:
+    global _kv_dtypes
+    if _kv_dtypes is None:
+        import torch
+        _kv_dtypes = {torch.float16: LLM_F16, torch.bfloat16: LLM_BF16, torch.float32: LLM_F32,
+                      torch.int8: LLM_I8}
+    dtype = _kv_dtypes.get(t.dtype)
+    if dtype is None:
         raise TypeError(f"KV pool dtype {t.dtype} is not one of fp16/bf16/fp32/int8")
-    return m[t.dtype]
+    return dtype
 
 
 def kv_view(k_pool, v_pool, page_table, *, num_beams=None) -> PaKvView:
@@ -248,21 +268,19 @@ def kv_view(k_pool, v_pool, page_table, *, num_beams=None) -> PaKvView:
     [num_pages][2][ts][D] tensor: K and V pages interleaved) as long as each
     page is contiguous; the view's page_stride is then the page-to-page step."""
     nb, H, mt = page_table.shape
-    for t in (k_pool, v_pool):
-        if t.dim() != 3 or t.stride(2) != 1 or t.stride(1) != t.shape[2]:
+    shape, stride, v_shape, v_stride = k_pool.shape, k_pool.stride(), v_pool.shape, v_pool.stride()
+    for n, step in ((shape, stride), (v_shape, v_stride)):
+        if len(n) != 3 or step[2] != 1 or step[1] != n[2]:
             raise ValueError("KV pools must be [num_pages][ts][D] with contiguous pages")
-    if k_pool.stride(0) != v_pool.stride(0):
+    if stride[0] != v_stride[0]:
         raise ValueError("k_pool and v_pool must share one page stride")
-    v = PaKvView()
-    v.k_pool, v.v_pool, v.page_table = k_pool.data_ptr(), v_pool.data_ptr(), page_table.data_ptr()
-    v.num_pages, v.page_size, v.head_dim = k_pool.shape[0], k_pool.shape[1], k_pool.shape[2]
-    v.num_beams, v.num_heads, v.max_tiles = num_beams or nb, H, mt
     if k_pool.dtype != v_pool.dtype:
         raise TypeError("k_pool and v_pool must have the same dtype")
-    v.kv_dtype = kv_dtype_of(k_pool)
-    dense = k_pool.shape[1] * k_pool.shape[2]
-    v.page_stride = 0 if k_pool.stride(0) == dense else k_pool.stride(0) * k_pool.element_size()
-    return v
+    pages, ts, D = shape
+    dtype = kv_dtype_of(k_pool)
+    return PaKvView(k_pool.data_ptr(), v_pool.data_ptr(), page_table.data_ptr(), pages, ts, D,
+                    num_beams or nb, H, mt, dtype,
+                    0 if stride[0] == ts * D else stride[0] * k_pool.element_size())
 
 
 def pa_decode(q, k_pool, v_pool, page_table, *, T, beam_ids=None, context_lens=None,
@@ -279,13 +297,13 @@ def pa_decode(q, k_pool, v_pool, page_table, *, T, beam_ids=None, context_lens=N
     ws_bytes = lib.pa_decode_workspace_bytes(B, H, D, page_table.shape[2], pages_per_split)
     ws = torch.empty(max(ws_bytes, 4), dtype=torch.uint8, device=q.device)
     if row_group > 1:
-        check(lib.pa_decode_grouped(ctypes.byref(view), ptr(q), ptr(out), ptr(beam_ids),
-                                    ptr(context_lens), B, H, D, T, sm_scale, pages_per_split,
-                                    row_group, ptr(ws), ws_bytes, stream_ptr(stream)))
+        check(lib.pa_decode_grouped(ctypes.byref(view), q.data_ptr(), out.data_ptr(), _at(beam_ids),
+                                    _at(context_lens), B, H, D, T, sm_scale, pages_per_split,
+                                    row_group, ws.data_ptr(), ws_bytes, _stream(stream)))
     else:
-        check(lib.pa_decode(ctypes.byref(view), ptr(q), ptr(out), ptr(beam_ids),
-                            ptr(context_lens), B, H, D, T, sm_scale, pages_per_split, ptr(ws),
-                            ws_bytes, stream_ptr(stream)))
+        check(lib.pa_decode(ctypes.byref(view), q.data_ptr(), out.data_ptr(), _at(beam_ids),
+                            _at(context_lens), B, H, D, T, sm_scale, pages_per_split,
+                            ws.data_ptr(), ws_bytes, _stream(stream)))
     return out
 
 
@@ -301,15 +319,13 @@ def pa_decode_ex(q, k_pool, v_pool, page_table, *, T, beam_ids=None, context_len
     probs = torch.empty((B, H, T), dtype=torch.float32, device=q.device) if want_probs else None
     scores = torch.empty((B, H, T), dtype=torch.float32, device=q.device) if want_probs else None
     view = kv_view(k_pool, v_pool, page_table)
-    opt = PaDecodeOptions(temperature=temperature, top_k=top_k, top_p=top_p, eos_token=eos_token,
-                          eos_threshold=eos_threshold,
-                          probs_out=None if probs is None else probs.data_ptr(),
-                          scores_out=None if scores is None else scores.data_ptr())
+    opt = PaDecodeOptions(temperature, top_k, top_p, eos_token, eos_threshold, _at(probs), _at(scores))
     ws_bytes = max(lib.pa_decode_workspace_bytes(B, H, D, page_table.shape[2], 0),
                    lib.pa_decode_ex_workspace_bytes(B, H, T))
     ws = torch.empty(max(ws_bytes, 8), dtype=torch.uint8, device=q.device)
-    check(lib.pa_decode_ex(ctypes.byref(view), ptr(q), ptr(out), ptr(beam_ids), ptr(context_lens),
-                           B, H, D, T, ctypes.byref(opt), ptr(ws), ws_bytes, stream_ptr(stream)))
+    check(lib.pa_decode_ex(ctypes.byref(view), q.data_ptr(), out.data_ptr(), _at(beam_ids),
+                           _at(context_lens), B, H, D, T, ctypes.byref(opt), ws.data_ptr(), ws_bytes,
+                           _stream(stream)))
     return (out, probs, scores) if want_probs else out
 
 
@@ -415,8 +431,8 @@ def sample_rows(logits, temperature=1.0, top_k=0, top_p=1.0, seed=0, counter=0, 
     lib = load()
     R, V = logits.shape
     out = torch.empty(R, dtype=torch.int32, device=logits.device)
-    check(lib.sample_rows(ptr(logits), R, V, temperature, top_k, top_p, seed, counter, ptr(out),
-                          stream_ptr(stream)))
+    check(lib.sample_rows(logits.data_ptr(), R, V, temperature, top_k, top_p, seed, counter,
+                          out.data_ptr(), _stream(stream)))
     return out
 
 
