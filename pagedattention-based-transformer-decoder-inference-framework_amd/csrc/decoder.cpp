@@ -156,6 +156,8 @@ struct llm_decoder {
 
   int layer_pre(int l, hipStream_t st, const struct Rows& R);
   int layer_attn(int l, hipStream_t st, const struct Rows& R, PaPlan* plan = nullptr);
+  bool ln_prologue(const struct Rows& R) const;
+  bool one_pass(const struct Rows& R) const;
   bool quant_prologue(const struct Rows& R) const;
   bool oproj_shape(const struct Rows& R) const;
   bool oproj_fusable(const struct Rows& R);
@@ -493,6 +495,14 @@ int llm_decoder::layer_pre(int l, hipStream_t st, const Rows& R) {
   return tap(l, 0, R, hid, st);
 }
 
+// Up to 32 prompt rows too: a launch less for each product behind a LayerNorm (4 layers of 4 x 64 fp16,
+// prompts of 9 tokens 264 -> 236 us, of 17 279 -> 254; 64 rows took a workgroup longer than the launch,
+// int8 313 -> 339).
+constexpr int kPrologueRows = 32;
+bool llm_decoder::ln_prologue(const Rows& R) const {
+  return (R.prefill_row < 0 || R.n <= kPrologueRows) && ln_fusable(wdtype, R.n, hid);
+}
+
 // LN(x) as the GEMM's A: fused into the GEMM as its LayerNorm prologue when
 // the rows' A image fits in LDS (decode rows), else a LayerNorm (+ quant)
 // launch writing the packed A the GEMM reads.
@@ -501,7 +511,7 @@ int llm_decoder::layer_norm_into(WeightGemm& g, const Rows& R, const float* gamm
   // the first LayerNorm reads the token embedding rows (embed_rows)
   LnSource src = embed_src;
   embed_src = LnSource{};
-  if (R.prefill_row < 0 && ln_fusable(wdtype, R.n, hid)) {
+  if (ln_prologue(R)) {
     g.ln_x = R.x; g.ln_g = gamma; g.ln_b = beta; g.ln_eps = 1e-5f;
     g.ln_emb = src.emb; g.ln_tok = src.tok; g.ln_V = src.V;
     if (tap_q) { g.act_out = R.act; g.sa_out = R.sa; }  // the taps read A and the scales back
@@ -522,8 +532,15 @@ int llm_decoder::layer_norm_into(WeightGemm& g, const Rows& R, const float* gamm
 // launch.  Beam groups keep the merge launch (the beam kernel's workgroups
 // are 4 beams of one split), as do prefill chunks.
 bool llm_decoder::quant_prologue(const Rows& R) const {
-  return wdtype == LLM_I8 && R.prefill_row < 0 && R.row_group == 1 &&
-         quant_prologue_ok(R.n, hid, hid);
+  return wdtype == LLM_I8 && R.row_group == 1 && quant_prologue_ok(R.n, hid, hid) &&
+         (R.prefill_row < 0 || one_pass(R));
+}
+
+// Prompt rows whose attention is one pass, no merge to make the o_proj's input: few of them it quantises
+// itself (4 layers of 4 x 64, 17 tokens 296 -> 284 us with the LayerNorms; 16 x 128 450 -> 461, so not there).
+bool llm_decoder::one_pass(const Rows& R) const {
+  pa_kv_view v;
+  return !R.mixed && R.n <= kPrologueRows && hid <= 1024 && kv_cache_view(kv, 0, &v) == LLM_OK && pa_prefill_one_pass(&v, R.prefill_p0, R.n);
 }
 
 bool llm_decoder::oproj_shape(const Rows& R) const {
@@ -591,7 +608,7 @@ bool llm_decoder::fc2_split(const Rows& R) const {
 // hidden 256: 1 row 190 and 180, 8 rows 203 and 193, 16 rows 223 and 225; 512: 208 and 197, 229
 // and 225, 257 and 266).
 bool llm_decoder::fc2_quant_prologue(const Rows& R) const {
-  return wdtype == LLM_I8 && R.prefill_row < 0 && R.n <= 8 && quant_prologue_ok(R.n, hid, inter);
+  return wdtype == LLM_I8 && R.n <= 8 && quant_prologue_ok(R.n, hid, inter);
 }
 
 int llm_decoder::layer_attn(int l, hipStream_t st, const Rows& R, PaPlan* plan) {
@@ -605,7 +622,9 @@ int llm_decoder::layer_attn(int l, hipStream_t st, const Rows& R, PaPlan* plan) 
     PaRowOutputs ro;
     ro.pack = 1;
     ro.keep_out = 0;
-    if (wdtype == LLM_I8) {
+    if (quant_prologue(R)) {
+      // fp32 rows in R.o, for the o_proj's prologue
+    } else if (wdtype == LLM_I8) {
       ro.q = static_cast<int8_t*>(R.act);
       ro.inv_scale = R.sa;
     } else {

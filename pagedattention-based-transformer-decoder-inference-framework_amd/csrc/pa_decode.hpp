@@ -87,9 +87,12 @@ int pa_merge_splits_internal(const float* part_acc, const float* part_ml, float*
 // positions 0 .. p0 + i of page-table row `row`.
 // With workspace (pa_prefill_workspace_bytes) the key range is split over
 // workgroups and merged by pa_merge_rows_internal, which also writes `rows`
-// (the o_proj input); without, one pass writes out and `rows` is converted by
-// the row quantiser.  `out` may be NULL only when it splits and rows is set.
+// (the o_proj input); without, one pass writes out, or packed fp16 `rows` in its
+// place if it is not kept, and int8 `rows` are made by the row quantiser.  `out`
+// may be NULL when it splits and rows is set, or fp16 rows take its place.
 bool pa_prefill_supported(const pa_kv_view* kv);
+// Whether m queries at p0 are one pass whatever the workspace.
+bool pa_prefill_one_pass(const pa_kv_view* kv, int p0, int m);
 // (pa_prefill_ws_bytes: enough for m queries at p0 and at any shorter context)
 size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m);
 int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, float* out,

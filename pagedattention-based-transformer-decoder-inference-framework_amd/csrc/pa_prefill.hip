@@ -48,6 +48,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "ln_wave.hpp"
 #include "pa_decode.hpp"
 #include "row_ops.hpp"
 
@@ -72,6 +73,7 @@ struct PaPrefillArgs {
   int nsplit, pps;
   float* part_acc;
   float* part_ml;
+  _Float16* out16;  // one pass: packed fp16 rows of H * D (a_frag_off_f16) in place of out
 };
 
 constexpr int stage_keys(int D) { return D == 64 ? 64 : 32; }
@@ -342,6 +344,12 @@ __global__ __launch_bounds__(64 * kWaves, KEYS == stage_keys(D) ? 4 : 2) void pa
     for (int nd = 0; nd < ND; ++nd)
       *reinterpret_cast<f32x4*>(o + 16 * nd) = O[nd] * (1.0f / kPScale);
     if (g == 0) *reinterpret_cast<float2*>(a.part_ml + pidx * 2) = float2{mtop, lrun};
+  } else if (a.out16) {
+    const float inv = 1.0f / (lrun + 1e-6f) * (1.0f / kPScale);
+    _Float16* o = a.out16 + a_frag_off_f16(qi, h * D + 4 * g, a.H * D / 32);
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd)  // (16 dims further: 2 of a fragment's 4 groups of 8)
+      *reinterpret_cast<ln_f16x4*>(o + nd / 2 * 512 + nd % 2 * 256) = ln_half4(O[nd] * inv);
   } else {
     const float inv = 1.0f / (lrun + 1e-6f) * (1.0f / kPScale);
     float* o = a.out + (size_t)qi * a.out_stride + h * D + 4 * g;
@@ -415,6 +423,10 @@ bool pa_prefill_supported(const pa_kv_view* kv) {
 // A plan has no more splits than split_bound and its stages allow, but fewer at one p0
 // than at a shorter one (2048 queries x 16 heads: three at p0 0, one from p0 2048 on), so
 // the size is of the most that any context up to this one takes.
+bool pa_prefill_one_pass(const pa_kv_view* kv, int p0, int m) {
+  return pa_prefill_supported(kv) && m > 0 && p0 >= 0 && prefill_plan(kv, p0, m).nsplit == 1;
+}
+
 size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m) {
   if (!pa_prefill_supported(kv) || m <= 0 || p0 < 0) return 0;
   const int most = (int)(((long long)p0 + m - 1) / stage_keys(kv->head_dim)) + 1;
@@ -447,7 +459,8 @@ int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, floa
   const bool split = pl.nsplit > 1 && workspace && workspace_bytes >= need &&
                      (out == nullptr || out_stride == hid) &&
                      (!row_out || rows->pack);  // the merge writes packed o_proj inputs
-  LLM_REQUIRE(out || (split && row_out), "pa_prefill: out is NULL");
+  const bool direct16 = !split && row_out && rows->out16 && !rows->q && !rows->keep_out && rows->pack;
+  LLM_REQUIRE(out || (split && row_out) || direct16, "pa_prefill: out is NULL");
   PaPrefillArgs a{};
   a.q = q;
   a.q_stride = q_stride;
@@ -471,6 +484,7 @@ int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, floa
   } else {
     a.nsplit = 1;
     a.pps = kv->max_tiles;
+    if (direct16) a.out16 = static_cast<_Float16*>(rows->out16);
   }
   hipError_t e;
   const int TS = kv->page_size;
@@ -483,7 +497,7 @@ int pa_prefill_internal(const pa_kv_view* kv, const float* q, int q_stride, floa
     return pa_merge_rows_internal(a.part_acc, a.part_ml, (rows && !rows->keep_out) ? nullptr : out,
                                   rows, nullptr, p0, m, H, D, p0 + m, TS, pl.pps, pl.nsplit,
                                   kv->max_tiles, st);
-  if (row_out) {  // one pass: convert the fp32 rows into the o_proj input
+  if (row_out && !direct16) {  // one pass: convert the fp32 rows into the o_proj input
     if (rows->q)
       LLM_HIP_RET(launch_quantize_rows(out, m, hid, rows->q, rows->inv_scale, st, rows->pack));
     if (rows->out16)

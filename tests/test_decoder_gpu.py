@@ -817,6 +817,18 @@ def test_prefill_last_rows(gpu, n, L, D):
     assert rel_err(lb, la) < 1e-3, rel_err(lb, la)
 
 
+@pytest.mark.parametrize("H,D", [(4, 64), (8, 64), (16, 128)])
+@pytest.mark.parametrize("n", [2, 9, 10, 17, 18, 33, 34, 65])
+def test_prefill_short_int8(gpu, oracle, n, H, D):
+    """Prompts whose products make their own int8 rows (up to 32 rows, and 8 of fc2's), at the edges; a
+    step's bar of free running."""
+    w = _int8_model(oracle, L=2, H=H, D=D, V=300, S=96, seed=23)
+    prompt = np.random.default_rng(24).integers(0, 300, n).tolist()
+    la, lb, nxt = _prefill_vs_stepping(lambda k: _make_gpu_decoder(w, max_batch=k), [prompt], 300)
+    assert rel_err(lb[0], la[0]) < FREE_RUN_TOL, rel_err(lb[0], la[0])
+    assert (la[0].max() - la[0][nxt[0]]) / np.abs(la[0]).max() <= FREE_RUN_TOL
+
+
 def test_prefill_decode_kernel_fallback(gpu, oracle):
     """Head dims the MFMA prefill kernel does not take (D = 256) prefill
     through the decode kernel, one row per prompt token (beam_ids = the row,
