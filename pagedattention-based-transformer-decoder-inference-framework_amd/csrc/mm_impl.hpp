@@ -1202,9 +1202,20 @@ hipError_t launch(const KernelArgs& p, hipStream_t st) {
       return stream<T, EPI, 1, 2, 4, 8>(p, 1, N, st);
   if (M <= 16) return stream<T, EPI, 1, 1>(p, 1, N, st);
   if constexpr (EPI == kSplit) {
-    // narrow products: all columns in two blocks, so a row is read twice
-    if (M > 64 && ntiles <= 10 && (M + 31) / 32 * 2 < 1024)
-      return stream<T, EPI, 2, 5>(p, (M + 31) / 32, N, st);
+    // Narrow products: the fewest column tiles a block that are one round, as a block takes the time of
+    // its chain of K whatever its width allows (K 4096, 160 columns, us by 1 / 2 / 3 / 5 tiles and 16 rows, 5
+    // and 32: 333 rows 7.8 / 8.7 / 9.4 / 11.4, 15.0; 700 12.5 / 9.8 / 9.8 / 11.6, 15.1; 2011 25.4 / 23.1 /
+    // 18.3 / 12.5, 15.5; K 2048, 96 columns: 333 4.8, 8.7; 1400 9.6 / 9.1 / 6.1 / 7.6, 9.5); past that all
+    // columns in two blocks of 32 rows, so a row is read twice.
+    if (M > 64 && ntiles <= 10) {
+      const int rb = (M + 15) / 16;
+      const auto one_round = [&](int nt) { return (ntiles + nt - 1) / nt * rb <= 256; };
+      if (one_round(1)) return stream<T, EPI, 1, 1>(p, rb, N, st);
+      if (one_round(2)) return stream<T, EPI, 1, 2>(p, rb, N, st);
+      if (one_round(3)) return stream<T, EPI, 1, 3>(p, rb, N, st);
+      if (one_round(5)) return stream<T, EPI, 1, 5>(p, rb, N, st);
+      if ((M + 31) / 32 * 2 < 1024) return stream<T, EPI, 2, 5>(p, (M + 31) / 32, N, st);
+    }
   }
   // Blocks once the smallest of them are more than half a round, else streams:
   // 64 x 6144 x 1024 5.1 us as blocks (streams 5.3), 64 x 2048 x 6144 10.7 as

@@ -169,6 +169,20 @@ def test_chunks_of_a_scan(serve, n):  # noqa: F811
     check_cuts(serve(cfg, w), cfg, w, t, "float32", [n, 1, 1])
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rank,state,rows", [
+    (128, 16, (65, 400, 401, 816, 817, 1024, 1025, 2049)), (64, 16, (672, 673, 1360, 1361, 1377)), (5, 8, (67, 1365))])
+def test_narrow_products_of_prompts(serve, rank, state, rows, dtype):  # noqa: F811
+    """The inputs of a scan at the row counts where a block of their product gets more columns."""
+    cfg = N.config([(N.mamba(inner=200, dt_rank=rank, state=state), None)], width=40, vocab=60, streams=1)
+    w = N.weights(cfg, 49)
+    eng = serve(cfg, w, dtype, max_seqs=1, max_tokens=64 * 40)
+    t = tokens(cfg, max(rows), 50)
+    want = T.logits(cfg, w, t)
+    for n in rows:
+        T.check_rows(run_whole(eng, t[:n]), want[:n], dtype)
+
+
 @pytest.mark.parametrize("state", [8, 128])
 def test_memory_of_the_first_token(serve, state):  # noqa: F811
     """Slow decay and a strong first input: the token at position 0 decides rows
