@@ -432,7 +432,8 @@ int LayerStack::ensure_rows(int M) {
   const size_t slack = (size_t)64 * es_;
   RET_IF(alloc_zero(q_, (size_t)n * ld_q_ * es_ + slack));
   RET_IF(alloc_zero(att_, (size_t)n * ld_att_ * es_));
-  RET_IF(alloc_zero(y_, (size_t)n * (max_top_ + 1) * ldx_));
+  const size_t part_rows = std::min<size_t>((size_t)n * kMmMostParts, kMmPartRows);
+  RET_IF(alloc_zero(y_, std::max((size_t)n * (max_top_ + 1), part_rows) * ldx_));
   RET_IF(alloc_zero(act_, (size_t)n * std::max(max_top_, 1) * ld_act_ * es_));
   RET_IF(alloc_zero(q_lat_, (size_t)n * ld_qlat_ * es_ + slack));
   RET_IF(alloc_zero(o_lat_, (size_t)n * ld_olat_ * es_ + slack));
@@ -747,9 +748,17 @@ int LayerStack::out_product(const Layer& l, const void* A, int lda, int K, int M
   o.N = cfg_.width;
   o.K = K;
   o.w_nt = w_nt_;
-  o.C = y_.p;
-  o.ldc = ldx_;
-  LLM_HIP_RET(mm(dt_, o, st));
+  return sublayer_product(o, st);
+}
+
+// The sums of K's slices lie side by side: rows m y_parts_ .. of y_.
+int LayerStack::sublayer_product(MmArgs& a, hipStream_t st) {
+  y_parts_ = mm_parts(dt_, a.M, a.N, a.K);
+  a.C = y_.p;
+  a.ldc = y_parts_ * ldx_;
+  a.parts = y_parts_;
+  a.c_part = ldx_;
+  LLM_HIP_RET(mm(dt_, a, st));
   return LLM_OK;
 }
 
@@ -769,10 +778,7 @@ int LayerStack::ffn(const Layer& l, int M, hipStream_t st) {
   a.W = l.ffn_out.p;
   a.N = cfg_.width;
   a.K = l.s.ffn.ff;
-  a.C = y_.p;
-  a.ldc = ldx_;
-  LLM_HIP_RET(mm(dt_, a, st));
-  return LLM_OK;
+  return sublayer_product(a, st);
 }
 
 int LayerStack::moe(const Layer& l, int M, hipStream_t st) {
@@ -884,7 +890,7 @@ int LayerStack::enqueue(int M, int n_want, float* logits, hipStream_t st) {
       case Mixer::kMamba: RET_IF(mamba(l, r, M, tail, st)); break;
     }
     if (n_want == 0 && tail) return LLM_OK;
-    leave(l.norm1b, l.ls1, l.hc1, 1, false);
+    leave(l.norm1b, l.ls1, l.hc1, y_parts_, false);
     if (tail) {  // from here on row i is wanted row i
       n.rows = meta<int32_t>(at_want_);
       n.M = n_want;
@@ -896,7 +902,7 @@ int LayerStack::enqueue(int M, int n_want, float* logits, hipStream_t st) {
       const int rows = tail ? n_want : M;
       if (l.s.dense) {
         RET_IF(ffn(l, rows, st));
-        leave(l.norm2b, l.ls2, l.hc2, 1, false);
+        leave(l.norm2b, l.ls2, l.hc2, y_parts_, false);
       } else {
         RET_IF(moe(l, rows, st));
         leave(l.norm2b, l.ls2, l.hc2, l.s.moe.top, l.s.moe.has_shared);

@@ -191,6 +191,7 @@ class LayerStack final : public StepModel {
   int latent(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st);
   int mamba(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st);
   int out_product(const Layer& l, const void* A, int lda, int K, int M, hipStream_t st);
+  int sublayer_product(MmArgs& a, hipStream_t st);
   int moe(const Layer& l, int M, hipStream_t st);
   int ffn(const Layer& l, int M, hipStream_t st);
   const int32_t* table_of(const Geometry& g, const Run& r) const {
@@ -223,6 +224,7 @@ class LayerStack final : public StepModel {
   // step buffers, sized for rows_ tokens
   int rows_ = 0;
   int ld_q_ = 0, ld_att_ = 0, ld_act_ = 0, ld_shared_ = 0, max_top_ = 0, max_e_ = 0;
+  int y_parts_ = 1;  // of the sublayer that was enqueued last
   DevBuf<float> x_, x_tail_, y_, z_, weight_, part_o_, part_ml_, tap_rows_;
   DevBuf<uint8_t> h_, q_, att_, act_, act_shared_;
   // latent: queries in the latent space, values in it, projected-down rows

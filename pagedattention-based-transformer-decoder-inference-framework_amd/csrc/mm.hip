@@ -60,6 +60,42 @@ static KernelArgs plain_args(int dtype, const MmArgs& a) {
   return p;
 }
 
+// A product of few blocks takes the time of its chain of K, so slices of K fill the chip, and the reader
+// of the sums, a norm, adds them up as it reads.  Priced by the form that each count of slices would take,
+// of whose time K / 2048 is the product's, 0.5 us for a slice more and its sums' way to memory and
+// back at 3 TB/s, and more slices only for 2 % and more.  With the norm behind it (us, weights from memory, 1 / 2 / 4 slices; the choice):
+// bf16 2048 columns of K 4096: 16 rows 13.0 / 10.7 / 10.9 (2), 64 14.4 / 13.5 / 11.4 (4), 333 26.3 / 19.7 /
+// 18.5 (4), 1000 32.7 / 28.4 / 30.8 (2); K 6144: 333 rows 34.2 / 24.5 / 22.3 (4); K 2048: 16 rows 9.0 / 8.2 /
+// 8.1 (2), 333 16.1 / 15.3 / 16.7 (2), 1400 24.8 / 26.4 / 31.2 (1); 1024 columns of K 1024: 1000 rows 13.3 /
+// 14.6 / 17.7 (1).  Over 1 to 2011 rows and 1024 to 4096 columns and K 0.88 of the time in bf16 (the best
+// count each: 0.86), 0.93 in fp32 (0.91).
+template <typename T>
+static int parts_of(KernelArgs p) {
+  int best = 1;
+  float least = 0.f;
+  for (int parts = 1; parts <= kMmMostParts; parts *= 2) {
+    if (parts > 1 && (p.KS / parts < 24 || p.a.M * parts > kMmPartRows)) break;
+    p.a.parts = parts;
+    const float us = form_of<T, kStore>(p).us;
+    if (us == 0.f) break;
+    const float all = kFixedUs + (us - kFixedUs) * (float)p.a.K / (2048.f * (float)parts) +
+                      (float)(parts - 1) * (0.5f + 1.33e-6f * (float)p.a.M * (float)p.a.N);
+    if (parts > 1 && all >= 0.98f * least) continue;
+    best = parts;
+    least = all;
+  }
+  return best;
+}
+
+int mm_parts(int dtype, int M, int N, int K) {
+  MmArgs a;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  const KernelArgs p = plain_args(dtype, a);
+  return dtype == LLM_F32 ? parts_of<float>(p) : parts_of<__bf16>(p);
+}
+
 hipError_t mm(int dtype, const MmArgs& a, hipStream_t st) {
   const KernelArgs p = plain_args(dtype, a);
   return dtype == LLM_F32 ? launch<float, kStore>(p, st) : launch<__bf16, kStore>(p, st);

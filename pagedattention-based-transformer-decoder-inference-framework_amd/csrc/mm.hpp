@@ -103,6 +103,10 @@ struct MmArgs {
   float* C = nullptr;       // [M][ldc]
   float* const* C_at = nullptr;  // (mm only) device word: in place of C, if it holds a pointer
   int ldc = 0;
+  // (mm only) K in `parts` slices, each summed by blocks of its own: C + i c_part has the sums of
+  // slice i (no softcap then)
+  int parts = 1;
+  size_t c_part = 0;
   float softcap = 0.f;      // C = softcap tanh(C / softcap) when set
 };
 
@@ -172,6 +176,10 @@ struct MmPageRows {
 };
 
 hipError_t mm(int dtype, const MmArgs& a, hipStream_t st);
+// Slices of K that mm is fastest with, the sum of them by its reader included; M times as many are at
+// most kMmPartRows rows.
+constexpr int kMmMostParts = 4, kMmPartRows = 8192;
+int mm_parts(int dtype, int M, int N, int K);
 hipError_t mm_split(int dtype, const MmArgs& a, const MmSplit& e, hipStream_t st);
 // W holds gate and up rows interleaved (N = 2 ff); act [M][ld] = glu
 hipError_t mm_glu(int dtype, const MmArgs& a, const GluParams& p, void* act, int ld, hipStream_t st);

@@ -74,7 +74,7 @@ struct KernelArgs {
 // blocks' own stores to the host's memory).
 __device__ __forceinline__ float* stored_to(const KernelArgs& p) {
   float* c = p.a.C_at ? *p.a.C_at : nullptr;
-  return c ? c : p.a.C;
+  return (c ? c : p.a.C) + blockIdx.z * p.a.c_part;
 }
 
 __device__ __forceinline__ float glu(float gate, float up, const GluParams& p) {
@@ -118,6 +118,7 @@ struct Block {
   const T* A = nullptr;
   const char* W = nullptr;
   int lda = 0, M = 0, N = 0, KS = 0, m0 = 0;
+  size_t w_tile = 0;  // bytes from a column tile of W to the next
   bool shared = false;
   GluParams glu;
 };
@@ -158,7 +159,18 @@ __device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_block,
       b.A += blockIdx.z * p.heads.a_head;
       b.W += blockIdx.z * p.heads.w_head;
     }
+    if constexpr (EPI == kStore) {
+      b.w_tile = (size_t)p.KS * 1024;
+      if (p.a.parts > 1) {
+        const int z = blockIdx.z, k0 = z * p.KS / p.a.parts;
+        b.A += (size_t)k0 * (64 / sizeof(T));
+        b.W += (size_t)k0 * 1024;
+        b.KS = (z + 1) * p.KS / p.a.parts - k0;
+      }
+      return b;
+    }
   }
+  b.w_tile = (size_t)b.KS * 1024;
   return b;
 }
 
@@ -882,7 +894,7 @@ __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kerne
   const char* bp[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
-    bp[j] = b.W + (size_t)min(nt0 + j, ntiles - 1) * b.KS * 1024 + lane * 16;
+    bp[j] = b.W + min(nt0 + j, ntiles - 1) * b.w_tile + lane * 16;
 
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -1044,7 +1056,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p)
   block_product<false, !Kind<T>::BF16, MB, NB, WM, WN, ST>(
       lds, acc, KS, b.m0 + 16 * wm * MT < b.M,
       [&](int r) { return a_row<T, EPI>(p, b, b.m0 + r); },
-      [&](int t) { return b.W + (size_t)min(nt0 + t, ntiles - 1) * KS * 1024; },
+      [&](int t) { return b.W + min(nt0 + t, ntiles - 1) * b.w_tile; },
       [](u32x4 x, u32x4 y, f32x4 c) { return Kind<T>::mma(x, y, c); });
   // (block_product has read all of LDS before its last barrier)
   constexpr int STRIDE = 16 * NB + 4;
@@ -1087,7 +1099,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mm_strip_kernel(KernelArgs p) {
   f32x4 acc[MB][NT];
   strip_product<MB, NT, WAVES, ST, AHEAD>(
       lds, acc, KS, [&](int r) { return a_row<T, EPI>(p, b, b.m0 + r); },
-      [&](int j) { return b.W + (size_t)min(nt0 + j, ntiles - 1) * KS * 1024; },
+      [&](int j) { return b.W + min(nt0 + j, ntiles - 1) * b.w_tile; },
       [](u32x4 x, u32x4 y, f32x4 c) { return Kind<T>::mma(x, y, c); });
   if (16 * nt0 >= b.N) return;
   float* sums = reinterpret_cast<float*>(&lds[0][0][0]) + w * 16 * SR * STRIDE;
@@ -1103,8 +1115,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mm_strip_kernel(KernelArgs p) {
 }
 
 template <int EPI>
-int heads_of(const KernelArgs& p) {
-  return EPI == kHeads ? p.heads.heads : 1;
+int heads_of(const KernelArgs& p) {  // and parts of K
+  return EPI == kHeads ? p.heads.heads : EPI == kStore ? p.a.parts : 1;
 }
 
 template <typename T, int EPI, int MT, int NT, int WK = 8, int PARTS = WK>
@@ -1136,6 +1148,22 @@ hipError_t strips(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
   return hipGetLastError();
 }
 
+// How a product runs, and about how long at K = 2048 (us; 0: not told), kFixedUs of it whatever K is.
+struct Form {
+  using Go = hipError_t (*)(const KernelArgs&, int, int, hipStream_t);
+  Go go = nullptr;
+  int row_blocks = 0;
+  float us = 0.f;
+};
+constexpr float kFixedUs = 2.f;
+
+// Rounds of stream blocks, priced by a block's column tiles and the rows it reads (128 column tiles, us of
+// bf16 / fp32: 16 rows 4.7 / 8, 48 to 64 rows 5.5 / 12).
+template <typename T>
+inline float stream_us(int groups, float tiles) {
+  return kFixedUs + (float)((groups + 255) / 256) * (Kind<T>::BF16 ? 1.8f : 4.5f) * tiles;
+}
+
 // A block form, the blocks of it a CU holds (by their LDS), and the time of a round of them at
 // K = 2048 with one, two and three a CU (us, weights from memory).  A product takes the form
 // whose rounds take least.  Two blocks of 64 x 128 a CU hide each other's first loads and last
@@ -1154,23 +1182,19 @@ hipError_t strips(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
 // is nearly the same: over 65 to 2048 rows and 1024 to 12288 columns of bf16 the form so chosen is
 // on average 0.1 to 0.3 % off the best from K 1024 to 8192, 0.8 % at 512, 2.3 % at 256.
 template <typename T, int EPI>
-hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipStream_t st) {
-  hipError_t (*best)(const KernelArgs&, int, int, hipStream_t) = nullptr;
-  int best_y = 0;
-  float least = 0.f;
-  const bool long_k = (EPI == kGroupIn || EPI == kGroupOut ? p.g.min_ks : p.KS) >= 32;
+Form block_form(const KernelArgs& p, int min_mb, int max_mb, int N) {
+  Form best;
+  const bool long_k = (EPI == kGroupIn || EPI == kGroupOut ? p.g.min_ks : EPI == kStore ? p.KS / p.a.parts : p.KS) >= 32;
   const auto consider = [&](int mb, int nb, int per, const float (&bf16)[3], float fp32,
-                            hipError_t (*go)(const KernelArgs&, int, int, hipStream_t), bool strip = false) {
+                            Form::Go go, bool strip = false) {
     if (mb < min_mb || mb > max_mb) return;
     const int y = (p.a.M + 16 * mb - 1) / (16 * mb);
     const dim3 g = block_grid<EPI>(p, y, N, nb);
     const int groups = g.x * g.y * g.z;
     if (strip && groups <= 256 && !long_k) return;
     const float cost = Kind<T>::BF16 ? rounds_us(groups, per, bf16) : (float)((groups + 255) / 256) * fp32;
-    if (best && cost >= least) return;
-    best = go;
-    best_y = y;
-    least = cost;
+    if (best.go && cost >= best.us) return;
+    best = Form{go, y, cost};
   };
   consider(4, 2, 3, {10.8f, 12.1f, 15.6f}, 21.5f, blocks<T, EPI, 4, 2, 4, 1, 4>);
   consider(4, 4, 3, {13.3f, 15.4f, 20.4f}, 37.f, blocks<T, EPI, 4, 4, 2, 2, 3>);
@@ -1183,11 +1207,11 @@ hipError_t launch_block(const KernelArgs& p, int min_mb, int max_mb, int N, hipS
     consider(8, 8, 2, {17.f, 31.f}, 0.f, strips<T, EPI, 8, 2, 4, 4, 8>, true);
     consider(8, 16, 2, {27.f, 53.f}, 0.f, strips<T, EPI, 8, 4, 4, 4, 4>, true);
   }
-  return best(p, best_y, N, st);
+  return best;
 }
 
 template <typename T, int EPI>
-hipError_t launch(const KernelArgs& p, hipStream_t st) {
+Form form_of(const KernelArgs& p) {
   const int M = p.a.M, N = p.a.N;
   const int ntiles = (N + 15) / 16;
   // A model's head: blocks of two tiles read A half as often, which counts once A's rows are
@@ -1199,8 +1223,8 @@ hipError_t launch(const KernelArgs& p, hipStream_t st) {
   // rows: 6.0 / 6.2, 9.4 / 8.9, 16.7 / 17.0.
   if constexpr (EPI == kStore && Kind<T>::BF16)
     if (M <= 16 && M > (p.KS > 64 ? 14 : 8) && p.KS <= 128 && ntiles >= 1000)
-      return stream<T, EPI, 1, 2, 4, 8>(p, 1, N, st);
-  if (M <= 16) return stream<T, EPI, 1, 1>(p, 1, N, st);
+      return Form{stream<T, EPI, 1, 2, 4, 8>, 1};
+  if (M <= 16) return Form{stream<T, EPI, 1, 1>, 1, stream_us<T>(ntiles * heads_of<EPI>(p), 1.5f)};
   if constexpr (EPI == kSplit) {
     // Narrow products: the fewest column tiles a block that are one round, as a block takes the time of
     // its chain of K whatever its width allows (K 4096, 160 columns, us by 1 / 2 / 3 / 5 tiles and 16 rows, 5
@@ -1210,42 +1234,42 @@ hipError_t launch(const KernelArgs& p, hipStream_t st) {
     if (M > 64 && ntiles <= 10) {
       const int rb = (M + 15) / 16;
       const auto one_round = [&](int nt) { return (ntiles + nt - 1) / nt * rb <= 256; };
-      if (one_round(1)) return stream<T, EPI, 1, 1>(p, rb, N, st);
-      if (one_round(2)) return stream<T, EPI, 1, 2>(p, rb, N, st);
-      if (one_round(3)) return stream<T, EPI, 1, 3>(p, rb, N, st);
-      if (one_round(5)) return stream<T, EPI, 1, 5>(p, rb, N, st);
-      if ((M + 31) / 32 * 2 < 1024) return stream<T, EPI, 2, 5>(p, (M + 31) / 32, N, st);
+      if (one_round(1)) return Form{stream<T, EPI, 1, 1>, rb};
+      if (one_round(2)) return Form{stream<T, EPI, 1, 2>, rb};
+      if (one_round(3)) return Form{stream<T, EPI, 1, 3>, rb};
+      if (one_round(5)) return Form{stream<T, EPI, 1, 5>, rb};
+      if ((M + 31) / 32 * 2 < 1024) return Form{stream<T, EPI, 2, 5>, (M + 31) / 32};
     }
   }
   // Blocks once the smallest of them are more than half a round, else streams:
   // 64 x 6144 x 1024 5.1 us as blocks (streams 5.3), 64 x 2048 x 6144 10.7 as
   // streams (blocks 15.4), 128 x 2048 x 6144 16.3 as streams (blocks 17.5).
   if (M > 32 && (M + 63) / 64 * ((N + 31) / 32) * heads_of<EPI>(p) > 128)
-    return launch_block<T, EPI>(p, 4, 8, N, st);
+    return block_form<T, EPI>(p, 4, 8, N);
   // The stream form with the fewest rounds of workgroups, a round priced by its
   // column tiles and the rows it reads.
-  struct Form {
+  struct Tiles {
     int mt, nt;
     float rows;
-    hipError_t (*go)(const KernelArgs&, int, int, hipStream_t);
+    Form::Go go;
   };
-  static constexpr Form forms[] = {{1, 1, 0.5f, stream<T, EPI, 1, 1>},
-                                   {1, 2, 0.5f, stream<T, EPI, 1, 2>},
-                                   {2, 2, 1.5f, stream<T, EPI, 2, 2>},
-                                   {2, 3, 1.5f, stream<T, EPI, 2, 3>}};
-  const Form* best = nullptr;
-  int row_blocks = 0;
-  float least = 0.f;
-  for (const Form& f : forms) {
+  static constexpr Tiles forms[] = {{1, 1, 0.5f, stream<T, EPI, 1, 1>},
+                                    {1, 2, 0.5f, stream<T, EPI, 1, 2>},
+                                    {2, 2, 1.5f, stream<T, EPI, 2, 2>},
+                                    {2, 3, 1.5f, stream<T, EPI, 2, 3>}};
+  Form best;
+  for (const Tiles& f : forms) {
     const int rb = (M + 16 * f.mt - 1) / (16 * f.mt);
-    const int groups = (ntiles + f.nt - 1) / f.nt * rb * heads_of<EPI>(p);
-    const float cost = (float)((groups + 255) / 256) * ((float)f.nt + f.rows);
-    if (best && cost >= least) continue;
-    best = &f;
-    least = cost;
-    row_blocks = rb;
+    const float us = stream_us<T>((ntiles + f.nt - 1) / f.nt * rb * heads_of<EPI>(p), (float)f.nt + f.rows);
+    if (!best.go || us < best.us) best = Form{f.go, rb, us};
   }
-  return best->go(p, row_blocks, N, st);
+  return best;
+}
+
+template <typename T, int EPI>
+hipError_t launch(const KernelArgs& p, hipStream_t st) {
+  const Form f = form_of<T, EPI>(p);
+  return f.go(p, f.row_blocks, p.a.N, st);
 }
 
 template <typename T, int EPI>
@@ -1253,8 +1277,10 @@ hipError_t launch_grouped(const MmGrouped& g, int w_nt, hipStream_t st) {
   KernelArgs p{};
   p.g = g;
   p.a.w_nt = w_nt;
-  if (g.tile_rows > 16)
-    return launch_block<T, EPI>(p, g.tile_rows / 16, g.tile_rows / 16, g.max_n, st);
+  if (g.tile_rows > 16) {
+    const Form f = block_form<T, EPI>(p, g.tile_rows / 16, g.tile_rows / 16, g.max_n);
+    return f.go(p, f.row_blocks, g.max_n, st);
+  }
   // bf16: at least eight k-steps a wave (an expert's output product of 32 k-steps over 37 tiles
   // 26 us by eight waves, 20.5 by four; of 16 over 52 15.2, 10.5 by two), the sums in as many
   // parts as by eight.  Two waves a workgroup are too few in flight while a CU has but two or

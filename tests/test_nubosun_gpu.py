@@ -516,6 +516,22 @@ def test_long_prompts_of_wide_layers(serve, dtype):  # noqa: F811
         T.check_rows(got[i], want[i], dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("inner,ff", [(1570, 800), (3100, 3200), (6200, 1540)])
+def test_slices_of_an_output_product(serve, inner, ff, dtype):  # noqa: F811
+    """Output products whose K is summed in slices, of even and odd numbers of k-steps, by every
+    form; last rows alone, of which there are other slices than of the prompt."""
+    cfg = N.config([(N.mamba(inner=inner, state=2), N.dense(ff=ff)), (N.mamba(inner=inner, state=2), None)],
+                   width=90, vocab=80, streams=2)
+    w = N.weights(cfg, 51)
+    eng = serve(cfg, w, dtype, max_seqs=2, max_tokens=64 * 14)
+    t = tokens(cfg, 800, 52)
+    want = T.logits(cfg, w, t)
+    for n in (1, 17, 33, 65, 130, 800):
+        T.check_rows(run_whole(eng, t[:n]), want[:n], dtype)
+    T.check_last_rows(eng, cfg, w, dtype, t[:100], tokens(cfg, 130, 53))
+
+
 def test_greedy_generation_through_the_scheduler(serve):  # noqa: F811
     cfg = MODELS["plain"]
     w = N.weights(cfg, 45)
