@@ -703,7 +703,15 @@ int LayerStack::attention(const Layer& l, const Run& r, int M, const Tail* tail,
   e.k_pool = kv.k_pool;
   e.v_pool = kv.v_pool;
   e.page_stride = kv.page_stride();
-  LLM_HIP_RET(mm_qkv(dt_, p, e, st));
+  MmArgs queries;
+  if (some_rows(p, tail, 0, a.heads * a.dim, &queries)) {
+    MmQkv rest = e;
+    rest.H = 0;
+    LLM_HIP_RET(mm_qkv(dt_, p, rest, st));
+    if (tail->n > 0) LLM_HIP_RET(mm_qkv(dt_, queries, e, st));
+  } else {
+    LLM_HIP_RET(mm_qkv(dt_, p, e, st));
+  }
   if (tail && tail->n == 0) return LLM_OK;
 
   const Plan& plan = *plans_[l.plan];
@@ -737,6 +745,22 @@ int LayerStack::attention(const Layer& l, const Run& r, int M, const Tail* tail,
   }
 
   return out_product(l, att_.p, ldo, a.heads * a.vdim, tail ? tail->n : M, st);
+}
+
+// Of a tail's input product, the columns [c0, c0 + cols) that its wanted rows alone need (queries, gates; the
+// first or the last ones) leave `a` for a product of those rows where that is faster.  Prompts of two
+// layers, us: Gefarax large 2,048 tokens 590 -> 565, float32 500 979 -> 897; Nubosun large 2,011 653 -> 633.
+bool LayerStack::some_rows(MmArgs& a, const Tail* tail, int c0, int cols, MmArgs* some) const {
+  if (!tail || c0 % 16 != 0 || (a.N - cols) % 16 != 0 || !mm_apart(dt_, a.M, a.N, a.K, tail->n, cols)) return false;
+  const auto columns = [&](int n) { return static_cast<const uint8_t*>(a.W) + mm_packed_bytes(dt_, n, a.K); };
+  *some = a;
+  some->W = columns(c0);
+  some->N = cols;
+  some->M = tail->n;
+  some->rows = meta<int32_t>(at_want_);
+  if (c0 == 0) a.W = columns(cols);
+  a.N -= cols;
+  return true;
 }
 
 int LayerStack::out_product(const Layer& l, const void* A, int lda, int K, int M, hipStream_t st) {

@@ -192,6 +192,7 @@ class LayerStack final : public StepModel {
   int mamba(const Layer& l, const Run& r, int M, const Tail* tail, hipStream_t st);
   int out_product(const Layer& l, const void* A, int lda, int K, int M, hipStream_t st);
   int sublayer_product(MmArgs& a, hipStream_t st);
+  bool some_rows(MmArgs& a, const Tail* tail, int c0, int cols, MmArgs* some) const;
   int moe(const Layer& l, int M, hipStream_t st);
   int ffn(const Layer& l, int M, hipStream_t st);
   const int32_t* table_of(const Geometry& g, const Run& r) const {

@@ -159,7 +159,15 @@ int LayerStack::latent(const Layer& l, const Run& r, int M, const Tail* tail, hi
   e.lat_rot = latent_rot_at(a.rank);
   e.down = down_.p;
   e.ldd = rank + a.rot_dim;
-  LLM_HIP_RET(mm_latent(dt_, p, e, st));
+  MmArgs queries;
+  if (some_rows(p, tail, 0, a.heads * (dim + a.rot_dim), &queries)) {
+    MmLatent rest = e;
+    rest.H = 0;
+    LLM_HIP_RET(mm_latent(dt_, p, rest, st));
+    if (tail->n > 0) LLM_HIP_RET(mm_latent(dt_, queries, e, st));
+  } else {
+    LLM_HIP_RET(mm_latent(dt_, p, e, st));
+  }
 
   MmPageRows rows;  // the new tokens' rows
   rows.pos = meta<int32_t>(at_pos_);

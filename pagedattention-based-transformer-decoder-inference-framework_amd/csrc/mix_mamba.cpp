@@ -143,7 +143,13 @@ int LayerStack::mamba(const Layer& l, const Run& r, int M, const Tail* tail, hip
     MmSplit s;
     s.t = xz_.p;
     s.ldt = s.n_t = 2 * ldc;
+    MmArgs gates;
+    const bool apart = some_rows(a, tail, ldc, ldc, &gates);
     LLM_HIP_RET(mm_split(dt_, a, s, st));
+    if (apart && tail->n > 0) {
+      s.t = z;
+      LLM_HIP_RET(mm_split(dt_, gates, s, st));
+    }
     ConvArgs c;
     c.M = M;
     c.channels = m.inner;

@@ -3,6 +3,8 @@
 // in mm_impl.hpp; mm_mix.hip has the epilogues of the other mixers.
 #include "mm_impl.hpp"
 
+#include <cmath>
+
 namespace llm {
 namespace {
 
@@ -94,6 +96,30 @@ int mm_parts(int dtype, int M, int N, int K) {
   a.K = K;
   const KernelArgs p = plain_args(dtype, a);
   return dtype == LLM_F32 ? parts_of<float>(p) : parts_of<__bf16>(p);
+}
+
+template <typename T>
+static float whole_us(KernelArgs p, int M, int N) {
+  if (M == 0) return 0.f;
+  p.a.M = M;
+  p.a.N = N;
+  const float us = form_of<T, kStore>(p).us;
+  if (us == 0.f) return NAN;  // not priced
+  return kFixedUs + (us - kFixedUs) * (float)p.a.K / 2048.f;
+}
+
+// By mm's prices: a launch more is in them, the rows' pages and rotations are not (2048 rows x 2560 columns
+// x 2048 to pages 39 us, priced 28; their 512 columns of keys and values 15.6 and one row's queries 5.7, priced
+// 12.1 and 4.7; a scan's 2011 x 8192 60, priced 53; 4096 of its columns 34.8 and three rows' 6.9, priced 27 and 4.7).
+bool mm_apart(int dtype, int M, int N, int K, int rows, int cols) {
+  if (cols % 16 != 0 || cols >= N) return false;  // (a column tile of packed weights holds 16)
+  MmArgs a;
+  a.K = K;
+  const KernelArgs p = plain_args(dtype, a);
+  const auto us = [&](int m, int n) {
+    return dtype == LLM_F32 ? whole_us<float>(p, m, n) : whole_us<__bf16>(p, m, n);
+  };
+  return us(M, N - cols) + us(rows, cols) < us(M, N);
 }
 
 hipError_t mm(int dtype, const MmArgs& a, hipStream_t st) {

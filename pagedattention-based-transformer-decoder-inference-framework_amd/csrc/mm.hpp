@@ -107,6 +107,9 @@ struct MmArgs {
   // slice i (no softcap then)
   int parts = 1;
   size_t c_part = 0;
+  // (mm_qkv, mm_latent, mm_split) only these rows of A, of the results and of what belongs to rows take
+  // part (M: their number)
+  const int32_t* rows = nullptr;
   float softcap = 0.f;      // C = softcap tanh(C / softcap) when set
 };
 
@@ -180,6 +183,9 @@ hipError_t mm(int dtype, const MmArgs& a, hipStream_t st);
 // most kMmPartRows rows.
 constexpr int kMmMostParts = 4, kMmPartRows = 8192;
 int mm_parts(int dtype, int M, int N, int K);
+// Whether `cols` of the N columns, of which `rows` of the M rows are wanted alone, are faster as a product
+// of their own behind that of the others.
+bool mm_apart(int dtype, int M, int N, int K, int rows, int cols);
 hipError_t mm_split(int dtype, const MmArgs& a, const MmSplit& e, hipStream_t st);
 // W holds gate and up rows interleaved (N = 2 ff); act [M][ld] = glu
 hipError_t mm_glu(int dtype, const MmArgs& a, const GluParams& p, void* act, int ld, hipStream_t st);

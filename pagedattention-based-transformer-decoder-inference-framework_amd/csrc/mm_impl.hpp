@@ -174,6 +174,12 @@ __device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_block,
   return b;
 }
 
+// Products of which only some rows may be wanted (MmArgs::rows).
+template <int EPI>
+constexpr bool some_rows() {
+  return EPI == kQkv || EPI == kLatent || EPI == kSplit;
+}
+
 // Row m of A (the last one for rows past it).
 template <typename T, int EPI>
 __device__ __forceinline__ const char* a_row(const KernelArgs& p, const Block<T>& b, int m) {
@@ -183,6 +189,9 @@ __device__ __forceinline__ const char* a_row(const KernelArgs& p, const Block<T>
   }
   if constexpr (EPI == kHeads) {
     if (p.heads.rows) m = p.heads.rows[m];
+  }
+  if constexpr (some_rows<EPI>()) {
+    if (p.a.rows) m = p.a.rows[m];
   }
   if constexpr (EPI == kExpand) {
     const MmPageRows& r = p.page_rows;
@@ -218,6 +227,9 @@ struct RowOf {
   __device__ __forceinline__ RowOf(const KernelArgs& p, const Block<T>& b, int row) {
     if (row >= b.M) return;
     m = row;
+    if constexpr (some_rows<EPI>()) {
+      if (p.a.rows) m = p.a.rows[row];
+    }
     if constexpr (PAGED) {
       const MmQkv& e = p.q;
       pos = e.pos[m];

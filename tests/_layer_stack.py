@@ -186,6 +186,23 @@ def check_last_rows(eng, cfg, w, dtype, a, b):
         eng.close_seq(s)
 
 
+def check_long_last_rows(eng, cfg, w, dtype, t, n):
+    """A prompt of n tokens of which the last row is wanted, and the same in two portions, of the
+    first of which none is, each with two tokens behind it."""
+    full = logits(cfg, w, t[:n + 2])
+    for sizes in ([n], [n - 40, 40]):
+        s, at, got, where = eng.open_seq(), 0, [], []
+        for size in sizes + [1, 1]:
+            at += size
+            want = at >= n
+            out = np.asarray(eng.step([(s, t[at - size:at], [size - 1] if want else [])]))
+            if want:
+                got.append(out[0])
+                where.append(at - 1)
+        eng.close_seq(s)
+        check_rows(np.stack(got), full[where], dtype)
+
+
 def random_schedule(requests, live, seed):
     """Mixed steps: some requests decode, others bring portions, some pause."""
     rng = np.random.default_rng(seed)

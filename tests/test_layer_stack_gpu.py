@@ -269,6 +269,19 @@ def test_last_layer_of_few_wanted_rows(serve, name, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,dim", [(64, 32), (63, 36)])
+def test_queries_of_the_wanted_rows_alone(serve, heads, dim, dtype):
+    """Prompts past and below the rows from which the last layer's queries are a product of their
+    own; heads that end inside a column tile of the packed weights, which stay one product."""
+    cfg = T.config([(T.attn(heads=heads, kv_heads=1, dim=dim), None)], width=1024, vocab=60)
+    w = model_weights(cfg, 61, dtype)
+    eng = serve(cfg, w, dtype, max_seqs=2, max_tokens=64 * 18)
+    t = tokens(cfg, 1030, 62)
+    for n in (60, 220, 1028):
+        T.check_long_last_rows(eng, cfg, w, dtype, t, n)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", sorted(MODELS))
 def test_mixed_batches_with_pages_and_slots_used_again(serve, name, dtype):
     """A pool that just holds the live requests: unequal requests, together and

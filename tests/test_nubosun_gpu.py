@@ -242,6 +242,20 @@ def test_last_layer_of_few_wanted_rows(serve, name, dtype):  # noqa: F811
     T.check_last_rows(serve(cfg, w, dtype), cfg, w, dtype, tokens(cfg, 110, 50), tokens(cfg, 140, 51))
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("layer", [N.latent(heads=32, dim=48, vdim=8, rot=16, rank=32), N.mamba(inner=2030, state=4)],
+                         ids=["latent", "scan"])
+def test_queries_and_gates_of_the_wanted_rows_alone(serve, layer, dtype):  # noqa: F811
+    """Prompts past and below the rows from which the last layer's queries or gates are a product
+    of their own."""
+    cfg = N.config([(layer, None)], width=1024, vocab=60, streams=1)
+    w = N.weights(cfg, 61)
+    eng = serve(cfg, w, dtype, max_seqs=2, max_tokens=64 * 18)
+    t = tokens(cfg, 1030, 62)
+    for n in (60, 220, 1028):
+        T.check_long_last_rows(eng, cfg, w, dtype, t, n)
+
+
 def test_residual_after_every_layer(serve):  # noqa: F811
     cfg = N.config([(N.latent(), N.dense()), (N.mamba(), None)], loop=(0, 2, 2), width=100)
     w = N.weights(cfg, 21)
