@@ -575,7 +575,6 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
   }
   const Layer& last = *layers_[runs_.back().layer];
   tail_.small = tail_.big = Launch();
-  tail_.n_scan = 0;
   if (last.plan >= 0) {
     launch_of(wanted, *plans_[last.plan], false, tail_.small);
     launch_of(wanted, *plans_[last.plan], true, tail_.big);
@@ -611,21 +610,19 @@ int LayerStack::build_meta(const std::vector<StepSeq>& batch, int M, int n_want,
     }
   }
   size_t parts = 0;
-  for (ScanPlan& p : scans_) {
+  const auto scan_of = [&](bool tail, ScanPlan& p) {
     std::vector<ScanItem> items, chunks;
     std::vector<ScanCarry> carry;
-    plan_scan(batch, false, p, items, chunks, carry);
+    plan_scan(batch, tail, p, items, chunks, carry);
     p.items_at = place(items);
     p.chunks_at = place(chunks);
     p.carry_at = place(carry);
     parts = std::max(parts, (size_t)p.parts);
-    if (!tail_.on || last.scan < 0 || &p != &scans_[last.scan]) continue;
-    items.clear();
-    ScanPlan again = p;
-    again.parts = 0;
-    plan_scan(batch, true, again, items, chunks, carry);
-    tail_.n_scan = (int)items.size();
-    tail_.scan_at = place(items);
+  };
+  for (ScanPlan& p : scans_) scan_of(false, p);
+  if (tail_.on && last.scan >= 0) {
+    tail_.scan = scans_[last.scan];
+    scan_of(true, tail_.scan);
   }
   if (part_o > part_o_.n || part_ml > part_ml_.n || at > meta_cap_ ||
       parts * carry_floats_ > carry_.n) {

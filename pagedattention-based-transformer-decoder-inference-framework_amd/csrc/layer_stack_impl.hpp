@@ -144,8 +144,7 @@ class LayerStack final : public StepModel {
     bool on = false;
     int n = 0;           // wanted rows
     Launch small, big;   // attention of the wanted rows, a portion each
-    int n_scan = 0;
-    size_t scan_at = 0;
+    ScanPlan scan;
   };
 
   int init_latent(Layer& l);
