@@ -504,7 +504,8 @@ int llm_decoder_set_taps(llm_decoder* d, int8_t* q_dev, float* s_dev);
  * LLM_PA_FORM_SPLIT_MERGE_ROW | LLM_PA_FORM_BEAM.  FP16
  * decoders (head_dim <= 128, <= 64 heads) whose launch merges in the workgroup
  * run o_proj inside it: LLM_PA_FORM_WG_MERGE | LLM_PA_FORM_OPROJ; LLM_PA_FORM_DIRECT
- * and LLM_PA_FORM_SPLIT_MERGE_ROW write its packed fp16 input. */
+ * and LLM_PA_FORM_SPLIT_MERGE_ROW write its packed fp16 input.  (A step of up to 8 rows of an INT8
+ * decoder of hidden 256 has no such launch while they are short: csrc/row_step.hip.) */
 int llm_decoder_attention_plan(llm_decoder* d, int* nsplit, int* form);
 /* Enqueue layer `layer`'s attention launch of the decoder's step on `stream`
  * (NULL: the decoder's) -- the same kernels, grid and outputs as inside the

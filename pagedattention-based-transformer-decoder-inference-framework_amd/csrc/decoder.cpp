@@ -31,6 +31,7 @@
 #include "common.hpp"
 #include "dev_buf.hpp"
 #include "gemm.hpp"
+#include "row_step.hpp"
 #include "kv_cache_impl.hpp"
 #include "model.hpp"
 #include "pa_decode.hpp"
@@ -125,6 +126,7 @@ struct llm_decoder {
 
   hipGraphExec_t graph = nullptr;
   int graph_batch = -1;
+  bool graph_rows = false;  // by row_step
 
   // activation taps (llm_decoder_set_taps): the int8 GEMM inputs and row scales
   // of every layer, copied out by the step for teacher-forced parity checks
@@ -166,6 +168,8 @@ struct llm_decoder {
   bool fc2_quant_prologue(const struct Rows& R) const;
   int layer_post(int l, hipStream_t st, const struct Rows& R);
   int layers(hipStream_t st, const struct Rows& R, int r0);
+  bool rows_alone() const;
+  int run_rows(hipStream_t st);
   struct Rows step_rows(int r0, int n, uint8_t* ws);
   void embed_rows(const int32_t* tok);
   int step_tail(hipStream_t st, int r0, int n, float* const* place, float* to);
@@ -831,8 +835,45 @@ int llm_decoder::step_tail(hipStream_t st, int r0, int n, float* const* place, f
                      place, to);
 }
 
+// Whether the step's rows each go through all layers in a workgroup of their own (row_step.hip).
+bool llm_decoder::rows_alone() const {
+  if (wdtype != LLM_I8 || row_group != 1 || tap_q) return false;
+  return row_step_ok(hid, inter, D, TS, batch, 1 + *std::max_element(h_pos.begin(), h_pos.begin() + batch));
+}
+
+int llm_decoder::run_rows(hipStream_t st) {
+  pa_kv_view view;
+  RET_IF(kv_cache_view(kv, 0, &view));
+  RowStep a;
+  a.L = L; a.D = D; a.V = V; a.rows = batch;
+  a.emb = reinterpret_cast<const _Float16*>(emb.p);
+  a.tok = tokens.p;
+  a.pos = pos.p;
+  a.ln1_g = ln1_g.p; a.ln1_b = ln1_b.p; a.ln2_g = ln2_g.p; a.ln2_b = ln2_b.p;
+  a.qkv = RowProduct{wqkv.p, sz_qkv, sw_qkv.p, nullptr};
+  a.o = RowProduct{wo.p, sz_o, sw_o.p, nullptr};
+  a.fc1 = RowProduct{w1.p, sz_1, sw1.p, b1.p};
+  a.fc2 = RowProduct{w2.p, sz_2, sw2.p, b2.p};
+  a.page_table = view.page_table;
+  a.beams = view.num_beams;
+  a.max_tiles = view.max_tiles;
+  a.num_pages = view.num_pages;
+  a.page_shift = __builtin_ctz((unsigned)view.page_size);
+  a.k_pool = static_cast<_Float16*>(kv_cache_k_pool(kv));
+  a.v_pool = static_cast<_Float16*>(kv_cache_v_pool(kv));
+  a.page_stride = (size_t)view.page_stride / sizeof(_Float16);
+  a.attn_scale = cfg.attn_scale;
+  a.x = x.p;
+  LLM_HIP_RET(row_step(a, st));
+  return LLM_OK;
+}
+
 // One decode step of all active rows (captured into the step graph).
 int llm_decoder::enqueue_step(hipStream_t st, float* const* place, float* to) {
+  if (rows_alone()) {
+    RET_IF(run_rows(st));
+    return step_tail(st, 0, batch, place, to);
+  }
   Rows R = step_rows(0, batch, attn_ws.p);
   if (oproj_fusable(R)) R.oacc = oacc.p, R.oproj_out = R.x, R.oflag = oflag.p;
   R.wgm_quant = wgm_quant_ok(R);
@@ -892,7 +933,7 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
   if (!use_graph) {
     RET_IF(enqueue_step(st, nullptr, to));
   } else {
-    if (graph_batch != batch) {
+    if (graph_batch != batch || graph_rows != rows_alone()) {
       if (graph) { (void)hipGraphExecDestroy(graph); graph = nullptr; }
       hipGraph_t g;
       LLM_HIP_RET(hipStreamSynchronize(st));
@@ -907,6 +948,7 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
       if (e != hipSuccess)
         return fail(LLM_ERR_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
       graph_batch = batch;
+      graph_rows = rows_alone();
     }
     LLM_HIP_RET(hipGraphLaunch(graph, st));
   }

@@ -1066,3 +1066,60 @@ def test_synthetic_context_bits(gpu, oracle, max_batch, max_seq):
         want = (x.astype(np.float64) * np.float64(scale)).astype(np.float16)
         got = pool[:, which].reshape(-1)[at]
         assert np.array_equal(got.view(np.uint16), want.view(np.uint16)), which
+
+
+@pytest.mark.parametrize("H,D,page,rows", [(4, 64, 16, 1), (4, 64, 32, 8), (2, 128, 16, 3), (8, 32, 32, 2),
+                                           (8, 32, 16, 5)])
+def test_rows_of_hidden_256_by_themselves(gpu, oracle, H, D, page, rows):
+    """Up to 8 rows of up to 512 tokens go through all layers in one workgroup each: against the
+    launches of 9 rows (the same ones and copies of the first), at contexts around pages, the lanes' and waves'
+    shares and the bound, where the next step goes by launches again.  Of the steps, whose activations on the
+    edge of two int8 values may take the other, more than half agree to fp32 sums' order."""
+    import llm_decoder
+    torch = _torch()
+    V, S = 300, 600
+    w = _int8_model(oracle, L=2, H=H, D=D, V=V, S=S, seed=71)
+    prompts = np.random.default_rng(72).integers(0, V, (rows, S))
+    got = []
+    for n_rows in (rows, 9):
+        c = w["cfg"]
+        dec = llm_decoder.INT8Decoder(c["L"], H, D, c["hid"], V, S, max_batch=n_rows, page_size=page)
+        dec.set_weights(_weights_dict(w))
+        dec.begin_synthetic(n_rows, 0, 0, False)
+        logits = torch.empty((n_rows, V), device="cuda")
+        mine, at = [], 0
+        for n in (0, 1, 15, 16, 31, 32, 33, 63, 64, 127, 128, 129, 257, 400, 510, 511, 512, 513):
+            own = [r if r < rows else 0 for r in range(n_rows)]
+            if n > at:
+                for r in range(n_rows):
+                    dec.prefill(r, prompts[own[r]][at:n].tolist())
+            dec.step([int(prompts[own[r]][n]) for r in range(n_rows)], logits_ptr=logits.data_ptr())
+            torch.cuda.synchronize()
+            mine.append(logits[:rows].cpu().numpy())
+            at = n + 1
+        got.append(np.stack(mine))
+    assert np.isfinite(got[0]).all()
+    err = np.abs(got[0] - got[1]).max(axis=-1) / np.abs(got[1]).max(axis=-1)
+    assert err.max() < FREE_RUN_TOL, err.max()
+    assert np.median(err) < 1e-5, err
+
+
+def test_rows_of_other_lengths_by_themselves(gpu, oracle):
+    """Rows of lengths of their own in one step, against each alone."""
+    torch = _torch()
+    V, S = 300, 300
+    w = _int8_model(oracle, L=2, V=V, S=S, seed=73)
+    prompts = [np.random.default_rng(74 + r).integers(0, V, n).tolist() for r, n in enumerate((2, 17, 130, 255))]
+    together = None
+    for batch in ([0, 1, 2, 3], [0], [1], [2], [3]):
+        dec = _make_gpu_decoder(w, max_batch=len(batch))
+        dec.begin_synthetic(len(batch), 0, 0, False)
+        for r, p in enumerate(batch):
+            dec.prefill(r, prompts[p][:-1])
+        logits = torch.empty((len(batch), V), device="cuda")
+        dec.step([prompts[p][-1] for p in batch], logits_ptr=logits.data_ptr())
+        torch.cuda.synchronize()
+        if together is None:
+            together = logits.cpu().numpy()
+        else:
+            assert (logits[0].cpu().numpy() == together[batch[0]]).all()
