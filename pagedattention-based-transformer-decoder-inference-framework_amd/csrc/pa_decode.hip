@@ -586,10 +586,13 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
 // make 9 to 95 splits of few pairs, most of them empty where the sequences are short of the longest held,
 // T, and merged in odd batches.  Steps of 2 layers, rows x heads of D, T (held), us, before -> now:
 //  * at most 16 up to 64 pairs (24 of more than 8 pairs of 128 past 9,600 tokens): 1 x 4 of 64 T 7,144 (1,000) 68 -> 62, T 12,144 (6,000) 93 -> 75; 1 x 16 of
-//    128 T 7,144 (1,000) 134 -> 125, T 4,520 (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 11, 16
-//    in place of more: 16 x 4 of 64 T 4,520 (4,500) 97 -> 95, T 7,144 (1,000) 80 -> 77;
+//    128 T 7,144 (1,000) 134 -> 125, T 4,520 (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 12, 16
+//    in place of more than 16: 16 x 4 of 64 T 4,520 (4,500) 97 -> 95;
 //  * 8 up to 128: 8 x 16 of 128 T 4,520 (4,500) 243 -> 220, 32 x 4 of 64 146 -> 133; past that merged in the
 //    workgroup: 16 x 12 of 64 T 8,192 (2,048) 140 -> 133, T 12,144 (6,000) 217 -> 194;
+//  * 13 to 16 of 33 to 128 pairs stay: three decoders in turns, 4 layers, 16 x 4 of 64 T 6,744 14 splits 83.1, 16
+//    86.0; 32 x 4 T 7,144 14 splits 120.5, 8 125.6; 8 x 16 of 128 209.8, 212.7 (alone the same), where 25 x 4 T 10,144
+//    20 splits 147.9, 8 140.6; 3 x 16 T 12,144 24 splits 129.0, 16 122.3;
 //  * more than 256 pairs of 64: 4 in place of 8 (64 x 12 T 8,192 (2,048) 275 -> 257, 32 x 12 186 -> 177), and
 //    past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
 struct F32Form {
@@ -600,8 +603,9 @@ F32Form f32_step_form(long long bh, int D, int tiles, int nsplit) {
   const bool wgm = nsplit <= kWgmMaxSplits;
   if (nsplit >= 2 && bh > 512 && tiles <= kMaxPps) return {1, false};
   if (wgm) return {D <= 64 && bh > 256 && tiles <= 4 * kMaxPps ? std::min(nsplit, 4) : nsplit, true};
+  if (bh > 32 && bh <= 128 && nsplit > 12 && nsplit <= 16) return {nsplit, wgm};
   const int few = D > 64 && bh > 8 && tiles > 600 ? 24 : 16;
-  const int n = bh <= 32 ? std::min(nsplit, few) : bh <= 64 ? (nsplit > 12 ? 16 : 12) : 8;
+  const int n = bh <= 32 ? std::min(nsplit, few) : bh <= 64 ? (nsplit > 16 ? 16 : 12) : 8;
   if ((long long)n * kMaxPps < tiles) return {nsplit, false};
   return {n, bh > 128};
 }

@@ -200,7 +200,7 @@ def test_f16_step_forms(gpu, B, H, D, S, nsplit, form):
 
 @pytest.mark.parametrize("B,H,D,S,nsplit,form", [
     (64, 12, 64, 700, 1, 0), (48, 12, 64, 8100, 4, 3), (16, 12, 64, 8300, 8, 3),  # past 512, 256, 128 pairs
-    (1, 4, 64, 12100, 16, 1), (1, 16, 128, 12100, 24, 1), (4, 12, 64, 4600, 12, 1), (16, 4, 64, 7100, 16, 1),
+    (1, 4, 64, 12100, 16, 1), (1, 16, 128, 12100, 24, 1), (4, 12, 64, 4600, 12, 1), (16, 4, 64, 7100, 14, 1), (16, 4, 64, 9000, 16, 1),
     (8, 16, 128, 4600, 8, 1), (2, 3, 64, 90, 1, 0), (16, 16, 128, 700, 2, 3),
 ], ids=str)
 def test_int8_step_forms(gpu, oracle, B, H, D, S, nsplit, form):
