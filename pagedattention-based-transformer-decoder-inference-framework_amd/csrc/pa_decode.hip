@@ -552,10 +552,13 @@ int choose_nsplit(int B, int H, int ntiles, int pps_fixed, long long resident,
 //  * few pairs of long rows leave CUs idle, so splits over more workgroups: 4 x 16 of 128 T 1,920 241 ->
 //    216, T 8,192 with 2,048 held 246 -> 222; 16 x 4 of 64 T 8,300 180 -> 151 by 12.  Heads of 64 with 17 to
 //    64 pairs do so past 8,192 tokens, as a step's sequences may be far shorter than T (T 7,144 with 1,000
-//    held: 4 x 16 of 64 by 4 waves 120, 12 splits 134).  And 16 of them at most, 12 from 33 pairs on, not 24
+//    held: 4 x 16 of 64 by 4 waves 120, 12 splits 134), more than 64 pairs of 128 never (three decoders in turns, 8 x 16
+//    T 7,144 with 1,000 held and more 220, 8 splits 228).  And 16 of them at most, 12 from 33 pairs on, not 24
 //    to 64 (1 x 8 of 128 T 7,144 with 1,000 held 103 -> 94, T 12,144 with 6,000 129 -> 118).
 //  * else 4 waves: 16 x 12 of 64 T 8,192 with 2,048 held 162 -> 156 (by 8), T 2,720 167 -> 161 (by 3).
-//    Up to 32 KB of W_o, which one wave's columns cover, 2 to 4 as before (64 x 4 of 64 T 1,920 175; by 4 179).
+//    Up to 128 pairs as before (three decoders in turns, 4 layers, 5 x 16 of 64 T 6,644 by 7 101.5, by 4 111.0;
+//    10 x 12 T 7,644 118.5, 125.9; 12 x 16 by 8 157.1, by 4 155.4), and up to 32 KB of W_o, which one wave's columns cover (64 x 4 of 64 T 1,920 175; by 4 179; three
+//    decoders in turns, 16 x 4 T 6,744 with 600 held and more, by 8 76.4, by 4 85.5).
 struct F16Form {
   int nsplit;
   bool fused;
@@ -567,16 +570,16 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
                         : kb >= 256 ? (bh > 256 ? 20 : 0)
                                     : (bh > 400 ? 25 : bh > 256 ? 10 : 0);
   if (fits && tiles <= kMaxPps && (bh > 512 || tiles <= one)) return {1, false};
-  const bool apart = D > 64 ? bh <= 128 && tiles > (kb >= 512 || bh <= 64 ? 45 : 200)
+  const bool apart = D > 64 ? tiles > (bh <= 64 ? 45 : INT_MAX)
                             : tiles > (bh <= 16 ? 110 : bh <= 64 ? 512 : INT_MAX);
   if (nsplit > 1 && apart) {
-    int n = bh <= 32 ? (fits ? 8 : 16) : bh > 64 || (D > 64 && tiles <= 256) ? 8 : 12;
+    int n = bh <= 32 ? (fits ? 8 : 16) : D > 64 && tiles <= 256 ? 8 : 12;
     if (!fits) n = std::min(n, nsplit);
     if ((long long)n * kMaxPps >= tiles) return {n, false};
   }
   if (!fits) return {nsplit, false};
   if (tiles <= 4 * kMaxPps && bh > (kb >= 512 ? 400 : 512) && kb >= 256) return {4, false};
-  int n = kb >= 512 || (kb >= 256 && bh <= 256) ? 8 : kb <= 32 ? std::min(nsplit, 4) : 4;
+  int n = kb >= 512 || (kb >= 256 && bh <= 256) ? 8 : kb <= 32 || bh <= 128 ? nsplit : 4;
   while (n < kWgmMaxSplits && (long long)n * kMaxPps < tiles) n *= 2;
   return {std::min(n, kWgmMaxSplits), true};
 }
@@ -593,8 +596,8 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
 //  * 13 to 16 of 33 to 128 pairs stay: three decoders in turns, 4 layers, 16 x 4 of 64 T 6,744 14 splits 83.1, 16
 //    86.0; 32 x 4 T 7,144 14 splits 120.5, 8 125.6; 8 x 16 of 128 209.8, 212.7 (alone the same), where 25 x 4 T 10,144
 //    20 splits 147.9, 8 140.6; 3 x 16 T 12,144 24 splits 129.0, 16 122.3;
-//  * more than 256 pairs of 64: 4 in place of 8 (64 x 12 T 8,192 (2,048) 275 -> 257, 32 x 12 186 -> 177), and
-//    past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
+//  * 257 to 512 pairs of 64: 4 in place of 8 (32 x 12 T 8,192 (2,048) 186 -> 177; 64 x 12 275 -> 257, but three
+//    decoders in turns 307 -> 313), and past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
 struct F32Form {
   int nsplit;
   bool wgm;
@@ -602,7 +605,7 @@ struct F32Form {
 F32Form f32_step_form(long long bh, int D, int tiles, int nsplit) {
   const bool wgm = nsplit <= kWgmMaxSplits;
   if (nsplit >= 2 && bh > 512 && tiles <= kMaxPps) return {1, false};
-  if (wgm) return {D <= 64 && bh > 256 && tiles <= 4 * kMaxPps ? std::min(nsplit, 4) : nsplit, true};
+  if (wgm) return {D <= 64 && bh > 256 && bh <= 512 && tiles <= 4 * kMaxPps ? std::min(nsplit, 4) : nsplit, true};
   if (bh > 32 && bh <= 128 && nsplit > 12 && nsplit <= 16) return {nsplit, wgm};
   const int few = D > 64 && bh > 8 && tiles > 600 ? 24 : 16;
   const int n = bh <= 32 ? std::min(nsplit, few) : bh <= 64 ? (nsplit > 16 ? 16 : 12) : 8;
