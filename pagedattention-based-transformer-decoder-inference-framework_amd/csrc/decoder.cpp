@@ -31,11 +31,12 @@
 #include "common.hpp"
 #include "dev_buf.hpp"
 #include "gemm.hpp"
-#include "row_step.hpp"
 #include "kv_cache_impl.hpp"
 #include "model.hpp"
 #include "pa_decode.hpp"
 #include "row_ops.hpp"
+#include "row_step.hpp"
+#include "step_graph.hpp"
 #include "step_put.hpp"
 
 using namespace llm;
@@ -124,9 +125,7 @@ struct llm_decoder {
   int batch = 0;
   std::vector<int> h_pos;  // host mirror of the next position of each row
 
-  hipGraphExec_t graph = nullptr;
-  int graph_batch = -1;
-  bool graph_rows = false;  // by row_step
+  StepGraphs<hipGraphExec_t, 2> graphs;  // by launches, by row_step
 
   // activation taps (llm_decoder_set_taps): the int8 GEMM inputs and row scales
   // of every layer, copied out by the step for teacher-forced parity checks
@@ -140,7 +139,7 @@ struct llm_decoder {
   ~llm_decoder() {
     if (h_oflag) (void)hipHostFree(h_oflag);
     if (h_prompt) (void)hipHostFree(h_prompt);
-    if (graph) (void)hipGraphExecDestroy(graph);
+    graphs.clear([](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); });
     if (kv) kv_cache_destroy(kv);
     if (stream) (void)hipStreamDestroy(stream);
   }
@@ -375,7 +374,7 @@ extern "C" int llm_decoder_set_int8_weights(llm_decoder* d, const llm_int8_weigh
   RET_IF(upload(d->b1, w->b1, (size_t)L * inter, "b1"));
   RET_IF(upload(d->b2, w->b2, (size_t)L * hid, "b2"));
   d->w_keep = w_keep_for(d);
-  d->graph_batch = -1;
+  d->graphs.stale();
   d->weights_ready = true;
   return LLM_OK;
 }
@@ -415,7 +414,7 @@ extern "C" int llm_decoder_set_f16_weights(llm_decoder* d, const llm_f16_weights
   RET_IF(upload(d->b1, w->b1, (size_t)L * inter, "b1"));
   RET_IF(upload(d->b2, w->b2, (size_t)L * hid, "b2"));
   d->w_keep = w_keep_for(d);
-  d->graph_batch = -1;
+  d->graphs.stale();
   d->weights_ready = true;
   return LLM_OK;
 }
@@ -933,23 +932,29 @@ int llm_decoder::run_step(const int32_t* tokens_host, float* logits_dev, int32_t
   if (!use_graph) {
     RET_IF(enqueue_step(st, nullptr, to));
   } else {
-    if (graph_batch != batch || graph_rows != rows_alone()) {
-      if (graph) { (void)hipGraphExecDestroy(graph); graph = nullptr; }
-      hipGraph_t g;
-      LLM_HIP_RET(hipStreamSynchronize(st));
-      LLM_HIP_RET(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
-      int rc = enqueue_step(stream, logits_at.p, nullptr);
-      hipError_t e = hipStreamEndCapture(stream, &g);
-      if (rc) return rc;
-      if (e != hipSuccess)
-        return fail(LLM_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
-      e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
-      (void)hipGraphDestroy(g);
-      if (e != hipSuccess)
-        return fail(LLM_ERR_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
-      graph_batch = batch;
-      graph_rows = rows_alone();
-    }
+    hipGraphExec_t graph = nullptr;
+    RET_IF(graphs.get(
+        rows_alone(), batch,
+        [&]() -> int {
+          LLM_HIP_RET(hipStreamSynchronize(st));
+          return LLM_OK;
+        },
+        [](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); },
+        [&](hipGraphExec_t* made) -> int {
+          hipGraph_t g;
+          LLM_HIP_RET(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
+          const int rc = enqueue_step(stream, logits_at.p, nullptr);
+          hipError_t e = hipStreamEndCapture(stream, &g);
+          if (rc) return rc;
+          if (e != hipSuccess)
+            return fail(LLM_ERR_HIP, std::string("graph capture: ") + hipGetErrorString(e));
+          e = hipGraphInstantiate(made, g, nullptr, nullptr, 0);
+          (void)hipGraphDestroy(g);
+          if (e != hipSuccess)
+            return fail(LLM_ERR_HIP, std::string("graph instantiate: ") + hipGetErrorString(e));
+          return LLM_OK;
+        },
+        &graph));
     LLM_HIP_RET(hipGraphLaunch(graph, st));
   }
   for (int b = 0; b < batch; ++b) h_pos[b] += 1;
@@ -1187,7 +1192,7 @@ static int reset_rows(llm_decoder* d, int batch, int start_pos) {
   LLM_REQUIRE(batch > 0 && batch <= d->maxB, "decoder: batch must be in [1, max_batch]");
   RET_IF(kv_cache_clear(d->kv));
   d->batch = batch;
-  if (d->row_group != 1) d->graph_batch = -1;  // the captured attention launch used the beam group
+  if (d->row_group != 1) d->graphs.stale();  // the captured attention launch used the beam group
   d->row_group = 1;
   d->h_pos.assign(d->maxB, 0);
   for (int b = 0; b < batch; ++b) d->h_pos[b] = start_pos;
@@ -1274,7 +1279,7 @@ extern "C" int llm_decoder_begin_beams(llm_decoder* d, int num_seqs, int beam_wi
                                      d->stream));
   LLM_HIP_RET(hipStreamSynchronize(d->stream));
   d->row_group = beam_width;
-  d->graph_batch = -1;  // re-capture: the attention launch depends on row_group
+  d->graphs.stale();  // re-capture: the attention launch depends on row_group
   return LLM_OK;
 }
 
@@ -1295,7 +1300,7 @@ extern "C" int llm_decoder_set_sampling(llm_decoder* d, float temperature, int t
   d->top_k = top_k;
   d->top_p = top_p;
   d->sample_seed = seed;
-  d->graph_batch = -1;  // the step graph changes
+  d->graphs.stale();  // the step graph changes
   return LLM_OK;
 }
 
@@ -1307,7 +1312,7 @@ extern "C" int llm_decoder_set_taps(llm_decoder* d, int8_t* q_dev, float* s_dev)
   LLM_HIP_RET(hipStreamSynchronize(d->stream));
   d->tap_q = q_dev;
   d->tap_s = s_dev;
-  d->graph_batch = -1;  // the step graph gains / loses the tap copies
+  d->graphs.stale();  // the step graph gains / loses the tap copies
   return LLM_OK;
 }
 
@@ -1415,10 +1420,10 @@ extern "C" int llm_decoder_generate(llm_decoder* d, const int32_t* prompts,
     bool active;
     explicit SamplingGuard(llm_decoder* dd)
         : d(dd), t(dd->temperature), active(dd->temperature > 0.f && dd->top_k != 1) {
-      if (active) { d->temperature = 0.f; d->graph_batch = -1; }
+      if (active) { d->temperature = 0.f; d->graphs.stale(); }
     }
     ~SamplingGuard() {
-      if (active) { d->temperature = t; d->graph_batch = -1; }
+      if (active) { d->temperature = t; d->graphs.stale(); }
     }
   } sampling_guard(d);
   LLM_REQUIRE(batch >= 1 && batch <= d->maxB, "llm_decoder_generate: batch out of range");

@@ -1123,3 +1123,27 @@ def test_rows_of_other_lengths_by_themselves(gpu, oracle):
             together = logits.cpu().numpy()
         else:
             assert (logits[0].cpu().numpy() == together[batch[0]]).all()
+
+
+def test_rows_of_hidden_256_past_the_bound_unwaited(gpu, oracle):
+    """Steps on both sides of 512 tokens enqueued one behind the other, and again in a second sequence:
+    the same as each waited for."""
+    torch = _torch()
+    rows, V, S = 2, 300, 560
+    w = _int8_model(oracle, L=2, V=V, S=S, seed=75)
+    dec = _make_gpu_decoder(w, max_batch=rows)
+    ids = np.random.default_rng(76).integers(0, V, (rows, 520)).tolist()
+    got = []
+    for wait in (True, False, False):
+        dec.begin_synthetic(rows, 0, 0, False)
+        for r in range(rows):
+            dec.prefill(r, ids[r][:500])
+        logits = torch.zeros((20, rows, V), device="cuda")
+        for i in range(20):
+            dec.step([ids[r][500 + i] for r in range(rows)], logits[i].data_ptr(), 0, False)
+            if wait:
+                torch.cuda.synchronize()
+        torch.cuda.synchronize()
+        got.append(logits)
+    assert torch.isfinite(got[0]).all() and got[0].abs().max() > 0
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

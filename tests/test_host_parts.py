@@ -53,6 +53,51 @@ int main() {
     assert out == ["ok"]
 
 
+def test_step_graphs_are_dropped_idle_and_not_half_made(tmp_path):
+    """An executable is waited for before it is dropped, the other way's stays, and one that could not
+    be made (or not be waited for) is not taken for one of a later call."""
+    out = run(tmp_path, """
+#include <cstdio>
+#include "step_graph.hpp"
+using namespace llm;
+struct Graph { int way, rows; bool running; };
+StepGraphs<Graph*, 2> g;
+int made = 0, dropped = 0, early = 0, wait_rc = 0, make_rc = 0;
+Graph* running = nullptr;
+int step(int way, int rows) {
+  Graph* x = nullptr;
+  const int rc = g.get(way, rows,
+      [&] { if (!wait_rc && running) { running->running = false; running = nullptr; } return wait_rc; },
+      [&](Graph* d) { early += d->running; ++dropped; delete d; },
+      [&](Graph** m) { if (make_rc) return make_rc; *m = new Graph{way, rows, false}; ++made; return 0; }, &x);
+  if (rc) return rc;
+  if (!x || x->way != way || x->rows != rows) return 99;
+  if (running) running->running = false;  // launches go one after the other
+  (running = x)->running = true;
+  return 0;
+}
+int main() {
+  if (step(1, 2) || step(1, 2) || step(0, 2) || step(1, 2) || step(0, 2) || made != 2 || dropped) return 1;
+  if (step(0, 3) || step(1, 2) || made != 3 || dropped != 1 || early) return 2;
+  g.stale();
+  if (step(1, 2) || made != 4 || dropped != 2 || early) return 3;
+  make_rc = 7;  // dropped, and not made anew
+  if (step(1, 4) != 7 || dropped != 3 || early) return 4;
+  make_rc = 0;
+  if (step(1, 2) || made != 5 || step(1, 4) || made != 6) return 5;
+  wait_rc = 9;  // nothing happened
+  if (step(1, 2) != 9 || dropped != 4 || made != 6) return 6;
+  wait_rc = 0;
+  if (step(1, 4) || made != 6) return 7;
+  running->running = false;
+  g.clear([&](Graph* d) { ++dropped; delete d; });
+  if (made + 0 != dropped) return 8;
+  std::puts("ok");
+}
+""")
+    assert out == ["ok"]
+
+
 def test_pinned_rows_of_two_sizes_in_turns(tmp_path):
     """Results that do not fit the pool together: no block is pinned or given back at every step, the
     bound holds, and sizes that are no longer asked for make room."""
