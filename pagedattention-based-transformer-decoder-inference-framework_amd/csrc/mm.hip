@@ -128,6 +128,7 @@ hipError_t mm(int dtype, const MmArgs& a, hipStream_t st) {
 }
 
 hipError_t mm_qkv(int dtype, const MmArgs& a, const MmQkv& e, hipStream_t st) {
+  if (a.rows && a.N > (e.H + e.G) * e.D) return hipErrorInvalidValue;  // (value columns go by rows side by side)
   KernelArgs p = plain_args(dtype, a);
   p.q = e;
   return dtype == LLM_F32 ? launch<float, kQkv>(p, st) : launch<__bf16, kQkv>(p, st);

@@ -108,7 +108,7 @@ struct MmArgs {
   int parts = 1;
   size_t c_part = 0;
   // (mm_qkv, mm_latent, mm_split) only these rows of A, of the results and of what belongs to rows take
-  // part (M: their number)
+  // part (M: their number; no value columns among them)
   const int32_t* rows = nullptr;
   float softcap = 0.f;      // C = softcap tanh(C / softcap) when set
 };

@@ -115,6 +115,7 @@ __device__ __forceinline__ void put_pair(T* p, float v0, float v1) {
 // or the tile list.
 template <typename T>
 struct Block {
+  static constexpr bool kSome = false;
   const T* A = nullptr;
   const char* W = nullptr;
   int lda = 0, M = 0, N = 0, KS = 0, m0 = 0;
@@ -122,6 +123,14 @@ struct Block {
   bool shared = false;
   GluParams glu;
 };
+// One of MmArgs::rows.  A kernel of its own: the look-up costs the others registers (bf16 kSplit streams
+// 82 -> 87, 110 -> 120, 130 -> 136, and 5.8 -> 6.2 us for 64 rows x 96 columns of a decode step).
+template <typename T>
+struct SomeBlock : Block<T> {
+  static constexpr bool kSome = true;
+};
+template <typename T, bool SOME>
+using BlockOf = std::conditional_t<SOME, SomeBlock<T>, Block<T>>;
 
 template <typename T, int EPI>
 __device__ __forceinline__ Block<T> block_of(const KernelArgs& p, int row_block, int by) {
@@ -181,8 +190,8 @@ constexpr bool some_rows() {
 }
 
 // Row m of A (the last one for rows past it).
-template <typename T, int EPI>
-__device__ __forceinline__ const char* a_row(const KernelArgs& p, const Block<T>& b, int m) {
+template <typename T, int EPI, typename B>
+__device__ __forceinline__ const char* a_row(const KernelArgs& p, const B& b, int m) {
   m = min(m, b.M - 1);
   if constexpr (EPI == kGroupIn) {
     if (!b.shared) m = p.g.perm[m] / p.g.top;
@@ -190,9 +199,7 @@ __device__ __forceinline__ const char* a_row(const KernelArgs& p, const Block<T>
   if constexpr (EPI == kHeads) {
     if (p.heads.rows) m = p.heads.rows[m];
   }
-  if constexpr (some_rows<EPI>()) {
-    if (p.a.rows) m = p.a.rows[m];
-  }
+  if constexpr (B::kSome) m = p.a.rows[m];
   if constexpr (EPI == kExpand) {
     const MmPageRows& r = p.page_rows;
     const int pos = r.pos[m];
@@ -223,13 +230,11 @@ struct RowOf {
   float weight = 1.f;
 
   __device__ __forceinline__ RowOf() {}
-  template <typename T>
-  __device__ __forceinline__ RowOf(const KernelArgs& p, const Block<T>& b, int row) {
+  template <typename B>
+  __device__ __forceinline__ RowOf(const KernelArgs& p, const B& b, int row) {
     if (row >= b.M) return;
     m = row;
-    if constexpr (some_rows<EPI>()) {
-      if (p.a.rows) m = p.a.rows[row];
-    }
+    if constexpr (B::kSome) m = p.a.rows[row];
     if constexpr (PAGED) {
       const MmQkv& e = p.q;
       pos = e.pos[m];
@@ -725,8 +730,8 @@ constexpr int columns_each(int rows, int cols) {
 // 2011 rows of gate and up with their activation 108, now 105; the products alone 77), and a thread's rows
 // have one set of columns, whose bias, head and place are found once.  All that is loaded
 // is loaded before the first store: a load behind stores is waited for together with them.
-template <typename T, int EPI, int ROWS, int COLS, int STRIDE>
-__device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b, const float* sums,
+template <typename T, int EPI, int ROWS, int COLS, int STRIDE, typename B>
+__device__ __forceinline__ void emit_wave(const KernelArgs& p, const B& b, const float* sums,
                                           const RowOf<EPI>& row, int m0, int n0) {
   constexpr int E = columns_each<EPI>(ROWS, COLS), ACROSS = COLS / E, STEP = 64 / ACROSS, PER = ROWS / STEP;
   static_assert(64 % ACROSS == 0 && PER >= 1);
@@ -888,14 +893,14 @@ __device__ __forceinline__ void emit_wave(const KernelArgs& p, const Block<T>& b
 // and its WK waves split K, adding through LDS in a fixed order.  K is summed in PARTS parts,
 // PARTS / WK of them by a wave one after the other: a wave that streams more of K sums it no
 // further in one piece, and the bits do not depend on how many waves there are.
-template <typename T, int EPI, int MT, int NT, int WK, int PARTS>
+template <typename T, int EPI, int MT, int NT, int WK, int PARTS, bool SOME = false>
 __global__ __launch_bounds__(64 * WK, MT * NT == 1 ? 4 : 2) void mm_stream_kernel(KernelArgs p) {
   if constexpr (EPI == kGroupIn || EPI == kGroupOut)
     if ((int)blockIdx.y >= *p.g.n_tiles) return;
   constexpr int U = MT * NT >= 4 ? 2 : 4;  // k-steps per load batch
   const int lane = lane_id();
   const int w = wave_id_uniform();
-  const Block<T> b = block_of<T, EPI>(p, 16 * MT, blockIdx.y);
+  const BlockOf<T, SOME> b{block_of<T, EPI>(p, 16 * MT, blockIdx.y)};
   const int ntiles = (b.N + 15) >> 4;
   const int nt0 = (int)blockIdx.x * NT;
   if (nt0 >= ntiles) return;  // (groups differ in width)
@@ -1048,7 +1053,7 @@ __device__ __forceinline__ bool tile_of(const KernelArgs& p, TileAt& tile) {
 
 // A block of 16 MB rows x 16 NB columns, WM x WN waves (block_product.hpp).  Two waves a SIMD in
 // the bounds, for the blocks of four waves (gemm_impl.hpp, gemm_block_kernel).
-template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
+template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST, bool SOME = false>
 __global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p) {
   constexpr int MT = MB / WM, NT = NB / WN;
   __shared__ u32x4 lds[ST][2 * (MB + NB)][64];
@@ -1056,14 +1061,15 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p)
   if (!tile_of<EPI, NB>(p, tile)) return;
   const int lane = lane_id();
   const int w = wave_id_uniform();
-  const Block<T> b = block_of<T, EPI>(p, 16 * MB, tile.y);
+  const BlockOf<T, SOME> b{block_of<T, EPI>(p, 16 * MB, tile.y)};
   const int ntiles = (b.N + 15) >> 4;
   const int nt0 = tile.x * NB, KS = b.KS;
   const int wm = w / WN, wn = w % WN;
   const int m0 = 16 * wm * MT, n0 = 16 * wn * NT;
   RowOf<EPI> row(p, b, b.m0 + m0 + lane % (16 * MT));
   if (row.m >= 0) row.look_up(p, b);
-  std::conditional_t<RowOf<EPI>::PAGED, Starts<16 * MB>, NoStarts> starts(p.q, b);
+  constexpr bool VALUES = RowOf<EPI>::PAGED && !SOME;
+  std::conditional_t<VALUES, Starts<16 * MB>, NoStarts> starts(p.q, b);
   f32x4 acc[MT][NT];
   block_product<false, !Kind<T>::BF16, MB, NB, WM, WN, ST>(
       lds, acc, KS, b.m0 + 16 * wm * MT < b.M,
@@ -1076,7 +1082,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void mm_block_kernel(KernelArgs p)
   float* sums = reinterpret_cast<float*>(&lds[0][0][0]);
   spread_sums<STRIDE>(acc, sums, m0, n0);
   emit_wave<T, EPI, 16 * MT, 16 * NT, STRIDE>(p, b, sums + m0 * STRIDE + n0, row, b.m0 + m0, 16 * nt0 + n0);
-  if constexpr (RowOf<EPI>::PAGED) {
+  if constexpr (VALUES) {
     const int first = max(16 * nt0, (p.q.H + p.q.G) * p.q.D), last = min(16 * (nt0 + NB), b.N);
     if (first >= last) return;
     __syncthreads();
@@ -1098,7 +1104,7 @@ constexpr bool by_strips() {
 // epilogue to which they are handed down: a launch finds its code in no cache (2011 x 2048 x 2048
 // amid a model, a copy for each quarter 35 KB: 27.5 us; one, 12 KB: 20.4; blocks of eight waves
 // 25.5).
-template <typename T, int EPI, int MB, int NT, int WAVES, int ST, int AHEAD>
+template <typename T, int EPI, int MB, int NT, int WAVES, int ST, int AHEAD, bool SOME = false>
 __global__ __launch_bounds__(64 * WAVES, 2) void mm_strip_kernel(KernelArgs p) {
   constexpr int NB = NT * WAVES, SR = MB / 4, STRIDE = 16 * NT + 4;
   __shared__ u32x4 lds[ST][2 * MB][64];
@@ -1106,7 +1112,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void mm_strip_kernel(KernelArgs p) {
   TileAt tile;
   if (!tile_of<EPI, NB>(p, tile)) return;
   const int w = wave_id_uniform();
-  const Block<T> b = block_of<T, EPI>(p, 16 * MB, tile.y);
+  const BlockOf<T, SOME> b{block_of<T, EPI>(p, 16 * MB, tile.y)};
   const int ntiles = (b.N + 15) >> 4, nt0 = tile.x * NB + w * NT, KS = b.KS;
   f32x4 acc[MB][NT];
   strip_product<MB, NT, WAVES, ST, AHEAD>(
@@ -1134,8 +1140,13 @@ int heads_of(const KernelArgs& p) {  // and parts of K
 template <typename T, int EPI, int MT, int NT, int WK = 8, int PARTS = WK>
 hipError_t stream(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
   const dim3 grid(((N + 15) / 16 + NT - 1) / NT, row_blocks, heads_of<EPI>(p));
-  hipLaunchKernelGGL((mm_stream_kernel<T, EPI, MT, NT, WK, PARTS>), grid, dim3(64 * WK), 0, st, p);
-  return hipGetLastError();
+  const auto go = [&](void (*kernel)(KernelArgs)) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * WK), 0, st, p);
+    return hipGetLastError();
+  };
+  if constexpr (some_rows<EPI>())
+    if (p.a.rows) return go(mm_stream_kernel<T, EPI, MT, NT, WK, PARTS, true>);
+  return go(mm_stream_kernel<T, EPI, MT, NT, WK, PARTS>);
 }
 
 template <int EPI>
@@ -1148,16 +1159,24 @@ dim3 block_grid(const KernelArgs& p, int row_blocks, int N, int NB) {
 
 template <typename T, int EPI, int MB, int NB, int WM, int WN, int ST>
 hipError_t blocks(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
-  hipLaunchKernelGGL((mm_block_kernel<T, EPI, MB, NB, WM, WN, ST>), block_grid<EPI>(p, row_blocks, N, NB),
-                     dim3(64 * WM * WN), 0, st, p);
-  return hipGetLastError();
+  const auto go = [&](void (*kernel)(KernelArgs)) {
+    hipLaunchKernelGGL(kernel, block_grid<EPI>(p, row_blocks, N, NB), dim3(64 * WM * WN), 0, st, p);
+    return hipGetLastError();
+  };
+  if constexpr (some_rows<EPI>())
+    if (p.a.rows) return go(mm_block_kernel<T, EPI, MB, NB, WM, WN, ST, true>);
+  return go(mm_block_kernel<T, EPI, MB, NB, WM, WN, ST>);
 }
 
 template <typename T, int EPI, int MB, int NT, int WAVES, int ST, int AHEAD>
 hipError_t strips(const KernelArgs& p, int row_blocks, int N, hipStream_t st) {
-  hipLaunchKernelGGL((mm_strip_kernel<T, EPI, MB, NT, WAVES, ST, AHEAD>), block_grid<EPI>(p, row_blocks, N, NT * WAVES),
-                     dim3(64 * WAVES), 0, st, p);
-  return hipGetLastError();
+  const auto go = [&](void (*kernel)(KernelArgs)) {
+    hipLaunchKernelGGL(kernel, block_grid<EPI>(p, row_blocks, N, NT * WAVES), dim3(64 * WAVES), 0, st, p);
+    return hipGetLastError();
+  };
+  if constexpr (some_rows<EPI>())
+    if (p.a.rows) return go(mm_strip_kernel<T, EPI, MB, NT, WAVES, ST, AHEAD, true>);
+  return go(mm_strip_kernel<T, EPI, MB, NT, WAVES, ST, AHEAD>);
 }
 
 // How a product runs, and about how long at K = 2048 (us; 0: not told), kFixedUs of it whatever K is.
