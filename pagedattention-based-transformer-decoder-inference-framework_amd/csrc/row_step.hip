@@ -63,6 +63,7 @@ struct Weights {
 
   // column (wave T + t) 16 + (lane & 15) of a row of int8 in LDS with scale sa
   __device__ __forceinline__ void times(const uint8_t* a, float sa, float (&y)[T]) const {
+#pragma clang fp contract(off)  // scaled, then the bias added: rounded twice, as the launches do
     int s[T] = {};
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
@@ -74,8 +75,8 @@ struct Weights {
     }
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      y[t] = __fmul_rn((float)rows_sum(s[t]), __fmul_rn(sa, scale[t]));
-      if constexpr (BIAS) y[t] = __fadd_rn(y[t], bias[t]);
+      y[t] = (float)rows_sum(s[t]) * (sa * scale[t]);
+      if constexpr (BIAS) y[t] = y[t] + bias[t];
     }
   }
 };
@@ -284,11 +285,12 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
         sum += f * part_ml[head * PER + p][1];
         o += f * *reinterpret_cast<const f32x4*>(&part_o[head * PER + p][d]);
       }
+      const float inv = 1.0f / (sum + 1e-6f);
       float most = 0.f;
       LnRow<1> v;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v.v[0][e] = sum > 0.f ? o[e] / sum : 0.f;
+        v.v[0][e] = o[e] * inv;
         most = fmaxf(most, fabsf(v.v[0][e]));
       }
       const float sa = quantise(v, ln_wave_max(most), ints);

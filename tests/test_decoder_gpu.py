@@ -1073,8 +1073,10 @@ def test_synthetic_context_bits(gpu, oracle, max_batch, max_seq):
 def test_rows_of_hidden_256_by_themselves(gpu, oracle, H, D, page, rows):
     """Up to 8 rows of up to 512 tokens go through all layers in one workgroup each: against the
     launches of 9 rows (the same ones and copies of the first), at contexts around pages, the lanes' and waves'
-    shares and the bound, where the next step goes by launches again.  Of the steps, whose activations on the
-    edge of two int8 values may take the other, more than half agree to fp32 sums' order."""
+    shares and the bound, where the next step goes by launches again.  An activation on the edge of two int8 values
+    may take the other: 2e-7 of the row's largest, as two orders of attention's sums differ, is 2.5e-5 of a value,
+    so with 3,584 values a step about one step in six; each context begins anew, so that it does
+    not come along to the next, and more than half agree to fp32 sums' order."""
     import llm_decoder
     torch = _torch()
     V, S = 300, 600
@@ -1085,18 +1087,17 @@ def test_rows_of_hidden_256_by_themselves(gpu, oracle, H, D, page, rows):
         c = w["cfg"]
         dec = llm_decoder.INT8Decoder(c["L"], H, D, c["hid"], V, S, max_batch=n_rows, page_size=page)
         dec.set_weights(_weights_dict(w))
-        dec.begin_synthetic(n_rows, 0, 0, False)
         logits = torch.empty((n_rows, V), device="cuda")
-        mine, at = [], 0
+        mine = []
+        own = [r if r < rows else 0 for r in range(n_rows)]
         for n in (0, 1, 15, 16, 31, 32, 33, 63, 64, 127, 128, 129, 257, 400, 510, 511, 512, 513):
-            own = [r if r < rows else 0 for r in range(n_rows)]
-            if n > at:
+            dec.begin_synthetic(n_rows, 0, 0, False)
+            if n:
                 for r in range(n_rows):
-                    dec.prefill(r, prompts[own[r]][at:n].tolist())
+                    dec.prefill(r, prompts[own[r]][:n].tolist())
             dec.step([int(prompts[own[r]][n]) for r in range(n_rows)], logits_ptr=logits.data_ptr())
             torch.cuda.synchronize()
             mine.append(logits[:rows].cpu().numpy())
-            at = n + 1
         got.append(np.stack(mine))
     assert np.isfinite(got[0]).all()
     err = np.abs(got[0] - got[1]).max(axis=-1) / np.abs(got[1]).max(axis=-1)
@@ -1147,3 +1148,22 @@ def test_rows_of_hidden_256_past_the_bound_unwaited(gpu, oracle):
         got.append(logits)
     assert torch.isfinite(got[0]).all() and got[0].abs().max() > 0
     assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("H,D", [(4, 64), (2, 128), (8, 32)])
+def test_first_tokens_of_hidden_256_bits(gpu, oracle, H, D):
+    """A row's first token, whose attention has one term and so no order of sums: the bits of the
+    launches, its weight 1 / (1 + 1e-6) among them."""
+    torch = _torch()
+    V = 500
+    w = _int8_model(oracle, L=3, H=H, D=D, V=V, S=32, seed=77)
+    got = []
+    for rows in (8, 12):  # by row_step, by launches
+        dec = _make_gpu_decoder(w, max_batch=rows)
+        logits = torch.empty((20, rows, V), device="cuda")
+        for i in range(20):
+            dec.begin_synthetic(rows, 0, 0, False)
+            dec.step([(37 * i + 11 * r) % V for r in range(rows)], logits_ptr=logits[i].data_ptr())
+        torch.cuda.synchronize()
+        got.append(logits[:, :8].clone())
+    assert torch.equal(*got), (got[0] - got[1]).abs().max()
