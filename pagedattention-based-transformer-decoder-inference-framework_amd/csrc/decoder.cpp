@@ -836,7 +836,7 @@ int llm_decoder::step_tail(hipStream_t st, int r0, int n, float* const* place, f
 
 // Whether the step's rows each go through all layers in a workgroup of their own (row_step.hip).
 bool llm_decoder::rows_alone() const {
-  if (wdtype != LLM_I8 || row_group != 1 || tap_q) return false;
+  if (wdtype != LLM_I8 || row_group != 1) return false;
   return row_step_ok(hid, inter, D, TS, batch, 1 + *std::max_element(h_pos.begin(), h_pos.begin() + batch));
 }
 
@@ -863,6 +863,10 @@ int llm_decoder::run_rows(hipStream_t st) {
   a.page_stride = (size_t)view.page_stride / sizeof(_Float16);
   a.attn_scale = cfg.attn_scale;
   a.x = x.p;
+  a.tap_q = tap_q;
+  a.tap_s = tap_s;
+  a.tap_stride = b16 * qa_ld;
+  a.tap_rows = maxB;
   LLM_HIP_RET(row_step(a, st));
   return LLM_OK;
 }

@@ -88,7 +88,9 @@ __device__ __forceinline__ float quantise(const LnRow<1>& v, float largest, uint
   return 1.0f / scale;
 }
 
-template <int D>
+// TAP: the rows of int8 go to the taps too.  The same code; behind a branch it costs every step scalar registers
+// (24.5 -> 25.7 us for 2 layers).
+template <int D, bool TAP>
 __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
   constexpr int H = HID / D, PER = kWaves / H;      // waves of a head
   constexpr int ACROSS = D / 8, TOKENS = 64 / ACROSS;  // lanes of a token, tokens of a load
@@ -114,7 +116,15 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
   const auto put_gain = [&](float g) {
     if (w < 2 * HID / 64) gains[w * 64 + lane] = g;
   };
-  const auto normalise = [&]() {  // x -> ints, by wave 0
+  // A row of int8 (of HID, by wave 0) and its scale to the taps.
+  const auto tap = [&](int layer, int stage, float sa) {
+    if constexpr (!TAP) return;
+    const size_t slot = (size_t)layer * 4 + stage;
+    *reinterpret_cast<uint32_t*>(a.tap_q + slot * a.tap_stride + a_frag_off_i8(m, 4 * lane_id(), HID / 64)) =
+        *reinterpret_cast<const uint32_t*>(ints + 4 * lane_id());
+    if (lane_id() == 0) a.tap_s[slot * a.tap_rows + m] = sa;
+  };
+  const auto normalise = [&](int layer, int stage) {  // x -> ints, by wave 0
     if (w != 0) return;
     LnRow<1> v, gain, shift;
     v.v[0] = *reinterpret_cast<const f32x4*>(&x[4 * lane_id()]);
@@ -122,6 +132,7 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
     shift.v[0] = *reinterpret_cast<const f32x4*>(&gains[HID + 4 * lane_id()]);
     const float sa = quantise(v, ln_wave_compute(v, gain, shift, HID, a.eps), ints);
     if (lane_id() == 0) ints_scale = sa;
+    tap(layer, stage, sa);
   };
   put_gain(gain_of(a.ln1_g, a.ln1_b, 0));
   if (w == kWaves - 1) {
@@ -139,7 +150,7 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
     const int page_id = at < held ? table[(size_t)(w / PER) * a.max_tiles + at] : -1;
     wqkv.load(a.qkv, l, w, lane);
     pages[w * 64 + lane] = page_id < a.num_pages ? page_id : -1;
-    normalise();
+    normalise(l, 0);
     lds_barrier();
 
     {  // q | k | v
@@ -295,6 +306,7 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
       }
       const float sa = quantise(v, ln_wave_max(most), ints);
       if (lane == 0) ints_scale = sa;
+      tap(l, 1, sa);
     }
     lds_barrier();
 
@@ -305,7 +317,7 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
     }
     lds_barrier();
 
-    normalise();
+    normalise(l, 2);
     const float next_gain = gain_of(a.ln1_g, a.ln1_b, min(l + 1, a.L - 1));
     lds_barrier();
 
@@ -327,7 +339,13 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
     lds_barrier();
     put_gain(next_gain);
     const float scale = 127.f / (ln_wave_max(largest[lane & 15]) + 1e-6f);
-    ints[w * 64 + lane] = (uint8_t)ln_quant4(f32x4{h, 0.f, 0.f, 0.f}, scale);
+    const uint8_t mine = (uint8_t)ln_quant4(f32x4{h, 0.f, 0.f, 0.f}, scale);
+    ints[w * 64 + lane] = mine;
+    if constexpr (TAP) {
+      const size_t slot = (size_t)l * 4 + 3;
+      a.tap_q[slot * a.tap_stride + a_frag_off_i8(m, w * 64 + lane, INTER / 64)] = (int8_t)mine;
+      if (w == 0 && lane == 0) a.tap_s[slot * a.tap_rows + m] = 1.0f / scale;
+    }
     lds_barrier();
 
     {  // fc2
@@ -360,9 +378,9 @@ hipError_t row_step(const RowStep& a, hipStream_t st) {
     return hipGetLastError();
   };
   switch (a.D) {
-    case 32: return go(row_step_kernel<32>);
-    case 64: return go(row_step_kernel<64>);
-    case 128: return go(row_step_kernel<128>);
+    case 32: return go(a.tap_q ? row_step_kernel<32, true> : row_step_kernel<32, false>);
+    case 64: return go(a.tap_q ? row_step_kernel<64, true> : row_step_kernel<64, false>);
+    case 128: return go(a.tap_q ? row_step_kernel<128, true> : row_step_kernel<128, false>);
     default: return hipErrorInvalidValue;
   }
 }

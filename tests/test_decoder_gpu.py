@@ -1073,33 +1073,47 @@ def test_synthetic_context_bits(gpu, oracle, max_batch, max_seq):
 def test_rows_of_hidden_256_by_themselves(gpu, oracle, H, D, page, rows):
     """Up to 8 rows of up to 512 tokens go through all layers in one workgroup each: against the
     launches of 9 rows (the same ones and copies of the first), at contexts around pages, the lanes' and waves'
-    shares and the bound, where the next step goes by launches again.  An activation on the edge of two int8 values
-    may take the other: 2e-7 of the row's largest, as two orders of attention's sums differ, is 2.5e-5 of a value,
-    so with 3,584 values a step about one step in six; each context begins anew, so that it does
-    not come along to the next, and more than half agree to fp32 sums' order."""
+    shares and the bound, where the next step goes by launches again; with taps and without, to the same bits.
+    The first layer's attention, whose inputs are the same bits, is held to one int8 value and fp32's scale.  Behind it an
+    activation on the edge of two int8 values may take the other: 2e-7 of the row's largest, as two orders of
+    sums differ, is 2.5e-5 of a value, so with 3,584 values a step about one step in six; each context
+    begins anew, so that it does not come along to the next, and more than half agree to fp32 sums' order."""
     import llm_decoder
     torch = _torch()
     V, S = 300, 600
     w = _int8_model(oracle, L=2, H=H, D=D, V=V, S=S, seed=71)
     prompts = np.random.default_rng(72).integers(0, V, (rows, S))
-    got = []
+    got, rows_of = [], []
     for n_rows in (rows, 9):
         c = w["cfg"]
         dec = llm_decoder.INT8Decoder(c["L"], H, D, c["hid"], V, S, max_batch=n_rows, page_size=page)
         dec.set_weights(_weights_dict(w))
-        logits = torch.empty((n_rows, V), device="cuda")
-        mine = []
+        logits = torch.empty((2, n_rows, V), device="cuda")
+        mine, tapped = [], []
         own = [r if r < rows else 0 for r in range(n_rows)]
         for n in (0, 1, 15, 16, 31, 32, 33, 63, 64, 127, 128, 129, 257, 400, 510, 511, 512, 513):
-            dec.begin_synthetic(n_rows, 0, 0, False)
-            if n:
-                for r in range(n_rows):
-                    dec.prefill(r, prompts[own[r]][:n].tolist())
-            dec.step([int(prompts[own[r]][n]) for r in range(n_rows)], logits_ptr=logits.data_ptr())
+            for i in range(2):
+                if i:
+                    taps = _Taps(dec, w, n_rows)
+                dec.begin_synthetic(n_rows, 0, 0, False)
+                if n:
+                    for r in range(n_rows):
+                        dec.prefill(r, prompts[own[r]][:n].tolist())
+                dec.step([int(prompts[own[r]][n]) for r in range(n_rows)], logits_ptr=logits[i].data_ptr())
             torch.cuda.synchronize()
-            mine.append(logits[:rows].cpu().numpy())
+            tapped.append(taps.read(rows))
+            dec.set_taps(0, 0)
+            assert torch.equal(logits[0], logits[1]), n
+            mine.append(logits[0, :rows].cpu().numpy())
         got.append(np.stack(mine))
+        rows_of.append([np.stack(t) for t in zip(*tapped)])
     assert np.isfinite(got[0]).all()
+    (q0, s0), (q1, s1) = rows_of  # [contexts][L][4][rows]
+    np.testing.assert_array_equal(q0[:, 0, 0], q1[:, 0, 0])
+    np.testing.assert_array_equal(s0[:, 0, 0].view(np.uint32), s1[:, 0, 0].view(np.uint32))
+    differ = np.abs(q0[:, 0, 1].astype(int) - q1[:, 0, 1])
+    assert differ.max() <= 1 and (differ != 0).mean() < 1e-3
+    np.testing.assert_allclose(s0[:, 0, 1], s1[:, 0, 1], rtol=2e-6)
     err = np.abs(got[0] - got[1]).max(axis=-1) / np.abs(got[1]).max(axis=-1)
     assert err.max() < FREE_RUN_TOL, err.max()
     assert np.median(err) < 1e-5, err
