@@ -139,7 +139,8 @@ def attention_launch_bytes(cfg, T, B, unique=False):
 
 def time_attention(dec, layers, iters=24):
     """Live HIP-event timing of the decoder's own paged-attention launch
-    (llm_decoder_run_attention: the step graph's kernels, grid and outputs --
+    (llm_decoder_run_attention: the step graph's kernels, grid and outputs,
+    unless the step is row_step's (step_by_rows) --
     split + merge-and-quantise for INT8, the workgroup-merge form for FP16,
     the beam-group schedule for beams), enqueued on torch's current stream so
     the events bracket exactly those kernels.  The launches rotate over the
@@ -611,8 +612,10 @@ def main():
                 "kernel": f"pa_split_kernel<D={cfg['D']},TS={cfg['ts']}>"
                           + (" beam-group" if form & 16 else "") + ": " + FORM_NAMES[form & 15]
                           + (OPROJ_OUT if form & 32 else FORM_OUT.get(cfg["cls"], {}).get(form & 15, ""))
-                          + f", {nsplit} splits, {B} rows (the step's own launch, "
-                            "llm_decoder_run_attention)",
+                          + f", {nsplit} splits, {B} rows ("
+                          + ("not of this step, which takes its rows through all layers in one "
+                             "launch, row_step_kernel: that of longer rows, " if dec.step_by_rows()
+                             else "the step's own launch, ") + "llm_decoder_run_attention)",
                 "bytes_per_launch": attn_b, "launch_us": round(t_attn * 1e6, 2),
                 "launch_timing": f"HIP events over 24 launches rotating over the {cfg['L']} layers"}
         if "beams" in cfg:  # logical bytes: every beam reads its whole context

@@ -504,16 +504,21 @@ int llm_decoder_set_taps(llm_decoder* d, int8_t* q_dev, float* s_dev);
  * LLM_PA_FORM_SPLIT_MERGE_ROW | LLM_PA_FORM_BEAM.  FP16
  * decoders (head_dim <= 128, <= 64 heads) whose launch merges in the workgroup
  * run o_proj inside it: LLM_PA_FORM_WG_MERGE | LLM_PA_FORM_OPROJ; LLM_PA_FORM_DIRECT
- * and LLM_PA_FORM_SPLIT_MERGE_ROW write its packed fp16 input.  (A step of up to 8 rows of an INT8
- * decoder of hidden 256 has no such launch while they are short: csrc/row_step.hip.) */
+ * and LLM_PA_FORM_SPLIT_MERGE_ROW write its packed fp16 input.  Where llm_decoder_step_by_rows is 1 it
+ * is the launch of the steps that the rows take once they are longer. */
 int llm_decoder_attention_plan(llm_decoder* d, int* nsplit, int* form);
+/* 1 if the next step, at its rows' present lengths, takes them through all layers in one launch, a
+ * workgroup a row, and has no attention launch of its own (INT8 decoders of hidden 256, up to 8 rows of up
+ * to 512 tokens: csrc/row_step.hip), else 0. */
+int llm_decoder_step_by_rows(llm_decoder* d);
 /* Enqueue layer `layer`'s attention launch of the decoder's step on `stream`
  * (NULL: the decoder's) -- the same kernels, grid and outputs as inside the
  * step graph (q from the last step's projection, each row's live context, the
  * o_proj input written), for timing the step's own launch in isolation.  The
  * fused o_proj of an FP16 decoder accumulates into a scratch set of columns of
  * its own here (not the step's), so a run may overlap an in-flight step; two
- * runs of one decoder must not overlap each other. */
+ * runs of one decoder must not overlap each other.  Where llm_decoder_step_by_rows is 1 it is the
+ * launch of longer rows, on the same queries and contexts. */
 int llm_decoder_run_attention(llm_decoder* d, int layer, void* stream);
 int llm_decoder_context_len(const llm_decoder* d, int row);
 kv_cache* llm_decoder_kv(llm_decoder* d);

@@ -365,6 +365,7 @@ class Decoder {
     py::gil_scoped_release nogil;
     check(llm_decoder_run_attention(d_, layer, reinterpret_cast<void*>(stream)));
   }
+  bool step_by_rows() const { return llm_decoder_step_by_rows(d_) != 0; }
   // llm_decoder_oproj_status: (range guard tripped, accumulator columns not at zero)
   py::tuple oproj_status() {
     int clamped = 0;
@@ -594,6 +595,7 @@ PYBIND11_MODULE(llm_decoder, m) {
         .def("oproj_status", &Decoder::oproj_status)
         .def("run_attention", &Decoder::run_attention, py::arg("layer") = 0,
              py::arg("stream") = 0)
+        .def("step_by_rows", &Decoder::step_by_rows)
         .def_property_readonly("kv_handle", &Decoder::kv_handle);
   };
   py::class_<Decoder>(m, "_Decoder");

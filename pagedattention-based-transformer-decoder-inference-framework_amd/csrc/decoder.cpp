@@ -863,6 +863,7 @@ int llm_decoder::run_rows(hipStream_t st) {
   a.page_stride = (size_t)view.page_stride / sizeof(_Float16);
   a.attn_scale = cfg.attn_scale;
   a.x = x.p;
+  a.q = qkv.p;
   a.tap_q = tap_q;
   a.tap_s = tap_s;
   a.tap_stride = b16 * qa_ld;
@@ -1211,6 +1212,16 @@ static int reset_rows(llm_decoder* d, int batch, int start_pos) {
 }
 
 #if LLM_TUNING
+// The step's queries and attention's fp32 rows (tests).
+extern "C" int llm_decoder_tune_attention_rows(llm_decoder* d, float* q, float* o) {
+  std::lock_guard<std::mutex> g(d->mu);
+  const size_t bytes = sizeof(float) * d->batch * d->hid;
+  LLM_HIP_RET(hipDeviceSynchronize());
+  LLM_HIP_RET(hipMemcpy(q, d->qkv.p, bytes, hipMemcpyDeviceToHost));
+  LLM_HIP_RET(hipMemcpy(o, d->o.p, bytes, hipMemcpyDeviceToHost));
+  return LLM_OK;
+}
+
 // The head's words as a launch that was cut short would leave them (tests).
 extern "C" int llm_decoder_tune_head_words(llm_decoder* d, uint32_t arrived, uint64_t key) {
   std::lock_guard<std::mutex> g(d->mu);
@@ -1332,6 +1343,12 @@ extern "C" int llm_decoder_attention_plan(llm_decoder* d, int* nsplit, int* form
   *nsplit = p.nsplit;
   *form = p.form;
   return LLM_OK;
+}
+
+extern "C" int llm_decoder_step_by_rows(llm_decoder* d) {
+  if (!d) return 0;
+  std::lock_guard<std::mutex> g(d->mu);
+  return d->batch > 0 && d->rows_alone();
 }
 
 extern "C" int llm_decoder_run_attention(llm_decoder* d, int layer, void* stream) {

@@ -356,6 +356,7 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
     lds_barrier();
   }
   if (w == 0) *reinterpret_cast<f32x4*>(a.x + (size_t)m * HID + 4 * lane) = *reinterpret_cast<const f32x4*>(&x[4 * lane]);
+  if (w == 1) *reinterpret_cast<f32x4*>(a.q + (size_t)m * HID + 4 * lane) = *reinterpret_cast<const f32x4*>(&q[4 * lane]);
 }
 
 }  // namespace

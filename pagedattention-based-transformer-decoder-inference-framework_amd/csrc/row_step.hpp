@@ -36,6 +36,7 @@ struct RowStep {
   size_t page_stride = 0;  // elements
   float attn_scale = 1.f;
   float* x = nullptr;  // [rows][hidden] after the last layer
+  float* q = nullptr;  // [rows][hidden] the last layer's queries (llm_decoder_run_attention)
   // Taps (llm_decoder_set_taps; NULL: none): slot 4 layer + stage has int8 rows in packed-A order from
   // tap_q + slot tap_stride and their scales from tap_s + slot tap_rows.
   int8_t* tap_q = nullptr;

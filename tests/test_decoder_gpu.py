@@ -29,6 +29,9 @@ token) plus a margin.  That drift is the INT8 decoder's own: the oracle
 against itself with only its summation order reversed drifts 2.3e-2 at C1
 dims (tests/test_generate_free_run.py); test_generate_free_run_gpu.py holds
 free-running generate to that yardstick."""
+import contextlib
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -54,6 +57,38 @@ def _weights_dict(w):
     d = {k: np.ascontiguousarray(v) for k, v in w.items() if k != "cfg"}
     d["emb"] = w["emb"].view(np.uint16)
     return d
+
+
+@contextlib.contextmanager
+def _tune_int8(lib, w, max_batch):
+    """An INT8 decoder of a library loaded by ctypes (the tuning build's hooks)."""
+    import llm_capi
+    from test_wg_merge_gpu import _Cfg
+    c, vp = w["cfg"], ctypes.c_void_p
+    names = ("emb", "ln1_g", "ln1_b", "ln2_g", "ln2_b", "wqkv", "sw_qkv", "wo", "sw_o", "w1", "sw1", "b1",
+             "w2", "sw2", "b2")
+    d = {k: np.ascontiguousarray(w[k]) for k in names}
+
+    class Weights(ctypes.Structure):
+        _fields_ = [(n, vp) for n in names]
+
+    lib.llm_decoder_create.argtypes = [ctypes.POINTER(_Cfg), ctypes.POINTER(vp)]
+    lib.llm_decoder_set_int8_weights.argtypes = [vp, ctypes.POINTER(Weights)]
+    lib.llm_decoder_begin_synthetic.argtypes = [vp, ctypes.c_int, ctypes.c_int, ctypes.c_uint64, ctypes.c_int]
+    lib.llm_decoder_step.argtypes = [vp] * 5
+    lib.llm_decoder_run_attention.argtypes = [vp, ctypes.c_int, vp]
+    lib.llm_decoder_tune_attention_rows.argtypes = [vp] * 3
+    lib.llm_decoder_step_by_rows.argtypes = [vp]
+    lib.llm_decoder_destroy.argtypes = [vp]
+    lib.llm_decoder_destroy.restype = None
+    cfg = _Cfg(c["L"], c["H"], c["D"], c["hid"], c["V"], c["max_seq"], 0, 16, llm_capi.LLM_I8, max_batch, 1.0, 0)
+    dec = vp()
+    llm_capi.check(lib.llm_decoder_create(ctypes.byref(cfg), ctypes.byref(dec)), lib)
+    try:
+        llm_capi.check(lib.llm_decoder_set_int8_weights(dec, ctypes.byref(Weights(*[d[k].ctypes.data for k in names]))), lib)
+        yield dec
+    finally:
+        lib.llm_decoder_destroy(dec)
 
 
 def _make_gpu_decoder(w, max_batch, cls="INT8Decoder"):
@@ -1181,3 +1216,31 @@ def test_first_tokens_of_hidden_256_bits(gpu, oracle, H, D):
         torch.cuda.synchronize()
         got.append(logits[:, :8].clone())
     assert torch.equal(*got), (got[0] - got[1]).abs().max()
+
+
+@pytest.mark.parametrize("H,D", [(4, 64), (2, 128)])
+def test_run_attention_behind_row_step(gpu, oracle, H, D):
+    """llm_decoder_run_attention after a step that has no attention launch works on the queries of that
+    step's last layer, as after a step of 9 rows by launches (tuning build, which reads the buffers; of its
+    context, the token that the next step writes is not there yet).  The last layer's inputs may have taken
+    another int8 value on the way: FREE_RUN_TOL."""
+    import llm_capi
+    lib = llm_capi.load_tune()
+    w = _int8_model(oracle, L=2, H=H, D=D, V=300, S=64, seed=78)
+    hid, V = H * D, 300
+    got = []
+    for rows in (4, 9):
+        with _tune_int8(lib, w, rows) as dec:
+            llm_capi.check(lib.llm_decoder_begin_synthetic(dec, rows, 0, 0, 0), lib)
+            assert lib.llm_decoder_step_by_rows(dec) == (rows == 4)
+            for s in range(21):
+                tok = np.array([(13 * s + 29 * (r % 4)) % V for r in range(rows)], np.int32)
+                llm_capi.check(lib.llm_decoder_step(dec, tok.ctypes.data, None, None, None), lib)
+            llm_capi.check(lib.llm_decoder_run_attention(dec, 1, None), lib)
+            q, o = np.zeros((2, rows, hid), np.float32)
+            llm_capi.check(lib.llm_decoder_tune_attention_rows(dec, q.ctypes.data, o.ctypes.data), lib)
+            assert np.isfinite(o).all() and (np.abs(o).max(axis=1) > 0).all()
+            got.append(q[:4])
+    assert np.isfinite(got[0]).all() and (np.abs(got[1]).max(axis=1) > 0).all()
+    err = np.abs(got[0] - got[1]).max(axis=1) / np.abs(got[1]).max(axis=1)
+    assert err.max() < FREE_RUN_TOL, err
