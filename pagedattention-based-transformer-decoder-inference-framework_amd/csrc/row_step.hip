@@ -171,7 +171,8 @@ __global__ __launch_bounds__(64 * kWaves) void row_step_kernel(RowStep a) {
     const float gain = gain_of(a.ln2_g, a.ln2_b, l);
     lds_barrier();
 
-    // (a look-up past LDS would be waited for together with the weights on their way)
+    // (a look-up past LDS would be waited for together with the weights on their way.  Rows that row_step_ok admits are
+    // never so long, but the device's position can be past the host's count: replays of a captured step)
     const auto page_of = [&](int head, int t, bool in_lds) {
       const int i = t >> a.page_shift;
       if (in_lds) return pages[head * (64 * PER) + i];

@@ -1244,3 +1244,66 @@ def test_run_attention_behind_row_step(gpu, oracle, H, D):
     assert np.isfinite(got[0]).all() and (np.abs(got[1]).max(axis=1) > 0).all()
     err = np.abs(got[0] - got[1]).max(axis=1) / np.abs(got[1]).max(axis=1)
     assert err.max() < FREE_RUN_TOL, err
+
+
+def _graph_nodes(step):
+    """Kernels, copies and fills of what step(stream) captures on a stream of its own."""
+    torch = _torch()
+    hip = ctypes.CDLL("libamdhip64.so")
+    stream, graph, n = torch.cuda.Stream(), ctypes.c_void_p(), ctypes.c_size_t()
+    st = ctypes.c_void_p(stream.cuda_stream)
+    assert hip.hipStreamBeginCapture(st, 2) == 0  # relaxed
+    try:
+        step(stream.cuda_stream)
+    finally:
+        assert hip.hipStreamEndCapture(st, ctypes.byref(graph)) == 0
+    assert hip.hipGraphGetNodes(graph, None, ctypes.byref(n)) == 0
+    assert hip.hipGraphDestroy(graph) == 0
+    return n.value
+
+
+@pytest.mark.parametrize("H,D", [(4, 64), (8, 32)])
+def test_captured_steps_of_hidden_256_go_by_launches(gpu, oracle, monkeypatch, H, D):
+    """A step that a program captures (LLM_GRAPH=0) has the layers' launches however short its rows are
+    then, and replays far past 512 tokens; a plain step behind them, whose row the host still takes for
+    short, finds pages past those that row_step holds in LDS (1,024 / H of a head).  Against steps whose
+    prompt was taken in whole: FREE_RUN_TOL."""
+    import llm_capi
+    torch = _torch()
+    monkeypatch.setenv("LLM_GRAPH", "0")
+    V, times, tok = 300, 105 if H == 4 else 55, 7
+    toks = np.random.default_rng(80).integers(0, V, 40).tolist()
+    n, S = 40 * times, 40 * times + 100
+    w = _int8_model(oracle, L=2, H=H, D=D, V=V, S=S, seed=79)
+    dec = _make_gpu_decoder(w, max_batch=1)
+    dec.begin_synthetic(1, 0, 0, False)
+    lib = llm_capi.load()
+    kv = ctypes.c_void_p(dec.kv_handle)
+    llm_capi.check(lib.kv_cache_reserve(kv, 0, S))
+    llm_capi.check(lib.kv_cache_sync(kv, None))
+    torch.cuda.synchronize()
+    assert dec.step_by_rows()
+    dec.step([tok])
+    assert _graph_nodes(lambda st: dec.step([tok], 0, st, False)) > 2 * 3  # (row_step: 3 in all)
+    dec.begin_synthetic(1, 0, 0, False)
+    llm_capi.check(lib.kv_cache_reserve(kv, 0, S))
+    llm_capi.check(lib.kv_cache_sync(kv, None))
+    torch.cuda.synchronize()
+    graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=stream):
+        for t in toks:
+            dec.step([t], 0, stream.cuda_stream, False)
+    logits = torch.empty((2, 1, V), device="cuda")
+    for i in range(times):
+        graph.replay()
+    torch.cuda.synchronize()
+    assert dec.context_len(0) == 40 and dec.step_by_rows()
+    dec.step([tok], logits_ptr=logits[0].data_ptr())
+    torch.cuda.synchronize()
+    dec.begin_synthetic(1, 0, 0, False)
+    dec.prefill(0, toks * times)
+    assert not dec.step_by_rows()
+    dec.step([tok], logits_ptr=logits[1].data_ptr())
+    torch.cuda.synchronize()
+    got, want = logits.cpu().numpy()
+    assert np.isfinite(got).all() and rel_err(got, want) < FREE_RUN_TOL, rel_err(got, want)
