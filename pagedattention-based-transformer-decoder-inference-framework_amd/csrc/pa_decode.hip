@@ -542,8 +542,9 @@ int choose_nsplit(int B, int H, int ntiles, int pps_fixed, long long resident,
 // o_proj GEMM after them.  `nsplit` in: what the rules above give; their fused form (2..8) may become any
 // of the three, the others stay what they are (the fused sums have a range, the GEMM's none).
 //
-// Lines from steps of 2 to 3 layers, rows x heads of D, the longest sequence held T, sequences that fill it
-// unless said; us a step, before -> now (with them the best fixed choice):
+// Lines from steps of 2 to 3 layers of one decoder alone, rows x heads of D, the longest sequence held T, sequences
+// that fill it unless said; us a step, before -> now (with them the best fixed choice).  "In turns": steps of three
+// decoders of 4 layers that overlap.
 //  * a fused workgroup reads D x hidden of W_o whatever its row's length, and its 4 waves (8 where that
 //    is 256 KB or more: two rounds of columns for 8) fit the chip 512 (256) times.  Past that one split of up
 //    to 128 pages: 64 x 16 of 128 T 720 476 -> 422, 48 x 12 of 64 T 720 194 -> 182, T 1,920 286 -> 261; below
@@ -552,13 +553,19 @@ int choose_nsplit(int B, int H, int ntiles, int pps_fixed, long long resident,
 //  * few pairs of long rows leave CUs idle, so splits over more workgroups: 4 x 16 of 128 T 1,920 241 ->
 //    216, T 8,192 with 2,048 held 246 -> 222; 16 x 4 of 64 T 8,300 180 -> 151 by 12.  Heads of 64 with 17 to
 //    64 pairs do so past 8,192 tokens, as a step's sequences may be far shorter than T (T 7,144 with 1,000
-//    held: 4 x 16 of 64 by 4 waves 120, 12 splits 134), more than 64 pairs of 128 never (three decoders in turns, 8 x 16
+//    held, in turns: 4 x 16 of 64 by 4 waves 120, 12 splits 134), more than 64 pairs of 128 never (in turns, 8 x 16
 //    T 7,144 with 1,000 held and more 220, 8 splits 228).  And 16 of them at most, 12 from 33 pairs on, not 24
-//    to 64 (1 x 8 of 128 T 7,144 with 1,000 held 103 -> 94, T 12,144 with 6,000 129 -> 118).
+//    to 64 (1 x 8 of 128 T 7,144 with 1,000 held 103 -> 94, T 12,144 with 6,000 129 -> 118; in turns 4 x 12 of 64 T
+//    14,336 with 8,192 119 -> 114, 16 x 4 121 -> 115, 3 x 16 with 9,000 141 -> 134).
+//    64 pairs of 128, whose W_o a fused workgroup's waves also read, gain alone and pay in turns, where the other decoders
+//    fill the CUs that one leaves idle, until their rows are long: 4 layers of 4 x 16, fused -> apart, alone and (in turns): T 1,920
+//    with 300 held 239 -> 235 (135.5 -> 141.2), 1,500 288 -> 265 (157.7 -> 163.7); T 7,144 with 1,000 267 -> 255
+//    (147.5 -> 155.4), 3,000 343 -> 296 (190.0 -> 192.1), 6,000 455 -> 351 (260.5 -> 248.9).  A step alone decides.
 //  * else 4 waves: 16 x 12 of 64 T 8,192 with 2,048 held 162 -> 156 (by 8), T 2,720 167 -> 161 (by 3).
-//    Up to 128 pairs as before (three decoders in turns, 4 layers, 5 x 16 of 64 T 6,644 by 7 101.5, by 4 111.0;
-//    10 x 12 T 7,644 118.5, 125.9; 12 x 16 by 8 157.1, by 4 155.4), and up to 32 KB of W_o, which one wave's columns cover (64 x 4 of 64 T 1,920 175; by 4 179; three
-//    decoders in turns, 16 x 4 T 6,744 with 600 held and more, by 8 76.4, by 4 85.5).
+//    Up to 128 pairs as before (in turns, 5 x 16 of 64 T 6,644 by 7 101.5, by 4 111.0;
+//    10 x 12 T 7,644 118.5, 125.9; 12 x 16 by 8 157.1, by 4 155.4), and up to 32 KB of W_o, which one wave's
+//    columns cover (64 x 4 of 64 T 1,920 175; by 4 179; in turns 16 x 4 T 6,744 with 600 held and more, by 8 76.4,
+//    by 4 85.5).
 struct F16Form {
   int nsplit;
   bool fused;
@@ -587,17 +594,18 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
 // fp32 rows that the o_proj quantises (hidden up to 2,048): splits that a workgroup merges (2..8) or a
 // merge launch does.  `nsplit` in: what the rules above give; half_round's stay.  Whole rounds of waves
 // make 9 to 95 splits of few pairs, most of them empty where the sequences are short of the longest held,
-// T, and merged in odd batches.  Steps of 2 layers, rows x heads of D, T (held), us, before -> now:
-//  * at most 16 up to 64 pairs (24 of more than 8 pairs of 128 past 9,600 tokens): 1 x 4 of 64 T 7,144 (1,000) 68 -> 62, T 12,144 (6,000) 93 -> 75; 1 x 16 of
-//    128 T 7,144 (1,000) 134 -> 125, T 4,520 (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 12, 16
+// T, and merged in odd batches.  Steps of 2 layers of one decoder alone, rows x heads of D, T (held), us, before ->
+// now; "in turns" as above:
+//  * at most 16 up to 64 pairs (24 of more than 8 pairs of 128 past 9,600 tokens): 1 x 4 of 64 T 7,144 (1,000) 68 ->
+//    62, T 12,144 (6,000) 93 -> 75; 1 x 16 of 128 T 7,144 (1,000) 134 -> 125, T 4,520 (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 12, 16
 //    in place of more than 16: 16 x 4 of 64 T 4,520 (4,500) 97 -> 95;
 //  * 8 up to 128: 8 x 16 of 128 T 4,520 (4,500) 243 -> 220, 32 x 4 of 64 146 -> 133; past that merged in the
 //    workgroup: 16 x 12 of 64 T 8,192 (2,048) 140 -> 133, T 12,144 (6,000) 217 -> 194;
-//  * 13 to 16 of 33 to 128 pairs stay: three decoders in turns, 4 layers, 16 x 4 of 64 T 6,744 14 splits 83.1, 16
+//  * 13 to 16 of 33 to 128 pairs stay: in turns, 16 x 4 of 64 T 6,744 14 splits 83.1, 16
 //    86.0; 32 x 4 T 7,144 14 splits 120.5, 8 125.6; 8 x 16 of 128 209.8, 212.7 (alone the same), where 25 x 4 T 10,144
 //    20 splits 147.9, 8 140.6; 3 x 16 T 12,144 24 splits 129.0, 16 122.3;
-//  * 257 to 512 pairs of 64: 4 in place of 8 (32 x 12 T 8,192 (2,048) 186 -> 177; 64 x 12 275 -> 257, but three
-//    decoders in turns 307 -> 313), and past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
+//  * 257 to 512 pairs of 64: 4 in place of 8 (32 x 12 T 8,192 (2,048) 186 -> 177; 64 x 12 275 -> 257, but in
+//    turns 307 -> 313), and past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
 struct F32Form {
   int nsplit;
   bool wgm;

@@ -420,13 +420,13 @@ bool pa_prefill_supported(const pa_kv_view* kv) {
          (kv->page_size == 16 || kv->page_size == 32);
 }
 
-// A plan has no more splits than split_bound and its stages allow, but fewer at one p0
-// than at a shorter one (2048 queries x 16 heads: three at p0 0, one from p0 2048 on), so
-// the size is of the most that any context up to this one takes.
 bool pa_prefill_one_pass(const pa_kv_view* kv, int p0, int m) {
   return pa_prefill_supported(kv) && m > 0 && p0 >= 0 && prefill_plan(kv, p0, m).nsplit == 1;
 }
 
+// A plan has no more splits than split_bound and its stages allow, but fewer at one p0
+// than at a shorter one (2048 queries x 16 heads: three at p0 0, one from p0 2048 on), so
+// the size is of the most that any context up to this one takes.
 size_t pa_prefill_ws_bytes(const pa_kv_view* kv, int p0, int m) {
   if (!pa_prefill_supported(kv) || m <= 0 || p0 < 0) return 0;
   const int most = (int)(((long long)p0 + m - 1) / stage_keys(kv->head_dim)) + 1;
