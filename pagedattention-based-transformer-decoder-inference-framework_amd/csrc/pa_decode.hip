@@ -537,6 +537,33 @@ int choose_nsplit(int B, int H, int ntiles, int pps_fixed, long long resident,
   return (int)std::min(ns, max_nsplit(B, H, ntiles));
 }
 
+// Splits of up to 32 pairs of row and head whose whole rounds of waves make more than a workgroup merges: a merge of
+// few parts costs less (steps are short beside it where T, the longest sequence held, is not filled), more waves read
+// long rows sooner.  4 layers, T (held), us by 16 / 24 / 32 / 48 / 64 splits and by whole rounds (how many), alone and (in
+// turns, three decoders' steps that overlap):
+//  * 1 x 4 of 64 T 14,336 (12,902) 163 / 153 / 150 / 154 / 161, rounds 182 (112) (67 / 63 / 61 / 61 / 63, 69); T 20,480
+//    (18,432) 190 / 171 / 164 / 163 / 166, 197 (128) (78 / 71 / 68 / 66 / 66, 74);
+//  * 1 x 12 of 64 T 4,500 (4,050) 155 / 158 / 161, 161 (36); T 7,144 (6,429) 170 / 168 / 171, 177 (43) (76 / 74 / 74, 75); T
+//    9,600 (1,440) 145 / 147 / 153, 153 (43), (8,640) 180 / 173 / 176, 182 (82 / 78 / 77, 79); T 32,000 (28,800) 273 / 238 / 228 / 224,
+//    235 (63) (140 / 123 / 116 / 111, 113); 1 x 8 T 20,480 (18,432) 211 / 191 / 185 / 184, 186 (64) (95 / 85 / 81 / 80, 79);
+//  * 1 x 8 of 128 T 7,144 (1,071) 157 / 165 / 164 / 177, 178 (56), (6,429) 206 / 198 / 197 / 208, 213 (104 / 99 / 97 / 99, 100): 16 as a step
+//    alone decides; T 9,600 (8,640) 224 / 211 / 208 / 215, 228 (64) (116 / 109 / 103 / 104, 106); T 14,336 (12,902) 263 / 236 /
+//    228 / 232, 241 (142 / 126 / 119 / 115, 115); T 32,000 (28,800) 400 / 332 / 303 / 285, 284 (233 / 195 / 174 / 158, 152);
+//  * 1 x 16 of 128 T 7,144 (1,071) 249 / 257, 257 (32) (138 / 140, 140), (6,429) 300 / 292, 295 (174 / 166, 165); T 12,144 (6,000)
+//    294 / 289, 292 (170 / 163, 162), (1,821) by 24 264, 269 (143, 145), (10,929) 325, 320 (194, 186); T 14,336 (12,902) 362 / 336, 329 (222 / 204, 197); T 32,000 (28,800) 508 / 443 / 416 / 420, 446 (63) (333 /
+//    297 / 283 / 273, 283).
+//  * 17 pairs and more: 2 x 16 of 128 T 14,336 (8,192) 331 / 329, 338 (28) (217 / 211, 213); of 64 16 (T 20,480 (18,500) 258, 293 (40)).
+int few_pairs_splits(long long bh, int D, int tiles, int nsplit) {
+  const bool wide = D > 64;
+  int n;
+  if (bh > 16) n = wide && tiles > 560 ? 24 : 16;
+  else if (tiles <= (wide ? (bh <= 8 ? 512 : 320) : (bh <= 4 ? 900 : 416))) n = 16;
+  else if (tiles <= (wide ? (bh <= 8 ? 0 : 760) : 624)) n = 24;
+  else if (wide && tiles <= 640) n = 32;
+  else n = bh > 8 || tiles <= (wide ? 960 : 1248) ? 48 : 64;
+  return std::min(n, nsplit);
+}
+
 // The FP16 decoder's attention and what its o_proj is: `nsplit` splits that a workgroup merges and
 // multiplies by the head's rows of W_o (fused), splits and a merge launch, or one split, both with an
 // o_proj GEMM after them.  `nsplit` in: what the rules above give; their fused form (2..8) may become any
@@ -554,9 +581,10 @@ int choose_nsplit(int B, int H, int ntiles, int pps_fixed, long long resident,
 //    216, T 8,192 with 2,048 held 246 -> 222; 16 x 4 of 64 T 8,300 180 -> 151 by 12.  Heads of 64 with 17 to
 //    64 pairs do so past 8,192 tokens, as a step's sequences may be far shorter than T (T 7,144 with 1,000
 //    held, in turns: 4 x 16 of 64 by 4 waves 120, 12 splits 134), more than 64 pairs of 128 never (in turns, 8 x 16
-//    T 7,144 with 1,000 held and more 220, 8 splits 228).  And 16 of them at most, 12 from 33 pairs on, not 24
-//    to 64 (1 x 8 of 128 T 7,144 with 1,000 held 103 -> 94, T 12,144 with 6,000 129 -> 118; in turns 4 x 12 of 64 T
-//    14,336 with 8,192 119 -> 114, 16 x 4 121 -> 115, 3 x 16 with 9,000 141 -> 134).
+//    T 7,144 with 1,000 held and more 220, 8 splits 228).  As many as
+//    few_pairs_splits says, and 12 from 33 pairs on, not 16 to 40 (in turns 4 x 12 of 64 T 14,336 with 8,192 119 -> 114, 16 x 4
+//    121 -> 115, 3 x 16 with 9,000 141 -> 134; 4 x 16 T 20,480 with 18,500 259 -> 238, of 128 505 -> 491; 3 x 16 of 128 there
+//    406 -> 416, alone 548 -> 517).
 //    64 pairs of 128, whose W_o a fused workgroup's waves also read, gain alone and pay in turns, where the other decoders
 //    fill the CUs that one leaves idle, until their rows are long: 4 layers of 4 x 16, fused -> apart, alone and (in turns): T 1,920
 //    with 300 held 239 -> 235 (135.5 -> 141.2), 1,500 288 -> 265 (157.7 -> 163.7); T 7,144 with 1,000 267 -> 255
@@ -580,7 +608,7 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
   const bool apart = D > 64 ? tiles > (bh <= 64 ? 45 : INT_MAX)
                             : tiles > (bh <= 16 ? 110 : bh <= 64 ? 512 : INT_MAX);
   if (nsplit > 1 && apart) {
-    int n = bh <= 32 ? (fits ? 8 : 16) : D > 64 && tiles <= 256 ? 8 : 12;
+    int n = bh <= 32 ? (fits ? 8 : few_pairs_splits(bh, D, tiles, nsplit)) : D > 64 && tiles <= 256 ? 8 : 12;
     if (!fits) n = std::min(n, nsplit);
     if ((long long)n * kMaxPps >= tiles) return {n, false};
   }
@@ -596,9 +624,9 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
 // make 9 to 95 splits of few pairs, most of them empty where the sequences are short of the longest held,
 // T, and merged in odd batches.  Steps of 2 layers of one decoder alone, rows x heads of D, T (held), us, before ->
 // now; "in turns" as above:
-//  * at most 16 up to 64 pairs (24 of more than 8 pairs of 128 past 9,600 tokens): 1 x 4 of 64 T 7,144 (1,000) 68 ->
-//    62, T 12,144 (6,000) 93 -> 75; 1 x 16 of 128 T 7,144 (1,000) 134 -> 125, T 4,520 (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 12, 16
-//    in place of more than 16: 16 x 4 of 64 T 4,520 (4,500) 97 -> 95;
+//  * few_pairs_splits up to 32 pairs: 1 x 4 of 64 T 7,144 (1,000) 68 -> 62, T 12,144 (6,000) 93 -> 75; 1 x 16 of 128 T 4,520
+//    (4,500) 144 -> 143; from 33 pairs on 12 in place of 9 to 12, 16 in place of more than 16: 16 x 4 of 64 T 4,520
+//    (4,500) 97 -> 95; 4 layers in turns, 4 x 12 T 32,000 (29,000) 275 -> 249, 3 x 16 of 128 554 -> 525;
 //  * 8 up to 128: 8 x 16 of 128 T 4,520 (4,500) 243 -> 220, 32 x 4 of 64 146 -> 133; past that merged in the
 //    workgroup: 16 x 12 of 64 T 8,192 (2,048) 140 -> 133, T 12,144 (6,000) 217 -> 194;
 //  * 13 to 16 of 33 to 128 pairs stay: in turns, 16 x 4 of 64 T 6,744 14 splits 83.1, 16
@@ -615,8 +643,7 @@ F32Form f32_step_form(long long bh, int D, int tiles, int nsplit) {
   if (nsplit >= 2 && bh > 512 && tiles <= kMaxPps) return {1, false};
   if (wgm) return {D <= 64 && bh > 256 && bh <= 512 && tiles <= 4 * kMaxPps ? std::min(nsplit, 4) : nsplit, true};
   if (bh > 32 && bh <= 128 && nsplit > 12 && nsplit <= 16) return {nsplit, wgm};
-  const int few = D > 64 && bh > 8 && tiles > 600 ? 24 : 16;
-  const int n = bh <= 32 ? std::min(nsplit, few) : bh <= 64 ? (nsplit > 16 ? 16 : 12) : 8;
+  const int n = bh <= 32 ? few_pairs_splits(bh, D, tiles, nsplit) : bh <= 64 ? (nsplit > 16 ? 16 : 12) : 8;
   if ((long long)n * kMaxPps < tiles) return {nsplit, false};
   return {n, bh > 128};
 }

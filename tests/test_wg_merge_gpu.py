@@ -176,6 +176,9 @@ def test_fused_oproj(gpu, ctx, H, D, ts):
     (16, 16, 128, 700, 8, 35),
     (4, 16, 128, 1900, 8, 2), (4, 16, 128, 4500, 12, 2), (1, 8, 128, 8192, 16, 2),
     (32, 16, 128, 2100, 4, 2),
+    # few pairs: more splits the longer the longest sequence
+    (1, 4, 64, 14400, 16, 2), (1, 4, 64, 14500, 48, 2), (1, 4, 64, 20000, 64, 2), (1, 12, 64, 6700, 24, 2),
+    (1, 8, 128, 8300, 32, 2), (1, 8, 128, 16000, 64, 2), (1, 16, 128, 12300, 32, 2), (2, 16, 128, 9600, 19, 2),
 ], ids=str)
 def test_f16_step_forms(gpu, B, H, D, S, nsplit, form):
     """The forms an FP16 decoder's attention takes by rows, heads and the longest sequence, one and
@@ -200,7 +203,8 @@ def test_f16_step_forms(gpu, B, H, D, S, nsplit, form):
 
 @pytest.mark.parametrize("B,H,D,S,nsplit,form", [
     (64, 12, 64, 700, 1, 0), (48, 12, 64, 8100, 4, 3), (16, 12, 64, 8300, 8, 3),  # past 512, 256, 128 pairs
-    (1, 4, 64, 12100, 16, 1), (1, 8, 64, 12100, 16, 1), (1, 16, 128, 12100, 24, 1), (4, 12, 64, 4600, 12, 1), (16, 4, 64, 7100, 14, 1), (16, 4, 64, 9000, 16, 1),
+    (1, 4, 64, 12100, 16, 1), (1, 8, 64, 6000, 16, 1), (1, 16, 128, 12100, 24, 1), (4, 12, 64, 4600, 12, 1), (16, 4, 64, 7100, 14, 1), (16, 4, 64, 9000, 16, 1),
+    (1, 8, 64, 10100, 48, 1), (1, 8, 128, 10300, 48, 1), (1, 16, 64, 9900, 24, 1), (1, 16, 128, 12300, 32, 1),
     (8, 16, 128, 4600, 8, 1), (2, 3, 64, 90, 1, 0), (16, 16, 128, 700, 2, 3),
 ], ids=str)
 def test_int8_step_forms(gpu, oracle, B, H, D, S, nsplit, form):
