@@ -589,6 +589,10 @@ int few_pairs_splits(long long bh, int D, int tiles, int nsplit) {
 //    fill the CUs that one leaves idle, until their rows are long: 4 layers of 4 x 16, fused -> apart, alone and (in turns): T 1,920
 //    with 300 held 239 -> 235 (135.5 -> 141.2), 1,500 288 -> 265 (157.7 -> 163.7); T 7,144 with 1,000 267 -> 255
 //    (147.5 -> 155.4), 3,000 343 -> 296 (190.0 -> 192.1), 6,000 455 -> 351 (260.5 -> 248.9).  A step alone decides.
+//    Less than 512 KB of W_o is no load to part with for short rows: 8 x 8 of 128 T 800 with 120 held 139 -> 149 (74.9 -> 78.1), T
+//    1,920 with 288 145 -> 154 (77.5 -> 81.6), 1,728 199 -> 182 (100.8 -> 106.5), T 4,500 with 675 160 -> 165 (84.3 -> 87.7),
+//    4,050 285 -> 227 (142 -> 149); 4 x 8 T 800 with 120 134 -> 144 (71 -> 74): apart past 4,096 tokens there.
+//    9 to 12 splits of 33 to 64 pairs stay (4 x 12 of 128 T 4,000 with 3,600 held 261, by 8 270; 600 held 212, 210).
 //  * else 4 waves: 16 x 12 of 64 T 8,192 with 2,048 held 162 -> 156 (by 8), T 2,720 167 -> 161 (by 3).
 //    Up to 128 pairs as before (in turns, 5 x 16 of 64 T 6,644 by 7 101.5, by 4 111.0;
 //    10 x 12 T 7,644 118.5, 125.9; 12 x 16 by 8 157.1, by 4 155.4), and up to 32 KB of W_o, which one wave's
@@ -605,10 +609,10 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
                         : kb >= 256 ? (bh > 256 ? 20 : 0)
                                     : (bh > 400 ? 25 : bh > 256 ? 10 : 0);
   if (fits && tiles <= kMaxPps && (bh > 512 || tiles <= one)) return {1, false};
-  const bool apart = D > 64 ? tiles > (bh <= 64 ? 45 : INT_MAX)
+  const bool apart = D > 64 ? tiles > (bh > 64 ? INT_MAX : fits && kb < 512 ? 256 : 45)
                             : tiles > (bh <= 16 ? 110 : bh <= 64 ? 512 : INT_MAX);
   if (nsplit > 1 && apart) {
-    int n = bh <= 32 ? (fits ? 8 : few_pairs_splits(bh, D, tiles, nsplit)) : D > 64 && tiles <= 256 ? 8 : 12;
+    int n = bh <= 32 ? (fits ? 8 : few_pairs_splits(bh, D, tiles, nsplit)) : D > 64 && fits && tiles <= 256 ? 8 : 12;
     if (!fits) n = std::min(n, nsplit);
     if ((long long)n * kMaxPps >= tiles) return {n, false};
   }

@@ -176,6 +176,7 @@ def test_fused_oproj(gpu, ctx, H, D, ts):
     (16, 16, 128, 700, 8, 35),
     (4, 16, 128, 1900, 8, 2), (4, 16, 128, 4500, 12, 2), (1, 8, 128, 8192, 16, 2),
     (32, 16, 128, 2100, 4, 2),
+    (4, 12, 128, 4000, 11, 2), (4, 8, 128, 800, 8, 35), (8, 8, 128, 4090, 8, 35), (8, 8, 128, 4500, 12, 2),  # a smaller W_o stays fused
     # few pairs: more splits the longer the longest sequence
     (1, 4, 64, 14400, 16, 2), (1, 4, 64, 14500, 48, 2), (1, 4, 64, 20000, 64, 2), (1, 12, 64, 6700, 24, 2),
     (1, 8, 128, 8300, 32, 2), (1, 8, 128, 16000, 64, 2), (1, 16, 128, 12300, 32, 2), (2, 16, 128, 9600, 19, 2),
