@@ -638,13 +638,15 @@ F16Form f16_step_form(long long bh, int D, int hidden, int tiles, int nsplit) {
 //    20 splits 147.9, 8 140.6; 3 x 16 T 12,144 24 splits 129.0, 16 122.3;
 //  * 257 to 512 pairs of 64: 4 in place of 8 (32 x 12 T 8,192 (2,048) 186 -> 177; 64 x 12 275 -> 257, but in
 //    turns 307 -> 313), and past 512 pairs one for up to 128 pages (64 x 12 T 720 163 -> 157, 64 x 16 of 128 303 -> 299).
+//    Two and a half waves a CU of heads of 128 end unevenly where they are long: 4 layers of 40 x 16, T 1,920 (1,728) 622 ->
+//    609, in turns 499 -> 543, so below three a CU up to 720 tokens.
 struct F32Form {
   int nsplit;
   bool wgm;
 };
 F32Form f32_step_form(long long bh, int D, int tiles, int nsplit) {
   const bool wgm = nsplit <= kWgmMaxSplits;
-  if (nsplit >= 2 && bh > 512 && tiles <= kMaxPps) return {1, false};
+  if (nsplit >= 2 && bh > 512 && tiles <= (D > 64 && bh < 768 ? 45 : kMaxPps)) return {1, false};
   if (wgm) return {D <= 64 && bh > 256 && bh <= 512 && tiles <= 4 * kMaxPps ? std::min(nsplit, 4) : nsplit, true};
   if (bh > 32 && bh <= 128 && nsplit > 12 && nsplit <= 16) return {nsplit, wgm};
   const int n = bh <= 32 ? few_pairs_splits(bh, D, tiles, nsplit) : bh <= 64 ? (nsplit > 16 ? 16 : 12) : 8;

@@ -205,6 +205,7 @@ def test_f16_step_forms(gpu, B, H, D, S, nsplit, form):
 @pytest.mark.parametrize("B,H,D,S,nsplit,form", [
     (64, 12, 64, 700, 1, 0), (48, 12, 64, 8100, 4, 3), (16, 12, 64, 8300, 8, 3),  # past 512, 256, 128 pairs
     (1, 4, 64, 12100, 16, 1), (1, 8, 64, 6000, 16, 1), (1, 16, 128, 12100, 24, 1), (4, 12, 64, 4600, 12, 1), (16, 4, 64, 7100, 14, 1), (16, 4, 64, 9000, 16, 1),
+    (40, 16, 128, 700, 1, 0), (40, 16, 128, 1000, 2, 3),
     (1, 8, 64, 10100, 48, 1), (1, 8, 128, 10300, 48, 1), (1, 16, 64, 9900, 24, 1), (1, 16, 128, 12300, 32, 1),
     (8, 16, 128, 4600, 8, 1), (2, 3, 64, 90, 1, 0), (16, 16, 128, 700, 2, 3),
 ], ids=str)
